@@ -109,8 +109,16 @@ int resolve_algo(int algo, int T, int H, int E, int k, int I, int dtype, bool co
   return BIBO_OK;
 }
 
+// Whether the generic family's fp32 tile kernels take a shape, given 16-byte aligned operands.  Their pre-activations
+// [S, 2I] lie where the slot rows [S, H] go later (the last segment of the workspace).
+inline bool generic_tiles(int H, int I, int dtype) {
+  return tile_f32_supported(H, I) && (dtype == BIBO_DTYPE_F32 || !mfma_supported(H, I, dtype));
+}
+
 struct Workspace {
-  size_t hist, idx, w, counts, offsets, perm_slot, perm_token, hidden, gu, yw, total;
+  size_t hist, idx, w, counts, offsets, perm_slot, perm_token, hidden, gu, yw;
+  size_t least;        // with room for the slot rows only: what every kernel family can do with
+  size_t total;
 };
 
 Workspace carve(int T, int H, int E, int k, int I, int dtype) {
@@ -128,8 +136,9 @@ Workspace carve(int T, int H, int E, int k, int I, int dtype) {
   ws.hidden = o;     o += align_up(S * (size_t)I * elt_size(dtype));
   // bf16 gate/up pre-activations, only ever used when the streaming kernels are eligible
   ws.gu = o;         o += align_up(stream_possible(T, H, E, k, I, dtype, true) ? S * (size_t)2 * I * sizeof(bf16_t) : 0);
-  ws.yw = o;         o += align_up(S * (size_t)H * sizeof(float));
-  ws.total = o;
+  ws.yw = o;
+  ws.least = o + align_up(S * (size_t)H * sizeof(float));
+  ws.total = o + align_up(S * (size_t)(generic_tiles(H, I, dtype) && 2 * I > H ? 2 * I : H) * sizeof(float));
   return ws;
 }
 
@@ -168,8 +177,8 @@ int down_dispatch(const void* hidden, const void* wd, const float* w, const int3
 int experts_dispatch(const void* x, const void* wgu, const void* wd, const float* theta, const int32_t* idx,
                      const float* w, const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token,
                      const void* residual, bool idx_trusted, int T, int H, int Eg, int np, int nn, int k, int I, int dtype,
-                     int algo, int act, int flags, void* out, char* base, const Workspace& ws, hipStream_t s,
-                     void* preact = nullptr) {
+                     int algo, int act, int flags, void* out, char* base, const Workspace& ws, size_t ws_bytes,
+                     hipStream_t s, void* preact = nullptr) {
   float* yw = reinterpret_cast<float*>(base + ws.yw);
   CombineArgs ca;
   ca.residual = residual;
@@ -192,6 +201,14 @@ int experts_dispatch(const void* x, const void* wgu, const void* wd, const float
     hipError_t e = launch_experts_fused(x, wgu, wd, theta, w, offsets, perm_slot, perm_token, T, H, Eg, k, I, act, yw, preact, s);
     if (e != hipSuccess) return (int)e;
     return hip_rc(launch_combine(yw, 1, ca, T, H, k, dtype, out, s));
+  }
+  // (a bf16 shape of the MFMA families that a caller asks the generic one for runs the row kernels, like the stage calls)
+  if (algo == BIBO_ALGO_GENERIC && generic_tiles(H, I, dtype) && aligned16(x) && aligned16(wgu) && aligned16(wd) &&
+      ws_bytes >= ws.total) {
+    hipError_t e = launch_experts_tiled(x, wgu, wd, theta, w, offsets, perm_slot, perm_token, T, H, Eg, k, I, dtype, act, yw,
+                                        base + ws.hidden, yw, s);
+    if (e != hipSuccess) return (int)e;
+    return hip_rc(launch_combine(yw, 0, ca, T, H, k, dtype, out, s));
   }
   const int rc = gateup_dispatch(x, wgu, theta, offsets, perm_token, T, H, Eg, k, I, dtype, algo, act, base + ws.hidden, s);
   if (rc != BIBO_OK) return rc;
@@ -240,7 +257,7 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
   if (T > 0 && (!x || !w_router || !bias || !w_gate_up || !w_down || !out)) return BIBO_ERR_NULL_POINTER;
   if (T > 0 && !theta && sh->act != BIBO_ACT_SILU) return BIBO_ERR_NULL_POINTER;
   const Workspace ws = carve(T, H, E, k, I, dtype);
-  if (workspace_bytes < ws.total) return BIBO_ERR_WORKSPACE_TOO_SMALL;
+  if (workspace_bytes < ws.least) return BIBO_ERR_WORKSPACE_TOO_SMALL;
   char* base = static_cast<char*>(workspace);
   hipStream_t s = static_cast<hipStream_t>(stream);
   int32_t* idx = idx_out ? idx_out : reinterpret_cast<int32_t*>(base + ws.idx);
@@ -283,7 +300,7 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
   }
   if (T == 0) return BIBO_OK;
   return experts_dispatch(x, w_gate_up, w_down, theta, idx, w, offsets, perm_slot, perm_token, residual, true, T, H, Eg,
-                          sh->n_pos, sh->n_neg, k, I, dtype, a, sh->act, sh->flags, out, base, ws, s, preact);
+                          sh->n_pos, sh->n_neg, k, I, dtype, a, sh->act, sh->flags, out, base, ws, workspace_bytes, s, preact);
 }
 
 
@@ -577,7 +594,7 @@ int bibo_moe_experts_fwd(const void* x, const int32_t* idx, const float* w, cons
   if (T > 0 && (!x || !idx || !w || !w_gate_up || !w_down || !out)) return BIBO_ERR_NULL_POINTER;
   if (T > 0 && !theta && sh->act != BIBO_ACT_SILU) return BIBO_ERR_NULL_POINTER;
   const Workspace ws = carve(T, H, E, k, I, dtype);
-  if (workspace_bytes < ws.total) return BIBO_ERR_WORKSPACE_TOO_SMALL;
+  if (workspace_bytes < ws.least) return BIBO_ERR_WORKSPACE_TOO_SMALL;
   char* base = static_cast<char*>(workspace);
   hipStream_t s = static_cast<hipStream_t>(stream);
   int32_t* counts = counts_out ? counts_out : reinterpret_cast<int32_t*>(base + ws.counts);
@@ -591,7 +608,7 @@ int bibo_moe_experts_fwd(const void* x, const int32_t* idx, const float* w, cons
     return rc;
   if (T == 0) return BIBO_OK;
   return experts_dispatch(x, w_gate_up, w_down, theta, idx, w, offsets, perm_slot, perm_token, nullptr, false, T, H, Eg,
-                          sh->n_pos, sh->n_neg, k, I, dtype, a, sh->act, 0, out, base, ws, s);
+                          sh->n_pos, sh->n_neg, k, I, dtype, a, sh->act, 0, out, base, ws, workspace_bytes, s);
 }
 
 int bibo_moe_forward(const void* x, const void* w_router, const float* bias, const void* w_gate_up, const void* w_down,
@@ -609,7 +626,7 @@ int bibo_moe_forward_static(const void* x, const void* w_router, const float* bi
   if (sh == nullptr) return BIBO_ERR_NULL_POINTER;
   int rc = check_dims(sh->T, sh->H, sh->E, sh->k, sh->I, sh->dtype, sh->n_pos, sh->n_neg);
   if (rc != BIBO_OK) return rc;
-  if (carve(sh->T, sh->H, sh->E, sh->k, sh->I, sh->dtype).total > (size_t)BIBO_MOE_STATIC_SCRATCH_BYTES)
+  if (carve(sh->T, sh->H, sh->E, sh->k, sh->I, sh->dtype).least > (size_t)BIBO_MOE_STATIC_SCRATCH_BYTES)
     return BIBO_ERR_STATIC_SCRATCH;
   void* ws = nullptr;
   if ((rc = static_scratch(&ws)) != BIBO_OK) return rc;
@@ -692,11 +709,16 @@ int bibo_moe_backward(const void* x, const void* d_out, const void* w_router, co
     int32_t* g_offsets = reinterpret_cast<int32_t*>(gb + gw.offsets);
     int32_t* g_slot = reinterpret_cast<int32_t*>(gb + gw.perm_slot);
     int32_t* g_token = reinterpret_cast<int32_t*>(gb + gw.perm_token);
+    int32_t* g_counts = reinterpret_cast<int32_t*>(gb + gw.counts);
+    int32_t* g_hist = reinterpret_cast<int32_t*>(gb + gw.hist);
+    int hist_tokens = 0;
+    const bool want_hist = T > 0 && permute_takes_router_hist(T, k);
     if (T > 0 && (rc = hip_rc(launch_router(x, w_router, bias, T, H, E, k, sh->dtype, norm_mode, g_logits, g_idx, g_w, nullptr,
-                                            nullptr, nullptr, gs))) != BIBO_OK)
+                                            want_hist ? g_hist : nullptr, &hist_tokens, gs))) != BIBO_OK)
       return rc;
-    if ((rc = hip_rc(launch_permute(g_idx, T, E, k, reinterpret_cast<int32_t*>(gb + gw.counts), g_offsets, g_slot, g_token,
-                                    gb + gw.hist, gs))) != BIBO_OK)
+    if ((rc = hip_rc((want_hist && hist_tokens > 0)
+                         ? launch_permute_from_hist(g_idx, T, E, k, g_hist, hist_tokens, g_counts, g_offsets, g_slot, g_token, gs)
+                         : launch_permute(g_idx, T, E, k, g_counts, g_offsets, g_slot, g_token, g_hist, gs))) != BIBO_OK)
       return rc;
     GenericBackwardBuffers g;
     g.dgu = reinterpret_cast<float*>(gb + gw.dgu); g.hw = reinterpret_cast<float*>(gb + gw.hw);

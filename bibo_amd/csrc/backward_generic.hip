@@ -3,10 +3,11 @@
 // gradients in fp32 at tiny sizes, tests/test_moe.py:53-63, ablate/common/test_eager_radial.py:63-69) and sizes that
 // are no multiples of 128.  The gradients are those torch.autograd derives for the eager layer
 // (src/modeling/ffn/moe.py:46-101,157-183, src/modeling/ffn/router.py:25-47) with the selection held fixed; the
-// formulas are the ones spelled out at the top of backward.hip.  One workgroup per routed row for the row-wise part,
-// one workgroup per weight row for the weight gradients, which loop over an expert's rows in permuted order: every sum
-// has a fixed order, so the results are the same bits on every call.
-#include "common.h"
+// formulas are the ones spelled out at the top of backward.hip.  Sizes that are multiples of four run on the fp32 MFMA
+// GEMMs of tile_f32.h with a row-wise activation kernel between them; the rest takes one workgroup per routed row for the
+// row-wise part and one workgroup per weight row for the weight gradients, which loop over an expert's rows in permuted
+// order.  Every sum has a fixed order, so the results are the same bits on every call.
+#include "tile_f32.h"
 
 namespace bibo {
 namespace {
@@ -121,87 +122,196 @@ __global__ __launch_bounds__(256) void row_bwd_generic_kernel(const TIn* __restr
   }
 }
 
-// +/-Identity experts (moe.py:95-99): dw[slot] = sign <d_out[t], x[t]>, dxs[slot] = sign w[slot] d_out[t].  One
-// workgroup per permuted row behind the GLU experts' rows.
+// Radial NormSiLU backward of one permuted row per wave (formulas at the top of row_bwd_generic_kernel and backward.hip), in
+// place: gu [S, 2I] holds [g, u] and receives [dg, du], dhp [S, I] holds dh' and receives w h.  The row is read three times,
+// from L1 after the first.
+__global__ __launch_bounds__(256) void act_bwd_f32_kernel(float* __restrict__ gu, float* __restrict__ dhp,
+                                                          const float* __restrict__ w, const float* __restrict__ theta,
+                                                          const int32_t* __restrict__ offsets,
+                                                          const int32_t* __restrict__ perm_slot, int S, int E, int I, int act,
+                                                          float* __restrict__ dw_slot, float* __restrict__ dtheta_row) {
+  const int lane = threadIdx.x & 63;
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= S) return;
+  const int e = expert_of_row(offsets, E, row);
+  if (e < 0) return;
+  const int slot = perm_slot[row];
+  const float ws = w[slot];
+  float* gr = gu + (size_t)row * 2 * I;
+  float* dr = dhp + (size_t)row * I;
+  float ss = 0.f;
+  for (int c = lane * 4; c < I; c += 4 * kWave) {
+    const floatx4 g = load4<float>(gr + c);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) ss = fmaf(g[q], g[q], ss);
+  }
+  ss = wave_sum(ss);
+  const bool radial = act != BIBO_ACT_SILU;
+  float p = 0.f, r = 1.f, gain = 1.f;
+  if (radial) {
+    p = radial_exponent(theta, e, act);
+    r = sqrtf(ss / (float)I + kNormSiluEps);         // moe.py:88
+    gain = powf(r, p);
+  }
+  const float rinv = 1.f / r;
+  float dot_h = 0.f, sum_qa = 0.f, inner = 0.f;
+  for (int c = lane * 4; c < I; c += 4 * kWave) {
+    const floatx4 g = load4<float>(gr + c), u = load4<float>(gr + I + c), d = load4<float>(dr + c);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float z = g[q] * rinv, s = 1.f / (1.f + expf(-z));
+      const float a = z * s, ad = s * (1.f + z * (1.f - s));
+      dot_h = fmaf(d[q], gain * a * u[q], dot_h);
+      const float qq = ws * d[q] * u[q];
+      sum_qa = fmaf(qq, a, sum_qa);
+      inner = fmaf(qq, gain * rinv * (p * a - ad * z), inner);
+    }
+  }
+  dot_h = wave_sum(dot_h);
+  sum_qa = wave_sum(sum_qa);
+  inner = wave_sum(inner);
+  for (int c = lane * 4; c < I; c += 4 * kWave) {
+    const floatx4 g = load4<float>(gr + c), u = load4<float>(gr + I + c), d = load4<float>(dr + c);
+    floatx4 og, ou, oh;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float z = g[q] * rinv, s = 1.f / (1.f + expf(-z));
+      const float a = z * s, ad = s * (1.f + z * (1.f - s));
+      const float dh = ws * d[q];
+      float dg = dh * u[q] * gain * rinv * ad;
+      if (radial) dg = fmaf(g[q] * rinv / (float)I, inner, dg);
+      og[q] = dg;
+      ou[q] = dh * gain * a;
+      oh[q] = ws * gain * a * u[q];
+    }
+    store4(gr + c, og);
+    store4(gr + I + c, ou);
+    store4(dr + c, oh);
+  }
+  if (lane == 0) {
+    dw_slot[slot] = dot_h;
+    const float dp = act == BIBO_ACT_RADIAL_TANH ? 1.f - p * p : p * (1.f - p);
+    dtheta_row[row] = radial ? dp * logf(r) * gain * sum_qa : 0.f;
+  }
+}
+
+// Everything per token behind the experts, one wave per token: the combine-weight gradients of +/-Identity slots
+// (sign <d_out[t], x[t]>, moe.py:95-99), dlogit of the k selected experts (router.py:31,41-47; w_router == NULL: none), and
+//   dx[t, h] = sum_j dx of slot j + sum_j dl[t, j] W_router[idx[t, j], h]
+// where the dx of a slot is its dxs row or, for an Identity slot, sign w d_out[t].  A slot whose expert id lies outside
+// [0, E + n_pos + n_neg) is left out and its dw_slot entry is set to zero.
 template <typename TIn>
-__global__ __launch_bounds__(256) void special_bwd_generic_kernel(const TIn* __restrict__ x, const TIn* __restrict__ d_out,
-                                                                  const float* __restrict__ w,
+__global__ __launch_bounds__(256) void token_bwd_generic_kernel(const TIn* __restrict__ x, const TIn* __restrict__ d_out,
+                                                                const float* __restrict__ dxs, const float* __restrict__ logits,
+                                                                const int32_t* __restrict__ idx, const float* __restrict__ w,
+                                                                const TIn* __restrict__ w_router, int T, int H, int E, int n_pos,
+                                                                int n_neg, int k, int norm_mode, float* __restrict__ dw_slot,
+                                                                float* __restrict__ dl, TIn* __restrict__ dx) {
+  const int lane = threadIdx.x & 63;
+  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (t >= T) return;
+  const int Et = E + n_pos + n_neg;
+  // lane j < k holds slot j
+  int e_ = -1;
+  float w_ = 0.f, dw_ = 0.f, s_ = 0.f;
+  if (lane < k) {
+    e_ = idx[t * k + lane];
+    w_ = w[t * k + lane];
+    if (e_ < 0 || e_ >= Et) e_ = -1;
+    if (e_ >= 0 && e_ < E) dw_ = dw_slot[t * k + lane];
+    if (w_router != nullptr) s_ = 1.f / (1.f + expf(-logits[(size_t)t * Et + e_]));
+  }
+  if (__ballot(e_ >= E) != 0ull) {
+    float dot = 0.f;
+    for (int h = lane; h < H; h += kWave) dot = fmaf(to_float(d_out[(size_t)t * H + h]), to_float(x[(size_t)t * H + h]), dot);
+    dot = wave_sum(dot);
+    if (e_ >= E) dw_ = e_ < E + n_pos ? dot : -dot;
+  }
+  if (lane < k && (e_ < 0 || e_ >= E)) dw_slot[t * k + lane] = dw_;
+  float dl_ = 0.f;
+  if (w_router != nullptr) {
+    float sum = 0.f, dot = 0.f;
+    for (int j = 0; j < k; ++j) {
+      sum += __shfl(s_, j, kWave);
+      dot = fmaf(__shfl(dw_, j, kWave), __shfl(w_, j, kWave), dot);
+    }
+    float ds = dw_;
+    if (k > 1 && norm_mode == BIBO_NORM_SUM) ds = (ds - dot) / (sum + 1e-20f);
+    else if (k > 1 && norm_mode == BIBO_NORM_SOFTMAX) ds = w_ * (ds - dot);
+    dl_ = ds * s_ * (1.f - s_);
+    if (lane < k) dl[t * k + lane] = dl_;
+  }
+  int ej[kMaxK];                                     // the k slots, the same in every lane
+  float wj[kMaxK], dlj[kMaxK];
+#pragma unroll
+  for (int j = 0; j < kMaxK; ++j) {
+    ej[j] = j < k ? __builtin_amdgcn_readlane(e_, j) : -1;
+    wj[j] = __shfl(w_, j, kWave);
+    dlj[j] = __shfl(dl_, j, kWave);
+  }
+  for (int h = lane; h < H; h += kWave) {
+    float acc = 0.f;
+#pragma unroll
+    for (int j = 0; j < kMaxK; ++j) {
+      const int e = ej[j];
+      if (e < 0) continue;
+      if (e < E) acc += dxs[((size_t)t * k + j) * H + h];
+      else acc = fmaf(e < E + n_pos ? wj[j] : -wj[j], to_float(d_out[(size_t)t * H + h]), acc);
+      if (w_router != nullptr) acc = fmaf(dlj[j], to_float(w_router[(size_t)e * H + h]), acc);
+    }
+    dx[(size_t)t * H + h] = from_float<TIn>(acc);
+  }
+}
+
+// grid (Et, ceil(H / 64) + 1).  Blocks y < ceil(H / 64): dW_router[e, h] = sum over the rows r of expert e of dl[slot(r)]
+// x[token(r), h] for 64 columns: 16 row groups of 16 threads x 4 columns, the groups' sums added in order (dwr == NULL: none).
+// The last y: dtheta[e] = the sum of its rows' shares (e < E).
+template <typename TIn>
+__global__ __launch_bounds__(256) void expert_sums_generic_kernel(const TIn* __restrict__ x, const float* __restrict__ dl,
                                                                   const int32_t* __restrict__ offsets,
                                                                   const int32_t* __restrict__ perm_slot,
-                                                                  const int32_t* __restrict__ perm_token, int Eg, int n_pos,
-                                                                  int n_neg, int H, float* __restrict__ dw_slot,
-                                                                  float* __restrict__ dxs) {
-  __shared__ float red[4];
-  const int row = offsets[Eg] + blockIdx.x;
-  if (row >= offsets[Eg + n_pos + n_neg]) return;
-  const float sign = row < offsets[Eg + n_pos] ? 1.f : -1.f;
-  const int slot = perm_slot[row];
-  const size_t t = (size_t)perm_token[row];
-  const float sw = sign * w[slot];
-  float dot = 0.f;
-  for (int h = threadIdx.x; h < H; h += 256) {
-    const float dv = to_float(d_out[t * H + h]);
-    dot = fmaf(dv, to_float(x[t * H + h]), dot);
-    dxs[(size_t)slot * H + h] = sw * dv;
+                                                                  const int32_t* __restrict__ perm_token, int H, int E,
+                                                                  const float* __restrict__ dtheta_row,
+                                                                  float* __restrict__ dtheta, TIn* __restrict__ dwr) {
+  __shared__ float red[16][65];
+  const int e = blockIdx.x, tid = threadIdx.x;
+  const int lo = offsets[e], hi = offsets[e + 1];
+  if (blockIdx.y + 1 == gridDim.y) {
+    if (e >= E) return;
+    float acc = 0.f;
+    for (int r = lo + tid; r < hi; r += 256) acc += dtheta_row[r];
+    acc = block_sum(acc, red[0]);
+    if (tid == 0) dtheta[e] = acc;
+    return;
   }
-  dot = block_sum(dot, red);
-  if (threadIdx.x == 0) dw_slot[slot] = sign * dot;
-}
-
-// dtheta[e] = sum of its rows' contributions, in row order
-__global__ __launch_bounds__(256) void dtheta_generic_kernel(const float* __restrict__ dtheta_row,
-                                                             const int32_t* __restrict__ offsets,
-                                                             float* __restrict__ dtheta) {
-  __shared__ float red[4];
-  const int e = blockIdx.x;
-  float acc = 0.f;
-  for (int r = offsets[e] + threadIdx.x; r < offsets[e + 1]; r += 256) acc += dtheta_row[r];
-  acc = block_sum(acc, red);
-  if (threadIdx.x == 0) dtheta[e] = acc;
-}
-
-// One thread per token: dlogit of the k selected experts from the gradients of the combine weights (router.py:31,41-47).
-__global__ void router_bwd_generic_kernel(const float* __restrict__ logits, const int32_t* __restrict__ idx,
-                                          const float* __restrict__ w, const float* __restrict__ dw, int T, int E, int k,
-                                          int norm_mode, float* __restrict__ dl) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= T) return;
-  float s[kMaxK], sum = 0.f, dot = 0.f;
-  for (int j = 0; j < k; ++j) {
-    s[j] = 1.f / (1.f + expf(-logits[(size_t)t * E + idx[t * k + j]]));
-    sum += s[j];
-    dot = fmaf(dw[t * k + j], w[t * k + j], dot);
-  }
-  for (int j = 0; j < k; ++j) {
-    float dsc = dw[t * k + j];
-    if (k > 1 && norm_mode == BIBO_NORM_SUM) dsc = (dsc - dot) / (sum + 1e-20f);
-    else if (k > 1 && norm_mode == BIBO_NORM_SOFTMAX) dsc = w[t * k + j] * (dsc - dot);
-    dl[t * k + j] = dsc * s[j] * (1.f - s[j]);
-  }
-}
-
-// dx[t, h] = sum_j dxs[t k + j, h] + sum_j dl[t, j] W_router[idx[t, j], h].  dl == NULL: the slot rows alone.  A slot
-// whose expert id lies outside [0, n_experts) has no dxs row: left out, and its dw_slot entry is set to zero.
-template <typename TIn>
-__global__ __launch_bounds__(256) void dx_combine_generic_kernel(const float* __restrict__ dxs, const float* __restrict__ dl,
-                                                                 const int32_t* __restrict__ idx,
-                                                                 const TIn* __restrict__ w_router, int T, int H, int k,
-                                                                 int n_experts, float* __restrict__ dw_slot,
-                                                                 TIn* __restrict__ dx) {
-  const long long gid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= (long long)T * H) return;
-  const int t = (int)(gid / H), h = (int)(gid - (long long)t * H);
-  float acc = 0.f;
-  for (int j = 0; j < k; ++j) {
-    const int e = idx[t * k + j];
-    if (e < 0 || e >= n_experts) {
-      if (h == 0) dw_slot[t * k + j] = 0.f;
-      continue;
+  if (dwr == nullptr) return;
+  const int rl = tid >> 4, c4 = (tid & 15) * 4, h0 = blockIdx.y * 64;
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  constexpr int kU = 4;                                        // rows of a thread whose loads are in flight together
+  for (int r = lo + rl; r < hi; r += 16 * kU) {
+    float d[kU], v[kU][4];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int rr = r + 16 * u;
+      d[u] = rr < hi ? dl[perm_slot[rr]] : 0.f;
+      const size_t t = rr < hi ? perm_token[rr] : 0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[u][q] = rr < hi && h0 + c4 + q < H ? to_float(x[t * H + h0 + c4 + q]) : 0.f;
     }
-    acc += dxs[((size_t)t * k + j) * H + h];
-    if (dl != nullptr) acc = fmaf(dl[t * k + j], to_float(w_router[(size_t)e * H + h]), acc);
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc[q] = fmaf(d[u], v[u][q], acc[q]);
   }
-  dx[(size_t)t * H + h] = from_float<TIn>(acc);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) red[rl][c4 + q] = acc[q];
+  __syncthreads();
+  if (tid < 64 && h0 + tid < H) {
+    float sum = 0.f;
+#pragma unroll
+    for (int g = 0; g < 16; ++g) sum += red[g][tid];
+    dwr[(size_t)e * H + h0 + tid] = from_float<TIn>(sum);
+  }
 }
 
 // dW[e][n][m] = sum over the rows r of expert e, in row order, of P[srcP(r)][n] Q[srcQ(r)][m]; grid = (N, E), threads
@@ -222,22 +332,6 @@ __global__ __launch_bounds__(256) void wgrad_generic_kernel(const TP* __restrict
       if (m < M) acc = fmaf(pv, to_float(Q[(size_t)(GATHER_Q ? ix : r) * M + m]), acc);
     }
     if (m < M) dW[((size_t)e * N + n) * M + m] = from_float<TOut>(acc);
-  }
-}
-
-// dW_router[e, h] = sum over the rows r of expert e, in row order, of dl[slot(r)] x[token(r), h]; grid = E.
-template <typename TIn>
-__global__ __launch_bounds__(256) void dwr_generic_kernel(const TIn* __restrict__ x, const float* __restrict__ dl,
-                                                          const int32_t* __restrict__ offsets,
-                                                          const int32_t* __restrict__ perm_slot,
-                                                          const int32_t* __restrict__ perm_token, int H,
-                                                          TIn* __restrict__ dwr) {
-  const int e = blockIdx.x;
-  const int lo = offsets[e], hi = offsets[e + 1];
-  for (int h = threadIdx.x; h < H; h += 256) {
-    float acc = 0.f;
-    for (int r = lo; r < hi; ++r) acc = fmaf(dl[perm_slot[r]], to_float(x[(size_t)perm_token[r] * H + h]), acc);
-    dwr[(size_t)e * H + h] = from_float<TIn>(acc);
   }
 }
 
@@ -273,23 +367,31 @@ hipError_t launch_t(const void* x_, const void* d_out_, const void* w_router_, c
     zero_elems(static_cast<TIn*>(d_wd_), (size_t)E * H * I, s);
     return hipGetLastError();
   }
-  const size_t shm = (size_t)(2 * H + 5 * I) * sizeof(float);
-  hipLaunchKernelGGL(row_bwd_generic_kernel<TIn>, dim3(S), dim3(256), shm, s, x, d_out, wgu, wd, theta, w, offsets, perm_slot,
-                     perm_token, H, E, I, act, b.dgu, b.hw, b.dxs, b.dw_slot, b.dtheta_row);
-  hipLaunchKernelGGL(dtheta_generic_kernel, dim3(E), dim3(256), 0, s, b.dtheta_row, offsets, d_theta);
-  if (n_pos + n_neg > 0)   // (as many workgroups as there could be rows: how many there are is only known on the device)
-    hipLaunchKernelGGL(special_bwd_generic_kernel<TIn>, dim3(S), dim3(256), 0, s, x, d_out, w, offsets, perm_slot, perm_token, E,
-                       n_pos, n_neg, H, b.dw_slot, b.dxs);
+  const bool tiles = tile_f32_supported(H, I) && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(d_out) |
+                                                    reinterpret_cast<uintptr_t>(wgu) | reinterpret_cast<uintptr_t>(wd)) & 15) == 0;
+  hipError_t err = hipSuccess;
+  if (tiles) {
+    // gu = x W_gate_up^T; dh' = d W_down; [dg, du] and w h in their places; dx of every slot = [dg, du] W_gate_up
+    if ((err = launch_ggemm_f32<TIn, TIn, false, true, false>(x, perm_token, wgu, offsets, nullptr, nullptr, S, H, 2 * I, E, b.dgu, s)) != hipSuccess) return err;
+    if ((err = launch_ggemm_f32<TIn, TIn, true, true, false>(d_out, perm_token, wd, offsets, nullptr, nullptr, S, H, I, E, b.hw, s)) != hipSuccess) return err;
+    hipLaunchKernelGGL(act_bwd_f32_kernel, dim3((S + 3) / 4), dim3(256), 0, s, b.dgu, b.hw, w, theta, offsets, perm_slot, S, E, I, act,
+                       b.dw_slot, b.dtheta_row);
+    if ((err = launch_ggemm_f32<float, TIn, true, false, true>(b.dgu, nullptr, wgu, offsets, perm_slot, nullptr, S, 2 * I, H, E, b.dxs, s)) != hipSuccess) return err;
+  } else {
+    const size_t shm = (size_t)(2 * H + 5 * I) * sizeof(float);
+    hipLaunchKernelGGL(row_bwd_generic_kernel<TIn>, dim3(S), dim3(256), shm, s, x, d_out, wgu, wd, theta, w, offsets, perm_slot,
+                       perm_token, H, E, I, act, b.dgu, b.hw, b.dxs, b.dw_slot, b.dtheta_row);
+  }
   const bool with_router = w_router != nullptr;      // else: the experts alone, the caller owns the routing
-  if (with_router)
-    hipLaunchKernelGGL(router_bwd_generic_kernel, dim3((T + 255) / 256), dim3(256), 0, s, logits, idx, w, b.dw_slot, T, Et, k,
-                       norm_mode, b.dl);
-  hipLaunchKernelGGL(dx_combine_generic_kernel<TIn>, dim3((unsigned)(((long long)T * H + 255) / 256)), dim3(256), 0, s, b.dxs,
-                     with_router ? b.dl : nullptr, idx, w_router, T, H, k, Et, b.dw_slot, static_cast<TIn*>(dx_));
-  if (with_router)
-    hipLaunchKernelGGL(dwr_generic_kernel<TIn>, dim3(Et), dim3(256), 0, s, x, b.dl, offsets, perm_slot, perm_token, H,
-                       static_cast<TIn*>(d_w_router_));
+  hipLaunchKernelGGL(token_bwd_generic_kernel<TIn>, dim3((T + 3) / 4), dim3(256), 0, s, x, d_out, b.dxs, logits, idx, w, w_router, T,
+                     H, E, n_pos, n_neg, k, norm_mode, b.dw_slot, b.dl, static_cast<TIn*>(dx_));
+  hipLaunchKernelGGL(expert_sums_generic_kernel<TIn>, dim3(Et, (H + 63) / 64 + 1), dim3(256), 0, s, x, b.dl, offsets, perm_slot,
+                     perm_token, H, E, b.dtheta_row, d_theta, with_router ? static_cast<TIn*>(d_w_router_) : nullptr);
   // dW_down[e] = d^T (w h), d gathered by token; dW_gate_up[e] = [dg, du]^T x, x gathered by token
+  if (tiles) {
+    if ((err = launch_wgrad_f32<TIn, float, TIn, true, false>(d_out, b.hw, perm_token, offsets, H, I, E, static_cast<TIn*>(d_wd_), s)) != hipSuccess) return err;
+    return launch_wgrad_f32<float, TIn, TIn, false, true>(b.dgu, x, perm_token, offsets, 2 * I, H, E, static_cast<TIn*>(d_wgu_), s);
+  }
   hipLaunchKernelGGL((wgrad_generic_kernel<TIn, float, TIn, true, false>), dim3(H, E), dim3(256), 0, s, d_out, b.hw, perm_token,
                      offsets, H, I, static_cast<TIn*>(d_wd_));
   hipLaunchKernelGGL((wgrad_generic_kernel<float, TIn, TIn, false, true>), dim3(2 * I, E), dim3(256), 0, s, b.dgu, x, perm_token,

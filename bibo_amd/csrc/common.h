@@ -181,6 +181,10 @@ hipError_t launch_gateup_generic(const void* x, const void* wgu, const float* th
 hipError_t launch_down_generic(const void* hidden, const void* wd, const float* w, const int32_t* offsets,
                                const int32_t* perm_slot, int T, int H, int E, int k, int I, int dtype, float* yw,
                                hipStream_t s);
+bool tile_f32_supported(int H, int I);
+hipError_t launch_experts_tiled(const void* x, const void* wgu, const void* wd, const float* theta, const float* w,
+                                const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int T, int H,
+                                int E, int k, int I, int dtype, int act, float* gu, void* hidden, float* yw, hipStream_t s);
 // What the combine folds in besides the slot rows; every pointer may be NULL (see combine_kernel).
 struct CombineArgs {
   const int32_t* idx = nullptr;    // [T,k]; needed for specials and for skipping out-of-range slots

@@ -1,8 +1,9 @@
-// Generic expert kernels: one workgroup per routed row, any H and I, bf16 or fp32 operands, fp32
-// accumulation.  They serve shapes the MFMA tiles do not cover and fp32 modules, and double as an
-// independent implementation the MFMA kernels are cross-checked against.
+// Generic expert kernels: any H and I, bf16 or fp32 operands, fp32 arithmetic.  They serve shapes the bf16 MFMA
+// tiles do not cover and fp32 modules, and double as an independent implementation the MFMA kernels are cross-checked
+// against.  Two ways through them: grouped GEMMs on fp32 MFMAs (tile_f32.h) for sizes that are multiples of four, and one
+// workgroup per routed row for the rest and for the stage entry points, which have no room for pre-activations.
 // Follow BiBoFusedExperts.forward, src/modeling/ffn/moe.py:73-101 of the reference.
-#include "common.h"
+#include "tile_f32.h"
 
 namespace bibo {
 namespace {
@@ -87,6 +88,39 @@ __global__ __launch_bounds__(256) void down_generic_kernel(const TIn* __restrict
   }
 }
 
+// hidden[row, :] = r^p SiLU(g/r) up (moe.py:87-92) from the fp32 pre-activations gu [S, 2I], one wave per permuted row.
+// Bound by memory (a row is read twice, the second time from L1): 4 rows per workgroup keep enough loads in flight.
+template <typename TIn>
+__global__ __launch_bounds__(256) void activate_f32_kernel(const float* __restrict__ gu, const float* __restrict__ theta,
+                                                           const int32_t* __restrict__ offsets, int S, int E, int I, int act,
+                                                           TIn* __restrict__ hidden) {
+  const int lane = threadIdx.x & 63;
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= S) return;
+  const int e = expert_of_row(offsets, E, row);
+  if (e < 0) return;
+  const float* g = gu + (size_t)row * 2 * I;
+  float ss = 0.f;
+  for (int c = lane * 4; c < I; c += 4 * kWave) {
+    const floatx4 v = load4<float>(g + c);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) ss = fmaf(v[q], v[q], ss);
+  }
+  ss = wave_sum(ss);
+  const float r = act == BIBO_ACT_SILU ? 1.f : sqrtf(ss / (float)I + kNormSiluEps);   // moe.py:88
+  const float gain = act == BIBO_ACT_SILU ? 1.f : powf(r, radial_exponent(theta, e, act));
+  for (int c = lane * 4; c < I; c += 4 * kWave) {
+    const floatx4 v = load4<float>(g + c), u = load4<float>(g + I + c);
+    floatx4 h;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float z = v[q] / r;
+      h[q] = z / (1.f + expf(-z)) * gain * u[q];                       // SiLU(g/r) r^p up
+    }
+    store4(hidden + (size_t)row * I + c, h);
+  }
+}
+
 // out[t, :] = round(residual[t, :] + sum_j contribution(t, j))  in fp32, ascending j   (moe.py:93-101; the residual
 // add of the caller, src/modeling/layers.py:62, when `residual` is given).  contribution = yw[t*k + j, :] for a GLU
 // expert; with `idx` given, +/- w[t,j] * x[t, :] for a +/-Identity special (moe.py:95-99) and nothing for an index
@@ -161,10 +195,13 @@ __global__ __launch_bounds__(256) void combine_bf16x8_kernel(const bf16_t* __res
   }
 }
 
-// fp32 slot rows -> bf16 output, 4 columns per thread: the decode-size combine, whose duration is one round trip of
+// fp32 slot rows -> bf16 or fp32 output, 4 columns per thread: the decode-size combine, whose duration is one round trip of
 // its loads, issues a quarter of the threads and all k loads of a thread at once.  Same sum as combine_kernel.
+template <typename TOut>
 __global__ __launch_bounds__(256) void combine_f32x4_kernel(const float* __restrict__ yw, CombineArgs a, int T, int H4,
-                                                            int k, bf16_t* __restrict__ out) {
+                                                            int k, TOut* __restrict__ out) {
+  const TOut* x = static_cast<const TOut*>(a.x);
+  const TOut* residual = static_cast<const TOut*>(a.residual);
   const size_t n = (size_t)T * H4;
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
     const size_t t = i / H4, c = i - t * H4;
@@ -175,7 +212,7 @@ __global__ __launch_bounds__(256) void combine_f32x4_kernel(const float* __restr
 #pragma unroll
     for (int j = 0; j < kMaxK; ++j)
       if (j < k) {
-        special[j] = special_slot<bf16_t>(a, t * k + j, &sign[j]);
+        special[j] = special_slot<TOut>(a, t * k + j, &sign[j]);
         if (!special[j]) v[j] = src[(size_t)j * H4];
       }
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
@@ -185,22 +222,21 @@ __global__ __launch_bounds__(256) void combine_f32x4_kernel(const float* __restr
         if (special[j]) {
           if (sign[j] != 0) {
             const float sw = (float)sign[j] * a.w[t * k + j];
-            const bf16x4 xv = reinterpret_cast<const bf16x4*>(a.x)[i];
+            const floatx4 xv = load4<TOut>(x + i * 4);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) acc[q] += sw * (float)xv[q];
+            for (int q = 0; q < 4; ++q) acc[q] += sw * xv[q];
           }
         } else {
 #pragma unroll
           for (int q = 0; q < 4; ++q) acc[q] += v[j][q];
         }
       }
-    if (a.residual != nullptr) {
-      const bf16x4 r = reinterpret_cast<const bf16x4*>(a.residual)[i];
+    if (residual != nullptr) {
+      const floatx4 r = load4<TOut>(residual + i * 4);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) acc[q] = (a.round_block ? (float)(bf16_t)acc[q] : acc[q]) + (float)r[q];
+      for (int q = 0; q < 4; ++q) acc[q] = (a.round_block ? to_float(from_float<TOut>(acc[q])) : acc[q]) + r[q];
     }
-    bf16x4 o = {(bf16_t)acc[0], (bf16_t)acc[1], (bf16_t)acc[2], (bf16_t)acc[3]};
-    reinterpret_cast<bf16x4*>(out)[i] = o;
+    store4(out + i * 4, floatx4{acc[0], acc[1], acc[2], acc[3]});
   }
 }
 
@@ -238,6 +274,33 @@ hipError_t launch_down_generic(const void* hidden, const void* wd, const float* 
   return hipGetLastError();
 }
 
+bool tile_f32_supported(int H, int I) { return H % 4 == 0 && I % 4 == 0; }
+
+// The experts of the generic family as three launches: gu = x W_gate_up^T (fp32, [S, 2I], permuted rows), the activation,
+// yw[slot] = w[slot] hidden W_down^T.  `gu` may share its memory with `yw`.  At T = 2048, H = 768, E = 64, k = 6, I = 384 in
+// fp32 the row kernels took 5088 + 2688 us: every routed row read its expert's 3.5 MB through one CU.
+template <typename TIn>
+static hipError_t launch_experts_tiled_t(const TIn* x, const TIn* wgu, const TIn* wd, const float* theta, const float* w,
+                                         const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int S,
+                                         int H, int E, int I, int act, float* gu, TIn* hidden, float* yw, hipStream_t s) {
+  hipError_t err = launch_ggemm_f32<TIn, TIn, false, true, false>(x, perm_token, wgu, offsets, nullptr, nullptr, S, H, 2 * I, E, gu, s);
+  if (err != hipSuccess) return err;
+  hipLaunchKernelGGL(activate_f32_kernel<TIn>, dim3((S + 3) / 4), dim3(256), 0, s, gu, theta, offsets, S, E, I, act, hidden);
+  return launch_ggemm_f32<TIn, TIn, false, false, true>(hidden, nullptr, wd, offsets, perm_slot, w, S, I, H, E, yw, s);
+}
+
+hipError_t launch_experts_tiled(const void* x, const void* wgu, const void* wd, const float* theta, const float* w,
+                                const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int T, int H,
+                                int E, int k, int I, int dtype, int act, float* gu, void* hidden, float* yw, hipStream_t s) {
+  const int S = T * k;
+  if (S == 0) return hipSuccess;
+  if (dtype == BIBO_DTYPE_BF16)
+    return launch_experts_tiled_t(static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(wgu), static_cast<const bf16_t*>(wd), theta,
+                                  w, offsets, perm_slot, perm_token, S, H, E, I, act, gu, static_cast<bf16_t*>(hidden), yw, s);
+  return launch_experts_tiled_t(static_cast<const float*>(x), static_cast<const float*>(wgu), static_cast<const float*>(wd), theta, w,
+                                offsets, perm_slot, perm_token, S, H, E, I, act, gu, static_cast<float*>(hidden), yw, s);
+}
+
 hipError_t launch_combine(const void* yw, int yw_is_bf16, const CombineArgs& a, int T, int H, int k, int dtype,
                           void* out, hipStream_t s) {
   const size_t n = (size_t)T * H;
@@ -254,19 +317,21 @@ hipError_t launch_combine(const void* yw, int yw_is_bf16, const CombineArgs& a, 
     } else
       hipLaunchKernelGGL((combine_kernel<bf16_t, bf16_t>), dim3(grid), dim3(256), 0, s,
                          static_cast<const bf16_t*>(yw), a, T, H, k, static_cast<bf16_t*>(out));
-  } else if (dtype == BIBO_DTYPE_BF16) {
-    if ((H % 4) == 0 && ((reinterpret_cast<uintptr_t>(yw) | reinterpret_cast<uintptr_t>(out) |
-                          reinterpret_cast<uintptr_t>(a.residual) | reinterpret_cast<uintptr_t>(a.x)) & 15) == 0) {
-      const size_t n4 = n / 4;
-      const int g4 = (int)((n4 + 255) / 256 < 65536 ? (n4 + 255) / 256 : 65536);
-      hipLaunchKernelGGL(combine_f32x4_kernel, dim3(g4), dim3(256), 0, s, static_cast<const float*>(yw), a, T, H / 4, k,
-                         static_cast<bf16_t*>(out));
-    } else
-      hipLaunchKernelGGL((combine_kernel<float, bf16_t>), dim3(grid), dim3(256), 0, s, static_cast<const float*>(yw), a, T,
-                         H, k, static_cast<bf16_t*>(out));
   } else {
-    hipLaunchKernelGGL((combine_kernel<float, float>), dim3(grid), dim3(256), 0, s, static_cast<const float*>(yw), a, T,
-                       H, k, static_cast<float*>(out));
+    const bool vec = (H % 4) == 0 && ((reinterpret_cast<uintptr_t>(yw) | reinterpret_cast<uintptr_t>(out) |
+                                       reinterpret_cast<uintptr_t>(a.residual) | reinterpret_cast<uintptr_t>(a.x)) & 15) == 0;
+    const size_t n4 = n / 4;
+    const int g4 = (int)((n4 + 255) / 256 < 65536 ? (n4 + 255) / 256 : 65536);
+    const float* yp = static_cast<const float*>(yw);
+    if (dtype == BIBO_DTYPE_BF16) {
+      bf16_t* op = static_cast<bf16_t*>(out);
+      if (vec) hipLaunchKernelGGL(combine_f32x4_kernel<bf16_t>, dim3(g4), dim3(256), 0, s, yp, a, T, H / 4, k, op);
+      else hipLaunchKernelGGL((combine_kernel<float, bf16_t>), dim3(grid), dim3(256), 0, s, yp, a, T, H, k, op);
+    } else {
+      float* op = static_cast<float*>(out);
+      if (vec) hipLaunchKernelGGL(combine_f32x4_kernel<float>, dim3(g4), dim3(256), 0, s, yp, a, T, H / 4, k, op);
+      else hipLaunchKernelGGL((combine_kernel<float, float>), dim3(grid), dim3(256), 0, s, yp, a, T, H, k, op);
+    }
   }
   return hipGetLastError();
 }

@@ -1,141 +1,12 @@
 // Kernel 1: fused router.  fp32 logits x @ w_router^T, canonical sigmoid, selection on score + bias
 // (ties to the lowest expert index), gather of the unbiased scores, normalisation.
 // Follows BiBoMoERouter.forward, src/modeling/ffn/router.py:25-51 of the reference.
-#include "common.h"
+#include "tile_f32.h"
 
 namespace bibo {
 namespace {
 
 constexpr int kRowPad = kMaxE + 1;   // LDS row stride (floats): lane = token reads are conflict-free
-
-// One lane owns one token: scan the E scores in ascending expert order and keep the k best
-// (score + bias) in a sorted register list.  Strict '>' keeps the earlier, i.e. lower-index, expert
-// ahead of an equal later one, which is the tie rule.  Emits experts in ascending index order.
-__device__ __forceinline__ void select_row(const float* __restrict__ sc, const float* __restrict__ bias_s, int E,
-                                           int k, int norm_mode, int32_t* __restrict__ idx_out,
-                                           float* __restrict__ w_out, float* __restrict__ gap_out) {
-  float sel[kMaxK];
-  int id[kMaxK];
-#pragma unroll
-  for (int j = 0; j < kMaxK; ++j) { sel[j] = -INFINITY; id[j] = j; }
-  for (int e = 0; e < E; ++e) {
-    const float v = sc[e] + bias_s[e];                       // router.py:38
-#pragma unroll
-    for (int j = kMaxK - 1; j >= 0; --j) {
-      if (j < k) {
-        const bool gt_prev = (j > 0) && (v > sel[j > 0 ? j - 1 : 0]);
-        if (gt_prev) { sel[j] = sel[j - (j > 0)]; id[j] = id[j - (j > 0)]; }
-        else if (v > sel[j]) { sel[j] = v; id[j] = e; }
-      }
-    }
-  }
-  unsigned long long mask = 0;
-#pragma unroll
-  for (int j = 0; j < kMaxK; ++j)
-    if (j < k) mask |= 1ull << id[j];
-  // ascending expert order; weights are the UNBIASED scores (router.py:41)
-  float raw[kMaxK];
-  float sum = 0.f, mx = -INFINITY;
-  unsigned long long m = mask;
-#pragma unroll
-  for (int j = 0; j < kMaxK; ++j) {
-    raw[j] = 0.f;
-    if (j < k) {
-      const int e = __ffsll((long long)m) - 1;
-      m &= m - 1;
-      idx_out[j] = e;
-      raw[j] = sc[e];
-      sum += raw[j];                                         // sequential fp32 adds, ascending expert
-      mx = fmaxf(mx, raw[j]);
-    }
-  }
-  if (k > 1 && norm_mode == BIBO_NORM_SOFTMAX) {             // router.py:42-43
-    float ex[kMaxK];
-    float es = 0.f;
-#pragma unroll
-    for (int j = 0; j < kMaxK; ++j) { ex[j] = (j < k) ? expf(raw[j] - mx) : 0.f; es += ex[j]; }
-#pragma unroll
-    for (int j = 0; j < kMaxK; ++j) if (j < k) w_out[j] = ex[j] / es;
-  } else if (k > 1 && norm_mode == BIBO_NORM_SUM) {          // router.py:44-45
-    const float den = sum + kSumNormEps;
-#pragma unroll
-    for (int j = 0; j < kMaxK; ++j) if (j < k) w_out[j] = raw[j] / den;
-  } else {                                                   // router.py:46-47
-#pragma unroll
-    for (int j = 0; j < kMaxK; ++j) if (j < k) w_out[j] = raw[j];
-  }
-  if (gap_out != nullptr) {                                  // router.py:33-36, unbiased scores
-    float top[kMaxK + 1];
-#pragma unroll
-    for (int j = 0; j <= kMaxK; ++j) top[j] = -INFINITY;
-    for (int e = 0; e < E; ++e) {
-      const float v = sc[e];
-#pragma unroll
-      for (int j = kMaxK; j >= 0; --j) {
-        if (j <= k) {
-          const bool gt_prev = (j > 0) && (v > top[j > 0 ? j - 1 : 0]);
-          if (gt_prev) top[j] = top[j - (j > 0)];
-          else if (v > top[j]) top[j] = v;
-        }
-      }
-    }
-    float a = 0.f, b = 0.f;
-#pragma unroll
-    for (int j = 0; j <= kMaxK; ++j) { if (j == k - 1) a = top[j]; if (j == k) b = top[j]; }
-    *gap_out = (k < E) ? (a - b) : 0.f;
-  }
-}
-
-// ---- generic router: any H, bf16 or fp32 inputs, plain FMA -------------------------------------
-constexpr int kGenTokens = 64;
-
-template <typename TIn>
-__global__ __launch_bounds__(256) void router_generic_kernel(const TIn* __restrict__ x, const TIn* __restrict__ wr,
-                                                             const float* __restrict__ bias, int T, int H, int E, int k,
-                                                             int norm_mode, float* __restrict__ logits,
-                                                             int32_t* __restrict__ idx, float* __restrict__ w,
-                                                             float* __restrict__ gap) {
-  __shared__ float sc[kGenTokens * kRowPad];
-  __shared__ float bias_s[kMaxE];
-  const int tid = threadIdx.x;
-  const int t0 = blockIdx.x * kGenTokens;
-  if (tid < kMaxE) bias_s[tid] = (tid < E) ? bias[tid] : 0.f;
-  {
-    const int tl = tid >> 2, q = tid & 3;
-    const int t = min(t0 + tl, T - 1);
-    float acc[kMaxE / 4];
-#pragma unroll
-    for (int j = 0; j < kMaxE / 4; ++j) acc[j] = 0.f;
-    const TIn* xr = x + (size_t)t * H;
-    for (int h = 0; h < H; ++h) {
-      const float xv = to_float(xr[h]);
-#pragma unroll
-      for (int j = 0; j < kMaxE / 4; ++j) {
-        const int e = q + 4 * j;
-        if (e < E) acc[j] = fmaf(xv, to_float(wr[(size_t)e * H + h]), acc[j]);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < kMaxE / 4; ++j) {
-      const int e = q + 4 * j;
-      if (e < E) sc[tl * kRowPad + e] = acc[j];
-    }
-  }
-  __syncthreads();
-  const int ntok = min(kGenTokens, T - t0);
-  for (int i = tid; i < ntok * E; i += 256) {
-    const int tl = i / E, e = i - tl * E;
-    const float lg = sc[tl * kRowPad + e];
-    if (logits != nullptr) logits[(size_t)(t0 + tl) * E + e] = lg;
-    sc[tl * kRowPad + e] = sigmoid32_canonical(lg);          // router.py:31
-  }
-  __syncthreads();
-  if (tid < ntok) {
-    const int t = t0 + tid;
-    select_row(sc + tid * kRowPad, bias_s, E, k, norm_mode, idx + (size_t)t * k, w + (size_t)t * k,
-               gap ? gap + t : nullptr);
-  }
-}
 
 // Integer key of a score whose unsigned order is the order of the floats (-0 counts as +0): the row-wide maximum
 // is then one v_max_u32 per butterfly step instead of a compare-and-select on (value, expert) pairs under exec
@@ -253,6 +124,110 @@ __device__ __forceinline__ unsigned long long select_tokens16(const float* __res
   return live ? mask : 0ull;
 }
 
+// Histogram of the selections of this workgroup's TOK tokens (16 threads each), for the permutation kernel.
+template <int TOK>
+__device__ __forceinline__ void write_chunk_hist(unsigned long long mask, int32_t* __restrict__ chunk_hist) {
+  __shared__ unsigned long long mask_s[TOK];
+  const int tid = threadIdx.x;
+  if ((tid & 15) == 0) mask_s[tid >> 4] = mask;
+  __syncthreads();
+  if (tid < kMaxE) {
+    int c = 0;
+#pragma unroll
+    for (int t = 0; t < TOK; ++t) c += (int)((mask_s[t] >> tid) & 1ull);
+    chunk_hist[blockIdx.x * kMaxE + tid] = c;
+  }
+}
+
+// ---- generic router: any H, bf16 or fp32 inputs, plain FMA -------------------------------------
+// One workgroup = 16 tokens x 64 experts; thread = 2 tokens x 2 experts.  K chunks of 64 elements pass through LDS (the next
+// one waits in registers meanwhile).  A logit is one chain of FMAs over ascending h, so it does not depend on the tiling.
+// Bound by its LDS reads, four 16-byte ones per sixteen FMAs; with 16 tokens per workgroup even a few hundred tokens
+// reach many CUs (64 tokens per workgroup and operands straight from memory: 940 us at T = 2048, H = 768 in fp32).
+// VEC: rows are 16-byte (bf16: 8-byte) aligned and H % 4 == 0.
+constexpr int kGenTokens = 16;
+constexpr int kGenKC = 64;
+
+template <typename TIn, bool VEC>
+__global__ __launch_bounds__(256) void router_fma_kernel(const TIn* __restrict__ x, const TIn* __restrict__ wr,
+                                                         const float* __restrict__ bias, int T, int H, int E, int k,
+                                                         int norm_mode, float* __restrict__ logits, int32_t* __restrict__ idx,
+                                                         float* __restrict__ w, float* __restrict__ gap,
+                                                         int32_t* __restrict__ chunk_hist) {
+  constexpr int kStride = kGenKC + 4;                          // floats: 16 rows of a 16-byte read hit distinct banks
+  __shared__ __attribute__((aligned(16))) float xs[kGenTokens * kStride];
+  __shared__ __attribute__((aligned(16))) float ws[kMaxE * kStride];
+  __shared__ float sc[kGenTokens * kRowPad];
+  __shared__ float bias_s[kMaxE];
+  const int tid = threadIdx.x;
+  const int t0 = blockIdx.x * kGenTokens;
+  if (tid < kMaxE) bias_s[tid] = (tid < E) ? bias[tid] : 0.f;
+  // fill side: thread = granule tid % 16 (four elements) of rows tid / 16 + 16 i; row group 0 = the tokens, 1 .. 4 = w_router
+  const int fr = tid >> 4, fc = (tid & 15) * 4;
+  const TIn* src[5];
+  bool live[5];
+#pragma unroll
+  for (int i = 0; i < 5; ++i) {
+    const int e = fr + 16 * (i - 1);
+    live[i] = i == 0 || e < E;
+    src[i] = i == 0 ? x + (size_t)min(t0 + fr, T - 1) * H : wr + (size_t)min(e, E - 1) * H;
+  }
+  floatx4 r[5];
+  auto load = [&](int h0) {
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+      r[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (VEC) {
+        if (live[i] && h0 + fc < H) r[i] = load4<TIn>(src[i] + h0 + fc);
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (live[i] && h0 + fc + q < H) r[i][q] = to_float(src[i][h0 + fc + q]);
+      }
+    }
+  };
+  const int e5 = tid & 31, tp = tid >> 5;                      // experts e5, e5 + 32; tokens tp, tp + 8
+  float acc[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
+  load(0);
+  for (int h0 = 0; h0 < H; h0 += kGenKC) {
+    *reinterpret_cast<floatx4*>(xs + fr * kStride + fc) = r[0];
+#pragma unroll
+    for (int i = 1; i < 5; ++i) *reinterpret_cast<floatx4*>(ws + (fr + 16 * (i - 1)) * kStride + fc) = r[i];
+    __syncthreads();
+    if (h0 + kGenKC < H) load(h0 + kGenKC);
+#pragma unroll
+    for (int h = 0; h < kGenKC; h += 4) {
+      floatx4 xv[2], wv[2];
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        xv[a] = *reinterpret_cast<const floatx4*>(xs + (tp + 8 * a) * kStride + h);
+        wv[a] = *reinterpret_cast<const floatx4*>(ws + (e5 + 32 * a) * kStride + h);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+          for (int b = 0; b < 2; ++b) acc[a][b] = fmaf(xv[a][q], wv[b][q], acc[a][b]);
+    }
+    __syncthreads();
+  }
+  const int ntok = min(kGenTokens, T - t0);
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int tl = tp + 8 * a, e = e5 + 32 * b;
+      if (tl < ntok && e < E) {
+        if (logits != nullptr) logits[(size_t)(t0 + tl) * E + e] = acc[a][b];
+        sc[tl * kRowPad + e] = sigmoid32_canonical(acc[a][b]);   // router.py:31
+      }
+    }
+  __syncthreads();
+  const unsigned long long mask = select_tokens16(sc, bias_s, E, k, norm_mode, t0, ntok, idx, w, gap);
+  if (chunk_hist != nullptr) write_chunk_hist<kGenTokens>(mask, chunk_hist);
+}
+
 // ---- MFMA router: bf16, H % 128 == 0 ------------------------------------------------------------
 // One workgroup = TOK tokens (16 or 32), TOK/16 x 4 waves: wave (tm, en) owns the 16x16 logits tile of
 // token tile tm and expert tile en over the whole K, so no partial sums cross waves and the fp32
@@ -290,17 +265,7 @@ __device__ __forceinline__ void router_finish(const floatx4& acc, float* sc, con
   }
   __syncthreads();
   const unsigned long long mask = select_tokens16(sc, bias_s, E, k, norm_mode, t0, ntok, idx, w, gap);
-  if (chunk_hist != nullptr) {           // histogram of this workgroup's selections, for the permutation kernel
-    __shared__ unsigned long long mask_s[TOK];
-    if ((tid & 15) == 0) mask_s[tid >> 4] = mask;
-    __syncthreads();
-    if (tid < kMaxE) {
-      int c = 0;
-#pragma unroll
-      for (int t = 0; t < TOK; ++t) c += (int)((mask_s[t] >> tid) & 1ull);
-      chunk_hist[blockIdx.x * kMaxE + tid] = c;
-    }
-  }
+  if (chunk_hist != nullptr) write_chunk_hist<TOK>(mask, chunk_hist);
 }
 
 template <int TOK>
@@ -492,7 +457,7 @@ __global__ __launch_bounds__(256) void router_mfma_split_kernel(const bf16_t* __
                                                                 const float* __restrict__ bias, int T, int H, int E,
                                                                 int k, int norm_mode, float* __restrict__ logits,
                                                                 int32_t* __restrict__ idx, float* __restrict__ w,
-                                                                float* __restrict__ gap) {
+                                                                float* __restrict__ gap, int32_t* __restrict__ chunk_hist) {
   __shared__ float part[4 * kMfmaTokens * kRowPad];
   __shared__ float sc[kMfmaTokens * kRowPad];
   __shared__ float bias_s[kMaxE];
@@ -548,7 +513,8 @@ __global__ __launch_bounds__(256) void router_mfma_split_kernel(const bf16_t* __
     }
   }
   __syncthreads();
-  select_tokens16(sc, bias_s, E, k, norm_mode, t0, ntok, idx, w, gap);
+  const unsigned long long mask = select_tokens16(sc, bias_s, E, k, norm_mode, t0, ntok, idx, w, gap);
+  if (chunk_hist != nullptr) write_chunk_hist<kMfmaTokens>(mask, chunk_hist);
 }
 
 }  // namespace
@@ -613,17 +579,27 @@ hipError_t launch_router(const void* x, const void* w_router, const float* bias,
                          chunk_hist);
     if (hist_tokens != nullptr && chunk_hist != nullptr) *hist_tokens = T >= 32 * 256 ? 32 : 16;
   } else if (dtype == BIBO_DTYPE_BF16 && (H % 32) == 0 && aligned) {
+    chunk_hist = T < 32 * 256 ? chunk_hist : nullptr;   // (one per 16 tokens: too many to add up for larger batches)
     const int grid = (T + kMfmaTokens - 1) / kMfmaTokens;
     hipLaunchKernelGGL(router_mfma_split_kernel, dim3(grid), dim3(256), 0, s, static_cast<const bf16_t*>(x),
-                       static_cast<const bf16_t*>(w_router), bias, T, H, E, k, norm_mode, logits, idx, w, gap);
+                       static_cast<const bf16_t*>(w_router), bias, T, H, E, k, norm_mode, logits, idx, w, gap, chunk_hist);
+    if (hist_tokens != nullptr && chunk_hist != nullptr) *hist_tokens = kMfmaTokens;
   } else {
-    const int grid = (T + kGenTokens - 1) / kGenTokens;
-    if (dtype == BIBO_DTYPE_BF16)
-      hipLaunchKernelGGL(router_generic_kernel<bf16_t>, dim3(grid), dim3(256), 0, s, static_cast<const bf16_t*>(x),
-                         static_cast<const bf16_t*>(w_router), bias, T, H, E, k, norm_mode, logits, idx, w, gap);
-    else
-      hipLaunchKernelGGL(router_generic_kernel<float>, dim3(grid), dim3(256), 0, s, static_cast<const float*>(x),
-                         static_cast<const float*>(w_router), bias, T, H, E, k, norm_mode, logits, idx, w, gap);
+    chunk_hist = T < 32 * 256 ? chunk_hist : nullptr;
+    const dim3 grid((T + kGenTokens - 1) / kGenTokens);
+    const bool vec = aligned && H % 4 == 0;
+    auto launch = [&](auto kernel, auto* xp) {
+      hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, xp, static_cast<decltype(xp)>(w_router), bias, T, H, E, k, norm_mode,
+                         logits, idx, w, gap, chunk_hist);
+    };
+    if (dtype == BIBO_DTYPE_BF16) {
+      const bf16_t* xp = static_cast<const bf16_t*>(x);
+      if (vec) launch(router_fma_kernel<bf16_t, true>, xp); else launch(router_fma_kernel<bf16_t, false>, xp);
+    } else {
+      const float* xp = static_cast<const float*>(x);
+      if (vec) launch(router_fma_kernel<float, true>, xp); else launch(router_fma_kernel<float, false>, xp);
+    }
+    if (hist_tokens != nullptr && chunk_hist != nullptr) *hist_tokens = kGenTokens;
   }
   return hipGetLastError();
 }

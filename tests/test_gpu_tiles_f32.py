@@ -1,0 +1,47 @@
+"""The fp32 tile kernels of the generic family (tile_f32.h) at the edges of their tiles: row counts around 16 and 64 per
+expert, widths below, at and past 64 columns, contractions that end inside a step of 32, widths that are no multiples of
+four (the row kernels), +/-Identity experts; forward and backward against the fp64 oracle."""
+import numpy as np
+import pytest
+import torch
+
+from bibo_amd import ops
+from oracle import bibo_moe_oracle as O
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+def _rel(a, ref):
+    return float((a.double().cpu() - ref.double()).abs().max() / ref.double().abs().max().clamp_min(1e-30))
+
+
+@pytest.mark.parametrize("T,H,Eg,pairs,k,I", [(1, 64, 8, 0, 2, 32), (12, 68, 2, 0, 2, 36), (24, 132, 4, 0, 2, 64), (63, 100, 2, 0, 1, 28),
+                                              (65, 64, 1, 1, 2, 64), (129, 192, 14, 1, 3, 88), (200, 66, 4, 0, 2, 33),
+                                              (17, 260, 64, 0, 8, 132), (300, 516, 5, 2, 4, 260)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_tile_edges(T, H, Eg, pairs, k, I, dtype):
+    E = Eg + 2 * pairs
+    p = O.make_inputs(T=T, H=H, E=Eg, k=min(k, Eg), I=I, theta="normal", seed=T + H, dtype=dtype)
+    g = torch.Generator().manual_seed(T)
+    p["w_router"] = (torch.randn(E, H, generator=g) * 0.1).to(dtype)
+    p["bias"] = torch.rand(E, generator=g) * 0.02 - 0.01
+    d_out = torch.randn(T, H, generator=g).to(dtype)
+    args = [p[n].to(DEV) for n in ("w_router", "bias", "w_gate_up", "w_down", "theta")]
+    kw = dict(n_pos=pairs, n_neg=pairs)
+    out, idx, w, counts, logits = ops.moe_forward(p["x"].to(DEV), *args, k, want_routing=True, want_counts=True, want_logits=True, **kw)
+    got = ops.moe_backward(p["x"].to(DEV), d_out.to(DEV), *args, k, want_dw=True, **kw)
+    torch.cuda.synchronize()
+    idx, w = idx.cpu().numpy(), w.cpu().numpy()
+    lg = p["x"].double() @ p["w_router"].double().t()
+    assert _rel(logits, lg) <= 1e-5
+    ri, rw = O.route_from_logits(logits.cpu().numpy(), p["bias"].numpy(), k)[:2]
+    assert np.array_equal(ri, idx) and np.array_equal(rw, w)
+    assert np.array_equal(np.bincount(ri.ravel(), minlength=E), counts.cpu().numpy())
+    tol = 1e-5 if dtype == torch.float32 else 2e-2
+    ref = O.experts_forward(p["x"], idx, w, p["w_gate_up"], p["w_down"], p["theta"], dtype=torch.float64, **kw)
+    assert _rel(out, ref) <= tol
+    grads = O.moe_backward(p["x"], p["w_router"], p["w_gate_up"], p["w_down"], p["theta"], idx, d_out, **kw)
+    # one token: a single cancelling dot product decides a tensor's largest entry
+    for name, a in zip(("x", "w_router", "w_gate_up", "w_down", "theta", "w"), got):
+        assert _rel(a, grads[name]) <= (tol if T > 1 else 4 * tol), name
