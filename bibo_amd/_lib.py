@@ -1,4 +1,4 @@
-"""ctypes binding of libbibo_moe.so (declared in include/bibo_moe.h).
+"""ctypes binding of libbibo_moe.so (declared in include/bibo_moe.h), and the loader of the modules' native host path.
 
 The library is the product: there is no Python or CPU fallback.  If it is missing, `lib()` raises."""
 from __future__ import annotations
@@ -24,7 +24,7 @@ SYMBOLS = (
     "bibo_moe_combine_fwd", "bibo_moe_combine_ex_fwd", "bibo_moe_experts_fwd", "bibo_moe_forward", "bibo_moe_rmsnorm_fwd",
     "bibo_moe_ffn_workspace_bytes", "bibo_moe_ffn_forward", "bibo_moe_forward_static", "bibo_moe_backward_workspace_bytes", "bibo_moe_backward", "bibo_moe_experts_backward",
     "bibo_moe_train_state_bytes", "bibo_moe_forward_train", "bibo_moe_backward_saved",
-    "bibo_moe_exp_attn_res_fwd",
+    "bibo_moe_exp_attn_res_fwd", "bibo_moe_balance_step",
 )
 STATIC_SCRATCH_BYTES = 16 << 20
 
@@ -37,6 +37,7 @@ class Shape(ctypes.Structure):
 
 _lock = threading.Lock()
 _lib = None
+_native = None
 
 
 def _declare(l):
@@ -88,6 +89,8 @@ def _declare(l):
                                           sz, vp]
     l.bibo_moe_exp_attn_res_fwd.restype = ci
     l.bibo_moe_exp_attn_res_fwd.argtypes = [vp, ci, vp, ctypes.c_float, ci, ci, ci, vp, vp]
+    l.bibo_moe_balance_step.restype = ci
+    l.bibo_moe_balance_step.argtypes = [vp, vp, vp, ci, ctypes.c_float, ci, vp]
     l.bibo_moe_forward_static.argtypes = [vp, vp, vp, vp, vp, vp, ctypes.POINTER(Shape), ci, ci, vp, vp, vp, vp, vp, vp]
     l.bibo_moe_forward.restype = ci
     l.bibo_moe_forward.argtypes = [vp, vp, vp, vp, vp, vp, ctypes.POINTER(Shape), ci, ci, vp, vp, vp, vp, vp, vp, sz, vp]
@@ -113,6 +116,22 @@ def lib():
                 raise RuntimeError(f"{LIB_PATH} has ABI {l.bibo_moe_abi_version()}, binding expects {ABI_VERSION}")
             _lib = l
     return _lib
+
+
+def native():
+    """The native host path of the modules (csrc/binding.cpp); raises RuntimeError if it has not been built."""
+    global _native
+    if _native is None:
+        lib()
+        try:
+            from . import _native as n
+        except ImportError as e:
+            raise RuntimeError(f"bibo_amd/_native.so cannot be loaded ({e}): build it with `python -m bibo_amd.build`. "
+                               "bibo_amd has no fallback path.") from e
+        if n.abi_version() != ABI_VERSION:
+            raise RuntimeError(f"bibo_amd/_native.so has ABI {n.abi_version()}, binding expects {ABI_VERSION}")
+        _native = n
+    return _native
 
 
 def check(code: int, what: str) -> None:

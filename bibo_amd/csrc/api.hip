@@ -833,6 +833,12 @@ int bibo_moe_experts_backward(const void* x, const void* d_out, const int32_t* i
                                 nullptr, d_w_gate_up, d_w_down, d_theta, s));
 }
 
+int bibo_moe_balance_step(const int32_t* counts, float* accumulated, float* bias, int E, float factor, int update, void* stream) {
+  if (E < 1 || E > kMaxE) return BIBO_ERR_BAD_SHAPE;
+  if (!counts || !accumulated || !bias) return BIBO_ERR_NULL_POINTER;
+  return hip_rc(launch_balance_step(counts, accumulated, bias, E, factor, update, static_cast<hipStream_t>(stream)));
+}
+
 int bibo_moe_exp_attn_res_fwd(const void* const* candidates, int n_candidates, const float* score_weight, float eps, int T, int H,
                           int dtype, void* out, void* stream) {
   const int rc = check_dims(T, H, 1, 1, 1, dtype);

@@ -175,6 +175,8 @@ bool permute_takes_router_hist(int T, int k);
 hipError_t launch_permute_from_hist(const int32_t* idx, int T, int E, int k, int32_t* hist, int hist_tokens,
                                     int32_t* counts, int32_t* offsets, int32_t* perm_slot, int32_t* perm_token,
                                     hipStream_t s);
+hipError_t launch_balance_step(const int32_t* counts, float* accumulated, float* bias, int E, float factor, int update,
+                               hipStream_t s);
 hipError_t launch_gateup_generic(const void* x, const void* wgu, const float* theta, const int32_t* offsets,
                                  const int32_t* perm_token, int T, int H, int E, int k, int I, int dtype, int act,
                                  void* hidden, hipStream_t s);

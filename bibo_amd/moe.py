@@ -4,9 +4,11 @@ Class names, constructor argument, attribute names, parameter shapes and state_d
 src/modeling/ffn/router.py and src/modeling/ffn/moe.py of the reference, so a reference checkpoint
 loads with strict=True and code that pokes at `layer.gate.bias` or `layer.experts.radial_theta`
 keeps working.  The modules are differentiable: `BiBoMoELayer.forward` is one autograd node (backward =
-bibo_moe_backward); with hooks present, or called on their own, `BiBoFusedExperts` is one node (backward =
-bibo_moe_experts_backward) and `BiBoMoERouter` returns the kernel's selection with differentiable weights.  bf16
-compute on sizes that are multiples of 128 trains on the MFMA kernels, fp32 compute and other sizes on generic ones."""
+bibo_moe_backward or, where the forward kept its activations, bibo_moe_backward_saved); with hooks present, or called on
+their own, `BiBoFusedExperts` is one node (backward = bibo_moe_experts_backward) and `BiBoMoERouter` returns the kernel's
+selection with differentiable weights.  bf16 compute on sizes that are multiples of 128 trains on the MFMA kernels, fp32
+compute and other sizes on generic ones.  The layer's calls go through the native host path (csrc/binding.cpp): at decode
+sizes the host is what bounds them, so `forward` does little more in Python than read its parameters."""
 from __future__ import annotations
 
 import torch
@@ -23,63 +25,26 @@ except AttributeError:                                    # older torch
     _no_compile = torch._dynamo.disable
 
 
+def _param(module, name):
+    """module.name without nn.Module's attribute lookup where it is a plain parameter."""
+    p = module._parameters.get(name)
+    return getattr(module, name) if p is None else p
+
+
+_codes_seen: dict = {}
+
+
+def _codes(norm, algo, act):
+    """(norm mode, algorithm, activation) as the library's codes; the module's settings are looked up, not parsed, per call."""
+    key = (norm, type(norm), algo, act)
+    hit = _codes_seen.get(key)
+    if hit is None:
+        hit = _codes_seen[key] = (ops.norm_mode(norm), ops.algo_code(algo), ops.act_code(act))
+    return hit
+
+
 def _wants_grad(*tensors) -> bool:
     return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
-
-
-class _MoELayerFn(torch.autograd.Function):
-    """The whole layer as one autograd node.  Gradients are what autograd gives the reference's eager layer with the
-    selection held fixed (moe.py:157-183); the balancing bias gets none (router.py:38).  The per-expert row counts come
-    out as a second, non-differentiable result.  `cd` is the compute dtype: bf16 runs the MFMA backward where its tiles
-    divide the sizes, anything else the generic kernels.  Two ways through the library: with `keep` and a shape that
-    has the pair, forward = bibo_moe_forward_train, which leaves routing, permutation and pre-activations in a state
-    tensor (about 4 I bytes per routed slot), and backward = bibo_moe_backward_saved; otherwise forward =
-    bibo_moe_forward and backward = bibo_moe_backward, which computes all of that again from the saved input rows.
-    The gradients are the same bits either way."""
-
-    @staticmethod
-    def forward(ctx, x, w_router, w_gate_up, w_down, theta, bias, k, norm, act, algo, want_counts, n_pos=0, n_neg=0,
-                casts=None, cd=torch.bfloat16, keep=True):
-        cast = lambda t, d: (t if t.dtype == d else t.to(d)).contiguous()
-        xb = cast(x.detach(), cd)
-        # `casts`: kernel-dtype copies of the three weight tensors the caller already holds (the layer's cast cache), so
-        # fp32 master weights are rounded once per optimiser step, not once per forward
-        wr, gu, dn = casts if casts is not None else (cast(w_router.detach(), cd), cast(w_gate_up.detach(), cd),
-                                                      cast(w_down.detach(), cd))
-        th = cast(theta.detach(), torch.float32)
-        # A private copy of the E selection biases: the layer's balancing step writes gate.bias in place later in the
-        # same forward (update_bias), and the backward pass has to route with the values the forward saw.
-        b = bias.detach().to(torch.float32).clone()
-        T, H = xb.shape
-        state = None
-        if keep and algo in ("auto", "fused") and ops.train_state_bytes(T, H, wr.shape[0], k, gu.shape[1] // 2, cd, n_pos,
-                                                                        n_neg, act) is not None:
-            out, counts, state = ops.moe_forward_train(xb, wr, b, gu, dn, th, k, norm=norm, want_counts=want_counts, act=act,
-                                                       n_pos=n_pos, n_neg=n_neg)
-        else:
-            out, _, _, counts, _ = ops.moe_forward(xb, wr, b, gu, dn, th, k, norm=norm, algo=algo, want_counts=want_counts,
-                                                   act=act, n_pos=n_pos, n_neg=n_neg)
-        ctx.has_state = state is not None
-        ctx.save_for_backward(xb, wr, gu, dn, th, b, *((state,) if state is not None else ()))
-        ctx.conf = (k, norm, act, n_pos, n_neg)
-        ctx.in_dtypes = (x.dtype, w_router.dtype, w_gate_up.dtype, w_down.dtype, theta.dtype)
-        if counts is None:
-            counts = torch.empty(0, dtype=torch.int32, device=x.device)
-        ctx.mark_non_differentiable(counts)
-        return out, counts
-
-    @staticmethod
-    def backward(ctx, d_out, _d_counts):
-        saved = ctx.saved_tensors                        # read once: activation checkpointing unpacks on access
-        xb, wr, gu, dn, th, b = saved[:6]
-        k, norm, act, n_pos, n_neg = ctx.conf
-        d = d_out.to(xb.dtype).contiguous()
-        if ctx.has_state:
-            grads = ops.moe_backward_saved(xb, d, wr, gu, dn, th, k, saved[6], norm=norm, act=act, n_pos=n_pos,
-                                           n_neg=n_neg)[:5]
-        else:
-            grads = ops.moe_backward(xb, d, wr, b, gu, dn, th, k, norm=norm, act=act, n_pos=n_pos, n_neg=n_neg)[:5]
-        return tuple(g.to(dt) for g, dt in zip(grads, ctx.in_dtypes)) + (None,) * 11
 
 
 class _ExpertsFn(torch.autograd.Function):
@@ -408,17 +373,54 @@ class BiBoMoELayer(nn.Module):
         self.accumulated_tpe.zero_()
         return tpe
 
+    def _balance(self, counts, num_tokens):
+        """_balance_step and update_bias of this forward in one launch, where neither is overridden, the state is fp32 on the
+        GPU and no process group has to see the counts first."""
+        cls, bias, acc = type(self), _param(self._modules["gate"], "bias"), self.accumulated_tpe
+        if (cls._balance_step is BiBoMoELayer._balance_step and cls.update_bias is BiBoMoELayer.update_bias
+                and "update_bias" not in self.__dict__ and "_balance_step" not in self.__dict__
+                and counts is not None and counts.is_cuda and acc.device == bias.device == counts.device
+                and acc.dtype == bias.dtype == torch.float32 and acc.is_contiguous() and bias.is_contiguous()):
+            if self._update_every is None:
+                self._update_every = max(1, round(self.bias_update_threshold / max(num_tokens, 1)))
+            fires = (self._fwd_step + 1) % self._update_every == 0
+            if not (fires and torch.distributed.is_available() and torch.distributed.is_initialized()):
+                self._fwd_step += 1
+                L.native().balance_step(counts, acc, bias, self.bias_update_factor, fires)
+                return
+        tpe = self._balance_step(None, num_tokens, counts=counts)
+        if tpe is not None:
+            self.update_bias(tpe)
+
     def _hooks_present(self) -> bool:
-        g, e = self.gate, self.experts
+        g, e = self._modules["gate"], self._modules["experts"]
         return bool(g._forward_hooks or g._forward_pre_hooks or e._forward_hooks or e._forward_pre_hooks
                     or g._probe_gap or nn.modules.module._global_forward_hooks
                     or nn.modules.module._global_forward_pre_hooks)
+
+    def _parameters_of_call(self):
+        """The five parameters the layer's output depends on: router weight, gate/up, down, theta, selection bias."""
+        g, e = self._modules["gate"], self._modules["experts"]
+        return (_param(g._modules["gate_proj"], "weight"), _param(e, "gate_up_proj"), _param(e, "down_proj"),
+                _param(e, "radial_theta"), _param(g, "bias"))
+
+    def _kernel_operands(self, params, cd):
+        """The same in kernel dtype, in the native calls' order: router weight, bias, gate/up, down, theta."""
+        gc, ec = self._modules["gate"]._cache, self._modules["experts"]._cache
+        wr, gu, dn, th, b = params
+        f32 = torch.float32
+        return (wr if wr.dtype == cd and wr.is_contiguous() else gc.get("w", wr, cd),
+                b if b.dtype == f32 and b.is_contiguous() else gc.get("b", b, f32),
+                gu if gu.dtype == cd and gu.is_contiguous() else ec.get("gu", gu, cd),
+                dn if dn.dtype == cd and dn.is_contiguous() else ec.get("dn", dn, cd),
+                th if th.dtype == f32 and th.is_contiguous() else ec.get("th", th, f32))
 
     @_no_compile
     def forward(self, hidden_states: torch.Tensor) -> torch.Tensor:
         bsz, seq, hdim = hidden_states.shape
         num_tokens = bsz * seq
         balancing = self.training and self.bias_update_factor > 0
+        top_idx = None
         if self._hooks_present():
             # module-by-module, so hooks on `gate` and `experts` observe exactly what the reference's
             # would (ablate/common/router_trace.py hooks both)
@@ -426,47 +428,34 @@ class BiBoMoELayer(nn.Module):
             res = self.experts(hidden_states.reshape(num_tokens, hdim), top_idx.view(num_tokens, -1),
                                top_w.view(num_tokens, -1), _want_counts=balancing)
             out, counts = res if balancing else (res, None)
-        elif _wants_grad(hidden_states, self.gate.gate_proj.weight, self.experts.gate_up_proj, self.experts.down_proj,
-                         self.experts.radial_theta):
-            out, counts = self._differentiable_forward(hidden_states.reshape(num_tokens, hdim), balancing)
-            out = out if out.dtype == hidden_states.dtype else out.to(hidden_states.dtype)
-            top_idx = None
+            out = out.view(bsz, seq, hdim)
         else:
             cd = _compute_dtype(hidden_states)
-            x = hidden_states.detach().reshape(num_tokens, hdim)
-            x = (x.to(cd) if x.dtype != cd else x).contiguous()
-            gu, dn, th = self.experts._weights(cd)
-            wr = self.gate._cache.get("w", self.gate.gate_proj.weight, cd)
-            b = self.gate._cache.get("b", self.gate.bias, torch.float32)
-            out, _, _, counts, _ = ops.moe_forward(x, wr, b, gu, dn, th, self.num_experts_per_tok,
-                                                   norm=self.gate.norm_topk_prob, algo=self.experts.algo,
-                                                   want_counts=balancing, n_pos=self.experts.num_pos,
-                                                   n_neg=self.experts.num_neg, act=self.experts.act)
+            e = self._modules["experts"]
+            params = self._parameters_of_call()
+            operands = self._kernel_operands(params, cd)
+            norm, algo, act = _codes(self._modules["gate"].norm_topk_prob, e.algo, e.act)
+            settings = (self.num_experts_per_tok, norm, algo, e.num_pos, e.num_neg, act, balancing, cd)
+            if torch.is_grad_enabled() and (hidden_states.requires_grad or any(p.requires_grad for p in params[:4])):
+                if not self._differentiable(cd):
+                    raise NotImplementedError(_NO_BACKWARD)
+                out, counts = L.native().layer_train(hidden_states, *params[:4], *operands, *settings, self.keep_activations)
+            else:
+                out, counts = L.native().layer_forward(hidden_states, *operands, *settings)
             out = out if out.dtype == hidden_states.dtype else out.to(hidden_states.dtype)
-            top_idx = None
-        out = out.view(bsz, seq, hdim)
         if self.use_shared_expert:                             # moe.py:174-176
             out = out + self.shared_experts_list[0](hidden_states).to(out.dtype)
         if balancing:                                          # exactly once per training forward
-            tpe = self._balance_step(top_idx, num_tokens, counts=counts)
-            if tpe is not None:
-                self.update_bias(tpe)
+            self._balance(counts, num_tokens)
         return out
 
-    def _differentiable_forward(self, x: torch.Tensor, want_counts: bool):
-        """x [T,H] -> (out [T,H] in the compute dtype with an autograd graph, counts|None).  bf16 compute (bf16
-        activations, or fp32 activations under bf16 autocast) with H and I multiples of 128 and I <= 512 runs the MFMA
-        backward; fp32 compute and every other size run the generic kernels."""
-        e = self.experts
-        cd = _compute_dtype(x)
-        if not _backward_covers(e, cd):
-            raise NotImplementedError(_NO_BACKWARD)
-        gu, dn, _ = e._weights(cd)
-        casts = (self.gate._cache.get("w", self.gate.gate_proj.weight, cd), gu, dn)
-        out, counts = _MoELayerFn.apply(x, self.gate.gate_proj.weight, e.gate_up_proj, e.down_proj, e.radial_theta,
-                                        self.gate.bias, self.num_experts_per_tok, self.gate.norm_topk_prob, e.act, e.algo,
-                                        want_counts, e.num_pos, e.num_neg, casts, cd, self.keep_activations)
-        return out, (counts if want_counts else None)
+    def _differentiable(self, cd) -> bool:
+        """bf16 compute (bf16 activations, or fp32 activations under bf16 autocast) with H and I multiples of 128 and
+        I <= 512 runs the MFMA backward; fp32 compute and every other size run the generic kernels, up to their limit."""
+        hit = self.__dict__.setdefault("_covers", {})
+        if cd not in hit:
+            hit[cd] = _backward_covers(self.experts, cd)
+        return hit[cd]
 
     @_no_compile
     def ffn_forward(self, hidden_states: torch.Tensor, norm_weight: torch.Tensor, eps: float,
@@ -496,24 +485,25 @@ class BiBoMoELayer(nn.Module):
             out = blk.to(hidden_states.dtype) if residual is False else base + blk.to(hidden_states.dtype)   # layers.py:64
             return out.to(torch.bfloat16) if bf16_stream else out
         balancing = self.training and self.bias_update_factor > 0
-        cd = _compute_dtype(hidden_states)
-        h = hidden_states.detach().reshape(num_tokens, hdim)
-        h = (h.to(cd) if h.dtype != cd else h).contiguous()
-        gu, dn, th = self.experts._weights(cd)
-        wr = self.gate._cache.get("w", self.gate.gate_proj.weight, cd)
-        b = self.gate._cache.get("b", self.gate.bias, torch.float32)
-        nw = norm_weight.detach().float().contiguous()
-        out, _, _, counts = ops.ffn_forward(h, nw, float(eps), wr, b, gu, dn, th, self.num_experts_per_tok,
-                                            norm=self.gate.norm_topk_prob, algo=self.experts.algo, want_counts=balancing,
-                                            n_pos=self.experts.num_pos, n_neg=self.experts.num_neg, act=self.experts.act,
-                                            round_block_out=bf16_moe_out and cd == torch.bfloat16,
-                                            residual=(residual if residual is None or residual is False
-                                                      else residual.detach().reshape(num_tokens, hdim).to(cd).contiguous()))
+        e = self._modules["experts"]
+        operands = self._kernel_operands(self._parameters_of_call(), hidden_states.dtype)
+        norm, algo, act = _codes(self._modules["gate"].norm_topk_prob, e.algo, e.act)
+        flags = L.FLAG_ROUND_BLOCK_OUT if bf16_moe_out else 0
+        if residual is False:
+            flags, residual = flags | L.FLAG_NO_RESIDUAL, None
+        out, counts = L.native().ffn_forward(hidden_states, self._norm_weight(norm_weight), float(eps), residual, *operands,
+                                             self.num_experts_per_tok, norm, algo, e.num_pos, e.num_neg, act, flags, balancing)
         if balancing:                                          # exactly once per training forward
-            tpe = self._balance_step(None, num_tokens, counts=counts)
-            if tpe is not None:
-                self.update_bias(tpe)
-        out = out.view(bsz, seq, hdim)
-        out = out if out.dtype == hidden_states.dtype else out.to(hidden_states.dtype)
+            self._balance(counts, num_tokens)
         return out.to(torch.bfloat16) if bf16_stream else out
 
+    def _norm_weight(self, w):
+        """fp32 copy of the caller's norm weight; a parameter's copy is kept until the parameter changes."""
+        if w.dtype == torch.float32 and w.is_contiguous():
+            return w
+        if not isinstance(w, nn.Parameter):
+            return w.detach().float().contiguous()
+        hit = self.__dict__.get("_norm_copy")
+        if hit is None or hit[0] is not w or hit[1] != (w._version, w.data_ptr()):
+            hit = self.__dict__["_norm_copy"] = (w, (w._version, w.data_ptr()), w.detach().float().contiguous())
+        return hit[2]

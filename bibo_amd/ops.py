@@ -83,17 +83,21 @@ def _stream(dev) -> ctypes.c_void_p:
     return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
 
 
-_workspaces: dict = {}
+class _Workspaces:
+    """The grow-only byte buffers, one per (device, stream): calls on one stream are ordered, so they may share one.  They
+    live in the native host path, which the modules' calls take them from."""
+
+    @staticmethod
+    def clear():
+        L.native().workspace_clear()
+
+
+_workspaces = _Workspaces()
 
 
 def workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
-    """A grow-only byte buffer per (device, stream): calls on one stream are ordered, so they may share it."""
-    key = (dev.index, torch.cuda.current_stream(dev).cuda_stream)
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
-        _workspaces[key] = ws
-    return ws
+    """The current stream's byte buffer, at least `nbytes` long."""
+    return L.native().workspace(dev.index if dev.index is not None else torch.cuda.current_device(), nbytes)
 
 
 def workspace_bytes(T, H, E, k, I, dtype_code) -> int:

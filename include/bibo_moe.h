@@ -326,6 +326,14 @@ int bibo_moe_experts_backward(const void* x, const void* d_out, const int32_t* i
                               void* stream);
 
 /*
+ * One balancing step on device tensors (_balance_step / update_bias, src/modeling/ffn/moe.py:131-155), all [E]:
+ *   accumulated += counts;  with `update` != 0 also, for load = accumulated / max(sum(accumulated), 1):
+ *   bias += factor * (mean(load) - load),  accumulated = 0.
+ * E <= 64.  Asynchronous on `stream`; needs no workspace.
+ */
+int bibo_moe_balance_step(const int32_t* counts, float* accumulated, float* bias, int E, float factor, int update, void* stream);
+
+/*
  * Depth mix of the experimental model's Block Attention Residuals: apply_attention_residual
  * (exp/modeling_bibo.py:119-232; softmax scores, dense), the operation the reference hands to its optional external
  * kernel `kernels.sm120.attn_res.attn_res(block_residual, prefix, score_weight, eps, ...)` (exp/modeling_bibo.py:44,
