@@ -25,6 +25,8 @@ SYMBOLS = (
     "bibo_moe_ffn_workspace_bytes", "bibo_moe_ffn_forward", "bibo_moe_forward_static", "bibo_moe_backward_workspace_bytes", "bibo_moe_backward", "bibo_moe_experts_backward",
     "bibo_moe_train_state_bytes", "bibo_moe_forward_train", "bibo_moe_backward_saved",
     "bibo_moe_exp_attn_res_fwd", "bibo_moe_balance_step",
+    "bibo_moe_exp_attn_res_norm_fwd", "bibo_moe_exp_carry_fwd", "bibo_moe_exp_silu_mul_fwd", "bibo_moe_exp_qk_norm_rope",
+    "bibo_moe_exp_attention_fwd",
 )
 STATIC_SCRATCH_BYTES = 16 << 20
 
@@ -89,6 +91,13 @@ def _declare(l):
                                           sz, vp]
     l.bibo_moe_exp_attn_res_fwd.restype = ci
     l.bibo_moe_exp_attn_res_fwd.argtypes = [vp, ci, vp, ctypes.c_float, ci, ci, ci, vp, vp]
+    cf = ctypes.c_float
+    for name, args in (("bibo_moe_exp_attn_res_norm_fwd", [vp, ci, vp, cf, vp, cf, ci, ci, ci, vp, vp, vp]),
+                       ("bibo_moe_exp_carry_fwd", [vp, vp, vp, vp, ci, ci, vp, vp, vp]),
+                       ("bibo_moe_exp_silu_mul_fwd", [vp, ci, ci, vp, vp]),
+                       ("bibo_moe_exp_qk_norm_rope", [vp, ci, ci, ci, ci, ci, ci, vp, vp, cf, vp, vp, vp]),
+                       ("bibo_moe_exp_attention_fwd", [vp, ci, ci, ci, ci, ci, ci, ci, cf, vp, vp, vp])):
+        getattr(l, name).restype, getattr(l, name).argtypes = ci, args
     l.bibo_moe_balance_step.restype = ci
     l.bibo_moe_balance_step.argtypes = [vp, vp, vp, ci, ctypes.c_float, ci, vp]
     l.bibo_moe_forward_static.argtypes = [vp, vp, vp, vp, vp, vp, ctypes.POINTER(Shape), ci, ci, vp, vp, vp, vp, vp, vp]

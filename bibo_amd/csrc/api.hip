@@ -839,20 +839,73 @@ int bibo_moe_balance_step(const int32_t* counts, float* accumulated, float* bias
   return hip_rc(launch_balance_step(counts, accumulated, bias, E, factor, update, static_cast<hipStream_t>(stream)));
 }
 
-int bibo_moe_exp_attn_res_fwd(const void* const* candidates, int n_candidates, const float* score_weight, float eps, int T, int H,
-                          int dtype, void* out, void* stream) {
+int bibo_moe_exp_attn_res_norm_fwd(const void* const* candidates, int n_candidates, const float* score_weight, float eps,
+                                   const float* norm_weight, float norm_eps, int T, int H, int dtype, void* out, void* normed,
+                                   void* stream) {
   const int rc = check_dims(T, H, 1, 1, 1, dtype);
   if (rc != BIBO_OK) return rc;
   if (!attn_res_supported(H, n_candidates, dtype)) return BIBO_ERR_UNSUPPORTED;
-  if (!candidates || !score_weight) return BIBO_ERR_NULL_POINTER;
+  if (!candidates || !score_weight || (normed && !norm_weight)) return BIBO_ERR_NULL_POINTER;
   if (T == 0) return BIBO_OK;
   if (!out) return BIBO_ERR_NULL_POINTER;
   for (int i = 0; i < n_candidates; ++i) {
     if (!candidates[i]) return BIBO_ERR_NULL_POINTER;
     if (!aligned16(candidates[i])) return BIBO_ERR_MISALIGNED;
   }
-  if (!aligned16(out)) return BIBO_ERR_MISALIGNED;
-  return hip_rc(launch_attn_res(candidates, n_candidates, score_weight, eps, T, H, out, static_cast<hipStream_t>(stream)));
+  if (!aligned16(out) || !aligned16(normed)) return BIBO_ERR_MISALIGNED;
+  return hip_rc(launch_attn_res(candidates, n_candidates, score_weight, eps, T, H, out, norm_weight, norm_eps, normed,
+                                static_cast<hipStream_t>(stream)));
+}
+
+int bibo_moe_exp_attn_res_fwd(const void* const* candidates, int n_candidates, const float* score_weight, float eps, int T, int H,
+                              int dtype, void* out, void* stream) {
+  return bibo_moe_exp_attn_res_norm_fwd(candidates, n_candidates, score_weight, eps, nullptr, 0.f, T, H, dtype, out, nullptr, stream);
+}
+
+int bibo_moe_exp_carry_fwd(const void* attn_read, const void* a, const float* theta, const void* prefix, int T, int H, void* hs,
+                           void* prefix_out, void* stream) {
+  const int rc = check_dims(T, H, 1, 1, 1, BIBO_DTYPE_BF16);
+  if (rc != BIBO_OK) return rc;
+  if (H % 8 != 0) return BIBO_ERR_UNSUPPORTED;
+  if (T == 0) return BIBO_OK;
+  if (!attn_read || !a || !hs || (prefix && !prefix_out)) return BIBO_ERR_NULL_POINTER;
+  if (!aligned16(attn_read) || !aligned16(a) || !aligned16(hs) || !aligned16(prefix) || !aligned16(prefix_out)) return BIBO_ERR_MISALIGNED;
+  return hip_rc(launch_carry(attn_read, a, theta, prefix, T, H, hs, prefix_out, static_cast<hipStream_t>(stream)));
+}
+
+int bibo_moe_exp_silu_mul_fwd(const void* gate_up, int T, int I, void* out, void* stream) {
+  const int rc = check_dims(T, 1, 1, 1, I, BIBO_DTYPE_BF16);
+  if (rc != BIBO_OK) return rc;
+  if (I % 8 != 0) return BIBO_ERR_UNSUPPORTED;
+  if (T == 0) return BIBO_OK;
+  if (!gate_up || !out) return BIBO_ERR_NULL_POINTER;
+  if (!aligned16(gate_up) || !aligned16(out)) return BIBO_ERR_MISALIGNED;
+  return hip_rc(launch_silu_mul(gate_up, T, I, out, static_cast<hipStream_t>(stream)));
+}
+
+int bibo_moe_exp_qk_norm_rope(void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, const float* q_weight,
+                              const float* k_weight, float eps, const float* cos, const float* sin, void* stream) {
+  if (B < 0 || S < 0 || (long long)B * S > 0x3fffffffLL) return BIBO_ERR_BAD_SHAPE;
+  if (!exp_attention_supported(n_heads, n_kv_heads, head_dim) || ld < (n_heads + 2 * n_kv_heads) * head_dim || ld % 8 != 0 ||
+      (cos == nullptr) != (sin == nullptr))
+    return BIBO_ERR_UNSUPPORTED;
+  if (B == 0 || S == 0) return BIBO_OK;
+  if (!qkv) return BIBO_ERR_NULL_POINTER;
+  if (!aligned16(qkv)) return BIBO_ERR_MISALIGNED;
+  return hip_rc(launch_qk_norm_rope(qkv, ld, B * S, S, n_heads, n_kv_heads, head_dim, q_weight, k_weight, eps, cos, sin,
+                                    static_cast<hipStream_t>(stream)));
+}
+
+int bibo_moe_exp_attention_fwd(const void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, int window,
+                               float scale, const float* xsa_alpha, void* out, void* stream) {
+  if (B < 0 || S < 0 || window < 0 || (long long)B * S * n_heads > 0x3fffffffLL) return BIBO_ERR_BAD_SHAPE;
+  if (!exp_attention_supported(n_heads, n_kv_heads, head_dim) || ld < (n_heads + 2 * n_kv_heads) * head_dim || ld % 8 != 0)
+    return BIBO_ERR_UNSUPPORTED;
+  if (B == 0 || S == 0) return BIBO_OK;
+  if (!qkv || !out) return BIBO_ERR_NULL_POINTER;
+  if (!aligned16(qkv) || !aligned16(out)) return BIBO_ERR_MISALIGNED;
+  return hip_rc(launch_exp_attention(qkv, ld, B, S, n_heads, n_kv_heads, head_dim, window, scale, xsa_alpha, out,
+                                     static_cast<hipStream_t>(stream)));
 }
 
 }  // extern "C"

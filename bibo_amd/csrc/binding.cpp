@@ -263,6 +263,101 @@ void balance_step(const Tensor& counts, Tensor accumulated, Tensor bias, double 
   if (update) bias.unsafeGetTensorImpl()->bump_version();
 }
 
+// ---- the 10-layer forward's own launches (bibo_amd/exp_model.py); bf16, no autograd -------------------------------
+void check_rows(const Tensor& t, const char* name, int64_t cols) {
+  TORCH_CHECK(t.is_cuda(), name, " must live on the GPU (got ", t.device(), "); bibo_amd has no CPU path");
+  TORCH_CHECK_VALUE(t.is_contiguous() && t.dim() >= 1 && t.size(-1) == cols, name, " must be contiguous rows of ", cols);
+  TORCH_CHECK_TYPE(t.scalar_type() == at::kBFloat16, name, " must be bfloat16");
+}
+const float* f32_or_null(const c10::optional<Tensor>& t, const char* name, at::IntArrayRef shape) {
+  if (!t.has_value()) return nullptr;
+  check_tensor(*t, name, at::kFloat, shape);
+  return f32(*t);
+}
+hipStream_t stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+// candidates [T, H] -> (their depth mix, its RMSNorm or None)
+py::tuple exp_attn_res_norm(const std::vector<Tensor>& candidates, const Tensor& score_weight, double eps,
+                            const c10::optional<Tensor>& norm_weight, double norm_eps) {
+  TORCH_CHECK_VALUE(!candidates.empty() && candidates.size() <= 8, "1 to 8 candidates");
+  const Tensor& c0 = candidates[0];
+  const int64_t H = c0.size(-1), T = c0.numel() / H;
+  const void* ptrs[8];
+  for (size_t i = 0; i < candidates.size(); ++i) {
+    check_rows(candidates[i], "candidate", H);
+    TORCH_CHECK_VALUE(candidates[i].numel() == c0.numel(), "candidates must have one size");
+    ptrs[i] = candidates[i].data_ptr();
+  }
+  check_tensor(score_weight, "score_weight", at::kFloat, {H});
+  const float* nw = f32_or_null(norm_weight, "norm_weight", {H});
+  c10::DeviceGuard guard(c0.device());
+  Tensor out = at::empty_like(c0), normed;
+  if (nw != nullptr) normed = at::empty_like(c0);
+  check(bibo_moe_exp_attn_res_norm_fwd(ptrs, (int)candidates.size(), f32(score_weight), (float)eps, nw, (float)norm_eps, (int)T, (int)H,
+                                       BIBO_DTYPE_BF16, out.data_ptr(), nw != nullptr ? normed.data_ptr() : nullptr, stream_of(c0)),
+        "bibo_moe_exp_attn_res_norm_fwd");
+  return py::make_tuple(out, maybe(normed));
+}
+
+// x [B, S, H] -> attention output [B, S, H]: one projection to q|k|v rows, norm and RoPE in place, attention with XSA, output
+// projection (the two products are library GEMMs)
+Tensor exp_attention(const Tensor& x, const Tensor& w_qkv, const Tensor& w_o, const c10::optional<Tensor>& q_weight,
+                     const c10::optional<Tensor>& k_weight, double eps, const c10::optional<Tensor>& cos,
+                     const c10::optional<Tensor>& sin, const c10::optional<Tensor>& xsa_alpha, int n_heads, int n_kv_heads,
+                     int head_dim, int window, double scale) {
+  at::NoGradGuard no_grad;
+  const int64_t B = x.size(0), S = x.size(1);
+  check_rows(x, "x", x.size(2));
+  const float *qw = f32_or_null(q_weight, "q_weight", {head_dim}), *kw = f32_or_null(k_weight, "k_weight", {head_dim});
+  const float *co = f32_or_null(cos, "cos", {S, head_dim / 2}), *si = f32_or_null(sin, "sin", {S, head_dim / 2});
+  const float* alpha = f32_or_null(xsa_alpha, "xsa_alpha", {n_heads});
+  c10::DeviceGuard guard(x.device());
+  const Tensor qkv = at::linear(x, w_qkv);
+  const int ld = (int)qkv.size(-1);
+  hipStream_t s = stream_of(x);
+  if (qw != nullptr || kw != nullptr || co != nullptr)
+    check(bibo_moe_exp_qk_norm_rope(qkv.data_ptr(), ld, (int)B, (int)S, n_heads, n_kv_heads, head_dim, qw, kw, (float)eps, co, si, s),
+          "bibo_moe_exp_qk_norm_rope");
+  const Tensor y = at::empty({B, S, (int64_t)n_heads * head_dim}, x.options());
+  check(bibo_moe_exp_attention_fwd(qkv.data_ptr(), ld, (int)B, (int)S, n_heads, n_kv_heads, head_dim, window, (float)scale, alpha,
+                                   y.data_ptr(), s),
+        "bibo_moe_exp_attention_fwd");
+  return at::linear(y, w_o);
+}
+
+// (attn_read + theta a, prefix + a or a itself)
+py::tuple exp_carry(const Tensor& attn_read, const Tensor& a, const c10::optional<Tensor>& theta, const c10::optional<Tensor>& prefix) {
+  const int64_t H = a.size(-1);
+  check_rows(attn_read, "attn_read", H);
+  check_rows(a, "a", H);
+  TORCH_CHECK_VALUE(attn_read.numel() == a.numel(), "attn_read must have the size of a");
+  const float* th = f32_or_null(theta, "theta", {H});
+  Tensor out = at::empty_like(a), prefix_out;
+  if (prefix.has_value()) {
+    check_rows(*prefix, "prefix", H);
+    TORCH_CHECK_VALUE(prefix->numel() == a.numel(), "prefix must have the size of a");
+    prefix_out = at::empty_like(a);
+  }
+  c10::DeviceGuard guard(a.device());
+  check(bibo_moe_exp_carry_fwd(attn_read.data_ptr(), a.data_ptr(), th, prefix.has_value() ? prefix->data_ptr() : nullptr,
+                               (int)(a.numel() / H), (int)H, out.data_ptr(), prefix.has_value() ? prefix_out.data_ptr() : nullptr,
+                               stream_of(a)),
+        "bibo_moe_exp_carry_fwd");
+  return py::make_tuple(out, prefix.has_value() ? prefix_out : a);
+}
+
+// base + SwiGLU(x): gate and up in one library product, SiLU(gate) * up in one launch, base added by the down product
+Tensor exp_mlp(const Tensor& x, const Tensor& w_gate_up, const Tensor& w_down, const Tensor& base) {
+  at::NoGradGuard no_grad;
+  const int64_t H = x.size(-1), T = x.numel() / H, I = w_gate_up.size(0) / 2;
+  check_rows(x, "x", H);
+  c10::DeviceGuard guard(x.device());
+  const Tensor gu = at::linear(x.view({T, H}), w_gate_up);
+  Tensor h = at::empty({T, I}, x.options());
+  check(bibo_moe_exp_silu_mul_fwd(gu.data_ptr(), (int)T, (int)I, h.data_ptr(), stream_of(x)), "bibo_moe_exp_silu_mul_fwd");
+  return at::addmm(base.reshape({T, w_down.size(0)}), h, w_down.t()).view_as(base);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_native, m) {
@@ -273,4 +368,8 @@ PYBIND11_MODULE(_native, m) {
   m.def("ffn_forward", &ffn_forward);
   m.def("layer_train", &layer_train);
   m.def("balance_step", &balance_step);
+  m.def("exp_attn_res_norm", &exp_attn_res_norm);
+  m.def("exp_attention", &exp_attention);
+  m.def("exp_carry", &exp_carry);
+  m.def("exp_mlp", &exp_mlp);
 }

@@ -221,7 +221,15 @@ hipError_t launch_down_stream(const void* gu, const void* wd, const float* theta
 
 bool attn_res_supported(int H, int n_cand, int dtype);
 hipError_t launch_attn_res(const void* const* cands, int n_cand, const float* score_w, float eps, int T, int H, void* out,
-                           hipStream_t s);
+                           const float* norm_w, float norm_eps, void* normed, hipStream_t s);
+hipError_t launch_carry(const void* attn_read, const void* a, const float* theta, const void* prefix, int T, int H, void* hs,
+                        void* prefix_out, hipStream_t s);
+hipError_t launch_silu_mul(const void* gu, int T, int I, void* out, hipStream_t s);
+bool exp_attention_supported(int nq, int nkv, int D);
+hipError_t launch_qk_norm_rope(void* qkv, int ld, int T, int S, int nq, int nkv, int D, const float* qw, const float* kw, float eps,
+                               const float* cos, const float* sin, hipStream_t s);
+hipError_t launch_exp_attention(const void* qkv, int ld, int B, int S, int nq, int nkv, int D, int window, float scale,
+                                const float* xsa_alpha, void* out, hipStream_t s);
 
 // ---- backward pass (backward.hip) ----
 struct BackwardBuffers {

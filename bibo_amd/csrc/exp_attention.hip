@@ -1,0 +1,310 @@
+// Attention of the 10-layer experimental forward (BiBoAttention.forward, src/modeling/attn/base.py:55-128 without cache):
+// QK-norm and RoPE in place on the rows of one q|k|v projection, and causal or banded attention with the XSA correction
+// (attn/xsa.py:41-54) in its epilogue, written token-major for the output projection.  bf16 operands, fp32 arithmetic.
+#include "stripe.h"
+
+namespace bibo {
+namespace {
+
+__device__ __forceinline__ float row16_sum(float v) {      // sum over a DPP row of 16 lanes, the same in every lane
+  auto dpp = [](float x, auto ctrl) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, false));
+  };
+  v += dpp(v, std::integral_constant<int, 0xB1>{});
+  v += dpp(v, std::integral_constant<int, 0x4E>{});
+  v += dpp(v, std::integral_constant<int, 0x141>{});
+  return v + dpp(v, std::integral_constant<int, 0x140>{});
+}
+
+// ---- QK-norm (norm.py:19-24 on head rows) and RoPE (attn/rope.py, rotate-half), in place --------------------------
+// rows of qkv: [T, ld], the nq query heads first, then the nkv key heads, D elements each.  Sixteen lanes per head row; lane
+// c < D / 16 owns elements 8c .. 8c + 7 of the first half and of the second half, i.e. whole rotation pairs.  Memory-bound:
+// one read and one write of the q and k columns.  qw, kw (fp32 [D], or NULL: no norm); cos, sin (fp32 [S, D / 2] or NULL).
+template <int D>
+__global__ __launch_bounds__(256) void qk_norm_rope_kernel(bf16_t* __restrict__ qkv, int ld, int T, int S, int nq, int nkv,
+                                                           const float* __restrict__ qw, const float* __restrict__ kw, float eps,
+                                                           const float* __restrict__ cos, const float* __restrict__ sin) {
+  constexpr int kLanes = D / 16;
+  const int heads = nq + nkv;
+  const long long g = ((long long)blockIdx.x * 256 + threadIdx.x) >> 4;
+  if (g >= (long long)T * heads) return;                   // whole groups of 16 lanes
+  const int t = (int)(g / heads), hd = (int)(g - (long long)t * heads);
+  const int c = threadIdx.x & 15;
+  const bool live = c < kLanes;
+  bf16_t* row = qkv + (size_t)t * ld + hd * D;
+  float a[8], b[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) a[q] = b[q] = 0.f;
+  if (live) {
+    const bf16x8 va = *reinterpret_cast<const bf16x8*>(row + c * 8), vb = *reinterpret_cast<const bf16x8*>(row + D / 2 + c * 8);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) { a[q] = (float)va[q]; b[q] = (float)vb[q]; }
+  }
+  const float* w = hd < nq ? qw : kw;
+  if (w != nullptr) {
+    float ss = 0.f;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) ss = fmaf(a[q], a[q], fmaf(b[q], b[q], ss));
+    const float rinv = rsqrtf(row16_sum(ss) / (float)D + eps);
+    if (live) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        a[q] = w[c * 8 + q] * (float)(bf16_t)(a[q] * rinv);
+        b[q] = w[D / 2 + c * 8 + q] * (float)(bf16_t)(b[q] * rinv);
+      }
+    }
+  }
+  if (!live || (w == nullptr && cos == nullptr)) return;
+  if (cos != nullptr) {
+    const size_t p = (size_t)(t % S) * (D / 2) + c * 8;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const float x = a[q], y = b[q], co = cos[p + q], si = sin[p + q];
+      a[q] = x * co - y * si;
+      b[q] = y * co + x * si;
+    }
+  }
+  bf16x8 oa, ob;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) { oa[q] = (bf16_t)a[q]; ob[q] = (bf16_t)b[q]; }
+  *reinterpret_cast<bf16x8*>(row + c * 8) = oa;
+  *reinterpret_cast<bf16x8*>(row + D / 2 + c * 8) = ob;
+}
+
+// ---- attention -------------------------------------------------------------------------------------------------
+// One workgroup = four waves; a wave owns 32 consecutive queries of one head, and 1, 2 or 4 query heads that share a key
+// head share the workgroup (hpw), so that a block of 32 keys and values passes through LDS once for all of them.
+//   S^T = K Q^T  (v_mfma_f32_32x32x16_bf16, Q fragments in registers): lane = query, registers = keys, so a row's maximum
+//     and sum are in-lane but for the other half of the keys in lane ^ 32;
+//   O^T = V^T P^T: the probabilities a lane holds (keys 4h .. +4 and 8 + 4h .. +4 of sixteen) are, rounded to bf16, the MFMA
+//     operand as they are, with V's operand read in the same key order by transposing LDS reads; O^T has lane = query
+//     again, so rescaling and the final division are per-lane scalars.
+// The running maximum is raised (and O rescaled, D/32 x 16 multiplies) only when a row's maximum passes it by more than 8
+// in log2 units: the sums stay exact, the probabilities at most 256.
+// K and V blocks arrive by LDS-DMA in two stages; the next one is requested right after the barrier that frees its stage.
+// 16-byte granule g of a K row r sits at g ^ swz, so the 16 rows of a fragment read hit distinct banks; V rows are
+// swizzled so that the four rows of a transposing read do.
+// Two workgroups per CU (D = 192: 48 KB of LDS, 96 accumulator and 48 query registers per lane): one's softmax runs beside the
+// other's MFMAs.  Causal blocks are dealt longest first, then shortest first, so that the two of a CU add up alike.
+typedef short attn_v4i16 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) attn_v4i16 attn_lds_v4i16;
+
+template <int D> __device__ __forceinline__ int kswz(int row) { return D == 128 ? (row & 15) : ((row >> 1) & 7); }
+template <int D> __device__ __forceinline__ int vswz(int row) { return D == 128 ? ((row & 3) << 2) : (((row >> 1) & 1) << 2); }
+
+template <int D>
+__global__ __launch_bounds__(256, 2) void attention_kernel(const bf16_t* __restrict__ qkv, int ld, int S, int nq, int nkv, int hpw,
+                                                           int heads, int nqb, int window, float scale_log2,
+                                                           const float* __restrict__ xsa_alpha, bf16_t* __restrict__ out) {
+  constexpr int KB = 32, GPR = D / 8, NI = KB * GPR / 256;      // keys per block, granules per row, DMA instructions per operand
+  constexpr int DT = D / 32, KS = D / 16;
+  static_assert(KB * GPR % 256 == 0, "a block does not divide over the threads");
+  __shared__ __attribute__((aligned(16))) bf16_t K0[KB * D];
+  __shared__ __attribute__((aligned(16))) bf16_t K1[KB * D];
+  __shared__ __attribute__((aligned(16))) bf16_t V0[KB * D];
+  __shared__ __attribute__((aligned(16))) bf16_t V1[KB * D];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 31, h = lane >> 5;
+  // block id -> (query block, group of hpw query heads of one batch); heads = groups over all batches
+  const int r = blockIdx.x / heads, grp = blockIdx.x - r * heads;
+  const int qb = r < nqb / 2 ? nqb - 1 - r : r - nqb / 2;
+  const int gpb = nq / hpw;                                     // groups per batch
+  const int b = grp / gpb, gi = grp - b * gpb;
+  const int wph = 4 / hpw;                                      // waves per head
+  const int head = gi * hpw + wave / wph;
+  const int kvh = gi * hpw / (nq / nkv);
+  const int QB = 32 * wph;
+  const int q0 = qb * QB, q0w = q0 + (wave % wph) * 32;         // the workgroup's and this wave's first query
+  const bf16_t* base = qkv + (size_t)b * S * ld;
+  const bf16_t* kbase = base + (size_t)(nq + kvh) * D;
+  const bf16_t* vbase = base + (size_t)(nq + nkv + kvh) * D;
+
+  int krow[NI], kg[NI], vg[NI];                                 // this thread's row of a block and source granules
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int p = i * 256 + tid, row = p / GPR, pos = p - row * GPR;
+    krow[i] = row;
+    kg[i] = (pos ^ kswz<D>(row)) * 8;
+    vg[i] = (pos ^ vswz<D>(row)) * 8;
+  }
+  auto request = [&](int kv0, bf16_t* ks, bf16_t* vs) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const size_t o = (size_t)min(kv0 + krow[i], S - 1) * ld;
+      dma16(kbase + o + kg[i], ks + (i * 256 + wave * 64) * 8);
+      dma16(vbase + o + vg[i], vs + (i * 256 + wave * 64) * 8);
+    }
+  };
+  const int kv_first = window > 0 ? max(0, (q0 - window + 1)) & ~(KB - 1) : 0;
+  const int kv_end = min(q0 + QB, S);                           // keys [kv_first, kv_end)
+  request(kv_first, K0, V0);
+
+  bf16x8 q[KS];
+  {
+    const bf16_t* qrow = base + (size_t)min(q0w + n, S - 1) * ld + head * D + h * 8;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) q[s] = *reinterpret_cast<const bf16x8*>(qrow + s * 16);
+  }
+  floatx16 o[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
+  float m = -1.0e30f, l = 0.f;                                  // running maximum (log2 units) and this lane's part of the sum
+  // V operand: lane r16 of a 16-lane group points at key 4h + r16 / 4, columns 16 ((lane >> 4) & 1) + 4 (r16 % 4)
+  const int r16 = lane & 15;
+  const int vkey = 4 * h + (r16 >> 2), vcol = 16 * ((lane >> 4) & 1) + 4 * (r16 & 3);
+  const int vsw = vswz<D>(r16 >> 2);                            // the same for every key this lane reads (keys = r16 / 4 mod 4)
+  const int ksw = kswz<D>(n);
+
+  auto block = [&](int kv0, const bf16_t* ks, const bf16_t* vs) {
+    // nothing of this block is visible to this wave's queries?
+    if (kv0 > q0w + 31 || (window > 0 && kv0 + KB - 1 <= q0w - window)) return;
+    floatx16 st;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) st[i] = 0.f;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const bf16x8 kf = *reinterpret_cast<const bf16x8*>(ks + n * D + (((2 * s + h) ^ ksw) << 3));
+      st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, q[s], st, 0, 0, 0);
+    }
+    // register i: key kv0 + 8 (i / 4) + 4 h + i % 4
+    if (kv0 + KB - 1 > q0w || (window > 0 && q0w + 31 - kv0 >= window)) {
+      const int qi = q0w + n;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int key = kv0 + 8 * (i >> 2) + 4 * h + (i & 3);
+        if (key > qi || (window > 0 && qi - key >= window)) st[i] = -INFINITY;
+      }
+    }
+    float mx = st[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) mx = fmaxf(mx, st[i]);
+    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave)) * scale_log2;
+    if (__any(mx > m + 8.f)) {
+      const float mn = fmaxf(m, mx), al = __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+      l *= al;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[dt][i] *= al;
+    }
+    bf16x8 p[2];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float e = __builtin_amdgcn_exp2f(fmaf(st[i], scale_log2, -m));
+      l += e;
+      p[i >> 3][i & 7] = (bf16_t)e;
+    }
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const int gcol = dt * 32 + vcol;
+        const bf16_t* a = vs + (16 * kk + vkey) * D + (((gcol >> 3) ^ vsw) << 3) + (gcol & 4);
+        const attn_v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((attn_lds_v4i16*)a);
+        const attn_v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((attn_lds_v4i16*)(a + 8 * D));
+        typedef short v8i16 __attribute__((ext_vector_type(8)));
+        const v8i16 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, v), p[kk], o[dt], 0, 0, 0);
+      }
+  };
+  for (int kv0 = kv_first; kv0 < kv_end; kv0 += 2 * KB) {
+    sync_keep_loads<0>();                    // block kv0 has landed in every wave; nobody reads the other stage any more
+    if (kv0 + KB < kv_end) request(kv0 + KB, K1, V1);
+    block(kv0, K0, V0);
+    if (kv0 + KB < kv_end) {
+      sync_keep_loads<0>();
+      if (kv0 + 2 * KB < kv_end) request(kv0 + 2 * KB, K0, V0);
+      block(kv0 + KB, K1, V1);
+    }
+  }
+  // y = O / l, then XSA: y -= tanh(alpha) <y, vn> vn with vn = v / |v| of the query's own token
+  const int qi = q0w + n;
+  l += __shfl_xor(l, 32, kWave);
+  const float inv = 1.f / l;
+  if (xsa_alpha != nullptr) {
+    const bf16_t* vrow = vbase + (size_t)min(qi, S - 1) * ld + 4 * h;
+    bf16x4 v[DT][4];
+    float vv = 0.f, yv = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) v[dt][c] = *reinterpret_cast<const bf16x4*>(vrow + dt * 32 + c * 8);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const float f = (float)v[dt][i >> 2][i & 3];
+        o[dt][i] *= inv;
+        vv = fmaf(f, f, vv);
+        yv = fmaf(f, o[dt][i], yv);
+      }
+    vv += __shfl_xor(vv, 32, kWave);
+    yv += __shfl_xor(yv, 32, kWave);
+    const float vn = 1.f / fmaxf(sqrtf(vv), 1e-12f);            // F.normalize
+    const float coeff = yv * vn * vn * tanhf(xsa_alpha[head]);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[dt][i] = fmaf(-coeff, (float)v[dt][i >> 2][i & 3], o[dt][i]);
+  } else {
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[dt][i] *= inv;
+  }
+  if (qi >= S) return;
+  bf16_t* orow = out + ((size_t)b * S + qi) * nq * D + head * D + 4 * h;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      *reinterpret_cast<bf16x4*>(orow + dt * 32 + c * 8) =
+          bf16x4{(bf16_t)o[dt][4 * c], (bf16_t)o[dt][4 * c + 1], (bf16_t)o[dt][4 * c + 2], (bf16_t)o[dt][4 * c + 3]};
+}
+
+}  // namespace
+
+bool exp_attention_supported(int nq, int nkv, int D) {
+  const int g = nkv > 0 ? nq / nkv : 0;
+  return (D == 64 || D == 128 || D == 192) && nkv >= 1 && nq % nkv == 0 && (g == 1 || g % 2 == 0);
+}
+
+hipError_t launch_qk_norm_rope(void* qkv, int ld, int T, int S, int nq, int nkv, int D, const float* qw, const float* kw, float eps,
+                               const float* cos, const float* sin, hipStream_t s) {
+  const long long groups = (long long)T * (nq + nkv);
+  if (groups == 0) return hipSuccess;
+  const dim3 grid((unsigned)((groups + 15) / 16));
+  bf16_t* p = static_cast<bf16_t*>(qkv);
+  switch (D) {
+    case 64: hipLaunchKernelGGL(qk_norm_rope_kernel<64>, grid, dim3(256), 0, s, p, ld, T, S, nq, nkv, qw, kw, eps, cos, sin); break;
+    case 128: hipLaunchKernelGGL(qk_norm_rope_kernel<128>, grid, dim3(256), 0, s, p, ld, T, S, nq, nkv, qw, kw, eps, cos, sin); break;
+    case 192: hipLaunchKernelGGL(qk_norm_rope_kernel<192>, grid, dim3(256), 0, s, p, ld, T, S, nq, nkv, qw, kw, eps, cos, sin); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_exp_attention(const void* qkv, int ld, int B, int S, int nq, int nkv, int D, int window, float scale,
+                                const float* xsa_alpha, void* out, hipStream_t s) {
+  if (B == 0 || S == 0) return hipSuccess;
+  const int g = nq / nkv;
+  const int hpw = g % 4 == 0 ? 4 : (g % 2 == 0 ? 2 : 1);
+  const int QB = 128 / hpw, nqb = (S + QB - 1) / QB, heads = B * nq / hpw;
+  const dim3 grid((unsigned)(heads * nqb));
+  const float sl = scale * 1.4426950408889634f;
+  const bf16_t* p = static_cast<const bf16_t*>(qkv);
+  bf16_t* o = static_cast<bf16_t*>(out);
+  switch (D) {
+    case 64: hipLaunchKernelGGL(attention_kernel<64>, grid, dim3(256), 0, s, p, ld, S, nq, nkv, hpw, heads, nqb, window, sl, xsa_alpha, o); break;
+    case 128: hipLaunchKernelGGL(attention_kernel<128>, grid, dim3(256), 0, s, p, ld, S, nq, nkv, hpw, heads, nqb, window, sl, xsa_alpha, o); break;
+    case 192: hipLaunchKernelGGL(attention_kernel<192>, grid, dim3(256), 0, s, p, ld, S, nq, nkv, hpw, heads, nqb, window, sl, xsa_alpha, o); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+}  // namespace bibo

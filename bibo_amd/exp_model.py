@@ -5,9 +5,12 @@ Block Attention Residuals with one depth mix per layer and the carry write `attn
 [global, window, window] attention (NoPE on global layers, full RoPE on windowed ones), QK-norm, XSA, dense SwiGLU in
 `mlp_only_layers` and `BiBoMoELayer` everywhere else.  Only the MoE block runs on this package's HIP kernels, one
 library call per layer: `out = prefix_sum + moe(rmsnorm(h))` (`bibo_moe_ffn_forward` with its own residual operand).
-Everything around it is stock PyTorch tensor operations: attention through `scaled_dot_product_attention` (the
-windowed layers as block-local attention over a two-block key window instead of the reference's eager S x S band
-mask, `src/modeling/attn/swa.py:93-112`), the depth mix in fp32 as `apply_attention_residual` spells it out.
+Around it a bf16 model on the GPU without autograd runs a handful of launches per layer (csrc/exp_attention.hip, csrc/ffn.hip
+through the native calls): depth mix + input norm, one q|k|v product, QK-norm + RoPE in place, attention + XSA, output product,
+the two residual sums.  Everything else (fp32, autograd, hooks on inner modules, head sizes the attention kernel does not
+take) is stock PyTorch tensor operations: attention through `scaled_dot_product_attention` (the windowed layers as
+block-local attention over a two-block key window instead of the reference's eager S x S band mask,
+`src/modeling/attn/swa.py:93-112`), the depth mix in fp32 as `apply_attention_residual` spells it out.
 
 Parameter names follow the reference's `state_dict()` (`model.layers.N.self_attn.q_proj.weight`, ...,
 `model.layers.N.attn_res_carry_theta`, `model.output_attn_res_proj.weight`, tied `lm_head.weight`), so a checkpoint
@@ -20,6 +23,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .config import BiBoMoEConfig
+from . import _lib as L
 from . import ops
 from .moe import BiBoMoELayer
 
@@ -95,20 +99,42 @@ def _hip_ok(x) -> bool:
     return x.is_cuda and x.dtype == torch.bfloat16 and not (torch.is_grad_enabled() and x.requires_grad)
 
 
-def _fp32_copy(module, name):
-    """fp32 copy of a small parameter, refreshed when the parameter changes (storage address or version counter)."""
-    p = getattr(module, name)
-    tag = (p.data_ptr(), p._version, p.device)
-    hit = module.__dict__.get("_fp32_" + name)
+def _derived(module, key, params, make):
+    """make() from parameters, kept in `module` until one of them changes (storage address or version counter; the cache
+    holds the tensors, so an address cannot pass to another one meanwhile)."""
+    tag = tuple((p.data_ptr(), p._version, p.device) for p in params)
+    hit = module.__dict__.get("_derived_" + key)
     if hit is None or hit[0] != tag:
-        hit = (tag, p.detach().float().contiguous())
-        module.__dict__["_fp32_" + name] = hit
+        with torch.no_grad():
+            hit = module.__dict__["_derived_" + key] = (tag, make(), params)
     return hit[1]
+
+
+def _fp32_copy(module, name):
+    """fp32 copy of a small parameter."""
+    p = getattr(module, name)
+    return _derived(module, name, (p,), lambda: p.detach().float().contiguous())
+
+
+def _plain(*modules) -> bool:
+    """None of the modules' own calls is observed: their work may be done inside another launch."""
+    g = nn.modules.module
+    return not (g._global_forward_hooks or g._global_forward_pre_hooks
+                or any(m._forward_hooks or m._forward_pre_hooks for m in modules))
+
+
+def _native_ok(x) -> bool:
+    """bf16 rows on the GPU with autograd off: what the native launches around the block take."""
+    return x.is_cuda and x.dtype == torch.bfloat16 and not torch.is_grad_enabled() and x.is_contiguous()
 
 
 def _rotate_half(x):
     h = x.shape[-1] // 2
     return torch.cat((-x[..., h:], x[..., :h]), dim=-1)
+
+
+def _score_weight(module, proj_w, norm_w):
+    return _derived(module, "score", (proj_w, norm_w), lambda: (norm_w.float() * proj_w.reshape(-1).float()).contiguous())
 
 
 def attention_residual(prefix, blocks, proj_w, norm_w, eps):
@@ -173,7 +199,29 @@ class BiBoExpAttention(nn.Module):
         self.xsa_alpha = (nn.Parameter(torch.full((self.num_heads,), float(config.xsa_alpha_init)))
                           if config.use_xsa else None)
 
+    def _native(self, x, cos, sin):
+        """The whole block in the native call, or None where its kernels do not take it."""
+        nh, nkv, d = self.num_heads, self.num_key_value_heads, self.head_dim
+        projs = (self.q_proj, self.k_proj, self.v_proj, self.o_proj)
+        normed = isinstance(self.q_norm, RMSNorm)
+        if not (_native_ok(x) and d in (64, 128, 192) and (nh == nkv or (nh // nkv) % 2 == 0)
+                and all(p.weight.dtype == torch.bfloat16 for p in projs) and _plain(*projs, self.q_norm, self.k_norm)):
+            return None
+        ws = (self.q_proj.weight, self.k_proj.weight, self.v_proj.weight)
+        w_qkv = _derived(self, "qkv", ws, lambda: torch.cat(ws, 0).contiguous())
+        half = (None, None)
+        if self.is_swa:                                                         # base.py:87-91
+            half = _derived(self, "rope", (cos, sin), lambda: tuple(t[:, :d // 2].float().contiguous() for t in (cos, sin)))
+        return L.native().exp_attention(x, w_qkv, self.o_proj.weight, _fp32_copy(self.q_norm, "weight") if normed else None,
+                                        _fp32_copy(self.k_norm, "weight") if normed else None,
+                                        self.q_norm.variance_epsilon if normed else 0.0, *half,
+                                        None if self.xsa_alpha is None else _fp32_copy(self, "xsa_alpha"), nh, nkv, d,
+                                        self.sliding_window or 0, self.scaling)
+
     def forward(self, x, cos, sin):
+        out = self._native(x, cos, sin)
+        if out is not None:
+            return out
         B, S, _ = x.shape
         nh, nkv, d = self.num_heads, self.num_key_value_heads, self.head_dim
         g = nh // nkv
@@ -210,6 +258,16 @@ class BiBoExpMLP(nn.Module):
     def forward(self, x):
         return self.down_proj(F.silu(self.gate_proj(x)) * self.up_proj(x))
 
+    def added_to(self, base, x):
+        """base + self(x)"""
+        projs = (self.gate_proj, self.up_proj, self.down_proj)
+        if (_native_ok(x) and x.dtype == base.dtype and self.gate_proj.weight.shape[0] % 8 == 0
+                and all(p.weight.dtype == torch.bfloat16 for p in projs) and _plain(self, *projs)):
+            ws = (self.gate_proj.weight, self.up_proj.weight)
+            return L.native().exp_mlp(x, _derived(self, "gate_up", ws, lambda: torch.cat(ws, 0).contiguous()),
+                                      self.down_proj.weight, base)
+        return base + self(x)
+
 
 class BiBoExpDecoderLayer(nn.Module):
     """One layer of `_forward_attention_residuals` (exp/modeling_bibo.py:466-671) with sites = 1 and carry."""
@@ -233,21 +291,32 @@ class BiBoExpDecoderLayer(nn.Module):
     def forward(self, hidden_states, blocks, cos, sin, collect_routing=False):
         B, S, H = hidden_states.shape
         prefix = hidden_states
-        hs = hidden_states
+        native = _native_ok(hidden_states) and H % 8 == 0 and H <= 1024 and len(blocks) < 8
+        hs, xn = hidden_states, None
         if blocks:                                                              # depth-mix read (:484-492)
-            hs = attention_residual(prefix.reshape(-1, H), blocks, self.self_attention_res_proj.weight,
-                                    self.self_attention_res_norm.weight,
-                                    self.self_attention_res_norm.variance_epsilon).view(B, S, H)
+            res = self.self_attention_res_norm
+            if native and _plain(res, self.self_attention_res_proj, self.input_layernorm):
+                ln = self.input_layernorm
+                hs, xn = L.native().exp_attn_res_norm(
+                    [*(b.view(B, S, H) for b in blocks), prefix],
+                    _score_weight(self, self.self_attention_res_proj.weight, res.weight), res.variance_epsilon,
+                    _fp32_copy(ln, "weight"), ln.variance_epsilon)
+            else:
+                hs = attention_residual(prefix.reshape(-1, H), blocks, self.self_attention_res_proj.weight, res.weight,
+                                        res.variance_epsilon).view(B, S, H)
         attn_read = hs
         if self.layer_idx % self.attn_res_block_size == 0:                      # block boundary (:526-531)
             blocks = blocks + [prefix.reshape(-1, H)]
             prefix = None
-        a = self.self_attn(self.input_layernorm(hs), cos, sin)
-        prefix = a if prefix is None else prefix + a
-        if self.attn_res_carry_theta is not None:                               # carry write (:640-648)
-            hs = attn_read + self.attn_res_carry_theta.float().to(a.dtype) * a
+        a = self.self_attn(self.input_layernorm(hs) if xn is None else xn, cos, sin)
+        theta = self.attn_res_carry_theta
+        if native and a.is_contiguous() and a.dtype == hidden_states.dtype:     # carry write (:640-648)
+            th = (None if theta is None else
+                  _derived(self, "carry", (theta,), lambda: theta.detach().float().to(a.dtype).float().expand(H).contiguous()))
+            hs, prefix = L.native().exp_carry(attn_read, a, th, prefix)
         else:
-            hs = attn_read + a
+            prefix = a if prefix is None else prefix + a
+            hs = attn_read + (a if theta is None else theta.float().to(a.dtype) * a)
         ln = self.post_attention_layernorm
         if self.is_moe_layer:
             # prefix_sum + mlp(post_attention_layernorm(hs)) (:429-431, :666) as one library call
@@ -259,7 +328,7 @@ class BiBoExpDecoderLayer(nn.Module):
                 out = self.mlp.ffn_forward(hs, ln.weight, ln.variance_epsilon, residual=prefix,
                                            bf16_moe_out=hs.dtype == torch.bfloat16)
         else:
-            out = prefix + self.mlp(ln(hs))
+            out = self.mlp.added_to(prefix, ln(hs))
         return out, blocks
 
     def _moe_with_routing(self, hs, prefix):
@@ -298,15 +367,34 @@ class BiBoExpModel(nn.Module):
         h = self.embed_tokens(input_ids)
         if self.config.bf16_residual_stream:                                    # exp/modeling_bibo.py:858-859
             h = h.to(torch.bfloat16)
-        ang = torch.arange(S, device=h.device, dtype=torch.float32)[:, None] * self.inv_freq.float()[None, :]
-        ang = torch.cat((ang, ang), dim=-1)
-        cos, sin = ang.cos().to(h.dtype), ang.sin().to(h.dtype)                 # embed.py:63-74
+        cos, sin = self._rope_tables(S, h)
         blocks = []
         for layer in self.layers:
             h, blocks = layer(h, blocks, cos, sin, collect_routing)
-        h = attention_residual(h.reshape(-1, H), blocks, self.output_attn_res_proj.weight, self.output_attn_res_norm.weight,
-                               self.output_attn_res_norm.variance_epsilon).view(B, S, H)     # :916-920
+        res = self.output_attn_res_norm                                         # :916-920
+        if (_native_ok(h) and H % 8 == 0 and H <= 1024 and len(blocks) < 8 and _plain(res, self.output_attn_res_proj, self.norm)):
+            return L.native().exp_attn_res_norm([*(b.view(B, S, H) for b in blocks), h],
+                                                _score_weight(self, self.output_attn_res_proj.weight, res.weight),
+                                                res.variance_epsilon, _fp32_copy(self.norm, "weight"),
+                                                self.norm.variance_epsilon)[1]
+        h = attention_residual(h.reshape(-1, H), blocks, self.output_attn_res_proj.weight, res.weight,
+                               res.variance_epsilon).view(B, S, H)
         return self.norm(h)
+
+    def _rope_tables(self, S, h):
+        """cos and sin [S, head_dim] in the stream's dtype (embed.py:63-74); those of the last sequence length are kept."""
+        def make():
+            ang = torch.arange(S, device=h.device, dtype=torch.float32)[:, None] * self.inv_freq.float()[None, :]
+            ang = torch.cat((ang, ang), dim=-1)
+            return ang.cos().to(h.dtype), ang.sin().to(h.dtype)
+        if torch.is_grad_enabled():
+            return make()
+        kept = self.__dict__.get("_rope_kept")
+        key = (S, h.dtype, h.device)
+        if kept is None or kept[0] != key:
+            self.__dict__["_rope_kept"] = (key,)
+            self.__dict__.pop("_derived_tables", None)
+        return _derived(self, "tables", (self.inv_freq,), make)
 
 
 class BiBoExpForCausalLM(nn.Module):

@@ -1,0 +1,107 @@
+"""The launches around the MoE block in the 10-layer forward, through the C ABI, against plain fp32 PyTorch on the CPU: QK-norm
+and RoPE in place, causal / banded attention with XSA at the edges of its 32-key blocks and query blocks, the depth mix with
+its norm, the carry sums and SwiGLU's product."""
+import ctypes
+
+import pytest
+import torch
+
+from bibo_amd import _lib as L
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+def _ptr(t):
+    return None if t is None else ctypes.c_void_p(t.data_ptr())
+
+
+def _call(name, *args):
+    L.check(getattr(L.lib(), name)(*args, ctypes.c_void_p(torch.cuda.current_stream(DEV).cuda_stream)), name)
+    torch.cuda.synchronize()
+
+
+def _rel(a, ref):
+    return float((a.float().cpu() - ref).abs().max() / ref.abs().max().clamp_min(1e-30))
+
+
+@pytest.mark.parametrize("D,nq,nkv", [(64, 2, 2), (64, 4, 1), (128, 2, 1), (192, 4, 2)])
+@pytest.mark.parametrize("S,window", [(1, 0), (31, 0), (33, 16), (64, 64), (65, 0), (129, 32), (200, 128), (300, 0), (390, 33)])
+def test_attention(D, nq, nkv, S, window):
+    B, ld = 2, (nq + 2 * nkv) * D + 8
+    g = torch.Generator().manual_seed(S + D)
+    qkv = torch.randn(B, S, ld, generator=g).bfloat16()
+    qkv[0, S // 2, :nq * D] *= 30                                  # a row whose maximum jumps late
+    qw, kw = torch.rand(D, generator=g) + 0.5, torch.rand(D, generator=g) + 0.5
+    ang = torch.arange(S)[:, None] * (10000.0 ** (-torch.arange(0, D, 2) / D))[None]
+    cos, sin = ang.cos(), ang.sin()
+    alpha = torch.randn(nq, generator=g)
+    scale = D ** -0.5
+    d = qkv.to(DEV)
+    dev = [t.to(DEV).contiguous() for t in (qw, kw, cos, sin, alpha)]
+    _call("bibo_moe_exp_qk_norm_rope", _ptr(d), ld, B, S, nq, nkv, D, _ptr(dev[0]), _ptr(dev[1]), ctypes.c_float(1e-6), _ptr(dev[2]), _ptr(dev[3]))
+    x = qkv.float()
+
+    def heads(lo, n):
+        return x[..., lo * D:(lo + n) * D].reshape(B, S, n, D)
+
+    def norm_rope(t, w):
+        t = (t * torch.rsqrt(t.pow(2).mean(-1, keepdim=True) + 1e-6)).bfloat16().float() * w
+        a, b = t[..., :D // 2], t[..., D // 2:]
+        c, s = cos[None, :, None], sin[None, :, None]
+        return torch.cat((a * c - b * s, b * c + a * s), -1)
+
+    q, k, v = norm_rope(heads(0, nq), qw), norm_rope(heads(nq, nkv), kw), heads(nq + nkv, nkv)
+    got = d.cpu().float()
+    assert _rel(got[..., :nq * D].reshape(q.shape), q) <= 8e-3 and _rel(got[..., nq * D:(nq + nkv) * D].reshape(k.shape), k) <= 8e-3
+    assert torch.equal(got[..., (nq + nkv) * D:], x[..., (nq + nkv) * D:])          # v and the padding stay as they are
+    q, k = got[..., :nq * D].reshape(q.shape), got[..., nq * D:(nq + nkv) * D].reshape(k.shape)
+    rep = nq // nkv
+    kx, vx = k.repeat_interleave(rep, 2), v.repeat_interleave(rep, 2)
+    i = torch.arange(S)
+    allow = (i[None] <= i[:, None]) & ((i[:, None] - i[None] < window) if window else True)
+    for xsa in (None, dev[4]):
+        out = torch.full((B, S, nq * D), float("nan"), dtype=torch.bfloat16, device=DEV)
+        _call("bibo_moe_exp_attention_fwd", _ptr(d), ld, B, S, nq, nkv, D, window, ctypes.c_float(scale), _ptr(xsa), _ptr(out))
+        y = torch.empty(B, S, nq, D)
+        for h in range(nq):
+            p = (q[:, :, h] @ k[:, :, h // rep].transpose(1, 2).contiguous() * scale).masked_fill(~allow, -torch.inf).softmax(-1)
+            y[:, :, h] = p @ vx[:, :, h]
+        if xsa is not None:
+            vn = torch.nn.functional.normalize(vx, dim=-1)
+            y = y - (y * vn).sum(-1, keepdim=True) * torch.tanh(alpha)[None, None, :, None] * vn
+        assert _rel(out, y.reshape(B, S, nq * D)) <= 1e-2, (xsa is not None)
+
+
+def test_attention_refuses_what_it_does_not_take():
+    args = lambda nq, nkv, D: (None, 4096, 1, 4, nq, nkv, D, 0, ctypes.c_float(1.0), None, None, None)
+    for nq, nkv, D in ((4, 2, 96), (3, 2, 64), (3, 1, 64), (4, 0, 64)):
+        assert L.lib().bibo_moe_exp_attention_fwd(*args(nq, nkv, D)) == -6
+    assert L.lib().bibo_moe_exp_attention_fwd(*args(4, 2, 64)) == -1
+
+
+@pytest.mark.parametrize("T,H", [(1, 8), (3, 520), (7, 768), (65, 1024)])
+def test_depth_mix_carry_and_swiglu(T, H):
+    g = torch.Generator().manual_seed(T + H)
+    rows = lambda: torch.randn(T, H, generator=g).bfloat16()
+    sw, nw, theta = torch.randn(H, generator=g) * 0.1, torch.rand(H, generator=g) + 0.5, torch.rand(H, generator=g)
+    for n in (1, 2, 5, 8):
+        cands = [rows() for _ in range(n)]
+        dc = [c.to(DEV) for c in cands]
+        mixed, normed = L.native().exp_attn_res_norm(dc, sw.to(DEV), 1e-6, nw.to(DEV), 1e-6)
+        v = torch.stack([c.float() for c in cands], 1)
+        ref = (((v @ sw) * torch.rsqrt(v.pow(2).mean(-1) + 1e-6)).softmax(-1)[..., None] * v).sum(1)
+        assert _rel(mixed, ref) <= 8e-3
+        m = mixed.cpu().float()
+        assert _rel(normed, (m * torch.rsqrt(m.pow(2).mean(-1, keepdim=True) + 1e-6)) * nw) <= 1.2e-2
+        assert torch.equal(L.native().exp_attn_res_norm(dc, sw.to(DEV), 1e-6, None, 0.0)[0], mixed)
+    r, a, p = rows(), rows(), rows()
+    hs, prefix = L.native().exp_carry(r.to(DEV), a.to(DEV), theta.to(DEV), p.to(DEV))
+    assert _rel(hs, r.float() + theta * a.float()) <= 8e-3 and torch.equal(prefix.cpu(), p + a)
+    hs, prefix = L.native().exp_carry(r.to(DEV), a.to(DEV), None, None)
+    assert torch.equal(hs.cpu(), r + a) and torch.equal(prefix.cpu(), a)
+    gu = torch.randn(T, 2 * H, generator=g).bfloat16().to(DEV)
+    out = torch.empty(T, H, dtype=torch.bfloat16, device=DEV)
+    _call("bibo_moe_exp_silu_mul_fwd", _ptr(gu), T, H, _ptr(out))
+    f = gu.cpu().float()
+    assert _rel(out, torch.nn.functional.silu(f[:, :H]) * f[:, H:]) <= 8e-3
