@@ -439,7 +439,7 @@ int backward_mfma(const void* x, const void* d_out, const void* w_router, const 
   b.wgrad_plan = reinterpret_cast<int*>(base + ws.wgrad_plan);
   return hip_rc(launch_backward(x, d_out, w_router, w_gate_up, w_down, theta, logits, idx, w, offsets, perm_slot, perm_token,
                                 T, H, E - sh->n_pos - sh->n_neg, sh->n_pos, sh->n_neg, k, I, norm_mode, sh->act, b, d_x,
-                                d_w_router, d_w_gate_up, d_w_down, d_theta, s, gu_saved));
+                                d_w_router, d_w_gate_up, d_w_down, d_theta, (sh->flags & BIBO_FLAG_GRAD_F32) != 0, s, gu_saved));
 }
 
 // whether a shape has the training forward that keeps its state: the fused forward kernel and the MFMA backward both take it
@@ -727,7 +727,8 @@ int bibo_moe_backward(const void* x, const void* d_out, const void* w_router, co
     g.dl = reinterpret_cast<float*>(gb + gw.dl); g.dtheta_row = reinterpret_cast<float*>(gb + gw.dtheta_row);
     return hip_rc(launch_backward_generic(x, d_out, w_router, w_gate_up, w_down, theta, g_logits, g_idx, g_w, g_offsets, g_slot,
                                           g_token, T, H, E - sh->n_pos - sh->n_neg, sh->n_pos, sh->n_neg, k, I, sh->dtype,
-                                          norm_mode, sh->act, g, d_x, d_w_router, d_w_gate_up, d_w_down, d_theta, gs));
+                                          norm_mode, sh->act, g, d_x, d_w_router, d_w_gate_up, d_w_down, d_theta,
+                                          (sh->flags & BIBO_FLAG_GRAD_F32) != 0, gs));
   }
   return backward_mfma(x, d_out, w_router, bias, w_gate_up, w_down, theta, sh, norm_mode, nullptr, d_x, d_w_router,
                        d_w_gate_up, d_w_down, d_theta, d_w_out, workspace, workspace_bytes, stream);
@@ -804,7 +805,7 @@ int bibo_moe_experts_backward(const void* x, const void* d_out, const int32_t* i
     g.dl = reinterpret_cast<float*>(gb + gw.dl); g.dtheta_row = reinterpret_cast<float*>(gb + gw.dtheta_row);
     return hip_rc(launch_backward_generic(x, d_out, nullptr, w_gate_up, w_down, theta, nullptr, idx, w, g_offsets, g_slot, g_token,
                                           T, H, E - sh->n_pos - sh->n_neg, sh->n_pos, sh->n_neg, k, I, sh->dtype, BIBO_NORM_SUM,
-                                          sh->act, g, d_x, nullptr, d_w_gate_up, d_w_down, d_theta, gs));
+                                          sh->act, g, d_x, nullptr, d_w_gate_up, d_w_down, d_theta, (sh->flags & BIBO_FLAG_GRAD_F32) != 0, gs));
   }
   if (!aligned16(x) || !aligned16(d_out) || !aligned16(w_gate_up) || !aligned16(w_down) || !aligned16(d_x) ||
       !aligned16(d_w_gate_up) || !aligned16(d_w_down))
@@ -830,7 +831,7 @@ int bibo_moe_experts_backward(const void* x, const void* d_out, const int32_t* i
   b.wgrad_plan = reinterpret_cast<int*>(base + ws.wgrad_plan);
   return hip_rc(launch_backward(x, d_out, nullptr, w_gate_up, w_down, theta, nullptr, idx, w, offsets, perm_slot, perm_token,
                                 T, H, E - sh->n_pos - sh->n_neg, sh->n_pos, sh->n_neg, k, I, BIBO_NORM_SUM, sh->act, b, d_x,
-                                nullptr, d_w_gate_up, d_w_down, d_theta, s));
+                                nullptr, d_w_gate_up, d_w_down, d_theta, (sh->flags & BIBO_FLAG_GRAD_F32) != 0, s));
 }
 
 int bibo_moe_balance_step(const int32_t* counts, float* accumulated, float* bias, int E, float factor, int update, void* stream) {

@@ -169,29 +169,29 @@ hipError_t launch_dgrad(const bf16_t* A, const int32_t* a_index, const bf16_t* W
 // dW[e] = P(rows of e)^T Q(rows of e), P [.., N] and Q [.., M] row-major (kmajor.h)
 template <int MT, bool GATHER_P, bool GATHER_Q>
 hipError_t launch_wgrad_t(const bf16_t* P, const bf16_t* Q, const int32_t* index, const int32_t* offsets, const bf16_t* zrow,
-                          int N, int M, int E, int slots, const int* plan, float* part, bf16_t* dW, hipStream_t s) {
+                          int N, int M, int E, int slots, const int* plan, float* part, void* dW, int f32, hipStream_t s) {
   const dim3 block(512);               // (the partial tiles of cut experts are added up by backward_sums_kernel)
   auto grid = [&](int bn) { return dim3((unsigned)((slots * (N / (64 * MT)) * (M / bn) + 7) & ~7)); };
   if (M % 384 == 0)
     hipLaunchKernelGGL((wgrad_kmajor_kernel<MT, 3, GATHER_P, GATHER_Q>), grid(384), block, 0, s, P, Q, index, offsets, zrow, N,
-                       M, E, plan, part, dW);
+                       M, E, plan, part, dW, f32);
   else if (M % 256 == 0)
     hipLaunchKernelGGL((wgrad_kmajor_kernel<MT, 2, GATHER_P, GATHER_Q>), grid(256), block, 0, s, P, Q, index, offsets, zrow, N,
-                       M, E, plan, part, dW);
+                       M, E, plan, part, dW, f32);
   else
     hipLaunchKernelGGL((wgrad_kmajor_kernel<MT, 1, GATHER_P, GATHER_Q>), grid(128), block, 0, s, P, Q, index, offsets, zrow, N,
-                       M, E, plan, part, dW);
+                       M, E, plan, part, dW, f32);
   return hipGetLastError();
 }
 
 // 256 rows of dW per workgroup where N allows and the experts have rows enough for the streams to matter
 template <bool GATHER_P, bool GATHER_Q>
 hipError_t launch_wgrad(const bf16_t* P, const bf16_t* Q, const int32_t* index, const int32_t* offsets, const bf16_t* zrow,
-                        int N, int M, int S_rows, int E, int slots, const int* plan, float* part, bf16_t* dW, hipStream_t s) {
+                        int N, int M, int S_rows, int E, int slots, const int* plan, float* part, void* dW, int f32, hipStream_t s) {
   const int bn = M % 384 == 0 ? 384 : (M % 256 == 0 ? 256 : 128);
   if (N % 256 == 0 && tall_tiles(S_rows, E, (long long)E * (N / 128) * (M / bn), (long long)E * (N / 256) * (M / bn)))
-    return launch_wgrad_t<4, GATHER_P, GATHER_Q>(P, Q, index, offsets, zrow, N, M, E, slots, plan, part, dW, s);
-  return launch_wgrad_t<2, GATHER_P, GATHER_Q>(P, Q, index, offsets, zrow, N, M, E, slots, plan, part, dW, s);
+    return launch_wgrad_t<4, GATHER_P, GATHER_Q>(P, Q, index, offsets, zrow, N, M, E, slots, plan, part, dW, f32, s);
+  return launch_wgrad_t<2, GATHER_P, GATHER_Q>(P, Q, index, offsets, zrow, N, M, E, slots, plan, part, dW, f32, s);
 }
 
 // ---- Radial NormSiLU backward (moe.py:87-92), one wave per permuted row ----------------------------------------
@@ -439,13 +439,13 @@ __global__ __launch_bounds__(256) void dwr_partial_kernel(const bf16_t* __restri
 __global__ __launch_bounds__(256) void backward_sums_kernel(int nb_w, const float* __restrict__ part_a,
                                                             const float* __restrict__ part_b, const int* __restrict__ plan,
                                                             int slots, int NMa, int NMb, int E, int Et,
-                                                            bf16_t* __restrict__ dWa, bf16_t* __restrict__ dWb,
+                                                            void* __restrict__ dWa, void* __restrict__ dWb, int f32,
                                                             const float* __restrict__ dtheta_row, float* __restrict__ dtheta,
                                                             const float* __restrict__ dwr_part, int H,
-                                                            bf16_t* __restrict__ dwr) {
+                                                            void* __restrict__ dwr) {
   const int block = blockIdx.x;
   if (block < nb_w) {
-    wgrad_reduce_block(block, part_a, part_b, plan, slots, NMa, NMb, E, dWa, dWb);
+    wgrad_reduce_block(block, part_a, part_b, plan, slots, NMa, NMb, E, dWa, dWb, f32);
     return;
   }
   const int* experts = plan + 4 + 4 * (slots + Et);            // {first chunk, chunks, ., .} per expert
@@ -474,7 +474,8 @@ __global__ __launch_bounds__(256) void backward_sums_kernel(int nb_w, const floa
   const int first = experts[4 * e], chunks = experts[4 * e + 1];
   float acc = 0.f;
   for (int j = 0; j < chunks * kDwrSplit; ++j) acc += dwr_part[((size_t)first * kDwrSplit + j) * H + c];
-  dwr[i] = (bf16_t)acc;
+  if (f32) static_cast<float*>(dwr)[i] = acc;
+  else static_cast<bf16_t*>(dwr)[i] = (bf16_t)acc;
 }
 
 // zero n 4-byte words (a kernel rather than a memset node, so that the call can be captured into a graph)
@@ -524,7 +525,9 @@ hipError_t launch_backward(const void* x, const void* d_out, const void* w_route
                            const float* theta, const float* logits, const int32_t* idx, const float* w,
                            const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int T, int H, int E,
                            int n_pos, int n_neg, int k, int I, int norm_mode, int act, const BackwardBuffers& b, void* dx,
-                           void* d_w_router, void* d_wgu, void* d_wd, float* d_theta, hipStream_t s, const void* gu_saved) {
+                           void* d_w_router, void* d_wgu, void* d_wd, float* d_theta, int grad_f32,
+                           hipStream_t s, const void* gu_saved) {
+  const size_t gb = grad_f32 ? sizeof(float) : sizeof(bf16_t);      // bytes per element of the weight gradients
   // E = GLU experts (with weights); the router and the permutation know Et experts, the +/-Identity ones last
   const int Et = E + n_pos + n_neg;
   const int S = T * k;
@@ -544,9 +547,9 @@ hipError_t launch_backward(const void* x, const void* d_out, const void* w_route
   hipError_t err = hipSuccess;
   if (S == 0) {
     zero_bytes(d_theta, (size_t)E * sizeof(float), s);
-    if (d_w_router != nullptr) zero_bytes(d_w_router, (size_t)Et * H * sizeof(bf16_t), s);
-    zero_bytes(d_wgu, (size_t)E * 2 * I * H * sizeof(bf16_t), s);
-    zero_bytes(d_wd, (size_t)E * H * I * sizeof(bf16_t), s);
+    if (d_w_router != nullptr) zero_bytes(d_w_router, (size_t)Et * H * gb, s);
+    zero_bytes(d_wgu, (size_t)E * 2 * I * H * gb, s);
+    zero_bytes(d_wd, (size_t)E * H * I * gb, s);
     return hipGetLastError();
   }
   // pre-activations again (moe.py:84): x W_gate_up^T, both contiguous along H - by the first phase of the forward
@@ -581,17 +584,17 @@ hipError_t launch_backward(const void* x, const void* d_out, const void* w_route
                        perm_slot, perm_token, H, b.dwr_part);
   // weight gradients, contracted over each expert's rows: dW_down[e] = d^T (w h) (d gathered by token, `hidden`
   // already carries w), dW_gate_up[e] = [dg, du]^T x (x gathered by token)
-  err = launch_wgrad<true, false>(dop, hidden, perm_token, offsets, zrow, H, I, S, E, slots, b.wgrad_plan, b.wgrad_part, static_cast<bf16_t*>(d_wd), s);
+  err = launch_wgrad<true, false>(dop, hidden, perm_token, offsets, zrow, H, I, S, E, slots, b.wgrad_plan, b.wgrad_part, d_wd, grad_f32, s);
   if (err != hipSuccess) return err;
   float* part_gu = b.wgrad_part + (size_t)slots * H * I;
-  err = launch_wgrad<false, true>(dgu, xp, perm_token, offsets, zrow, 2 * I, H, S, E, slots, b.wgrad_plan, part_gu, static_cast<bf16_t*>(d_wgu), s);
+  err = launch_wgrad<false, true>(dgu, xp, perm_token, offsets, zrow, 2 * I, H, S, E, slots, b.wgrad_plan, part_gu, d_wgu, grad_f32, s);
   if (err != hipSuccess) return err;
   // the sums that end the pass: cut experts' partial tiles, dtheta, the router's weight gradient
   const int nb_w = (int)(((size_t)2 * I * H / 4 + 255) / 256);
   const int nb_r = with_router ? (Et * H + 255) / 256 : 0;
   hipLaunchKernelGGL(backward_sums_kernel, dim3(nb_w + E + nb_r), dim3(256), 0, s, nb_w, b.wgrad_part, part_gu, b.wgrad_plan,
-                     slots, H * I, 2 * I * H, E, Et, static_cast<bf16_t*>(d_wd), static_cast<bf16_t*>(d_wgu), b.dtheta_row,
-                     d_theta, b.dwr_part, H, with_router ? static_cast<bf16_t*>(d_w_router) : nullptr);
+                     slots, H * I, 2 * I * H, E, Et, d_wd, d_wgu, grad_f32, b.dtheta_row,
+                     d_theta, b.dwr_part, H, with_router ? d_w_router : nullptr);
   return hipGetLastError();
 }
 

@@ -266,13 +266,13 @@ __global__ __launch_bounds__(256) void token_bwd_generic_kernel(const TIn* __res
 // grid (Et, ceil(H / 64) + 1).  Blocks y < ceil(H / 64): dW_router[e, h] = sum over the rows r of expert e of dl[slot(r)]
 // x[token(r), h] for 64 columns: 16 row groups of 16 threads x 4 columns, the groups' sums added in order (dwr == NULL: none).
 // The last y: dtheta[e] = the sum of its rows' shares (e < E).
-template <typename TIn>
+template <typename TIn, typename TG>
 __global__ __launch_bounds__(256) void expert_sums_generic_kernel(const TIn* __restrict__ x, const float* __restrict__ dl,
                                                                   const int32_t* __restrict__ offsets,
                                                                   const int32_t* __restrict__ perm_slot,
                                                                   const int32_t* __restrict__ perm_token, int H, int E,
                                                                   const float* __restrict__ dtheta_row,
-                                                                  float* __restrict__ dtheta, TIn* __restrict__ dwr) {
+                                                                  float* __restrict__ dtheta, TG* __restrict__ dwr) {
   __shared__ float red[16][65];
   const int e = blockIdx.x, tid = threadIdx.x;
   const int lo = offsets[e], hi = offsets[e + 1];
@@ -310,7 +310,7 @@ __global__ __launch_bounds__(256) void expert_sums_generic_kernel(const TIn* __r
     float sum = 0.f;
 #pragma unroll
     for (int g = 0; g < 16; ++g) sum += red[g][tid];
-    dwr[(size_t)e * H + h0 + tid] = from_float<TIn>(sum);
+    dwr[(size_t)e * H + h0 + tid] = from_float<TG>(sum);
   }
 }
 
@@ -348,7 +348,8 @@ void zero_elems(TIn* p, size_t n, hipStream_t s) {
   hipLaunchKernelGGL(zero_generic_kernel<TIn>, dim3(grid), dim3(256), 0, s, p, n);
 }
 
-template <typename TIn>
+// TG: type of the weight gradients
+template <typename TIn, typename TG>
 hipError_t launch_t(const void* x_, const void* d_out_, const void* w_router_, const void* wgu_, const void* wd_,
                     const float* theta, const float* logits, const int32_t* idx, const float* w, const int32_t* offsets,
                     const int32_t* perm_slot, const int32_t* perm_token, int T, int H, int E, int n_pos, int n_neg, int k, int I,
@@ -362,9 +363,9 @@ hipError_t launch_t(const void* x_, const void* d_out_, const void* w_router_, c
   const int Et = E + n_pos + n_neg, S = T * k;
   if (S == 0) {
     zero_elems(d_theta, (size_t)E, s);
-    if (d_w_router_ != nullptr) zero_elems(static_cast<TIn*>(d_w_router_), (size_t)Et * H, s);
-    zero_elems(static_cast<TIn*>(d_wgu_), (size_t)E * 2 * I * H, s);
-    zero_elems(static_cast<TIn*>(d_wd_), (size_t)E * H * I, s);
+    if (d_w_router_ != nullptr) zero_elems(static_cast<TG*>(d_w_router_), (size_t)Et * H, s);
+    zero_elems(static_cast<TG*>(d_wgu_), (size_t)E * 2 * I * H, s);
+    zero_elems(static_cast<TG*>(d_wd_), (size_t)E * H * I, s);
     return hipGetLastError();
   }
   const bool tiles = tile_f32_supported(H, I) && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(d_out) |
@@ -385,17 +386,17 @@ hipError_t launch_t(const void* x_, const void* d_out_, const void* w_router_, c
   const bool with_router = w_router != nullptr;      // else: the experts alone, the caller owns the routing
   hipLaunchKernelGGL(token_bwd_generic_kernel<TIn>, dim3((T + 3) / 4), dim3(256), 0, s, x, d_out, b.dxs, logits, idx, w, w_router, T,
                      H, E, n_pos, n_neg, k, norm_mode, b.dw_slot, b.dl, static_cast<TIn*>(dx_));
-  hipLaunchKernelGGL(expert_sums_generic_kernel<TIn>, dim3(Et, (H + 63) / 64 + 1), dim3(256), 0, s, x, b.dl, offsets, perm_slot,
-                     perm_token, H, E, b.dtheta_row, d_theta, with_router ? static_cast<TIn*>(d_w_router_) : nullptr);
+  hipLaunchKernelGGL((expert_sums_generic_kernel<TIn, TG>), dim3(Et, (H + 63) / 64 + 1), dim3(256), 0, s, x, b.dl, offsets, perm_slot,
+                     perm_token, H, E, b.dtheta_row, d_theta, with_router ? static_cast<TG*>(d_w_router_) : nullptr);
   // dW_down[e] = d^T (w h), d gathered by token; dW_gate_up[e] = [dg, du]^T x, x gathered by token
   if (tiles) {
-    if ((err = launch_wgrad_f32<TIn, float, TIn, true, false>(d_out, b.hw, perm_token, offsets, H, I, E, static_cast<TIn*>(d_wd_), s)) != hipSuccess) return err;
-    return launch_wgrad_f32<float, TIn, TIn, false, true>(b.dgu, x, perm_token, offsets, 2 * I, H, E, static_cast<TIn*>(d_wgu_), s);
+    if ((err = launch_wgrad_f32<TIn, float, TG, true, false>(d_out, b.hw, perm_token, offsets, H, I, E, static_cast<TG*>(d_wd_), s)) != hipSuccess) return err;
+    return launch_wgrad_f32<float, TIn, TG, false, true>(b.dgu, x, perm_token, offsets, 2 * I, H, E, static_cast<TG*>(d_wgu_), s);
   }
-  hipLaunchKernelGGL((wgrad_generic_kernel<TIn, float, TIn, true, false>), dim3(H, E), dim3(256), 0, s, d_out, b.hw, perm_token,
-                     offsets, H, I, static_cast<TIn*>(d_wd_));
-  hipLaunchKernelGGL((wgrad_generic_kernel<float, TIn, TIn, false, true>), dim3(2 * I, E), dim3(256), 0, s, b.dgu, x, perm_token,
-                     offsets, 2 * I, H, static_cast<TIn*>(d_wgu_));
+  hipLaunchKernelGGL((wgrad_generic_kernel<TIn, float, TG, true, false>), dim3(H, E), dim3(256), 0, s, d_out, b.hw, perm_token,
+                     offsets, H, I, static_cast<TG*>(d_wd_));
+  hipLaunchKernelGGL((wgrad_generic_kernel<float, TIn, TG, false, true>), dim3(2 * I, E), dim3(256), 0, s, b.dgu, x, perm_token,
+                     offsets, 2 * I, H, static_cast<TG*>(d_wgu_));
   return hipGetLastError();
 }
 
@@ -413,11 +414,14 @@ hipError_t launch_backward_generic(const void* x, const void* d_out, const void*
                                    const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int T, int H,
                                    int E, int n_pos, int n_neg, int k, int I, int dtype, int norm_mode, int act,
                                    const GenericBackwardBuffers& b, void* dx, void* d_w_router, void* d_wgu, void* d_wd,
-                                   float* d_theta, hipStream_t s) {
-  if (dtype == BIBO_DTYPE_BF16)
-    return launch_t<bf16_t>(x, d_out, w_router, wgu, wd, theta, logits, idx, w, offsets, perm_slot, perm_token, T, H, E, n_pos,
+                                   float* d_theta, int grad_f32, hipStream_t s) {
+  if (dtype == BIBO_DTYPE_BF16 && !grad_f32)
+    return launch_t<bf16_t, bf16_t>(x, d_out, w_router, wgu, wd, theta, logits, idx, w, offsets, perm_slot, perm_token, T, H, E, n_pos,
                             n_neg, k, I, norm_mode, act, b, dx, d_w_router, d_wgu, d_wd, d_theta, s);
-  return launch_t<float>(x, d_out, w_router, wgu, wd, theta, logits, idx, w, offsets, perm_slot, perm_token, T, H, E, n_pos,
+  if (dtype == BIBO_DTYPE_BF16)
+    return launch_t<bf16_t, float>(x, d_out, w_router, wgu, wd, theta, logits, idx, w, offsets, perm_slot, perm_token, T, H, E, n_pos,
+                            n_neg, k, I, norm_mode, act, b, dx, d_w_router, d_wgu, d_wd, d_theta, s);
+  return launch_t<float, float>(x, d_out, w_router, wgu, wd, theta, logits, idx, w, offsets, perm_slot, perm_token, T, H, E, n_pos,
                          n_neg, k, I, norm_mode, act, b, dx, d_w_router, d_wgu, d_wd, d_theta, s);
 }
 

@@ -209,10 +209,15 @@ class LayerFn : public torch::autograd::Function<LayerFn> {
     c10::DeviceGuard guard(x.device());
     const Tensor d = in_dtype(grads[0], x.scalar_type());
     const int64_t Eg = l.w_gate_up.size(0);
+    // fp32 master weights behind bf16 operands: the kernels' fp32 sums are the gradients
+    const bool grad_f32 = x.scalar_type() != at::kFloat && dtypes[1] == (int64_t)at::kFloat && dtypes[2] == (int64_t)at::kFloat &&
+                          dtypes[3] == (int64_t)at::kFloat;
     const bibo_moe_shape sh{(int32_t)(x.numel() / x.size(-1)), (int32_t)x.size(-1), (int32_t)(Eg + l.n_pos + l.n_neg), l.k,
-                            (int32_t)(l.w_gate_up.size(1) / 2), dtype_code(x), l.n_pos, l.n_neg, l.act, 0};
-    Tensor d_x = at::empty_like(x), d_wr = at::empty_like(l.w_router), d_gu = at::empty_like(l.w_gate_up),
-           d_dn = at::empty_like(l.w_down), d_th = at::empty_like(l.theta);
+                            (int32_t)(l.w_gate_up.size(1) / 2), dtype_code(x), l.n_pos, l.n_neg, l.act,
+                            grad_f32 ? BIBO_FLAG_GRAD_F32 : 0};
+    const at::TensorOptions wopt = l.w_gate_up.options().requires_grad(false).dtype(grad_f32 ? at::kFloat : x.scalar_type());
+    Tensor d_x = at::empty_like(x), d_wr = at::empty(l.w_router.sizes(), wopt), d_gu = at::empty(l.w_gate_up.sizes(), wopt),
+           d_dn = at::empty(l.w_down.sizes(), wopt), d_th = at::empty_like(l.theta);
     hipStream_t s = c10::hip::getCurrentHIPStream(x.device().index()).stream();
     size_t bytes = 0;
     check(bibo_moe_backward_workspace_bytes(&sh, &bytes), "bibo_moe_backward_workspace_bytes");

@@ -257,11 +257,12 @@ hipError_t launch_backward_generic(const void* x, const void* d_out, const void*
                                    const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int T, int H,
                                    int E, int n_pos, int n_neg, int k, int I, int dtype, int norm_mode, int act,
                                    const GenericBackwardBuffers& b, void* dx, void* d_w_router, void* d_wgu, void* d_wd,
-                                   float* d_theta, hipStream_t s);
+                                   float* d_theta, int grad_f32, hipStream_t s);
 hipError_t launch_backward(const void* x, const void* d_out, const void* w_router, const void* wgu, const void* wd,
                            const float* theta, const float* logits, const int32_t* idx, const float* w,
                            const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int T, int H, int E,
                            int n_pos, int n_neg, int k, int I, int norm_mode, int act, const BackwardBuffers& b, void* dx,
-                           void* d_w_router, void* d_wgu, void* d_wd, float* d_theta, hipStream_t s, const void* gu_saved = nullptr);
+                           void* d_w_router, void* d_wgu, void* d_wd, float* d_theta, int grad_f32, hipStream_t s,
+                           const void* gu_saved = nullptr);
 
 }  // namespace bibo

@@ -293,7 +293,8 @@ __global__ __launch_bounds__(512) void dgrad_kmajor_kernel(const bf16_t* __restr
 // An expert with more than `chunk` rows is cut into chunks of that many rows, each a workgroup of its own per tile of
 // dW, so that a few experts holding most of the rows do not leave a few workgroups with most of the work; such an
 // expert's chunks write fp32 partial tiles to `part` (one [N, M] slot per chunk, slots numbered over all experts'
-// chunks) and wgrad_reduce_block adds them in chunk order.  Experts of one chunk write dW directly.  The chunks are
+// chunks) and wgrad_reduce_block adds them in chunk order.  Experts of one chunk write dW directly, in bf16 or, with `f32`
+// (gradients of fp32 master weights), as they are: a conversion pass afterwards cost 61 us at T = 8192.  The chunks are
 // listed once per backward pass by wgrad_plan (below), so that a workgroup finds its chunk with one load.
 struct WgradPlan {
   int total;         // chunks over all experts
@@ -328,7 +329,7 @@ __global__ __launch_bounds__(512) void wgrad_kmajor_kernel(const bf16_t* __restr
                                                            const int32_t* __restrict__ offsets,
                                                            const bf16_t* __restrict__ zrow, int N, int M, int E,
                                                            const int* __restrict__ plan, float* __restrict__ part,
-                                                           bf16_t* __restrict__ dW) {
+                                                           void* __restrict__ dW, int f32) {
   static_assert(MT == 2 || MT == 4, "128 or 256 rows of dW per workgroup");
   constexpr int BM = 64 * MT, BN = kSubW * NTW;
   constexpr int R = MT == 4 ? 3 : kRing;                 // stages that fit LDS (MT = 4: 40 KB each)
@@ -450,8 +451,8 @@ __global__ __launch_bounds__(512) void wgrad_kmajor_kernel(const bf16_t* __restr
   // m0 + (wn NTW + j) 32 + 8 q + 4 (lane / 32) + r
   const int n = lane & 31, hh = lane >> 5;
   const size_t oofs = ((size_t)n0 + wm * MT * 32 + n) * M + m0 + wn * NTW * 32 + 4 * hh;
-  if (e_chunks == 1) {
-    bf16_t* orow = dW + (size_t)e * N * M + oofs;
+  if (e_chunks == 1 && !f32) {
+    bf16_t* orow = static_cast<bf16_t*>(dW) + (size_t)e * N * M + oofs;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -464,7 +465,7 @@ __global__ __launch_bounds__(512) void wgrad_kmajor_kernel(const bf16_t* __restr
           *reinterpret_cast<bf16x4*>(orow + (size_t)mt * 32 * M + j * 32 + 8 * q) = v;
         }
   } else {
-    float* prow = part + (size_t)cg * N * M + oofs;
+    float* prow = (e_chunks == 1 ? static_cast<float*>(dW) + (size_t)e * N * M : part + (size_t)cg * N * M) + oofs;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -484,12 +485,12 @@ __global__ __launch_bounds__(512) void wgrad_kmajor_kernel(const bf16_t* __restr
 // second in `part_b`).  Workgroup `block` of 256 threads, a thread per four elements.  E = experts with weights.
 __device__ __forceinline__ void wgrad_reduce_block(int block, const float* __restrict__ part_a, const float* __restrict__ part_b,
                                                    const int* __restrict__ plan, int slots, int NMa, int NMb, int E,
-                                                   bf16_t* __restrict__ dWa, bf16_t* __restrict__ dWb) {
+                                                   void* __restrict__ dWa, void* __restrict__ dWb, int f32) {
   const int n_cut = plan[1];
   if (n_cut == 0) return;
   const size_t i = ((size_t)block * 256 + threadIdx.x) * 4;
   const int* cut = plan + 4 + 4 * slots;
-  auto reduce = [&](const float* part, int NM, bf16_t* dW, int e, int first, int n) {
+  auto reduce = [&](const float* part, int NM, void* dW, int e, int first, int n) {
     if (i >= (size_t)NM) return;
     floatx4 acc = *reinterpret_cast<const floatx4*>(part + (size_t)first * NM + i);
     for (int c = 1; c < n; ++c) {
@@ -497,10 +498,14 @@ __device__ __forceinline__ void wgrad_reduce_block(int block, const float* __res
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[r] += v[r];
     }
+    if (f32) {
+      *reinterpret_cast<floatx4*>(static_cast<float*>(dW) + (size_t)e * NM + i) = acc;
+      return;
+    }
     bf16x4 o;
 #pragma unroll
     for (int r = 0; r < 4; ++r) o[r] = (bf16_t)acc[r];
-    *reinterpret_cast<bf16x4*>(dW + (size_t)e * NM + i) = o;
+    *reinterpret_cast<bf16x4*>(static_cast<bf16_t*>(dW) + (size_t)e * NM + i) = o;
   };
   for (int q = 0; q < n_cut; ++q) {
     const int e = cut[4 * q], first = cut[4 * q + 1], n = cut[4 * q + 2];

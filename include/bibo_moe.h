@@ -68,7 +68,10 @@ enum bibo_flags {
   /* bibo_moe_ffn_forward only: no residual at all, out = moe(rmsnorm(h)): the block as the reference's experimental
      decoder layer calls it under Block Attention Residuals (exp/modeling_bibo.py:429-431), where the caller owns
      the sum. */
-  BIBO_FLAG_NO_RESIDUAL = 2
+  BIBO_FLAG_NO_RESIDUAL = 2,
+  /* the backward calls only: d_w_router, d_w_gate_up and d_w_down are fp32 whatever `dtype` is (gradients of fp32 master
+     weights: the fp32 sums leave as they are, and no conversion pass follows). */
+  BIBO_FLAG_GRAD_F32 = 4
 };
 
 /* kernel family for the expert GEMMs */
@@ -270,7 +273,8 @@ int bibo_moe_ffn_forward(const void* h, const float* norm_weight, float eps, con
  * the selection, router.py:38, and gets no gradient; nor does anything flow through which experts were chosen).
  * x is the block's input as in bibo_moe_forward; the routing is recomputed from it by the forward's router kernel,
  * so the selection and the combine weights are those of the forward call on the same operands.
- *   d_x [T,H], d_w_router [E,H], d_w_gate_up [Eg,2I,H], d_w_down [Eg,H,I] in `dtype`; d_theta fp32 [Eg], with
+ *   d_x [T,H], d_w_router [E,H], d_w_gate_up [Eg,2I,H], d_w_down [Eg,H,I] in `dtype` (the last three in fp32 with
+ *   BIBO_FLAG_GRAD_F32); d_theta fp32 [Eg], with
  *   Eg = E - n_pos - n_neg GLU experts
  *   (reference pins: theta receives gradient, tests/test_moe.py:53-63, ablate/common/test_eager_radial.py:63-69);
  *   d_w_out fp32 [T,k] or NULL: gradient with respect to the combine weights (router.py:47), for inspection.
