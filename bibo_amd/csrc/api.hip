@@ -115,6 +115,13 @@ inline bool generic_tiles(int H, int I, int dtype) {
   return tile_f32_supported(H, I) && (dtype == BIBO_DTYPE_F32 || !mfma_supported(H, I, dtype));
 }
 
+// Whether a composite call that resolved to `algo` runs the few-token kernels (experts_few.hip).  A bf16 shape of the MFMA
+// families that a caller asks the generic one for does not.
+inline bool few_taken(int algo, int T, int H, int k, int I, int dtype, const void* x, const void* wgu, const void* wd) {
+  return few_supported(T, H, k, I) && (algo == BIBO_ALGO_STREAM || (algo == BIBO_ALGO_GENERIC && generic_tiles(H, I, dtype))) &&
+         aligned16(x) && aligned16(wgu) && aligned16(wd);
+}
+
 struct Workspace {
   size_t hist, idx, w, counts, offsets, perm_slot, perm_token, hidden, gu, yw;
   size_t least;        // with room for the slot rows only: what every kernel family can do with
@@ -134,8 +141,9 @@ Workspace carve(int T, int H, int E, int k, int I, int dtype) {
   ws.perm_slot = o;  o += align_up(S * sizeof(int32_t));
   ws.perm_token = o; o += align_up(S * sizeof(int32_t));
   ws.hidden = o;     o += align_up(S * (size_t)I * elt_size(dtype));
-  // bf16 gate/up pre-activations, only ever used when the streaming kernels are eligible
-  ws.gu = o;         o += align_up(stream_possible(T, H, E, k, I, dtype, true) ? S * (size_t)2 * I * sizeof(bf16_t) : 0);
+  // gate/up pre-activations of the few-token kernels (fp32) and of the streaming kernels (bf16), where they are eligible
+  ws.gu = o;         o += align_up(few_supported(T, H, k, I) ? S * (size_t)2 * I * sizeof(float)
+                                   : stream_possible(T, H, E, k, I, dtype, true) ? S * (size_t)2 * I * sizeof(bf16_t) : 0);
   ws.yw = o;
   ws.least = o + align_up(S * (size_t)H * sizeof(float));
   ws.total = o + align_up(S * (size_t)(generic_tiles(H, I, dtype) && 2 * I > H ? 2 * I : H) * sizeof(float));
@@ -186,6 +194,11 @@ int experts_dispatch(const void* x, const void* wgu, const void* wd, const float
   // indices that come straight from the router kernel are in range; a caller's may hold padding values, whose
   // slots the combine has to skip; specials are the combine's work either way (moe.py:95-99)
   if (!idx_trusted || np + nn > 0) { ca.idx = idx; ca.w = w; ca.x = x; ca.E_glu = Eg; ca.n_pos = np; ca.n_neg = nn; }
+  if (few_taken(algo, T, H, k, I, dtype, x, wgu, wd)) {
+    ca.x = x; ca.n_pos = np; ca.n_neg = nn;
+    return hip_rc(launch_experts_few(x, wgu, wd, theta, idx, w, ca, T, H, Eg, k, I, dtype, act, reinterpret_cast<float*>(base + ws.gu),
+                                     out, s));
+  }
   if (algo == BIBO_ALGO_STREAM) {
     if (!aligned16(x) || !aligned16(wgu) || !aligned16(wd)) return BIBO_ERR_MISALIGNED;
     if (!stream_possible(T, H, Eg + np + nn, k, I, dtype, idx_trusted)) return BIBO_ERR_UNSUPPORTED;   // no pre-activation segment carved, or more rows than a row list holds
@@ -277,8 +290,9 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
     perm_token = reinterpret_cast<int32_t*>(state + st.perm_token);
     preact = state + st.gu;
   }
-  // the streaming kernels find their rows themselves; the permutation then only serves the counts
-  const bool need_permute = a != BIBO_ALGO_STREAM || counts_out != nullptr || T == 0;
+  // the streaming and few-token kernels find their rows themselves; the permutation then only serves the counts
+  const bool need_permute = (a != BIBO_ALGO_STREAM && !few_taken(a, T, H, k, I, dtype, x, w_gate_up, w_down)) ||
+                            counts_out != nullptr || T == 0;
   // the router kernel can leave per-workgroup histograms of its selections, which save the permutation its
   // histogram launch and its counting pass
   int32_t* hist = reinterpret_cast<int32_t*>(base + ws.hist);
@@ -601,8 +615,9 @@ int bibo_moe_experts_fwd(const void* x, const int32_t* idx, const float* w, cons
   int32_t* offsets = reinterpret_cast<int32_t*>(base + ws.offsets);
   int32_t* perm_slot = reinterpret_cast<int32_t*>(base + ws.perm_slot);
   int32_t* perm_token = reinterpret_cast<int32_t*>(base + ws.perm_token);
-  // the streaming kernels find their rows themselves; the permutation then only serves the counts
-  const bool need_permute = a != BIBO_ALGO_STREAM || counts_out != nullptr || T == 0;
+  // the streaming and few-token kernels find their rows themselves; the permutation then only serves the counts
+  const bool need_permute = (a != BIBO_ALGO_STREAM && !few_taken(a, T, H, k, I, dtype, x, w_gate_up, w_down)) ||
+                            counts_out != nullptr || T == 0;
   if (need_permute &&
       (rc = hip_rc(launch_permute(idx, T, E, k, counts, offsets, perm_slot, perm_token, base + ws.hist, s))) != BIBO_OK)
     return rc;

@@ -19,6 +19,7 @@ constexpr float kSumNormEps = 1e-20f;   // src/modeling/ffn/router.py:45
 // tokens handled by one workgroup of the histogram / permutation kernels
 constexpr int kPermTokens = 128;   // tokens per permutation workgroup (256 and 64 measured slower)
 constexpr int kStreamMaxSlots = 4096;   // routed slots the weight-streaming kernels can scan per workgroup
+constexpr int kFewSlots = 48;           // routed slots up to which the few-token kernels run
 constexpr int kStreamMaxRows = 2048;    // rows (= tokens) one expert can get in them
 
 typedef __bf16 bf16_t;
@@ -184,6 +185,7 @@ hipError_t launch_down_generic(const void* hidden, const void* wd, const float* 
                                const int32_t* perm_slot, int T, int H, int E, int k, int I, int dtype, float* yw,
                                hipStream_t s);
 bool tile_f32_supported(int H, int I);
+bool few_supported(int T, int H, int k, int I);
 hipError_t launch_experts_tiled(const void* x, const void* wgu, const void* wd, const float* theta, const float* w,
                                 const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int T, int H,
                                 int E, int k, int I, int dtype, int act, float* gu, void* hidden, float* yw, hipStream_t s);
@@ -196,6 +198,9 @@ struct CombineArgs {
   const void* residual = nullptr;  // [T,H] in the output dtype
   int round_block = 0;             // round the sum of the slot rows to the output dtype before the residual is added
 };
+hipError_t launch_experts_few(const void* x, const void* wgu, const void* wd, const float* theta, const int32_t* idx, const float* w,
+                              const CombineArgs& a, int T, int H, int E, int k, int I, int dtype, int act, float* gu, void* out,
+                              hipStream_t s);
 hipError_t launch_combine(const void* yw, int yw_is_bf16, const CombineArgs& a, int T, int H, int k, int dtype,
                           void* out, hipStream_t s);
 hipError_t launch_rmsnorm(const void* x, const float* weight, float eps, int T, int H, int dtype, void* out,

@@ -1,0 +1,215 @@
+// The layer for a handful of tokens (single-stream decoding), bf16 or fp32: two launches behind the router, no permutation.
+//
+// With a few routed slots the weight-streaming kernels are all latency: one workgroup per 64 weight rows leaves most CUs
+// idle (72 workgroups for one token's six experts), each pulls 98 KB through one CU, and the slot rows cross memory to a
+// combine launch.  Here a workgroup takes 32 rows of ONE slot's expert (or 8 output columns of one token) with all of its
+// loads in flight at once, so a launch is one round trip of an index and one of the weights.  Slots that share an expert read its
+// weights again (from L2), which is why the range ends at kFewSlots.
+//   gateup_few_kernel: gu[slot] = W_gate_up[e] x_t, fp32                              (src/modeling/ffn/moe.py:84)
+//   down_few_kernel:   out[t] = round(residual + sum_j w_j W_down[e_j] h_j), h = r^p SiLU(g/r) u recomputed by every workgroup,
+//                      one wave per slot of the token; +/-Identity slots add +/- w x   (moe.py:87-101)
+// Plain FMAs: a matrix instruction would use one of its sixteen columns.  Sixteen lanes share a weight row, 16 bytes (fp32:
+// 32) each at a time, i.e. whole 256-byte pieces of a row per request.
+#include "tile_f32.h"
+
+namespace bibo {
+namespace {
+
+__device__ __forceinline__ void load8(float (&v)[8], const float* p) {
+  const floatx4 a = *reinterpret_cast<const floatx4*>(p), b = *reinterpret_cast<const floatx4*>(p + 4);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) { v[q] = a[q]; v[4 + q] = b[q]; }
+}
+
+// eight weights as they come from memory
+template <typename T> struct Raw8;
+template <> struct Raw8<bf16_t> {
+  bf16x8 v;
+  __device__ __forceinline__ void load(const bf16_t* p) { v = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p)); }
+  __device__ __forceinline__ void zero() {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = (bf16_t)0.f;
+  }
+  __device__ __forceinline__ float get(int q) const { return (float)v[q]; }
+};
+template <> struct Raw8<float> {
+  floatx4 a, b;
+  __device__ __forceinline__ void load(const float* p) {
+    a = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(p));
+    b = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(p + 4));
+  }
+  __device__ __forceinline__ void zero() { a = b = floatx4{0.f, 0.f, 0.f, 0.f}; }
+  __device__ __forceinline__ float get(int q) const { return q < 4 ? a[q] : b[q - 4]; }
+};
+
+__device__ __forceinline__ float sum16(float v) {          // over the 16 lanes of a DPP row, the same in every lane
+  auto dpp = [](float x, auto ctrl) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, false));
+  };
+  v += dpp(v, std::integral_constant<int, 0xB1>{});
+  v += dpp(v, std::integral_constant<int, 0x4E>{});
+  v += dpp(v, std::integral_constant<int, 0x141>{});
+  return v + dpp(v, std::integral_constant<int, 0x140>{});
+}
+
+constexpr int kGateRows = 32;           // weight rows per workgroup of the gate/up kernel: two per 16 lanes
+
+// grid (ceil(2I / 32), S).  NG = ceil(H / 128): 8-element granules of a row per lane.
+template <typename T, int NG>
+__global__ __launch_bounds__(256) void gateup_few_kernel(const T* __restrict__ x, const T* __restrict__ wgu,
+                                                         const int32_t* __restrict__ idx, int k, int H, int I2, int E,
+                                                         float* __restrict__ gu) {
+  const int slot = blockIdx.y, c = threadIdx.x & 15, rg = threadIdx.x >> 4;
+  const int e = idx[slot];
+  Raw8<T> xv[NG], wv[2][NG];
+  const T* xr = x + (size_t)(slot / k) * H;
+#pragma unroll
+  for (int u = 0; u < NG; ++u) {
+    const int g = (u * 16 + c) * 8;
+    if (g < H) xv[u].load(xr + g); else xv[u].zero();
+  }
+  if ((unsigned)e >= (unsigned)E) return;                      // no GLU expert
+  const int row0 = blockIdx.x * kGateRows + rg;
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const T* wr = wgu + ((size_t)e * I2 + min(row0 + 16 * r, I2 - 1)) * H;
+#pragma unroll
+    for (int u = 0; u < NG; ++u) {
+      const int g = (u * 16 + c) * 8;
+      if (g < H) wv[r][u].load(wr + g); else wv[r][u].zero();
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    float acc = 0.f;
+#pragma unroll
+    for (int u = 0; u < NG; ++u)
+#pragma unroll
+      for (int q = 0; q < 8; ++q) acc = fmaf(wv[r][u].get(q), xv[u].get(q), acc);
+    acc = sum16(acc);
+    if (c == 0 && row0 + 16 * r < I2) gu[(size_t)slot * I2 + row0 + 16 * r] = acc;
+  }
+}
+
+// grid (H / CH, T), 64 k threads: wave j = slot j of the token.  NG = ceil(I / 128).
+template <typename T, int NG, int CH>
+__global__ __launch_bounds__(64 * kMaxK) void down_few_kernel(const float* __restrict__ gu, const T* __restrict__ wd,
+                                                              const float* __restrict__ theta, const float* __restrict__ w,
+                                                              const int32_t* __restrict__ idx, CombineArgs a, int k, int H, int E,
+                                                              int I, int act, T* __restrict__ out) {
+  __shared__ float part[kMaxK][CH];
+  const int t = blockIdx.y, c0 = blockIdx.x * CH;
+  const int j = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int c = lane & 15, rg = lane >> 4;
+  const int slot = t * k + j, e = idx[slot];
+  const float ws = w[slot];
+  if (e >= 0 && e < E) {
+    const float p = radial_exponent(theta, e, act);
+    constexpr int kIt = CH / 4;
+    Raw8<T> wv[kIt][NG];
+#pragma unroll
+    for (int it = 0; it < kIt; ++it) {
+      const T* wr = wd + ((size_t)e * H + c0 + it * 4 + rg) * I;
+#pragma unroll
+      for (int u = 0; u < NG; ++u) {
+        const int g = (u * 16 + c) * 8;
+        if (g < I) wv[it][u].load(wr + g); else wv[it][u].zero();
+      }
+    }
+    float gv[NG][8], h[NG][8];                                 // gate, then up -> h
+    const float* gr = gu + (size_t)slot * 2 * I;
+    float ss = 0.f;
+#pragma unroll
+    for (int u = 0; u < NG; ++u) {
+      const int g = (u * 16 + c) * 8;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) gv[u][q] = h[u][q] = 0.f;
+      if (g < I) {
+        load8(gv[u], gr + g);
+        load8(h[u], gr + I + g);
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) ss = fmaf(gv[u][q], gv[u][q], ss);
+    }
+    ss = sum16(ss);
+    float rinv, gain;                                                                              // 1/r, r^p (moe.py:88-89)
+    radial_row_scalars(ss, I, p, act, rinv, gain);
+    const float nrl = -1.4426950408889634f * rinv, rgn = rinv * gain;
+#pragma unroll
+    for (int u = 0; u < NG; ++u)
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const float sig = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(gv[u][q] * nrl));
+        h[u][q] *= gv[u][q] * rgn * sig;                                                            // SiLU(g/r) r^p up
+      }
+#pragma unroll
+    for (int it = 0; it < kIt; ++it) {
+      float acc = 0.f;
+#pragma unroll
+      for (int u = 0; u < NG; ++u)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) acc = fmaf(wv[it][u].get(q), h[u][q], acc);
+      acc = sum16(acc);
+      if (c == 0) part[j][it * 4 + rg] = ws * acc;                                                 // moe.py:93
+    }
+  } else if (lane < CH) {                                      // +/-Identity (moe.py:95-99), or no expert at all
+    float v = 0.f;
+    if (e >= E && e < E + a.n_pos + a.n_neg) {
+      const float xv = to_float(static_cast<const T*>(a.x)[(size_t)t * H + c0 + lane]);
+      v = e < E + a.n_pos ? ws * xv : -ws * xv;
+    }
+    part[j][lane] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x < CH) {
+    const size_t o = (size_t)t * H + c0 + threadIdx.x;
+    float acc = 0.f;
+    for (int i = 0; i < k; ++i) acc += part[i][threadIdx.x];
+    if (a.residual != nullptr)
+      acc = (a.round_block ? to_float(from_float<T>(acc)) : acc) + to_float(static_cast<const T*>(a.residual)[o]);
+    out[o] = from_float<T>(acc);
+  }
+}
+
+template <typename T>
+hipError_t launch_t(const T* x, const T* wgu, const T* wd, const float* theta, const int32_t* idx, const float* w,
+                    const CombineArgs& a, int Tn, int H, int E, int k, int I, int act, float* gu, T* out, hipStream_t s) {
+  auto gateup = [&](auto ng) {
+    hipLaunchKernelGGL((gateup_few_kernel<T, decltype(ng)::value>), dim3((2 * I + kGateRows - 1) / kGateRows, Tn * k), dim3(256), 0, s, x,
+                       wgu, idx, k, H, 2 * I, E, gu);
+  };
+  using std::integral_constant;
+  const int nh = (H + 127) / 128;
+  if (nh <= 2) gateup(integral_constant<int, 2>{});
+  else if (nh <= 4) gateup(integral_constant<int, 4>{});
+  else if (nh <= 6) gateup(integral_constant<int, 6>{});
+  else gateup(integral_constant<int, 8>{});
+  auto down = [&](auto ng) {
+    hipLaunchKernelGGL((down_few_kernel<T, decltype(ng)::value, 8>), dim3(H / 8, Tn), dim3(64 * k), 0, s, gu, wd, theta, w, idx, a, k, H,
+                       E, I, act, out);
+  };
+  const int ni = (I + 127) / 128;
+  if (ni <= 1) down(integral_constant<int, 1>{});
+  else if (ni == 2) down(integral_constant<int, 2>{});
+  else if (ni == 3) down(integral_constant<int, 3>{});
+  else down(integral_constant<int, 4>{});
+  return hipGetLastError();
+}
+
+}  // namespace
+
+bool few_supported(int T, int H, int k, int I) {
+  return T >= 1 && T * k <= kFewSlots && H % 8 == 0 && I % 8 == 0 && H <= 1024 && I <= 512;
+}
+
+hipError_t launch_experts_few(const void* x, const void* wgu, const void* wd, const float* theta, const int32_t* idx, const float* w,
+                              const CombineArgs& a, int T, int H, int E, int k, int I, int dtype, int act, float* gu, void* out,
+                              hipStream_t s) {
+  if (dtype == BIBO_DTYPE_BF16)
+    return launch_t(static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(wgu), static_cast<const bf16_t*>(wd), theta, idx, w, a, T,
+                    H, E, k, I, act, gu, static_cast<bf16_t*>(out), s);
+  return launch_t(static_cast<const float*>(x), static_cast<const float*>(wgu), static_cast<const float*>(wd), theta, idx, w, a, T, H, E,
+                  k, I, act, gu, static_cast<float*>(out), s);
+}
+
+}  // namespace bibo

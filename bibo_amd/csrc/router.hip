@@ -141,12 +141,13 @@ __device__ __forceinline__ void write_chunk_hist(unsigned long long mask, int32_
 
 // ---- generic router: any H, bf16 or fp32 inputs, plain FMA -------------------------------------
 // One workgroup = 16 tokens x 64 experts; thread = 2 tokens x 2 experts.  K chunks of 64 elements pass through LDS (the next
-// one waits in registers meanwhile).  A logit is one chain of FMAs over ascending h, so it does not depend on the tiling.
+// three are on their way to registers meanwhile: with a few tokens the kernel is one workgroup and its loads' latency).  A logit is one chain of FMAs over ascending h, so it does not depend on the tiling.
 // Bound by its LDS reads, four 16-byte ones per sixteen FMAs; with 16 tokens per workgroup even a few hundred tokens
 // reach many CUs (64 tokens per workgroup and operands straight from memory: 940 us at T = 2048, H = 768 in fp32).
 // VEC: rows are 16-byte (bf16: 8-byte) aligned and H % 4 == 0.
 constexpr int kGenTokens = 16;
 constexpr int kGenKC = 64;
+constexpr int kGenAhead = 3;
 
 template <typename TIn, bool VEC>
 __global__ __launch_bounds__(256) void router_fma_kernel(const TIn* __restrict__ x, const TIn* __restrict__ wr,
@@ -172,29 +173,30 @@ __global__ __launch_bounds__(256) void router_fma_kernel(const TIn* __restrict__
     live[i] = i == 0 || e < E;
     src[i] = i == 0 ? x + (size_t)min(t0 + fr, T - 1) * H : wr + (size_t)min(e, E - 1) * H;
   }
-  floatx4 r[5];
-  auto load = [&](int h0) {
+  floatx4 r[kGenAhead][5];
+  auto load = [&](auto set, int h0) {
+    constexpr int st = decltype(set)::value;
 #pragma unroll
     for (int i = 0; i < 5; ++i) {
-      r[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+      r[st][i] = floatx4{0.f, 0.f, 0.f, 0.f};
       if constexpr (VEC) {
-        if (live[i] && h0 + fc < H) r[i] = load4<TIn>(src[i] + h0 + fc);
+        if (live[i] && h0 + fc < H) r[st][i] = load4<TIn>(src[i] + h0 + fc);
       } else {
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          if (live[i] && h0 + fc + q < H) r[i][q] = to_float(src[i][h0 + fc + q]);
+          if (live[i] && h0 + fc + q < H) r[st][i][q] = to_float(src[i][h0 + fc + q]);
       }
     }
   };
   const int e5 = tid & 31, tp = tid >> 5;                      // experts e5, e5 + 32; tokens tp, tp + 8
   float acc[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
-  load(0);
-  for (int h0 = 0; h0 < H; h0 += kGenKC) {
-    *reinterpret_cast<floatx4*>(xs + fr * kStride + fc) = r[0];
+  auto chunk = [&](auto set, int h0) {
+    constexpr int st = decltype(set)::value;
+    *reinterpret_cast<floatx4*>(xs + fr * kStride + fc) = r[st][0];
 #pragma unroll
-    for (int i = 1; i < 5; ++i) *reinterpret_cast<floatx4*>(ws + (fr + 16 * (i - 1)) * kStride + fc) = r[i];
+    for (int i = 1; i < 5; ++i) *reinterpret_cast<floatx4*>(ws + (fr + 16 * (i - 1)) * kStride + fc) = r[st][i];
     __syncthreads();
-    if (h0 + kGenKC < H) load(h0 + kGenKC);
+    if (h0 + kGenAhead * kGenKC < H) load(set, h0 + kGenAhead * kGenKC);
 #pragma unroll
     for (int h = 0; h < kGenKC; h += 4) {
       floatx4 xv[2], wv[2];
@@ -211,6 +213,15 @@ __global__ __launch_bounds__(256) void router_fma_kernel(const TIn* __restrict__
           for (int b = 0; b < 2; ++b) acc[a][b] = fmaf(xv[a][q], wv[b][q], acc[a][b]);
     }
     __syncthreads();
+  };
+  using std::integral_constant;
+  load(integral_constant<int, 0>{}, 0);
+  load(integral_constant<int, 1>{}, kGenKC);
+  load(integral_constant<int, 2>{}, 2 * kGenKC);
+  for (int h0 = 0; h0 < H; h0 += kGenAhead * kGenKC) {
+    chunk(integral_constant<int, 0>{}, h0);
+    if (h0 + kGenKC < H) chunk(integral_constant<int, 1>{}, h0 + kGenKC);
+    if (h0 + 2 * kGenKC < H) chunk(integral_constant<int, 2>{}, h0 + 2 * kGenKC);
   }
   const int ntok = min(kGenTokens, T - t0);
 #pragma unroll
