@@ -139,106 +139,6 @@ __device__ __forceinline__ void write_chunk_hist(unsigned long long mask, int32_
   }
 }
 
-// ---- generic router: any H, bf16 or fp32 inputs, plain FMA -------------------------------------
-// One workgroup = 16 tokens x 64 experts; thread = 2 tokens x 2 experts.  K chunks of 64 elements pass through LDS (the next
-// three are on their way to registers meanwhile: with a few tokens the kernel is one workgroup and its loads' latency).  A logit is one chain of FMAs over ascending h, so it does not depend on the tiling.
-// Bound by its LDS reads, four 16-byte ones per sixteen FMAs; with 16 tokens per workgroup even a few hundred tokens
-// reach many CUs (64 tokens per workgroup and operands straight from memory: 940 us at T = 2048, H = 768 in fp32).
-// VEC: rows are 16-byte (bf16: 8-byte) aligned and H % 4 == 0.
-constexpr int kGenTokens = 16;
-constexpr int kGenKC = 64;
-constexpr int kGenAhead = 3;
-
-template <typename TIn, bool VEC>
-__global__ __launch_bounds__(256) void router_fma_kernel(const TIn* __restrict__ x, const TIn* __restrict__ wr,
-                                                         const float* __restrict__ bias, int T, int H, int E, int k,
-                                                         int norm_mode, float* __restrict__ logits, int32_t* __restrict__ idx,
-                                                         float* __restrict__ w, float* __restrict__ gap,
-                                                         int32_t* __restrict__ chunk_hist) {
-  constexpr int kStride = kGenKC + 4;                          // floats: 16 rows of a 16-byte read hit distinct banks
-  __shared__ __attribute__((aligned(16))) float xs[kGenTokens * kStride];
-  __shared__ __attribute__((aligned(16))) float ws[kMaxE * kStride];
-  __shared__ float sc[kGenTokens * kRowPad];
-  __shared__ float bias_s[kMaxE];
-  const int tid = threadIdx.x;
-  const int t0 = blockIdx.x * kGenTokens;
-  if (tid < kMaxE) bias_s[tid] = (tid < E) ? bias[tid] : 0.f;
-  // fill side: thread = granule tid % 16 (four elements) of rows tid / 16 + 16 i; row group 0 = the tokens, 1 .. 4 = w_router
-  const int fr = tid >> 4, fc = (tid & 15) * 4;
-  const TIn* src[5];
-  bool live[5];
-#pragma unroll
-  for (int i = 0; i < 5; ++i) {
-    const int e = fr + 16 * (i - 1);
-    live[i] = i == 0 || e < E;
-    src[i] = i == 0 ? x + (size_t)min(t0 + fr, T - 1) * H : wr + (size_t)min(e, E - 1) * H;
-  }
-  floatx4 r[kGenAhead][5];
-  auto load = [&](auto set, int h0) {
-    constexpr int st = decltype(set)::value;
-#pragma unroll
-    for (int i = 0; i < 5; ++i) {
-      r[st][i] = floatx4{0.f, 0.f, 0.f, 0.f};
-      if constexpr (VEC) {
-        if (live[i] && h0 + fc < H) r[st][i] = load4<TIn>(src[i] + h0 + fc);
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          if (live[i] && h0 + fc + q < H) r[st][i][q] = to_float(src[i][h0 + fc + q]);
-      }
-    }
-  };
-  const int e5 = tid & 31, tp = tid >> 5;                      // experts e5, e5 + 32; tokens tp, tp + 8
-  float acc[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
-  auto chunk = [&](auto set, int h0) {
-    constexpr int st = decltype(set)::value;
-    *reinterpret_cast<floatx4*>(xs + fr * kStride + fc) = r[st][0];
-#pragma unroll
-    for (int i = 1; i < 5; ++i) *reinterpret_cast<floatx4*>(ws + (fr + 16 * (i - 1)) * kStride + fc) = r[st][i];
-    __syncthreads();
-    if (h0 + kGenAhead * kGenKC < H) load(set, h0 + kGenAhead * kGenKC);
-#pragma unroll
-    for (int h = 0; h < kGenKC; h += 4) {
-      floatx4 xv[2], wv[2];
-#pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        xv[a] = *reinterpret_cast<const floatx4*>(xs + (tp + 8 * a) * kStride + h);
-        wv[a] = *reinterpret_cast<const floatx4*>(ws + (e5 + 32 * a) * kStride + h);
-      }
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-          for (int b = 0; b < 2; ++b) acc[a][b] = fmaf(xv[a][q], wv[b][q], acc[a][b]);
-    }
-    __syncthreads();
-  };
-  using std::integral_constant;
-  load(integral_constant<int, 0>{}, 0);
-  load(integral_constant<int, 1>{}, kGenKC);
-  load(integral_constant<int, 2>{}, 2 * kGenKC);
-  for (int h0 = 0; h0 < H; h0 += kGenAhead * kGenKC) {
-    chunk(integral_constant<int, 0>{}, h0);
-    if (h0 + kGenKC < H) chunk(integral_constant<int, 1>{}, h0 + kGenKC);
-    if (h0 + 2 * kGenKC < H) chunk(integral_constant<int, 2>{}, h0 + 2 * kGenKC);
-  }
-  const int ntok = min(kGenTokens, T - t0);
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const int tl = tp + 8 * a, e = e5 + 32 * b;
-      if (tl < ntok && e < E) {
-        if (logits != nullptr) logits[(size_t)(t0 + tl) * E + e] = acc[a][b];
-        sc[tl * kRowPad + e] = sigmoid32_canonical(acc[a][b]);   // router.py:31
-      }
-    }
-  __syncthreads();
-  const unsigned long long mask = select_tokens16(sc, bias_s, E, k, norm_mode, t0, ntok, idx, w, gap);
-  if (chunk_hist != nullptr) write_chunk_hist<kGenTokens>(mask, chunk_hist);
-}
-
 // ---- MFMA router: bf16, H % 128 == 0 ------------------------------------------------------------
 // One workgroup = TOK tokens (16 or 32), TOK/16 x 4 waves: wave (tm, en) owns the 16x16 logits tile of
 // token tile tm and expert tile en over the whole K, so no partial sums cross waves and the fp32
@@ -277,6 +177,82 @@ __device__ __forceinline__ void router_finish(const floatx4& acc, float* sc, con
   __syncthreads();
   const unsigned long long mask = select_tokens16(sc, bias_s, E, k, norm_mode, t0, ntok, idx, w, gap);
   if (chunk_hist != nullptr) write_chunk_hist<TOK>(mask, chunk_hist);
+}
+
+// ---- generic router: any H, bf16 or fp32 inputs, fp32 arithmetic ---------------------------------
+// One workgroup = 16 tokens x 64 experts, wave en = expert tile en.  K chunks of 64 elements, widened to fp32, pass through
+// LDS; the next three are on their way to registers meanwhile (with a few tokens the kernel is one workgroup and its loads'
+// latency).  v_mfma_f32_16x16x4_f32 with k ascending: one logit is one chain of FMAs over ascending h, bit for bit (checked
+// against scalar FMAs, which took 16 us for H = 768 at one wave per SIMD where the MFMA chain takes 2.6).
+// VEC: rows are 16-byte (bf16: 8-byte) aligned and H % 4 == 0.
+constexpr int kGenTokens = 16;
+constexpr int kGenKC = 64;
+constexpr int kGenAhead = 3;
+
+template <typename TIn, bool VEC>
+__global__ __launch_bounds__(256) void router_f32_kernel(const TIn* __restrict__ x, const TIn* __restrict__ wr,
+                                                         const float* __restrict__ bias, int T, int H, int E, int k,
+                                                         int norm_mode, float* __restrict__ logits, int32_t* __restrict__ idx,
+                                                         float* __restrict__ w, float* __restrict__ gap,
+                                                         int32_t* __restrict__ chunk_hist) {
+  constexpr int kStride = kGenKC + 4;                          // floats: 16 rows of a 16-byte read hit distinct banks
+  __shared__ __attribute__((aligned(16))) float xs[kGenTokens * kStride];
+  __shared__ __attribute__((aligned(16))) float ws[kMaxE * kStride];
+  __shared__ float sc[kGenTokens * kRowPad];
+  __shared__ float bias_s[kMaxE];
+  const int tid = threadIdx.x;
+  const int t0 = blockIdx.x * kGenTokens;
+  if (tid < kMaxE) bias_s[tid] = (tid < E) ? bias[tid] : 0.f;
+  // fill side: thread = granule tid % 16 (four elements) of rows tid / 16 + 16 i; row group 0 = the tokens, 1 .. 4 = w_router
+  const int fr = tid >> 4, fc = (tid & 15) * 4;
+  const TIn* src[5];
+  bool live[5];
+#pragma unroll
+  for (int i = 0; i < 5; ++i) {
+    const int e = fr + 16 * (i - 1);
+    live[i] = i == 0 || e < E;
+    src[i] = i == 0 ? x + (size_t)min(t0 + fr, T - 1) * H : wr + (size_t)min(e, E - 1) * H;
+  }
+  floatx4 r[kGenAhead][5];
+  auto load = [&](auto set, int h0) {
+    constexpr int st = decltype(set)::value;
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+      r[st][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (VEC) {
+        if (live[i] && h0 + fc < H) r[st][i] = load4<TIn>(src[i] + h0 + fc);
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (live[i] && h0 + fc + q < H) r[st][i][q] = to_float(src[i][h0 + fc + q]);
+      }
+    }
+  };
+  const int lane = tid & 63, r16 = lane & 15, g4 = lane >> 4;
+  const float* xrow = xs + r16 * kStride + g4;                 // A: token r16, k = 4 m + g4
+  const float* wrow = ws + ((tid >> 6) * 16 + r16) * kStride + g4;
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+  auto chunk = [&](auto set, int h0) {
+    constexpr int st = decltype(set)::value;
+    *reinterpret_cast<floatx4*>(xs + fr * kStride + fc) = r[st][0];
+#pragma unroll
+    for (int i = 1; i < 5; ++i) *reinterpret_cast<floatx4*>(ws + (fr + 16 * (i - 1)) * kStride + fc) = r[st][i];
+    __syncthreads();
+    if (h0 + kGenAhead * kGenKC < H) load(set, h0 + kGenAhead * kGenKC);
+#pragma unroll
+    for (int m = 0; m < kGenKC; m += 4) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xrow[m], wrow[m], acc, 0, 0, 0);
+    __syncthreads();
+  };
+  using std::integral_constant;
+  load(integral_constant<int, 0>{}, 0);
+  load(integral_constant<int, 1>{}, kGenKC);
+  load(integral_constant<int, 2>{}, 2 * kGenKC);
+  for (int h0 = 0; h0 < H; h0 += kGenAhead * kGenKC) {
+    chunk(integral_constant<int, 0>{}, h0);
+    if (h0 + kGenKC < H) chunk(integral_constant<int, 1>{}, h0 + kGenKC);
+    if (h0 + 2 * kGenKC < H) chunk(integral_constant<int, 2>{}, h0 + 2 * kGenKC);
+  }
+  router_finish<kGenTokens>(acc, sc, bias_s, T, E, k, norm_mode, t0, logits, idx, w, gap, chunk_hist);
 }
 
 template <int TOK>
@@ -605,10 +581,10 @@ hipError_t launch_router(const void* x, const void* w_router, const float* bias,
     };
     if (dtype == BIBO_DTYPE_BF16) {
       const bf16_t* xp = static_cast<const bf16_t*>(x);
-      if (vec) launch(router_fma_kernel<bf16_t, true>, xp); else launch(router_fma_kernel<bf16_t, false>, xp);
+      if (vec) launch(router_f32_kernel<bf16_t, true>, xp); else launch(router_f32_kernel<bf16_t, false>, xp);
     } else {
       const float* xp = static_cast<const float*>(x);
-      if (vec) launch(router_fma_kernel<float, true>, xp); else launch(router_fma_kernel<float, false>, xp);
+      if (vec) launch(router_f32_kernel<float, true>, xp); else launch(router_f32_kernel<float, false>, xp);
     }
     if (hist_tokens != nullptr && chunk_hist != nullptr) *hist_tokens = kGenTokens;
   }
