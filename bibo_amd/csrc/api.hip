@@ -78,6 +78,15 @@ inline bool stream_eligible(int T, int H, int E, int k, int I, int dtype, bool d
   return stream_possible(T, H, E, k, I, dtype, distinct) && (long long)T * k <= stream_rows_per_expert(H, I, dtype) * E;
 }
 
+// What `auto` runs in a composite call where it resolves to the MFMA family and the fused kernel takes I = 512 on shorter
+// tiles: H = 1024, I = 512, T = 3001, k = 8 in one launch instead of two.  An explicit request for the family runs its two kernels,
+// whose results the stage calls repeat bit for bit.
+constexpr int kAlgoFusedWide = 100;
+inline int composite_algo(int asked, int resolved, int T, int H, int I, int dtype) {
+  return asked == BIBO_ALGO_AUTO && resolved == BIBO_ALGO_MFMA && fused_wide_supported(H, I, dtype) && fused_fits(T, H) ? kAlgoFusedWide
+                                                                                                                       : resolved;
+}
+
 // `composite`: the caller is bibo_moe_experts_fwd / bibo_moe_forward, the only entry points that can run
 // the streaming kernels (they hand bf16 pre-activations, not `hidden`, from one kernel to the next) and
 // the fused kernel (its activations never reach memory).
@@ -209,7 +218,7 @@ int experts_dispatch(const void* x, const void* wgu, const void* wd, const float
     if (e != hipSuccess) return (int)e;
     return hip_rc(launch_combine(yw, 0, ca, T, H, k, dtype, out, s));
   }
-  if (algo == BIBO_ALGO_FUSED) {
+  if (algo == BIBO_ALGO_FUSED || algo == kAlgoFusedWide) {
     if (!aligned16(x) || !aligned16(wgu) || !aligned16(wd)) return BIBO_ERR_MISALIGNED;
     hipError_t e = launch_experts_fused(x, wgu, wd, theta, w, offsets, perm_slot, perm_token, T, H, Eg, k, I, act, yw, preact, s);
     if (e != hipSuccess) return (int)e;
@@ -265,6 +274,7 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
   if (norm_mode < BIBO_NORM_NONE || norm_mode > BIBO_NORM_SOFTMAX || !act_ok(sh->act)) return BIBO_ERR_UNSUPPORTED;
   int a;
   if ((rc = resolve_algo(algo, T, H, E, k, I, dtype, true, true, &a)) != BIBO_OK) return rc;
+  a = composite_algo(algo, a, T, H, I, dtype);
   if (!workspace) return BIBO_ERR_NULL_POINTER;
   if (!aligned_ws(workspace)) return BIBO_ERR_MISALIGNED;
   if (T > 0 && (!x || !w_router || !bias || !w_gate_up || !w_down || !out)) return BIBO_ERR_NULL_POINTER;
@@ -603,6 +613,7 @@ int bibo_moe_experts_fwd(const void* x, const int32_t* idx, const float* w, cons
   int a;
   // a caller's indices may repeat an expert inside a token (moe.py:46-71 accepts that)
   if ((rc = resolve_algo(algo, T, H, E, k, I, dtype, true, false, &a)) != BIBO_OK) return rc;
+  a = composite_algo(algo, a, T, H, I, dtype);
   if (!workspace) return BIBO_ERR_NULL_POINTER;
   if (!aligned_ws(workspace)) return BIBO_ERR_MISALIGNED;
   if (T > 0 && (!x || !idx || !w || !w_gate_up || !w_down || !out)) return BIBO_ERR_NULL_POINTER;

@@ -556,7 +556,7 @@ hipError_t launch_backward(const void* x, const void* d_out, const void* w_route
   // pass's fused kernel where it takes the shape (its ring of weight stages is the faster main loop)
   if (gu_saved != nullptr)
     err = hipSuccess;
-  else if (fused_supported(H, I, BIBO_DTYPE_BF16) && (long long)T * H < (1LL << 31))
+  else if ((fused_supported(H, I, BIBO_DTYPE_BF16) || fused_wide_supported(H, I, BIBO_DTYPE_BF16)) && (long long)T * H < (1LL << 31))
     err = launch_gateup_raw(xp, wgup, offsets, perm_token, T, H, E, k, I, b.gu, s);
   else
     err = launch_ggemm<true, false>(xp, perm_token, wgup, offsets, nullptr, S, H, 2 * I, E, static_cast<bf16_t*>(b.gu), s);

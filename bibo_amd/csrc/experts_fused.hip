@@ -38,15 +38,17 @@
 namespace bibo {
 namespace {
 
-template <int NT, int CT>
+template <int NT, int CT, int MT_ = 2>
 struct FusedShape {
-  static constexpr int MT = 2, BM = 128, BK = 64;
+  static constexpr int MT = MT_, BM = 64 * MT, BK = 64;
   static constexpr int I = 128 * NT;
   static constexpr int BN2 = 128 * CT;                             // output columns per block: 8 waves x CT x 16
   // I = 384: the three stages are the three sub-steps of a K step and the x rows alternate between two buffers.
   // I < 384 with at most 256 output columns per block (kDeep): three stages all the same, walked round by the running
   // sub-step, and a third x buffer, so that x rows are requested two K steps ahead.  Otherwise two stages.
-  static constexpr bool kDeep = NT < 3 && CT < 3;
+  // I = 512 (NT = 4) takes 64-row tiles (MT = 1): a row's 1024 accumulator columns leave registers for no more.  Its four
+  // sub-steps per K step walk the ring by the running sub-step too.
+  static constexpr bool kDeep = (NT < 3 && CT < 3) || NT == 4;
   static constexpr int kRing = (NT == 3 || kDeep) ? 3 : 2;         // weight stages in LDS
   static constexpr int kDist = kRing - 1;                          // sub-steps between a stage's request and its use
   static constexpr int kStageRows = 256;                           // 4 N waves x (gate tile + up tile) x 32 rows
@@ -56,7 +58,9 @@ struct FusedShape {
   static constexpr int kOutElems = kOutRows * BN2;
   static constexpr int kXElems = kAElems > kOutElems ? kAElems : kOutElems;   // a buffer that serves as either
   static constexpr int kBInstr = kStageRows * (BK / 8) / 512;      // load instructions per thread and weight stage
-  static_assert(kBInstr == 4 && BM * (BK / 8) == 2 * 512, "stage does not divide over the threads");
+  static constexpr int kAInstr = BM * (BK / 8) / 512;              // and per x stage
+  static_assert(kBInstr == 4 && kAInstr == MT && BM * (BK / 8) % 512 == 0, "stage does not divide over the threads");
+  static_assert(MT == 2 ? NT <= 3 : NT <= 4, "accumulators and activations of a tile");
 };
 
 // LDS-DMA through a buffer descriptor: the address is descriptor base + 32-bit per-thread byte offset (one
@@ -77,7 +81,7 @@ struct SubLoader {
   unsigned b_soff;         // byte offset of the stage's first tile row, K offset included (uniform)
   unsigned bstep;          // bytes between the rows of consecutive instructions (uniform)
   bf16_t* b_dst;           // LDS stage
-  unsigned a_voff[2];      // byte offsets of this thread's two token rows and granule
+  unsigned a_voff[F::kAInstr];   // byte offsets of this thread's token rows and granule
   unsigned a_soff;         // K offset in bytes (uniform)
   bf16_t* a_dst;           // LDS x stage
   int wave_elems;          // this wave's place in an instruction's LDS block, in elements (uniform: a scalar register,
@@ -90,11 +94,11 @@ struct SubLoader {
 template <typename F, bool WITH_A>
 struct SubIssuer {
   const SubLoader<F>& d;
-  static constexpr int kInstr = F::kBInstr + (WITH_A ? 2 : 0);
+  static constexpr int kInstr = F::kBInstr + (WITH_A ? F::kAInstr : 0);
   template <int Q>
   __device__ __forceinline__ void issue(int, bf16_t*) const {
     if constexpr (Q < F::kBInstr) dma16_buf(d.w_rsrc, d.b_voff, d.b_soff + Q * d.bstep, d.b_dst + Q * 512 * 8 + d.wave_elems);
-    else if constexpr (WITH_A && Q < F::kBInstr + 2)
+    else if constexpr (WITH_A && Q < F::kBInstr + F::kAInstr)
       dma16_buf(d.x_rsrc, d.a_voff[Q - F::kBInstr], d.a_soff, d.a_dst + (Q - F::kBInstr) * 512 * 8 + d.wave_elems);
   }
 };
@@ -133,7 +137,7 @@ __device__ __forceinline__ bf16x8 to_operand_lanes(bf16x8 v, int sel) {
 // columns), staged through the LDS stages into whole row segments.  MODE 2: the training forward - the forward pass that
 // also leaves those pre-activations for its backward, in the same way (8-byte stores straight from the accumulator
 // registers during phase 2 were slower: 140 against 133 us at T = 8192).
-template <int NT, int CT, int MODE = 0>
+template <int NT, int CT, int MODE = 0, int MTP = 2>
 __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ wgu,
                                                             const bf16_t* __restrict__ wd,
                                                             const float* __restrict__ theta,
@@ -143,7 +147,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
                                                             const int32_t* __restrict__ perm_token, int H, int E,
                                                             int act, unsigned x_bytes, bf16_t* __restrict__ yw,
                                                             bf16_t* __restrict__ preact) {
-  using F = FusedShape<NT, CT>;
+  using F = FusedShape<NT, CT, MTP>;
   constexpr int MT = F::MT, BM = F::BM, I = F::I, BK = F::BK;
   // Every buffer that is read while LDS-DMA fills another is a variable of its own: the compiler orders a DMA
   // transfer against later LDS reads of the same variable with a full wait for the transfer.
@@ -165,7 +169,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
   e = __builtin_amdgcn_readfirstlane(e);                // the same for every lane: keep them in scalar registers
   row0 = __builtin_amdgcn_readfirstlane(row0);
   rows = __builtin_amdgcn_readfirstlane(rows);
-  const int nblocks = (rows + 31) >> 5;                 // 32-row blocks that hold rows: 1 .. 4
+  const int nblocks = (rows + 31) >> 5;                 // 32-row blocks that hold rows: 1 .. 2 MT
 
   // The rest of the kernel exists once per number of blocks, chosen here, where nothing is alive yet: the copies
   // share no values, so each gets the registers the kernel would get if it were the only one.
@@ -175,13 +179,17 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
   const int wn = wave & 3, wm = wave >> 2;
   // M wave wm owns blocks 2 wm and 2 wm + 1; blocks without rows are not multiplied.  The two waves of a SIMD
   // belong to different M waves, so what a SIMD's MFMA pipe has to do goes with the tile's blocks either way.
-  static_assert(MT == 2, "two blocks per M wave");
-  const int my_blocks = __builtin_amdgcn_readfirstlane(wm == 0 ? (kBlocks < 2 ? kBlocks : 2) : (kBlocks > 2 ? kBlocks - 2 : 0));
+  const int my_blocks = __builtin_amdgcn_readfirstlane(wm == 0 ? (kBlocks < MT ? kBlocks : MT) : (kBlocks > MT ? kBlocks - MT : 0));
   const int n = lane & 31;
   const int mbase = wm * MT * 32;
   auto stage = [&](auto ic) -> bf16_t* {
     constexpr int i = decltype(ic)::value;
     if constexpr (i == 0) return S0; else if constexpr (i == 1) return S1; else return S2;
+  };
+  // slice i of the activations, columns [128 i, 128 i + 128) of all BM rows: a whole stage (BM = 128) or half of one
+  auto slice = [&](int i) -> bf16_t* {
+    if constexpr (MT == 2) return i == 0 ? S0 : (i == 1 ? S1 : S2);
+    else return (i < 2 ? S0 : S1) + (i & 1) * (BM * 128);
   };
 
   // ---- phase 1: gate/up projection (moe.py:81-86) ----
@@ -201,7 +209,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
     ld.bstep = (unsigned)NT * 32 * hb;
     ld.wave_elems = __builtin_amdgcn_readfirstlane(wave) * 64 * 8;
 #pragma unroll
-    for (int a = 0; a < 2; ++a) {
+    for (int a = 0; a < F::kAInstr; ++a) {
       const int m = min(a * 64 + drow, rows - 1);                                // rows past the end re-read the last valid row
       ld.a_voff[a] = (unsigned)perm_token[row0 + m] * hb + chunk * 16;          // gather, moe.py:81
     }
@@ -230,9 +238,9 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
 #pragma unroll
       for (int q = 0; q < F::kBInstr; ++q) dma16_buf(ld.w_rsrc, ld.b_voff, q * ld.bstep, S0 + q * 512 * 8 + ld.wave_elems);
 #pragma unroll
-      for (int a = 0; a < 2; ++a) dma16_buf(ld.x_rsrc, ld.a_voff[a], 0, A0 + a * 512 * 8 + ld.wave_elems);
+      for (int a = 0; a < F::kAInstr; ++a) dma16_buf(ld.x_rsrc, ld.a_voff[a], 0, A0 + a * 512 * 8 + ld.wave_elems);
 #pragma unroll
-      for (int a = 0; a < 2; ++a) dma16_buf(ld.x_rsrc, ld.a_voff[a], kb, A1 + a * 512 * 8 + ld.wave_elems);
+      for (int a = 0; a < F::kAInstr; ++a) dma16_buf(ld.x_rsrc, ld.a_voff[a], kb, A1 + a * 512 * 8 + ld.wave_elems);
 #pragma unroll
       for (int q = 0; q < F::kBInstr; ++q)
         dma16_buf(ld.w_rsrc, ld.b_voff, (NT == 1 ? kb : 32 * hb) + q * ld.bstep, S1 + q * 512 * 8 + ld.wave_elems);
@@ -243,7 +251,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
         constexpr int cur = (ph * NT + t) % 3, target = (ph * NT + t + 2) % 3;
         constexpr int tn = (t + 2) % NT, ds = (t + 2) / NT;
         constexpr bool after_t0 = NT == 1 || t == 1;                   // the sub-step before also requested x rows
-        sync_keep_loads<F::kBInstr + (after_t0 ? 2 : 0)>();
+        sync_keep_loads<F::kBInstr + (after_t0 ? F::kAInstr : 0)>();
         const bf16_t* a0 = abuf(integral_constant<int, ph>{}) + (mbase + n) * BK + pos0;
         const bf16_t* b0 = stage(integral_constant<int, cur>{}) + n * BK;
         ld.b_soff = (unsigned)tn * 32 * hb + (unsigned)min(s + ds, nsteps - 1) * kb;
@@ -259,6 +267,8 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
       auto kstep = [&](auto mc, auto phc, int s) {
         substep(mc, phc, integral_constant<int, 0>{}, s);
         if constexpr (NT > 1) substep(mc, phc, integral_constant<int, 1>{}, s);
+        if constexpr (NT > 2) substep(mc, phc, integral_constant<int, 2>{}, s);
+        if constexpr (NT > 3) substep(mc, phc, integral_constant<int, 3>{}, s);
       };
       auto kloop = [&](auto mc) {
         for (int s = 0; s < nsteps; s += 3) {
@@ -267,7 +277,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
           if (s + 2 < nsteps) kstep(mc, integral_constant<int, 2>{}, s + 2);
         }
       };
-      if (my_blocks == 2) kloop(integral_constant<int, 2>{});
+      if (MT == 2 && my_blocks == 2) kloop(integral_constant<int, MT>{});
       else if (my_blocks == 1) kloop(integral_constant<int, 1>{});
       else kloop(integral_constant<int, 0>{});
     } else {
@@ -287,8 +297,8 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
     // for the row indices)
 #pragma unroll
     for (int q = 0; q < F::kBInstr; ++q) dma16_buf(ld.w_rsrc, ld.b_voff, q * ld.bstep, S0 + q * 512 * 8 + ld.wave_elems);
-    dma16_buf(ld.x_rsrc, ld.a_voff[0], 0, A0 + ld.wave_elems);
-    dma16_buf(ld.x_rsrc, ld.a_voff[1], 0, A0 + 512 * 8 + ld.wave_elems);
+#pragma unroll
+    for (int a = 0; a < F::kAInstr; ++a) dma16_buf(ld.x_rsrc, ld.a_voff[a], 0, A0 + a * 512 * 8 + ld.wave_elems);
     if constexpr (F::kDist == 2) {
 #pragma unroll
       for (int q = 0; q < F::kBInstr; ++q)
@@ -301,7 +311,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
       constexpr int cur = NT == 1 ? par : t;
       // loads still allowed in flight: those of the sub-steps after the one whose stage is read now
       if constexpr (F::kDist == 1) sync_keep_loads<0>();
-      else if constexpr (t == 1) sync_keep_loads<F::kBInstr + 2>();     // the sub-step before (t = 0) also requested x rows
+      else if constexpr (t == 1) sync_keep_loads<F::kBInstr + F::kAInstr>();     // the sub-step before (t = 0) also requested x rows
       else sync_keep_loads<F::kBInstr>();
       const bf16_t* a0 = (par ? A1 : A0) + (mbase + n) * BK + pos0;
       const bf16_t* b0 = stage(std::integral_constant<int, cur>{}) + n * BK;
@@ -324,8 +334,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
         if constexpr (NT > 2) substep(mc, integral_constant<int, 2>{}, integral_constant<int, 1>{}, s + 1);
       }
     };
-    static_assert(MT == 2, "the three copies below are 2, 1 and 0 M tiles");
-    if (my_blocks == 2) kloop(integral_constant<int, 2>{});
+    if (MT == 2 && my_blocks == 2) kloop(integral_constant<int, MT>{});
     else if (my_blocks == 1) kloop(integral_constant<int, 1>{});
     else kloop(integral_constant<int, 0>{});
       }
@@ -345,7 +354,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
           const int tile32 = wn * NT + j;
-          bf16_t* hrow = ((tile32 >> 2) == 0 ? S0 : ((tile32 >> 2) == 1 ? S1 : S2)) + m * 128 + 4 * hh;
+          bf16_t* hrow = slice(tile32 >> 2) + m * 128 + 4 * hh;
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
             bf16x4 hv;
@@ -359,12 +368,12 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
       __syncthreads();
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        const bf16_t* slice = t == 0 ? S0 : (t == 1 ? S1 : S2);
+        const bf16_t* from = slice(t);
         for (int g = tid; g < BM * 16; g += 512) {
           const int m = g >> 4, pos = g & 15;
           if (m < rows)
             *reinterpret_cast<u32x4*>(preact + (size_t)(row0 + m) * (2 * I) + half * I + t * 128 + ((pos ^ (m & 15)) * 8)) =
-                *reinterpret_cast<const u32x4*>(slice + m * 128 + pos * 8);
+                *reinterpret_cast<const u32x4*>(from + m * 128 + pos * 8);
         }
       }
       __syncthreads();                     // the stages are free for the other half
@@ -422,7 +431,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
         const int tile32 = wn * NT + j;      // 32-column tile of the activation row: slice tile32 / 4, granules (tile32 % 4) * 4 + q
-        bf16_t* hrow = ((tile32 >> 2) == 0 ? S0 : ((tile32 >> 2) == 1 ? S1 : S2)) + m * 128 + 4 * hh;
+        bf16_t* hrow = slice(tile32 >> 2) + m * 128 + 4 * hh;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {        // columns tile32*32 + 8*q + 4*hh + 0..3: half of a granule
           bf16x4 hv;
@@ -458,8 +467,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
     auto frag = [&](int kb, int rt, int s) {
       // K elements 64 kb + 32 s + 8 g4 .. + 8 of row 16 rt + r16: slice kb / 2, granule (kb % 2) * 8 + 4 s + g4
       const int gq = ((((kb & 1) * 8 + g4) ^ r16) * 8) ^ (s * 32);
-      const bf16_t* slice = (kb >> 1) == 0 ? S0 : ((kb >> 1) == 1 ? S1 : S2);
-      return *reinterpret_cast<const bf16x8*>(slice + (rt * 16 + r16) * 128 + gq);
+      return *reinterpret_cast<const bf16x8*>(slice(kb >> 1) + (rt * 16 + r16) * 128 + gq);
     };
     // The multiply walks half K blocks (32 elements, one MFMA deep): while half hs is multiplied with all NRT
     // row tiles, the weights of half hs + 1 change lanes and the activation fragment of the next row tile is read.
@@ -546,23 +554,23 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
   };
   for (int nb = 0; nb < nblk; ++nb) down_block(std::integral_constant<int, 2 * kBlocks>{}, nb);
   };   // body
-  if (nblocks == 4) body(std::integral_constant<int, 4>{});
-  else if (nblocks == 3) body(std::integral_constant<int, 3>{});
+  if (MT == 2 && nblocks == 4) body(std::integral_constant<int, 2 * MT>{});
+  else if (MT == 2 && nblocks == 3) body(std::integral_constant<int, 2 * MT - 1>{});
   else if (nblocks == 2) body(std::integral_constant<int, 2>{});
   else body(std::integral_constant<int, 1>{});
 }
 
 
-template <int NT, int CT>
+template <int NT, int CT, int MT>
 void launch_fused_t(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const float* theta, const float* w,
                     const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int S, int H, int E,
                     int act, unsigned x_bytes, bf16_t* yw, bf16_t* preact, hipStream_t s) {
-  const int grid = ((S / 128 + E + 7) & ~7) + 8;
+  const int grid = ((S / (64 * MT) + E + 7) & ~7) + 8;
   if (preact != nullptr)
-    hipLaunchKernelGGL((experts_fused_kernel<NT, CT, 2>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta, w, offsets,
+    hipLaunchKernelGGL((experts_fused_kernel<NT, CT, 2, MT>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta, w, offsets,
                        perm_slot, perm_token, H, E, act, x_bytes, yw, preact);
   else
-    hipLaunchKernelGGL((experts_fused_kernel<NT, CT, 0>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta, w, offsets,
+    hipLaunchKernelGGL((experts_fused_kernel<NT, CT, 0, MT>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta, w, offsets,
                        perm_slot, perm_token, H, E, act, x_bytes, yw, preact);
 }
 
@@ -570,18 +578,27 @@ template <int NT>
 void launch_fused_nt(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const float* theta, const float* w,
                      const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int S, int H, int E,
                      int act, unsigned x_bytes, bf16_t* yw, bf16_t* preact, hipStream_t s) {
-  // (blocks of 256 columns leave room for the third x buffer of the deeper ring where I < 384)
-  if (H % 384 == 0 && (NT == 3 || H % 256 != 0))
-    launch_fused_t<NT, 3>(x, wgu, wd, theta, w, offsets, perm_slot, perm_token, S, H, E, act, x_bytes, yw, preact, s);
-  else if (H % 256 == 0) launch_fused_t<NT, 2>(x, wgu, wd, theta, w, offsets, perm_slot, perm_token, S, H, E, act, x_bytes, yw, preact, s);
-  else launch_fused_t<NT, 1>(x, wgu, wd, theta, w, offsets, perm_slot, perm_token, S, H, E, act, x_bytes, yw, preact, s);
+  constexpr int MT = NT == 4 ? 1 : 2;
+  auto launch = [&](auto ct) {
+    launch_fused_t<NT, decltype(ct)::value, MT>(x, wgu, wd, theta, w, offsets, perm_slot, perm_token, S, H, E, act, x_bytes, yw, preact, s);
+  };
+  // (blocks of 256 columns leave room for the third x buffer of the deeper ring where I is not 384)
+  if constexpr (NT != 4) {
+    if (H % 384 == 0 && (NT == 3 || H % 256 != 0)) {
+      launch(std::integral_constant<int, 3>{});
+      return;
+    }
+  }
+  if (H % 256 == 0) launch(std::integral_constant<int, 2>{});
+  else launch(std::integral_constant<int, 1>{});
 }
 
 template <int NT>
 void launch_raw_nt(const bf16_t* x, const bf16_t* wgu, const int32_t* offsets, const int32_t* perm_token, int S, int H, int E,
                    unsigned x_bytes, bf16_t* gu, hipStream_t s) {
-  const int grid = ((S / 128 + E + 7) & ~7) + 8;
-  hipLaunchKernelGGL((experts_fused_kernel<NT, 1, 1>), dim3(grid), dim3(512), 0, s, x, wgu, nullptr, nullptr, nullptr,
+  constexpr int MT = NT == 4 ? 1 : 2;
+  const int grid = ((S / (64 * MT) + E + 7) & ~7) + 8;
+  hipLaunchKernelGGL((experts_fused_kernel<NT, 1, 1, MT>), dim3(grid), dim3(512), 0, s, x, wgu, nullptr, nullptr, nullptr,
                      offsets, nullptr, perm_token, H, E, 0, x_bytes, nullptr, gu);
 }
 
@@ -602,6 +619,7 @@ hipError_t launch_gateup_raw(const void* x, const void* wgu, const int32_t* offs
     case 128: launch_raw_nt<1>(xp, gp, offsets, perm_token, S, H, E, xb, out, s); break;
     case 256: launch_raw_nt<2>(xp, gp, offsets, perm_token, S, H, E, xb, out, s); break;
     case 384: launch_raw_nt<3>(xp, gp, offsets, perm_token, S, H, E, xb, out, s); break;
+    case 512: launch_raw_nt<4>(xp, gp, offsets, perm_token, S, H, E, xb, out, s); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -611,6 +629,9 @@ bool fused_supported(int H, int I, int dtype) {
   // the activation tile plus two weight stages have to fit 160 KB of LDS: I <= 384
   return dtype == BIBO_DTYPE_BF16 && H >= 128 && (H % 128) == 0 && (I == 128 || I == 256 || I == 384);
 }
+
+// I = 512 on 64-row tiles: what `auto` runs for the shape, under the name of the two-kernel family the stage calls run
+bool fused_wide_supported(int H, int I, int dtype) { return dtype == BIBO_DTYPE_BF16 && H >= 128 && H % 128 == 0 && I == 512; }
 
 hipError_t launch_experts_fused(const void* x, const void* wgu, const void* wd, const float* theta, const float* w,
                                 const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int T,
@@ -628,6 +649,7 @@ hipError_t launch_experts_fused(const void* x, const void* wgu, const void* wd, 
     case 128: launch_fused_nt<1>(xp, gp, dp, theta, w, offsets, perm_slot, perm_token, S, H, E, act, xb, yp, pp, s); break;
     case 256: launch_fused_nt<2>(xp, gp, dp, theta, w, offsets, perm_slot, perm_token, S, H, E, act, xb, yp, pp, s); break;
     case 384: launch_fused_nt<3>(xp, gp, dp, theta, w, offsets, perm_slot, perm_token, S, H, E, act, xb, yp, pp, s); break;
+    case 512: launch_fused_nt<4>(xp, gp, dp, theta, w, offsets, perm_slot, perm_token, S, H, E, act, xb, yp, pp, s); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
