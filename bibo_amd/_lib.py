@@ -14,7 +14,7 @@ NORM_NONE, NORM_SUM, NORM_SOFTMAX = 0, 1, 2
 ALGO_AUTO, ALGO_GENERIC, ALGO_MFMA, ALGO_STREAM, ALGO_FUSED = 0, 1, 2, 3, 4
 MAX_EXPERTS, MAX_TOPK = 64, 8
 ACT_RADIAL_SIGMOID, ACT_RADIAL_TANH, ACT_SILU = 0, 1, 2
-FLAG_ROUND_BLOCK_OUT, FLAG_NO_RESIDUAL, FLAG_GRAD_F32 = 1, 2, 4
+FLAG_ROUND_BLOCK_OUT, FLAG_NO_RESIDUAL, FLAG_GRAD_F32, FLAG_TRAIN_AUTO = 1, 2, 4, 8
 ABI_VERSION = 3
 
 # every symbol include/bibo_moe.h declares

@@ -78,13 +78,16 @@ inline bool stream_eligible(int T, int H, int E, int k, int I, int dtype, bool d
   return stream_possible(T, H, E, k, I, dtype, distinct) && (long long)T * k <= stream_rows_per_expert(H, I, dtype) * E;
 }
 
-// What `auto` runs in a composite call where it resolves to the MFMA family and the fused kernel takes I = 512 on shorter
-// tiles: H = 1024, I = 512, T = 3001, k = 8 in one launch instead of two.  An explicit request for the family runs its two kernels,
-// whose results the stage calls repeat bit for bit.
-constexpr int kAlgoFusedWide = 100;
-inline int composite_algo(int asked, int resolved, int T, int H, int I, int dtype) {
-  return asked == BIBO_ALGO_AUTO && resolved == BIBO_ALGO_MFMA && fused_wide_supported(H, I, dtype) && fused_fits(T, H) ? kAlgoFusedWide
-                                                                                                                       : resolved;
+// What `auto` runs in a composite call under the name of a family: the fused kernel on shorter tiles where it resolves to the
+// MFMA family at I = 512 (H = 1024, T = 3001, k = 8: 199 -> 167 us), and the fused kernel's two halves with a tile's columns cut over
+// several workgroups where there are few tiles (split_columns).  An explicit request for a family runs the kernels its stage
+// calls run, whose results they repeat bit for bit.
+constexpr int kAlgoFusedWide = 100, kAlgoSplit = 101;
+inline int composite_algo(bool automatic, int resolved, int T, int H, int E, int k, int I, int dtype) {
+  if (!automatic) return resolved;
+  const bool wide = resolved == BIBO_ALGO_MFMA && fused_wide_supported(H, I, dtype) && fused_fits(T, H);
+  if ((wide || resolved == BIBO_ALGO_FUSED) && split_columns(T * k, E, H, I)) return kAlgoSplit;
+  return wide ? kAlgoFusedWide : resolved;
 }
 
 // `composite`: the caller is bibo_moe_experts_fwd / bibo_moe_forward, the only entry points that can run
@@ -132,7 +135,7 @@ inline bool few_taken(int algo, int T, int H, int k, int I, int dtype, const voi
 }
 
 struct Workspace {
-  size_t hist, idx, w, counts, offsets, perm_slot, perm_token, hidden, gu, yw;
+  size_t hist, idx, w, counts, offsets, perm_slot, perm_token, hidden, gu, yw, pre;
   size_t least;        // with room for the slot rows only: what every kernel family can do with
   size_t total;
 };
@@ -156,6 +159,13 @@ Workspace carve(int T, int H, int E, int k, int I, int dtype) {
   ws.yw = o;
   ws.least = o + align_up(S * (size_t)H * sizeof(float));
   ws.total = o + align_up(S * (size_t)(generic_tiles(H, I, dtype) && 2 * I > H ? 2 * I : H) * sizeof(float));
+  // bf16 pre-activations of a call whose tiles are cut by columns: the streaming kernels' segment, or one behind the others
+  ws.pre = ws.gu;
+  if (dtype == BIBO_DTYPE_BF16 && mfma_supported(H, I, dtype) && split_columns(T * k, E, H, I) &&
+      !stream_possible(T, H, E, k, I, dtype, true)) {
+    ws.pre = ws.total;
+    ws.total += align_up(S * (size_t)2 * I * sizeof(bf16_t));
+  }
   return ws;
 }
 
@@ -218,6 +228,14 @@ int experts_dispatch(const void* x, const void* wgu, const void* wd, const float
     if (e != hipSuccess) return (int)e;
     return hip_rc(launch_combine(yw, 0, ca, T, H, k, dtype, out, s));
   }
+  if (algo == kAlgoSplit) {
+    if (!aligned16(x) || !aligned16(wgu) || !aligned16(wd)) return BIBO_ERR_MISALIGNED;
+    void* pre = preact != nullptr ? preact : static_cast<void*>(base + ws.pre);
+    hipError_t e = launch_gateup_raw(x, wgu, offsets, perm_token, T, H, Eg, k, I, pre, true, s);
+    if (e != hipSuccess) return (int)e;
+    if ((e = launch_down_act(pre, wd, theta, w, offsets, perm_slot, T * k, H, Eg, I, act, yw, s)) != hipSuccess) return (int)e;
+    return hip_rc(launch_combine(yw, 1, ca, T, H, k, dtype, out, s));
+  }
   if (algo == BIBO_ALGO_FUSED || algo == kAlgoFusedWide) {
     if (!aligned16(x) || !aligned16(wgu) || !aligned16(wd)) return BIBO_ERR_MISALIGNED;
     hipError_t e = launch_experts_fused(x, wgu, wd, theta, w, offsets, perm_slot, perm_token, T, H, Eg, k, I, act, yw, preact, s);
@@ -274,7 +292,8 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
   if (norm_mode < BIBO_NORM_NONE || norm_mode > BIBO_NORM_SOFTMAX || !act_ok(sh->act)) return BIBO_ERR_UNSUPPORTED;
   int a;
   if ((rc = resolve_algo(algo, T, H, E, k, I, dtype, true, true, &a)) != BIBO_OK) return rc;
-  a = composite_algo(algo, a, T, H, I, dtype);
+  a = composite_algo(algo == BIBO_ALGO_AUTO || (state != nullptr && (sh->flags & BIBO_FLAG_TRAIN_AUTO) != 0), a, T, H, E, k, I, dtype);
+  if (a == kAlgoSplit && state == nullptr && workspace_bytes < carve(T, H, E, k, I, dtype).total) a = BIBO_ALGO_FUSED;
   if (!workspace) return BIBO_ERR_NULL_POINTER;
   if (!aligned_ws(workspace)) return BIBO_ERR_MISALIGNED;
   if (T > 0 && (!x || !w_router || !bias || !w_gate_up || !w_down || !out)) return BIBO_ERR_NULL_POINTER;
@@ -613,7 +632,8 @@ int bibo_moe_experts_fwd(const void* x, const int32_t* idx, const float* w, cons
   int a;
   // a caller's indices may repeat an expert inside a token (moe.py:46-71 accepts that)
   if ((rc = resolve_algo(algo, T, H, E, k, I, dtype, true, false, &a)) != BIBO_OK) return rc;
-  a = composite_algo(algo, a, T, H, I, dtype);
+  a = composite_algo(algo == BIBO_ALGO_AUTO, a, T, H, E, k, I, dtype);
+  if (a == kAlgoSplit && workspace_bytes < carve(T, H, E, k, I, dtype).total) a = BIBO_ALGO_FUSED;
   if (!workspace) return BIBO_ERR_NULL_POINTER;
   if (!aligned_ws(workspace)) return BIBO_ERR_MISALIGNED;
   if (T > 0 && (!x || !idx || !w || !w_gate_up || !w_down || !out)) return BIBO_ERR_NULL_POINTER;

@@ -132,6 +132,113 @@ __device__ __forceinline__ bf16x8 to_operand_lanes(bf16x8 v, int sel) {
   return __builtin_bit_cast(bf16x8, u);
 }
 
+// One block of F::BN2 output columns (from column n0 on) for the first NRT 16-row tiles of a tile whose activations sit in LDS
+// (`slice(i)`: columns [128 i, 128 i + 128) of all rows), and its way out through the staging buffers O0 and O1 (moe.py:92-93).
+// wb: the first D K blocks of this wave's w_down rows, already requested; with `more`, the next column block's are on return.
+template <typename F, int CT, int KB, int D, int NB, int NRT, typename Slice>
+__device__ __forceinline__ void down_block(Slice slice, WBlock<CT> (&wb)[NB], const bf16_t*& wp, size_t tile_stride, bool more, int n0,
+                                           const float* w_s, const int* slot_s, int rows, bf16_t* O0, bf16_t* O1, int H,
+                                           bf16_t* __restrict__ yw) {
+  constexpr int I = F::I;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int r16 = lane & 15, g4 = lane >> 4;
+  const int sel = 4 * (4 * r16 + g4);
+  floatx4 acc2[CT][NRT];
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+    for (int rt = 0; rt < NRT; ++rt) acc2[ct][rt] = floatx4{0.f, 0.f, 0.f, 0.f};
+  // Activation fragments are read a row tile ahead of the MFMAs that consume them (across K block
+  // boundaries too).
+  auto frag = [&](int kb, int rt, int s) {
+    // K elements 64 kb + 32 s + 8 g4 .. + 8 of row 16 rt + r16: slice kb / 2, granule (kb % 2) * 8 + 4 s + g4
+    const int gq = ((((kb & 1) * 8 + g4) ^ r16) * 8) ^ (s * 32);
+    return *reinterpret_cast<const bf16x8*>(slice(kb >> 1) + (rt * 16 + r16) * 128 + gq);
+  };
+  // The multiply walks half K blocks (32 elements, one MFMA deep): while half hs is multiplied with all NRT
+  // row tiles, the weights of half hs + 1 change lanes and the activation fragment of the next row tile is read.
+  bf16x8 wc[2][CT], xa[2];
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) wc[0][ct] = to_operand_lanes(wb[0].w[ct][0], sel);
+  xa[0] = frag(0, 0, 0);
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    if (kb + D < KB) load_wblock<CT>(wb[(kb + D) % NB], wp, tile_stride, kb + D);
+    __builtin_amdgcn_sched_barrier(0);     // keep the loads D blocks ahead of their use
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int hs = 2 * kb + s;
+#pragma unroll
+      for (int rt = 0; rt < NRT; ++rt) {
+        const int g = hs * NRT + rt;         // running (half K block, row tile) index
+        if (g + 1 < KB * 2 * NRT) xa[(g + 1) & 1] = frag(((g + 1) / NRT) >> 1, (g + 1) % NRT, ((g + 1) / NRT) & 1);
+        // the CT lane exchanges of the next half are spread over the row tiles (the last tile takes what is left)
+#pragma unroll
+        for (int cx = 0; cx < CT; ++cx)
+          if ((cx == rt || (rt == NRT - 1 && cx > rt)) && hs + 1 < 2 * KB)
+            wc[(hs + 1) & 1][cx] = to_operand_lanes(wb[((hs + 1) >> 1) % NB].w[cx][(hs + 1) & 1], sel);
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+          acc2[ct][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc[hs & 1][ct], xa[g & 1], acc2[ct][rt], 0, 0, 0);
+      }
+    }
+  }
+  wp += (size_t)F::BN2 * I;                                  // next block of columns: in flight during the epilogue
+  if (more) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) load_wblock<CT>(wb[d], wp, tile_stride, d);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  // accumulator: lane holds row 16*rt + r16, columns wave*16*CT + 16*ct + 4*g4 + i.  The block leaves 32 rows at
+  // a time through the two x buffers in turn; between two barriers a wave stages the next 32 rows into one
+  // buffer and copies the previous 32 out of the other.  Staged row r keeps granule c at position c ^ (r & 15): the 8-byte writes of a half wave
+  // then cover all banks.  Copy-out: 16 consecutive threads move 256 contiguous bytes of one row.
+  // (The thread index goes through an empty asm so the staging addresses are formed here, per block,
+  // instead of being hoisted out of the loop and kept alive across the multiply.)
+  int tid_o = tid;
+  asm volatile("" : "+v"(tid_o));
+  const int r16o = tid_o & 15, g4o = (tid_o >> 4) & 3;
+  const int ro = tid_o >> 4, pco = tid_o & 15;             // copy-out: staged row, first granule position
+  auto stage_rows = [&](int hf) {          // rows 32 hf .. + 32 of the block into buffer hf % 2
+    bf16_t* const O = (hf & 1) ? O1 : O0;
+#pragma unroll
+    for (int rq = 0; rq < F::kOutRows / 16; ++rq) {
+      const int rt = hf * (F::kOutRows / 16) + rq;
+      const float ws = w_s[rt * 16 + r16o];                                            // moe.py:93
+      bf16_t* orow = O + (rq * 16 + r16o) * F::BN2 + (g4o & 1) * 4;
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) {
+        const int c = wave * (2 * CT) + ct * 2 + (g4o >> 1);
+        bf16x4 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = (bf16_t)(ws * acc2[ct][rt][i]);
+        *reinterpret_cast<bf16x4*>(orow + (c ^ r16o) * 8) = v;
+      }
+    }
+  };
+  auto copy_out = [&](int hf) {
+    const bf16_t* const O = (hf & 1) ? O1 : O0;
+    const int m = hf * F::kOutRows + ro;
+    if (m < rows) {
+      bf16_t* dst = yw + (size_t)slot_s[m] * H + n0;
+      const bf16_t* src = O + ro * F::BN2;
+#pragma unroll
+      for (int q = 0; q < CT; ++q) {                         // 16 CT granules per row, 16 threads per row
+        const int pc = pco + 16 * q;
+        *reinterpret_cast<u32x4*>(dst + (pc ^ (ro & 15)) * 8) = *reinterpret_cast<const u32x4*>(src + pc * 8);
+      }
+    }
+  };
+  constexpr int NR = NRT * 16 / F::kOutRows;
+  stage_rows(0);
+#pragma unroll
+  for (int hf = 0; hf < NR; ++hf) {
+    __syncthreads();                       // rows of round hf are staged; round hf - 1 has left its buffer
+    if (hf + 1 < NR) stage_rows(hf + 1);
+    copy_out(hf);
+  }
+}
+
 // MODE 0: the forward pass.  MODE 1: the backward pass's recomputation - the kernel stops after phase 1 and writes the
 // pre-activations themselves, rounded to bf16, to `preact` [S, 2I] in permuted row order (gate columns, then up
 // columns), staged through the LDS stages into whole row segments.  MODE 2: the training forward - the forward pass that
@@ -146,7 +253,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
                                                             const int32_t* __restrict__ perm_slot,
                                                             const int32_t* __restrict__ perm_token, int H, int E,
                                                             int act, unsigned x_bytes, bf16_t* __restrict__ yw,
-                                                            bf16_t* __restrict__ preact) {
+                                                            bf16_t* __restrict__ preact, int column_blocks) {
   using F = FusedShape<NT, CT, MTP>;
   constexpr int MT = F::MT, BM = F::BM, I = F::I, BK = F::BK;
   // Every buffer that is read while LDS-DMA fills another is a variable of its own: the compiler orders a DMA
@@ -161,9 +268,13 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
   __shared__ float rinv_s[BM], gain_s[BM], w_s[BM];
   __shared__ int slot_s[BM];
 
+  // MODE 1 may cut a tile's columns over several workgroups (the other modes need whole rows): workgroup cb of a tile then
+  // owns gate columns [cb I, cb I + I) of a row of row_i = column_blocks I and the up columns behind the same gate columns.
+  const int ncb = MODE == 1 ? column_blocks : 1, row_i = I * ncb;
   const TileMap tm = make_tile_map(offsets, E, BM);
-  const int tile = xcd_tile(blockIdx.x, tm.total);
-  if (tile >= tm.total) return;
+  const int flat = xcd_tile(blockIdx.x, tm.total * ncb);
+  if (flat >= tm.total * ncb) return;
+  const int tile = flat / ncb, cb = flat - tile * ncb;
   int e, row0, rows;
   find_tile(tm, offsets, BM, tile, e, row0, rows);
   e = __builtin_amdgcn_readfirstlane(e);                // the same for every lane: keep them in scalar registers
@@ -203,9 +314,9 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
     const unsigned hb = (unsigned)H * sizeof(bf16_t);                            // bytes per weight / hidden-state row
     const int nsteps = H / BK;
     SubLoader<F> ld;
-    ld.w_rsrc = make_rsrc(wgu + (size_t)e * 2 * I * H, 2u * I * hb);
+    ld.w_rsrc = make_rsrc(wgu + (size_t)e * 2 * row_i * H, 2u * row_i * hb);
     ld.x_rsrc = make_rsrc(x, x_bytes);
-    ld.b_voff = ((unsigned)((drow >> 5) * I + (drow & 31))) * hb + chunk * 16;
+    ld.b_voff = ((unsigned)((drow >> 5) * row_i + cb * I + (drow & 31))) * hb + chunk * 16;
     ld.bstep = (unsigned)NT * 32 * hb;
     ld.wave_elems = __builtin_amdgcn_readfirstlane(wave) * 64 * 8;
 #pragma unroll
@@ -372,7 +483,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
         for (int g = tid; g < BM * 16; g += 512) {
           const int m = g >> 4, pos = g & 15;
           if (m < rows)
-            *reinterpret_cast<u32x4*>(preact + (size_t)(row0 + m) * (2 * I) + half * I + t * 128 + ((pos ^ (m & 15)) * 8)) =
+            *reinterpret_cast<u32x4*>(preact + (size_t)(row0 + m) * (2 * row_i) + half * row_i + cb * I + t * 128 + ((pos ^ (m & 15)) * 8)) =
                 *reinterpret_cast<const u32x4*>(from + m * 128 + pos * 8);
         }
       }
@@ -450,109 +561,9 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
   __syncthreads();                         // the activation tile is complete
 
   // ---- phase 3: down projection, routing weight, scatter to slot order (moe.py:92-93) ----
-  const int r16 = lane & 15, g4 = lane >> 4;
   const int nblk = H / F::BN2;
-  const int sel = 4 * (4 * r16 + g4);
-  // One block of F::BN2 output columns for the first NRT 16-row tiles of the tile (NRT = 2 per block that holds rows).
-  auto down_block = [&](auto nrt_c, int nb) {
-    constexpr int NRT = decltype(nrt_c)::value;
-    const int n0 = nb * F::BN2;
-    floatx4 acc2[CT][NRT];
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-      for (int rt = 0; rt < NRT; ++rt) acc2[ct][rt] = floatx4{0.f, 0.f, 0.f, 0.f};
-    // Activation fragments are read a row tile ahead of the MFMAs that consume them (across K block
-    // boundaries too).
-    auto frag = [&](int kb, int rt, int s) {
-      // K elements 64 kb + 32 s + 8 g4 .. + 8 of row 16 rt + r16: slice kb / 2, granule (kb % 2) * 8 + 4 s + g4
-      const int gq = ((((kb & 1) * 8 + g4) ^ r16) * 8) ^ (s * 32);
-      return *reinterpret_cast<const bf16x8*>(slice(kb >> 1) + (rt * 16 + r16) * 128 + gq);
-    };
-    // The multiply walks half K blocks (32 elements, one MFMA deep): while half hs is multiplied with all NRT
-    // row tiles, the weights of half hs + 1 change lanes and the activation fragment of the next row tile is read.
-    bf16x8 wc[2][CT], xa[2];
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct) wc[0][ct] = to_operand_lanes(wb[0].w[ct][0], sel);
-    xa[0] = frag(0, 0, 0);
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
-      if (kb + D < KB) load_wblock<CT>(wb[(kb + D) % NB], wp, tile_stride, kb + D);
-      __builtin_amdgcn_sched_barrier(0);     // keep the loads D blocks ahead of their use
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const int hs = 2 * kb + s;
-#pragma unroll
-        for (int rt = 0; rt < NRT; ++rt) {
-          const int g = hs * NRT + rt;         // running (half K block, row tile) index
-          if (g + 1 < KB * 2 * NRT) xa[(g + 1) & 1] = frag(((g + 1) / NRT) >> 1, (g + 1) % NRT, ((g + 1) / NRT) & 1);
-          // the CT lane exchanges of the next half are spread over the row tiles (the last tile takes what is left)
-#pragma unroll
-          for (int cx = 0; cx < CT; ++cx)
-            if ((cx == rt || (rt == NRT - 1 && cx > rt)) && hs + 1 < 2 * KB)
-              wc[(hs + 1) & 1][cx] = to_operand_lanes(wb[((hs + 1) >> 1) % NB].w[cx][(hs + 1) & 1], sel);
-#pragma unroll
-          for (int ct = 0; ct < CT; ++ct)
-            acc2[ct][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc[hs & 1][ct], xa[g & 1], acc2[ct][rt], 0, 0, 0);
-        }
-      }
-    }
-    wp += (size_t)F::BN2 * I;                                  // next block of columns: in flight during the epilogue
-    if (nb + 1 < nblk) {
-#pragma unroll
-      for (int d = 0; d < D; ++d) load_wblock<CT>(wb[d], wp, tile_stride, d);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    // accumulator: lane holds row 16*rt + r16, columns wave*16*CT + 16*ct + 4*g4 + i.  The block leaves 32 rows at
-    // a time through the two x buffers in turn; between two barriers a wave stages the next 32 rows into one
-    // buffer and copies the previous 32 out of the other.  Staged row r keeps granule c at position c ^ (r & 15): the 8-byte writes of a half wave
-    // then cover all banks.  Copy-out: 16 consecutive threads move 256 contiguous bytes of one row.
-    // (The thread index goes through an empty asm so the staging addresses are formed here, per block,
-    // instead of being hoisted out of the loop and kept alive across the multiply.)
-    int tid_o = tid;
-    asm volatile("" : "+v"(tid_o));
-    const int r16o = tid_o & 15, g4o = (tid_o >> 4) & 3;
-    const int ro = tid_o >> 4, pco = tid_o & 15;             // copy-out: staged row, first granule position
-    auto stage_rows = [&](int hf) {          // rows 32 hf .. + 32 of the block into buffer hf % 2
-      bf16_t* const O = (hf & 1) ? A1 : A0;
-#pragma unroll
-      for (int rq = 0; rq < F::kOutRows / 16; ++rq) {
-        const int rt = hf * (F::kOutRows / 16) + rq;
-        const float ws = w_s[rt * 16 + r16o];                                            // moe.py:93
-        bf16_t* orow = O + (rq * 16 + r16o) * F::BN2 + (g4o & 1) * 4;
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-          const int c = wave * (2 * CT) + ct * 2 + (g4o >> 1);
-          bf16x4 v;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) v[i] = (bf16_t)(ws * acc2[ct][rt][i]);
-          *reinterpret_cast<bf16x4*>(orow + (c ^ r16o) * 8) = v;
-        }
-      }
-    };
-    auto copy_out = [&](int hf) {
-      const bf16_t* const O = (hf & 1) ? A1 : A0;
-      const int m = hf * F::kOutRows + ro;
-      if (m < rows) {
-        bf16_t* dst = yw + (size_t)slot_s[m] * H + n0;
-        const bf16_t* src = O + ro * F::BN2;
-#pragma unroll
-        for (int q = 0; q < CT; ++q) {                         // 16 CT granules per row, 16 threads per row
-          const int pc = pco + 16 * q;
-          *reinterpret_cast<u32x4*>(dst + (pc ^ (ro & 15)) * 8) = *reinterpret_cast<const u32x4*>(src + pc * 8);
-        }
-      }
-    };
-    constexpr int NR = NRT * 16 / F::kOutRows;
-    stage_rows(0);
-#pragma unroll
-    for (int hf = 0; hf < NR; ++hf) {
-      __syncthreads();                       // rows of round hf are staged; round hf - 1 has left its buffer
-      if (hf + 1 < NR) stage_rows(hf + 1);
-      copy_out(hf);
-    }
-  };
-  for (int nb = 0; nb < nblk; ++nb) down_block(std::integral_constant<int, 2 * kBlocks>{}, nb);
+  for (int nb = 0; nb < nblk; ++nb)
+    down_block<F, CT, KB, D, NB, 2 * kBlocks>(slice, wb, wp, tile_stride, nb + 1 < nblk, nb * F::BN2, w_s, slot_s, rows, A0, A1, H, yw);
   };   // body
   if (MT == 2 && nblocks == 4) body(std::integral_constant<int, 2 * MT>{});
   else if (MT == 2 && nblocks == 3) body(std::integral_constant<int, 2 * MT - 1>{});
@@ -561,6 +572,123 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
 }
 
 
+// The second half of the fused kernel on its own, for calls with fewer tiles than CUs: the activations of a tile from the bf16
+// pre-activations [S, 2I] that the first half left (phase 2), and ONE block of output columns (phase 3), so that an expert's
+// w_down passes through H / BN2 CUs at once.  Every one of them computes the tile's activations again, one wave per row, while
+// its first weights are on their way.
+template <int NT, int CT, int MTP>
+__global__ __launch_bounds__(512) void down_act_kernel(const bf16_t* __restrict__ gu, const bf16_t* __restrict__ wd,
+                                                       const float* __restrict__ theta, const float* __restrict__ w,
+                                                       const int32_t* __restrict__ offsets, const int32_t* __restrict__ perm_slot,
+                                                       int H, int E, int act, bf16_t* __restrict__ yw) {
+  using F = FusedShape<NT, CT, MTP>;
+  constexpr int BM = F::BM, I = F::I;
+  __shared__ __attribute__((aligned(16))) bf16_t acts[NT * BM * 128];
+  __shared__ __attribute__((aligned(16))) bf16_t O0[F::kOutElems];
+  __shared__ __attribute__((aligned(16))) bf16_t O1[F::kOutElems];
+  __shared__ float w_s[BM];
+  __shared__ int slot_s[BM];
+  const int nblk = H / F::BN2;
+  const TileMap tm = make_tile_map(offsets, E, BM);
+  const int flat = xcd_tile(blockIdx.x, tm.total * nblk);
+  if (flat >= tm.total * nblk) return;
+  const int tile = flat / nblk, nb = flat - tile * nblk;
+  int e, row0, rows;
+  find_tile(tm, offsets, BM, tile, e, row0, rows);
+  e = __builtin_amdgcn_readfirstlane(e);
+  row0 = __builtin_amdgcn_readfirstlane(row0);
+  rows = __builtin_amdgcn_readfirstlane(rows);
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  constexpr int KB = I / 64;                 // every K block of the weights is requested up front
+  const size_t tile_stride = (size_t)16 * I;
+  const bf16_t* wp = wd + ((size_t)e * H + nb * F::BN2 + wave * (16 * CT) + (lane >> 2)) * I + (lane & 3) * 8;
+  WBlock<CT> wb[KB];
+  // a wave's rows are wave, wave + 8, ...; the first kRowsAhead of them are requested ahead of the weights, which a CU would
+  // otherwise serve first
+  constexpr int kRowsAhead = 8;
+  const bool live = lane * 8 < I;
+  bf16x8 g[kRowsAhead], u[kRowsAhead];
+  auto request = [&](int m0) {
+#pragma unroll
+    for (int i = 0; i < kRowsAhead; ++i) {
+      const bf16_t* src = gu + (size_t)(row0 + min(m0 + 8 * i, rows - 1)) * 2 * I + lane * 8;
+      if (live && m0 + 8 * i < rows) {
+        g[i] = *reinterpret_cast<const bf16x8*>(src);
+        u[i] = *reinterpret_cast<const bf16x8*>(src + I);
+      }
+    }
+  };
+  request(wave);
+  if (tid < BM) {
+    const int slot = perm_slot[row0 + min(tid, rows - 1)];
+    slot_s[tid] = slot;
+    w_s[tid] = w[slot];
+  }
+  const float p = radial_exponent(theta, e, act);                                   // moe.py:89
+#pragma unroll
+  for (int d = 0; d < KB; ++d) load_wblock<CT>(wb[d], wp, tile_stride, d);
+  for (int m0 = wave; m0 < rows; m0 += 8 * kRowsAhead) {
+    if (m0 > wave) request(m0);
+#pragma unroll
+    for (int i = 0; i < kRowsAhead; ++i) {
+      const int m = m0 + 8 * i;
+      if (m >= rows) break;
+      float ss = 0.f;
+      if (live) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) ss = fmaf((float)g[i][q], (float)g[i][q], ss);
+      }
+      ss = wave_sum(ss);
+      float rinv, gain;
+      radial_row_scalars(ss, I, p, act, rinv, gain);                                // 1/r and r^p, moe.py:88-89
+      const float nrl = -1.44269504f * rinv, rg = rinv * gain;
+      if (live) {
+        bf16x8 h;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const float gq = (float)g[i][q];
+          const float sg = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(gq * nrl));
+          h[q] = (bf16_t)(gq * rg * sg * (float)u[i][q]);                           // SiLU(g/r) r^p up
+        }
+        *reinterpret_cast<bf16x8*>(acts + (lane >> 4) * (BM * 128) + m * 128 + (((lane & 15) ^ (m & 15)) << 3)) = h;
+      }
+    }
+  }
+  __syncthreads();
+  auto slice = [&](int i) -> const bf16_t* { return acts + i * (BM * 128); };
+  auto body = [&](auto nblocks_c) {
+    down_block<F, CT, KB, KB, KB, 2 * decltype(nblocks_c)::value>(slice, wb, wp, tile_stride, false, nb * F::BN2, w_s, slot_s, rows, O0,
+                                                                 O1, H, yw);
+  };
+  const int nblocks = (rows + 31) >> 5;
+  if (MTP == 2 && nblocks == 4) body(std::integral_constant<int, 2 * MTP>{});
+  else if (MTP == 2 && nblocks == 3) body(std::integral_constant<int, 2 * MTP - 1>{});
+  else if (nblocks == 2) body(std::integral_constant<int, 2>{});
+  else body(std::integral_constant<int, 1>{});
+}
+
+template <int NT>
+void launch_down_act_nt(const bf16_t* gu, const bf16_t* wd, const float* theta, const float* w, const int32_t* offsets,
+                        const int32_t* perm_slot, int S, int H, int E, int act, bf16_t* yw, hipStream_t s) {
+  auto launch = [&](auto mt, auto ct) {
+    constexpr int MT = decltype(mt)::value, CT = decltype(ct)::value;
+    const int tiles = S / (64 * MT) + E < S ? S / (64 * MT) + E : S;
+    const int grid = ((tiles * (H / (128 * CT)) + 7) & ~7) + 8;
+    hipLaunchKernelGGL((down_act_kernel<NT, CT, MT>), dim3(grid), dim3(512), 0, s, gu, wd, theta, w, offsets, perm_slot, H, E, act, yw);
+  };
+  // 64-row tiles while they and their column blocks leave no workgroup waiting for a CU: shorter, and more of them pull weights
+  using std::integral_constant;
+  const bool two = H % 256 == 0;
+  const bool tall = (S / 64 + E / 2) * (H / (two ? 256 : 128)) > 256;
+  if constexpr (NT < 4) {
+    if (tall) {
+      if (two) launch(integral_constant<int, 2>{}, integral_constant<int, 2>{}); else launch(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+      return;
+    }
+  }
+  if (two) launch(integral_constant<int, 1>{}, integral_constant<int, 2>{}); else launch(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+}
+
 template <int NT, int CT, int MT>
 void launch_fused_t(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const float* theta, const float* w,
                     const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int S, int H, int E,
@@ -568,10 +696,10 @@ void launch_fused_t(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const 
   const int grid = ((S / (64 * MT) + E + 7) & ~7) + 8;
   if (preact != nullptr)
     hipLaunchKernelGGL((experts_fused_kernel<NT, CT, 2, MT>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta, w, offsets,
-                       perm_slot, perm_token, H, E, act, x_bytes, yw, preact);
+                       perm_slot, perm_token, H, E, act, x_bytes, yw, preact, 1);
   else
     hipLaunchKernelGGL((experts_fused_kernel<NT, CT, 0, MT>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta, w, offsets,
-                       perm_slot, perm_token, H, E, act, x_bytes, yw, preact);
+                       perm_slot, perm_token, H, E, act, x_bytes, yw, preact, 1);
 }
 
 template <int NT>
@@ -595,19 +723,21 @@ void launch_fused_nt(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const
 
 template <int NT>
 void launch_raw_nt(const bf16_t* x, const bf16_t* wgu, const int32_t* offsets, const int32_t* perm_token, int S, int H, int E,
-                   unsigned x_bytes, bf16_t* gu, hipStream_t s) {
+                   unsigned x_bytes, bf16_t* gu, int column_blocks, hipStream_t s) {
   constexpr int MT = NT == 4 ? 1 : 2;
-  const int grid = ((S / (64 * MT) + E + 7) & ~7) + 8;
+  const int tiles = S / (64 * MT) + E < S ? S / (64 * MT) + E : S;
+  const int grid = ((tiles * column_blocks + 7) & ~7) + 8;
   hipLaunchKernelGGL((experts_fused_kernel<NT, 1, 1, MT>), dim3(grid), dim3(512), 0, s, x, wgu, nullptr, nullptr, nullptr,
-                     offsets, nullptr, perm_token, H, E, 0, x_bytes, nullptr, gu);
+                     offsets, nullptr, perm_token, H, E, 0, x_bytes, nullptr, gu, column_blocks);
 }
 
 }  // namespace
 
 // Phase 1 of the fused kernel alone: gu[row] = [x W_gate^T, x W_up^T] in bf16 for every permuted row (what the backward
 // pass recomputes, moe.py:84).  Same shapes as launch_experts_fused.
+// `split`: one workgroup per 128 gate (and up) columns of a tile, for calls with fewer tiles than CUs.
 hipError_t launch_gateup_raw(const void* x, const void* wgu, const int32_t* offsets, const int32_t* perm_token, int T, int H,
-                             int E, int k, int I, void* gu, hipStream_t s) {
+                             int E, int k, int I, void* gu, bool split, hipStream_t s) {
   const int S = T * k;
   if (S == 0) return hipSuccess;
   if ((unsigned long long)T * H * sizeof(bf16_t) >= (1ull << 32)) return hipErrorInvalidValue;
@@ -615,11 +745,43 @@ hipError_t launch_gateup_raw(const void* x, const void* wgu, const int32_t* offs
   const bf16_t* xp = static_cast<const bf16_t*>(x);
   const bf16_t* gp = static_cast<const bf16_t*>(wgu);
   bf16_t* out = static_cast<bf16_t*>(gu);
+  if (split) {
+    launch_raw_nt<1>(xp, gp, offsets, perm_token, S, H, E, xb, out, I / 128, s);
+    return hipGetLastError();
+  }
   switch (I) {
-    case 128: launch_raw_nt<1>(xp, gp, offsets, perm_token, S, H, E, xb, out, s); break;
-    case 256: launch_raw_nt<2>(xp, gp, offsets, perm_token, S, H, E, xb, out, s); break;
-    case 384: launch_raw_nt<3>(xp, gp, offsets, perm_token, S, H, E, xb, out, s); break;
-    case 512: launch_raw_nt<4>(xp, gp, offsets, perm_token, S, H, E, xb, out, s); break;
+    case 128: launch_raw_nt<1>(xp, gp, offsets, perm_token, S, H, E, xb, out, 1, s); break;
+    case 256: launch_raw_nt<2>(xp, gp, offsets, perm_token, S, H, E, xb, out, 1, s); break;
+    case 384: launch_raw_nt<3>(xp, gp, offsets, perm_token, S, H, E, xb, out, 1, s); break;
+    case 512: launch_raw_nt<4>(xp, gp, offsets, perm_token, S, H, E, xb, out, 1, s); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+// Whether a tile's columns are cut over several workgroups.  The fused kernel keeps a row's tile on one CU, which is what pulls the
+// expert's weights then: with fewer tiles than CUs most of the chip idles.  Cut (launch_gateup_raw, launch_down_act), the
+// pre-activations make a round trip and every column block computes the activations again, which pays up to about 80 tiles
+// (expected: an expert's last one half full): H = 768, I = 384, E = 64, k = 6: 62 -> 48 us at T = 128, 68 -> 55 at T = 512, 77 -> 64 at
+// T = 1024, but 79 -> 94 at T = 1500; H = 2048, I = 384, E = 16, k = 4: 132 -> 72 at T = 512.  Lighter experts stream faster and gain
+// less: I = 256 up to about 64 tiles at H = 1024 (E = 16, k = 3: 60 -> 43 at T = 512), 40 at H = 512.
+bool split_columns(int S, int E, int H, int I) {
+  const int limit = I >= 384 ? 80 : (H * I >= 256 * 1024 ? 64 : 40);
+  return S / 128 + E / 2 <= limit && I >= 256;
+}
+
+// gu [S, 2I] bf16 -> routing-weighted rows in slot order (down_act_kernel); shapes as launch_gateup_raw takes them
+hipError_t launch_down_act(const void* gu, const void* wd, const float* theta, const float* w, const int32_t* offsets,
+                           const int32_t* perm_slot, int S, int H, int E, int I, int act, void* yw, hipStream_t s) {
+  if (S == 0) return hipSuccess;
+  const bf16_t* gp = static_cast<const bf16_t*>(gu);
+  const bf16_t* dp = static_cast<const bf16_t*>(wd);
+  bf16_t* yp = static_cast<bf16_t*>(yw);
+  switch (I) {
+    case 128: launch_down_act_nt<1>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yp, s); break;
+    case 256: launch_down_act_nt<2>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yp, s); break;
+    case 384: launch_down_act_nt<3>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yp, s); break;
+    case 512: launch_down_act_nt<4>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yp, s); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

@@ -71,7 +71,10 @@ enum bibo_flags {
   BIBO_FLAG_NO_RESIDUAL = 2,
   /* the backward calls only: d_w_router, d_w_gate_up and d_w_down are fp32 whatever `dtype` is (gradients of fp32 master
      weights: the fp32 sums leave as they are, and no conversion pass follows). */
-  BIBO_FLAG_GRAD_F32 = 4
+  BIBO_FLAG_GRAD_F32 = 4,
+  /* bibo_moe_forward_train only: pick the expert kernels as `auto` does in bibo_moe_forward (few tiles: two launches over more
+     workgroups) instead of always running the fused kernel. */
+  BIBO_FLAG_TRAIN_AUTO = 8
 };
 
 /* kernel family for the expert GEMMs */
