@@ -289,107 +289,107 @@ __global__ __launch_bounds__(256) void act_bwd_kernel(const bf16_t* __restrict__
   }
 }
 
-// +/-Identity experts (moe.py:95-99): a slot routed to one contributes sign w x[t] to the output, so
-//   dw[slot] = sign <d_out[t], x[t]>,  dx_slot[slot] = sign w[slot] d_out[t]
-// (the per-slot dx rows are summed over a token's slots by dx_combine_kernel like those of the GLU experts).
-// One wave per permuted row behind the GLU experts' rows: rows offsets[Eg] .. offsets[Eg + n_pos + n_neg).
-__global__ __launch_bounds__(256) void special_bwd_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ d_out,
-                                                          const float* __restrict__ w, const int32_t* __restrict__ offsets,
-                                                          const int32_t* __restrict__ perm_slot,
-                                                          const int32_t* __restrict__ perm_token, int Eg, int n_pos,
-                                                          int n_neg, int H, float* __restrict__ dw_slot,
-                                                          bf16_t* __restrict__ dxs) {
+__device__ __forceinline__ float lane_value(float v, int lane) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
+}
+
+// Everything per token behind the experts, one wave per token and run of up to 512 columns (`parts` runs of equal length):
+//   +/-Identity slots (moe.py:95-99): dw = +/- <d_out[t], x[t]>, their share of dx is +/- w d_out[t];
+//   router (router.py:31,41-47; w_router == NULL: none): lane j < k turns the gradients of the combine weights into dlogit of
+//     slot j, the sums over a token's slots in ascending j;
+//   dx[t, c] = sum_j (dx row of slot j + dl[t, j] W_router[idx[t, j], c]).
+// A slot whose expert id lies outside [0, E + n_pos + n_neg) (padding in a caller's indices, which the forward pass skips) has no
+// dx row and no combine-weight gradient: it is left out and its dw_slot entry set to zero.  Every wave of a token works out the k
+// scalars, the first one stores them.  Bound by reading the slots' dx rows (T = 8192, H = 768, k = 6: 75 MB), which are requested
+// before the indices that decide about them are back.  K = k at compile time, and no load under a condition: the compiler
+// drains all loads where a branch around one ends (k at run time: 26 us at that size, 21 like this).
+template <int K>
+__global__ __launch_bounds__(256) void token_bwd_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ d_out,
+                                                        const bf16_t* __restrict__ dxs, const float* __restrict__ logits,
+                                                        const int32_t* __restrict__ idx, const float* __restrict__ w,
+                                                        const bf16_t* __restrict__ w_router, int T, int H, int E, int n_pos,
+                                                        int n_neg, int norm_mode, int parts, float* __restrict__ dw_slot,
+                                                        float* __restrict__ dl, bf16_t* __restrict__ dx) {
   const int lane = threadIdx.x & 63;
-  const int row = offsets[Eg] + blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= offsets[Eg + n_pos + n_neg]) return;
-  const float sign = row < offsets[Eg + n_pos] ? 1.f : -1.f;
-  const int slot = perm_slot[row];
-  const size_t t = (size_t)perm_token[row];
-  const float sw = sign * w[slot];
-  float dot = 0.f;
-  for (int c = lane * 8; c < H; c += 64 * 8) {
-    const bf16x8 xv = *reinterpret_cast<const bf16x8*>(x + t * H + c);
-    const bf16x8 dv = *reinterpret_cast<const bf16x8*>(d_out + t * H + c);
-    bf16x8 o;
+  const int unit = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  const int t = unit / parts, part = unit - t * parts;
+  if (t >= T) return;
+  const int Et = E + n_pos + n_neg, gran = H / 8, run = (gran + parts - 1) / parts;
+  const int c = part * run + lane, cc = min(c, gran - 1);
+  const bool mine = lane < run && c < gran;
+  const bf16x8* const dtok = reinterpret_cast<const bf16x8*>(d_out) + (size_t)t * gran;
+  // lane j < k: slot j.  Loads are waited for in the order of their requests: the indices first, then the rows, which do not need them.
+  const int sl = t * K + min(lane, K - 1);
+  int e_ = idx[sl];
+  const float w_ = w[sl];
+  float dw_ = dw_slot[sl], s_ = 0.f;
+  bf16x8 v[K], r[K];
+  const bf16x8* const rows = reinterpret_cast<const bf16x8*>(dxs) + (size_t)t * K * gran + cc;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      dot = fmaf((float)dv[q], (float)xv[q], dot);
-      o[q] = (bf16_t)(sw * (float)dv[q]);
-    }
-    *reinterpret_cast<bf16x8*>(dxs + (size_t)slot * H + c) = o;
-  }
-  dot = wave_sum(dot);
-  if (lane == 0) dw_slot[slot] = sign * dot;
-}
-
-// ---- router backward (router.py:31,41-47) --------------------------------------------------------------------
-// Eight lanes per token, lane j < k for slot j: dlogit of the k selected experts from the gradients of the combine
-// weights.  The sums over a token's slots are taken in ascending j by every lane, so they are the same bits in all.
-__global__ __launch_bounds__(256) void router_bwd_kernel(const float* __restrict__ logits, const int32_t* __restrict__ idx,
-                                                         const float* __restrict__ w, const float* __restrict__ dw, int T,
-                                                         int E, int k, int norm_mode, float* __restrict__ dl) {
-  static_assert(kMaxK <= 8, "eight lanes per token");
-  const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-  const int t = gid >> 3, j = gid & 7;
-  const bool live = t < T && j < k;
-  float sj = 0.f, dwj = 0.f, wj = 0.f;
-  if (live) {
-    sj = 1.f / (1.f + __expf(-logits[(size_t)t * E + idx[t * k + j]]));
-    dwj = dw[t * k + j];
-    wj = w[t * k + j];
-  }
-  const int base = (threadIdx.x & 63) & ~7;
-  float sum = 0.f, dot = 0.f;
+  for (int j = 0; j < K; ++j) v[j] = rows[(size_t)j * gran];
+  __builtin_amdgcn_sched_barrier(0);
+  if (e_ >= Et) e_ = -1;
+  if (e_ < 0 || e_ >= E) dw_ = 0.f;
+  if (w_router != nullptr) {
+    const float logit = logits[(size_t)t * Et + max(e_, 0)];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float si = __shfl(sj, base + i, kWave), di = __shfl(dwj, base + i, kWave), wi = __shfl(wj, base + i, kWave);
-    if (i < k) {
-      sum += si;
-      dot = fmaf(di, wi, dot);
-    }
+    for (int j = 0; j < K; ++j)
+      r[j] = reinterpret_cast<const bf16x8*>(w_router)[(size_t)max(__builtin_amdgcn_readlane(e_, j), 0) * gran + cc];
+    s_ = 1.f / (1.f + __expf(-logit));
   }
-  if (!live) return;
-  float ds = dwj;
-  if (k > 1 && norm_mode == BIBO_NORM_SUM) ds = (ds - dot) / (sum + 1e-20f);
-  else if (k > 1 && norm_mode == BIBO_NORM_SOFTMAX) ds = wj * (ds - dot);
-  dl[t * k + j] = ds * sj * (1.f - sj);
-}
-
-// dx[t, c] = sum_j dxs[t k + j, c] + sum_j dl[t, j] W_router[idx[t, j], c]; one thread per 8 columns.  dl == NULL: the
-// slot rows alone (the experts without their router).  A slot whose expert id lies outside [0, n_experts) (padding in
-// a caller's indices, which the forward pass skips) has no dxs row and no combine-weight gradient: it is left out of
-// the sum and its dw_slot entry is set to zero here.
-__global__ __launch_bounds__(256) void dx_combine_kernel(const bf16_t* __restrict__ dxs, const float* __restrict__ dl,
-                                                         const int32_t* __restrict__ idx,
-                                                         const bf16_t* __restrict__ w_router, int T, int H, int k,
-                                                         int n_experts, float* __restrict__ dw_slot,
-                                                         bf16_t* __restrict__ dx) {
-  const int gpr = H / 8;
-  const long long gid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= (long long)T * gpr) return;
-  const int t = (int)(gid / gpr), c = (int)(gid - (long long)t * gpr) * 8;
+  if (__ballot(e_ >= E) != 0ull) {
+    float dot = 0.f;
+    for (int g = lane; g < gran; g += kWave) {
+      const bf16x8 xv = reinterpret_cast<const bf16x8*>(x)[(size_t)t * gran + g];
+      const bf16x8 dv = dtok[g];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) dot = fmaf((float)dv[q], (float)xv[q], dot);
+    }
+    dot = wave_sum(dot);
+    if (e_ >= E) dw_ = e_ < E + n_pos ? dot : -dot;
+  }
+  float dl_ = 0.f;
+  if (w_router != nullptr) {
+    float sum = 0.f, dot = 0.f;
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+      sum += lane_value(s_, j);
+      dot = fmaf(lane_value(dw_, j), lane_value(w_, j), dot);
+    }
+    float ds = dw_;
+    if (K > 1 && norm_mode == BIBO_NORM_SUM) ds = (ds - dot) / (sum + 1e-20f);
+    else if (K > 1 && norm_mode == BIBO_NORM_SOFTMAX) ds = w_ * (ds - dot);
+    dl_ = ds * s_ * (1.f - s_);
+  }
+  if (part == 0 && lane < K) {
+    if (e_ < 0 || e_ >= E) dw_slot[t * K + lane] = dw_;
+    if (w_router != nullptr) dl[t * K + lane] = dl_;
+  }
+  if (!mine) return;
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int j = 0; j < k; ++j) {
-    const int e = idx[t * k + j];
-    if (e < 0 || e >= n_experts) {
-      if (c == 0) dw_slot[t * k + j] = 0.f;
-      continue;
-    }
-    const bf16x8 v = *reinterpret_cast<const bf16x8*>(dxs + ((size_t)t * k + j) * H + c);
-    if (dl != nullptr) {
-      const bf16x8 r = *reinterpret_cast<const bf16x8*>(w_router + (size_t)e * H + c);
-      const float d = dl[t * k + j];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) acc[q] += (float)v[q] + d * (float)r[q];
+  for (int j = 0; j < K; ++j) {
+    const int e = __builtin_amdgcn_readlane(e_, j);
+    if (e < 0) continue;
+    if (e >= E) {
+      const float wj = lane_value(w_, j);
+      const bf16x8 dv = dtok[c];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) acc[q] = fmaf(e < E + n_pos ? wj : -wj, (float)dv[q], acc[q]);
     } else {
 #pragma unroll
-      for (int q = 0; q < 8; ++q) acc[q] += (float)v[q];
+      for (int q = 0; q < 8; ++q) acc[q] += (float)v[j][q];
+    }
+    if (w_router != nullptr) {
+      const float dj = lane_value(dl_, j);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) acc[q] = fmaf(dj, (float)r[j][q], acc[q]);
     }
   }
   bf16x8 o;
 #pragma unroll
   for (int q = 0; q < 8; ++q) o[q] = (bf16_t)acc[q];
-  *reinterpret_cast<bf16x8*>(dx + (size_t)t * H + c) = o;
+  reinterpret_cast<bf16x8*>(dx)[(size_t)t * gran + c] = o;
 }
 
 // dW_router[e, c] = sum over the rows r of expert e of dl[slot(r)] x[token(r), c], in two steps.  Step 1, grid =
@@ -570,15 +570,24 @@ hipError_t launch_backward(const void* x, const void* d_out, const void* w_route
   // dx of every slot, in slot order: [dg, du] W_gate_up, contracts over the 2I rows of w_gate_up [E, 2I, H]
   err = launch_dgrad<false, true>(dgu, nullptr, wgup, offsets, perm_slot, S, 2 * I, H, E, dxs, s);
   if (err != hipSuccess) return err;
-  if (n_pos + n_neg > 0)   // (as many waves as there could be rows: how many there are is only known on the device)
-    hipLaunchKernelGGL(special_bwd_kernel, dim3((S + 3) / 4), dim3(256), 0, s, xp, dop, w, offsets, perm_slot, perm_token, E,
-                       n_pos, n_neg, H, b.dw_slot, dxs);
   const bool with_router = w_router != nullptr;      // else: the experts alone, the caller owns the routing
-  if (with_router)
-    hipLaunchKernelGGL(router_bwd_kernel, dim3((T + 31) / 32), dim3(256), 0, s, logits, idx, w, b.dw_slot, T, Et, k, norm_mode,
-                       b.dl);
-  hipLaunchKernelGGL(dx_combine_kernel, dim3((unsigned)(((long long)T * (H / 8) + 255) / 256)), dim3(256), 0, s, dxs,
-                     with_router ? b.dl : nullptr, idx, wrp, T, H, k, Et, b.dw_slot, static_cast<bf16_t*>(dx));
+  const int parts = (H / 8 + kWave - 1) / kWave;     // runs of columns a lane each
+  auto token_bwd = [&](auto kc) {
+    hipLaunchKernelGGL(token_bwd_kernel<decltype(kc)::value>, dim3((unsigned)(((long long)T * parts + 3) / 4)), dim3(256), 0, s, xp, dop,
+                       dxs, logits, idx, w, wrp, T, H, E, n_pos, n_neg, norm_mode, parts, b.dw_slot, b.dl, static_cast<bf16_t*>(dx));
+  };
+  static_assert(kMaxK == 8, "a case per k");
+  using std::integral_constant;
+  switch (k) {
+    case 1: token_bwd(integral_constant<int, 1>{}); break;
+    case 2: token_bwd(integral_constant<int, 2>{}); break;
+    case 3: token_bwd(integral_constant<int, 3>{}); break;
+    case 4: token_bwd(integral_constant<int, 4>{}); break;
+    case 5: token_bwd(integral_constant<int, 5>{}); break;
+    case 6: token_bwd(integral_constant<int, 6>{}); break;
+    case 7: token_bwd(integral_constant<int, 7>{}); break;
+    default: token_bwd(integral_constant<int, 8>{});
+  }
   if (with_router)
     hipLaunchKernelGGL(dwr_partial_kernel, dim3((H + 255) / 256, slots, kDwrSplit), dim3(256), 0, s, xp, b.dl, b.wgrad_plan,
                        perm_slot, perm_token, H, b.dwr_part);
