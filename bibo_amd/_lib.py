@@ -92,11 +92,11 @@ def _declare(l):
     l.bibo_moe_exp_attn_res_fwd.restype = ci
     l.bibo_moe_exp_attn_res_fwd.argtypes = [vp, ci, vp, ctypes.c_float, ci, ci, ci, vp, vp]
     cf = ctypes.c_float
-    for name, args in (("bibo_moe_exp_attn_res_norm_fwd", [vp, ci, vp, cf, vp, cf, ci, ci, ci, vp, vp, vp]),
-                       ("bibo_moe_exp_carry_fwd", [vp, vp, vp, vp, ci, ci, vp, vp, vp]),
+    for name, args in (("bibo_moe_exp_attn_res_norm_fwd", [vp, ci, vp, vp, cf, vp, cf, ci, ci, ci, ci, vp, vp, vp]),
+                       ("bibo_moe_exp_carry_fwd", [vp, vp, vp, ci, vp, ci, ci, vp, vp, vp]),
                        ("bibo_moe_exp_silu_mul_fwd", [vp, ci, ci, vp, vp]),
-                       ("bibo_moe_exp_qk_norm_rope", [vp, ci, ci, ci, ci, ci, ci, vp, vp, cf, vp, vp, vp]),
-                       ("bibo_moe_exp_attention_fwd", [vp, ci, ci, ci, ci, ci, ci, ci, cf, vp, vp, vp])):
+                       ("bibo_moe_exp_qk_norm_rope", [vp, ci, ci, ci, ci, ci, ci, vp, vp, ci, cf, vp, vp, ci, ci, vp]),
+                       ("bibo_moe_exp_attention_fwd", [vp, ci, ci, ci, ci, ci, ci, ci, cf, vp, ci, vp, vp])):
         getattr(l, name).restype, getattr(l, name).argtypes = ci, args
     l.bibo_moe_balance_step.restype = ci
     l.bibo_moe_balance_step.argtypes = [vp, vp, vp, ci, ctypes.c_float, ci, vp]

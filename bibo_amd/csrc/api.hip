@@ -40,6 +40,8 @@ inline size_t elt_size(int dtype) { return dtype == BIBO_DTYPE_BF16 ? 2 : 4; }
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 inline bool aligned_ws(const void* p) { return (reinterpret_cast<uintptr_t>(p) & (kAlign - 1)) == 0; }
 
+inline Vec vec(const void* p, int dtype) { return Vec{p, dtype == BIBO_DTYPE_BF16}; }
+inline bool vec_ok(const void* p, int dtype) { return dtype != BIBO_DTYPE_BF16 || aligned16(p); }
 inline bool act_ok(int act) { return act >= BIBO_ACT_RADIAL_SIGMOID && act <= BIBO_ACT_SILU; }
 
 int check_dims(int T, int H, int E, int k, int I, int dtype, int n_pos = 0, int n_neg = 0) {
@@ -886,13 +888,14 @@ int bibo_moe_balance_step(const int32_t* counts, float* accumulated, float* bias
   return hip_rc(launch_balance_step(counts, accumulated, bias, E, factor, update, static_cast<hipStream_t>(stream)));
 }
 
-int bibo_moe_exp_attn_res_norm_fwd(const void* const* candidates, int n_candidates, const float* score_weight, float eps,
-                                   const float* norm_weight, float norm_eps, int T, int H, int dtype, void* out, void* normed,
-                                   void* stream) {
+int bibo_moe_exp_attn_res_norm_fwd(const void* const* candidates, int n_candidates, const void* score_a, const void* score_b,
+                                   float eps, const void* norm_weight, float norm_eps, int weight_dtype, int T, int H, int dtype,
+                                   void* out, void* normed, void* stream) {
   const int rc = check_dims(T, H, 1, 1, 1, dtype);
   if (rc != BIBO_OK) return rc;
   if (!attn_res_supported(H, n_candidates, dtype)) return BIBO_ERR_UNSUPPORTED;
-  if (!candidates || !score_weight || (normed && !norm_weight)) return BIBO_ERR_NULL_POINTER;
+  if (!candidates || !score_a || (normed && !norm_weight)) return BIBO_ERR_NULL_POINTER;
+  if (!vec_ok(score_a, weight_dtype) || !vec_ok(score_b, weight_dtype) || !vec_ok(norm_weight, weight_dtype)) return BIBO_ERR_MISALIGNED;
   if (T == 0) return BIBO_OK;
   if (!out) return BIBO_ERR_NULL_POINTER;
   for (int i = 0; i < n_candidates; ++i) {
@@ -900,24 +903,27 @@ int bibo_moe_exp_attn_res_norm_fwd(const void* const* candidates, int n_candidat
     if (!aligned16(candidates[i])) return BIBO_ERR_MISALIGNED;
   }
   if (!aligned16(out) || !aligned16(normed)) return BIBO_ERR_MISALIGNED;
-  return hip_rc(launch_attn_res(candidates, n_candidates, score_weight, eps, T, H, out, norm_weight, norm_eps, normed,
-                                static_cast<hipStream_t>(stream)));
+  return hip_rc(launch_attn_res(candidates, n_candidates, vec(score_a, weight_dtype), vec(score_b, weight_dtype), eps, T, H, out,
+                                vec(norm_weight, weight_dtype), norm_eps, normed, static_cast<hipStream_t>(stream)));
 }
 
 int bibo_moe_exp_attn_res_fwd(const void* const* candidates, int n_candidates, const float* score_weight, float eps, int T, int H,
                               int dtype, void* out, void* stream) {
-  return bibo_moe_exp_attn_res_norm_fwd(candidates, n_candidates, score_weight, eps, nullptr, 0.f, T, H, dtype, out, nullptr, stream);
+  return bibo_moe_exp_attn_res_norm_fwd(candidates, n_candidates, score_weight, nullptr, eps, nullptr, 0.f, BIBO_DTYPE_F32, T, H, dtype,
+                                        out, nullptr, stream);
 }
 
-int bibo_moe_exp_carry_fwd(const void* attn_read, const void* a, const float* theta, const void* prefix, int T, int H, void* hs,
-                           void* prefix_out, void* stream) {
+int bibo_moe_exp_carry_fwd(const void* attn_read, const void* a, const void* theta, int theta_dtype, const void* prefix, int T, int H,
+                           void* hs, void* prefix_out, void* stream) {
   const int rc = check_dims(T, H, 1, 1, 1, BIBO_DTYPE_BF16);
   if (rc != BIBO_OK) return rc;
   if (H % 8 != 0) return BIBO_ERR_UNSUPPORTED;
   if (T == 0) return BIBO_OK;
   if (!attn_read || !a || !hs || (prefix && !prefix_out)) return BIBO_ERR_NULL_POINTER;
-  if (!aligned16(attn_read) || !aligned16(a) || !aligned16(hs) || !aligned16(prefix) || !aligned16(prefix_out)) return BIBO_ERR_MISALIGNED;
-  return hip_rc(launch_carry(attn_read, a, theta, prefix, T, H, hs, prefix_out, static_cast<hipStream_t>(stream)));
+  if (!aligned16(attn_read) || !aligned16(a) || !aligned16(hs) || !aligned16(prefix) || !aligned16(prefix_out) ||
+      !vec_ok(theta, theta_dtype))
+    return BIBO_ERR_MISALIGNED;
+  return hip_rc(launch_carry(attn_read, a, vec(theta, theta_dtype), prefix, T, H, hs, prefix_out, static_cast<hipStream_t>(stream)));
 }
 
 int bibo_moe_exp_silu_mul_fwd(const void* gate_up, int T, int I, void* out, void* stream) {
@@ -930,28 +936,32 @@ int bibo_moe_exp_silu_mul_fwd(const void* gate_up, int T, int I, void* out, void
   return hip_rc(launch_silu_mul(gate_up, T, I, out, static_cast<hipStream_t>(stream)));
 }
 
-int bibo_moe_exp_qk_norm_rope(void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, const float* q_weight,
-                              const float* k_weight, float eps, const float* cos, const float* sin, void* stream) {
+int bibo_moe_exp_qk_norm_rope(void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, const void* q_weight,
+                              const void* k_weight, int weight_dtype, float eps, const void* cos, const void* sin, int rope_dtype,
+                              int ld_rope, void* stream) {
   if (B < 0 || S < 0 || (long long)B * S > 0x3fffffffLL) return BIBO_ERR_BAD_SHAPE;
   if (!exp_attention_supported(n_heads, n_kv_heads, head_dim) || ld < (n_heads + 2 * n_kv_heads) * head_dim || ld % 8 != 0 ||
-      (cos == nullptr) != (sin == nullptr))
+      (cos == nullptr) != (sin == nullptr) || (cos != nullptr && (ld_rope < head_dim / 2 || ld_rope % 8 != 0)))
     return BIBO_ERR_UNSUPPORTED;
   if (B == 0 || S == 0) return BIBO_OK;
   if (!qkv) return BIBO_ERR_NULL_POINTER;
-  if (!aligned16(qkv)) return BIBO_ERR_MISALIGNED;
-  return hip_rc(launch_qk_norm_rope(qkv, ld, B * S, S, n_heads, n_kv_heads, head_dim, q_weight, k_weight, eps, cos, sin,
+  if (!aligned16(qkv) || !vec_ok(q_weight, weight_dtype) || !vec_ok(k_weight, weight_dtype) || !vec_ok(cos, rope_dtype) ||
+      !vec_ok(sin, rope_dtype))
+    return BIBO_ERR_MISALIGNED;
+  return hip_rc(launch_qk_norm_rope(qkv, ld, B * S, S, n_heads, n_kv_heads, head_dim, vec(q_weight, weight_dtype),
+                                    vec(k_weight, weight_dtype), eps, vec(cos, rope_dtype), vec(sin, rope_dtype), ld_rope,
                                     static_cast<hipStream_t>(stream)));
 }
 
 int bibo_moe_exp_attention_fwd(const void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, int window,
-                               float scale, const float* xsa_alpha, void* out, void* stream) {
+                               float scale, const void* xsa_alpha, int alpha_dtype, void* out, void* stream) {
   if (B < 0 || S < 0 || window < 0 || (long long)B * S * n_heads > 0x3fffffffLL) return BIBO_ERR_BAD_SHAPE;
   if (!exp_attention_supported(n_heads, n_kv_heads, head_dim) || ld < (n_heads + 2 * n_kv_heads) * head_dim || ld % 8 != 0)
     return BIBO_ERR_UNSUPPORTED;
   if (B == 0 || S == 0) return BIBO_OK;
   if (!qkv || !out) return BIBO_ERR_NULL_POINTER;
   if (!aligned16(qkv) || !aligned16(out)) return BIBO_ERR_MISALIGNED;
-  return hip_rc(launch_exp_attention(qkv, ld, B, S, n_heads, n_kv_heads, head_dim, window, scale, xsa_alpha, out,
+  return hip_rc(launch_exp_attention(qkv, ld, B, S, n_heads, n_kv_heads, head_dim, window, scale, vec(xsa_alpha, alpha_dtype), out,
                                      static_cast<hipStream_t>(stream)));
 }
 

@@ -128,7 +128,8 @@ py::tuple ffn_forward(const Tensor& h, const Tensor& norm_weight, double eps, co
   c10::DeviceGuard guard(h.device());
   const Tensor x = h.contiguous();
   const bibo_moe_shape sh = shape_of(x, l, flags);
-  check_tensor(norm_weight, "norm_weight", at::kFloat, {sh.H});
+  const Tensor nw = in_dtype(norm_weight.detach(), at::kFloat);
+  check_tensor(nw, "norm_weight", at::kFloat, {sh.H});
   Tensor res;
   if (residual.has_value()) {
     res = in_dtype(*residual, x.scalar_type());
@@ -140,7 +141,7 @@ py::tuple ffn_forward(const Tensor& h, const Tensor& norm_weight, double eps, co
   size_t bytes = 0;
   check(bibo_moe_ffn_workspace_bytes(&sh, &bytes), "bibo_moe_ffn_workspace_bytes");
   const Tensor ws = workspace_on(x.device(), s, bytes);
-  check(bibo_moe_ffn_forward(x.data_ptr(), f32(norm_weight), (float)eps, res.defined() ? res.data_ptr() : nullptr,
+  check(bibo_moe_ffn_forward(x.data_ptr(), f32(nw), (float)eps, res.defined() ? res.data_ptr() : nullptr,
                              w_router.data_ptr(), f32(bias), w_gate_up.data_ptr(), w_down.data_ptr(), f32(theta), &sh, norm, algo,
                              out.data_ptr(), nullptr, nullptr, int_ptr(counts), ws.data_ptr(), (size_t)ws.numel(), s),
         "bibo_moe_ffn_forward");
@@ -274,16 +275,35 @@ void check_rows(const Tensor& t, const char* name, int64_t cols) {
   TORCH_CHECK_VALUE(t.is_contiguous() && t.dim() >= 1 && t.size(-1) == cols, name, " must be contiguous rows of ", cols);
   TORCH_CHECK_TYPE(t.scalar_type() == at::kBFloat16, name, " must be bfloat16");
 }
-const float* f32_or_null(const c10::optional<Tensor>& t, const char* name, at::IntArrayRef shape) {
-  if (!t.has_value()) return nullptr;
-  check_tensor(*t, name, at::kFloat, shape);
-  return f32(*t);
+// Small parameter vectors of one launch in the type the kernels read them in: bf16 in place where every one is bf16 and
+// 16-byte aligned, else fp32 (copies of those that are not).
+struct Vecs {
+  std::vector<Tensor> t;
+  int dtype;
+  const void* operator[](size_t i) const { return t[i].defined() ? t[i].data_ptr() : nullptr; }
+};
+Vecs vecs(std::initializer_list<c10::optional<Tensor>> in, int64_t n, const char* what) {
+  Vecs v{{}, BIBO_DTYPE_BF16};
+  for (const auto& o : in) {
+    const Tensor t = o.has_value() ? o->detach().reshape({-1}).contiguous() : Tensor();
+    if (t.defined()) {
+      TORCH_CHECK(t.is_cuda(), what, " must live on the GPU (got ", t.device(), "); bibo_amd has no CPU path");
+      TORCH_CHECK_VALUE(t.numel() == n, what, " must have ", n, " elements, got ", t.numel());
+      if (t.scalar_type() != at::kBFloat16 || reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 != 0) v.dtype = BIBO_DTYPE_F32;
+    }
+    v.t.push_back(t);
+  }
+  if (v.dtype == BIBO_DTYPE_F32)
+    for (Tensor& t : v.t)
+      if (t.defined()) t = t.to(at::kFloat);
+  return v;
 }
 hipStream_t stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
-// candidates [T, H] -> (their depth mix, its RMSNorm or None)
-py::tuple exp_attn_res_norm(const std::vector<Tensor>& candidates, const Tensor& score_weight, double eps,
-                            const c10::optional<Tensor>& norm_weight, double norm_eps) {
+// candidates [T, H] -> (their depth mix with score weight score_a * score_b, its RMSNorm or None)
+py::tuple exp_attn_res_norm(const std::vector<Tensor>& candidates, const Tensor& score_a, const c10::optional<Tensor>& score_b,
+                            double eps, const c10::optional<Tensor>& norm_weight, double norm_eps) {
+  at::NoGradGuard no_grad;
   TORCH_CHECK_VALUE(!candidates.empty() && candidates.size() <= 8, "1 to 8 candidates");
   const Tensor& c0 = candidates[0];
   const int64_t H = c0.size(-1), T = c0.numel() / H;
@@ -293,58 +313,61 @@ py::tuple exp_attn_res_norm(const std::vector<Tensor>& candidates, const Tensor&
     TORCH_CHECK_VALUE(candidates[i].numel() == c0.numel(), "candidates must have one size");
     ptrs[i] = candidates[i].data_ptr();
   }
-  check_tensor(score_weight, "score_weight", at::kFloat, {H});
-  const float* nw = f32_or_null(norm_weight, "norm_weight", {H});
   c10::DeviceGuard guard(c0.device());
+  const Vecs v = vecs({score_a, score_b, norm_weight}, H, "score and norm weights");
+  const void* nw = v[2];
   Tensor out = at::empty_like(c0), normed;
   if (nw != nullptr) normed = at::empty_like(c0);
-  check(bibo_moe_exp_attn_res_norm_fwd(ptrs, (int)candidates.size(), f32(score_weight), (float)eps, nw, (float)norm_eps, (int)T, (int)H,
+  check(bibo_moe_exp_attn_res_norm_fwd(ptrs, (int)candidates.size(), v[0], v[1], (float)eps, nw, (float)norm_eps, v.dtype, (int)T, (int)H,
                                        BIBO_DTYPE_BF16, out.data_ptr(), nw != nullptr ? normed.data_ptr() : nullptr, stream_of(c0)),
         "bibo_moe_exp_attn_res_norm_fwd");
   return py::make_tuple(out, maybe(normed));
 }
 
 // x [B, S, H] -> attention output [B, S, H]: one projection to q|k|v rows, norm and RoPE in place, attention with XSA, output
-// projection (the two products are library GEMMs)
-Tensor exp_attention(const Tensor& x, const Tensor& w_qkv, const Tensor& w_o, const c10::optional<Tensor>& q_weight,
+// projection (the two products are library GEMMs).  The three projection weights are joined here on every call (2.4 MB at
+// H = 768: 1 % of the call at 8 x 2048 tokens): a joined copy that is kept would not see a write through `.data`.
+Tensor exp_attention(const Tensor& x, const Tensor& w_q, const Tensor& w_k, const Tensor& w_v, const Tensor& w_o, const c10::optional<Tensor>& q_weight,
                      const c10::optional<Tensor>& k_weight, double eps, const c10::optional<Tensor>& cos,
                      const c10::optional<Tensor>& sin, const c10::optional<Tensor>& xsa_alpha, int n_heads, int n_kv_heads,
                      int head_dim, int window, double scale) {
   at::NoGradGuard no_grad;
   const int64_t B = x.size(0), S = x.size(1);
   check_rows(x, "x", x.size(2));
-  const float *qw = f32_or_null(q_weight, "q_weight", {head_dim}), *kw = f32_or_null(k_weight, "k_weight", {head_dim});
-  const float *co = f32_or_null(cos, "cos", {S, head_dim / 2}), *si = f32_or_null(sin, "sin", {S, head_dim / 2});
-  const float* alpha = f32_or_null(xsa_alpha, "xsa_alpha", {n_heads});
   c10::DeviceGuard guard(x.device());
-  const Tensor qkv = at::linear(x, w_qkv);
+  const Vecs norm = vecs({q_weight, k_weight}, head_dim, "q and k norm weights"), rope = vecs({cos, sin}, S * head_dim, "cos and sin"),
+             alpha = vecs({xsa_alpha}, n_heads, "xsa_alpha");
+  const Tensor qkv = at::linear(x, at::cat({w_q, w_k, w_v}));
+  check_rows(qkv, "q|k|v rows", (int64_t)(n_heads + 2 * n_kv_heads) * head_dim);
   const int ld = (int)qkv.size(-1);
   hipStream_t s = stream_of(x);
-  if (qw != nullptr || kw != nullptr || co != nullptr)
-    check(bibo_moe_exp_qk_norm_rope(qkv.data_ptr(), ld, (int)B, (int)S, n_heads, n_kv_heads, head_dim, qw, kw, (float)eps, co, si, s),
+  if (q_weight.has_value() || k_weight.has_value() || cos.has_value())
+    check(bibo_moe_exp_qk_norm_rope(qkv.data_ptr(), ld, (int)B, (int)S, n_heads, n_kv_heads, head_dim, norm[0], norm[1], norm.dtype,
+                                    (float)eps, rope[0], rope[1], rope.dtype, head_dim, s),
           "bibo_moe_exp_qk_norm_rope");
   const Tensor y = at::empty({B, S, (int64_t)n_heads * head_dim}, x.options());
-  check(bibo_moe_exp_attention_fwd(qkv.data_ptr(), ld, (int)B, (int)S, n_heads, n_kv_heads, head_dim, window, (float)scale, alpha,
-                                   y.data_ptr(), s),
+  check(bibo_moe_exp_attention_fwd(qkv.data_ptr(), ld, (int)B, (int)S, n_heads, n_kv_heads, head_dim, window, (float)scale, alpha[0],
+                                   alpha.dtype, y.data_ptr(), s),
         "bibo_moe_exp_attention_fwd");
   return at::linear(y, w_o);
 }
 
 // (attn_read + theta a, prefix + a or a itself)
 py::tuple exp_carry(const Tensor& attn_read, const Tensor& a, const c10::optional<Tensor>& theta, const c10::optional<Tensor>& prefix) {
+  at::NoGradGuard no_grad;
   const int64_t H = a.size(-1);
   check_rows(attn_read, "attn_read", H);
   check_rows(a, "a", H);
   TORCH_CHECK_VALUE(attn_read.numel() == a.numel(), "attn_read must have the size of a");
-  const float* th = f32_or_null(theta, "theta", {H});
+  c10::DeviceGuard guard(a.device());
+  const Vecs th = vecs({theta}, H, "theta");
   Tensor out = at::empty_like(a), prefix_out;
   if (prefix.has_value()) {
     check_rows(*prefix, "prefix", H);
     TORCH_CHECK_VALUE(prefix->numel() == a.numel(), "prefix must have the size of a");
     prefix_out = at::empty_like(a);
   }
-  c10::DeviceGuard guard(a.device());
-  check(bibo_moe_exp_carry_fwd(attn_read.data_ptr(), a.data_ptr(), th, prefix.has_value() ? prefix->data_ptr() : nullptr,
+  check(bibo_moe_exp_carry_fwd(attn_read.data_ptr(), a.data_ptr(), th[0], th.dtype, prefix.has_value() ? prefix->data_ptr() : nullptr,
                                (int)(a.numel() / H), (int)H, out.data_ptr(), prefix.has_value() ? prefix_out.data_ptr() : nullptr,
                                stream_of(a)),
         "bibo_moe_exp_carry_fwd");
@@ -352,12 +375,13 @@ py::tuple exp_carry(const Tensor& attn_read, const Tensor& a, const c10::optiona
 }
 
 // base + SwiGLU(x): gate and up in one library product, SiLU(gate) * up in one launch, base added by the down product
-Tensor exp_mlp(const Tensor& x, const Tensor& w_gate_up, const Tensor& w_down, const Tensor& base) {
+Tensor exp_mlp(const Tensor& x, const Tensor& w_gate, const Tensor& w_up, const Tensor& w_down, const Tensor& base) {
   at::NoGradGuard no_grad;
-  const int64_t H = x.size(-1), T = x.numel() / H, I = w_gate_up.size(0) / 2;
+  const int64_t H = x.size(-1), T = x.numel() / H, I = w_gate.size(0);
   check_rows(x, "x", H);
   c10::DeviceGuard guard(x.device());
-  const Tensor gu = at::linear(x.view({T, H}), w_gate_up);
+  const Tensor gu = at::linear(x.view({T, H}), at::cat({w_gate, w_up}));        // joined per call, as in exp_attention
+  check_rows(gu, "gate|up rows", 2 * I);
   Tensor h = at::empty({T, I}, x.options());
   check(bibo_moe_exp_silu_mul_fwd(gu.data_ptr(), (int)T, (int)I, h.data_ptr(), stream_of(x)), "bibo_moe_exp_silu_mul_fwd");
   return at::addmm(base.reshape({T, w_down.size(0)}), h, w_down.t()).view_as(base);

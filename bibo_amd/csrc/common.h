@@ -229,17 +229,37 @@ hipError_t launch_gateup_stream(const void* x, const void* wgu, const int32_t* i
 hipError_t launch_down_stream(const void* gu, const void* wd, const float* theta, const float* w, const int32_t* idx,
                               int T, int H, int E, int k, int I, int act, void* hidden, float* yw, hipStream_t s);
 
+// A small parameter vector as its owner holds it: fp32, or bf16 (then 16-byte aligned, checked at the entry points).  Read in
+// place: a widened copy kept between calls would go stale, and one made per call is a launch.  p NULL: absent.
+struct Vec {
+  const void* p;
+  int bf16;
+  __device__ __forceinline__ float operator[](size_t i) const {
+    return bf16 ? (float)static_cast<const bf16_t*>(p)[i] : static_cast<const float*>(p)[i];
+  }
+};
+__device__ __forceinline__ void load8(const Vec& v, size_t at, float (&out)[8]) {      // at: a multiple of 8
+  if (v.bf16) {
+    const bf16x8 r = *reinterpret_cast<const bf16x8*>(static_cast<const bf16_t*>(v.p) + at);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) out[q] = (float)r[q];
+  } else {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) out[q] = static_cast<const float*>(v.p)[at + q];
+  }
+}
+
 bool attn_res_supported(int H, int n_cand, int dtype);
-hipError_t launch_attn_res(const void* const* cands, int n_cand, const float* score_w, float eps, int T, int H, void* out,
-                           const float* norm_w, float norm_eps, void* normed, hipStream_t s);
-hipError_t launch_carry(const void* attn_read, const void* a, const float* theta, const void* prefix, int T, int H, void* hs,
+hipError_t launch_attn_res(const void* const* cands, int n_cand, Vec score_a, Vec score_b, float eps, int T, int H, void* out,
+                           Vec norm_w, float norm_eps, void* normed, hipStream_t s);
+hipError_t launch_carry(const void* attn_read, const void* a, Vec theta, const void* prefix, int T, int H, void* hs,
                         void* prefix_out, hipStream_t s);
 hipError_t launch_silu_mul(const void* gu, int T, int I, void* out, hipStream_t s);
 bool exp_attention_supported(int nq, int nkv, int D);
-hipError_t launch_qk_norm_rope(void* qkv, int ld, int T, int S, int nq, int nkv, int D, const float* qw, const float* kw, float eps,
-                               const float* cos, const float* sin, hipStream_t s);
+hipError_t launch_qk_norm_rope(void* qkv, int ld, int T, int S, int nq, int nkv, int D, Vec qw, Vec kw, float eps, Vec cos, Vec sin,
+                               int ld_rope, hipStream_t s);
 hipError_t launch_exp_attention(const void* qkv, int ld, int B, int S, int nq, int nkv, int D, int window, float scale,
-                                const float* xsa_alpha, void* out, hipStream_t s);
+                                Vec xsa_alpha, void* out, hipStream_t s);
 
 // ---- backward pass (backward.hip) ----
 struct BackwardBuffers {

@@ -19,11 +19,10 @@ __device__ __forceinline__ float row16_sum(float v) {      // sum over a DPP row
 // ---- QK-norm (norm.py:19-24 on head rows) and RoPE (attn/rope.py, rotate-half), in place --------------------------
 // rows of qkv: [T, ld], the nq query heads first, then the nkv key heads, D elements each.  Sixteen lanes per head row; lane
 // c < D / 16 owns elements 8c .. 8c + 7 of the first half and of the second half, i.e. whole rotation pairs.  Memory-bound:
-// one read and one write of the q and k columns.  qw, kw (fp32 [D], or NULL: no norm); cos, sin (fp32 [S, D / 2] or NULL).
+// one read and one write of the q and k columns.  qw, kw: [D], or NULL: no norm; cos, sin: rows of D / 2 at stride ld_rope, or NULL.
 template <int D>
 __global__ __launch_bounds__(256) void qk_norm_rope_kernel(bf16_t* __restrict__ qkv, int ld, int T, int S, int nq, int nkv,
-                                                           const float* __restrict__ qw, const float* __restrict__ kw, float eps,
-                                                           const float* __restrict__ cos, const float* __restrict__ sin) {
+                                                           Vec qw, Vec kw, float eps, Vec cos, Vec sin, int ld_rope) {
   constexpr int kLanes = D / 16;
   const int heads = nq + nkv;
   const long long g = ((long long)blockIdx.x * 256 + threadIdx.x) >> 4;
@@ -40,28 +39,34 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(bf16_t* __restrict__ 
 #pragma unroll
     for (int q = 0; q < 8; ++q) { a[q] = (float)va[q]; b[q] = (float)vb[q]; }
   }
-  const float* w = hd < nq ? qw : kw;
-  if (w != nullptr) {
+  const Vec w = hd < nq ? qw : kw;
+  if (w.p != nullptr) {
     float ss = 0.f;
 #pragma unroll
     for (int q = 0; q < 8; ++q) ss = fmaf(a[q], a[q], fmaf(b[q], b[q], ss));
     const float rinv = rsqrtf(row16_sum(ss) / (float)D + eps);
     if (live) {
+      float wa[8], wb[8];
+      load8(w, c * 8, wa);
+      load8(w, D / 2 + c * 8, wb);
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
-        a[q] = w[c * 8 + q] * (float)(bf16_t)(a[q] * rinv);
-        b[q] = w[D / 2 + c * 8 + q] * (float)(bf16_t)(b[q] * rinv);
+        a[q] = wa[q] * (float)(bf16_t)(a[q] * rinv);
+        b[q] = wb[q] * (float)(bf16_t)(b[q] * rinv);
       }
     }
   }
-  if (!live || (w == nullptr && cos == nullptr)) return;
-  if (cos != nullptr) {
-    const size_t p = (size_t)(t % S) * (D / 2) + c * 8;
+  if (!live || (w.p == nullptr && cos.p == nullptr)) return;
+  if (cos.p != nullptr) {
+    const size_t p = (size_t)(t % S) * ld_rope + c * 8;
+    float co[8], si[8];
+    load8(cos, p, co);
+    load8(sin, p, si);
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-      const float x = a[q], y = b[q], co = cos[p + q], si = sin[p + q];
-      a[q] = x * co - y * si;
-      b[q] = y * co + x * si;
+      const float x = a[q], y = b[q];
+      a[q] = x * co[q] - y * si[q];
+      b[q] = y * co[q] + x * si[q];
     }
   }
   bf16x8 oa, ob;
@@ -95,7 +100,7 @@ template <int D> __device__ __forceinline__ int vswz(int row) { return D == 128 
 template <int D>
 __global__ __launch_bounds__(256, 2) void attention_kernel(const bf16_t* __restrict__ qkv, int ld, int S, int nq, int nkv, int hpw,
                                                            int heads, int nqb, int window, float scale_log2,
-                                                           const float* __restrict__ xsa_alpha, bf16_t* __restrict__ out) {
+                                                           Vec xsa_alpha, bf16_t* __restrict__ out) {
   constexpr int KB = 32, GPR = D / 8, NI = KB * GPR / 256;      // keys per block, granules per row, DMA instructions per operand
   constexpr int DT = D / 32, KS = D / 16;
   static_assert(KB * GPR % 256 == 0, "a block does not divide over the threads");
@@ -225,7 +230,7 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const bf16_t* __restr
   const int qi = q0w + n;
   l += __shfl_xor(l, 32, kWave);
   const float inv = 1.f / l;
-  if (xsa_alpha != nullptr) {
+  if (xsa_alpha.p != nullptr) {
     const bf16_t* vrow = vbase + (size_t)min(qi, S - 1) * ld + 4 * h;
     bf16x4 v[DT][4];
     float vv = 0.f, yv = 0.f;
@@ -273,23 +278,23 @@ bool exp_attention_supported(int nq, int nkv, int D) {
   return (D == 64 || D == 128 || D == 192) && nkv >= 1 && nq % nkv == 0 && (g == 1 || g % 2 == 0);
 }
 
-hipError_t launch_qk_norm_rope(void* qkv, int ld, int T, int S, int nq, int nkv, int D, const float* qw, const float* kw, float eps,
-                               const float* cos, const float* sin, hipStream_t s) {
+hipError_t launch_qk_norm_rope(void* qkv, int ld, int T, int S, int nq, int nkv, int D, Vec qw, Vec kw, float eps, Vec cos, Vec sin,
+                               int ld_rope, hipStream_t s) {
   const long long groups = (long long)T * (nq + nkv);
   if (groups == 0) return hipSuccess;
   const dim3 grid((unsigned)((groups + 15) / 16));
   bf16_t* p = static_cast<bf16_t*>(qkv);
   switch (D) {
-    case 64: hipLaunchKernelGGL(qk_norm_rope_kernel<64>, grid, dim3(256), 0, s, p, ld, T, S, nq, nkv, qw, kw, eps, cos, sin); break;
-    case 128: hipLaunchKernelGGL(qk_norm_rope_kernel<128>, grid, dim3(256), 0, s, p, ld, T, S, nq, nkv, qw, kw, eps, cos, sin); break;
-    case 192: hipLaunchKernelGGL(qk_norm_rope_kernel<192>, grid, dim3(256), 0, s, p, ld, T, S, nq, nkv, qw, kw, eps, cos, sin); break;
+    case 64: hipLaunchKernelGGL(qk_norm_rope_kernel<64>, grid, dim3(256), 0, s, p, ld, T, S, nq, nkv, qw, kw, eps, cos, sin, ld_rope); break;
+    case 128: hipLaunchKernelGGL(qk_norm_rope_kernel<128>, grid, dim3(256), 0, s, p, ld, T, S, nq, nkv, qw, kw, eps, cos, sin, ld_rope); break;
+    case 192: hipLaunchKernelGGL(qk_norm_rope_kernel<192>, grid, dim3(256), 0, s, p, ld, T, S, nq, nkv, qw, kw, eps, cos, sin, ld_rope); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
 
 hipError_t launch_exp_attention(const void* qkv, int ld, int B, int S, int nq, int nkv, int D, int window, float scale,
-                                const float* xsa_alpha, void* out, hipStream_t s) {
+                                Vec xsa_alpha, void* out, hipStream_t s) {
   if (B == 0 || S == 0) return hipSuccess;
   const int g = nq / nkv;
   const int hpw = g % 4 == 0 ? 4 : (g % 2 == 0 ? 2 : 1);

@@ -80,7 +80,7 @@ __global__ __launch_bounds__(256) void rmsnorm_bf16x8_kernel(const bf16_t* __res
 
 // Depth mix of Block Attention Residuals (apply_attention_residual, exp/modeling_bibo.py:119-232, softmax scores,
 // dense): candidates = the completed block representatives and the running prefix sum of a token; score of a
-// candidate = rsqrt(mean(c^2) + eps) * <c, score_w> with score_w = norm weight * pseudo-query (fp32); out = the
+// candidate = rsqrt(mean(c^2) + eps) * <c, score_a * score_b> (norm weight and pseudo-query; their product in fp32); out = the
 // candidates averaged with the softmax of their scores, fp32, rounded once.  With `normed`, the RMSNorm of the rounded row
 // that the attention behind it reads (input_layernorm) leaves with it.  One wave per token, all N candidate rows
 // requested at once and kept in registers (two 16-byte granules per lane: H <= 1024): bound by memory.
@@ -90,8 +90,8 @@ struct AttnResPtrs {
 };
 
 template <int N>
-__global__ __launch_bounds__(256) void attn_res_kernel(AttnResPtrs cand, const float* __restrict__ score_w, float eps, int T, int H,
-                                                       bf16_t* __restrict__ out, const float* __restrict__ norm_w, float norm_eps,
+__global__ __launch_bounds__(256) void attn_res_kernel(AttnResPtrs cand, Vec score_a, Vec score_b, float eps, int T, int H,
+                                                       bf16_t* __restrict__ out, Vec norm_w, float norm_eps,
                                                        bf16_t* __restrict__ normed) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -114,9 +114,16 @@ __global__ __launch_bounds__(256) void attn_res_kernel(AttnResPtrs cand, const f
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     const int c = u * kWave + lane;
-    float sw[8];
+    float sw[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (c < nchunk) {
+      load8(score_a, c * 8, sw);
+      if (score_b.p != nullptr) {
+        float sb[8];
+        load8(score_b, c * 8, sb);
 #pragma unroll
-    for (int q = 0; q < 8; ++q) sw[q] = c < nchunk ? score_w[c * 8 + q] : 0.f;
+        for (int q = 0; q < 8; ++q) sw[q] *= sb[q];
+      }
+    }
 #pragma unroll
     for (int i = 0; i < N; ++i)
 #pragma unroll
@@ -165,8 +172,10 @@ __global__ __launch_bounds__(256) void attn_res_kernel(AttnResPtrs cand, const f
     const int c = u * kWave + lane;
     if (c < nchunk) {
       bf16x8 w;
+      float nw[8];
+      load8(norm_w, c * 8, nw);
 #pragma unroll
-      for (int q = 0; q < 8; ++q) w[q] = (bf16_t)(norm_w[c * 8 + q] * (float)(bf16_t)((float)o[u][q] * rinv));   // norm.py:24
+      for (int q = 0; q < 8; ++q) w[q] = (bf16_t)(nw[q] * (float)(bf16_t)((float)o[u][q] * rinv));   // norm.py:24
       reinterpret_cast<bf16x8*>(normed + (size_t)row * H)[c] = w;
     }
   }
@@ -175,15 +184,17 @@ __global__ __launch_bounds__(256) void attn_res_kernel(AttnResPtrs cand, const f
 // The two sums behind an attention block (exp/modeling_bibo.py:526-531,640-648), 8 elements per thread: hs = attn_read +
 // theta a (theta NULL: a), and prefix_out = prefix + a where the block has a prefix already.
 __global__ __launch_bounds__(256) void carry_kernel(const bf16_t* __restrict__ attn_read, const bf16_t* __restrict__ a,
-                                                    const float* __restrict__ theta, const bf16_t* __restrict__ prefix,
+                                                    Vec theta, const bf16_t* __restrict__ prefix,
                                                     long long n8, int H8, bf16_t* __restrict__ hs, bf16_t* __restrict__ prefix_out) {
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= n8) return;
   const int c = (int)(i % H8);
   const bf16x8 av = reinterpret_cast<const bf16x8*>(a)[i], rv = reinterpret_cast<const bf16x8*>(attn_read)[i];
+  float th[8] = {1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f};
+  if (theta.p != nullptr) load8(theta, c * 8, th);
   bf16x8 o;
 #pragma unroll
-  for (int q = 0; q < 8; ++q) o[q] = (bf16_t)fmaf(theta != nullptr ? theta[c * 8 + q] : 1.f, (float)av[q], (float)rv[q]);
+  for (int q = 0; q < 8; ++q) o[q] = (bf16_t)fmaf(th[q], (float)av[q], (float)rv[q]);
   reinterpret_cast<bf16x8*>(hs)[i] = o;
   if (prefix != nullptr) {
     const bf16x8 pv = reinterpret_cast<const bf16x8*>(prefix)[i];
@@ -214,13 +225,13 @@ bool attn_res_supported(int H, int n_cand, int dtype) {
   return dtype == BIBO_DTYPE_BF16 && H % 8 == 0 && H <= 1024 && n_cand >= 1 && n_cand <= kAttnResMaxCand;
 }
 
-hipError_t launch_attn_res(const void* const* cands, int n_cand, const float* score_w, float eps, int T, int H, void* out,
-                           const float* norm_w, float norm_eps, void* normed, hipStream_t s) {
+hipError_t launch_attn_res(const void* const* cands, int n_cand, Vec score_a, Vec score_b, float eps, int T, int H, void* out,
+                           Vec norm_w, float norm_eps, void* normed, hipStream_t s) {
   if (T == 0) return hipSuccess;
   AttnResPtrs p;
   for (int i = 0; i < kAttnResMaxCand; ++i) p.c[i] = static_cast<const bf16_t*>(i < n_cand ? cands[i] : cands[0]);
   auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3((T + 3) / 4), dim3(256), 0, s, p, score_w, eps, T, H, static_cast<bf16_t*>(out), norm_w, norm_eps,
+    hipLaunchKernelGGL(kernel, dim3((T + 3) / 4), dim3(256), 0, s, p, score_a, score_b, eps, T, H, static_cast<bf16_t*>(out), norm_w, norm_eps,
                        static_cast<bf16_t*>(normed));
   };
   switch (n_cand) {
@@ -237,7 +248,7 @@ hipError_t launch_attn_res(const void* const* cands, int n_cand, const float* sc
   return hipGetLastError();
 }
 
-hipError_t launch_carry(const void* attn_read, const void* a, const float* theta, const void* prefix, int T, int H, void* hs,
+hipError_t launch_carry(const void* attn_read, const void* a, Vec theta, const void* prefix, int T, int H, void* hs,
                         void* prefix_out, hipStream_t s) {
   const long long n8 = (long long)T * H / 8;
   if (n8 == 0) return hipSuccess;

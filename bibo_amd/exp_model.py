@@ -99,21 +99,15 @@ def _hip_ok(x) -> bool:
     return x.is_cuda and x.dtype == torch.bfloat16 and not (torch.is_grad_enabled() and x.requires_grad)
 
 
-def _derived(module, key, params, make):
-    """make() from parameters, kept in `module` until one of them changes (storage address or version counter; the cache
-    holds the tensors, so an address cannot pass to another one meanwhile)."""
-    tag = tuple((p.data_ptr(), p._version, p.device) for p in params)
-    hit = module.__dict__.get("_derived_" + key)
-    if hit is None or hit[0] != tag:
-        with torch.no_grad():
-            hit = module.__dict__["_derived_" + key] = (tag, make(), params)
-    return hit[1]
-
-
 def _fp32_copy(module, name):
-    """fp32 copy of a small parameter."""
+    """fp32 copy of a small parameter, refreshed when the parameter changes (storage address or version counter)."""
     p = getattr(module, name)
-    return _derived(module, name, (p,), lambda: p.detach().float().contiguous())
+    tag = (p.data_ptr(), p._version, p.device)
+    hit = module.__dict__.get("_fp32_" + name)
+    if hit is None or hit[0] != tag:
+        hit = (tag, p.detach().float().contiguous())
+        module.__dict__["_fp32_" + name] = hit
+    return hit[1]
 
 
 def _plain(*modules) -> bool:
@@ -124,17 +118,15 @@ def _plain(*modules) -> bool:
 
 
 def _native_ok(x) -> bool:
-    """bf16 rows on the GPU with autograd off: what the native launches around the block take."""
-    return x.is_cuda and x.dtype == torch.bfloat16 and not torch.is_grad_enabled() and x.is_contiguous()
+    """bf16 rows on the GPU with autograd off, products in bf16: what the native launches around the block take."""
+    return (x.is_cuda and x.dtype == torch.bfloat16 and not torch.is_grad_enabled() and x.is_contiguous()
+            and x.data_ptr() % 16 == 0
+            and not (torch.is_autocast_enabled() and torch.get_autocast_dtype("cuda") != torch.bfloat16))
 
 
 def _rotate_half(x):
     h = x.shape[-1] // 2
     return torch.cat((-x[..., h:], x[..., :h]), dim=-1)
-
-
-def _score_weight(module, proj_w, norm_w):
-    return _derived(module, "score", (proj_w, norm_w), lambda: (norm_w.float() * proj_w.reshape(-1).float()).contiguous())
 
 
 def attention_residual(prefix, blocks, proj_w, norm_w, eps):
@@ -207,15 +199,10 @@ class BiBoExpAttention(nn.Module):
         if not (_native_ok(x) and d in (64, 128, 192) and (nh == nkv or (nh // nkv) % 2 == 0)
                 and all(p.weight.dtype == torch.bfloat16 for p in projs) and _plain(*projs, self.q_norm, self.k_norm)):
             return None
-        ws = (self.q_proj.weight, self.k_proj.weight, self.v_proj.weight)
-        w_qkv = _derived(self, "qkv", ws, lambda: torch.cat(ws, 0).contiguous())
-        half = (None, None)
-        if self.is_swa:                                                         # base.py:87-91
-            half = _derived(self, "rope", (cos, sin), lambda: tuple(t[:, :d // 2].float().contiguous() for t in (cos, sin)))
-        return L.native().exp_attention(x, w_qkv, self.o_proj.weight, _fp32_copy(self.q_norm, "weight") if normed else None,
-                                        _fp32_copy(self.k_norm, "weight") if normed else None,
-                                        self.q_norm.variance_epsilon if normed else 0.0, *half,
-                                        None if self.xsa_alpha is None else _fp32_copy(self, "xsa_alpha"), nh, nkv, d,
+        rope = (cos, sin) if self.is_swa else (None, None)                      # base.py:87-91
+        return L.native().exp_attention(x, *(p.weight for p in projs), self.q_norm.weight if normed else None,
+                                        self.k_norm.weight if normed else None,
+                                        self.q_norm.variance_epsilon if normed else 0.0, *rope, self.xsa_alpha, nh, nkv, d,
                                         self.sliding_window or 0, self.scaling)
 
     def forward(self, x, cos, sin):
@@ -263,9 +250,7 @@ class BiBoExpMLP(nn.Module):
         projs = (self.gate_proj, self.up_proj, self.down_proj)
         if (_native_ok(x) and x.dtype == base.dtype and self.gate_proj.weight.shape[0] % 8 == 0
                 and all(p.weight.dtype == torch.bfloat16 for p in projs) and _plain(self, *projs)):
-            ws = (self.gate_proj.weight, self.up_proj.weight)
-            return L.native().exp_mlp(x, _derived(self, "gate_up", ws, lambda: torch.cat(ws, 0).contiguous()),
-                                      self.down_proj.weight, base)
+            return L.native().exp_mlp(x, *(p.weight for p in projs), base)
         return base + self(x)
 
 
@@ -298,9 +283,8 @@ class BiBoExpDecoderLayer(nn.Module):
             if native and _plain(res, self.self_attention_res_proj, self.input_layernorm):
                 ln = self.input_layernorm
                 hs, xn = L.native().exp_attn_res_norm(
-                    [*(b.view(B, S, H) for b in blocks), prefix],
-                    _score_weight(self, self.self_attention_res_proj.weight, res.weight), res.variance_epsilon,
-                    _fp32_copy(ln, "weight"), ln.variance_epsilon)
+                    [*(b.contiguous().view(B, S, H) for b in blocks), prefix], res.weight, self.self_attention_res_proj.weight,
+                    res.variance_epsilon, ln.weight, ln.variance_epsilon)
             else:
                 hs = attention_residual(prefix.reshape(-1, H), blocks, self.self_attention_res_proj.weight, res.weight,
                                         res.variance_epsilon).view(B, S, H)
@@ -311,8 +295,7 @@ class BiBoExpDecoderLayer(nn.Module):
         a = self.self_attn(self.input_layernorm(hs) if xn is None else xn, cos, sin)
         theta = self.attn_res_carry_theta
         if native and a.is_contiguous() and a.dtype == hidden_states.dtype:     # carry write (:640-648)
-            th = (None if theta is None else
-                  _derived(self, "carry", (theta,), lambda: theta.detach().float().to(a.dtype).float().expand(H).contiguous()))
+            th = None if theta is None else theta.to(a.dtype).expand(H)
             hs, prefix = L.native().exp_carry(attn_read, a, th, prefix)
         else:
             prefix = a if prefix is None else prefix + a
@@ -367,34 +350,20 @@ class BiBoExpModel(nn.Module):
         h = self.embed_tokens(input_ids)
         if self.config.bf16_residual_stream:                                    # exp/modeling_bibo.py:858-859
             h = h.to(torch.bfloat16)
-        cos, sin = self._rope_tables(S, h)
+        ang = torch.arange(S, device=h.device, dtype=torch.float32)[:, None] * self.inv_freq.float()[None, :]
+        ang = torch.cat((ang, ang), dim=-1)
+        cos, sin = ang.cos().to(h.dtype), ang.sin().to(h.dtype)                 # embed.py:63-74
         blocks = []
         for layer in self.layers:
             h, blocks = layer(h, blocks, cos, sin, collect_routing)
         res = self.output_attn_res_norm                                         # :916-920
         if (_native_ok(h) and H % 8 == 0 and H <= 1024 and len(blocks) < 8 and _plain(res, self.output_attn_res_proj, self.norm)):
-            return L.native().exp_attn_res_norm([*(b.view(B, S, H) for b in blocks), h],
-                                                _score_weight(self, self.output_attn_res_proj.weight, res.weight),
-                                                res.variance_epsilon, _fp32_copy(self.norm, "weight"),
+            return L.native().exp_attn_res_norm([*(b.contiguous().view(B, S, H) for b in blocks), h], res.weight,
+                                                self.output_attn_res_proj.weight, res.variance_epsilon, self.norm.weight,
                                                 self.norm.variance_epsilon)[1]
         h = attention_residual(h.reshape(-1, H), blocks, self.output_attn_res_proj.weight, res.weight,
                                res.variance_epsilon).view(B, S, H)
         return self.norm(h)
-
-    def _rope_tables(self, S, h):
-        """cos and sin [S, head_dim] in the stream's dtype (embed.py:63-74); those of the last sequence length are kept."""
-        def make():
-            ang = torch.arange(S, device=h.device, dtype=torch.float32)[:, None] * self.inv_freq.float()[None, :]
-            ang = torch.cat((ang, ang), dim=-1)
-            return ang.cos().to(h.dtype), ang.sin().to(h.dtype)
-        if torch.is_grad_enabled():
-            return make()
-        kept = self.__dict__.get("_rope_kept")
-        key = (S, h.dtype, h.device)
-        if kept is None or kept[0] != key:
-            self.__dict__["_rope_kept"] = (key,)
-            self.__dict__.pop("_derived_tables", None)
-        return _derived(self, "tables", (self.inv_freq,), make)
 
 
 class BiBoExpForCausalLM(nn.Module):

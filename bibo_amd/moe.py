@@ -491,19 +491,8 @@ class BiBoMoELayer(nn.Module):
         flags = L.FLAG_ROUND_BLOCK_OUT if bf16_moe_out else 0
         if residual is False:
             flags, residual = flags | L.FLAG_NO_RESIDUAL, None
-        out, counts = L.native().ffn_forward(hidden_states, self._norm_weight(norm_weight), float(eps), residual, *operands,
+        out, counts = L.native().ffn_forward(hidden_states, norm_weight, float(eps), residual, *operands,
                                              self.num_experts_per_tok, norm, algo, e.num_pos, e.num_neg, act, flags, balancing)
         if balancing:                                          # exactly once per training forward
             self._balance(counts, num_tokens)
         return out.to(torch.bfloat16) if bf16_stream else out
-
-    def _norm_weight(self, w):
-        """fp32 copy of the caller's norm weight; a parameter's copy is kept until the parameter changes."""
-        if w.dtype == torch.float32 and w.is_contiguous():
-            return w
-        if not isinstance(w, nn.Parameter):
-            return w.detach().float().contiguous()
-        hit = self.__dict__.get("_norm_copy")
-        if hit is None or hit[0] is not w or hit[1] != (w._version, w.data_ptr()):
-            hit = self.__dict__["_norm_copy"] = (w, (w._version, w.data_ptr()), w.detach().float().contiguous())
-        return hit[2]

@@ -354,31 +354,33 @@ int bibo_moe_exp_attn_res_fwd(const void* const* candidates, int n_candidates, c
                           int dtype, void* out, void* stream);
 
 /*
- * Further caller-side kernels of the 10-layer forward; bf16 rows, 16-byte aligned.
+ * Further caller-side kernels of the 10-layer forward; bf16 rows, 16-byte aligned.  The small
+ * parameter vectors are fp32 or bf16 (then 16-byte aligned too), as the dtype beside them says, and used in fp32.
  *
- * bibo_moe_exp_attn_res_norm_fwd: the depth mix above, and in `normed` (or NULL) also norm_weight * round(out *
+ * bibo_moe_exp_attn_res_norm_fwd: the depth mix above with score_weight = score_a * score_b (score_b NULL: score_a), and in `normed` (or NULL) also norm_weight * round(out *
  *   rsqrt(mean(out^2) + norm_eps)), the RMSNorm (src/modeling/norm.py:19-24) of the mixed row.
- * bibo_moe_exp_carry_fwd: hs = attn_read + theta * a (theta fp32 [H] or NULL for 1) and, with `prefix` given, prefix_out =
+ * bibo_moe_exp_carry_fwd: hs = attn_read + theta * a (theta [H] or NULL for 1) and, with `prefix` given, prefix_out =
  *   prefix + a (exp/modeling_bibo.py:526-531,640-648).  H % 8 == 0.
  * bibo_moe_exp_silu_mul_fwd: out[t] = SiLU(gate) * up of rows [gate (I) | up (I)] (src/modeling/ffn/mlp.py:34-35).  I % 8 == 0.
  * bibo_moe_exp_qk_norm_rope: in place on rows [q heads | k heads | v heads] (row stride ld elements) of B x S tokens: RMSNorm
- *   per query and key head (q_weight, k_weight fp32 [head_dim], NULL: none), then the rotate-half RoPE (cos, sin fp32
- *   [S, head_dim / 2], NULL: none) (src/modeling/attn/base.py:70-91).
+ *   per query and key head (q_weight, k_weight [head_dim], NULL: none), then the rotate-half RoPE (cos, sin: the first
+ *   head_dim / 2 entries of S rows at stride ld_rope, a multiple of 8; NULL: none) (src/modeling/attn/base.py:70-91).
  * bibo_moe_exp_attention_fwd: out [B*S, n_heads * head_dim] = causal attention of those rows (window > 0: restricted to the
- *   last `window` keys), softmax in fp32, with the XSA correction y - tanh(alpha) <y, vn> vn (xsa_alpha fp32 [n_heads] or NULL;
+ *   last `window` keys), softmax in fp32, with the XSA correction y - tanh(alpha) <y, vn> vn (xsa_alpha [n_heads] or NULL;
  *   src/modeling/attn/xsa.py:41-54).  head_dim in {64, 128, 192}; n_heads / n_kv_heads = 1 or even (BIBO_ERR_UNSUPPORTED
  *   otherwise).
  */
-int bibo_moe_exp_attn_res_norm_fwd(const void* const* candidates, int n_candidates, const float* score_weight, float eps,
-                                   const float* norm_weight, float norm_eps, int T, int H, int dtype, void* out, void* normed,
-                                   void* stream);
-int bibo_moe_exp_carry_fwd(const void* attn_read, const void* a, const float* theta, const void* prefix, int T, int H, void* hs,
-                           void* prefix_out, void* stream);
+int bibo_moe_exp_attn_res_norm_fwd(const void* const* candidates, int n_candidates, const void* score_a, const void* score_b,
+                                   float eps, const void* norm_weight, float norm_eps, int weight_dtype, int T, int H, int dtype,
+                                   void* out, void* normed, void* stream);
+int bibo_moe_exp_carry_fwd(const void* attn_read, const void* a, const void* theta, int theta_dtype, const void* prefix, int T, int H,
+                           void* hs, void* prefix_out, void* stream);
 int bibo_moe_exp_silu_mul_fwd(const void* gate_up, int T, int I, void* out, void* stream);
-int bibo_moe_exp_qk_norm_rope(void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, const float* q_weight,
-                              const float* k_weight, float eps, const float* cos, const float* sin, void* stream);
+int bibo_moe_exp_qk_norm_rope(void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, const void* q_weight,
+                              const void* k_weight, int weight_dtype, float eps, const void* cos, const void* sin, int rope_dtype,
+                              int ld_rope, void* stream);
 int bibo_moe_exp_attention_fwd(const void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, int window,
-                               float scale, const float* xsa_alpha, void* out, void* stream);
+                               float scale, const void* xsa_alpha, int alpha_dtype, void* out, void* stream);
 
 #ifdef __cplusplus
 }

@@ -39,7 +39,7 @@ def test_attention(D, nq, nkv, S, window):
     scale = D ** -0.5
     d = qkv.to(DEV)
     dev = [t.to(DEV).contiguous() for t in (qw, kw, cos, sin, alpha)]
-    _call("bibo_moe_exp_qk_norm_rope", _ptr(d), ld, B, S, nq, nkv, D, _ptr(dev[0]), _ptr(dev[1]), ctypes.c_float(1e-6), _ptr(dev[2]), _ptr(dev[3]))
+    _call("bibo_moe_exp_qk_norm_rope", _ptr(d), ld, B, S, nq, nkv, D, _ptr(dev[0]), _ptr(dev[1]), 1, ctypes.c_float(1e-6), _ptr(dev[2]), _ptr(dev[3]), 1, D // 2)
     x = qkv.float()
 
     def heads(lo, n):
@@ -62,7 +62,7 @@ def test_attention(D, nq, nkv, S, window):
     allow = (i[None] <= i[:, None]) & ((i[:, None] - i[None] < window) if window else True)
     for xsa in (None, dev[4]):
         out = torch.full((B, S, nq * D), float("nan"), dtype=torch.bfloat16, device=DEV)
-        _call("bibo_moe_exp_attention_fwd", _ptr(d), ld, B, S, nq, nkv, D, window, ctypes.c_float(scale), _ptr(xsa), _ptr(out))
+        _call("bibo_moe_exp_attention_fwd", _ptr(d), ld, B, S, nq, nkv, D, window, ctypes.c_float(scale), _ptr(xsa), 1, _ptr(out))
         y = torch.empty(B, S, nq, D)
         for h in range(nq):
             p = (q[:, :, h] @ k[:, :, h // rep].transpose(1, 2).contiguous() * scale).masked_fill(~allow, -torch.inf).softmax(-1)
@@ -74,7 +74,7 @@ def test_attention(D, nq, nkv, S, window):
 
 
 def test_attention_refuses_what_it_does_not_take():
-    args = lambda nq, nkv, D: (None, 4096, 1, 4, nq, nkv, D, 0, ctypes.c_float(1.0), None, None, None)
+    args = lambda nq, nkv, D: (None, 4096, 1, 4, nq, nkv, D, 0, ctypes.c_float(1.0), None, 1, None, None)
     for nq, nkv, D in ((4, 2, 96), (3, 2, 64), (3, 1, 64), (4, 0, 64)):
         assert L.lib().bibo_moe_exp_attention_fwd(*args(nq, nkv, D)) == -6
     assert L.lib().bibo_moe_exp_attention_fwd(*args(4, 2, 64)) == -1
@@ -88,13 +88,13 @@ def test_depth_mix_carry_and_swiglu(T, H):
     for n in (1, 2, 5, 8):
         cands = [rows() for _ in range(n)]
         dc = [c.to(DEV) for c in cands]
-        mixed, normed = L.native().exp_attn_res_norm(dc, sw.to(DEV), 1e-6, nw.to(DEV), 1e-6)
+        mixed, normed = L.native().exp_attn_res_norm(dc, sw.to(DEV), None, 1e-6, nw.to(DEV), 1e-6)
         v = torch.stack([c.float() for c in cands], 1)
         ref = (((v @ sw) * torch.rsqrt(v.pow(2).mean(-1) + 1e-6)).softmax(-1)[..., None] * v).sum(1)
         assert _rel(mixed, ref) <= 8e-3
         m = mixed.cpu().float()
         assert _rel(normed, (m * torch.rsqrt(m.pow(2).mean(-1, keepdim=True) + 1e-6)) * nw) <= 1.2e-2
-        assert torch.equal(L.native().exp_attn_res_norm(dc, sw.to(DEV), 1e-6, None, 0.0)[0], mixed)
+        assert torch.equal(L.native().exp_attn_res_norm(dc, sw.to(DEV), None, 1e-6, None, 0.0)[0], mixed)
     r, a, p = rows(), rows(), rows()
     hs, prefix = L.native().exp_carry(r.to(DEV), a.to(DEV), theta.to(DEV), p.to(DEV))
     assert _rel(hs, r.float() + theta * a.float()) <= 8e-3 and torch.equal(prefix.cpu(), p + a)

@@ -1,0 +1,99 @@
+"""The 10-layer forward keeps nothing between calls: parameters written through `.data`, another sequence length, inference
+mode, autocast and graph replays all see the values of their own call; vectors in bf16 give the bits of their fp32 copies."""
+import pytest
+import torch
+
+from bibo_amd import _lib as L
+from bibo_amd import exp_model as X
+from test_exp_model import randomize
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+def _model(seed=0):
+    cfg = X.BiBoExpConfig(vocab_size=97, hidden_size=256, num_hidden_layers=4, num_attention_heads=4, num_key_value_heads=2,
+                          intermediate_size=256, moe_intermediate_size=128, num_routed_experts=8, num_experts_per_tok=2,
+                          sliding_window=16, mlp_only_layers=(0, 3))
+    model = randomize(X.BiBoExpForCausalLM(cfg), seed).to(DEV, torch.bfloat16).eval()
+    return model
+
+
+def _ids(B, S, seed):
+    return torch.randint(0, 97, (B, S), generator=torch.Generator().manual_seed(seed)).to(DEV)
+
+
+@torch.no_grad()
+def test_writes_through_data_are_seen():
+    model, ids = _model(), _ids(2, 40, 1)
+    before = model(ids)
+    new = _model(seed=5)
+    for p, q in zip(model.parameters(), new.parameters()):
+        p.data.copy_(q)
+    for m in model.modules():                       # what the layers keep in kernel dtype, and row norms, are told of it
+        if hasattr(m, "refresh_weights"):
+            m.refresh_weights()
+        if isinstance(m, X.RMSNorm):
+            m.__dict__.pop("_fp32_weight", None)
+    after = model(ids)
+    assert not torch.equal(before, after) and torch.equal(after, new(ids))
+
+
+def test_inference_mode_sequence_lengths_and_autocast():
+    model = _model()
+    want = {}
+    with torch.no_grad():
+        for S in (40, 17):
+            want[S] = model(_ids(2, S, S))
+    with torch.inference_mode():
+        for S in (40, 17, 40):
+            assert torch.equal(model(_ids(2, S, S)), want[S])
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        assert torch.equal(model(_ids(2, 40, 40)), want[40])
+
+
+@torch.no_grad()
+def test_replays_after_calls_of_another_length():
+    model, ids, other = _model(), _ids(2, 40, 1), _ids(1, 65, 2)
+    side = torch.cuda.Stream(device=DEV)
+    side.wait_stream(torch.cuda.current_stream(DEV))
+    with torch.cuda.stream(side):
+        model(ids)
+    side.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = model(ids)
+    for seed in (3, 4, 3):
+        ids.copy_(_ids(2, 40, seed))
+        model(other)                                # tables of another length in between
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, model(ids))
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("H,S", [(256, 33), (768, 5)])
+def test_bf16_vectors_give_the_bits_of_their_fp32_copies(H, S):
+    g = torch.Generator().manual_seed(H + S)
+    r = lambda *s: torch.randn(*s, generator=g).to(DEV, torch.bfloat16)
+    nat, d, nh, nkv = L.native(), H // 4, 4, 2
+    cands, a, b, w = [r(1, S, H) for _ in range(3)], r(H), r(1, H), r(H)
+    odd = r(H + 1)[1:]                              # a view no 16-byte load may read
+    full = lambda t: None if t is None else t.float()
+    for x, y, z in ((a, b, w), (a, None, w), (odd, b, w), (a, b, None)):
+        for got, ref in zip(nat.exp_attn_res_norm(cands, x, y, 1e-6, z, 1e-6),
+                            nat.exp_attn_res_norm(cands, full(x), full(y), 1e-6, full(z), 1e-6)):
+            assert got is ref or torch.equal(got, ref)
+    product = (a.float() * b.float().view(-1)).contiguous()
+    assert torch.equal(nat.exp_attn_res_norm(cands, a, b, 1e-6, None, 0.0)[0], nat.exp_attn_res_norm(cands, product, None, 1e-6, None, 0.0)[0])
+    for th in (a, odd):
+        assert all(torch.equal(p, q) for p, q in zip(nat.exp_carry(cands[0], cands[1], th, cands[2]),
+                                                     nat.exp_carry(cands[0], cands[1], th.float(), cands[2])))
+    x, wq, wk, wv, wo = r(2, S, H), r(nh * d, H), r(nkv * d, H), r(nkv * d, H), r(H, nh * d)
+    qw, kw, alpha = r(d), r(d), r(nh)
+    cos, sin = r(S, d), r(S, d)
+    vecs = (qw, kw, 1e-6, cos, sin, alpha)
+    one = nat.exp_attention(x, wq, wk, wv, wo, *vecs, nh, nkv, d, 0, d ** -0.5)
+    two = nat.exp_attention(x, wq, wk, wv, wo, *(v.float() if torch.is_tensor(v) else v for v in vecs), nh, nkv, d, 0, d ** -0.5)
+    assert torch.equal(one, two)
