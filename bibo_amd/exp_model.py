@@ -111,10 +111,12 @@ def _fp32_copy(module, name):
 
 
 def _plain(*modules) -> bool:
-    """None of the modules' own calls is observed: their work may be done inside another launch."""
+    """The modules are the ones built here and nobody observes their own calls: their work may be done inside another launch.
+    A wrapped or subclassed projection (an adapter, a parametrization), a replaced forward and hooks run as modules."""
     g = nn.modules.module
-    return not (g._global_forward_hooks or g._global_forward_pre_hooks
-                or any(m._forward_hooks or m._forward_pre_hooks for m in modules))
+    return not (g._global_forward_hooks or g._global_forward_pre_hooks) and all(
+        type(m) in (nn.Linear, RMSNorm, nn.Identity, BiBoExpMLP) and not m._forward_hooks and not m._forward_pre_hooks
+        and "forward" not in m.__dict__ and m._parameters.get("bias") is None for m in modules)
 
 
 def _native_ok(x) -> bool:

@@ -73,6 +73,26 @@ def test_replays_after_calls_of_another_length():
 
 
 @torch.no_grad()
+@pytest.mark.parametrize("name", ["self_attn.q_proj", "self_attn.o_proj", "self_attn.k_norm", "input_layernorm", "mlp.up_proj"])
+@pytest.mark.parametrize("how", ["forward", "subclass", "hook"])
+def test_replaced_and_observed_modules_are_called(name, how):
+    model, ids, seen = _model(), _ids(2, 20, 1), []
+    layer = model.model.layers[3 if "mlp" in name else 1]
+    module = layer.get_submodule(name)
+    model(ids)
+    if how == "forward":
+        plain = module.forward
+        module.forward = lambda x: seen.append(1) or plain(x)
+    elif how == "subclass":
+        base = type(module)
+        module.__class__ = type("Wrapped", (base,), {"forward": lambda self, x: seen.append(1) or base.forward(self, x)})
+    else:
+        module.register_forward_hook(lambda *a: seen.append(1))
+    model(ids)
+    assert seen == [1]
+
+
+@torch.no_grad()
 @pytest.mark.parametrize("H,S", [(256, 33), (768, 5)])
 def test_bf16_vectors_give_the_bits_of_their_fp32_copies(H, S):
     g = torch.Generator().manual_seed(H + S)
