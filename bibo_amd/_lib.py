@@ -14,7 +14,7 @@ NORM_NONE, NORM_SUM, NORM_SOFTMAX = 0, 1, 2
 ALGO_AUTO, ALGO_GENERIC, ALGO_MFMA, ALGO_STREAM, ALGO_FUSED = 0, 1, 2, 3, 4
 MAX_EXPERTS, MAX_TOPK = 64, 8
 ACT_RADIAL_SIGMOID, ACT_RADIAL_TANH, ACT_SILU = 0, 1, 2
-FLAG_ROUND_BLOCK_OUT, FLAG_NO_RESIDUAL, FLAG_GRAD_F32, FLAG_TRAIN_AUTO = 1, 2, 4, 8
+FLAG_ROUND_BLOCK_OUT, FLAG_NO_RESIDUAL, FLAG_GRAD_F32, FLAG_TRAIN_AUTO, FLAG_NORM_BF16 = 1, 2, 4, 8, 16
 ABI_VERSION = 3
 
 # every symbol include/bibo_moe.h declares
@@ -26,7 +26,7 @@ SYMBOLS = (
     "bibo_moe_train_state_bytes", "bibo_moe_forward_train", "bibo_moe_backward_saved",
     "bibo_moe_exp_attn_res_fwd", "bibo_moe_balance_step",
     "bibo_moe_exp_attn_res_norm_fwd", "bibo_moe_exp_carry_fwd", "bibo_moe_exp_silu_mul_fwd", "bibo_moe_exp_qk_norm_rope",
-    "bibo_moe_exp_attention_fwd",
+    "bibo_moe_exp_attention_fwd", "bibo_moe_exp_rope_tables",
 )
 STATIC_SCRATCH_BYTES = 16 << 20
 
@@ -96,6 +96,7 @@ def _declare(l):
                        ("bibo_moe_exp_carry_fwd", [vp, vp, vp, ci, vp, ci, ci, vp, vp, vp]),
                        ("bibo_moe_exp_silu_mul_fwd", [vp, ci, ci, vp, vp]),
                        ("bibo_moe_exp_qk_norm_rope", [vp, ci, ci, ci, ci, ci, ci, vp, vp, ci, cf, vp, vp, ci, ci, vp]),
+                       ("bibo_moe_exp_rope_tables", [vp, ci, ci, ci, vp, vp, vp]),
                        ("bibo_moe_exp_attention_fwd", [vp, ci, ci, ci, ci, ci, ci, ci, cf, vp, ci, vp, vp])):
         getattr(l, name).restype, getattr(l, name).argtypes = ci, args
     l.bibo_moe_balance_step.restype = ci

@@ -284,7 +284,7 @@ TrainState carve_state(int T, int E, int k, int I) {
 int forward_impl(const void* x, const void* w_router, const float* bias, const void* w_gate_up, const void* w_down,
                  const float* theta, const bibo_moe_shape* sh, int norm_mode, int algo, const void* residual, void* out,
                  int32_t* idx_out, float* w_out, int32_t* counts_out, float* logits_out, void* workspace,
-                 size_t workspace_bytes, void* stream, const void* norm_src = nullptr, const float* norm_weight = nullptr,
+                 size_t workspace_bytes, void* stream, const void* norm_src = nullptr, Vec norm_weight = Vec{nullptr, 0},
                  float eps = 0.f, char* state = nullptr) {
   if (sh == nullptr) return BIBO_ERR_NULL_POINTER;
   const int T = sh->T, H = sh->H, E = sh->E, k = sh->k, I = sh->I, dtype = sh->dtype;
@@ -688,7 +688,7 @@ int bibo_moe_rmsnorm_fwd(const void* x, const float* norm_weight, float eps, int
   if (rc != BIBO_OK) return rc;
   if (T == 0) return BIBO_OK;
   if (!x || !norm_weight || !out) return BIBO_ERR_NULL_POINTER;
-  return hip_rc(launch_rmsnorm(x, norm_weight, eps, T, H, dtype, out, static_cast<hipStream_t>(stream)));
+  return hip_rc(launch_rmsnorm(x, vec(norm_weight, BIBO_DTYPE_F32), eps, T, H, dtype, out, static_cast<hipStream_t>(stream)));
 }
 
 int bibo_moe_ffn_workspace_bytes(const bibo_moe_shape* sh, size_t* out) {
@@ -709,6 +709,8 @@ int bibo_moe_ffn_forward(const void* h, const float* norm_weight, float eps, con
   if (!workspace) return BIBO_ERR_NULL_POINTER;
   if (!aligned_ws(workspace)) return BIBO_ERR_MISALIGNED;
   if (sh->T > 0 && (!h || !norm_weight || !out)) return BIBO_ERR_NULL_POINTER;
+  const Vec nw = vec(norm_weight, (sh->flags & BIBO_FLAG_NORM_BF16) ? BIBO_DTYPE_BF16 : BIBO_DTYPE_F32);
+  if (nw.bf16 && !aligned16(norm_weight)) return BIBO_ERR_MISALIGNED;
   const size_t inner = carve(sh->T, sh->H, sh->E, sh->k, sh->I, sh->dtype).total;
   const size_t xn_bytes = align_up((size_t)sh->T * sh->H * elt_size(sh->dtype));
   if (workspace_bytes < inner + xn_bytes) return BIBO_ERR_WORKSPACE_TOO_SMALL;
@@ -718,8 +720,8 @@ int bibo_moe_ffn_forward(const void* h, const float* norm_weight, float eps, con
   if (sh->T > 0 && w_router != nullptr && router_norm_supported(sh->H, sh->dtype, h, w_router, xn))
     // the router kernel normalises the rows it reads and leaves them in xn: no norm launch, one read of h
     return forward_impl(xn, w_router, bias, w_gate_up, w_down, theta, sh, norm_mode, algo, res, out, idx_out, w_out,
-                        counts_out, nullptr, workspace, inner, stream, h, norm_weight, eps);
-  const hipError_t e = launch_rmsnorm(h, norm_weight, eps, sh->T, sh->H, sh->dtype, xn, static_cast<hipStream_t>(stream));
+                        counts_out, nullptr, workspace, inner, stream, h, nw, eps);
+  const hipError_t e = launch_rmsnorm(h, nw, eps, sh->T, sh->H, sh->dtype, xn, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return (int)e;
   return forward_impl(xn, w_router, bias, w_gate_up, w_down, theta, sh, norm_mode, algo, res, out, idx_out, w_out,
                       counts_out, nullptr, workspace, inner, stream);
@@ -801,7 +803,7 @@ int bibo_moe_forward_train(const void* x, const void* w_router, const float* bia
   if (!aligned_ws(state)) return BIBO_ERR_MISALIGNED;
   if (state_bytes < carve_state(sh->T, sh->E, sh->k, sh->I).total) return BIBO_ERR_WORKSPACE_TOO_SMALL;
   return forward_impl(x, w_router, bias, w_gate_up, w_down, theta, sh, norm_mode, BIBO_ALGO_FUSED, nullptr, out, nullptr,
-                      nullptr, counts_out, nullptr, workspace, workspace_bytes, stream, nullptr, nullptr, 0.f,
+                      nullptr, counts_out, nullptr, workspace, workspace_bytes, stream, nullptr, Vec{nullptr, 0}, 0.f,
                       static_cast<char*>(state));
 }
 
@@ -951,6 +953,13 @@ int bibo_moe_exp_qk_norm_rope(void* qkv, int ld, int B, int S, int n_heads, int 
   return hip_rc(launch_qk_norm_rope(qkv, ld, B * S, S, n_heads, n_kv_heads, head_dim, vec(q_weight, weight_dtype),
                                     vec(k_weight, weight_dtype), eps, vec(cos, rope_dtype), vec(sin, rope_dtype), ld_rope,
                                     static_cast<hipStream_t>(stream)));
+}
+
+int bibo_moe_exp_rope_tables(const void* inv_freq, int inv_freq_dtype, int S, int half, void* cos, void* sin, void* stream) {
+  if (S < 0 || half < 1) return BIBO_ERR_BAD_SHAPE;
+  if (S == 0) return BIBO_OK;
+  if (!inv_freq || !cos || !sin) return BIBO_ERR_NULL_POINTER;
+  return hip_rc(launch_rope_tables(vec(inv_freq, inv_freq_dtype), S, half, cos, sin, static_cast<hipStream_t>(stream)));
 }
 
 int bibo_moe_exp_attention_fwd(const void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, int window,

@@ -127,9 +127,13 @@ py::tuple ffn_forward(const Tensor& h, const Tensor& norm_weight, double eps, co
   const Layer l{w_router, bias, w_gate_up, w_down, theta, k, norm, algo, n_pos, n_neg, act};
   c10::DeviceGuard guard(h.device());
   const Tensor x = h.contiguous();
+  Tensor nw = norm_weight.detach();
+  if (nw.scalar_type() == at::kBFloat16 && nw.is_contiguous() && reinterpret_cast<uintptr_t>(nw.data_ptr()) % 16 == 0)
+    flags |= BIBO_FLAG_NORM_BF16;                        // read in place
+  else
+    nw = in_dtype(nw, at::kFloat);
   const bibo_moe_shape sh = shape_of(x, l, flags);
-  const Tensor nw = in_dtype(norm_weight.detach(), at::kFloat);
-  check_tensor(nw, "norm_weight", at::kFloat, {sh.H});
+  check_tensor(nw, "norm_weight", nw.scalar_type(), {sh.H});
   Tensor res;
   if (residual.has_value()) {
     res = in_dtype(*residual, x.scalar_type());
@@ -324,9 +328,34 @@ py::tuple exp_attn_res_norm(const std::vector<Tensor>& candidates, const Tensor&
   return py::make_tuple(out, maybe(normed));
 }
 
+// Weights [n_i, K] of one dtype as a single matrix: in place where they lie one behind the other in one storage (where the
+// modules put them), else a copy of the call's own (2.4 MB of q|k|v at H = 768: 6.5 us and a launch).
+Tensor joined(std::initializer_list<Tensor> ws) {
+  const Tensor& first = *ws.begin();
+  int64_t rows = 0;
+  bool adjacent = true;
+  for (const Tensor& w : ws) {
+    adjacent = adjacent && w.dim() == 2 && w.is_contiguous() && w.size(1) == first.size(1) && w.scalar_type() == first.scalar_type() &&
+               w.storage().is_alias_of(first.storage()) && w.storage_offset() == first.storage_offset() + rows * first.size(1);
+    rows += w.size(0);
+  }
+  return adjacent ? first.as_strided({rows, first.size(1)}, {first.size(1), 1}) : at::cat(at::ITensorListRef(ws.begin(), ws.size()));
+}
+
+// inv_freq [d / 2] -> cos, sin bf16 [S, d]
+py::tuple exp_rope_tables(const Tensor& inv_freq, int64_t S) {
+  at::NoGradGuard no_grad;
+  c10::DeviceGuard guard(inv_freq.device());
+  const int64_t half = inv_freq.numel();
+  const Vecs f = vecs({inv_freq}, half, "inv_freq");
+  const at::TensorOptions opt = inv_freq.options().requires_grad(false).dtype(at::kBFloat16);
+  Tensor cos = at::empty({S, 2 * half}, opt), sin = at::empty({S, 2 * half}, opt);
+  check(bibo_moe_exp_rope_tables(f[0], f.dtype, (int)S, (int)half, cos.data_ptr(), sin.data_ptr(), stream_of(cos)), "bibo_moe_exp_rope_tables");
+  return py::make_tuple(cos, sin);
+}
+
 // x [B, S, H] -> attention output [B, S, H]: one projection to q|k|v rows, norm and RoPE in place, attention with XSA, output
-// projection (the two products are library GEMMs).  The three projection weights are joined here on every call (2.4 MB at
-// H = 768: 1 % of the call at 8 x 2048 tokens): a joined copy that is kept would not see a write through `.data`.
+// projection (the two products are library GEMMs)
 Tensor exp_attention(const Tensor& x, const Tensor& w_q, const Tensor& w_k, const Tensor& w_v, const Tensor& w_o, const c10::optional<Tensor>& q_weight,
                      const c10::optional<Tensor>& k_weight, double eps, const c10::optional<Tensor>& cos,
                      const c10::optional<Tensor>& sin, const c10::optional<Tensor>& xsa_alpha, int n_heads, int n_kv_heads,
@@ -337,7 +366,7 @@ Tensor exp_attention(const Tensor& x, const Tensor& w_q, const Tensor& w_k, cons
   c10::DeviceGuard guard(x.device());
   const Vecs norm = vecs({q_weight, k_weight}, head_dim, "q and k norm weights"), rope = vecs({cos, sin}, S * head_dim, "cos and sin"),
              alpha = vecs({xsa_alpha}, n_heads, "xsa_alpha");
-  const Tensor qkv = at::linear(x, at::cat({w_q, w_k, w_v}));
+  const Tensor qkv = at::linear(x, joined({w_q, w_k, w_v}));
   check_rows(qkv, "q|k|v rows", (int64_t)(n_heads + 2 * n_kv_heads) * head_dim);
   const int ld = (int)qkv.size(-1);
   hipStream_t s = stream_of(x);
@@ -380,7 +409,7 @@ Tensor exp_mlp(const Tensor& x, const Tensor& w_gate, const Tensor& w_up, const 
   const int64_t H = x.size(-1), T = x.numel() / H, I = w_gate.size(0);
   check_rows(x, "x", H);
   c10::DeviceGuard guard(x.device());
-  const Tensor gu = at::linear(x.view({T, H}), at::cat({w_gate, w_up}));        // joined per call, as in exp_attention
+  const Tensor gu = at::linear(x.view({T, H}), joined({w_gate, w_up}));
   check_rows(gu, "gate|up rows", 2 * I);
   Tensor h = at::empty({T, I}, x.options());
   check(bibo_moe_exp_silu_mul_fwd(gu.data_ptr(), (int)T, (int)I, h.data_ptr(), stream_of(x)), "bibo_moe_exp_silu_mul_fwd");
@@ -398,6 +427,7 @@ PYBIND11_MODULE(_native, m) {
   m.def("layer_train", &layer_train);
   m.def("balance_step", &balance_step);
   m.def("exp_attn_res_norm", &exp_attn_res_norm);
+  m.def("exp_rope_tables", &exp_rope_tables);
   m.def("exp_attention", &exp_attention);
   m.def("exp_carry", &exp_carry);
   m.def("exp_mlp", &exp_mlp);

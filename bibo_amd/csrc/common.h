@@ -158,6 +158,26 @@ struct LdsLimitOnce {
   }
 };
 
+// A small parameter vector as its owner holds it: fp32, or bf16 (then 16-byte aligned, checked at the entry points).  Read in
+// place: a widened copy kept between calls would go stale, and one made per call is a launch.  p NULL: absent.
+struct Vec {
+  const void* p;
+  int bf16;
+  __device__ __forceinline__ float operator[](size_t i) const {
+    return bf16 ? (float)static_cast<const bf16_t*>(p)[i] : static_cast<const float*>(p)[i];
+  }
+};
+__device__ __forceinline__ void load8(const Vec& v, size_t at, float (&out)[8]) {      // at: a multiple of 8
+  if (v.bf16) {
+    const bf16x8 r = *reinterpret_cast<const bf16x8*>(static_cast<const bf16_t*>(v.p) + at);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) out[q] = (float)r[q];
+  } else {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) out[q] = static_cast<const float*>(v.p)[at + q];
+  }
+}
+
 // ---- host-side launchers (one per translation unit) -------------------------------------------
 // `chunk_hist` (or NULL): per-workgroup histograms of the selected experts, [ceil(T / *hist_tokens)][64]; *hist_tokens
 // comes back 0 when the kernel that ran does not write them.
@@ -165,7 +185,7 @@ hipError_t launch_router(const void* x, const void* w_router, const float* bias,
                          int norm_mode, float* logits, int32_t* idx, float* w, float* gap, int32_t* chunk_hist,
                          int* hist_tokens, hipStream_t s);
 bool router_norm_supported(int H, int dtype, const void* h, const void* w_router, const void* xn);
-hipError_t launch_router_norm(const void* h, const float* norm_weight, float eps, const void* w_router, const float* bias,
+hipError_t launch_router_norm(const void* h, Vec norm_weight, float eps, const void* w_router, const float* bias,
                               int T, int H, int E, int k, int norm_mode, void* xn, float* logits, int32_t* idx, float* w,
                               int32_t* chunk_hist, int* hist_tokens, hipStream_t s);
 size_t permute_workspace_bytes(int T);
@@ -203,7 +223,7 @@ hipError_t launch_experts_few(const void* x, const void* wgu, const void* wd, co
                               hipStream_t s);
 hipError_t launch_combine(const void* yw, int yw_is_bf16, const CombineArgs& a, int T, int H, int k, int dtype,
                           void* out, hipStream_t s);
-hipError_t launch_rmsnorm(const void* x, const float* weight, float eps, int T, int H, int dtype, void* out,
+hipError_t launch_rmsnorm(const void* x, Vec weight, float eps, int T, int H, int dtype, void* out,
                           hipStream_t s);
 bool mfma_supported(int H, int I, int dtype);
 hipError_t launch_gateup_mfma(const void* x, const void* wgu, const float* theta, const int32_t* offsets,
@@ -229,26 +249,6 @@ hipError_t launch_gateup_stream(const void* x, const void* wgu, const int32_t* i
 hipError_t launch_down_stream(const void* gu, const void* wd, const float* theta, const float* w, const int32_t* idx,
                               int T, int H, int E, int k, int I, int act, void* hidden, float* yw, hipStream_t s);
 
-// A small parameter vector as its owner holds it: fp32, or bf16 (then 16-byte aligned, checked at the entry points).  Read in
-// place: a widened copy kept between calls would go stale, and one made per call is a launch.  p NULL: absent.
-struct Vec {
-  const void* p;
-  int bf16;
-  __device__ __forceinline__ float operator[](size_t i) const {
-    return bf16 ? (float)static_cast<const bf16_t*>(p)[i] : static_cast<const float*>(p)[i];
-  }
-};
-__device__ __forceinline__ void load8(const Vec& v, size_t at, float (&out)[8]) {      // at: a multiple of 8
-  if (v.bf16) {
-    const bf16x8 r = *reinterpret_cast<const bf16x8*>(static_cast<const bf16_t*>(v.p) + at);
-#pragma unroll
-    for (int q = 0; q < 8; ++q) out[q] = (float)r[q];
-  } else {
-#pragma unroll
-    for (int q = 0; q < 8; ++q) out[q] = static_cast<const float*>(v.p)[at + q];
-  }
-}
-
 bool attn_res_supported(int H, int n_cand, int dtype);
 hipError_t launch_attn_res(const void* const* cands, int n_cand, Vec score_a, Vec score_b, float eps, int T, int H, void* out,
                            Vec norm_w, float norm_eps, void* normed, hipStream_t s);
@@ -258,6 +258,7 @@ hipError_t launch_silu_mul(const void* gu, int T, int I, void* out, hipStream_t 
 bool exp_attention_supported(int nq, int nkv, int D);
 hipError_t launch_qk_norm_rope(void* qkv, int ld, int T, int S, int nq, int nkv, int D, Vec qw, Vec kw, float eps, Vec cos, Vec sin,
                                int ld_rope, hipStream_t s);
+hipError_t launch_rope_tables(Vec inv_freq, int S, int half, void* cos, void* sin, hipStream_t s);
 hipError_t launch_exp_attention(const void* qkv, int ld, int B, int S, int nq, int nkv, int D, int window, float scale,
                                 Vec xsa_alpha, void* out, hipStream_t s);
 

@@ -76,6 +76,19 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(bf16_t* __restrict__ 
   *reinterpret_cast<bf16x8*>(row + D / 2 + c * 8) = ob;
 }
 
+// cos and sin of position * inv_freq, bf16 [S, 2 half], both halves of a row alike (embed.py:63-74): one launch for what is
+// nine as tensor operations, of 2 to 5 us each.
+__global__ __launch_bounds__(256) void rope_tables_kernel(Vec inv_freq, int S, int half, bf16_t* __restrict__ cos_t,
+                                                          bf16_t* __restrict__ sin_t) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (long long)S * half) return;
+  const int s = (int)(i / half), c = (int)(i - (long long)s * half);
+  const float ang = (float)s * inv_freq[c];
+  const size_t at = (size_t)s * 2 * half + c;
+  cos_t[at] = cos_t[at + half] = (bf16_t)cosf(ang);
+  sin_t[at] = sin_t[at + half] = (bf16_t)sinf(ang);
+}
+
 // ---- attention -------------------------------------------------------------------------------------------------
 // One workgroup = four waves; a wave owns 32 consecutive queries of one head, and 1, 2 or 4 query heads that share a key
 // head share the workgroup (hpw), so that a block of 32 keys and values passes through LDS once for all of them.
@@ -290,6 +303,14 @@ hipError_t launch_qk_norm_rope(void* qkv, int ld, int T, int S, int nq, int nkv,
     case 192: hipLaunchKernelGGL(qk_norm_rope_kernel<192>, grid, dim3(256), 0, s, p, ld, T, S, nq, nkv, qw, kw, eps, cos, sin, ld_rope); break;
     default: return hipErrorInvalidValue;
   }
+  return hipGetLastError();
+}
+
+hipError_t launch_rope_tables(Vec inv_freq, int S, int half, void* cos, void* sin, hipStream_t s) {
+  const long long n = (long long)S * half;
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(rope_tables_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, inv_freq, S, half,
+                     static_cast<bf16_t*>(cos), static_cast<bf16_t*>(sin));
   return hipGetLastError();
 }
 

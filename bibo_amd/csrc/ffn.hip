@@ -10,8 +10,7 @@ namespace {
 constexpr int kNormMaxPerLane = 32;      // elements a lane keeps in registers (rows up to 2048 wide)
 
 template <typename TIn>
-__global__ __launch_bounds__(256) void rmsnorm_kernel(const TIn* __restrict__ x, const float* __restrict__ weight,
-                                                      float eps, int T, int H, TIn* __restrict__ out) {
+__global__ __launch_bounds__(256) void rmsnorm_kernel(const TIn* __restrict__ x, Vec weight, float eps, int T, int H, TIn* __restrict__ out) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= T) return;
@@ -45,8 +44,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const TIn* __restrict__ x,
 }
 
 // bf16 rows of up to 2048 elements, H % 8 == 0, 16-byte aligned: 16-byte accesses, the row stays in registers
-__global__ __launch_bounds__(256) void rmsnorm_bf16x8_kernel(const bf16_t* __restrict__ x, const float* __restrict__ weight,
-                                                             float eps, int T, int H, bf16_t* __restrict__ out) {
+__global__ __launch_bounds__(256) void rmsnorm_bf16x8_kernel(const bf16_t* __restrict__ x, Vec weight, float eps, int T, int H, bf16_t* __restrict__ out) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= T) return;
@@ -71,8 +69,10 @@ __global__ __launch_bounds__(256) void rmsnorm_bf16x8_kernel(const bf16_t* __res
     const int c = u * kWave + lane;
     if (c < nchunk) {
       bf16x8 o;
+      float nw[8];
+      load8(weight, c * 8, nw);
 #pragma unroll
-      for (int q = 0; q < 8; ++q) o[q] = (bf16_t)(weight[c * 8 + q] * (float)(bf16_t)((float)v[u][q] * rinv));   // norm.py:24
+      for (int q = 0; q < 8; ++q) o[q] = (bf16_t)(nw[q] * (float)(bf16_t)((float)v[u][q] * rinv));   // norm.py:24
       orow[c] = o;
     }
   }
@@ -266,7 +266,7 @@ hipError_t launch_silu_mul(const void* gu, int T, int I, void* out, hipStream_t 
   return hipGetLastError();
 }
 
-hipError_t launch_rmsnorm(const void* x, const float* weight, float eps, int T, int H, int dtype, void* out,
+hipError_t launch_rmsnorm(const void* x, Vec weight, float eps, int T, int H, int dtype, void* out,
                           hipStream_t s) {
   if (T == 0) return hipSuccess;
   const int grid = (T + 3) / 4;

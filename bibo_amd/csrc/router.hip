@@ -328,8 +328,8 @@ __global__ __launch_bounds__(TOK * 16) void router_mfma_kernel(const bf16_t* __r
 // row back to LDS in place and to `xn` in memory, and the logits are then multiplied from the resident rows while
 // w_router streams through two LDS stages as in router_mfma_kernel.  x rows are stored as H/128 chunks of
 // [TOK][128], granule c of a chunk row r at position c ^ (r & 15).
-template <int TOK>
-__global__ __launch_bounds__(TOK * 16) void router_norm_mfma_kernel(const bf16_t* __restrict__ h, const float* __restrict__ nw,
+template <int TOK, typename TN>
+__global__ __launch_bounds__(TOK * 16) void router_norm_mfma_kernel(const bf16_t* __restrict__ h, const TN* __restrict__ nw,
                                                                     float eps, const bf16_t* __restrict__ wr,
                                                                     const float* __restrict__ bias, int T, int H, int E,
                                                                     int k, int norm_mode, bf16_t* __restrict__ xn,
@@ -400,8 +400,13 @@ __global__ __launch_bounds__(TOK * 16) void router_norm_mfma_kernel(const bf16_t
         const int c = u * kWave + lane;
         if (c < ngran) {
           bf16x8 o;
+          TN wv[8];
+          if constexpr (sizeof(TN) == 2) *reinterpret_cast<bf16x8*>(wv) = reinterpret_cast<const bf16x8*>(nw)[c];
+          else
 #pragma unroll
-          for (int q = 0; q < 8; ++q) o[q] = (bf16_t)(nw[c * 8 + q] * (float)(bf16_t)((float)v[u][q] * rinv));   // norm.py:24
+            for (int q = 0; q < 8; ++q) wv[q] = nw[c * 8 + q];
+#pragma unroll
+          for (int q = 0; q < 8; ++q) o[q] = (bf16_t)((float)wv[q] * (float)(bf16_t)((float)v[u][q] * rinv));   // norm.py:24
           *reinterpret_cast<bf16x8*>(loc[u]) = o;
           if (live) *reinterpret_cast<bf16x8*>(xn + (size_t)(t0 + r) * H + c * 8) = o;
         }
@@ -516,14 +521,14 @@ bool router_norm_supported(int H, int dtype, const void* h, const void* w_router
 }
 
 // the kernel's TOK whole rows sit in dynamic LDS: allowed once per device, for the widest rows it takes
-template <int TOK>
+template <int TOK, typename TN>
 hipError_t allow_dynamic_lds() {
   static LdsLimitOnce once;
-  return once.raise(reinterpret_cast<const void*>(&router_norm_mfma_kernel<TOK>), (int)(TOK * kNormRouterMaxH * sizeof(bf16_t)));
+  return once.raise(reinterpret_cast<const void*>(&router_norm_mfma_kernel<TOK, TN>), (int)(TOK * kNormRouterMaxH * sizeof(bf16_t)));
 }
 
 // RMSNorm + router in one launch (see router_norm_mfma_kernel); `xn` receives the normalised rows.
-hipError_t launch_router_norm(const void* h, const float* norm_weight, float eps, const void* w_router, const float* bias,
+hipError_t launch_router_norm(const void* h, Vec norm_weight, float eps, const void* w_router, const float* bias,
                               int T, int H, int E, int k, int norm_mode, void* xn, float* logits, int32_t* idx, float* w,
                               int32_t* chunk_hist, int* hist_tokens, hipStream_t s) {
   if (hist_tokens != nullptr) *hist_tokens = 0;
@@ -531,20 +536,22 @@ hipError_t launch_router_norm(const void* h, const float* norm_weight, float eps
   const bf16_t* hp = static_cast<const bf16_t*>(h);
   const bf16_t* wp = static_cast<const bf16_t*>(w_router);
   bf16_t* xp = static_cast<bf16_t*>(xn);
-  hipError_t e;
-  if (T >= 32 * 256) {
-    const size_t shm = (size_t)32 * H * sizeof(bf16_t);
-    if ((e = allow_dynamic_lds<32>()) != hipSuccess) return e;
-    hipLaunchKernelGGL(router_norm_mfma_kernel<32>, dim3((T + 31) / 32), dim3(512), shm, s, hp, norm_weight, eps, wp, bias, T,
-                       H, E, k, norm_mode, xp, logits, idx, w, nullptr, chunk_hist);
-  } else {
-    const size_t shm = (size_t)16 * H * sizeof(bf16_t);
-    if ((e = allow_dynamic_lds<16>()) != hipSuccess) return e;
-    hipLaunchKernelGGL(router_norm_mfma_kernel<16>, dim3((T + 15) / 16), dim3(256), shm, s, hp, norm_weight, eps, wp, bias, T,
-                       H, E, k, norm_mode, xp, logits, idx, w, nullptr, chunk_hist);
-  }
+  auto launch = [&](auto tok, auto* nw) -> hipError_t {
+    constexpr int TOK = decltype(tok)::value;
+    using TN = std::remove_const_t<std::remove_pointer_t<decltype(nw)>>;
+    const hipError_t e = allow_dynamic_lds<TOK, TN>();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((router_norm_mfma_kernel<TOK, TN>), dim3((T + TOK - 1) / TOK), dim3(TOK * 16), (size_t)TOK * H * sizeof(bf16_t), s,
+                       hp, nw, eps, wp, bias, T, H, E, k, norm_mode, xp, logits, idx, w, nullptr, chunk_hist);
+    return hipGetLastError();
+  };
+  auto typed = [&](auto tok) {
+    return norm_weight.bf16 ? launch(tok, static_cast<const bf16_t*>(norm_weight.p)) : launch(tok, static_cast<const float*>(norm_weight.p));
+  };
+  const hipError_t e = T >= 32 * 256 ? typed(std::integral_constant<int, 32>()) : typed(std::integral_constant<int, 16>());
+  if (e != hipSuccess) return e;
   if (hist_tokens != nullptr && chunk_hist != nullptr) *hist_tokens = T >= 32 * 256 ? 32 : 16;
-  return hipGetLastError();
+  return hipSuccess;
 }
 
 hipError_t launch_router(const void* x, const void* w_router, const float* bias, int T, int H, int E, int k, int dtype,

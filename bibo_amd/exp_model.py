@@ -126,6 +126,26 @@ def _native_ok(x) -> bool:
             and not (torch.is_autocast_enabled() and torch.get_autocast_dtype("cuda") != torch.bfloat16))
 
 
+def _lay_out(*linears):
+    """The layers' weights one behind the other in one block of GPU memory, so that one product reads them all in place.  They
+    stay parameters of their own; wherever they end up elsewhere (a copy, a replaced parameter) the native call joins them."""
+    ps = [m._parameters.get("weight") for m in linears]
+    if not all(type(p) is nn.Parameter and type(p.data) is torch.Tensor and p.is_cuda and p.is_contiguous() and not p.is_inference()
+               and p.dtype == ps[0].dtype and p.device == ps[0].device for p in ps):
+        return
+    at = ps[0].data_ptr()
+    for p in ps:
+        if p.data_ptr() != at or p.untyped_storage().data_ptr() != ps[0].untyped_storage().data_ptr():
+            break
+        at += p.numel() * p.element_size()
+    else:
+        return
+    with torch.no_grad():
+        block = torch.cat([p.data for p in ps])
+    for p, part in zip(ps, block.split([p.shape[0] for p in ps])):
+        p.data = part
+
+
 def _rotate_half(x):
     h = x.shape[-1] // 2
     return torch.cat((-x[..., h:], x[..., :h]), dim=-1)
@@ -192,6 +212,12 @@ class BiBoExpAttention(nn.Module):
         self.k_norm = RMSNorm(d, config.rms_norm_eps) if qk_norm else nn.Identity()
         self.xsa_alpha = (nn.Parameter(torch.full((self.num_heads,), float(config.xsa_alpha_init)))
                           if config.use_xsa else None)
+        _lay_out(self.q_proj, self.k_proj, self.v_proj)
+
+    def _apply(self, fn, *a, **kw):
+        out = super()._apply(fn, *a, **kw)
+        _lay_out(self.q_proj, self.k_proj, self.v_proj)
+        return out
 
     def _native(self, x, cos, sin):
         """The whole block in the native call, or None where its kernels do not take it."""
@@ -243,6 +269,12 @@ class BiBoExpMLP(nn.Module):
         self.gate_proj = nn.Linear(config.hidden_size, config.intermediate_size, bias=False)
         self.up_proj = nn.Linear(config.hidden_size, config.intermediate_size, bias=False)
         self.down_proj = nn.Linear(config.intermediate_size, config.hidden_size, bias=False)
+        _lay_out(self.gate_proj, self.up_proj)
+
+    def _apply(self, fn, *a, **kw):
+        out = super()._apply(fn, *a, **kw)
+        _lay_out(self.gate_proj, self.up_proj)
+        return out
 
     def forward(self, x):
         return self.down_proj(F.silu(self.gate_proj(x)) * self.up_proj(x))
@@ -352,9 +384,12 @@ class BiBoExpModel(nn.Module):
         h = self.embed_tokens(input_ids)
         if self.config.bf16_residual_stream:                                    # exp/modeling_bibo.py:858-859
             h = h.to(torch.bfloat16)
-        ang = torch.arange(S, device=h.device, dtype=torch.float32)[:, None] * self.inv_freq.float()[None, :]
-        ang = torch.cat((ang, ang), dim=-1)
-        cos, sin = ang.cos().to(h.dtype), ang.sin().to(h.dtype)                 # embed.py:63-74
+        if _native_ok(h) and self.inv_freq.is_cuda:
+            cos, sin = L.native().exp_rope_tables(self.inv_freq, S)
+        else:
+            ang = torch.arange(S, device=h.device, dtype=torch.float32)[:, None] * self.inv_freq.float()[None, :]
+            ang = torch.cat((ang, ang), dim=-1)
+            cos, sin = ang.cos().to(h.dtype), ang.sin().to(h.dtype)             # embed.py:63-74
         blocks = []
         for layer in self.layers:
             h, blocks = layer(h, blocks, cos, sin, collect_routing)

@@ -74,7 +74,9 @@ enum bibo_flags {
   BIBO_FLAG_GRAD_F32 = 4,
   /* bibo_moe_forward_train only: pick the expert kernels as `auto` does in bibo_moe_forward (few tiles: two launches over more
      workgroups) instead of always running the fused kernel. */
-  BIBO_FLAG_TRAIN_AUTO = 8
+  BIBO_FLAG_TRAIN_AUTO = 8,
+  /* bibo_moe_ffn_forward only: norm_weight points to bf16 values, 16-byte aligned (used in fp32, as the fp32 ones are). */
+  BIBO_FLAG_NORM_BF16 = 16
 };
 
 /* kernel family for the expert GEMMs */
@@ -365,6 +367,7 @@ int bibo_moe_exp_attn_res_fwd(const void* const* candidates, int n_candidates, c
  * bibo_moe_exp_qk_norm_rope: in place on rows [q heads | k heads | v heads] (row stride ld elements) of B x S tokens: RMSNorm
  *   per query and key head (q_weight, k_weight [head_dim], NULL: none), then the rotate-half RoPE (cos, sin: the first
  *   head_dim / 2 entries of S rows at stride ld_rope, a multiple of 8; NULL: none) (src/modeling/attn/base.py:70-91).
+ * bibo_moe_exp_rope_tables: cos, sin bf16 [S, 2 half] of position * inv_freq[half] in fp32, both halves of a row alike.
  * bibo_moe_exp_attention_fwd: out [B*S, n_heads * head_dim] = causal attention of those rows (window > 0: restricted to the
  *   last `window` keys), softmax in fp32, with the XSA correction y - tanh(alpha) <y, vn> vn (xsa_alpha [n_heads] or NULL;
  *   src/modeling/attn/xsa.py:41-54).  head_dim in {64, 128, 192}; n_heads / n_kv_heads = 1 or even (BIBO_ERR_UNSUPPORTED
@@ -379,6 +382,7 @@ int bibo_moe_exp_silu_mul_fwd(const void* gate_up, int T, int I, void* out, void
 int bibo_moe_exp_qk_norm_rope(void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, const void* q_weight,
                               const void* k_weight, int weight_dtype, float eps, const void* cos, const void* sin, int rope_dtype,
                               int ld_rope, void* stream);
+int bibo_moe_exp_rope_tables(const void* inv_freq, int inv_freq_dtype, int S, int half, void* cos, void* sin, void* stream);
 int bibo_moe_exp_attention_fwd(const void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, int window,
                                float scale, const void* xsa_alpha, int alpha_dtype, void* out, void* stream);
 

@@ -117,3 +117,49 @@ def test_bf16_vectors_give_the_bits_of_their_fp32_copies(H, S):
     one = nat.exp_attention(x, wq, wk, wv, wo, *vecs, nh, nkv, d, 0, d ** -0.5)
     two = nat.exp_attention(x, wq, wk, wv, wo, *(v.float() if torch.is_tensor(v) else v for v in vecs), nh, nkv, d, 0, d ** -0.5)
     assert torch.equal(one, two)
+
+
+@torch.no_grad()
+def test_weights_lie_in_one_block_until_one_is_replaced():
+    import copy
+    model, ids = _model(), _ids(2, 20, 1)
+    attn, mlp = model.model.layers[1].self_attn, model.model.layers[3].mlp
+    for group in ((attn.q_proj, attn.k_proj, attn.v_proj), (mlp.gate_proj, mlp.up_proj)):
+        assert len({m.weight.untyped_storage().data_ptr() for m in group}) == 1
+    want = model(ids)
+    assert torch.equal(copy.deepcopy(model)(ids), want)                            # copies lie apart
+    other = _model(seed=3)
+    other.load_state_dict(model.state_dict())
+    for m in other.modules():
+        m.__dict__.pop("_fp32_weight", None)
+    assert torch.equal(other(ids), want)
+    for m in (attn.k_proj, mlp.up_proj):
+        m.weight = torch.nn.Parameter(m.weight.clone())
+    assert torch.equal(model(ids), want)
+    attn.v_proj.weight.data.mul_(2.0)                # (a factor on q would vanish in its norm)
+    assert not torch.equal(model(ids), want)
+    attn.v_proj.weight.data.mul_(0.5)
+    assert torch.equal(model.float().to(torch.bfloat16)(ids), want)
+
+
+@pytest.mark.parametrize("S,half,dtype", [(1, 32, torch.float32), (77, 96, torch.float32), (2048, 64, torch.bfloat16)])
+def test_rope_tables_give_the_bits_of_the_tensor_operations(S, half, dtype):
+    inv = (10000.0 ** (-torch.arange(0, half, dtype=torch.float32) / half)).to(DEV, dtype)
+    ang = torch.arange(S, device=DEV, dtype=torch.float32)[:, None] * inv.float()[None, :]
+    ang = torch.cat((ang, ang), -1)
+    cos, sin = L.native().exp_rope_tables(inv, S)
+    assert torch.equal(cos, ang.cos().bfloat16()) and torch.equal(sin, ang.sin().bfloat16())
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("T,H", [(5, 256), (40, 96), (70, 2304)])
+def test_seam_reads_a_bf16_norm_weight_in_place(T, H):
+    import bibo_amd
+    cfg = bibo_amd.BiBoMoEConfig(hidden_size=H, moe_intermediate_size=32, num_routed_experts=8, num_experts_per_tok=2, special_expert_pairs=0)
+    with torch.device(DEV):
+        layer = bibo_amd.BiBoMoELayer(cfg).to(torch.bfloat16).eval()
+    g = torch.Generator().manual_seed(T)
+    h = torch.randn(1, T, H, generator=g).to(DEV, torch.bfloat16)
+    w = torch.randn(H + 1, generator=g).to(DEV, torch.bfloat16)
+    for nw in (w[:H], w[1:]):                       # the second on no 16-byte boundary
+        assert torch.equal(layer.ffn_forward(h, nw, 1e-6), layer.ffn_forward(h, nw.float(), 1e-6))
