@@ -97,6 +97,9 @@ __global__ __launch_bounds__(256) void rope_tables_kernel(Vec inv_freq, int S, i
 //   O^T = V^T P^T: the probabilities a lane holds (keys 4h .. +4 and 8 + 4h .. +4 of sixteen) are, rounded to bf16, the MFMA
 //     operand as they are, with V's operand read in the same key order by transposing LDS reads; O^T has lane = query
 //     again, so rescaling and the final division are per-lane scalars.
+// FINE (banded layers): a probability goes in as two bf16 parts, its rounding and what that left, so that it keeps 16 bits of
+// mantissa; the tensor operations these layers ran before multiplied their probabilities in fp32.  Causal layers' library kernel
+// rounded them to bf16, as the other variant does.
 // The running maximum is raised (and O rescaled, D/32 x 16 multiplies) only when a row's maximum passes it by more than 8
 // in log2 units: the sums stay exact, the probabilities at most 256.
 // K and V blocks arrive by LDS-DMA in two stages; the next one is requested right after the barrier that frees its stage.
@@ -110,7 +113,7 @@ typedef __attribute__((address_space(3))) attn_v4i16 attn_lds_v4i16;
 template <int D> __device__ __forceinline__ int kswz(int row) { return D == 128 ? (row & 15) : ((row >> 1) & 7); }
 template <int D> __device__ __forceinline__ int vswz(int row) { return D == 128 ? ((row & 3) << 2) : (((row >> 1) & 1) << 2); }
 
-template <int D>
+template <int D, bool FINE>
 __global__ __launch_bounds__(256, 2) void attention_kernel(const bf16_t* __restrict__ qkv, int ld, int S, int nq, int nkv, int hpw,
                                                            int heads, int nqb, int window, float scale_log2,
                                                            Vec xsa_alpha, bf16_t* __restrict__ out) {
@@ -209,12 +212,13 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const bf16_t* __restr
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[dt][i] *= al;
     }
-    bf16x8 p[2];
+    bf16x8 p[2], pf[2];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const float e = __builtin_amdgcn_exp2f(fmaf(st[i], scale_log2, -m));
       l += e;
       p[i >> 3][i & 7] = (bf16_t)e;
+      if constexpr (FINE) pf[i >> 3][i & 7] = (bf16_t)(e - (float)p[i >> 3][i & 7]);
     }
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk)
@@ -227,6 +231,7 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const bf16_t* __restr
         typedef short v8i16 __attribute__((ext_vector_type(8)));
         const v8i16 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
         o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, v), p[kk], o[dt], 0, 0, 0);
+        if constexpr (FINE) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, v), pf[kk], o[dt], 0, 0, 0);
       }
   };
   for (int kv0 = kv_first; kv0 < kv_end; kv0 += 2 * KB) {
@@ -324,10 +329,14 @@ hipError_t launch_exp_attention(const void* qkv, int ld, int B, int S, int nq, i
   const float sl = scale * 1.4426950408889634f;
   const bf16_t* p = static_cast<const bf16_t*>(qkv);
   bf16_t* o = static_cast<bf16_t*>(out);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, p, ld, S, nq, nkv, hpw, heads, nqb, window, sl, xsa_alpha, o);
+  };
+  const bool fine = window > 0;
   switch (D) {
-    case 64: hipLaunchKernelGGL(attention_kernel<64>, grid, dim3(256), 0, s, p, ld, S, nq, nkv, hpw, heads, nqb, window, sl, xsa_alpha, o); break;
-    case 128: hipLaunchKernelGGL(attention_kernel<128>, grid, dim3(256), 0, s, p, ld, S, nq, nkv, hpw, heads, nqb, window, sl, xsa_alpha, o); break;
-    case 192: hipLaunchKernelGGL(attention_kernel<192>, grid, dim3(256), 0, s, p, ld, S, nq, nkv, hpw, heads, nqb, window, sl, xsa_alpha, o); break;
+    case 64: if (fine) launch(attention_kernel<64, true>); else launch(attention_kernel<64, false>); break;
+    case 128: if (fine) launch(attention_kernel<128, true>); else launch(attention_kernel<128, false>); break;
+    case 192: if (fine) launch(attention_kernel<192, true>); else launch(attention_kernel<192, false>); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
