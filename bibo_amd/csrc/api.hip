@@ -161,13 +161,10 @@ Workspace carve(int T, int H, int E, int k, int I, int dtype) {
   ws.yw = o;
   ws.least = o + align_up(S * (size_t)H * sizeof(float));
   ws.total = o + align_up(S * (size_t)(generic_tiles(H, I, dtype) && 2 * I > H ? 2 * I : H) * sizeof(float));
-  // bf16 pre-activations of a call whose tiles are cut by columns: the streaming kernels' segment, or one behind the others
-  ws.pre = ws.gu;
-  if (dtype == BIBO_DTYPE_BF16 && mfma_supported(H, I, dtype) && split_columns(T * k, E, H, I) &&
-      !stream_possible(T, H, E, k, I, dtype, true)) {
-    ws.pre = ws.total;
-    ws.total += align_up(S * (size_t)2 * I * sizeof(bf16_t));
-  }
+  // fp32 pre-activations of a call whose tiles are cut by columns, behind the others
+  ws.pre = ws.total;
+  if (dtype == BIBO_DTYPE_BF16 && mfma_supported(H, I, dtype) && split_columns(T * k, E, H, I))
+    ws.total += align_up(S * (size_t)2 * I * sizeof(float));
   return ws;
 }
 
@@ -232,10 +229,10 @@ int experts_dispatch(const void* x, const void* wgu, const void* wd, const float
   }
   if (algo == kAlgoSplit) {
     if (!aligned16(x) || !aligned16(wgu) || !aligned16(wd)) return BIBO_ERR_MISALIGNED;
-    void* pre = preact != nullptr ? preact : static_cast<void*>(base + ws.pre);
-    hipError_t e = launch_gateup_raw(x, wgu, offsets, perm_token, T, H, Eg, k, I, pre, true, s);
+    void* pre = base + ws.pre;
+    hipError_t e = launch_gateup_raw(x, wgu, offsets, perm_token, T, H, Eg, k, I, pre, true, true, s);
     if (e != hipSuccess) return (int)e;
-    if ((e = launch_down_act(pre, wd, theta, w, offsets, perm_slot, T * k, H, Eg, I, act, yw, s)) != hipSuccess) return (int)e;
+    if ((e = launch_down_act(pre, wd, theta, w, offsets, perm_slot, T * k, H, Eg, I, act, yw, preact, s)) != hipSuccess) return (int)e;
     return hip_rc(launch_combine(yw, 1, ca, T, H, k, dtype, out, s));
   }
   if (algo == BIBO_ALGO_FUSED || algo == kAlgoFusedWide) {
@@ -295,7 +292,7 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
   int a;
   if ((rc = resolve_algo(algo, T, H, E, k, I, dtype, true, true, &a)) != BIBO_OK) return rc;
   a = composite_algo(algo == BIBO_ALGO_AUTO || (state != nullptr && (sh->flags & BIBO_FLAG_TRAIN_AUTO) != 0), a, T, H, E, k, I, dtype);
-  if (a == kAlgoSplit && state == nullptr && workspace_bytes < carve(T, H, E, k, I, dtype).total) a = BIBO_ALGO_FUSED;
+  if (a == kAlgoSplit && workspace_bytes < carve(T, H, E, k, I, dtype).total) a = BIBO_ALGO_FUSED;
   if (!workspace) return BIBO_ERR_NULL_POINTER;
   if (!aligned_ws(workspace)) return BIBO_ERR_MISALIGNED;
   if (T > 0 && (!x || !w_router || !bias || !w_gate_up || !w_down || !out)) return BIBO_ERR_NULL_POINTER;

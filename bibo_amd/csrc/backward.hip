@@ -557,7 +557,7 @@ hipError_t launch_backward(const void* x, const void* d_out, const void* w_route
   if (gu_saved != nullptr)
     err = hipSuccess;
   else if ((fused_supported(H, I, BIBO_DTYPE_BF16) || fused_wide_supported(H, I, BIBO_DTYPE_BF16)) && (long long)T * H < (1LL << 31))
-    err = launch_gateup_raw(xp, wgup, offsets, perm_token, T, H, E, k, I, b.gu, split_columns(S, E, H, I), s);
+    err = launch_gateup_raw(xp, wgup, offsets, perm_token, T, H, E, k, I, b.gu, split_columns(S, E, H, I), false, s);
   else
     err = launch_ggemm<true, false>(xp, perm_token, wgup, offsets, nullptr, S, H, 2 * I, E, static_cast<bf16_t*>(b.gu), s);
   if (err != hipSuccess) return err;

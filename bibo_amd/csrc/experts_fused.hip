@@ -243,7 +243,8 @@ __device__ __forceinline__ void down_block(Slice slice, WBlock<CT> (&wb)[NB], co
 // pre-activations themselves, rounded to bf16, to `preact` [S, 2I] in permuted row order (gate columns, then up
 // columns), staged through the LDS stages into whole row segments.  MODE 2: the training forward - the forward pass that
 // also leaves those pre-activations for its backward, in the same way (8-byte stores straight from the accumulator
-// registers during phase 2 were slower: 140 against 133 us at T = 8192).
+// registers during phase 2 were slower: 140 against 133 us at T = 8192).  MODE 3: as MODE 1, but the fp32 sums as they are, for
+// down_act_kernel (`preact` points to floats): 16-byte stores from the accumulators, a row's 128 bytes in four of them.
 template <int NT, int CT, int MODE = 0, int MTP = 2>
 __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ wgu,
                                                             const bf16_t* __restrict__ wd,
@@ -268,9 +269,9 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
   __shared__ float rinv_s[BM], gain_s[BM], w_s[BM];
   __shared__ int slot_s[BM];
 
-  // MODE 1 may cut a tile's columns over several workgroups (the other modes need whole rows): workgroup cb of a tile then
+  // MODE 1 and 3 may cut a tile's columns over several workgroups (the others need whole rows): workgroup cb of a tile then
   // owns gate columns [cb I, cb I + I) of a row of row_i = column_blocks I and the up columns behind the same gate columns.
-  const int ncb = MODE == 1 ? column_blocks : 1, row_i = I * ncb;
+  const int ncb = MODE == 1 || MODE == 3 ? column_blocks : 1, row_i = I * ncb;
   const TileMap tm = make_tile_map(offsets, E, BM);
   const int flat = xcd_tile(blockIdx.x, tm.total * ncb);
   if (flat >= tm.total * ncb) return;
@@ -452,6 +453,24 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
   }
   wait_loads_and_sync();                   // every transfer has landed and every wave is done with the stages
 
+  if constexpr (MODE == 3) {
+    float* pre = reinterpret_cast<float*>(preact);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const int m = mbase + mt * 32 + n;
+      if (mt >= my_blocks || m >= rows) continue;
+      float* prow = pre + (size_t)(row0 + m) * (2 * row_i) + cb * I + 4 * (lane >> 5);
+#pragma unroll
+      for (int j = 0; j < 2 * NT; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int half = j / NT, col = (wn * NT + j % NT) * 32 + 8 * q;
+          *reinterpret_cast<floatx4*>(prow + half * row_i + col) =
+              floatx4{acc[mt][j][4 * q], acc[mt][j][4 * q + 1], acc[mt][j][4 * q + 2], acc[mt][j][4 * q + 3]};
+        }
+    }
+    return;
+  }
   if constexpr (MODE != 0) {
     // gate half, then up half: accumulators -> the stages in the activation layout (stage t = columns [128 t, 128 t + 128)
     // of the half, granule c of row m at c ^ (m & 15)) -> whole 256-byte row segments to memory
@@ -572,15 +591,17 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
 }
 
 
-// The second half of the fused kernel on its own, for calls with fewer tiles than CUs: the activations of a tile from the bf16
+// The second half of the fused kernel on its own, for calls with fewer tiles than CUs: the activations of a tile from the fp32
 // pre-activations [S, 2I] that the first half left (phase 2), and ONE block of output columns (phase 3), so that an expert's
 // w_down passes through H / BN2 CUs at once.  Every one of them computes the tile's activations again, one wave per row, while
-// its first weights are on their way.
+// its first weights are on their way.  With `preact`, the workgroups of column block 0 also leave the pre-activations rounded to
+// bf16, for a backward pass.
 template <int NT, int CT, int MTP>
-__global__ __launch_bounds__(512) void down_act_kernel(const bf16_t* __restrict__ gu, const bf16_t* __restrict__ wd,
+__global__ __launch_bounds__(512) void down_act_kernel(const float* __restrict__ gu, const bf16_t* __restrict__ wd,
                                                        const float* __restrict__ theta, const float* __restrict__ w,
                                                        const int32_t* __restrict__ offsets, const int32_t* __restrict__ perm_slot,
-                                                       int H, int E, int act, bf16_t* __restrict__ yw) {
+                                                       int H, int E, int act, bf16_t* __restrict__ yw,
+                                                       bf16_t* __restrict__ preact) {
   using F = FusedShape<NT, CT, MTP>;
   constexpr int BM = F::BM, I = F::I;
   __shared__ __attribute__((aligned(16))) bf16_t acts[NT * BM * 128];
@@ -605,16 +626,19 @@ __global__ __launch_bounds__(512) void down_act_kernel(const bf16_t* __restrict_
   WBlock<CT> wb[KB];
   // a wave's rows are wave, wave + 8, ...; the first kRowsAhead of them are requested ahead of the weights, which a CU would
   // otherwise serve first
-  constexpr int kRowsAhead = 8;
+  constexpr int kRowsAhead = NT == 4 ? 6 : 8;            // (what the registers hold beside I = 512 worth of weights)
   const bool live = lane * 8 < I;
-  bf16x8 g[kRowsAhead], u[kRowsAhead];
+  floatx4 g[kRowsAhead][2], u[kRowsAhead][2];
   auto request = [&](int m0) {
 #pragma unroll
     for (int i = 0; i < kRowsAhead; ++i) {
-      const bf16_t* src = gu + (size_t)(row0 + min(m0 + 8 * i, rows - 1)) * 2 * I + lane * 8;
+      const float* src = gu + (size_t)(row0 + min(m0 + 8 * i, rows - 1)) * 2 * I + lane * 8;
       if (live && m0 + 8 * i < rows) {
-        g[i] = *reinterpret_cast<const bf16x8*>(src);
-        u[i] = *reinterpret_cast<const bf16x8*>(src + I);
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+          g[i][v] = *reinterpret_cast<const floatx4*>(src + 4 * v);
+          u[i][v] = *reinterpret_cast<const floatx4*>(src + I + 4 * v);
+        }
       }
     }
   };
@@ -636,7 +660,7 @@ __global__ __launch_bounds__(512) void down_act_kernel(const bf16_t* __restrict_
       float ss = 0.f;
       if (live) {
 #pragma unroll
-        for (int q = 0; q < 8; ++q) ss = fmaf((float)g[i][q], (float)g[i][q], ss);
+        for (int q = 0; q < 8; ++q) ss = fmaf(g[i][q >> 2][q & 3], g[i][q >> 2][q & 3], ss);
       }
       ss = wave_sum(ss);
       float rinv, gain;
@@ -646,9 +670,20 @@ __global__ __launch_bounds__(512) void down_act_kernel(const bf16_t* __restrict_
         bf16x8 h;
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-          const float gq = (float)g[i][q];
+          const float gq = g[i][q >> 2][q & 3];
           const float sg = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(gq * nrl));
-          h[q] = (bf16_t)(gq * rg * sg * (float)u[i][q]);                           // SiLU(g/r) r^p up
+          h[q] = (bf16_t)(gq * rg * sg * u[i][q >> 2][q & 3]);                      // SiLU(g/r) r^p up
+        }
+        if (preact != nullptr && nb == 0) {
+          bf16x8 gb, ub;
+#pragma unroll
+          for (int q = 0; q < 8; ++q) {
+            gb[q] = (bf16_t)g[i][q >> 2][q & 3];
+            ub[q] = (bf16_t)u[i][q >> 2][q & 3];
+          }
+          bf16_t* dst = preact + (size_t)(row0 + m) * 2 * I + lane * 8;
+          *reinterpret_cast<bf16x8*>(dst) = gb;
+          *reinterpret_cast<bf16x8*>(dst + I) = ub;
         }
         *reinterpret_cast<bf16x8*>(acts + (lane >> 4) * (BM * 128) + m * 128 + (((lane & 15) ^ (m & 15)) << 3)) = h;
       }
@@ -668,13 +703,15 @@ __global__ __launch_bounds__(512) void down_act_kernel(const bf16_t* __restrict_
 }
 
 template <int NT>
-void launch_down_act_nt(const bf16_t* gu, const bf16_t* wd, const float* theta, const float* w, const int32_t* offsets,
-                        const int32_t* perm_slot, int S, int H, int E, int act, bf16_t* yw, hipStream_t s) {
+void launch_down_act_nt(const float* gu, const bf16_t* wd, const float* theta, const float* w, const int32_t* offsets,
+                        const int32_t* perm_slot, int S, int H, int E, int act, bf16_t* yw, bf16_t* preact,
+                        hipStream_t s) {
   auto launch = [&](auto mt, auto ct) {
     constexpr int MT = decltype(mt)::value, CT = decltype(ct)::value;
     const int tiles = S / (64 * MT) + E < S ? S / (64 * MT) + E : S;
     const int grid = ((tiles * (H / (128 * CT)) + 7) & ~7) + 8;
-    hipLaunchKernelGGL((down_act_kernel<NT, CT, MT>), dim3(grid), dim3(512), 0, s, gu, wd, theta, w, offsets, perm_slot, H, E, act, yw);
+    hipLaunchKernelGGL((down_act_kernel<NT, CT, MT>), dim3(grid), dim3(512), 0, s, gu, wd, theta, w, offsets, perm_slot, H, E, act, yw,
+                       preact);
   };
   // 64-row tiles while they and their column blocks leave no workgroup waiting for a CU: shorter, and more of them pull weights
   using std::integral_constant;
@@ -721,13 +758,13 @@ void launch_fused_nt(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const
   else launch(std::integral_constant<int, 1>{});
 }
 
-template <int NT>
+template <int NT, int MODE = 1>
 void launch_raw_nt(const bf16_t* x, const bf16_t* wgu, const int32_t* offsets, const int32_t* perm_token, int S, int H, int E,
                    unsigned x_bytes, bf16_t* gu, int column_blocks, hipStream_t s) {
   constexpr int MT = NT == 4 ? 1 : 2;
   const int tiles = S / (64 * MT) + E < S ? S / (64 * MT) + E : S;
   const int grid = ((tiles * column_blocks + 7) & ~7) + 8;
-  hipLaunchKernelGGL((experts_fused_kernel<NT, 1, 1, MT>), dim3(grid), dim3(512), 0, s, x, wgu, nullptr, nullptr, nullptr,
+  hipLaunchKernelGGL((experts_fused_kernel<NT, 1, MODE, MT>), dim3(grid), dim3(512), 0, s, x, wgu, nullptr, nullptr, nullptr,
                      offsets, nullptr, perm_token, H, E, 0, x_bytes, nullptr, gu, column_blocks);
 }
 
@@ -737,7 +774,7 @@ void launch_raw_nt(const bf16_t* x, const bf16_t* wgu, const int32_t* offsets, c
 // pass recomputes, moe.py:84).  Same shapes as launch_experts_fused.
 // `split`: one workgroup per 128 gate (and up) columns of a tile, for calls with fewer tiles than CUs.
 hipError_t launch_gateup_raw(const void* x, const void* wgu, const int32_t* offsets, const int32_t* perm_token, int T, int H,
-                             int E, int k, int I, void* gu, bool split, hipStream_t s) {
+                             int E, int k, int I, void* gu, bool split, bool f32, hipStream_t s) {
   const int S = T * k;
   if (S == 0) return hipSuccess;
   if ((unsigned long long)T * H * sizeof(bf16_t) >= (1ull << 32)) return hipErrorInvalidValue;
@@ -745,6 +782,11 @@ hipError_t launch_gateup_raw(const void* x, const void* wgu, const int32_t* offs
   const bf16_t* xp = static_cast<const bf16_t*>(x);
   const bf16_t* gp = static_cast<const bf16_t*>(wgu);
   bf16_t* out = static_cast<bf16_t*>(gu);
+  if (f32 && !split) return hipErrorInvalidValue;
+  if (f32) {
+    launch_raw_nt<1, 3>(xp, gp, offsets, perm_token, S, H, E, xb, out, I / 128, s);
+    return hipGetLastError();
+  }
   if (split) {
     launch_raw_nt<1>(xp, gp, offsets, perm_token, S, H, E, xb, out, I / 128, s);
     return hipGetLastError();
@@ -762,26 +804,30 @@ hipError_t launch_gateup_raw(const void* x, const void* wgu, const int32_t* offs
 // Whether a tile's columns are cut over several workgroups.  The fused kernel keeps a row's tile on one CU, which is what pulls the
 // expert's weights then: with fewer tiles than CUs most of the chip idles.  Cut (launch_gateup_raw, launch_down_act), the
 // pre-activations make a round trip and every column block computes the activations again, which pays up to about 80 tiles
-// (expected: an expert's last one half full): H = 768, I = 384, E = 64, k = 6: 62 -> 48 us at T = 128, 68 -> 55 at T = 512, 77 -> 64 at
-// T = 1024, but 79 -> 94 at T = 1500; H = 2048, I = 384, E = 16, k = 4: 132 -> 72 at T = 512.  Lighter experts stream faster and gain
-// less: I = 256 up to about 64 tiles at H = 1024 (E = 16, k = 3: 60 -> 43 at T = 512), 40 at H = 512.
+// (expected: an expert's last one half full).  Whole layer, one set of weights read again and again, uncut -> cut: H = 768,
+// I = 384, E = 64, k = 6: 47 -> 44.5 us at T = 128, 52 -> 51 at T = 512, 66 -> 63 at T = 1024, but 79 -> 94 at T = 1500; H = 1024,
+// I = 512, k = 8: 87 -> 78 at T = 512 (E = 16, k = 3: 79 -> 53 at T = 1000).  Lighter experts stream faster and gain less: I = 256 up to
+// about 64 tiles at H = 1024 (E = 16, k = 3: 60 -> 44 at T = 512), 40 at H = 512 (45 -> 34).  Pre-activations in bf16 were 1 to 5 us
+// faster and half again as far from the exact result (3.5e-3 against 2.3e-3).
 bool split_columns(int S, int E, int H, int I) {
   const int limit = I >= 384 ? 80 : (H * I >= 256 * 1024 ? 64 : 40);
   return S / 128 + E / 2 <= limit && I >= 256;
 }
 
-// gu [S, 2I] bf16 -> routing-weighted rows in slot order (down_act_kernel); shapes as launch_gateup_raw takes them
+// gu [S, 2I] fp32 -> routing-weighted rows in slot order, and with `preact` their bf16 copy (down_act_kernel); shapes as
+// launch_gateup_raw takes them
 hipError_t launch_down_act(const void* gu, const void* wd, const float* theta, const float* w, const int32_t* offsets,
-                           const int32_t* perm_slot, int S, int H, int E, int I, int act, void* yw, hipStream_t s) {
+                           const int32_t* perm_slot, int S, int H, int E, int I, int act, void* yw, void* preact, hipStream_t s) {
   if (S == 0) return hipSuccess;
-  const bf16_t* gp = static_cast<const bf16_t*>(gu);
+  const float* gp = static_cast<const float*>(gu);
+  bf16_t* pp = static_cast<bf16_t*>(preact);
   const bf16_t* dp = static_cast<const bf16_t*>(wd);
   bf16_t* yp = static_cast<bf16_t*>(yw);
   switch (I) {
-    case 128: launch_down_act_nt<1>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yp, s); break;
-    case 256: launch_down_act_nt<2>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yp, s); break;
-    case 384: launch_down_act_nt<3>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yp, s); break;
-    case 512: launch_down_act_nt<4>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yp, s); break;
+    case 128: launch_down_act_nt<1>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yp, pp, s); break;
+    case 256: launch_down_act_nt<2>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yp, pp, s); break;
+    case 384: launch_down_act_nt<3>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yp, pp, s); break;
+    case 512: launch_down_act_nt<4>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yp, pp, s); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
