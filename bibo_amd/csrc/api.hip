@@ -161,10 +161,12 @@ Workspace carve(int T, int H, int E, int k, int I, int dtype) {
   ws.yw = o;
   ws.least = o + align_up(S * (size_t)H * sizeof(float));
   ws.total = o + align_up(S * (size_t)(generic_tiles(H, I, dtype) && 2 * I > H ? 2 * I : H) * sizeof(float));
-  // fp32 pre-activations of a call whose tiles are cut by columns, behind the others
-  ws.pre = ws.total;
-  if (dtype == BIBO_DTYPE_BF16 && mfma_supported(H, I, dtype) && split_columns(T * k, E, H, I))
-    ws.total += align_up(S * (size_t)2 * I * sizeof(float));
+  // fp32 pre-activations of a call whose tiles are cut by columns: behind its slot rows, which are bf16
+  ws.pre = o + align_up(S * (size_t)H * sizeof(bf16_t));
+  if (dtype == BIBO_DTYPE_BF16 && mfma_supported(H, I, dtype) && split_columns(T * k, E, H, I)) {
+    const size_t end = ws.pre + align_up(S * (size_t)2 * I * sizeof(float));
+    if (end > ws.total) ws.total = end;
+  }
   return ws;
 }
 
