@@ -9,6 +9,7 @@
 #include <torch/extension.h>
 
 #include <map>
+#include <memory>
 #include <mutex>
 
 #include "../../include/bibo_moe.h"
@@ -22,28 +23,48 @@ void check(int code, const char* what) {
 }
 
 // ---- workspace: one grow-only byte buffer per (device, stream); calls on one stream are ordered, so they may share it ----
+// A library call is several launches, so a thread keeps its stream's buffer (a Scratch) until the last of them is queued: the
+// autograd thread runs a backward pass while another thread runs a forward on the same stream.
+struct Buffer {
+  std::mutex busy;
+  Tensor bytes;
+};
 struct Pool {
   std::mutex m;
-  std::map<std::pair<int, hipStream_t>, Tensor> buffers;
+  std::map<std::pair<int, hipStream_t>, std::shared_ptr<Buffer>> buffers;
 };
 Pool& pool() {
   static Pool* p = new Pool;             // never destroyed: tensors must not outlive the allocator at exit
   return *p;
 }
 
-Tensor workspace_on(c10::Device dev, hipStream_t stream, size_t bytes) {
-  Pool& p = pool();
-  std::lock_guard<std::mutex> lock(p.m);
-  Tensor& t = p.buffers[{dev.index(), stream}];
-  if (!t.defined() || (size_t)t.numel() < bytes)
-    t = at::empty({(int64_t)std::max<size_t>(bytes, 1)}, at::TensorOptions().dtype(at::kByte).device(dev));
-  return t;
-}
+class Scratch {
+ public:
+  Scratch(c10::Device dev, hipStream_t stream, size_t bytes) : buffer_(find(dev, stream)), lock_(buffer_->busy) {
+    Tensor& t = buffer_->bytes;
+    if (!t.defined() || (size_t)t.numel() < bytes)
+      t = at::empty({(int64_t)std::max<size_t>(bytes, 1)}, at::TensorOptions().dtype(at::kByte).device(dev));
+  }
+  const Tensor& tensor() const { return buffer_->bytes; }
+  void* data_ptr() const { return tensor().data_ptr(); }
+  int64_t numel() const { return tensor().numel(); }
+
+ private:
+  static std::shared_ptr<Buffer> find(c10::Device dev, hipStream_t stream) {
+    Pool& p = pool();
+    std::lock_guard<std::mutex> lock(p.m);
+    std::shared_ptr<Buffer>& b = p.buffers[{dev.index(), stream}];
+    if (!b) b = std::make_shared<Buffer>();
+    return b;
+  }
+  std::shared_ptr<Buffer> buffer_;
+  std::unique_lock<std::mutex> lock_;
+};
 
 Tensor workspace(int device_index, int64_t bytes) {
   const c10::Device dev(c10::DeviceType::CUDA, (c10::DeviceIndex)device_index);
   c10::DeviceGuard guard(dev);
-  return workspace_on(dev, c10::hip::getCurrentHIPStream(dev.index()).stream(), (size_t)bytes);
+  return Scratch(dev, c10::hip::getCurrentHIPStream(dev.index()).stream(), (size_t)bytes).tensor();
 }
 
 void workspace_clear() {
@@ -111,7 +132,7 @@ py::tuple layer_forward(const Tensor& x_, const Tensor& w_router, const Tensor& 
   hipStream_t s = c10::hip::getCurrentHIPStream(x.device().index()).stream();
   size_t bytes = 0;
   check(bibo_moe_workspace_bytes(&sh, &bytes), "bibo_moe_workspace_bytes");
-  const Tensor ws = workspace_on(x.device(), s, bytes);
+  const Scratch ws(x.device(), s, bytes);
   check(bibo_moe_forward(x.data_ptr(), w_router.data_ptr(), f32(bias), w_gate_up.data_ptr(), w_down.data_ptr(), f32(theta), &sh, norm,
                          algo, out.data_ptr(), nullptr, nullptr, int_ptr(counts), nullptr, ws.data_ptr(), (size_t)ws.numel(), s),
         "bibo_moe_forward");
@@ -144,7 +165,7 @@ py::tuple ffn_forward(const Tensor& h, const Tensor& norm_weight, double eps, co
   hipStream_t s = c10::hip::getCurrentHIPStream(x.device().index()).stream();
   size_t bytes = 0;
   check(bibo_moe_ffn_workspace_bytes(&sh, &bytes), "bibo_moe_ffn_workspace_bytes");
-  const Tensor ws = workspace_on(x.device(), s, bytes);
+  const Scratch ws(x.device(), s, bytes);
   check(bibo_moe_ffn_forward(x.data_ptr(), f32(nw), (float)eps, res.defined() ? res.data_ptr() : nullptr,
                              w_router.data_ptr(), f32(bias), w_gate_up.data_ptr(), w_down.data_ptr(), f32(theta), &sh, norm, algo,
                              out.data_ptr(), nullptr, nullptr, int_ptr(counts), ws.data_ptr(), (size_t)ws.numel(), s),
@@ -176,7 +197,7 @@ class LayerFn : public torch::autograd::Function<LayerFn> {
     hipStream_t s = c10::hip::getCurrentHIPStream(xb.device().index()).stream();
     size_t bytes = 0, state_bytes = 0;
     check(bibo_moe_workspace_bytes(&sh, &bytes), "bibo_moe_workspace_bytes");
-    const Tensor ws = workspace_on(xb.device(), s, bytes);
+    const Scratch ws(xb.device(), s, bytes);
     const bool saved = c->keep && (l.algo == BIBO_ALGO_AUTO || l.algo == BIBO_ALGO_FUSED) &&
                        bibo_moe_train_state_bytes(&sh, &state_bytes) == BIBO_OK;
     Tensor last;           // the state or, where the backward pass routes again, the selection biases
@@ -226,7 +247,7 @@ class LayerFn : public torch::autograd::Function<LayerFn> {
     hipStream_t s = c10::hip::getCurrentHIPStream(x.device().index()).stream();
     size_t bytes = 0;
     check(bibo_moe_backward_workspace_bytes(&sh, &bytes), "bibo_moe_backward_workspace_bytes");
-    const Tensor ws = workspace_on(x.device(), s, bytes);
+    const Scratch ws(x.device(), s, bytes);
     if (saved)
       check(bibo_moe_backward_saved(x.data_ptr(), d.data_ptr(), l.w_router.data_ptr(), l.w_gate_up.data_ptr(), l.w_down.data_ptr(),
                                     f32(l.theta), &sh, l.norm, last.data_ptr(), (size_t)last.numel(), d_x.data_ptr(),
