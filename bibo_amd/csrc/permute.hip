@@ -57,7 +57,10 @@ __global__ __launch_bounds__(256) void hist_blocksum_kernel(const int32_t* __res
 // HT = tokens per histogram in `hist`: kPermTokens for hist_kernel's output (the wave counts its own slots
 // with ballots), 16 or 32 for the histograms the router kernel wrote per workgroup (a wave's count is the sum
 // of its 32/HT histograms and no counting pass is needed).
-template <int HT>
+// BATCH = histograms a wave requests together.  They are read whether a call has them or not (past the end: the last one again,
+// counted as zero), and each costs the wave 40 ns, so few histograms get a short batch: 6.7 -> 4.2 us at 32 of them (T = 512),
+// 6.3 -> 4.7 at 49.  Wave index and bounds are scalar: under per-lane conditions 256 of them took 7.3 us instead of 6.5 (T = 8192).
+template <int HT, int BATCH>
 __global__ __launch_bounds__(256) void scatter_kernel(const int32_t* __restrict__ idx, int S, int E, int k,
                                                       const int32_t* __restrict__ hist, int nhist,
                                                       const int32_t* __restrict__ block_sum,
@@ -65,7 +68,7 @@ __global__ __launch_bounds__(256) void scatter_kernel(const int32_t* __restrict_
                                                       int32_t* __restrict__ perm_slot, int32_t* __restrict__ perm_token) {
   static_assert(kPermTokens == 128 && (HT == kPermTokens || HT == 16 || HT == 32), "a wave owns 32 tokens");
   __shared__ int part_tot[4][kMaxE], part_bef[4][kMaxE], wave_cnt[4][kMaxE];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int b = blockIdx.x;
   const int s0 = (b * kPermTokens + wave * (kPermTokens / 4)) * k;
   const int s1 = min(S, s0 + (kPermTokens / 4) * k);
@@ -103,22 +106,23 @@ __global__ __launch_bounds__(256) void scatter_kernel(const int32_t* __restrict_
   wave_cnt[wave][lane] = mycnt;
 
   int tot = 0, bef = 0;
-  constexpr int kBatch = 64;                       // histograms requested together: one memory latency per batch
-  if (block_sum == nullptr) {
+  constexpr int kBatch = BATCH;                    // histograms requested together: one memory latency per batch
+  if (BATCH < 64 || block_sum == nullptr) {
     for (int bb0 = wave; bb0 < nhist; bb0 += 4 * kBatch) {
       int v[kBatch];
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
-        const int bb = bb0 + 4 * u;
-        v[u] = (bb < nhist) ? hist[bb * kMaxE + lane] : 0;
+        const int bb = min(bb0 + 4 * u, nhist - 1);
+        v[u] = (hist + (size_t)bb * kMaxE)[lane];
       }
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
-        tot += v[u];
-        bef += (bb0 + 4 * u < h0) ? v[u] : 0;
+        const int bb = bb0 + 4 * u;
+        tot += v[u] & (bb < nhist ? -1 : 0);
+        bef += v[u] & (bb < min(h0, nhist) ? -1 : 0);
       }
     }
-  } else {
+  } else if constexpr (BATCH == 64) {
     // two levels: the sums of whole blocks of histograms, then the histograms of this workgroup's own block in front
     // of its first one
     static_assert(kHistBlock == 4 * kBatch, "one batch per wave covers a block");
@@ -127,7 +131,7 @@ __global__ __launch_bounds__(256) void scatter_kernel(const int32_t* __restrict_
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
       const int bb = hb * kHistBlock + wave + 4 * u;
-      v[u] = (bb < h0) ? hist[bb * kMaxE + lane] : 0;
+      v[u] = (hist + (size_t)min(bb, nhist - 1) * kMaxE)[lane] & (bb < h0 ? -1 : 0);
     }
     for (int blk = wave; blk < nblk; blk += 4) {
       const int bs = block_sum[blk * kMaxE + lane];
@@ -252,6 +256,19 @@ static const int32_t* block_sums(int32_t* hist, int nhist, hipStream_t s) {
   return sums;
 }
 
+template <int HT>
+static void launch_scatter(const int32_t* idx, int S, int E, int k, const int32_t* hist, int nhist, const int32_t* block_sum, int grid,
+                           int32_t* counts, int32_t* offsets, int32_t* perm_slot, int32_t* perm_token, hipStream_t s) {
+  auto launch = [&](auto batch) {
+    hipLaunchKernelGGL((scatter_kernel<HT, decltype(batch)::value>), dim3(grid), dim3(256), 0, s, idx, S, E, k, hist, nhist, block_sum,
+                       counts, offsets, perm_slot, perm_token);
+  };
+  if (nhist <= 4 * 8) launch(std::integral_constant<int, 8>());
+  else if (nhist <= 4 * 24) launch(std::integral_constant<int, 24>());
+  else if (nhist <= 4 * 48) launch(std::integral_constant<int, 48>());
+  else launch(std::integral_constant<int, 64>());
+}
+
 hipError_t launch_permute(const int32_t* idx, int T, int E, int k, int32_t* counts, int32_t* offsets,
                           int32_t* perm_slot, int32_t* perm_token, void* ws, hipStream_t s) {
   const int nblk = (T + kPermTokens - 1) / kPermTokens;
@@ -264,8 +281,8 @@ hipError_t launch_permute(const int32_t* idx, int T, int E, int k, int32_t* coun
   }
   const int grid = nblk;
   hipLaunchKernelGGL(hist_kernel, dim3(grid), dim3(256), 0, s, idx, S, E, k, block_hist);
-  hipLaunchKernelGGL(scatter_kernel<kPermTokens>, dim3(grid), dim3(256), 0, s, idx, S, E, k, block_hist, grid,
-                     block_sums(block_hist, grid, s), counts, offsets, perm_slot, perm_token);
+  launch_scatter<kPermTokens>(idx, S, E, k, block_hist, grid, block_sums(block_hist, grid, s), grid, counts, offsets, perm_slot,
+                              perm_token, s);
   return hipGetLastError();
 }
 
@@ -279,11 +296,9 @@ hipError_t launch_permute_from_hist(const int32_t* idx, int T, int E, int k, int
   const int grid = (T + kPermTokens - 1) / kPermTokens;
   const int nhist = (T + hist_tokens - 1) / hist_tokens;
   if (hist_tokens == 32)
-    hipLaunchKernelGGL(scatter_kernel<32>, dim3(grid), dim3(256), 0, s, idx, T * k, E, k, hist, nhist,
-                       block_sums(hist, nhist, s), counts, offsets, perm_slot, perm_token);
+    launch_scatter<32>(idx, T * k, E, k, hist, nhist, block_sums(hist, nhist, s), grid, counts, offsets, perm_slot, perm_token, s);
   else if (hist_tokens == 16)   // (fewer than 8192 tokens: never enough histograms for block sums, and no room for them)
-    hipLaunchKernelGGL(scatter_kernel<16>, dim3(grid), dim3(256), 0, s, idx, T * k, E, k, hist, nhist,
-                       static_cast<const int32_t*>(nullptr), counts, offsets, perm_slot, perm_token);
+    launch_scatter<16>(idx, T * k, E, k, hist, nhist, nullptr, grid, counts, offsets, perm_slot, perm_token, s);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();

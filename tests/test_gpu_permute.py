@@ -65,3 +65,16 @@ def test_router_output_feeds_the_permutation():
     assert np.array_equal(np.sort(ps), np.arange(idx_np.size))
     assert (np.bincount(perm_token.cpu().numpy(), minlength=512) == 6).all()
     assert (np.diff(idx_np.reshape(-1)[ps]) >= 0).all()
+
+
+@pytest.mark.parametrize("n", [32, 33, 96, 97, 192, 193, 256, 257])
+def test_histogram_counts_around_the_batches(n):
+    """n histograms of 128 tokens (its own launch) and of 16 or 32 tokens (the router's): a wave requests 8, 24, 48 or 64 at once."""
+    _check(_random_idx(128 * n - 5, 16, 2, n), 16)
+    T = (16 if 16 * n < 8192 else 32) * n - 3
+    p = O.make_inputs(T=T, H=128, E=16, k=2, I=128, seed=n)
+    x, *ops_in = (p[name].to("cuda:0") for name in ("x", "w_router", "bias", "w_gate_up", "w_down", "theta"))
+    out, idx, w, counts, _ = ops.moe_forward(x, *ops_in, 2, algo="fused", want_routing=True, want_counts=True)
+    again, counts2 = ops.experts_fwd(x, idx, w, *ops_in[2:], algo="fused", want_counts=True)
+    assert torch.equal(counts, counts2) and torch.equal(out, again)
+    assert np.array_equal(counts.cpu().numpy(), np.bincount(idx.cpu().numpy().ravel(), minlength=16))
