@@ -212,7 +212,6 @@ class BiBoExpAttention(nn.Module):
         self.k_norm = RMSNorm(d, config.rms_norm_eps) if qk_norm else nn.Identity()
         self.xsa_alpha = (nn.Parameter(torch.full((self.num_heads,), float(config.xsa_alpha_init)))
                           if config.use_xsa else None)
-        _lay_out(self.q_proj, self.k_proj, self.v_proj)
 
     def _apply(self, fn, *a, **kw):
         out = super()._apply(fn, *a, **kw)
@@ -269,7 +268,6 @@ class BiBoExpMLP(nn.Module):
         self.gate_proj = nn.Linear(config.hidden_size, config.intermediate_size, bias=False)
         self.up_proj = nn.Linear(config.hidden_size, config.intermediate_size, bias=False)
         self.down_proj = nn.Linear(config.intermediate_size, config.hidden_size, bias=False)
-        _lay_out(self.gate_proj, self.up_proj)
 
     def _apply(self, fn, *a, **kw):
         out = super()._apply(fn, *a, **kw)
