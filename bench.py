@@ -358,8 +358,8 @@ def full_model(dev, batch=8, seq=2048, steps=10, warmup=3):
             "tokens_per_s": batch * seq / sec, "ms_per_forward": sec * 1e3, "ms_per_forward_runs": [r * 1e3 for r in runs],
             "logits_finite": finite, "params": sum(p.numel() for p in model.parameters()),
             "note": "HIP MoE block per layer through bibo_moe_ffn_forward (norm + block + residual in one call), HIP depth "
-                    "mix (bibo_moe_exp_attn_res_fwd) and row norms (bibo_moe_rmsnorm_fwd); attention, dense layers and the "
-                    "head are stock PyTorch-ROCm operations"}
+                    "mix + norm, QK-norm + RoPE, attention with XSA, residual sums and SwiGLU product (bibo_moe_exp_*); the "
+                    "dense products and the head are library GEMMs"}
 
 
 def main():
