@@ -94,14 +94,25 @@ class _CastCache:
 
     A change is seen through the parameter's storage address, version counter, device and dtype.  In-place writes
     through `p.data` (`p.data.copy_(...)`, `p.data.fill_(...)`) bump none of them; after such a write call
-    `invalidate()` (the modules below expose it as `refresh_weights()`), as `load_state_dict` and `Module._apply`
-    (`.to()`, `.cuda()`, `.bfloat16()`) do by themselves here."""
+    `invalidate()` (the modules below expose it as `refresh_weights()`), as `load_state_dict` does by itself here;
+    `Module._apply` (`.to()`, `.cuda()`, `.bfloat16()`) calls `after_move()`."""
 
     def __init__(self):
         self._store = {}
 
     def invalidate(self):
         self._store.clear()
+
+    @torch.no_grad()
+    def after_move(self, **params):
+        """Copies of parameters that a move has left where they were keep their memory, which a captured graph reads, and take
+        the values anew; the others are dropped."""
+        for (name, dtype), (tag, copy) in list(self._store.items()):
+            p = params[name]
+            if tag == (p.data_ptr(), p._version, p.device, p.dtype):
+                copy.data.copy_(p)
+            else:
+                del self._store[name, dtype]
 
     def get(self, name: str, p: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
         if p.dtype == dtype and p.is_contiguous():
@@ -150,8 +161,9 @@ class BiBoMoERouter(nn.Module):
         self._cache.invalidate()
 
     def _apply(self, fn, *a, **kw):
-        self._cache.invalidate()
-        return super()._apply(fn, *a, **kw)
+        out = super()._apply(fn, *a, **kw)
+        self._cache.after_move(w=self.gate_proj.weight, b=self.bias)
+        return out
 
     def _operands(self, hidden_states):
         cd = _compute_dtype(hidden_states)
@@ -238,8 +250,9 @@ class BiBoFusedExperts(nn.Module):
         self._cache.invalidate()
 
     def _apply(self, fn, *a, **kw):
-        self._cache.invalidate()
-        return super()._apply(fn, *a, **kw)
+        out = super()._apply(fn, *a, **kw)
+        self._cache.after_move(gu=self.gate_up_proj, dn=self.down_proj, th=self.radial_theta)
+        return out
 
     def _weights(self, cd):
         return (self._cache.get("gu", self.gate_up_proj, cd), self._cache.get("dn", self.down_proj, cd),

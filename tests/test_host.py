@@ -255,6 +255,23 @@ def test_cast_cache_refreshes_on_load_and_on_request():
     assert not layer.experts._cache._store
 
 
+def test_kernel_dtype_copies_keep_their_memory_over_a_move_that_moves_nothing():
+    """A captured graph reads the copies, so `.to()` of the device and type a layer has must not free them; it takes up what was
+    written through `.data`.  A copy whose parameter did move is dropped."""
+    layer = bibo_amd.BiBoMoELayer(make_config())
+    e, g = layer.experts, layer.gate
+    held = {(m, n): m._cache.get(n, p, torch.bfloat16) for m, n, p in ((e, "gu", e.gate_up_proj), (e, "th", e.radial_theta),
+                                                                       (g, "w", g.gate_proj.weight), (g, "b", g.bias))}
+    e.radial_theta.data.fill_(3.0)
+    for move in (lambda: layer.to("cpu"), lambda: layer.float(), lambda: layer.cpu()):
+        move()
+        for (m, n), copy in held.items():
+            assert m._cache._store[n, torch.bfloat16][1] is copy
+    assert float(held[e, "th"][0]) == 3.0
+    layer.double()
+    assert not e._cache._store and not g._cache._store
+
+
 def test_specials_and_shared_expert_follow_the_reference_layout():
     """moe.py:19-44,118-127: the weight tensors hold only the GLU experts, the router has a row per routed expert
     (specials included), the shared expert is a SwiGLU of width moe_intermediate_size * num_shared_experts."""
