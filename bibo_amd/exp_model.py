@@ -126,19 +126,26 @@ def _native_ok(x) -> bool:
             and not (torch.is_autocast_enabled() and torch.get_autocast_dtype("cuda") != torch.bfloat16))
 
 
-def _lay_out(*linears):
-    """The layers' weights one behind the other in one block of GPU memory, so that one product reads them all in place.  They
-    stay parameters of their own; wherever they end up elsewhere (a copy, a replaced parameter) the native call joins them."""
+def _weights_held(*linears):
+    """The storages of the layers' weights, held so that no address of theirs is given out again (None: no plain parameter)."""
     ps = [m._parameters.get("weight") for m in linears]
-    if not all(type(p) is nn.Parameter and type(p.data) is torch.Tensor and p.is_cuda and p.is_contiguous() and not p.is_inference()
-               and p.dtype == ps[0].dtype and p.device == ps[0].device for p in ps):
+    if not all(type(p) is nn.Parameter and type(p.data) is torch.Tensor for p in ps):
+        return None
+    return [p.untyped_storage() for p in ps]
+
+
+def _lay_out(held, *linears):
+    """The layers' weights one behind the other in one block of GPU memory, so that one product reads them all in place: after a
+    move that gave every one of them a storage of its own (`held`: the storages before it).  A move that leaves them where they
+    are (`.to()` of the device and type they have) leaves them alone: captured graphs, assigned state dicts and flat buffers
+    read and write them there.  They stay parameters of their own; wherever they lie apart the native call joins them."""
+    ps = [m._parameters.get("weight") for m in linears]
+    if held is None or not all(
+            type(p) is nn.Parameter and type(p.data) is torch.Tensor and p.is_cuda and p.is_contiguous() and not p.is_inference()
+            and p.dtype == ps[0].dtype and p.device == ps[0].device
+            and p.untyped_storage().nbytes() == p.numel() * p.element_size() for p in ps):
         return
-    at = ps[0].data_ptr()
-    for p in ps:
-        if p.data_ptr() != at or p.untyped_storage().data_ptr() != ps[0].untyped_storage().data_ptr():
-            break
-        at += p.numel() * p.element_size()
-    else:
+    if {p.data_ptr() for p in ps} & {s.data_ptr() for s in held}:
         return
     with torch.no_grad():
         block = torch.cat([p.data for p in ps])
@@ -214,8 +221,9 @@ class BiBoExpAttention(nn.Module):
                           if config.use_xsa else None)
 
     def _apply(self, fn, *a, **kw):
+        held = _weights_held(self.q_proj, self.k_proj, self.v_proj)
         out = super()._apply(fn, *a, **kw)
-        _lay_out(self.q_proj, self.k_proj, self.v_proj)
+        _lay_out(held, self.q_proj, self.k_proj, self.v_proj)
         return out
 
     def _native(self, x, cos, sin):
@@ -270,8 +278,9 @@ class BiBoExpMLP(nn.Module):
         self.down_proj = nn.Linear(config.intermediate_size, config.hidden_size, bias=False)
 
     def _apply(self, fn, *a, **kw):
+        held = _weights_held(self.gate_proj, self.up_proj)
         out = super()._apply(fn, *a, **kw)
-        _lay_out(self.gate_proj, self.up_proj)
+        _lay_out(held, self.gate_proj, self.up_proj)
         return out
 
     def forward(self, x):

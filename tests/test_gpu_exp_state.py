@@ -142,6 +142,47 @@ def test_weights_lie_in_one_block_until_one_is_replaced():
     assert torch.equal(model.float().to(torch.bfloat16)(ids), want)
 
 
+@torch.no_grad()
+@pytest.mark.parametrize("source", ["built", "assigned", "flat"])
+def test_a_move_that_moves_nothing_leaves_the_weights_where_they_are(source):
+    model, ids = _model(), _ids(2, 20, 1)
+    want = model(ids)
+    tensors = {n: p.detach().clone() for n, p in model.named_parameters()}
+    if source == "built":                            # on the device and in the type of every later move
+        for m in model.modules():
+            if isinstance(m, torch.nn.Linear):
+                m.weight = torch.nn.Parameter(m.weight.clone())
+    elif source == "assigned":
+        model.load_state_dict(tensors, strict=False, assign=True)
+    else:                                            # views of a flat buffer with gaps between them
+        flat = torch.zeros(sum(t.numel() + 128 for t in tensors.values()), dtype=torch.bfloat16, device=DEV)
+        at = 0
+        for n, p in model.named_parameters():
+            p.data = flat[at:at + p.numel()].view_as(p).copy_(tensors[n])
+            tensors[n] = p.data
+            at += (p.numel() + 127) // 64 * 64
+    where = {n: p.data_ptr() for n, p in model.named_parameters()}
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream(device=DEV)
+    side.wait_stream(torch.cuda.current_stream(DEV))
+    with torch.cuda.stream(side):
+        model(ids)
+    side.synchronize()
+    with torch.cuda.graph(graph, stream=side):
+        out = model(ids)
+    for move in (lambda: model.cuda(), lambda: model.to(DEV), lambda: model.to(torch.bfloat16), lambda: model.bfloat16()):
+        move()
+        assert {n: p.data_ptr() for n, p in model.named_parameters()} == where
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(out, want) and torch.equal(model(ids), want)
+    if source != "built":                            # a write through the other name of a weight is seen
+        tensors["model.layers.1.self_attn.v_proj.weight"].mul_(2.0)
+        changed = model(ids)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert not torch.equal(changed, want) and torch.equal(out, changed)
+
+
 @pytest.mark.parametrize("S,half,dtype", [(1, 32, torch.float32), (77, 96, torch.float32), (2048, 64, torch.bfloat16)])
 def test_rope_tables_give_the_bits_of_the_tensor_operations(S, half, dtype):
     inv = (10000.0 ** (-torch.arange(0, half, dtype=torch.float32) / half)).to(DEV, dtype)
