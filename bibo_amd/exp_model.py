@@ -112,10 +112,11 @@ def _fp32_copy(module, name):
 
 def _plain(*modules) -> bool:
     """The modules are the ones built here and nobody observes their own calls: their work may be done inside another launch.
-    A wrapped or subclassed projection (an adapter, a parametrization), a replaced forward and hooks run as modules."""
+    A wrapped or subclassed projection (an adapter, a parametrization), a replaced forward, on the module or on its class, and
+    hooks run as modules."""
     g = nn.modules.module
     return not (g._global_forward_hooks or g._global_forward_pre_hooks) and all(
-        type(m) in (nn.Linear, RMSNorm, nn.Identity, BiBoExpMLP) and not m._forward_hooks and not m._forward_pre_hooks
+        _METHODS.get(type(m)) == (type(m).forward, type(m).__call__) and not m._forward_hooks and not m._forward_pre_hooks
         and "forward" not in m.__dict__ and m._parameters.get("bias") is None for m in modules)
 
 
@@ -293,6 +294,10 @@ class BiBoExpMLP(nn.Module):
                 and all(p.weight.dtype == torch.bfloat16 for p in projs) and _plain(self, *projs)):
             return L.native().exp_mlp(x, *(p.weight for p in projs), base)
         return base + self(x)
+
+
+# what a call of the modules whose work other launches take over runs, unless somebody replaces it
+_METHODS = {cls: (cls.forward, cls.__call__) for cls in (nn.Linear, nn.Identity, RMSNorm, BiBoExpMLP)}
 
 
 class BiBoExpDecoderLayer(nn.Module):

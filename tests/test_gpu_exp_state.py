@@ -93,6 +93,33 @@ def test_replaced_and_observed_modules_are_called(name, how):
 
 
 @torch.no_grad()
+@pytest.mark.parametrize("cls,method", [(X.RMSNorm, "forward"), (X.RMSNorm, "__call__"), (torch.nn.Linear, "forward"), (X.BiBoExpMLP, "forward")])
+def test_methods_replaced_on_the_class_are_called(cls, method, monkeypatch):
+    model, ids, seen = _model(), _ids(2, 20, 1), set()
+    want = model(ids)
+    plain = getattr(cls, method)
+    monkeypatch.setattr(cls, method, lambda self, x: seen.add(self) or plain(self, x))
+    got = model(ids)
+    layers, dense = model.model.layers, [l for l in model.model.layers if not l.is_moe_layer]
+    if cls is X.RMSNorm:
+        expected = {model.model.norm, *(l.post_attention_layernorm for l in dense)}
+        for l in layers:
+            expected |= {l.input_layernorm, l.self_attn.q_norm, l.self_attn.k_norm}
+    elif cls is torch.nn.Linear:
+        expected = {model.lm_head, *(m for l in layers for m in (l.self_attn.q_proj, l.self_attn.k_proj, l.self_attn.v_proj, l.self_attn.o_proj)),
+                    *(m for l in dense for m in (l.mlp.gate_proj, l.mlp.up_proj, l.mlp.down_proj))}
+    else:
+        expected = {l.mlp for l in dense}
+    assert expected <= seen
+    monkeypatch.undo()
+    assert torch.equal(model(ids), want)
+    for m in model.modules():                        # observed modules run by themselves too: the same route, the same bits
+        if type(m) is cls:
+            m.register_forward_hook(lambda *a: None)
+    assert torch.equal(model(ids), got)
+
+
+@torch.no_grad()
 @pytest.mark.parametrize("H,S", [(256, 33), (768, 5)])
 def test_bf16_vectors_give_the_bits_of_their_fp32_copies(H, S):
     g = torch.Generator().manual_seed(H + S)
