@@ -387,10 +387,10 @@ class BiBoMoELayer(nn.Module):
         return tpe
 
     def _balance(self, counts, num_tokens):
-        """_balance_step and update_bias of this forward in one launch, where neither is overridden, the state is fp32 on the
-        GPU and no process group has to see the counts first."""
+        """_balance_step and update_bias of this forward in one launch, where neither is overridden or replaced, the state is fp32 on
+        the GPU and no process group has to see the counts first."""
         cls, bias, acc = type(self), _param(self._modules["gate"], "bias"), self.accumulated_tpe
-        if (cls._balance_step is BiBoMoELayer._balance_step and cls.update_bias is BiBoMoELayer.update_bias
+        if ((cls._balance_step, cls.update_bias) == _BALANCING
                 and "update_bias" not in self.__dict__ and "_balance_step" not in self.__dict__
                 and counts is not None and counts.is_cuda and acc.device == bias.device == counts.device
                 and acc.dtype == bias.dtype == torch.float32 and acc.is_contiguous() and bias.is_contiguous()):
@@ -509,3 +509,6 @@ class BiBoMoELayer(nn.Module):
         if balancing:                                          # exactly once per training forward
             self._balance(counts, num_tokens)
         return out.to(torch.bfloat16) if bf16_stream else out
+
+
+_BALANCING = (BiBoMoELayer._balance_step, BiBoMoELayer.update_bias)      # unless somebody replaces them on the class

@@ -40,3 +40,14 @@ def test_training_forwards_move_the_bias_as_the_tensor_operations_do():
         assert (layer.gate.bias._version > version) == (step % 2 == 1)
         assert torch.equal(layer.accumulated_tpe, plain.accumulated_tpe)
         assert torch.allclose(layer.gate.bias, plain.gate.bias, rtol=0, atol=1e-8)
+
+
+@pytest.mark.parametrize("method", ["update_bias", "_balance_step"])
+def test_balancing_methods_replaced_on_the_class_are_called(method, monkeypatch):
+    cfg = bibo_amd.BiBoMoEConfig(hidden_size=128, moe_intermediate_size=128, num_routed_experts=16, num_experts_per_tok=4,
+                                 special_expert_pairs=0, bias_update_threshold=60)
+    layer, seen = bibo_amd.BiBoMoELayer(cfg).to(DEV), []
+    plain = getattr(bibo_amd.BiBoMoELayer, method)
+    monkeypatch.setattr(bibo_amd.BiBoMoELayer, method, lambda self, *a, **kw: seen.append(1) or plain(self, *a, **kw))
+    layer(torch.randn(1, 60, 128, device=DEV))
+    assert seen == [1]
