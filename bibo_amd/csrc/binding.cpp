@@ -192,7 +192,8 @@ class LayerFn : public torch::autograd::Function<LayerFn> {
                         const Tensor& w_down, const Tensor& theta, TrainCall* c) {
     const Layer& l = c->l;
     const Tensor xb = in_dtype(x, c->compute);
-    const bibo_moe_shape sh = shape_of(xb, l, BIBO_FLAG_TRAIN_AUTO);
+    // a family that was asked for by name runs in training as well
+    const bibo_moe_shape sh = shape_of(xb, l, l.algo == BIBO_ALGO_AUTO ? BIBO_FLAG_TRAIN_AUTO : 0);
     Tensor out = at::empty_like(xb);
     hipStream_t s = c10::hip::getCurrentHIPStream(xb.device().index()).stream();
     size_t bytes = 0, state_bytes = 0;

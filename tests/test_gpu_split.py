@@ -74,3 +74,19 @@ def test_training_on_cut_tiles():
         out.backward(d)
         grads.append([xg.grad] + [p.grad for p in layer.parameters() if p.requires_grad])
     assert all(torch.equal(a, b) for a, b in zip(*grads))
+
+
+@pytest.mark.parametrize("algo", ["fused", "mfma"])
+def test_a_named_family_runs_in_training_too(algo):
+    """A layer asked for a family by name runs it in training as in inference: the same bits, also where `auto` cuts the tiles."""
+    torch.manual_seed(0)
+    cfg = bibo_amd.BiBoMoEConfig(hidden_size=768, moe_intermediate_size=384, num_routed_experts=16, num_experts_per_tok=3,
+                                 special_expert_pairs=0, bias_update_factor=0.0)
+    layer = bibo_amd.BiBoMoELayer(cfg).to(DEV).bfloat16()
+    x = torch.randn(1, 500, 768, device=DEV).bfloat16()
+    with torch.no_grad():
+        auto = layer(x)
+        layer.experts.algo = algo
+        plain = layer(x)
+    assert not torch.equal(plain, auto)                 # `auto` does cut here
+    assert torch.equal(layer(x.clone().requires_grad_()), plain)
