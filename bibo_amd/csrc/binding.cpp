@@ -25,12 +25,18 @@ void check(int code, const char* what) {
 // ---- workspace: one grow-only byte buffer per (device, stream); calls on one stream are ordered, so they may share it ----
 // A library call is several launches, so a thread keeps its stream's buffer (a Scratch) until the last of them is queued: the
 // autograd thread runs a backward pass while another thread runs a forward on the same stream.
+//
+// Order of locks: nobody waits for a buffer with the interpreter lock in hand, and nothing is allocated or dropped with a
+// buffer in hand (a tensor that Python has seen takes the interpreter lock when it goes, and so does an allocation with
+// memory recording on).  A Python caller (Held) runs Python code with a buffer in hand, in which a finaliser may call the
+// library again: the same thread may take its buffer twice.  The inner call's launches then lie whole between two of the
+// outer's statements, and the outer holds the tensor it began with.
 struct Buffer {
-  std::mutex busy;
+  std::recursive_mutex busy;
   Tensor bytes;
 };
 struct Pool {
-  std::mutex m;
+  std::mutex m;                          // held for a look-up only
   std::map<std::pair<int, hipStream_t>, std::shared_ptr<Buffer>> buffers;
 };
 Pool& pool() {
@@ -40,14 +46,19 @@ Pool& pool() {
 
 class Scratch {
  public:
-  Scratch(c10::Device dev, hipStream_t stream, size_t bytes) : buffer_(find(dev, stream)), lock_(buffer_->busy) {
-    Tensor& t = buffer_->bytes;
-    if (!t.defined() || (size_t)t.numel() < bytes)
-      t = at::empty({(int64_t)std::max<size_t>(bytes, 1)}, at::TensorOptions().dtype(at::kByte).device(dev));
+  Scratch(c10::Device dev, hipStream_t stream, size_t bytes) : buffer_(find(dev, stream)), lock_(buffer_->busy, std::defer_lock) {
+    take();
+    if (small(bytes)) {
+      lock_.unlock();
+      spare_ = at::empty({(int64_t)std::max<size_t>(bytes, 1)}, at::TensorOptions().dtype(at::kByte).device(dev));
+      take();
+      if (small(bytes)) std::swap(buffer_->bytes, spare_);       // (or another thread has been here: the spare one goes)
+    }
+    bytes_ = buffer_->bytes;
   }
-  const Tensor& tensor() const { return buffer_->bytes; }
-  void* data_ptr() const { return tensor().data_ptr(); }
-  int64_t numel() const { return tensor().numel(); }
+  const Tensor& tensor() const { return bytes_; }
+  void* data_ptr() const { return bytes_.data_ptr(); }
+  int64_t numel() const { return bytes_.numel(); }
 
  private:
   static std::shared_ptr<Buffer> find(c10::Device dev, hipStream_t stream) {
@@ -57,20 +68,52 @@ class Scratch {
     if (!b) b = std::make_shared<Buffer>();
     return b;
   }
+  bool small(size_t bytes) const { return !buffer_->bytes.defined() || (size_t)buffer_->bytes.numel() < bytes; }
+  void take() {
+    if (lock_.try_lock()) return;
+    if (PyGILState_Check()) {
+      py::gil_scoped_release no_gil;
+      lock_.lock();
+    } else {
+      lock_.lock();
+    }
+  }
+  // destroyed from the last to the first: the tensors go after the lock
   std::shared_ptr<Buffer> buffer_;
-  std::unique_lock<std::mutex> lock_;
+  Tensor spare_, bytes_;
+  std::unique_lock<std::recursive_mutex> lock_;
 };
 
-Tensor workspace(int device_index, int64_t bytes) {
+std::unique_ptr<Scratch> scratch_of(int device_index, int64_t bytes) {
   const c10::Device dev(c10::DeviceType::CUDA, (c10::DeviceIndex)device_index);
   c10::DeviceGuard guard(dev);
-  return Scratch(dev, c10::hip::getCurrentHIPStream(dev.index()).stream(), (size_t)bytes).tensor();
+  return std::make_unique<Scratch>(dev, c10::hip::getCurrentHIPStream(dev.index()).stream(), (size_t)bytes);
 }
 
+// the current stream's buffer as a Python context: (address, size), nobody else's until it ends
+class Held {
+ public:
+  Held(int device_index, int64_t bytes) : device_index_(device_index), bytes_(bytes) {}
+  std::pair<uintptr_t, int64_t> enter() {
+    scratch_ = scratch_of(device_index_, bytes_);
+    return {reinterpret_cast<uintptr_t>(scratch_->data_ptr()), scratch_->numel()};
+  }
+  void exit(py::args) { scratch_.reset(); }
+
+ private:
+  int device_index_;
+  int64_t bytes_;
+  std::unique_ptr<Scratch> scratch_;
+};
+
+// the same as a tensor, to look at or to fill: calls that use it take it as above
+Tensor workspace(int device_index, int64_t bytes) { return scratch_of(device_index, bytes)->tensor(); }
+
 void workspace_clear() {
+  std::map<std::pair<int, hipStream_t>, std::shared_ptr<Buffer>> gone;       // goes after the lock
   Pool& p = pool();
   std::lock_guard<std::mutex> lock(p.m);
-  p.buffers.clear();
+  gone.swap(p.buffers);
 }
 
 // ---- operands ----------------------------------------------------------------------------------------------------
@@ -132,10 +175,12 @@ py::tuple layer_forward(const Tensor& x_, const Tensor& w_router, const Tensor& 
   hipStream_t s = c10::hip::getCurrentHIPStream(x.device().index()).stream();
   size_t bytes = 0;
   check(bibo_moe_workspace_bytes(&sh, &bytes), "bibo_moe_workspace_bytes");
-  const Scratch ws(x.device(), s, bytes);
-  check(bibo_moe_forward(x.data_ptr(), w_router.data_ptr(), f32(bias), w_gate_up.data_ptr(), w_down.data_ptr(), f32(theta), &sh, norm,
-                         algo, out.data_ptr(), nullptr, nullptr, int_ptr(counts), nullptr, ws.data_ptr(), (size_t)ws.numel(), s),
-        "bibo_moe_forward");
+  {
+    const Scratch ws(x.device(), s, bytes);
+    check(bibo_moe_forward(x.data_ptr(), w_router.data_ptr(), f32(bias), w_gate_up.data_ptr(), w_down.data_ptr(), f32(theta), &sh, norm,
+                           algo, out.data_ptr(), nullptr, nullptr, int_ptr(counts), nullptr, ws.data_ptr(), (size_t)ws.numel(), s),
+          "bibo_moe_forward");
+  }
   return py::make_tuple(out, maybe(counts));
 }
 
@@ -165,11 +210,13 @@ py::tuple ffn_forward(const Tensor& h, const Tensor& norm_weight, double eps, co
   hipStream_t s = c10::hip::getCurrentHIPStream(x.device().index()).stream();
   size_t bytes = 0;
   check(bibo_moe_ffn_workspace_bytes(&sh, &bytes), "bibo_moe_ffn_workspace_bytes");
-  const Scratch ws(x.device(), s, bytes);
-  check(bibo_moe_ffn_forward(x.data_ptr(), f32(nw), (float)eps, res.defined() ? res.data_ptr() : nullptr,
-                             w_router.data_ptr(), f32(bias), w_gate_up.data_ptr(), w_down.data_ptr(), f32(theta), &sh, norm, algo,
-                             out.data_ptr(), nullptr, nullptr, int_ptr(counts), ws.data_ptr(), (size_t)ws.numel(), s),
-        "bibo_moe_ffn_forward");
+  {
+    const Scratch ws(x.device(), s, bytes);
+    check(bibo_moe_ffn_forward(x.data_ptr(), f32(nw), (float)eps, res.defined() ? res.data_ptr() : nullptr,
+                               w_router.data_ptr(), f32(bias), w_gate_up.data_ptr(), w_down.data_ptr(), f32(theta), &sh, norm, algo,
+                               out.data_ptr(), nullptr, nullptr, int_ptr(counts), ws.data_ptr(), (size_t)ws.numel(), s),
+          "bibo_moe_ffn_forward");
+  }
   return py::make_tuple(out, maybe(counts));
 }
 
@@ -198,12 +245,12 @@ class LayerFn : public torch::autograd::Function<LayerFn> {
     hipStream_t s = c10::hip::getCurrentHIPStream(xb.device().index()).stream();
     size_t bytes = 0, state_bytes = 0;
     check(bibo_moe_workspace_bytes(&sh, &bytes), "bibo_moe_workspace_bytes");
-    const Scratch ws(xb.device(), s, bytes);
     const bool saved = c->keep && (l.algo == BIBO_ALGO_AUTO || l.algo == BIBO_ALGO_FUSED) &&
                        bibo_moe_train_state_bytes(&sh, &state_bytes) == BIBO_OK;
     Tensor last;           // the state or, where the backward pass routes again, the selection biases
     if (saved) {
       last = at::empty({(int64_t)std::max<size_t>(state_bytes, 256)}, xb.options().dtype(at::kByte));
+      const Scratch ws(xb.device(), s, bytes);
       check(bibo_moe_forward_train(xb.data_ptr(), l.w_router.data_ptr(), f32(l.bias), l.w_gate_up.data_ptr(), l.w_down.data_ptr(),
                                    f32(l.theta), &sh, l.norm, out.data_ptr(), int_ptr(c->counts), last.data_ptr(),
                                    (size_t)last.numel(), ws.data_ptr(), (size_t)ws.numel(), s),
@@ -212,6 +259,7 @@ class LayerFn : public torch::autograd::Function<LayerFn> {
       // A private copy: the layer's balancing step writes gate.bias in place later in the same forward, and the backward
       // pass has to route with the values the forward saw.
       last = l.bias.detach().clone();
+      const Scratch ws(xb.device(), s, bytes);
       check(bibo_moe_forward(xb.data_ptr(), l.w_router.data_ptr(), f32(last), l.w_gate_up.data_ptr(), l.w_down.data_ptr(),
                              f32(l.theta), &sh, l.norm, l.algo, out.data_ptr(), nullptr, nullptr, int_ptr(c->counts), nullptr,
                              ws.data_ptr(), (size_t)ws.numel(), s),
@@ -248,18 +296,20 @@ class LayerFn : public torch::autograd::Function<LayerFn> {
     hipStream_t s = c10::hip::getCurrentHIPStream(x.device().index()).stream();
     size_t bytes = 0;
     check(bibo_moe_backward_workspace_bytes(&sh, &bytes), "bibo_moe_backward_workspace_bytes");
-    const Scratch ws(x.device(), s, bytes);
-    if (saved)
-      check(bibo_moe_backward_saved(x.data_ptr(), d.data_ptr(), l.w_router.data_ptr(), l.w_gate_up.data_ptr(), l.w_down.data_ptr(),
-                                    f32(l.theta), &sh, l.norm, last.data_ptr(), (size_t)last.numel(), d_x.data_ptr(),
-                                    d_wr.data_ptr(), d_gu.data_ptr(), d_dn.data_ptr(), f32_out(d_th), nullptr, ws.data_ptr(),
-                                    (size_t)ws.numel(), s),
-            "bibo_moe_backward_saved");
-    else
-      check(bibo_moe_backward(x.data_ptr(), d.data_ptr(), l.w_router.data_ptr(), f32(last), l.w_gate_up.data_ptr(),
-                              l.w_down.data_ptr(), f32(l.theta), &sh, l.norm, d_x.data_ptr(), d_wr.data_ptr(), d_gu.data_ptr(),
-                              d_dn.data_ptr(), f32_out(d_th), nullptr, ws.data_ptr(), (size_t)ws.numel(), s),
-            "bibo_moe_backward");
+    {
+      const Scratch ws(x.device(), s, bytes);
+      if (saved)
+        check(bibo_moe_backward_saved(x.data_ptr(), d.data_ptr(), l.w_router.data_ptr(), l.w_gate_up.data_ptr(), l.w_down.data_ptr(),
+                                      f32(l.theta), &sh, l.norm, last.data_ptr(), (size_t)last.numel(), d_x.data_ptr(),
+                                      d_wr.data_ptr(), d_gu.data_ptr(), d_dn.data_ptr(), f32_out(d_th), nullptr, ws.data_ptr(),
+                                      (size_t)ws.numel(), s),
+              "bibo_moe_backward_saved");
+      else
+        check(bibo_moe_backward(x.data_ptr(), d.data_ptr(), l.w_router.data_ptr(), f32(last), l.w_gate_up.data_ptr(),
+                                l.w_down.data_ptr(), f32(l.theta), &sh, l.norm, d_x.data_ptr(), d_wr.data_ptr(), d_gu.data_ptr(),
+                                d_dn.data_ptr(), f32_out(d_th), nullptr, ws.data_ptr(), (size_t)ws.numel(), s),
+              "bibo_moe_backward");
+    }
     torch::autograd::variable_list out{d_x, d_wr, d_gu, d_dn, d_th, Tensor()};
     for (int i = 0; i < 5; ++i)
       if (out[i].scalar_type() != (at::ScalarType)dtypes[i]) out[i] = out[i].to((at::ScalarType)dtypes[i]);
@@ -442,6 +492,7 @@ Tensor exp_mlp(const Tensor& x, const Tensor& w_gate, const Tensor& w_up, const 
 
 PYBIND11_MODULE(_native, m) {
   m.def("abi_version", [] { return bibo_moe_abi_version(); });
+  py::class_<Held>(m, "Held").def(py::init<int, int64_t>()).def("__enter__", &Held::enter).def("__exit__", &Held::exit);
   m.def("workspace", &workspace);
   m.def("workspace_clear", &workspace_clear);
   m.def("layer_forward", &layer_forward);

@@ -95,9 +95,19 @@ class _Workspaces:
 _workspaces = _Workspaces()
 
 
+def _index(dev: torch.device) -> int:
+    return dev.index if dev.index is not None else torch.cuda.current_device()
+
+
 def workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
-    """The current stream's byte buffer, at least `nbytes` long."""
-    return L.native().workspace(dev.index if dev.index is not None else torch.cuda.current_device(), nbytes)
+    """The current stream's byte buffer, at least `nbytes` long, to look at or to fill; calls take it with _held."""
+    return L.native().workspace(_index(dev), nbytes)
+
+
+def _held(dev: torch.device, nbytes: int):
+    """The current stream's byte buffer for one library call: `with _held(...) as (address, size)`; calls of other threads on the
+    stream wait until it ends."""
+    return L.native().Held(_index(dev), nbytes)
 
 
 def workspace_bytes(T, H, E, k, I, dtype_code) -> int:
@@ -136,10 +146,9 @@ def permute(idx, E):
     perm_token = torch.empty(T * k, dtype=torch.int32, device=dev)
     # one 64-entry histogram per 128 tokens and, for large batches, one sum per 256 histograms
     nb = (max(1, (T + 127) // 128) + (T + 32767) // 32768 + 1) * 64 * 4
-    ws = workspace(dev, nb)
-    with torch.cuda.device(dev):
+    with torch.cuda.device(dev), _held(dev, nb) as (ws, ws_bytes):
         L.check(L.lib().bibo_moe_permute(_ptr(idx), T, E, k, _ptr(counts), _ptr(offsets), _ptr(perm_slot),
-                                         _ptr(perm_token), _ptr(ws), ws.numel(), _stream(dev)), "bibo_moe_permute")
+                                         _ptr(perm_token), ctypes.c_void_p(ws), ws_bytes, _stream(dev)), "bibo_moe_permute")
     return counts, offsets, perm_slot, perm_token
 
 
@@ -169,10 +178,9 @@ def down_combine_fwd(hidden, w_down, w, offsets, perm_slot, T, algo="auto"):
     _chk(offsets, "offsets", torch.int32, (E + 1,)); _chk(perm_slot, "perm_slot", torch.int32, (T * k,))
     dev = hidden.device
     out = torch.empty(T, H, dtype=hidden.dtype, device=dev)
-    ws = workspace(dev, T * k * H * 4)
-    with torch.cuda.device(dev):
+    with torch.cuda.device(dev), _held(dev, T * k * H * 4) as (ws, ws_bytes):
         L.check(L.lib().bibo_moe_down_combine_fwd(_ptr(hidden), _ptr(w_down), _ptr(w), _ptr(offsets), _ptr(perm_slot),
-                                                  T, H, E, k, I, dc, algo_code(algo), _ptr(out), _ptr(ws), ws.numel(),
+                                                  T, H, E, k, I, dc, algo_code(algo), _ptr(out), ctypes.c_void_p(ws), ws_bytes,
                                                   _stream(dev)), "bibo_moe_down_combine_fwd")
     return out
 
@@ -238,12 +246,11 @@ def experts_fwd(x, idx, w, w_gate_up, w_down, theta, algo="auto", want_counts=Fa
     dev = x.device
     out = torch.empty(T, H, dtype=x.dtype, device=dev)
     counts = torch.empty(E, dtype=torch.int32, device=dev) if want_counts else None
-    ws = workspace(dev, workspace_bytes(T, H, E, k, I, dc))
     sh = L.Shape(T, H, E, k, I, dc, n_pos, n_neg, act_code(act), 0)
-    with torch.cuda.device(dev):
+    with torch.cuda.device(dev), _held(dev, workspace_bytes(T, H, E, k, I, dc)) as (ws, ws_bytes):
         L.check(L.lib().bibo_moe_experts_fwd(_ptr(x), _ptr(idx), _ptr(w), _ptr(w_gate_up), _ptr(w_down), _ptr(theta),
-                                             ctypes.byref(sh), algo_code(algo), _ptr(out), _ptr(counts), _ptr(ws),
-                                             ws.numel(), _stream(dev)), "bibo_moe_experts_fwd")
+                                             ctypes.byref(sh), algo_code(algo), _ptr(out), _ptr(counts), ctypes.c_void_p(ws),
+                                             ws_bytes, _stream(dev)), "bibo_moe_experts_fwd")
     return out, counts
 
 
@@ -265,12 +272,11 @@ def moe_forward(x, w_router, bias, w_gate_up, w_down, theta, k, norm="sum", algo
     w = torch.empty(T, k, dtype=torch.float32, device=dev) if want_routing else None
     counts = torch.empty(E, dtype=torch.int32, device=dev) if want_counts else None
     logits = torch.empty(T, E, dtype=torch.float32, device=dev) if want_logits else None
-    ws = workspace(dev, workspace_bytes(T, H, E, k, I, dc))
     sh = L.Shape(T, H, E, k, I, dc, n_pos, n_neg, act_code(act), 0)
-    with torch.cuda.device(dev):
+    with torch.cuda.device(dev), _held(dev, workspace_bytes(T, H, E, k, I, dc)) as (ws, ws_bytes):
         L.check(L.lib().bibo_moe_forward(_ptr(x), _ptr(w_router), _ptr(bias), _ptr(w_gate_up), _ptr(w_down),
                                          _ptr(theta), ctypes.byref(sh), norm_mode(norm), algo_code(algo), _ptr(out),
-                                         _ptr(idx), _ptr(w), _ptr(counts), _ptr(logits), _ptr(ws), ws.numel(),
+                                         _ptr(idx), _ptr(w), _ptr(counts), _ptr(logits), ctypes.c_void_p(ws), ws_bytes,
                                          _stream(dev)), "bibo_moe_forward")
     return out, idx, w, counts, logits
 
@@ -324,11 +330,10 @@ def moe_backward(x, d_out, w_router, bias, w_gate_up, w_down, theta, k, norm="su
     sh = L.Shape(T, H, E, k, I, dc, n_pos, n_neg, act_code(act), 0)
     nbytes = ctypes.c_size_t(0)
     L.check(L.lib().bibo_moe_backward_workspace_bytes(ctypes.byref(sh), ctypes.byref(nbytes)), "bibo_moe_backward_workspace_bytes")
-    ws = workspace(dev, nbytes.value)
-    with torch.cuda.device(dev):
+    with torch.cuda.device(dev), _held(dev, nbytes.value) as (ws, ws_bytes):
         L.check(L.lib().bibo_moe_backward(_ptr(x), _ptr(d_out), _ptr(w_router), _ptr(bias), _ptr(w_gate_up), _ptr(w_down),
                                           _ptr(theta), ctypes.byref(sh), norm_mode(norm), _ptr(d_x), _ptr(d_wr), _ptr(d_gu),
-                                          _ptr(d_dn), _ptr(d_theta), _ptr(d_w), _ptr(ws), ws.numel(), _stream(dev)),
+                                          _ptr(d_dn), _ptr(d_theta), _ptr(d_w), ctypes.c_void_p(ws), ws_bytes, _stream(dev)),
                 "bibo_moe_backward")
     return d_x, d_wr, d_gu, d_dn, d_theta, d_w
 
@@ -361,12 +366,11 @@ def moe_forward_train(x, w_router, bias, w_gate_up, w_down, theta, k, norm="sum"
     out = torch.empty(T, H, dtype=x.dtype, device=dev)
     counts = torch.empty(E, dtype=torch.int32, device=dev) if want_counts else None
     state = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=dev)
-    ws = workspace(dev, workspace_bytes(T, H, E, k, I, dc))
     sh = L.Shape(T, H, E, k, I, dc, n_pos, n_neg, act_code(act), 0)
-    with torch.cuda.device(dev):
+    with torch.cuda.device(dev), _held(dev, workspace_bytes(T, H, E, k, I, dc)) as (ws, ws_bytes):
         L.check(L.lib().bibo_moe_forward_train(_ptr(x), _ptr(w_router), _ptr(bias), _ptr(w_gate_up), _ptr(w_down), _ptr(theta),
                                                ctypes.byref(sh), norm_mode(norm), _ptr(out), _ptr(counts), _ptr(state),
-                                               state.numel(), _ptr(ws), ws.numel(), _stream(dev)), "bibo_moe_forward_train")
+                                               state.numel(), ctypes.c_void_p(ws), ws_bytes, _stream(dev)), "bibo_moe_forward_train")
     return out, counts, state
 
 
@@ -390,12 +394,11 @@ def moe_backward_saved(x, d_out, w_router, w_gate_up, w_down, theta, k, state, n
     sh = L.Shape(T, H, E, k, I, dc, n_pos, n_neg, act_code(act), 0)
     nbytes = ctypes.c_size_t(0)
     L.check(L.lib().bibo_moe_backward_workspace_bytes(ctypes.byref(sh), ctypes.byref(nbytes)), "bibo_moe_backward_workspace_bytes")
-    ws = workspace(dev, nbytes.value)
-    with torch.cuda.device(dev):
+    with torch.cuda.device(dev), _held(dev, nbytes.value) as (ws, ws_bytes):
         L.check(L.lib().bibo_moe_backward_saved(_ptr(x), _ptr(d_out), _ptr(w_router), _ptr(w_gate_up), _ptr(w_down),
                                                 _ptr(theta), ctypes.byref(sh), norm_mode(norm), _ptr(state), state.numel(),
                                                 _ptr(d_x), _ptr(d_wr), _ptr(d_gu), _ptr(d_dn), _ptr(d_theta), _ptr(d_w),
-                                                _ptr(ws), ws.numel(), _stream(dev)), "bibo_moe_backward_saved")
+                                                ctypes.c_void_p(ws), ws_bytes, _stream(dev)), "bibo_moe_backward_saved")
     return d_x, d_wr, d_gu, d_dn, d_theta, d_w
 
 
@@ -418,11 +421,10 @@ def experts_backward(x, d_out, idx, w, w_gate_up, w_down, theta, act="radial", n
     sh = L.Shape(T, H, E + n_pos + n_neg, k, I, dc, n_pos, n_neg, act_code(act), 0)
     nbytes = ctypes.c_size_t(0)
     L.check(L.lib().bibo_moe_backward_workspace_bytes(ctypes.byref(sh), ctypes.byref(nbytes)), "bibo_moe_backward_workspace_bytes")
-    ws = workspace(dev, nbytes.value)
-    with torch.cuda.device(dev):
+    with torch.cuda.device(dev), _held(dev, nbytes.value) as (ws, ws_bytes):
         L.check(L.lib().bibo_moe_experts_backward(_ptr(x), _ptr(d_out), _ptr(idx), _ptr(w), _ptr(w_gate_up), _ptr(w_down),
                                                   _ptr(theta), ctypes.byref(sh), _ptr(d_x), _ptr(d_w), _ptr(d_gu), _ptr(d_dn),
-                                                  _ptr(d_theta), _ptr(ws), ws.numel(), _stream(dev)),
+                                                  _ptr(d_theta), ctypes.c_void_p(ws), ws_bytes, _stream(dev)),
                 "bibo_moe_experts_backward")
     return d_x, d_w, d_gu, d_dn, d_theta
 
@@ -488,10 +490,9 @@ def ffn_forward(h, norm_weight, eps, w_router, bias, w_gate_up, w_down, theta, k
     sh = L.Shape(T, H, E, k, I, dc, n_pos, n_neg, act_code(act), flags)
     nbytes = ctypes.c_size_t(0)
     L.check(L.lib().bibo_moe_ffn_workspace_bytes(ctypes.byref(sh), ctypes.byref(nbytes)), "bibo_moe_ffn_workspace_bytes")
-    ws = workspace(dev, nbytes.value)
-    with torch.cuda.device(dev):
+    with torch.cuda.device(dev), _held(dev, nbytes.value) as (ws, ws_bytes):
         L.check(L.lib().bibo_moe_ffn_forward(_ptr(h), _ptr(norm_weight), ctypes.c_float(eps), _ptr(residual), _ptr(w_router), _ptr(bias),
                                              _ptr(w_gate_up), _ptr(w_down), _ptr(theta), ctypes.byref(sh),
                                              norm_mode(norm), algo_code(algo), _ptr(out), _ptr(idx), _ptr(w),
-                                             _ptr(counts), _ptr(ws), ws.numel(), _stream(dev)), "bibo_moe_ffn_forward")
+                                             _ptr(counts), ctypes.c_void_p(ws), ws_bytes, _stream(dev)), "bibo_moe_ffn_forward")
     return out, idx, w, counts
