@@ -31,6 +31,9 @@ void check(int code, const char* what) {
 // memory recording on).  A Python caller (Held) runs Python code with a buffer in hand, in which a finaliser may call the
 // library again: the same thread may take its buffer twice.  The inner call's launches then lie whole between two of the
 // outer's statements, and the outer holds the tensor it began with.
+//
+// A call under graph capture gets memory of its own, from the graph's pool, which lasts as long as the graph: the stream's
+// buffer goes when a larger call comes, and another graph's replays may run beside this one's.
 struct Buffer {
   std::recursive_mutex busy;
   Tensor bytes;
@@ -46,11 +49,18 @@ Pool& pool() {
 
 class Scratch {
  public:
-  Scratch(c10::Device dev, hipStream_t stream, size_t bytes) : buffer_(find(dev, stream)), lock_(buffer_->busy, std::defer_lock) {
+  Scratch(c10::Device dev, hipStream_t stream, size_t bytes) {
+    auto fresh = [&] { return at::empty({(int64_t)std::max<size_t>(bytes, 1)}, at::TensorOptions().dtype(at::kByte).device(dev)); };
+    if (capturing(stream)) {
+      bytes_ = fresh();
+      return;
+    }
+    buffer_ = find(dev, stream);
+    lock_ = std::unique_lock<std::recursive_mutex>(buffer_->busy, std::defer_lock);
     take();
     if (small(bytes)) {
       lock_.unlock();
-      spare_ = at::empty({(int64_t)std::max<size_t>(bytes, 1)}, at::TensorOptions().dtype(at::kByte).device(dev));
+      spare_ = fresh();
       take();
       if (small(bytes)) std::swap(buffer_->bytes, spare_);       // (or another thread has been here: the spare one goes)
     }
@@ -67,6 +77,12 @@ class Scratch {
     std::shared_ptr<Buffer>& b = p.buffers[{dev.index(), stream}];
     if (!b) b = std::make_shared<Buffer>();
     return b;
+  }
+  static bool capturing(hipStream_t stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return false;
   }
   bool small(size_t bytes) const { return !buffer_->bytes.defined() || (size_t)buffer_->bytes.numel() < bytes; }
   void take() {

@@ -99,3 +99,36 @@ def test_static_entry_point_replays():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out_s, eager), f"replay differs from the eager call (seed {seed})"
+
+
+@pytest.mark.parametrize("gone", ["grown", "cleared"])
+def test_replays_after_the_stream_has_got_another_buffer(gone):
+    """A graph's workspace is the graph's own: a larger call on the capturing stream, or ops._workspaces.clear(), does not give
+    memory back that replays write to, and buffers allocated afterwards keep what is in them."""
+    shape = dict(T=300, H=256, E=8, k=2, I=128)
+    p, _ = _inputs(1, **shape)
+    wts = [p[n].to(DEV) for n in NAMES]
+    x, big = p["x"].to(DEV), torch.randn(4000, 256, device=DEV).bfloat16()
+    side = torch.cuda.Stream(device=DEV)
+    side.wait_stream(torch.cuda.current_stream(DEV))
+    with torch.cuda.stream(side):
+        want = ops.moe_forward(x, *wts, 2)[0]
+    side.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = ops.moe_forward(x, *wts, 2)[0]
+    if gone == "grown":
+        with torch.cuda.stream(side):
+            ops.moe_forward(big, *wts, 2)
+    else:
+        ops._workspaces.clear()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):                      # what was given back on the stream is handed out again here
+        others = [torch.full((n,), 7, dtype=torch.uint8, device=DEV) for n in (1 << 20, 1 << 21, 3 << 20) for _ in range(4)]
+    for _ in range(3):
+        torch.cuda.synchronize()
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        assert all(bool((o == 7).all()) for o in others)
