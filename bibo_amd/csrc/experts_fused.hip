@@ -674,16 +674,18 @@ __global__ __launch_bounds__(512) void down_act_kernel(const float* __restrict__
           const float sg = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(gq * nrl));
           h[q] = (bf16_t)(gq * rg * sg * u[i][q >> 2][q & 3]);                      // SiLU(g/r) r^p up
         }
-        if (preact != nullptr && nb == 0) {
-          bf16x8 gb, ub;
+        if constexpr (NT < 4) {              // (a state-keeping forward has I <= 384)
+          if (preact != nullptr && nb == 0) {
+            bf16x8 gb, ub;
 #pragma unroll
-          for (int q = 0; q < 8; ++q) {
-            gb[q] = (bf16_t)g[i][q >> 2][q & 3];
-            ub[q] = (bf16_t)u[i][q >> 2][q & 3];
+            for (int q = 0; q < 8; ++q) {
+              gb[q] = (bf16_t)g[i][q >> 2][q & 3];
+              ub[q] = (bf16_t)u[i][q >> 2][q & 3];
+            }
+            bf16_t* dst = preact + (size_t)(row0 + m) * 2 * I + lane * 8;
+            *reinterpret_cast<bf16x8*>(dst) = gb;
+            *reinterpret_cast<bf16x8*>(dst + I) = ub;
           }
-          bf16_t* dst = preact + (size_t)(row0 + m) * 2 * I + lane * 8;
-          *reinterpret_cast<bf16x8*>(dst) = gb;
-          *reinterpret_cast<bf16x8*>(dst + I) = ub;
         }
         *reinterpret_cast<bf16x8*>(acts + (lane >> 4) * (BM * 128) + m * 128 + (((lane & 15) ^ (m & 15)) << 3)) = h;
       }
@@ -731,12 +733,15 @@ void launch_fused_t(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const 
                     const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int S, int H, int E,
                     int act, unsigned x_bytes, bf16_t* yw, bf16_t* preact, hipStream_t s) {
   const int grid = ((S / (64 * MT) + E + 7) & ~7) + 8;
-  if (preact != nullptr)
-    hipLaunchKernelGGL((experts_fused_kernel<NT, CT, 2, MT>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta, w, offsets,
-                       perm_slot, perm_token, H, E, act, x_bytes, yw, preact, 1);
-  else
-    hipLaunchKernelGGL((experts_fused_kernel<NT, CT, 0, MT>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta, w, offsets,
-                       perm_slot, perm_token, H, E, act, x_bytes, yw, preact, 1);
+  if constexpr (NT < 4) {                    // (a state-keeping forward has I <= 384)
+    if (preact != nullptr) {
+      hipLaunchKernelGGL((experts_fused_kernel<NT, CT, 2, MT>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta, w, offsets,
+                         perm_slot, perm_token, H, E, act, x_bytes, yw, preact, 1);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((experts_fused_kernel<NT, CT, 0, MT>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta, w, offsets, perm_slot,
+                     perm_token, H, E, act, x_bytes, yw, nullptr, 1);
 }
 
 template <int NT>
@@ -814,17 +819,17 @@ bool split_columns(int S, int E, int H, int I) {
   return S / 128 + E / 2 <= limit && I >= 256;
 }
 
-// gu [S, 2I] fp32 -> routing-weighted rows in slot order, and with `preact` their bf16 copy (down_act_kernel); shapes as
-// launch_gateup_raw takes them
+// gu [S, 2I] fp32 -> routing-weighted rows in slot order, and with `preact` their bf16 copy (down_act_kernel; I <= 384); shapes as
+// launch_gateup_raw takes them, I = 256 to 512
 hipError_t launch_down_act(const void* gu, const void* wd, const float* theta, const float* w, const int32_t* offsets,
                            const int32_t* perm_slot, int S, int H, int E, int I, int act, void* yw, void* preact, hipStream_t s) {
   if (S == 0) return hipSuccess;
+  if (I == 512 && preact != nullptr) return hipErrorInvalidValue;
   const float* gp = static_cast<const float*>(gu);
   bf16_t* pp = static_cast<bf16_t*>(preact);
   const bf16_t* dp = static_cast<const bf16_t*>(wd);
   bf16_t* yp = static_cast<bf16_t*>(yw);
   switch (I) {
-    case 128: launch_down_act_nt<1>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yp, pp, s); break;
     case 256: launch_down_act_nt<2>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yp, pp, s); break;
     case 384: launch_down_act_nt<3>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yp, pp, s); break;
     case 512: launch_down_act_nt<4>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yp, pp, s); break;
@@ -847,6 +852,7 @@ hipError_t launch_experts_fused(const void* x, const void* wgu, const void* wd, 
   const int S = T * k;
   if (S == 0) return hipSuccess;
   if ((unsigned long long)T * H * sizeof(bf16_t) >= (1ull << 32)) return hipErrorInvalidValue;   // 32-bit byte offsets into x
+  if (I == 512 && preact != nullptr) return hipErrorInvalidValue;
   const unsigned xb = (unsigned)((size_t)T * H * sizeof(bf16_t));
   const bf16_t* xp = static_cast<const bf16_t*>(x);
   const bf16_t* gp = static_cast<const bf16_t*>(wgu);

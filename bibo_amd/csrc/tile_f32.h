@@ -37,17 +37,17 @@ __device__ __forceinline__ int fswz(int row, int c) { return row * kFK + ((c ^ (
 // out[dst(r), n] = scale(r) * sum_k A[src(r), k] W[e](k, n) for the rows r of expert e.  src(r) = a_index[r] (GATHER) or
 // r; dst(r) = out_index[r] and scale(r) = out_scale[out_index[r]] (SCATTER; out_scale == NULL: 1) or r and 1.  W[e] is
 // [N, K] (K-contiguous) or, with W_KM, [K, N].  K, N multiples of 4, rows 16-byte (bf16: 8-byte) aligned.
-// BM = 64: 64 rows x 64 NJ columns, 2 x 2 waves of 32x32 tiles.  BM = 16 (few rows per expert): 16 rows x 64 NJ columns, four
+// BM = 64: 64 rows x 64 columns, 2 x 2 waves of 32x32 tiles.  BM = 16 (few rows per expert): 16 rows x 64 columns, four
 // waves along the columns, 16x16 tiles: a quarter of the MFMA time per streamed weight byte, which is what counts there.
-template <typename TA, typename TW, bool W_KM, bool GATHER, bool SCATTER, int BM, int NJ>
+template <typename TA, typename TW, bool W_KM, bool GATHER, bool SCATTER, int BM>
 __global__ __launch_bounds__(256) void ggemm_f32_kernel(const TA* __restrict__ A, const int32_t* __restrict__ a_index,
                                                         const TW* __restrict__ W, const int32_t* __restrict__ offsets,
                                                         const int32_t* __restrict__ out_index,
                                                         const float* __restrict__ out_scale, int K, int N, int E, int nblk_n,
                                                         float* __restrict__ out) {
   static_assert(BM == 64 || (BM == 16 && !W_KM), "tile shapes");
-  constexpr int BN = 64 * NJ;
-  constexpr int A_PER = BM == 64 ? 2 : 1, W_PER = 2 * NJ;       // granules of four elements per thread and step
+  constexpr int BN = 64;
+  constexpr int A_PER = BM == 64 ? 2 : 1, W_PER = 2;            // granules of four elements per thread and step
   __shared__ __attribute__((aligned(16))) float As[2][BM * kFK];
   __shared__ __attribute__((aligned(16))) float Ws[2][BN * kFK];
   __shared__ int dst_s[BM];
@@ -111,52 +111,42 @@ __global__ __launch_bounds__(256) void ggemm_f32_kernel(const TA* __restrict__ A
   __syncthreads();
   if constexpr (BM == 64) {
     const int wm = wave & 1, wn = wave >> 1, l32 = lane & 31, h = lane >> 5;
-    floatx16 acc[NJ];
+    floatx16 acc;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[j][i] = 0.f;
+    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
     for (int s = 0; s < nsteps; ++s) {
       if (s + 1 < nsteps) load((s + 1) * kFK);
       const float* as = As[s & 1];
       const float* ws = Ws[s & 1];
+      const int n = wn * 32 + l32;
 #pragma unroll
       for (int ks = 0; ks < kFK / 8; ++ks) {
         const floatx4 a = *reinterpret_cast<const floatx4*>(as + fswz(wm * 32 + l32, 2 * ks + h));
+        floatx4 b;
+        if constexpr (W_KM) {
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          floatx4 b;
-          const int n = (wn * NJ + j) * 32 + l32;
-          if constexpr (W_KM) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) b[q] = ws[(8 * ks + 4 * h + q) * BN + n];
-          } else {
-            b = *reinterpret_cast<const floatx4*>(ws + fswz(n, 2 * ks + h));
-          }
-#pragma unroll
-          for (int q = 0; q < 4; ++q) acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q], b[q], acc[j], 0, 0, 0);
+          for (int q = 0; q < 4; ++q) b[q] = ws[(8 * ks + 4 * h + q) * BN + n];
+        } else {
+          b = *reinterpret_cast<const floatx4*>(ws + fswz(n, 2 * ks + h));
         }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q], b[q], acc, 0, 0, 0);
       }
       if (s + 1 < nsteps) store((s + 1) & 1);
       __syncthreads();
     }
     // lane = column lane % 32, register i = row 8 (i / 4) + 4 (lane / 32) + i % 4: a store covers 128 bytes of two rows
+    const int n = n0 + wn * 32 + l32;
+    if (n < N) {
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int n = n0 + (wn * NJ + j) * 32 + l32;
-      if (n < N) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int m = wm * 32 + acc_row(i, lane);
-          if (m < rows) out[(size_t)dst_s[m] * N + n] = scale_s[m] * acc[j][i];
-        }
+      for (int i = 0; i < 16; ++i) {
+        const int m = wm * 32 + acc_row(i, lane);
+        if (m < rows) out[(size_t)dst_s[m] * N + n] = scale_s[m] * acc[i];
       }
     }
   } else {
     const int l16 = lane & 15, g4 = lane >> 4;
-    floatx4 acc[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) acc[j] = zero;
+    floatx4 acc = zero;
     for (int s = 0; s < nsteps; ++s) {
       if (s + 1 < nsteps) load((s + 1) * kFK);
       const float* as = As[s & 1];
@@ -164,25 +154,19 @@ __global__ __launch_bounds__(256) void ggemm_f32_kernel(const TA* __restrict__ A
 #pragma unroll
       for (int ks = 0; ks < kFK / 16; ++ks) {
         const floatx4 a = *reinterpret_cast<const floatx4*>(as + fswz(l16, 4 * ks + g4));
+        const floatx4 b = *reinterpret_cast<const floatx4*>(ws + fswz(wave * 16 + l16, 4 * ks + g4));
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          const floatx4 b = *reinterpret_cast<const floatx4*>(ws + fswz((wave * NJ + j) * 16 + l16, 4 * ks + g4));
-#pragma unroll
-          for (int q = 0; q < 4; ++q) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q], b[q], acc[j], 0, 0, 0);
-        }
+        for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q], b[q], acc, 0, 0, 0);
       }
       if (s + 1 < nsteps) store((s + 1) & 1);
       __syncthreads();
     }
+    const int n = n0 + wave * 16 + l16;
+    if (n < N) {
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int n = n0 + (wave * NJ + j) * 16 + l16;
-      if (n < N) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int m = 4 * g4 + i;
-          if (m < rows) out[(size_t)dst_s[m] * N + n] = scale_s[m] * acc[j][i];
-        }
+      for (int i = 0; i < 4; ++i) {
+        const int m = 4 * g4 + i;
+        if (m < rows) out[(size_t)dst_s[m] * N + n] = scale_s[m] * acc[i];
       }
     }
   }
@@ -199,16 +183,15 @@ hipError_t launch_ggemm_f32(const TA* A, const int32_t* a_index, const TW* W, co
     const long long tiles = (long long)(S / BM + E < S ? S / BM + E : S) * nblk_n;
     return dim3((unsigned)(((tiles + 7) & ~7ll) + 8));
   };
+  const int nblk = (N + 63) / 64;
   if constexpr (!W_KM) {
     if ((long long)S <= (long long)kFewRows * E) {
-      const int nblk = (N + 63) / 64;
-      hipLaunchKernelGGL((ggemm_f32_kernel<TA, TW, false, GATHER, SCATTER, 16, 1>), grid(16, nblk), dim3(256), 0, s, A, a_index, W,
+      hipLaunchKernelGGL((ggemm_f32_kernel<TA, TW, false, GATHER, SCATTER, 16>), grid(16, nblk), dim3(256), 0, s, A, a_index, W,
                          offsets, out_index, out_scale, K, N, E, nblk, out);
       return hipGetLastError();
     }
   }
-  const int nblk = (N + 63) / 64;
-  hipLaunchKernelGGL((ggemm_f32_kernel<TA, TW, W_KM, GATHER, SCATTER, 64, 1>), grid(64, nblk), dim3(256), 0, s, A, a_index, W,
+  hipLaunchKernelGGL((ggemm_f32_kernel<TA, TW, W_KM, GATHER, SCATTER, 64>), grid(64, nblk), dim3(256), 0, s, A, a_index, W,
                      offsets, out_index, out_scale, K, N, E, nblk, out);
   return hipGetLastError();
 }
