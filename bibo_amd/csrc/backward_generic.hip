@@ -182,7 +182,7 @@ __global__ __launch_bounds__(256) void act_bwd_f32_kernel(float* __restrict__ gu
       if (radial) dg = fmaf(g[q] * rinv / (float)I, inner, dg);
       og[q] = dg;
       ou[q] = dh * gain * a;
-      oh[q] = ws * gain * a * u[q];
+      oh[q] = (float)((double)ws * gain * a * u[q]);
     }
     store4(gr + c, og);
     store4(gr + I + c, ou);

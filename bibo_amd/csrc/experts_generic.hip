@@ -115,7 +115,7 @@ __global__ __launch_bounds__(256) void activate_f32_kernel(const float* __restri
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const float z = v[q] / r;
-      h[q] = z / (1.f + expf(-z)) * gain * u[q];                       // SiLU(g/r) r^p up
+      h[q] = (float)((double)(z / (1.f + expf(-z))) * gain * u[q]);    // SiLU(g/r) r^p up, rounded once
     }
     store4(hidden + (size_t)row * I + c, h);
   }

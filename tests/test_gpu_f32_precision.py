@@ -1,4 +1,4 @@
-"""How far fp32 results are from exact: the tile and few-token kernels of the generic family against the kernels that take one routed
+"""How far fp32 results are from exact: the tile kernels of the generic family against the kernels that take one routed
 row at a time, whose dot products are 64 partial sums and a tree.  The 2-norm error against float64 may not be larger (2 %: what
 two equally good orders of the same sums differ by at these counts of elements; 5 % where a result has under 10 000)."""
 import numpy as np
@@ -23,10 +23,9 @@ def _inputs(T, H, I, E, k):
     return p, [p[n].to(DEV) for n in NAMES]
 
 
-# 64-row tiles, 16-row tiles, few tokens; contractions shorter than one step of the tiles to the longest
+# 64-row tiles, 16-row tiles; contractions shorter than one step of the tiles to the longest
 SHAPES = [(600, 768, 384, 8, 3), (600, 1024, 512, 8, 2), (500, 192, 88, 16, 3), (700, 64, 32, 4, 2), (300, 340, 132, 8, 2),
-          (40, 768, 384, 16, 2), (60, 192, 88, 16, 3), (50, 1024, 512, 16, 2),
-          (1, 768, 384, 64, 6), (8, 1024, 512, 16, 6), (8, 192, 88, 16, 3), (16, 64, 32, 8, 3)]
+          (40, 768, 384, 16, 2), (60, 192, 88, 16, 3), (50, 1024, 512, 16, 2)]
 
 
 @pytest.mark.parametrize("T,H,I,E,k", SHAPES)
@@ -43,7 +42,7 @@ def test_forward(T, H, I, E, k):
     assert got <= want * (1.02 if T * H >= 10000 else 1.05)
 
 
-@pytest.mark.parametrize("T,H,I,E,k", SHAPES[:8])
+@pytest.mark.parametrize("T,H,I,E,k", SHAPES)
 def test_backward(T, H, I, E, k):
     p, args = _inputs(T, H, I, E, k)
     x = p["x"].to(DEV)
