@@ -52,6 +52,10 @@ __device__ __forceinline__ float sum16(float v) {          // over the 16 lanes 
   return v + dpp(v, std::integral_constant<int, 0x140>{});
 }
 
+// the end of a dot product: the lanes' four partial sums each.  Sixty-four chains and a tree, as where a wave's lanes share a row
+// (experts_generic.hip): one chain per lane was 1.3 times as far from exact in fp32 at H = 768
+__device__ __forceinline__ float sum64(const float (&part)[4]) { return sum16((part[0] + part[1]) + (part[2] + part[3])); }
+
 constexpr int kGateRows = 32;           // weight rows per workgroup of the gate/up kernel: two per 16 lanes
 
 // grid (ceil(2I / 32), S).  NG = ceil(H / 128): 8-element granules of a row per lane.
@@ -81,12 +85,12 @@ __global__ __launch_bounds__(256) void gateup_few_kernel(const T* __restrict__ x
   }
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
-    float acc = 0.f;
+    float part[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int u = 0; u < NG; ++u)
 #pragma unroll
-      for (int q = 0; q < 8; ++q) acc = fmaf(wv[r][u].get(q), xv[u].get(q), acc);
-    acc = sum16(acc);
+      for (int q = 0; q < 8; ++q) part[q & 3] = fmaf(wv[r][u].get(q), xv[u].get(q), part[q & 3]);
+    const float acc = sum64(part);
     if (c == 0 && row0 + 16 * r < I2) gu[(size_t)slot * I2 + row0 + 16 * r] = acc;
   }
 }
@@ -118,7 +122,7 @@ __global__ __launch_bounds__(64 * kMaxK) void down_few_kernel(const float* __res
     }
     float gv[NG][8], h[NG][8];                                 // gate, then up -> h
     const float* gr = gu + (size_t)slot * 2 * I;
-    float ss = 0.f;
+    float sq[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int u = 0; u < NG; ++u) {
       const int g = (u * 16 + c) * 8;
@@ -129,27 +133,40 @@ __global__ __launch_bounds__(64 * kMaxK) void down_few_kernel(const float* __res
         load8(h[u], gr + I + g);
       }
 #pragma unroll
-      for (int q = 0; q < 8; ++q) ss = fmaf(gv[u][q], gv[u][q], ss);
+      for (int q = 0; q < 8; ++q) sq[q & 3] = fmaf(gv[u][q], gv[u][q], sq[q & 3]);
     }
-    ss = sum16(ss);
-    float rinv, gain;                                                                              // 1/r, r^p (moe.py:88-89)
-    radial_row_scalars(ss, I, p, act, rinv, gain);
-    const float nrl = -1.4426950408889634f * rinv, rgn = rinv * gain;
-#pragma unroll
-    for (int u = 0; u < NG; ++u)
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const float sig = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(gv[u][q] * nrl));
-        h[u][q] *= gv[u][q] * rgn * sig;                                                            // SiLU(g/r) r^p up
-      }
-#pragma unroll
-    for (int it = 0; it < kIt; ++it) {
-      float acc = 0.f;
+    const float ss = sum64(sq);
+    if constexpr (sizeof(T) == 4) {
+      // fp32 layers: the math library and divisions, as in activate_f32_kernel
+      const float r = act == BIBO_ACT_SILU ? 1.f : sqrtf(ss / (float)I + kNormSiluEps);            // moe.py:88
+      const float gain = act == BIBO_ACT_SILU ? 1.f : powf(r, p);
 #pragma unroll
       for (int u = 0; u < NG; ++u)
 #pragma unroll
-        for (int q = 0; q < 8; ++q) acc = fmaf(wv[it][u].get(q), h[u][q], acc);
-      acc = sum16(acc);
+        for (int q = 0; q < 8; ++q) {
+          const float z = gv[u][q] / r;
+          h[u][q] = (float)((double)(z / (1.f + expf(-z))) * gain * h[u][q]);                       // SiLU(g/r) r^p up
+        }
+    } else {
+      float rinv, gain;                                                                            // 1/r, r^p (moe.py:88-89)
+      radial_row_scalars(ss, I, p, act, rinv, gain);
+      const float nrl = -1.4426950408889634f * rinv, rgn = rinv * gain;
+#pragma unroll
+      for (int u = 0; u < NG; ++u)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const float sig = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(gv[u][q] * nrl));
+          h[u][q] *= gv[u][q] * rgn * sig;                                                          // SiLU(g/r) r^p up
+        }
+    }
+#pragma unroll
+    for (int it = 0; it < kIt; ++it) {
+      float part_d[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int u = 0; u < NG; ++u)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) part_d[q & 3] = fmaf(wv[it][u].get(q), h[u][q], part_d[q & 3]);
+      const float acc = sum64(part_d);
       if (c == 0) part[j][it * 4 + rg] = ws * acc;                                                 // moe.py:93
     }
   } else if (lane < CH) {                                      // +/-Identity (moe.py:95-99), or no expert at all
