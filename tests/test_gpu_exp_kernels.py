@@ -73,6 +73,27 @@ def test_attention(D, nq, nkv, S, window):
         assert _rel(out, y.reshape(B, S, nq * D)) <= 1e-2, (xsa is not None)
 
 
+@pytest.mark.parametrize("B,S,nq,nkv,D,window,spread", [(1, 48, 4, 2, 192, 128, 1), (1, 700, 4, 2, 192, 128, 1), (1, 700, 4, 2, 192, 128, 3),
+                                                        (2, 333, 4, 1, 64, 128, 1), (1, 257, 2, 2, 128, 64, 3)])
+def test_banded_attention_is_as_exact_as_its_output_type(B, S, nq, nkv, D, window, spread):
+    """The probabilities' 16 bits of mantissa do not show: the result is as far from float64 as the float64 result rounded to bf16
+    is (2^-17 beside 2^-9, in quadrature: 1e-5 of it)."""
+    g = torch.Generator().manual_seed(S)
+    qkv = torch.randn(B, S, (nq + 2 * nkv) * D, generator=g)
+    qkv[..., :nq * D] *= spread
+    qkv = qkv.bfloat16()
+    out = torch.empty(B, S, nq * D, dtype=torch.bfloat16, device=DEV)
+    d = qkv.to(DEV)
+    _call("bibo_moe_exp_attention_fwd", _ptr(d), qkv.shape[-1], B, S, nq, nkv, D, window, ctypes.c_float(D ** -0.5), None, 1, _ptr(out))
+    q, k, v = (t.double().view(B, S, -1, D).transpose(1, 2) for t in qkv.split([nq * D, nkv * D, nkv * D], -1))
+    i = torch.arange(S)
+    allow = (i[None] <= i[:, None]) & (i[:, None] - i[None] < window)
+    rep = nq // nkv
+    p = (q @ k.repeat_interleave(rep, 1).transpose(-1, -2).contiguous() * D ** -0.5).masked_fill(~allow, -torch.inf).softmax(-1)
+    ref = (p @ v.repeat_interleave(rep, 1)).transpose(1, 2).reshape(B, S, nq * D)
+    assert float((out.cpu().double() - ref).norm()) <= 1.001 * float((ref.bfloat16().double() - ref).norm())
+
+
 def test_attention_refuses_what_it_does_not_take():
     args = lambda nq, nkv, D: (None, 4096, 1, 4, nq, nkv, D, 0, ctypes.c_float(1.0), None, 1, None, None)
     for nq, nkv, D in ((4, 2, 96), (3, 2, 64), (3, 1, 64), (4, 0, 64)):
