@@ -194,9 +194,12 @@ __global__ __launch_bounds__(256, 4) void ggemm_f32_kernel(const TA* __restrict_
   }
 }
 
-// 16-row tiles up to this many rows per expert on average: past it most experts need a second 16-row tile, which streams
-// their weights again, while a 64-row tile's MFMAs hide behind them.
-constexpr int kFewRows = 12;
+// 16-row tiles up to this many rows per expert on average: a 64-row tile multiplies up to 63 rows that are not there, a 16-row tile
+// streams its weights four times as often, from L2.  Layer times in fp32, 64-row -> 16-row tiles: H = 768, I = 384, E = 64, k = 6:
+// 116 -> 80 us at 9 rows, 117 -> 116 at 31, 213 -> 199 at 96, 221 -> 223 at 111, 326 -> 343 at 192; H = 1024, I = 512, k = 8: 175 -> 128
+// at 10, 311 -> 281 at 80, 322 -> 321 at 96, 347 -> 369 at 112; H = 192, I = 88, E = 16, k = 3: 34 -> 30 at 96, 49 -> 44 at 384.  (Where
+// the rows just fill 64, e.g. 36 to 40 at H = 768, the 64-row tiles are 2 % ahead.)
+constexpr int kFewRows = 96;
 
 template <typename TA, typename TW, bool W_KM, bool GATHER, bool SCATTER>
 hipError_t launch_ggemm_f32(const TA* A, const int32_t* a_index, const TW* W, const int32_t* offsets, const int32_t* out_index,

@@ -16,6 +16,16 @@ def _rel(a, ref):
     return float((a.double().cpu() - ref.double()).abs().max() / ref.double().abs().max().clamp_min(1e-30))
 
 
+# the same with more than 96 rows per expert on average, where the 64-row tiles run in both directions
+TALL = [(130, 100, 1, 0, 1, 28), (194, 68, 2, 0, 1, 36), (200, 132, 1, 1, 2, 64), (449, 64, 4, 0, 1, 128), (400, 260, 2, 1, 3, 132)]
+
+
+@pytest.mark.parametrize("T,H,Eg,pairs,k,I", TALL)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_tall_tile_edges(T, H, Eg, pairs, k, I, dtype):
+    test_tile_edges(T, H, Eg, pairs, k, I, dtype)
+
+
 @pytest.mark.parametrize("T,H,Eg,pairs,k,I", [(1, 64, 8, 0, 2, 32), (12, 68, 2, 0, 2, 36), (24, 132, 4, 0, 2, 64), (63, 100, 2, 0, 1, 28),
                                               (65, 64, 1, 1, 2, 64), (129, 192, 14, 1, 3, 88), (200, 66, 4, 0, 2, 33),
                                               (17, 260, 64, 0, 8, 132), (300, 516, 5, 2, 4, 260)])
