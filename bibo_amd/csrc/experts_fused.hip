@@ -808,14 +808,18 @@ hipError_t launch_gateup_raw(const void* x, const void* wgu, const int32_t* offs
 
 // Whether a tile's columns are cut over several workgroups.  The fused kernel keeps a row's tile on one CU, which is what pulls the
 // expert's weights then: with fewer tiles than CUs most of the chip idles.  Cut (launch_gateup_raw, launch_down_act), the
-// pre-activations make a round trip and every column block computes the activations again, which pays up to about 80 tiles
-// (expected: an expert's last one half full).  Whole layer, one set of weights read again and again, uncut -> cut: H = 768,
-// I = 384, E = 64, k = 6: 47 -> 44.5 us at T = 128, 52 -> 51 at T = 512, 66 -> 63 at T = 1024, but 79 -> 94 at T = 1500; H = 1024,
-// I = 512, k = 8: 87 -> 78 at T = 512 (E = 16, k = 3: 79 -> 53 at T = 1000).  Lighter experts stream faster and gain less: I = 256 up to
-// about 64 tiles at H = 1024 (E = 16, k = 3: 60 -> 44 at T = 512), 40 at H = 512 (45 -> 34).  Pre-activations in bf16 were 1 to 5 us
-// faster and half again as far from the exact result (3.5e-3 against 2.3e-3).
+// pre-activations make a round trip and every column block computes the activations again.  A workgroup fills a CU in either half, so
+// what decides is whether tiles x blocks (I / 128 in the first half, H / 256 or, where 256 does not divide H, H / 128 in the second)
+// still run in about one round of 256: a second round costs more than the cut gives.  The limits are in tiles as expected here (an
+// expert's last one half full).  Whole layer, uncut -> cut, six layers' weights in turn, bf16:
+//   I = 512 (4 blocks), H = 1024: 92 -> 70 us at 41 tiles, 89 -> 84 at 66, 97 -> 91 or 89 -> 94 at 72, 95 -> 101 at 80; H = 512: 60 -> 59 at 65
+//   I = 384 (3 blocks), H = 768: 64 -> 51 at 38, 76 -> 70 at 80, 78 -> 98 at 102; H = 1024: 90 -> 81 at 77, 90 -> 94 at 83; H = 512:
+//     58 -> 55 at 77, 58 -> 62 at 83; H = 640 (5 blocks in the second half): 59 -> 53 at 44, 64.5 -> 63 at 59, 66.5 -> 67 at 65
+//   I = 256, H = 1024 (4 blocks in the second half): 60 -> 51 at 38, 67 -> 63 at 64, 74 -> 74 at 80; H = 512, where the weights are too
+//     light to matter: within 1 us either way up to 56 tiles from memory, 45 -> 34 with 16 experts' weights in L2
+// Pre-activations in bf16 were 1 to 5 us faster and half again as far from the exact result (3.5e-3 against 2.3e-3).
 bool split_columns(int S, int E, int H, int I) {
-  const int limit = I >= 384 ? 80 : (H * I >= 256 * 1024 ? 64 : 40);
+  const int limit = I >= 512 ? 66 : I >= 384 ? (H % 256 == 0 ? 77 : 60) : (H * I >= 256 * 1024 ? 64 : 40);
   return S / 128 + E / 2 <= limit && I >= 256;
 }
 
