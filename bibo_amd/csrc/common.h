@@ -19,7 +19,11 @@ constexpr float kSumNormEps = 1e-20f;   // src/modeling/ffn/router.py:45
 // tokens handled by one workgroup of the histogram / permutation kernels
 constexpr int kPermTokens = 128;   // tokens per permutation workgroup (256 and 64 measured slower)
 constexpr int kStreamMaxSlots = 4096;   // routed slots the weight-streaming kernels can scan per workgroup
-constexpr int kFewSlots = 48;           // routed slots up to which the few-token kernels run
+// Routed slots up to which the few-token kernels run: every slot reads its expert's weights by itself there, so the widest layers
+// cross over first.  Layer times, other kernels -> few-token kernels, six layers' weights in turn: bf16 H = 1024, I = 512, k = 6:
+// 31 -> 17 us at 6 slots, 46 -> 41 at 48, 48 -> 53 at 72; H = 768, I = 384: 34 -> 26 at 48, 34 -> 33 at 72, 35 -> 40 at 96; H = 512,
+// I = 256: 24 -> 17 at 48, 25 -> 27 at 144; fp32 H = 1024, I = 512: 138 -> 100 at 48, 169 -> 175 at 96.
+constexpr int kFewSlots = 48;
 constexpr int kStreamMaxRows = 2048;    // rows (= tokens) one expert can get in them
 
 typedef __bf16 bf16_t;
