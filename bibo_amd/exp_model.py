@@ -105,8 +105,10 @@ def _fp32_copy(module, name):
     tag = (p.data_ptr(), p._version, p.device)
     hit = module.__dict__.get("_fp32_" + name)
     if hit is None or hit[0] != tag:
-        hit = (tag, p.detach().float().contiguous())
-        module.__dict__["_fp32_" + name] = hit
+        copy = p.detach().float().contiguous()
+        if p.is_cuda and torch.cuda.is_current_stream_capturing():
+            return copy                          # the graph's own: filled by its replays only
+        hit = module.__dict__["_fp32_" + name] = (tag, copy)
     return hit[1]
 
 

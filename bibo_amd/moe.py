@@ -121,8 +121,10 @@ class _CastCache:
         tag = (p.data_ptr(), p._version, p.device, p.dtype)
         hit = self._store.get(key)
         if hit is None or hit[0] != tag:
-            hit = (tag, p.detach().to(dtype).contiguous())
-            self._store[key] = hit
+            copy = p.detach().to(dtype).contiguous()
+            if p.is_cuda and torch.cuda.is_current_stream_capturing():
+                return copy                      # the graph's own: filled by its replays only
+            hit = self._store[key] = (tag, copy)
         return hit[1]
 
 

@@ -170,6 +170,28 @@ def test_weights_lie_in_one_block_until_one_is_replaced():
 
 
 @torch.no_grad()
+def test_weights_changed_before_a_capture_are_seen_outside_it():
+    """Copies in kernel dtype that a captured call makes are the graph's; a call outside makes its own."""
+    model, ids, new = _model(), _ids(2, 20, 1), _model(seed=5)
+    want = new(ids)
+    side = torch.cuda.Stream(device=DEV)
+    side.wait_stream(torch.cuda.current_stream(DEV))
+    with torch.cuda.stream(side):
+        model(ids)
+        for p, q in zip(model.parameters(), new.parameters()):
+            p.copy_(q)
+    side.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = model(ids)
+    assert torch.equal(model(ids), want)             # before any replay
+    for _ in range(2):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(model(ids), want)
+
+
+@torch.no_grad()
 @pytest.mark.parametrize("source", ["built", "assigned", "flat"])
 def test_a_move_that_moves_nothing_leaves_the_weights_where_they_are(source):
     model, ids = _model(), _ids(2, 20, 1)
