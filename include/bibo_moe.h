@@ -82,13 +82,13 @@ enum bibo_flags {
 /* kernel family for the expert GEMMs */
 enum bibo_algo {
   BIBO_ALGO_AUTO = 0,    /* pick by shape */
-  BIBO_ALGO_GENERIC = 1, /* one workgroup per routed row, any H and I, bf16 or fp32 */
+  BIBO_ALGO_GENERIC = 1, /* fp32 arithmetic, any H and I, bf16 or fp32: tiles of fp32 matrix instructions where H and I are
+                            multiples of 4 (bf16: and no MFMA tile divides them), else one workgroup per routed row */
   BIBO_ALGO_MFMA = 2,    /* grouped bf16 MFMA tiles, one kernel per GEMM; needs bf16, H % 128 == 0 and
                             I in {128,256,384,512} */
   BIBO_ALGO_STREAM = 3,  /* weight-streaming kernels for few rows per expert (decode); bf16, H and I
-                            multiples of 64 up to 1728; only the composite entry points; T*k <= 40*E when
-                            H, I <= 512, 32*E up to H = 768, 24*E above, and at most 4096 slots and 2048 rows per
-                            expert: T <= 2048 for bibo_moe_forward / bibo_moe_ffn_forward (a token's experts are
+                            multiples of 64 up to 1728; only the composite entry points; at most 4096 slots and
+                            2048 rows per expert: T <= 2048 for bibo_moe_forward / bibo_moe_ffn_forward (a token's experts are
                             distinct), T*k <= 2048 for bibo_moe_experts_fwd (a caller's indices may repeat) */
   BIBO_ALGO_FUSED = 4    /* both GEMMs of a 128-row tile in one kernel, activations stay in LDS; bf16,
                             H % 128 == 0, I in {128,256,384}; only bibo_moe_experts_fwd / bibo_moe_forward */
