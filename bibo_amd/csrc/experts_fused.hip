@@ -1,4 +1,4 @@
-// Kernels 3 and 4 in one launch: a workgroup takes 128 permuted rows of one expert through the gate/up
+// Kernels 3 and 4 in one launch: a workgroup takes up to 128 permuted rows of one expert through the gate/up
 // projection, Radial NormSiLU and the down projection without the activations leaving the CU.
 //
 // Phase 1 (gate/up GEMM, 2 x 4 waves, v_mfma_f32_32x32x16_bf16, operands swapped so that a lane ends up with
@@ -24,12 +24,10 @@
 // activations already fill most of the LDS.
 // Each block of columns is scaled by the routing weight, staged through LDS 32 rows at a time (in the two x
 // buffers, which are idle by then) and scattered to slot order as 256-byte row segments.
-// A tile may hold fewer than 128 rows (an expert's last tile, or all of its rows).  32-row blocks without rows are
-// not multiplied: the kernel body exists once per number of blocks (1 to 4), with the MFMAs, activations, down
-// projection row tiles and output rounds of the missing blocks left out; every wave still issues its share of
-// the weight requests.  A tile's duration hardly depends on its rows all the same (it is the stream of its
-// expert's weights through one CU: 3-block tiles take as long as 4-block tiles), which is why cutting the tiles
-// so that they fill whole rounds of the chip (512 tiles of 96 rows for the 410 of the prefill shape) gained nothing.
+// A tile may hold fewer than 128 rows: make_round_tile_map chooses the height of a call's tiles by the rounds of the chip they come to, and
+// an expert's last tile takes what is left.  32-row blocks without rows are not multiplied: the kernel body exists once per number of blocks
+// (1 to 4), with the MFMAs, activations, down projection row tiles and output rounds of the missing blocks left out, and of up to two blocks
+// each M wave takes one; every wave still issues its share of the weight requests, which is most of what a tile costs.
 // Reference: BiBoFusedExperts.forward, src/modeling/ffn/moe.py:81-93.
 #include <type_traits>
 
@@ -255,16 +253,16 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
                                                             const int32_t* __restrict__ perm_token, int H, int E,
                                                             int act, unsigned x_bytes, bf16_t* __restrict__ yw,
                                                             bf16_t* __restrict__ preact, int column_blocks) {
-  using F = FusedShape<NT, CT, MTP>;
-  constexpr int MT = F::MT, BM = F::BM, I = F::I, BK = F::BK;
+  using FT = FusedShape<NT, CT, MTP>;
+  constexpr int BM = FT::BM, I = FT::I, BK = FT::BK;
   // Every buffer that is read while LDS-DMA fills another is a variable of its own: the compiler orders a DMA
   // transfer against later LDS reads of the same variable with a full wait for the transfer.
-  __shared__ __attribute__((aligned(16))) bf16_t S0[F::kStageElems];  // weight stages, then the activations
-  __shared__ __attribute__((aligned(16))) bf16_t S1[F::kStageElems];
-  __shared__ __attribute__((aligned(16))) bf16_t S2[F::kRing == 3 ? F::kStageElems : 8];
-  __shared__ __attribute__((aligned(16))) bf16_t A0[F::kXElems];      // x rows of even K steps; then output staging,
-  __shared__ __attribute__((aligned(16))) bf16_t A1[F::kXElems];      // x rows of odd K steps;  alternating per 32 rows
-  __shared__ __attribute__((aligned(16))) bf16_t A2[F::kDeep ? F::kAElems : 8];   // kDeep: x rows of every third K step
+  __shared__ __attribute__((aligned(16))) bf16_t S0[FT::kStageElems];  // weight stages, then the activations
+  __shared__ __attribute__((aligned(16))) bf16_t S1[FT::kStageElems];
+  __shared__ __attribute__((aligned(16))) bf16_t S2[FT::kRing == 3 ? FT::kStageElems : 8];
+  __shared__ __attribute__((aligned(16))) bf16_t A0[FT::kXElems];      // x rows of even K steps; then output staging,
+  __shared__ __attribute__((aligned(16))) bf16_t A1[FT::kXElems];      // x rows of odd K steps;  alternating per 32 rows
+  __shared__ __attribute__((aligned(16))) bf16_t A2[FT::kDeep ? FT::kAElems : 8];   // kDeep: x rows of every third K step
   __shared__ float ssq[4 * BM];
   __shared__ float rinv_s[BM], gain_s[BM], w_s[BM];
   __shared__ int slot_s[BM];
@@ -272,24 +270,30 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
   // MODE 1 and 3 may cut a tile's columns over several workgroups (the others need whole rows): workgroup cb of a tile then
   // owns gate columns [cb I, cb I + I) of a row of row_i = column_blocks I and the up columns behind the same gate columns.
   const int ncb = MODE == 1 || MODE == 3 ? column_blocks : 1, row_i = I * ncb;
-  const TileMap tm = make_tile_map(offsets, E, BM);
+  const TileMap tm = MODE == 3 || ncb > 1 ? make_tile_map(offsets, E, BM) : make_round_tile_map<BM>(offsets, E);
   const int flat = xcd_tile(blockIdx.x, tm.total * ncb);
   if (flat >= tm.total * ncb) return;
   const int tile = flat / ncb, cb = flat - tile * ncb;
-  int e, row0, rows;
-  find_tile(tm, offsets, BM, tile, e, row0, rows);
-  e = __builtin_amdgcn_readfirstlane(e);                // the same for every lane: keep them in scalar registers
-  row0 = __builtin_amdgcn_readfirstlane(row0);
-  rows = __builtin_amdgcn_readfirstlane(rows);
-  const int nblocks = (rows + 31) >> 5;                 // 32-row blocks that hold rows: 1 .. 2 MT
+  int e, row0, rows, tile_e;                            // the same for every lane, in scalar registers
+  find_tile(tm, tile, e, row0, rows, tile_e);
+  // The tiles of an expert walk the weights of a K step from different blocks of columns on: of the tiles that run side by side on an XCD,
+  // one pays HBM's latency for a line and the others find it in L2.  A CU keeps about 40 KB of misses in flight, 47 GB/s from HBM and 90
+  // from L2.  (Not from different K offsets on: a row's sums would then depend on its place in the tile.)  Layer, weights from HBM, all tiles
+  // in the same order -> this: H = 768, I = 384, k = 6: 67 -> 63 us at T = 2049, 130 -> 126 at 6000; H = 1024, I = 512, k = 8: 160 -> 145 at
+  // 2049, 292 -> 287 at 6000, 370 -> 355 at 8192.  At I = 256 it is within 2 us either way; so is walking w_down's blocks like this, but at
+  // I = 512 (145 -> 155 us at T = 2049).
+  const int rot = NT >= 3 ? tile_e % NT : 0;
+  const int nblocks = (rows + 31) >> 5;                 // 32-row blocks that hold rows: 1 .. 2 MTP
 
   // The rest of the kernel exists once per number of blocks, chosen here, where nothing is alive yet: the copies
   // share no values, so each gets the registers the kernel would get if it were the only one.
   auto body = [&](auto nblocks_c) {
   constexpr int kBlocks = decltype(nblocks_c)::value;
+  constexpr int MT = kBlocks <= 2 ? 1 : MTP;
+  using F = FusedShape<NT, CT, MT>;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int wn = wave & 3, wm = wave >> 2;
-  // M wave wm owns blocks 2 wm and 2 wm + 1; blocks without rows are not multiplied.  The two waves of a SIMD
+  // M wave wm owns block wm of up to two, else blocks 2 wm and 2 wm + 1; blocks without rows are not multiplied.  The two waves of a SIMD
   // belong to different M waves, so what a SIMD's MFMA pipe has to do goes with the tile's blocks either way.
   const int my_blocks = __builtin_amdgcn_readfirstlane(wm == 0 ? (kBlocks < MT ? kBlocks : MT) : (kBlocks > MT ? kBlocks - MT : 0));
   const int n = lane & 31;
@@ -298,9 +302,11 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
     constexpr int i = decltype(ic)::value;
     if constexpr (i == 0) return S0; else if constexpr (i == 1) return S1; else return S2;
   };
+  // accumulator tile j of a wave holds its column tile block_of(j)
+  auto block_of = [&](int j) { const int b = j + rot; return b >= NT ? b - NT : b; };
   // slice i of the activations, columns [128 i, 128 i + 128) of all BM rows: a whole stage (BM = 128) or half of one
   auto slice = [&](int i) -> bf16_t* {
-    if constexpr (MT == 2) return i == 0 ? S0 : (i == 1 ? S1 : S2);
+    if constexpr (MTP == 2) return i == 0 ? S0 : (i == 1 ? S1 : S2);
     else return (i < 2 ? S0 : S1) + (i & 1) * (BM * 128);
   };
 
@@ -348,14 +354,15 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
       constexpr unsigned kb = BK * sizeof(bf16_t);
       // prologue, oldest first: sub-step 0, x rows of steps 0 and 1, sub-step 1
 #pragma unroll
-      for (int q = 0; q < F::kBInstr; ++q) dma16_buf(ld.w_rsrc, ld.b_voff, q * ld.bstep, S0 + q * 512 * 8 + ld.wave_elems);
+      for (int q = 0; q < F::kBInstr; ++q)
+        dma16_buf(ld.w_rsrc, ld.b_voff, (unsigned)block_of(0) * 32 * hb + q * ld.bstep, S0 + q * 512 * 8 + ld.wave_elems);
 #pragma unroll
       for (int a = 0; a < F::kAInstr; ++a) dma16_buf(ld.x_rsrc, ld.a_voff[a], 0, A0 + a * 512 * 8 + ld.wave_elems);
 #pragma unroll
       for (int a = 0; a < F::kAInstr; ++a) dma16_buf(ld.x_rsrc, ld.a_voff[a], kb, A1 + a * 512 * 8 + ld.wave_elems);
 #pragma unroll
       for (int q = 0; q < F::kBInstr; ++q)
-        dma16_buf(ld.w_rsrc, ld.b_voff, (NT == 1 ? kb : 32 * hb) + q * ld.bstep, S1 + q * 512 * 8 + ld.wave_elems);
+        dma16_buf(ld.w_rsrc, ld.b_voff, (NT == 1 ? kb : (unsigned)block_of(1) * 32 * hb) + q * ld.bstep, S1 + q * 512 * 8 + ld.wave_elems);
       zero_acc();
       auto substep = [&](auto mc, auto phc, auto tc, int s) {
         constexpr int nmt = decltype(mc)::value;
@@ -366,7 +373,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
         sync_keep_loads<F::kBInstr + (after_t0 ? F::kAInstr : 0)>();
         const bf16_t* a0 = abuf(integral_constant<int, ph>{}) + (mbase + n) * BK + pos0;
         const bf16_t* b0 = stage(integral_constant<int, cur>{}) + n * BK;
-        ld.b_soff = (unsigned)tn * 32 * hb + (unsigned)min(s + ds, nsteps - 1) * kb;
+        ld.b_soff = (unsigned)block_of(tn) * 32 * hb + (unsigned)min(s + ds, nsteps - 1) * kb;
         ld.b_dst = stage(integral_constant<int, target>{});
         ld.a_soff = (unsigned)min(s + 2, nsteps - 1) * kb;
         ld.a_dst = abuf(integral_constant<int, (ph + 2) % 3>{});
@@ -400,7 +407,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
       constexpr int t = decltype(tc)::value, par = decltype(pc)::value;
       constexpr int tn = (t + F::kDist) % NT, ds = (t + F::kDist) / NT;
       constexpr int target = NT == 1 ? (par + ds) % 2 : tn;
-      ld.b_soff = (unsigned)tn * 32 * hb + (unsigned)min(s + ds, nsteps - 1) * (unsigned)(BK * sizeof(bf16_t));
+      ld.b_soff = (unsigned)block_of(tn) * 32 * hb + (unsigned)min(s + ds, nsteps - 1) * (unsigned)(BK * sizeof(bf16_t));
       ld.b_dst = stage(std::integral_constant<int, target>{});
       ld.a_soff = (unsigned)min(s + 1, nsteps - 1) * (unsigned)(BK * sizeof(bf16_t));
       ld.a_dst = par ? A0 : A1;
@@ -408,13 +415,14 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
     // prologue: the first kDist sub-steps' weight rows and the x rows of step 0 (weight rows first: they do not wait
     // for the row indices)
 #pragma unroll
-    for (int q = 0; q < F::kBInstr; ++q) dma16_buf(ld.w_rsrc, ld.b_voff, q * ld.bstep, S0 + q * 512 * 8 + ld.wave_elems);
+    for (int q = 0; q < F::kBInstr; ++q)
+      dma16_buf(ld.w_rsrc, ld.b_voff, (unsigned)block_of(0) * 32 * hb + q * ld.bstep, S0 + q * 512 * 8 + ld.wave_elems);
 #pragma unroll
     for (int a = 0; a < F::kAInstr; ++a) dma16_buf(ld.x_rsrc, ld.a_voff[a], 0, A0 + a * 512 * 8 + ld.wave_elems);
     if constexpr (F::kDist == 2) {
 #pragma unroll
       for (int q = 0; q < F::kBInstr; ++q)
-        dma16_buf(ld.w_rsrc, ld.b_voff, 32 * hb + q * ld.bstep, S1 + q * 512 * 8 + ld.wave_elems);   // sub-step (0, 1)
+        dma16_buf(ld.w_rsrc, ld.b_voff, (unsigned)block_of(1) * 32 * hb + q * ld.bstep, S1 + q * 512 * 8 + ld.wave_elems);   // sub-step (0, 1)
     }
     zero_acc();
     auto substep = [&](auto mc, auto tc, auto pc, int s) {
@@ -464,7 +472,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
       for (int j = 0; j < 2 * NT; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const int half = j / NT, col = (wn * NT + j % NT) * 32 + 8 * q;
+          const int half = j / NT, col = (wn * NT + block_of(j % NT)) * 32 + 8 * q;
           *reinterpret_cast<floatx4*>(prow + half * row_i + col) =
               floatx4{acc[mt][j][4 * q], acc[mt][j][4 * q + 1], acc[mt][j][4 * q + 2], acc[mt][j][4 * q + 3]};
         }
@@ -483,7 +491,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
         const int m = mbase + mt * 32 + n;
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-          const int tile32 = wn * NT + j;
+          const int tile32 = wn * NT + block_of(j);
           bf16_t* hrow = slice(tile32 >> 2) + m * 128 + 4 * hh;
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
@@ -519,11 +527,21 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
   const int hh = lane >> 5;
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
+    float part[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      part[j] = 0.f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) part[j] = fmaf(acc[mt][j][i], acc[mt][j][i], part[j]);
+    }
     float sq = 0.f;
 #pragma unroll
-    for (int j = 0; j < NT; ++j)
+    for (int b = 0; b < NT; ++b) {            // in column order, whichever block the tile began with
+      float v = part[0];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) sq = fmaf(acc[mt][j][i], acc[mt][j][i], sq);
+      for (int j = 1; j < NT; ++j) v = block_of(j) == b ? part[j] : v;
+      sq += v;
+    }
     sq += __shfl_xor(sq, 32, kWave);
     if (hh == 0) ssq[wn * BM + mbase + mt * 32 + n] = sq;
   }
@@ -560,7 +578,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
       const float nrl = -1.44269504f * rinv, rg = rinv * gain_s[m];            // per-row constants folded once
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
-        const int tile32 = wn * NT + j;      // 32-column tile of the activation row: slice tile32 / 4, granules (tile32 % 4) * 4 + q
+        const int tile32 = wn * NT + block_of(j);      // 32-column tile of the activation row: slice tile32 / 4, granules (tile32 % 4) * 4 + q
         bf16_t* hrow = slice(tile32 >> 2) + m * 128 + 4 * hh;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {        // columns tile32*32 + 8*q + 4*hh + 0..3: half of a granule
@@ -584,8 +602,8 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
   for (int nb = 0; nb < nblk; ++nb)
     down_block<F, CT, KB, D, NB, 2 * kBlocks>(slice, wb, wp, tile_stride, nb + 1 < nblk, nb * F::BN2, w_s, slot_s, rows, A0, A1, H, yw);
   };   // body
-  if (MT == 2 && nblocks == 4) body(std::integral_constant<int, 2 * MT>{});
-  else if (MT == 2 && nblocks == 3) body(std::integral_constant<int, 2 * MT - 1>{});
+  if (MTP == 2 && nblocks == 4) body(std::integral_constant<int, 2 * MTP>{});
+  else if (MTP == 2 && nblocks == 3) body(std::integral_constant<int, 2 * MTP - 1>{});
   else if (nblocks == 2) body(std::integral_constant<int, 2>{});
   else body(std::integral_constant<int, 1>{});
 }
@@ -615,7 +633,7 @@ __global__ __launch_bounds__(512) void down_act_kernel(const float* __restrict__
   if (flat >= tm.total * nblk) return;
   const int tile = flat / nblk, nb = flat - tile * nblk;
   int e, row0, rows;
-  find_tile(tm, offsets, BM, tile, e, row0, rows);
+  find_tile(tm, tile, e, row0, rows);
   e = __builtin_amdgcn_readfirstlane(e);
   row0 = __builtin_amdgcn_readfirstlane(row0);
   rows = __builtin_amdgcn_readfirstlane(rows);
@@ -732,7 +750,7 @@ template <int NT, int CT, int MT>
 void launch_fused_t(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const float* theta, const float* w,
                     const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int S, int H, int E,
                     int act, unsigned x_bytes, bf16_t* yw, bf16_t* preact, hipStream_t s) {
-  const int grid = ((S / (64 * MT) + E + 7) & ~7) + 8;
+  const int grid = round_tiles_most(S, E, 64 * MT);
   if constexpr (NT < 4) {                    // (a state-keeping forward has I <= 384)
     if (preact != nullptr) {
       hipLaunchKernelGGL((experts_fused_kernel<NT, CT, 2, MT>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta, w, offsets,
@@ -768,7 +786,7 @@ void launch_raw_nt(const bf16_t* x, const bf16_t* wgu, const int32_t* offsets, c
                    unsigned x_bytes, bf16_t* gu, int column_blocks, hipStream_t s) {
   constexpr int MT = NT == 4 ? 1 : 2;
   const int tiles = S / (64 * MT) + E < S ? S / (64 * MT) + E : S;
-  const int grid = ((tiles * column_blocks + 7) & ~7) + 8;
+  const int grid = MODE == 3 || column_blocks > 1 ? ((tiles * column_blocks + 7) & ~7) + 8 : round_tiles_most(S, E, 64 * MT);
   hipLaunchKernelGGL((experts_fused_kernel<NT, 1, MODE, MT>), dim3(grid), dim3(512), 0, s, x, wgu, nullptr, nullptr, nullptr,
                      offsets, nullptr, perm_token, H, E, 0, x_bytes, nullptr, gu, column_blocks);
 }

@@ -40,7 +40,7 @@ __global__ __launch_bounds__(256 * WM) void gateup_dma_kernel(const bf16_t* __re
   const int tile = xcd_tile(blockIdx.x, tm.total);
   if (tile >= tm.total) return;
   int e, row0, rows;
-  find_tile(tm, offsets, BM, tile, e, row0, rows);
+  find_tile(tm, tile, e, row0, rows);
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int wn = wave & 3, wm = wave >> 2;
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(256 * WM) void down_dma_kernel(const bf16_t* __rest
   if (flat >= total) return;
   const int tile = flat / nblk_n, nb = flat - tile * nblk_n;
   int e, row0, rows;
-  find_tile(tm, offsets, BM, tile, e, row0, rows);
+  find_tile(tm, tile, e, row0, rows);
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int wn = wave & 3, wm = wave >> 2;

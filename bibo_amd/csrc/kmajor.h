@@ -169,7 +169,7 @@ __global__ __launch_bounds__(512) void dgrad_kmajor_kernel(const bf16_t* __restr
   if (flat >= total) return;
   const int tile = flat / nblk_n, nb = flat - tile * nblk_n;
   int e, row0, rows;
-  find_tile(tm, offsets, BM, tile, e, row0, rows);
+  find_tile(tm, tile, e, row0, rows);
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int wn = wave & 3, wm = wave >> 2;

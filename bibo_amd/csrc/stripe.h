@@ -12,32 +12,78 @@ namespace {
 constexpr int kLoadsPerPair = 1;   // load instructions of the next stage issued per (sub-step, N tile) pair
 constexpr int kBK = 32;        // default K elements per LDS stage
 
+// Everything but `total` is per lane (lane = expert) and stays in registers, so that a tile is found without a second read of the
+// offsets.  Built and searched by whole waves.
 struct TileMap {
-  int incl;    // lane = expert: inclusive tile count
-  int ntile;   // lane = expert: tiles of this expert
+  int lo, n;   // first row and rows of this expert
+  int ntile;   // its tiles
+  int incl;    // inclusive tile count
   int total;
+  int height;  // rows of a tile
 };
 
-__device__ __forceinline__ TileMap make_tile_map(const int32_t* __restrict__ offsets, int E, int BM) {
-  const int lane = lane_id();
-  int lo = 0, hi = 0;
-  if (lane < E) { lo = offsets[lane]; hi = offsets[lane + 1]; }
-  TileMap tm;
-  tm.ntile = (hi - lo + BM - 1) / BM;
+__device__ __forceinline__ void count_tiles(TileMap& tm, int height) {
+  tm.height = height;
+  tm.ntile = (int)((unsigned)(tm.n + height - 1) / (unsigned)height);
   tm.incl = wave_inclusive_scan(tm.ntile);
-  tm.total = __shfl(tm.incl, kWave - 1, kWave);
+  tm.total = __builtin_amdgcn_readlane(tm.incl, kWave - 1);
+}
+
+__device__ __forceinline__ TileMap load_tile_map(const int32_t* __restrict__ offsets, int E) {
+  const int lane = lane_id();
+  TileMap tm;
+  tm.lo = 0;
+  tm.n = 0;
+  if (lane < E) { tm.lo = offsets[lane]; tm.n = offsets[lane + 1] - tm.lo; }
   return tm;
 }
 
-// tile < tm.total required
-__device__ __forceinline__ void find_tile(const TileMap& tm, const int32_t* __restrict__ offsets, int BM, int tile,
-                                          int& expert, int& row0, int& rows) {
-  const unsigned long long m = __ballot(tm.incl > tile);
-  expert = __ffsll((long long)m) - 1;
-  const int excl = __shfl(tm.incl - tm.ntile, expert, kWave);
-  const int lo = offsets[expert], hi = offsets[expert + 1];
-  row0 = lo + (tile - excl) * BM;
-  rows = min(BM, hi - row0);
+__device__ __forceinline__ TileMap make_tile_map(const int32_t* __restrict__ offsets, int E, int BM) {
+  TileMap tm = load_tile_map(offsets, E);
+  count_tiles(tm, BM);
+  return tm;
+}
+
+// Tile heights for a kernel whose workgroups fill a CU each, in whole 32-row blocks up to BM.  What a tile costs is first of all the
+// stream of its expert's weights through its CU, whatever its rows (64 experts, H = 768, I = 384, 256 tiles: 38 us at 32 rows, 44 at 64,
+// 50 at 96, 57 at 128), so the rounds of kCUs tiles count first, and within them the height: the lowest tiles that still fit the rounds
+// that tiles of BM rows take.  Counted from the rows as routed: one tile more than a round is a round more.  T = 1024, k = 6: 57 -> 38 us,
+// 2049: 57 -> 45, 3001: 57 -> 50, 6000: 106 -> 88.
+constexpr int kCUs = 256, kBlockRows = 32;
+template <int BM>
+__device__ __forceinline__ TileMap make_round_tile_map(const int32_t* __restrict__ offsets, int E) {
+  static_assert(BM == 64 || BM == 128, "two or four blocks");
+  TileMap tm = load_tile_map(offsets, E);
+  count_tiles(tm, BM);
+  const int room = (int)((unsigned)(tm.total + kCUs - 1) / kCUs * kCUs);
+  count_tiles(tm, kBlockRows);
+  if (tm.total <= room) return tm;
+  if constexpr (BM == 128) {
+    count_tiles(tm, 2 * kBlockRows);
+    if (tm.total <= room) return tm;
+    count_tiles(tm, 3 * kBlockRows);
+    if (tm.total <= room) return tm;
+  }
+  count_tiles(tm, BM);
+  return tm;
+}
+// What such a map can come to, for the grid: the rounds that tiles of BM rows are sure to fit, or every tile at its lowest.
+inline int round_tiles_most(int S, int E, int BM) {
+  const long long rounds = ((long long)S / BM + E + kCUs - 1) / kCUs, low = (long long)S / kBlockRows + E;
+  return (int)((rounds * kCUs < low ? rounds * kCUs : low) + 7) & ~7;
+}
+
+// tile < tm.total required; tile_e: which of its expert's tiles it is.  (Rows spread evenly over an expert's tiles were 1 to 2 us slower:
+// the short last tiles end early.)
+__device__ __forceinline__ void find_tile(const TileMap& tm, int tile, int& expert, int& row0, int& rows, int& tile_e) {
+  expert = __ffsll((long long)__ballot(tm.incl > tile)) - 1;
+  tile_e = tile - (__builtin_amdgcn_readlane(tm.incl, expert) - __builtin_amdgcn_readlane(tm.ntile, expert));
+  row0 = __builtin_amdgcn_readlane(tm.lo, expert) + tile_e * tm.height;
+  rows = min(tm.height, __builtin_amdgcn_readlane(tm.n, expert) - tile_e * tm.height);
+}
+__device__ __forceinline__ void find_tile(const TileMap& tm, int tile, int& expert, int& row0, int& rows) {
+  int tile_e;
+  find_tile(tm, tile, expert, row0, rows, tile_e);
 }
 
 // ---- stage layout and loads ----------------------------------------------------------------------

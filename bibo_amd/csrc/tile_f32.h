@@ -67,7 +67,7 @@ __global__ __launch_bounds__(256, 4) void ggemm_f32_kernel(const TA* __restrict_
   if (flat >= total) return;
   const int tile = flat / nblk_n, nb = flat - tile * nblk_n;
   int e, row0, rows;
-  find_tile(tm, offsets, BM, tile, e, row0, rows);
+  find_tile(tm, tile, e, row0, rows);
   e = __builtin_amdgcn_readfirstlane(e);
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int n0 = nb * BN;
