@@ -52,12 +52,7 @@ int check_dims(int T, int H, int E, int k, int I, int dtype, int n_pos = 0, int 
   return BIBO_OK;
 }
 
-// Rows per expert at or below which the weight-streaming kernels are preferred (measured against the tile kernels
-// at E = 64, k = 6, whole layer).  With H and I up to 512 a wave's 16 weight rows stay in registers for all of the
-// expert's rows and a further 16-row pass only costs its staging: the crossover against the fused kernel is near 24
-// rows.  Wider rows are streamed again, from L2, for every pass: against the fused kernel they win up to about 10
-// rows (H = 768, I = 384), against the two-kernel MFMA path (shapes the fused kernel does not take) up to about 17
-// (H = 1024, I = 512).
+// Rows per expert up to which `auto` resolves to the weight-streaming family by name.
 inline long long stream_rows_per_expert(int H, int I, int dtype) {
   if (H <= 512 && I <= 512) return 24;
   return fused_supported(H, I, dtype) ? 10 : 17;
@@ -80,6 +75,17 @@ inline bool stream_eligible(int T, int H, int E, int k, int I, int dtype, bool d
   return stream_possible(T, H, E, k, I, dtype, distinct) && (long long)T * k <= stream_rows_per_expert(H, I, dtype) * E;
 }
 
+// Routed slots up to which a call that `auto` resolved to streaming does stream; beyond them the tile kernels take it under that name.  With H
+// and I up to 512 a wave's 16 weight rows stay in registers for all of the expert's rows, and a further 16-row pass only costs its
+// staging.  Wider rows are streamed again, from L2, for every pass of 16 that some expert needs.  Sum of the layer's kernels, streaming ->
+// tiles: H = 512, I = 256, E = 64: 31 -> 31 us at 9 rows per expert with weights in the Infinity Cache, 34 -> 35 at 12 and 39 -> 36 at 18
+// from HBM; E = 32: 27 -> 31 at 12, 32 -> 30 at 20; E = 16: 28 -> 30 at 20, 36 -> 29 at 36; E = 9: 24 -> 25 at 14, 30 -> 29 at 28.
+// H = 1024, I = 512, E = 64: 63 -> 63 at 10, 69 -> 63 at 12, 80 -> 63 at 16; E = 9: 30 -> 34 at 11, 38 -> 34 at 14.
+inline long long stream_slots(int E, int H, int I, int dtype) {
+  if (H <= 512 && I <= 512) return 24 * E < 704 ? 24 * E : 704;
+  return (fused_wide_supported(H, I, dtype) ? 11LL : 17LL) * E;
+}
+
 // What `auto` runs in a composite call under the name of a family: the fused kernel on shorter tiles where it resolves to the
 // MFMA family at I = 512 (H = 1024, T = 3001, k = 8: 199 -> 167 us), and the fused kernel's two halves with a tile's columns cut over
 // several workgroups where there are few tiles (split_columns).  An explicit request for a family runs the kernels its stage
@@ -87,7 +93,12 @@ inline bool stream_eligible(int T, int H, int E, int k, int I, int dtype, bool d
 constexpr int kAlgoFusedWide = 100, kAlgoSplit = 101;
 inline int composite_algo(bool automatic, int resolved, int T, int H, int E, int k, int I, int dtype) {
   if (!automatic) return resolved;
-  const bool wide = resolved == BIBO_ALGO_MFMA && fused_wide_supported(H, I, dtype) && fused_fits(T, H);
+  const bool fits = fused_fits(T, H);
+  if (resolved == BIBO_ALGO_STREAM && (long long)T * k > stream_slots(E, H, I, dtype) && fits) {
+    if (fused_supported(H, I, dtype)) resolved = BIBO_ALGO_FUSED;
+    else if (fused_wide_supported(H, I, dtype)) resolved = BIBO_ALGO_MFMA;
+  }
+  const bool wide = resolved == BIBO_ALGO_MFMA && fused_wide_supported(H, I, dtype) && fits;
   if ((wide || resolved == BIBO_ALGO_FUSED) && split_columns(T * k, E, H, I)) return kAlgoSplit;
   return wide ? kAlgoFusedWide : resolved;
 }

@@ -824,21 +824,22 @@ hipError_t launch_gateup_raw(const void* x, const void* wgu, const int32_t* offs
   return hipGetLastError();
 }
 
-// Whether a tile's columns are cut over several workgroups.  The fused kernel keeps a row's tile on one CU, which is what pulls the
-// expert's weights then: with fewer tiles than CUs most of the chip idles.  Cut (launch_gateup_raw, launch_down_act), the
-// pre-activations make a round trip and every column block computes the activations again.  A workgroup fills a CU in either half, so
-// what decides is whether tiles x blocks (I / 128 in the first half, H / 256 or, where 256 does not divide H, H / 128 in the second)
-// still run in about one round of 256: a second round costs more than the cut gives.  The limits are in tiles as expected here (an
-// expert's last one half full).  Whole layer, uncut -> cut, six layers' weights in turn, bf16:
-//   I = 512 (4 blocks), H = 1024: 92 -> 70 us at 41 tiles, 89 -> 84 at 66, 97 -> 91 or 89 -> 94 at 72, 95 -> 101 at 80; H = 512: 60 -> 59 at 65
-//   I = 384 (3 blocks), H = 768: 64 -> 51 at 38, 76 -> 70 at 80, 78 -> 98 at 102; H = 1024: 90 -> 81 at 77, 90 -> 94 at 83; H = 512:
-//     58 -> 55 at 77, 58 -> 62 at 83; H = 640 (5 blocks in the second half): 59 -> 53 at 44, 64.5 -> 63 at 59, 66.5 -> 67 at 65
-//   I = 256, H = 1024 (4 blocks in the second half): 60 -> 51 at 38, 67 -> 63 at 64, 74 -> 74 at 80; H = 512, where the weights are too
-//     light to matter: within 1 us either way up to 56 tiles from memory, 45 -> 34 with 16 experts' weights in L2
+// Whether a tile's columns are cut over several workgroups.  The fused kernel keeps a row's tile on one CU, which pulls all of the expert's
+// weights then, at HBM's latency where no other tile of the expert runs beside it.  Cut (launch_gateup_raw, launch_down_act), each CU pulls a
+// part of them, the pre-activations make a round trip and every column block computes the activations again.  So the limit, in routed slots,
+// goes with the weights of an expert, H x I; with the experts, because many of them share what the chip's L2s deliver; and with few experts
+// as the square of H x I, because their tiles are short streams then that the second launch outweighs.  At I = 512 the second half's tiles
+// of 64 rows come to two rounds from about 3600 slots on.  Sum of the layer's kernels, uncut -> cut, cold weights, bf16:
+//   E = 64, k = 6: H = 768, I = 384: 60 -> 46 us at 768 slots, 61 -> 56 at 3072, 57 -> 59 at 3600; H = 512, I = 384: 47 -> 46 at 1920,
+//     46 -> 47 at 2400; H = 1024, I = 256: 56 -> 53 at 2700, 55 -> 56 at 3072; H = 512, I = 256: 36 -> 35 at 768, 36 -> 37 at 1152
+//   E = 64, k = 8, H = 1024, I = 512: 90 -> 68 at 2048, 89 -> 72 at 2800, 84 -> 86 at 3600
+//   E = 16, k = 3: H = 768, I = 384: 42 -> 32 at 192, 44 -> 43 at 1536, 44 -> 45 at 1800; H = 768, I = 256: 37 -> 33 at 384, 35 -> 36 at 576;
+//     H = 512, I = 256: 30 -> 29 at 384, 29 -> 33 at 576; H = 1024, I = 512: 59 -> 53 at 3072, 60 -> 66 at 4095
+//   E = 9, k = 2, H = 512, I = 256: 29 -> 29 at 256, 30 -> 34 at 384, 30 -> 40 at 2048
 // Pre-activations in bf16 were 1 to 5 us faster and half again as far from the exact result (3.5e-3 against 2.3e-3).
 bool split_columns(int S, int E, int H, int I) {
-  const int limit = I >= 512 ? 66 : I >= 384 ? (H % 256 == 0 ? 77 : 60) : (H * I >= 256 * 1024 ? 64 : 40);
-  return S / 128 + E / 2 <= limit && I >= 256;
+  const long long hi = (long long)H * I / 1024;
+  return I >= 256 && S <= 3600 && S <= hi * (46 + E) / 10 && S <= hi * hi * E / 763;
 }
 
 // gu [S, 2I] fp32 -> routing-weighted rows in slot order, and with `preact` their bf16 copy (down_act_kernel; I <= 384); shapes as
