@@ -166,32 +166,41 @@ hipError_t launch_dgrad(const bf16_t* A, const int32_t* a_index, const bf16_t* W
   return launch_dgrad_t<1, GATHER, SCATTER>(A, a_index, W, offsets, out_index, S_rows, K, N, E, out, s);
 }
 
-// dW[e] = P(rows of e)^T Q(rows of e), P [.., N] and Q [.., M] row-major (kmajor.h)
-template <int MT, bool GATHER_P, bool GATHER_Q>
-hipError_t launch_wgrad_t(const bf16_t* P, const bf16_t* Q, const int32_t* index, const int32_t* offsets, const bf16_t* zrow,
-                          int N, int M, int E, int slots, const int* plan, float* part, void* dW, int f32, hipStream_t s) {
-  const dim3 block(512);               // (the partial tiles of cut experts are added up by backward_sums_kernel)
-  auto grid = [&](int bn) { return dim3((unsigned)((slots * (N / (64 * MT)) * (M / bn) + 7) & ~7)); };
-  if (M % 384 == 0)
-    hipLaunchKernelGGL((wgrad_kmajor_kernel<MT, 3, GATHER_P, GATHER_Q>), grid(384), block, 0, s, P, Q, index, offsets, zrow, N,
-                       M, E, plan, part, dW, f32);
-  else if (M % 256 == 0)
-    hipLaunchKernelGGL((wgrad_kmajor_kernel<MT, 2, GATHER_P, GATHER_Q>), grid(256), block, 0, s, P, Q, index, offsets, zrow, N,
-                       M, E, plan, part, dW, f32);
-  else
-    hipLaunchKernelGGL((wgrad_kmajor_kernel<MT, 1, GATHER_P, GATHER_Q>), grid(128), block, 0, s, P, Q, index, offsets, zrow, N,
-                       M, E, plan, part, dW, f32);
-  return hipGetLastError();
-}
+// How many 128-column sub-tiles a workgroup takes of an extent.
+inline int sub_tiles(int n) { return n % 384 == 0 ? 3 : n % 256 == 0 ? 2 : 1; }
 
-// 256 rows of dW per workgroup where N allows and the experts have rows enough for the streams to matter
-template <bool GATHER_P, bool GATHER_Q>
-hipError_t launch_wgrad(const bf16_t* P, const bf16_t* Q, const int32_t* index, const int32_t* offsets, const bf16_t* zrow,
-                        int N, int M, int S_rows, int E, int slots, const int* plan, float* part, void* dW, int f32, hipStream_t s) {
-  const int bn = M % 384 == 0 ? 384 : (M % 256 == 0 ? 256 : 128);
-  if (N % 256 == 0 && tall_tiles(S_rows, E, (long long)E * (N / 128) * (M / bn), (long long)E * (N / 256) * (M / bn)))
-    return launch_wgrad_t<4, GATHER_P, GATHER_Q>(P, Q, index, offsets, zrow, N, M, E, slots, plan, part, dW, f32, s);
-  return launch_wgrad_t<2, GATHER_P, GATHER_Q>(P, Q, index, offsets, zrow, N, M, E, slots, plan, part, dW, f32, s);
+// dx of every slot and both weight gradients (kmajor.h: backward_gemms_kernel).  256-row tiles, which stream the other operand half as
+// often and take 1.75 times as long, where the experts hold 192 rows on average and the launch is several rounds of workgroups, whose last
+// one the three products share.
+hipError_t launch_backward_gemms(BackwardGemms g, int S, int slots, hipStream_t s) {
+  const int H = g.H, I = g.I, E = g.E, nh = sub_tiles(H), ni = sub_tiles(I), bh = kSubW * nh, bi = kSubW * ni;
+  auto pad8 = [](long long n) { return (int)((n + 7) & ~7ll); };
+  auto dx = [&](int rows) { return ((long long)S / rows + E) * (H / bh); };
+  auto gu = [&](int rows) { return (long long)slots * (2 * I / rows) * (H / bh); };
+  auto down = [&](int rows) { return (long long)slots * (H / rows) * (I / bi); };
+  const bool tall = (long long)S >= 192ll * E && dx(128) + gu(128) + down(128) > 3 * kCUs;
+  g.tall_dx = tall;
+  g.tall_gu = tall && 2 * I % 256 == 0;
+  g.tall_d = tall && H % 256 == 0;
+  g.n_dx = pad8(dx(g.tall_dx ? 256 : 128));
+  g.n_gu = pad8(gu(g.tall_gu ? 256 : 128));
+  const int n_d = pad8(down(g.tall_d ? 256 : 128));
+  const dim3 grid((unsigned)(g.n_dx + g.n_gu + n_d));
+  using std::integral_constant;
+  auto launch = [&](auto hc, auto ic) {
+    constexpr int NH = decltype(hc)::value, NI = decltype(ic)::value;
+    if (g.tall_dx || g.tall_gu || g.tall_d) hipLaunchKernelGGL((backward_gemms_kernel<NH, NI, true>), grid, dim3(512), 0, s, g);
+    else hipLaunchKernelGGL((backward_gemms_kernel<NH, NI, false>), grid, dim3(512), 0, s, g);
+  };
+  auto by_i = [&](auto hc) {
+    if (ni == 3) launch(hc, integral_constant<int, 3>{});
+    else if (ni == 2) launch(hc, integral_constant<int, 2>{});
+    else launch(hc, integral_constant<int, 1>{});
+  };
+  if (nh == 3) by_i(integral_constant<int, 3>{});
+  else if (nh == 2) by_i(integral_constant<int, 2>{});
+  else by_i(integral_constant<int, 1>{});
+  return hipGetLastError();
 }
 
 // ---- Radial NormSiLU backward (moe.py:87-92), one wave per permuted row ----------------------------------------
@@ -567,9 +576,13 @@ hipError_t launch_backward(const void* x, const void* d_out, const void* w_route
   hipLaunchKernelGGL(act_bwd_kernel, dim3((S + 3) / 4), dim3(256), 0, s, gu, dhp, w, theta, offsets, perm_slot, S, E, I, act,
                      dgu, hidden, b.dw_slot, b.dtheta_row, reinterpret_cast<uint32_t*>(zrow),
                      (int)(backward_zero_row_bytes(H, I) / 4), b.wgrad_plan, Et, backward_chunk_rows(S, Et), slots);
-  // dx of every slot, in slot order: [dg, du] W_gate_up, contracts over the 2I rows of w_gate_up [E, 2I, H]
-  err = launch_dgrad<false, true>(dgu, nullptr, wgup, offsets, perm_slot, S, 2 * I, H, E, dxs, s);
-  if (err != hipSuccess) return err;
+  // dx of every slot, in slot order: [dg, du] W_gate_up, contracts over the 2I rows of w_gate_up [E, 2I, H].  Weight gradients,
+  // contracted over each expert's rows: dW_down[e] = d^T (w h) (d gathered by token, `hidden` already carries w), dW_gate_up[e] =
+  // [dg, du]^T x (x gathered by token)
+  float* part_gu = b.wgrad_part + (size_t)slots * H * I;
+  BackwardGemms gemms{xp, dop, dgu, hidden, wgup, zrow, offsets, perm_slot, perm_token, b.wgrad_plan, dxs, d_wgu, d_wd, part_gu,
+                      b.wgrad_part, H, I, E, grad_f32, 0, 0, false, false, false};
+  if ((err = launch_backward_gemms(gemms, S, slots, s)) != hipSuccess) return err;
   const bool with_router = w_router != nullptr;      // else: the experts alone, the caller owns the routing
   const int parts = (H / 8 + kWave - 1) / kWave;     // runs of columns a lane each
   auto token_bwd = [&](auto kc) {
@@ -591,13 +604,6 @@ hipError_t launch_backward(const void* x, const void* d_out, const void* w_route
   if (with_router)
     hipLaunchKernelGGL(dwr_partial_kernel, dim3((H + 255) / 256, slots, kDwrSplit), dim3(256), 0, s, xp, b.dl, b.wgrad_plan,
                        perm_slot, perm_token, H, b.dwr_part);
-  // weight gradients, contracted over each expert's rows: dW_down[e] = d^T (w h) (d gathered by token, `hidden`
-  // already carries w), dW_gate_up[e] = [dg, du]^T x (x gathered by token)
-  err = launch_wgrad<true, false>(dop, hidden, perm_token, offsets, zrow, H, I, S, E, slots, b.wgrad_plan, b.wgrad_part, d_wd, grad_f32, s);
-  if (err != hipSuccess) return err;
-  float* part_gu = b.wgrad_part + (size_t)slots * H * I;
-  err = launch_wgrad<false, true>(dgu, xp, perm_token, offsets, zrow, 2 * I, H, S, E, slots, b.wgrad_plan, part_gu, d_wgu, grad_f32, s);
-  if (err != hipSuccess) return err;
   // the sums that end the pass: cut experts' partial tiles, dtheta, the router's weight gradient
   const int nb_w = (int)(((size_t)2 * I * H / 4 + 255) / 256);
   const int nb_r = with_router ? (Et * H + 255) / 256 : 0;

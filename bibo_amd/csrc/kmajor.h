@@ -136,6 +136,13 @@ __device__ __forceinline__ void afill(const bf16_t* row, bf16_t* tile) {
 // waves, requests stage i + 3 into the buffer stage i - 1 was read from, and multiplies stage i.  Every step issues
 // the same number of transfers (a request past the last stage repeats the last one), so the wait count is a constant.
 
+// The stages of a ring, a row operand's and a column operand's each, as a kernel declares them; the fourth ones only for rings of four.
+struct Ring {
+  bf16_t *a0, *a1, *a2, *a3, *b0, *b1, *b2, *b3;
+  template <int I> __device__ __forceinline__ bf16_t* a() const { return I == 0 ? a0 : I == 1 ? a1 : I == 2 ? a2 : a3; }
+  template <int I> __device__ __forceinline__ bf16_t* b() const { return I == 0 ? b0 : I == 1 ? b1 : I == 2 ? b2 : b3; }
+};
+
 // ---- input gradients: out[dst(r), n] = sum_k A[src(r), k] W[e][k, n] for the rows r of expert e ----------------
 // A row-major (K contiguous), W K-major as stored: [K, N] per expert.  src(r) = a_index[r] (GATHER) or r; dst(r) =
 // out_index[r] (SCATTER) or r.  Workgroup = 64 MT rows x 128 NTW columns, 2 x 4 waves, 32x32x16 MFMA, operands swapped
@@ -143,29 +150,19 @@ __device__ __forceinline__ void afill(const bf16_t* row, bf16_t* tile) {
 // 256-row tiles for experts with many rows - an expert's weights then pass through LDS once per 256 rows instead of
 // once per 128, which is what these kernels are bound by; 192 accumulator registers and 40 KB stages, ring of three.
 template <int MT, int NTW, bool GATHER, bool SCATTER>
-__global__ __launch_bounds__(512) void dgrad_kmajor_kernel(const bf16_t* __restrict__ A, const int32_t* __restrict__ a_index,
-                                                           const bf16_t* __restrict__ W,
-                                                           const int32_t* __restrict__ offsets,
-                                                           const int32_t* __restrict__ out_index, int K, int N, int E,
-                                                           int nblk_n, bf16_t* __restrict__ out) {
+__device__ __forceinline__ void dgrad_block(const Ring& ring, int* dst_s, int block, const bf16_t* __restrict__ A,
+                                            const int32_t* __restrict__ a_index, const bf16_t* __restrict__ W,
+                                            const int32_t* __restrict__ offsets, const int32_t* __restrict__ out_index, int K, int N, int E,
+                                            int nblk_n, bf16_t* __restrict__ out) {
   static_assert(MT == 2 || MT == 4, "128- or 256-row tiles");
   constexpr int BM = 64 * MT, BN = kSubW * NTW;
   constexpr int R = MT == 4 ? 3 : kRing;                 // stages that fit LDS
   constexpr int kAOps = MT / 2;                          // 128-row blocks of the row operand
   constexpr int kOps = kAOps + NTW;                      // transfers per thread and stage
-  __shared__ __attribute__((aligned(16))) bf16_t a0[kAOps * kATile];
-  __shared__ __attribute__((aligned(16))) bf16_t a1[kAOps * kATile];
-  __shared__ __attribute__((aligned(16))) bf16_t a2[kAOps * kATile];
-  __shared__ __attribute__((aligned(16))) bf16_t a3[R == 4 ? kAOps * kATile : 8];
-  __shared__ __attribute__((aligned(16))) bf16_t b0[NTW * kSubElems];
-  __shared__ __attribute__((aligned(16))) bf16_t b1[NTW * kSubElems];
-  __shared__ __attribute__((aligned(16))) bf16_t b2[NTW * kSubElems];
-  __shared__ __attribute__((aligned(16))) bf16_t b3[R == 4 ? NTW * kSubElems : 8];
-  __shared__ int dst_s[BM];
 
   const TileMap tm = make_tile_map(offsets, E, BM);
   const int total = tm.total * nblk_n;
-  const int flat = xcd_tile(blockIdx.x, total);
+  const int flat = xcd_tile(block, total);
   if (flat >= total) return;
   const int tile = flat / nblk_n, nb = flat - tile * nblk_n;
   int e, row0, rows;
@@ -187,14 +184,8 @@ __global__ __launch_bounds__(512) void dgrad_kmajor_kernel(const bf16_t* __restr
   const int n0 = nb * BN;
   const bf16_t* wrow = W + (size_t)e * K * N + (size_t)(tid >> 4) * N + n0 + kfill_granule(tid) * 8;
   const int nstages = K / kKS;
-  auto abuf = [&](auto bc) -> bf16_t* {
-    constexpr int b = decltype(bc)::value;
-    if constexpr (b == 0) return a0; else if constexpr (b == 1) return a1; else if constexpr (b == 2) return a2; else return a3;
-  };
-  auto bbuf = [&](auto bc) -> bf16_t* {
-    constexpr int b = decltype(bc)::value;
-    if constexpr (b == 0) return b0; else if constexpr (b == 1) return b1; else if constexpr (b == 2) return b2; else return b3;
-  };
+  auto abuf = [&](auto bc) -> bf16_t* { return ring.template a<decltype(bc)::value>(); };
+  auto bbuf = [&](auto bc) -> bf16_t* { return ring.template b<decltype(bc)::value>(); };
   auto fill = [&](auto bc, int stage) {
     const int k0 = min(stage, nstages - 1) * kKS;
 #pragma unroll
@@ -254,8 +245,8 @@ __global__ __launch_bounds__(512) void dgrad_kmajor_kernel(const bf16_t* __restr
   constexpr int kOutCols = NTW * 32;
   constexpr int kOutStride = kOutCols + 8;          // +16 bytes staggers the rows over the banks
   static_assert(3 * 32 * kOutStride <= NTW * kSubElems, "output staging does not fit a weight stage");
-  bf16_t* otile = b0;                    // three waves per stage buffer
-  if (wave >= 6) otile = b2; else if (wave >= 3) otile = b1;
+  bf16_t* otile = ring.b0;               // three waves per stage buffer
+  if (wave >= 6) otile = ring.b2; else if (wave >= 3) otile = ring.b1;
   otile += (wave % 3) * (32 * kOutStride);
   constexpr int kGranPerRow = kOutCols / 8;
   const int colbase = n0 + wn * kOutCols;
@@ -282,6 +273,29 @@ __global__ __launch_bounds__(512) void dgrad_kmajor_kernel(const bf16_t* __restr
     __builtin_amdgcn_s_waitcnt(0xc07f);
     __builtin_amdgcn_wave_barrier();
   }
+}
+
+// Elements of a stage's row and column operand.
+constexpr int ring_a(int MT) { return MT / 2 * kATile; }
+constexpr int ring_b(int NTW) { return NTW * kSubElems; }
+
+template <int MT, int NTW, bool GATHER, bool SCATTER>
+__global__ __launch_bounds__(512) void dgrad_kmajor_kernel(const bf16_t* __restrict__ A, const int32_t* __restrict__ a_index,
+                                                           const bf16_t* __restrict__ W, const int32_t* __restrict__ offsets,
+                                                           const int32_t* __restrict__ out_index, int K, int N, int E, int nblk_n,
+                                                           bf16_t* __restrict__ out) {
+  constexpr bool four = MT == 2;
+  __shared__ __attribute__((aligned(16))) bf16_t a0[ring_a(MT)];
+  __shared__ __attribute__((aligned(16))) bf16_t a1[ring_a(MT)];
+  __shared__ __attribute__((aligned(16))) bf16_t a2[ring_a(MT)];
+  __shared__ __attribute__((aligned(16))) bf16_t a3[four ? ring_a(MT) : 8];
+  __shared__ __attribute__((aligned(16))) bf16_t b0[ring_b(NTW)];
+  __shared__ __attribute__((aligned(16))) bf16_t b1[ring_b(NTW)];
+  __shared__ __attribute__((aligned(16))) bf16_t b2[ring_b(NTW)];
+  __shared__ __attribute__((aligned(16))) bf16_t b3[four ? ring_b(NTW) : 8];
+  __shared__ int dst_s[64 * MT];
+  dgrad_block<MT, NTW, GATHER, SCATTER>(Ring{a0, a1, a2, a3, b0, b1, b2, b3}, dst_s, blockIdx.x, A, a_index, W, offsets, out_index, K, N, E,
+                                        nblk_n, out);
 }
 
 // ---- weight gradients: dW[e][n][m] = sum over the rows r of expert e of P[srcP(r)][n] Q[srcQ(r)][m] ------------
@@ -324,25 +338,14 @@ __device__ __forceinline__ void wgrad_plan(const int32_t* __restrict__ offsets, 
 }
 
 template <int MT, int NTW, bool GATHER_P, bool GATHER_Q>
-__global__ __launch_bounds__(512) void wgrad_kmajor_kernel(const bf16_t* __restrict__ P, const bf16_t* __restrict__ Q,
-                                                           const int32_t* __restrict__ index,
-                                                           const int32_t* __restrict__ offsets,
-                                                           const bf16_t* __restrict__ zrow, int N, int M, int E,
-                                                           const int* __restrict__ plan, float* __restrict__ part,
-                                                           void* __restrict__ dW, int f32) {
+__device__ __forceinline__ void wgrad_block(const Ring& ring, int block, const bf16_t* __restrict__ P, const bf16_t* __restrict__ Q,
+                                            const int32_t* __restrict__ index, const bf16_t* __restrict__ zrow, int N, int M, int E,
+                                            const int* __restrict__ plan, float* __restrict__ part, void* __restrict__ dW, int f32) {
   static_assert(MT == 2 || MT == 4, "128 or 256 rows of dW per workgroup");
   constexpr int BM = 64 * MT, BN = kSubW * NTW;
   constexpr int R = MT == 4 ? 3 : kRing;                 // stages that fit LDS (MT = 4: 40 KB each)
   constexpr int kPOps = MT / 2;                          // 128-column sub-tiles of P
   constexpr int kOps = kPOps + NTW;
-  __shared__ __attribute__((aligned(16))) bf16_t p0[kPOps * kSubElems];
-  __shared__ __attribute__((aligned(16))) bf16_t p1[kPOps * kSubElems];
-  __shared__ __attribute__((aligned(16))) bf16_t p2[kPOps * kSubElems];
-  __shared__ __attribute__((aligned(16))) bf16_t p3[R == 4 ? kPOps * kSubElems : 8];
-  __shared__ __attribute__((aligned(16))) bf16_t q0[NTW * kSubElems];
-  __shared__ __attribute__((aligned(16))) bf16_t q1[NTW * kSubElems];
-  __shared__ __attribute__((aligned(16))) bf16_t q2[NTW * kSubElems];
-  __shared__ __attribute__((aligned(16))) bf16_t q3[R == 4 ? NTW * kSubElems : 8];
   // Workgroup ids congruent mod 8 run on one XCD: they walk a contiguous range of (expert, m block, n block) triples,
   // so the workgroups that read the same rows of Q (and of P) share that XCD's L2.
   const int nblk_n = N / BM, nblk_m = M / BN;
@@ -351,7 +354,7 @@ __global__ __launch_bounds__(512) void wgrad_kmajor_kernel(const bf16_t* __restr
   // With experts cut into chunks the work per chunk is uneven (a cut expert's chunks are several times a small
   // expert's rows) and contiguous ranges of chunks per XCD would leave some XCDs with most of it: round robin then.
   const bool uneven = __builtin_amdgcn_readfirstlane(plan[1]) > 0;
-  const int item = uneven ? (int)blockIdx.x : xcd_tile(blockIdx.x, total_chunks * nblk_n * nblk_m);
+  const int item = uneven ? block : xcd_tile(block, total_chunks * nblk_n * nblk_m);
   if (item >= total_chunks * nblk_n * nblk_m) return;
   const int cg = item / (nblk_n * nblk_m), rest = item - cg * (nblk_n * nblk_m);      // chunk, numbered over all experts
   const int* entry = plan + 4 + 4 * cg;
@@ -369,14 +372,8 @@ __global__ __launch_bounds__(512) void wgrad_kmajor_kernel(const bf16_t* __restr
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[mt][j][i] = 0.f;
 
-  auto pbuf = [&](auto bc) -> bf16_t* {
-    constexpr int b = decltype(bc)::value;
-    if constexpr (b == 0) return p0; else if constexpr (b == 1) return p1; else if constexpr (b == 2) return p2; else return p3;
-  };
-  auto qbuf = [&](auto bc) -> bf16_t* {
-    constexpr int b = decltype(bc)::value;
-    if constexpr (b == 0) return q0; else if constexpr (b == 1) return q1; else if constexpr (b == 2) return q2; else return q3;
-  };
+  auto pbuf = [&](auto bc) -> bf16_t* { return ring.template a<decltype(bc)::value>(); };
+  auto qbuf = [&](auto bc) -> bf16_t* { return ring.template b<decltype(bc)::value>(); };
   const int nstages = (hi - lo + kKS - 1) / kKS;
   const int gofs = kfill_granule(tid) * 8;
   // This thread's row of stage `stage` (row tid / 16 of the stage's 32), the expert's last row past its end.
@@ -478,6 +475,62 @@ __global__ __launch_bounds__(512) void wgrad_kmajor_kernel(const bf16_t* __restr
           *reinterpret_cast<floatx4*>(prow + (size_t)mt * 32 * M + j * 32 + 8 * q) = v;
         }
   }
+}
+
+// ---- the three products behind act_bwd_kernel in one launch --------------------------------------------------------
+// dx of every slot = [dg, du] W_gate_up (blocks [0, n_dx)), dW_gate_up = [dg, du]^T x (the next n_gu), dW_down = d^T (w h) (the rest).
+// They need nothing from one another, and a workgroup fills a CU in each: as launches of their own each ended with a round in which most
+// CUs had none, and a small call spent three launches on three handfuls of workgroups.  Longest workgroups first.  NH, NI: what 128-column
+// sub-tiles H and I divide into.  TALL: each of the three has 256-row tiles by its flag, else none (their rings are smaller).  The three
+// launches -> this one: T = 8192, H = 768, I = 384, E = 64, k = 6: 259 -> 233 us; T = 2500: 118 -> 90; T = 1111, H = 512, I = 256, E = 9,
+// k = 2: 36 -> 14; T = 16000, H = 1024, I = 512, E = 64, k = 8: 750 -> 731.
+struct BackwardGemms {
+  const bf16_t *x, *d_out, *dgu, *hidden, *wgu, *zrow;
+  const int32_t *offsets, *perm_slot, *perm_token;
+  const int* plan;
+  bf16_t* dxs;
+  void *dwgu, *dwd;
+  float *part_gu, *part_d;
+  int H, I, E, f32, n_dx, n_gu;
+  bool tall_dx, tall_gu, tall_d;
+};
+
+template <int NH, int NI, bool TALL>
+__global__ __launch_bounds__(512) void backward_gemms_kernel(BackwardGemms g) {
+  constexpr int MT = TALL ? 4 : 2, NB = NH > NI ? NH : NI;
+  __shared__ __attribute__((aligned(16))) bf16_t a0[ring_a(MT)];
+  __shared__ __attribute__((aligned(16))) bf16_t a1[ring_a(MT)];
+  __shared__ __attribute__((aligned(16))) bf16_t a2[ring_a(MT)];
+  __shared__ __attribute__((aligned(16))) bf16_t a3[ring_a(2)];
+  __shared__ __attribute__((aligned(16))) bf16_t b0[ring_b(NB)];
+  __shared__ __attribute__((aligned(16))) bf16_t b1[ring_b(NB)];
+  __shared__ __attribute__((aligned(16))) bf16_t b2[ring_b(NB)];
+  __shared__ __attribute__((aligned(16))) bf16_t b3[ring_b(NB)];
+  __shared__ int dst_s[64 * MT];
+  const Ring ring{a0, a1, a2, a3, b0, b1, b2, b3};
+  const int block = blockIdx.x;
+  using std::integral_constant;
+  auto either = [](bool tall, auto run) {
+    if constexpr (TALL) {
+      if (tall) { run(integral_constant<int, 4>{}); return; }
+    }
+    run(integral_constant<int, 2>{});
+  };
+  if (block < g.n_dx)
+    either(g.tall_dx, [&](auto mt) {
+      dgrad_block<decltype(mt)::value, NH, false, true>(ring, dst_s, block, g.dgu, nullptr, g.wgu, g.offsets, g.perm_slot, 2 * g.I, g.H, g.E,
+                                                        g.H / (kSubW * NH), g.dxs);
+    });
+  else if (block < g.n_dx + g.n_gu)
+    either(g.tall_gu, [&](auto mt) {
+      wgrad_block<decltype(mt)::value, NH, false, true>(ring, block - g.n_dx, g.dgu, g.x, g.perm_token, g.zrow, 2 * g.I, g.H, g.E, g.plan,
+                                                        g.part_gu, g.dwgu, g.f32);
+    });
+  else
+    either(g.tall_d, [&](auto mt) {
+      wgrad_block<decltype(mt)::value, NI, true, false>(ring, block - g.n_dx - g.n_gu, g.d_out, g.hidden, g.perm_token, g.zrow, g.H, g.I, g.E,
+                                                        g.plan, g.part_d, g.dwd, g.f32);
+    });
 }
 
 // For the experts that were cut into chunks (none, when the tokens are spread evenly): dW[e] = the sum of expert e's
