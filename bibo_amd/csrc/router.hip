@@ -320,6 +320,83 @@ __global__ __launch_bounds__(TOK * 16) void router_mfma_kernel(const bf16_t* __r
   router_finish<TOK>(acc, sc, bias_s, T, E, k, norm_mode, t0, logits, idx, w, gap, chunk_hist);
 }
 
+// The same for calls of at most one workgroup per CU, which are a chain of memory latencies, one a chunk with two stages: here the first
+// six chunks of the rows and of w_router are requested up front (further ones as stages fall free), so that a workgroup waits for
+// one round trip and then for its bytes.  120 KB of LDS: one workgroup a CU.
+constexpr int kRouterRing = 6, kRingLeast = 128;
+__global__ __launch_bounds__(256) void router_ring_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ wr,
+                                                          const float* __restrict__ bias, int T, int H, int E, int k, int norm_mode,
+                                                          float* __restrict__ logits, int32_t* __restrict__ idx,
+                                                          float* __restrict__ w, float* __restrict__ gap,
+                                                          int32_t* __restrict__ chunk_hist) {
+  constexpr int TOK = 16, kThreads = TOK * 16, kRows = TOK + kMaxE, kPer = kRows * kRouterGran / kThreads;
+  constexpr int kElems = kRows * kRouterKC;
+  __shared__ __attribute__((aligned(16))) bf16_t st0[kElems];
+  __shared__ __attribute__((aligned(16))) bf16_t st1[kElems];
+  __shared__ __attribute__((aligned(16))) bf16_t st2[kElems];
+  __shared__ __attribute__((aligned(16))) bf16_t st3[kElems];
+  __shared__ __attribute__((aligned(16))) bf16_t st4[kElems];
+  __shared__ __attribute__((aligned(16))) bf16_t st5[kElems];
+  __shared__ float sc[TOK * kRowPad];
+  __shared__ float bias_s[kMaxE];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int t0 = blockIdx.x * TOK;
+  const float my_bias = tid < E ? bias[tid] : 0.f;
+  const bf16_t* src[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int row = (i * kThreads + tid) / kRouterGran;
+    const int c = (tid & (kRouterGran - 1)) ^ (row & 15);
+    src[i] = (row < TOK ? x + (size_t)min(t0 + row, T - 1) * H : wr + (size_t)min(row - TOK, E - 1) * H) + c * 8;
+  }
+  auto stage = [&](auto ic) -> bf16_t* {
+    constexpr int i = decltype(ic)::value;
+    if constexpr (i == 0) return st0; else if constexpr (i == 1) return st1; else if constexpr (i == 2) return st2;
+    else if constexpr (i == 3) return st3; else if constexpr (i == 4) return st4; else return st5;
+  };
+  auto issue = [&](int chunk, bf16_t* st) {
+#pragma unroll
+    for (int i = 0; i < kPer; ++i)
+      __builtin_amdgcn_global_load_lds((router_gbl_void*)(src[i] + chunk * kRouterKC), (router_lds_void*)(st + (i * kThreads + wave * 64) * 8),
+                                       16, 0, 0);
+  };
+  const int r16 = lane & 15, kc = lane >> 4;
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+  const int nchunks = H / kRouterKC;
+  using std::integral_constant;
+  for_each<kRouterRing>([&](auto ic) { if (decltype(ic)::value < nchunks) issue(decltype(ic)::value, stage(ic)); });
+  for (int c0 = 0; c0 < nchunks; c0 += kRouterRing)
+    for_each<kRouterRing>([&](auto ic) {
+      const int c = c0 + decltype(ic)::value;
+      if (c >= nchunks) return;
+      switch (min(nchunks - 1 - c, kRouterRing - 1)) {         // chunks that may still be on their way
+        case 0: sync_keep_loads<0>(); break;
+        case 1: sync_keep_loads<kPer>(); break;
+        case 2: sync_keep_loads<2 * kPer>(); break;
+        case 3: sync_keep_loads<3 * kPer>(); break;
+        case 4: sync_keep_loads<4 * kPer>(); break;
+        default: sync_keep_loads<5 * kPer>();
+      }
+      const bf16_t* st = stage(ic);
+      const bf16_t* arow = st + r16 * kRouterKC;
+      const bf16_t* brow = st + (TOK + wave * 16 + r16) * kRouterKC;
+#pragma unroll
+      for (int s = 0; s < kRouterKC / 32; ++s) {
+        const int pos = ((s * 4 + kc) ^ r16) * 8;
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(arow + pos);
+        const bf16x8 b = *reinterpret_cast<const bf16x8*>(brow + pos);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
+      }
+      if (c + kRouterRing < nchunks) {
+        __builtin_amdgcn_s_waitcnt(0xc07f);                    // this wave's reads of the stage have returned
+        __builtin_amdgcn_s_barrier();
+        issue(c + kRouterRing, stage(ic));
+      }
+    });
+  if (tid < kMaxE) bias_s[tid] = my_bias;
+  router_finish<TOK>(acc, sc, bias_s, T, E, k, norm_mode, t0, logits, idx, w, gap, chunk_hist);
+}
+
 // ---- MFMA router with the block's input RMSNorm in front (the caller's seam) ----------------------
 // out = h + moe(post_attention_layernorm(h)) (src/modeling/layers.py:57-64) needs the normalised rows twice: as the
 // router's operand and as the rows the expert kernels gather.  This kernel reads the raw rows once: all H elements of
@@ -565,6 +642,13 @@ hipError_t launch_router(const void* x, const void* w_router, const float* bias,
     // smaller tile keeps more CUs busy
     if (T >= 32 * 256)
       hipLaunchKernelGGL(router_mfma_kernel<32>, dim3((T + 31) / 32), dim3(512), 0, s, static_cast<const bf16_t*>(x),
+                         static_cast<const bf16_t*>(w_router), bias, T, H, E, k, norm_mode, logits, idx, w, gap,
+                         chunk_hist);
+    else if (T >= kRingLeast && T <= 16 * kCUs && H >= kRouterRing * kRouterKC)
+      // us, two stages -> ring: 9.3 -> 8.0 (H = 768, T = 128), 8.6 -> 7.6 (2049), 9.2 -> 8.0 (4096); 10.7 -> 8.9 (H = 1024, T = 128 to
+      // 2049), 11.0 -> 9.0 (4096).  Few workgroups have the memory to themselves and only pay the larger launch: 5.6 -> 6.4 (H = 768,
+      // T = 16), 6.7 -> 7.4 (H = 1024); four chunks and fewer gain 0.3 at most.
+      hipLaunchKernelGGL(router_ring_kernel, dim3((T + 15) / 16), dim3(256), 0, s, static_cast<const bf16_t*>(x),
                          static_cast<const bf16_t*>(w_router), bias, T, H, E, k, norm_mode, logits, idx, w, gap,
                          chunk_hist);
     else
