@@ -217,7 +217,7 @@ int experts_dispatch(const void* x, const void* wgu, const void* wd, const float
                      const float* w, const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token,
                      const void* residual, bool idx_trusted, int T, int H, int Eg, int np, int nn, int k, int I, int dtype,
                      int algo, int act, int flags, void* out, char* base, const Workspace& ws, size_t ws_bytes,
-                     hipStream_t s, void* preact = nullptr) {
+                     hipStream_t s, void* preact = nullptr, const ScanArgs& scan = ScanArgs()) {
   float* yw = reinterpret_cast<float*>(base + ws.yw);
   CombineArgs ca;
   ca.residual = residual;
@@ -243,14 +243,14 @@ int experts_dispatch(const void* x, const void* wgu, const void* wd, const float
   if (algo == kAlgoSplit) {
     if (!aligned16(x) || !aligned16(wgu) || !aligned16(wd)) return BIBO_ERR_MISALIGNED;
     void* pre = base + ws.pre;
-    hipError_t e = launch_gateup_raw(x, wgu, offsets, perm_token, T, H, Eg, k, I, pre, true, true, s);
+    hipError_t e = launch_gateup_raw(x, wgu, offsets, perm_token, T, H, Eg, k, I, pre, true, true, s, scan);
     if (e != hipSuccess) return (int)e;
     if ((e = launch_down_act(pre, wd, theta, w, offsets, perm_slot, T * k, H, Eg, I, act, yw, preact, s)) != hipSuccess) return (int)e;
     return hip_rc(launch_combine(yw, 1, ca, T, H, k, dtype, out, s));
   }
   if (algo == BIBO_ALGO_FUSED || algo == kAlgoFusedWide) {
     if (!aligned16(x) || !aligned16(wgu) || !aligned16(wd)) return BIBO_ERR_MISALIGNED;
-    hipError_t e = launch_experts_fused(x, wgu, wd, theta, w, offsets, perm_slot, perm_token, T, H, Eg, k, I, act, yw, preact, s);
+    hipError_t e = launch_experts_fused(x, wgu, wd, theta, w, offsets, perm_slot, perm_token, T, H, Eg, k, I, act, yw, preact, s, scan);
     if (e != hipSuccess) return (int)e;
     return hip_rc(launch_combine(yw, 1, ca, T, H, k, dtype, out, s));
   }
@@ -338,7 +338,11 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
   // histogram launch and its counting pass
   int32_t* hist = reinterpret_cast<int32_t*>(base + ws.hist);
   int hist_tokens = 0;
-  const bool want_hist = need_permute && T > 0 && permute_takes_router_hist(T, k);
+  // with few slots, the fused kernel and its first half find their rows themselves, and nobody needs the permutation
+  const bool may_scan = (a == BIBO_ALGO_FUSED || a == kAlgoFusedWide || a == kAlgoSplit) && T > 0 &&
+                        (long long)T * k <= (a == kAlgoFusedWide ? kScanSlots / 2 : kScanSlots) && counts_out == nullptr &&
+                        state == nullptr && aligned16(x) && aligned16(w_gate_up) && aligned16(w_down);
+  const bool want_hist = may_scan || (need_permute && T > 0 && permute_takes_router_hist(T, k));
   if (T > 0 && norm_src != nullptr) {
     rc = hip_rc(launch_router_norm(norm_src, norm_weight, eps, w_router, bias, T, H, E, k, norm_mode, const_cast<void*>(x),
                                    logits_out, idx, w, want_hist ? hist : nullptr, &hist_tokens, s));
@@ -346,8 +350,17 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
   } else if (T > 0 && (rc = hip_rc(launch_router(x, w_router, bias, T, H, E, k, dtype, norm_mode, logits_out, idx, w, nullptr,
                                                  want_hist ? hist : nullptr, &hist_tokens, s))) != BIBO_OK)
     return rc;
-  if (need_permute) {
-    const hipError_t e = (want_hist && hist_tokens > 0)
+  ScanArgs scan;
+  if (may_scan && hist_tokens == 16) {
+    scan.idx = idx;
+    scan.hist = hist;
+    scan.nhist = (T + 15) / 16;
+    scan.S = T * k;
+    scan.k = k;
+    scan.perm_slot = perm_slot;
+    scan.offsets = offsets;
+  } else if (need_permute) {
+    const hipError_t e = (want_hist && hist_tokens > 0 && permute_takes_router_hist(T, k))
                              ? launch_permute_from_hist(idx, T, E, k, hist, hist_tokens, counts, offsets, perm_slot,
                                                         perm_token, s)
                              : launch_permute(idx, T, E, k, counts, offsets, perm_slot, perm_token, hist, s);
@@ -355,7 +368,7 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
   }
   if (T == 0) return BIBO_OK;
   return experts_dispatch(x, w_gate_up, w_down, theta, idx, w, offsets, perm_slot, perm_token, residual, true, T, H, Eg,
-                          sh->n_pos, sh->n_neg, k, I, dtype, a, sh->act, sh->flags, out, base, ws, workspace_bytes, s, preact);
+                          sh->n_pos, sh->n_neg, k, I, dtype, a, sh->act, sh->flags, out, base, ws, workspace_bytes, s, preact, scan);
 }
 
 

@@ -238,17 +238,29 @@ hipError_t launch_gateup_mfma(const void* x, const void* wgu, const float* theta
 hipError_t launch_down_mfma(const void* hidden, const void* wd, const float* w, const int32_t* offsets,
                             const int32_t* perm_slot, int T, int H, int E, int k, int I, void* yw, hipStream_t s);
 
+// For a call that fills one round of the fused kernel's tiles at most (half of it on average: kScanSlots of 128-row tiles, half as many of
+// 64) and needs no permutation otherwise: the workgroups find their rows in the routing itself.  hist: the router's histograms, one per 16
+// tokens.  perm_slot, offsets: left behind by launch_gateup_raw for launch_down_act.
+constexpr int kScanSlots = 16384;
+struct ScanArgs {
+  const int32_t* idx = nullptr;
+  const int32_t* hist = nullptr;
+  int nhist = 0, S = 0, k = 0;
+  int32_t* perm_slot = nullptr;
+  int32_t* offsets = nullptr;
+};
 bool fused_supported(int H, int I, int dtype);
 bool fused_wide_supported(int H, int I, int dtype);
 hipError_t launch_gateup_raw(const void* x, const void* wgu, const int32_t* offsets, const int32_t* perm_token, int T, int H,
-                             int E, int k, int I, void* gu, bool split, bool f32, hipStream_t s);
+                             int E, int k, int I, void* gu, bool split, bool f32, hipStream_t s, const ScanArgs& scan = ScanArgs());
 // whether a tile's columns are cut over several workgroups (launch_gateup_raw + launch_down_act instead of the fused kernel)
 bool split_columns(int S, int E, int H, int I);
 hipError_t launch_down_act(const void* gu, const void* wd, const float* theta, const float* w, const int32_t* offsets,
                            const int32_t* perm_slot, int S, int H, int E, int I, int act, void* yw, void* preact, hipStream_t s);
 hipError_t launch_experts_fused(const void* x, const void* wgu, const void* wd, const float* theta, const float* w,
                                 const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int T,
-                                int H, int E, int k, int I, int act, void* yw, void* preact, hipStream_t s);
+                                int H, int E, int k, int I, int act, void* yw, void* preact, hipStream_t s,
+                                const ScanArgs& scan = ScanArgs());
 bool stream_supported(int H, int I, int dtype);
 hipError_t launch_gateup_stream(const void* x, const void* wgu, const int32_t* idx, int T, int H, int E, int k, int I,
                                 void* gu, hipStream_t s);

@@ -243,7 +243,14 @@ __device__ __forceinline__ void down_block(Slice slice, WBlock<CT> (&wb)[NB], co
 // also leaves those pre-activations for its backward, in the same way (8-byte stores straight from the accumulator
 // registers during phase 2 were slower: 140 against 133 us at T = 8192).  MODE 3: as MODE 1, but the fp32 sums as they are, for
 // down_act_kernel (`preact` points to floats): 16-byte stores from the accumulators, a row's 128 bytes in four of them.
-template <int NT, int CT, int MODE = 0, int MTP = 2>
+// SCAN (slots a thread looks at): no permutation has run.  A workgroup adds up the router's histograms for the tile map and looks through
+// all selections for its tile's rows, a wave 64 slots in a row at a time, in slot order as the permutation has them.  Reading offsets and
+// rows of a permutation takes two memory latencies too, and the launch in front of it is saved: 0.4 to 1.5 us more here (0.11 a slot of a
+// thread) against 3.0 to 5.9 of permuting and the gap between two launches.  Kernels of a layer, permutation -> this, us: H = 512,
+// I = 256, k = 6: 30.8 -> 27.5 (T = 256), 33.0 -> 29.1 (800), 38.3 -> 37.0 (2000); H = 768, I = 384: 49.9 -> 47.4, 57.3 -> 54.7,
+// 61.1 -> 60.7; nine experts, k = 2: 31.8 -> 26.5, 30.2 -> 26.6, 32.1 -> 28.4.  Beyond one round of tiles a CU would look twice: level at
+// 16,000 slots of H = 1024, I = 512.
+template <int NT, int CT, int MODE = 0, int MTP = 2, int SCAN = 0>
 __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ wgu,
                                                             const bf16_t* __restrict__ wd,
                                                             const float* __restrict__ theta,
@@ -252,7 +259,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
                                                             const int32_t* __restrict__ perm_slot,
                                                             const int32_t* __restrict__ perm_token, int H, int E,
                                                             int act, unsigned x_bytes, bf16_t* __restrict__ yw,
-                                                            bf16_t* __restrict__ preact, int column_blocks) {
+                                                            bf16_t* __restrict__ preact, int column_blocks, ScanArgs scan) {
   using FT = FusedShape<NT, CT, MTP>;
   constexpr int BM = FT::BM, I = FT::I, BK = FT::BK;
   // Every buffer that is read while LDS-DMA fills another is a variable of its own: the compiler orders a DMA
@@ -270,8 +277,46 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
   // MODE 1 and 3 may cut a tile's columns over several workgroups (the others need whole rows): workgroup cb of a tile then
   // owns gate columns [cb I, cb I + I) of a row of row_i = column_blocks I and the up columns behind the same gate columns.
   const int ncb = MODE == 1 || MODE == 3 ? column_blocks : 1, row_i = I * ncb;
-  const TileMap tm = MODE == 3 || ncb > 1 ? make_tile_map(offsets, E, BM) : make_round_tile_map<BM>(offsets, E);
+  __shared__ int found[SCAN ? 8 * kWave : 1];
+  int picked[SCAN ? SCAN : 1];                       // selections of this wave's slots, 64 in a row a time
+  const int scan_per = SCAN ? (scan.S + 511) >> 9 : 0;
+  int scan_first = 0;
+  TileMap tm;
+  if constexpr (SCAN > 0) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    scan_first = wave * scan_per * kWave;
+#pragma unroll
+    for (int q = 0; q < SCAN; ++q) picked[q] = scan.idx[min(scan_first + q * kWave + lane, scan.S - 1)];
+    int n = 0;
+    for (int c0 = 0; c0 < scan.nhist; c0 += 64) {
+      int v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = scan.hist[min(c0 + wave + 8 * u, scan.nhist - 1) * kMaxE + lane];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) n += c0 + wave + 8 * u < scan.nhist ? v[u] : 0;
+    }
+#pragma unroll
+    for (int q = 0; q < SCAN; ++q)
+      if (q >= scan_per || scan_first + q * kWave + lane >= scan.S) picked[q] = -1;
+    found[wave * kWave + lane] = n;
+    __syncthreads();
+    n = 0;
+#pragma unroll
+    for (int v = 0; v < 8; ++v) n += found[v * kWave + lane];
+    tm.n = lane < E ? n : 0;
+    tm.lo = wave_inclusive_scan(tm.n) - tm.n;
+  } else {
+    tm = load_tile_map(offsets, E);
+  }
+  if (MODE == 3 || ncb > 1) count_tiles(tm, BM);
+  else count_round_tiles<BM>(tm);
   const int flat = xcd_tile(blockIdx.x, tm.total * ncb);
+  if constexpr (SCAN > 0 && MODE == 3) {
+    if (blockIdx.x == 0 && threadIdx.x < (unsigned)E) {   // (also where every slot went to an expert that has no weights)
+      scan.offsets[threadIdx.x] = tm.lo;
+      if (threadIdx.x == (unsigned)E - 1) scan.offsets[E] = tm.lo + tm.n;
+    }
+  }
   if (flat >= tm.total * ncb) return;
   const int tile = flat / ncb, cb = flat - tile * ncb;
   int e, row0, rows, tile_e;                            // the same for every lane, in scalar registers
@@ -283,6 +328,30 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
   // 2049, 292 -> 287 at 6000, 370 -> 355 at 8192.  At I = 256 it is within 2 us either way; so is walking w_down's blocks like this, but at
   // I = 512 (145 -> 155 us at T = 2049).
   const int rot = NT >= 3 ? tile_e % NT : 0;
+  if constexpr (SCAN > 0) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int count = 0;
+#pragma unroll
+    for (int q = 0; q < SCAN; ++q) count += __popcll(__ballot(picked[q] == e));
+    __syncthreads();                                     // the histograms' sums have been read
+    if (lane == 0) found[wave] = count;
+    if (tid < BM) slot_s[tid] = 0;
+    __syncthreads();
+    int r0 = -tile_e * tm.height;
+#pragma unroll
+    for (int v = 0; v < 7; ++v) r0 += v < wave ? found[v] : 0;
+#pragma unroll
+    for (int q = 0; q < SCAN; ++q) {
+      const unsigned long long mine = __ballot(picked[q] == e);
+      const int r = r0 + __builtin_amdgcn_mbcnt_hi((unsigned)(mine >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mine, 0));
+      if (picked[q] == e && r >= 0 && r < rows) slot_s[r] = scan_first + q * kWave + lane;
+      r0 += __popcll(mine);
+    }
+    __syncthreads();
+    if constexpr (MODE == 3) {
+      if (cb == 0 && tid < rows) scan.perm_slot[row0 + tid] = slot_s[tid];
+    }
+  }
   const int nblocks = (rows + 31) >> 5;                 // 32-row blocks that hold rows: 1 .. 2 MTP
 
   // The rest of the kernel exists once per number of blocks, chosen here, where nothing is alive yet: the copies
@@ -329,7 +398,8 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
 #pragma unroll
     for (int a = 0; a < F::kAInstr; ++a) {
       const int m = min(a * 64 + drow, rows - 1);                                // rows past the end re-read the last valid row
-      ld.a_voff[a] = (unsigned)perm_token[row0 + m] * hb + chunk * 16;          // gather, moe.py:81
+      const int token = SCAN ? slot_s[m] / scan.k : perm_token[row0 + m];
+      ld.a_voff[a] = (unsigned)token * hb + chunk * 16;                          // gather, moe.py:81
     }
     const int pos0 = ((lane >> 5) ^ ((n >> 1) & 7)) * 8;    // fragment side: lane (n, h) reads logical granule 2*ss + h of rows congruent to n mod 32
     auto frag_row = [&](int j) { return (wn * 2 + j) * 32; };
@@ -550,8 +620,8 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
     const float p = radial_exponent(theta, e, act);                                   // moe.py:89
     const float ms = ((ssq[tid] + ssq[BM + tid]) + ssq[2 * BM + tid]) + ssq[3 * BM + tid];
     radial_row_scalars(ms, I, p, act, rinv_s[tid], gain_s[tid]);                      // 1/r and r^p, moe.py:88-89
-    const int slot = perm_slot[row0 + min(tid, rows - 1)];
-    slot_s[tid] = slot;
+    const int slot = SCAN ? slot_s[min(tid, rows - 1)] : perm_slot[row0 + min(tid, rows - 1)];
+    if constexpr (SCAN == 0) slot_s[tid] = slot;
     w_s[tid] = w[slot];
   }
   __syncthreads();
@@ -746,29 +816,44 @@ void launch_down_act_nt(const float* gu, const bf16_t* wd, const float* theta, c
   if (two) launch(integral_constant<int, 1>{}, integral_constant<int, 2>{}); else launch(integral_constant<int, 1>{}, integral_constant<int, 1>{});
 }
 
+// slots a thread of a SCAN kernel looks at, 512 threads
+template <typename Launch>
+void scan_variant(int S, Launch launch) {
+  if (S <= 8 * 512) launch(std::integral_constant<int, 8>());
+  else if (S <= 16 * 512) launch(std::integral_constant<int, 16>());
+  else launch(std::integral_constant<int, 32>());
+}
+
 template <int NT, int CT, int MT>
 void launch_fused_t(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const float* theta, const float* w,
                     const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int S, int H, int E,
-                    int act, unsigned x_bytes, bf16_t* yw, bf16_t* preact, hipStream_t s) {
+                    int act, unsigned x_bytes, bf16_t* yw, bf16_t* preact, const ScanArgs& scan, hipStream_t s) {
   const int grid = round_tiles_most(S, E, 64 * MT);
   if constexpr (NT < 4) {                    // (a state-keeping forward has I <= 384)
     if (preact != nullptr) {
       hipLaunchKernelGGL((experts_fused_kernel<NT, CT, 2, MT>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta, w, offsets,
-                         perm_slot, perm_token, H, E, act, x_bytes, yw, preact, 1);
+                         perm_slot, perm_token, H, E, act, x_bytes, yw, preact, 1, scan);
       return;
     }
   }
+  if (scan.idx != nullptr) {
+    scan_variant(S, [&](auto per) {
+      hipLaunchKernelGGL((experts_fused_kernel<NT, CT, 0, MT, decltype(per)::value>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta, w,
+                         nullptr, nullptr, nullptr, H, E, act, x_bytes, yw, nullptr, 1, scan);
+    });
+    return;
+  }
   hipLaunchKernelGGL((experts_fused_kernel<NT, CT, 0, MT>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta, w, offsets, perm_slot,
-                     perm_token, H, E, act, x_bytes, yw, nullptr, 1);
+                     perm_token, H, E, act, x_bytes, yw, nullptr, 1, scan);
 }
 
 template <int NT>
 void launch_fused_nt(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const float* theta, const float* w,
                      const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int S, int H, int E,
-                     int act, unsigned x_bytes, bf16_t* yw, bf16_t* preact, hipStream_t s) {
+                     int act, unsigned x_bytes, bf16_t* yw, bf16_t* preact, const ScanArgs& scan, hipStream_t s) {
   constexpr int MT = NT == 4 ? 1 : 2;
   auto launch = [&](auto ct) {
-    launch_fused_t<NT, decltype(ct)::value, MT>(x, wgu, wd, theta, w, offsets, perm_slot, perm_token, S, H, E, act, x_bytes, yw, preact, s);
+    launch_fused_t<NT, decltype(ct)::value, MT>(x, wgu, wd, theta, w, offsets, perm_slot, perm_token, S, H, E, act, x_bytes, yw, preact, scan, s);
   };
   // (blocks of 256 columns leave room for the third x buffer of the deeper ring where I is not 384)
   if constexpr (NT != 4) {
@@ -783,12 +868,21 @@ void launch_fused_nt(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const
 
 template <int NT, int MODE = 1>
 void launch_raw_nt(const bf16_t* x, const bf16_t* wgu, const int32_t* offsets, const int32_t* perm_token, int S, int H, int E,
-                   unsigned x_bytes, bf16_t* gu, int column_blocks, hipStream_t s) {
+                   unsigned x_bytes, bf16_t* gu, int column_blocks, hipStream_t s, const ScanArgs& scan = ScanArgs()) {
   constexpr int MT = NT == 4 ? 1 : 2;
   const int tiles = S / (64 * MT) + E < S ? S / (64 * MT) + E : S;
   const int grid = MODE == 3 || column_blocks > 1 ? ((tiles * column_blocks + 7) & ~7) + 8 : round_tiles_most(S, E, 64 * MT);
+  if constexpr (MODE == 3) {
+    if (scan.idx != nullptr) {
+      scan_variant(S, [&](auto per) {
+        hipLaunchKernelGGL((experts_fused_kernel<NT, 1, MODE, MT, decltype(per)::value>), dim3(grid), dim3(512), 0, s, x, wgu, nullptr,
+                           nullptr, nullptr, nullptr, nullptr, nullptr, H, E, 0, x_bytes, nullptr, gu, column_blocks, scan);
+      });
+      return;
+    }
+  }
   hipLaunchKernelGGL((experts_fused_kernel<NT, 1, MODE, MT>), dim3(grid), dim3(512), 0, s, x, wgu, nullptr, nullptr, nullptr,
-                     offsets, nullptr, perm_token, H, E, 0, x_bytes, nullptr, gu, column_blocks);
+                     offsets, nullptr, perm_token, H, E, 0, x_bytes, nullptr, gu, column_blocks, scan);
 }
 
 }  // namespace
@@ -797,7 +891,7 @@ void launch_raw_nt(const bf16_t* x, const bf16_t* wgu, const int32_t* offsets, c
 // pass recomputes, moe.py:84).  Same shapes as launch_experts_fused.
 // `split`: one workgroup per 128 gate (and up) columns of a tile, for calls with fewer tiles than CUs.
 hipError_t launch_gateup_raw(const void* x, const void* wgu, const int32_t* offsets, const int32_t* perm_token, int T, int H,
-                             int E, int k, int I, void* gu, bool split, bool f32, hipStream_t s) {
+                             int E, int k, int I, void* gu, bool split, bool f32, hipStream_t s, const ScanArgs& scan) {
   const int S = T * k;
   if (S == 0) return hipSuccess;
   if ((unsigned long long)T * H * sizeof(bf16_t) >= (1ull << 32)) return hipErrorInvalidValue;
@@ -805,9 +899,9 @@ hipError_t launch_gateup_raw(const void* x, const void* wgu, const int32_t* offs
   const bf16_t* xp = static_cast<const bf16_t*>(x);
   const bf16_t* gp = static_cast<const bf16_t*>(wgu);
   bf16_t* out = static_cast<bf16_t*>(gu);
-  if (f32 && !split) return hipErrorInvalidValue;
+  if ((f32 && !split) || (scan.idx != nullptr && !f32)) return hipErrorInvalidValue;
   if (f32) {
-    launch_raw_nt<1, 3>(xp, gp, offsets, perm_token, S, H, E, xb, out, I / 128, s);
+    launch_raw_nt<1, 3>(xp, gp, offsets, perm_token, S, H, E, xb, out, I / 128, s, scan);
     return hipGetLastError();
   }
   if (split) {
@@ -871,11 +965,11 @@ bool fused_wide_supported(int H, int I, int dtype) { return dtype == BIBO_DTYPE_
 
 hipError_t launch_experts_fused(const void* x, const void* wgu, const void* wd, const float* theta, const float* w,
                                 const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int T,
-                                int H, int E, int k, int I, int act, void* yw, void* preact, hipStream_t s) {
+                                int H, int E, int k, int I, int act, void* yw, void* preact, hipStream_t s, const ScanArgs& scan) {
   const int S = T * k;
   if (S == 0) return hipSuccess;
   if ((unsigned long long)T * H * sizeof(bf16_t) >= (1ull << 32)) return hipErrorInvalidValue;   // 32-bit byte offsets into x
-  if (I == 512 && preact != nullptr) return hipErrorInvalidValue;
+  if ((I == 512 || scan.idx != nullptr) && preact != nullptr) return hipErrorInvalidValue;
   const unsigned xb = (unsigned)((size_t)T * H * sizeof(bf16_t));
   const bf16_t* xp = static_cast<const bf16_t*>(x);
   const bf16_t* gp = static_cast<const bf16_t*>(wgu);
@@ -883,10 +977,10 @@ hipError_t launch_experts_fused(const void* x, const void* wgu, const void* wd, 
   bf16_t* yp = static_cast<bf16_t*>(yw);
   bf16_t* pp = static_cast<bf16_t*>(preact);
   switch (I) {
-    case 128: launch_fused_nt<1>(xp, gp, dp, theta, w, offsets, perm_slot, perm_token, S, H, E, act, xb, yp, pp, s); break;
-    case 256: launch_fused_nt<2>(xp, gp, dp, theta, w, offsets, perm_slot, perm_token, S, H, E, act, xb, yp, pp, s); break;
-    case 384: launch_fused_nt<3>(xp, gp, dp, theta, w, offsets, perm_slot, perm_token, S, H, E, act, xb, yp, pp, s); break;
-    case 512: launch_fused_nt<4>(xp, gp, dp, theta, w, offsets, perm_slot, perm_token, S, H, E, act, xb, yp, pp, s); break;
+    case 128: launch_fused_nt<1>(xp, gp, dp, theta, w, offsets, perm_slot, perm_token, S, H, E, act, xb, yp, pp, scan, s); break;
+    case 256: launch_fused_nt<2>(xp, gp, dp, theta, w, offsets, perm_slot, perm_token, S, H, E, act, xb, yp, pp, scan, s); break;
+    case 384: launch_fused_nt<3>(xp, gp, dp, theta, w, offsets, perm_slot, perm_token, S, H, E, act, xb, yp, pp, scan, s); break;
+    case 512: launch_fused_nt<4>(xp, gp, dp, theta, w, offsets, perm_slot, perm_token, S, H, E, act, xb, yp, pp, scan, s); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

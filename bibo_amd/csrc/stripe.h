@@ -51,21 +51,19 @@ __device__ __forceinline__ TileMap make_tile_map(const int32_t* __restrict__ off
 // 2049: 57 -> 45, 3001: 57 -> 50, 6000: 106 -> 88.
 constexpr int kCUs = 256, kBlockRows = 32;
 template <int BM>
-__device__ __forceinline__ TileMap make_round_tile_map(const int32_t* __restrict__ offsets, int E) {
+__device__ __forceinline__ void count_round_tiles(TileMap& tm) {
   static_assert(BM == 64 || BM == 128, "two or four blocks");
-  TileMap tm = load_tile_map(offsets, E);
   count_tiles(tm, BM);
   const int room = (int)((unsigned)(tm.total + kCUs - 1) / kCUs * kCUs);
   count_tiles(tm, kBlockRows);
-  if (tm.total <= room) return tm;
+  if (tm.total <= room) return;
   if constexpr (BM == 128) {
     count_tiles(tm, 2 * kBlockRows);
-    if (tm.total <= room) return tm;
+    if (tm.total <= room) return;
     count_tiles(tm, 3 * kBlockRows);
-    if (tm.total <= room) return tm;
+    if (tm.total <= room) return;
   }
   count_tiles(tm, BM);
-  return tm;
 }
 // What such a map can come to, for the grid: the rounds that tiles of BM rows are sure to fit, or every tile at its lowest.
 inline int round_tiles_most(int S, int E, int BM) {
