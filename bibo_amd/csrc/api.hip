@@ -338,10 +338,10 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
   // histogram launch and its counting pass
   int32_t* hist = reinterpret_cast<int32_t*>(base + ws.hist);
   int hist_tokens = 0;
-  // with few slots, the fused kernel and its first half find their rows themselves, and nobody needs the permutation
+  // with few slots, the fused kernel and its first half find their rows themselves; of a permutation they leave what a backward pass reads
   const bool may_scan = (a == BIBO_ALGO_FUSED || a == kAlgoFusedWide || a == kAlgoSplit) && T > 0 &&
-                        (long long)T * k <= (a == kAlgoFusedWide ? kScanSlots / 2 : kScanSlots) && counts_out == nullptr &&
-                        state == nullptr && aligned16(x) && aligned16(w_gate_up) && aligned16(w_down);
+                        (long long)T * k <= (a == BIBO_ALGO_FUSED ? kScanSlots : kScanSlots / 2) &&
+                        (state != nullptr ? Eg == E : counts_out == nullptr) && aligned16(x) && aligned16(w_gate_up) && aligned16(w_down);
   const bool want_hist = may_scan || (need_permute && T > 0 && permute_takes_router_hist(T, k));
   if (T > 0 && norm_src != nullptr) {
     rc = hip_rc(launch_router_norm(norm_src, norm_weight, eps, w_router, bias, T, H, E, k, norm_mode, const_cast<void*>(x),
@@ -359,6 +359,10 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
     scan.k = k;
     scan.perm_slot = perm_slot;
     scan.offsets = offsets;
+    if (state != nullptr) {
+      scan.perm_token = perm_token;
+      scan.counts = counts;
+    }
   } else if (need_permute) {
     const hipError_t e = (want_hist && hist_tokens > 0 && permute_takes_router_hist(T, k))
                              ? launch_permute_from_hist(idx, T, E, k, hist, hist_tokens, counts, offsets, perm_slot,

@@ -240,14 +240,17 @@ hipError_t launch_down_mfma(const void* hidden, const void* wd, const float* w, 
 
 // For a call that fills one round of the fused kernel's tiles at most (half of it on average: kScanSlots of 128-row tiles, half as many of
 // 64) and needs no permutation otherwise: the workgroups find their rows in the routing itself.  hist: the router's histograms, one per 16
-// tokens.  perm_slot, offsets: left behind by launch_gateup_raw for launch_down_act.
+// tokens.  Left behind for who reads them later: perm_slot and offsets by launch_gateup_raw (for launch_down_act), those, perm_token and
+// counts by a training forward (its experts all have weights: nobody would place the slots of the others).
 constexpr int kScanSlots = 16384;
 struct ScanArgs {
   const int32_t* idx = nullptr;
   const int32_t* hist = nullptr;
   int nhist = 0, S = 0, k = 0;
   int32_t* perm_slot = nullptr;
+  int32_t* perm_token = nullptr;
   int32_t* offsets = nullptr;
+  int32_t* counts = nullptr;
 };
 bool fused_supported(int H, int I, int dtype);
 bool fused_wide_supported(int H, int I, int dtype);

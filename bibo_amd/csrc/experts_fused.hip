@@ -311,10 +311,11 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
   if (MODE == 3 || ncb > 1) count_tiles(tm, BM);
   else count_round_tiles<BM>(tm);
   const int flat = xcd_tile(blockIdx.x, tm.total * ncb);
-  if constexpr (SCAN > 0 && MODE == 3) {
+  if constexpr (SCAN > 0 && MODE >= 2) {
     if (blockIdx.x == 0 && threadIdx.x < (unsigned)E) {   // (also where every slot went to an expert that has no weights)
       scan.offsets[threadIdx.x] = tm.lo;
       if (threadIdx.x == (unsigned)E - 1) scan.offsets[E] = tm.lo + tm.n;
+      if (scan.counts != nullptr) scan.counts[threadIdx.x] = tm.n;
     }
   }
   if (flat >= tm.total * ncb) return;
@@ -348,8 +349,12 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
       r0 += __popcll(mine);
     }
     __syncthreads();
-    if constexpr (MODE == 3) {
-      if (cb == 0 && tid < rows) scan.perm_slot[row0 + tid] = slot_s[tid];
+    if constexpr (MODE >= 2) {
+      if (cb == 0 && tid < rows) {
+        const int slot = slot_s[tid];
+        scan.perm_slot[row0 + tid] = slot;
+        if (scan.perm_token != nullptr) scan.perm_token[row0 + tid] = slot / scan.k;
+      }
     }
   }
   const int nblocks = (rows + 31) >> 5;                 // 32-row blocks that hold rows: 1 .. 2 MTP
@@ -829,22 +834,25 @@ void launch_fused_t(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const 
                     const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int S, int H, int E,
                     int act, unsigned x_bytes, bf16_t* yw, bf16_t* preact, const ScanArgs& scan, hipStream_t s) {
   const int grid = round_tiles_most(S, E, 64 * MT);
+  auto launch = [&](auto mode) {
+    constexpr int MODE = decltype(mode)::value;
+    if (scan.idx != nullptr) {
+      scan_variant(S, [&](auto per) {
+        hipLaunchKernelGGL((experts_fused_kernel<NT, CT, MODE, MT, decltype(per)::value>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta,
+                           w, nullptr, nullptr, nullptr, H, E, act, x_bytes, yw, preact, 1, scan);
+      });
+      return;
+    }
+    hipLaunchKernelGGL((experts_fused_kernel<NT, CT, MODE, MT>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta, w, offsets, perm_slot,
+                       perm_token, H, E, act, x_bytes, yw, preact, 1, scan);
+  };
   if constexpr (NT < 4) {                    // (a state-keeping forward has I <= 384)
     if (preact != nullptr) {
-      hipLaunchKernelGGL((experts_fused_kernel<NT, CT, 2, MT>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta, w, offsets,
-                         perm_slot, perm_token, H, E, act, x_bytes, yw, preact, 1, scan);
+      launch(std::integral_constant<int, 2>());
       return;
     }
   }
-  if (scan.idx != nullptr) {
-    scan_variant(S, [&](auto per) {
-      hipLaunchKernelGGL((experts_fused_kernel<NT, CT, 0, MT, decltype(per)::value>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta, w,
-                         nullptr, nullptr, nullptr, H, E, act, x_bytes, yw, nullptr, 1, scan);
-    });
-    return;
-  }
-  hipLaunchKernelGGL((experts_fused_kernel<NT, CT, 0, MT>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta, w, offsets, perm_slot,
-                     perm_token, H, E, act, x_bytes, yw, nullptr, 1, scan);
+  launch(std::integral_constant<int, 0>());
 }
 
 template <int NT>
@@ -969,7 +977,7 @@ hipError_t launch_experts_fused(const void* x, const void* wgu, const void* wd, 
   const int S = T * k;
   if (S == 0) return hipSuccess;
   if ((unsigned long long)T * H * sizeof(bf16_t) >= (1ull << 32)) return hipErrorInvalidValue;   // 32-bit byte offsets into x
-  if ((I == 512 || scan.idx != nullptr) && preact != nullptr) return hipErrorInvalidValue;
+  if (I == 512 && preact != nullptr) return hipErrorInvalidValue;
   const unsigned xb = (unsigned)((size_t)T * H * sizeof(bf16_t));
   const bf16_t* xp = static_cast<const bf16_t*>(x);
   const bf16_t* gp = static_cast<const bf16_t*>(wgu);

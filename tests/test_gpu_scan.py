@@ -62,3 +62,25 @@ def test_nothing_but_identity_after_a_full_call():
     """The scratch memory of a call with rows must not pass for a permutation of one without."""
     _same(300, 768, 384, 62, 6)
     _same(300, 768, 384, 62, 2, pairs=1, hot=(62, 63))
+
+
+@pytest.mark.parametrize("T,k,E", [(1, 1, 5), (100, 8, 64), (513, 8, 64), (1024, 8, 64), (1025, 8, 64), (1111, 2, 9), (2730, 6, 64),
+                                   (2731, 6, 64)])
+@pytest.mark.parametrize("H,I", [(128, 128), (256, 256), (768, 384)])
+def test_training_state(H, I, T, k, E):
+    """The state that a training forward leaves serves the backward pass as a permutation does (moe_backward makes its own)."""
+    g = torch.Generator().manual_seed(T + I)
+    x, d_out = (torch.randn(T, H, generator=g).bfloat16().to(DEV) for _ in range(2))
+    wr = (torch.randn(E, H, generator=g) * 0.1).bfloat16().to(DEV)
+    bias = (torch.rand(E, generator=g) * 0.02 - 0.01).to(DEV)
+    gu = (torch.randn(E, 2 * I, H, generator=g) * 0.05).bfloat16().to(DEV)
+    dn = (torch.randn(E, H, I, generator=g) * 0.05).bfloat16().to(DEV)
+    th = torch.randn(E, generator=g).to(DEV)
+    _, idx, _, _, _ = ops.moe_forward(x, wr, bias, gu, dn, th, k, want_routing=True)
+    out, counts, state = ops.moe_forward_train(x, wr, bias, gu, dn, th, k, want_counts=True)
+    assert torch.equal(torch.bincount(idx.flatten().long(), minlength=E).int(), counts)
+    assert torch.equal(out, ops.moe_forward(x, wr, bias, gu, dn, th, k, algo="fused")[0])
+    saved = ops.moe_backward_saved(x, d_out, wr, gu, dn, th, k, state, want_dw=True)
+    again = ops.moe_backward(x, d_out, wr, bias, gu, dn, th, k, want_dw=True)
+    for a, b in zip(saved, again):
+        assert torch.equal(a, b)
