@@ -217,7 +217,7 @@ int experts_dispatch(const void* x, const void* wgu, const void* wd, const float
                      const float* w, const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token,
                      const void* residual, bool idx_trusted, int T, int H, int Eg, int np, int nn, int k, int I, int dtype,
                      int algo, int act, int flags, void* out, char* base, const Workspace& ws, size_t ws_bytes,
-                     hipStream_t s, void* preact = nullptr, const ScanArgs& scan = ScanArgs()) {
+                     hipStream_t s, void* preact = nullptr, const ScanArgs& scan = ScanArgs(), bool gate_up_done = false) {
   float* yw = reinterpret_cast<float*>(base + ws.yw);
   CombineArgs ca;
   ca.residual = residual;
@@ -228,7 +228,7 @@ int experts_dispatch(const void* x, const void* wgu, const void* wd, const float
   if (few_taken(algo, T, H, k, I, dtype, x, wgu, wd)) {
     ca.x = x; ca.n_pos = np; ca.n_neg = nn;
     return hip_rc(launch_experts_few(x, wgu, wd, theta, idx, w, ca, T, H, Eg, k, I, dtype, act, reinterpret_cast<float*>(base + ws.gu),
-                                     out, s));
+                                     out, gate_up_done, s));
   }
   if (algo == BIBO_ALGO_STREAM) {
     if (!aligned16(x) || !aligned16(wgu) || !aligned16(wd)) return BIBO_ERR_MISALIGNED;
@@ -332,12 +332,13 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
     preact = state + st.gu;
   }
   // the streaming and few-token kernels find their rows themselves; the permutation then only serves the counts
-  const bool need_permute = (a != BIBO_ALGO_STREAM && !few_taken(a, T, H, k, I, dtype, x, w_gate_up, w_down)) ||
-                            counts_out != nullptr || T == 0;
+  const bool few = few_taken(a, T, H, k, I, dtype, x, w_gate_up, w_down);
+  const bool need_permute = (a != BIBO_ALGO_STREAM && !few) || counts_out != nullptr || T == 0;
   // the router kernel can leave per-workgroup histograms of its selections, which save the permutation its
   // histogram launch and its counting pass
   int32_t* hist = reinterpret_cast<int32_t*>(base + ws.hist);
   int hist_tokens = 0;
+  bool gate_up_done = false;
   // with few slots, the fused kernel and its first half find their rows themselves; of a permutation they leave what a backward pass reads
   const bool may_scan = (a == BIBO_ALGO_FUSED || a == kAlgoFusedWide || a == kAlgoSplit) && T > 0 &&
                         (long long)T * k <= (a == BIBO_ALGO_FUSED ? kScanSlots : kScanSlots / 2) &&
@@ -347,6 +348,11 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
     rc = hip_rc(launch_router_norm(norm_src, norm_weight, eps, w_router, bias, T, H, E, k, norm_mode, const_cast<void*>(x),
                                    logits_out, idx, w, want_hist ? hist : nullptr, &hist_tokens, s));
     if (rc != BIBO_OK) return rc;
+  } else if (few && !want_hist && router_gateup_supported(T, H, k, I, dtype, x, w_router)) {
+    rc = hip_rc(launch_router_gateup(x, w_router, bias, T, H, E, k, norm_mode, logits_out, idx, w, w_gate_up, Eg, I,
+                                     reinterpret_cast<float*>(base + ws.gu), s));
+    if (rc != BIBO_OK) return rc;
+    gate_up_done = true;
   } else if (T > 0 && (rc = hip_rc(launch_router(x, w_router, bias, T, H, E, k, dtype, norm_mode, logits_out, idx, w, nullptr,
                                                  want_hist ? hist : nullptr, &hist_tokens, s))) != BIBO_OK)
     return rc;
@@ -372,7 +378,7 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
   }
   if (T == 0) return BIBO_OK;
   return experts_dispatch(x, w_gate_up, w_down, theta, idx, w, offsets, perm_slot, perm_token, residual, true, T, H, Eg,
-                          sh->n_pos, sh->n_neg, k, I, dtype, a, sh->act, sh->flags, out, base, ws, workspace_bytes, s, preact, scan);
+                          sh->n_pos, sh->n_neg, k, I, dtype, a, sh->act, sh->flags, out, base, ws, workspace_bytes, s, preact, scan, gate_up_done);
 }
 
 

@@ -10,62 +10,19 @@
 //                      one wave per slot of the token; +/-Identity slots add +/- w x   (moe.py:87-101)
 // Plain FMAs: a matrix instruction would use one of its sixteen columns.  Sixteen lanes share a weight row, 16 bytes (fp32:
 // 32) each at a time, i.e. whole 256-byte pieces of a row per request.
-#include "tile_f32.h"
+#include "few.h"
 
 namespace bibo {
 namespace {
 
-__device__ __forceinline__ void load8(float (&v)[8], const float* p) {
-  const floatx4 a = *reinterpret_cast<const floatx4*>(p), b = *reinterpret_cast<const floatx4*>(p + 4);
-#pragma unroll
-  for (int q = 0; q < 4; ++q) { v[q] = a[q]; v[4 + q] = b[q]; }
-}
-
-// eight weights as they come from memory
-template <typename T> struct Raw8;
-template <> struct Raw8<bf16_t> {
-  bf16x8 v;
-  __device__ __forceinline__ void load(const bf16_t* p) { v = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p)); }
-  __device__ __forceinline__ void zero() {
-#pragma unroll
-    for (int q = 0; q < 8; ++q) v[q] = (bf16_t)0.f;
-  }
-  __device__ __forceinline__ float get(int q) const { return (float)v[q]; }
-};
-template <> struct Raw8<float> {
-  floatx4 a, b;
-  __device__ __forceinline__ void load(const float* p) {
-    a = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(p));
-    b = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(p + 4));
-  }
-  __device__ __forceinline__ void zero() { a = b = floatx4{0.f, 0.f, 0.f, 0.f}; }
-  __device__ __forceinline__ float get(int q) const { return q < 4 ? a[q] : b[q - 4]; }
-};
-
-__device__ __forceinline__ float sum16(float v) {          // over the 16 lanes of a DPP row, the same in every lane
-  auto dpp = [](float x, auto ctrl) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, false));
-  };
-  v += dpp(v, std::integral_constant<int, 0xB1>{});
-  v += dpp(v, std::integral_constant<int, 0x4E>{});
-  v += dpp(v, std::integral_constant<int, 0x141>{});
-  return v + dpp(v, std::integral_constant<int, 0x140>{});
-}
-
-// the end of a dot product: the lanes' four partial sums each.  Sixty-four chains and a tree, as where a wave's lanes share a row
-// (experts_generic.hip): one chain per lane was 1.3 times as far from exact in fp32 at H = 768
-__device__ __forceinline__ float sum64(const float (&part)[4]) { return sum16((part[0] + part[1]) + (part[2] + part[3])); }
-
-constexpr int kGateRows = 32;           // weight rows per workgroup of the gate/up kernel: two per 16 lanes
-
-// grid (ceil(2I / 32), S).  NG = ceil(H / 128): 8-element granules of a row per lane.
+// grid (ceil(2I / 32), S)
 template <typename T, int NG>
 __global__ __launch_bounds__(256) void gateup_few_kernel(const T* __restrict__ x, const T* __restrict__ wgu,
                                                          const int32_t* __restrict__ idx, int k, int H, int I2, int E,
                                                          float* __restrict__ gu) {
   const int slot = blockIdx.y, c = threadIdx.x & 15, rg = threadIdx.x >> 4;
   const int e = idx[slot];
-  Raw8<T> xv[NG], wv[2][NG];
+  Raw8<T> xv[NG];
   const T* xr = x + (size_t)(slot / k) * H;
 #pragma unroll
   for (int u = 0; u < NG; ++u) {
@@ -73,26 +30,7 @@ __global__ __launch_bounds__(256) void gateup_few_kernel(const T* __restrict__ x
     if (g < H) xv[u].load(xr + g); else xv[u].zero();
   }
   if ((unsigned)e >= (unsigned)E) return;                      // no GLU expert
-  const int row0 = blockIdx.x * kGateRows + rg;
-#pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    const T* wr = wgu + ((size_t)e * I2 + min(row0 + 16 * r, I2 - 1)) * H;
-#pragma unroll
-    for (int u = 0; u < NG; ++u) {
-      const int g = (u * 16 + c) * 8;
-      if (g < H) wv[r][u].load(wr + g); else wv[r][u].zero();
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    float part[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int u = 0; u < NG; ++u)
-#pragma unroll
-      for (int q = 0; q < 8; ++q) part[q & 3] = fmaf(wv[r][u].get(q), xv[u].get(q), part[q & 3]);
-    const float acc = sum64(part);
-    if (c == 0 && row0 + 16 * r < I2) gu[(size_t)slot * I2 + row0 + 16 * r] = acc;
-  }
+  gateup_rows<T, NG>(xv, wgu + (size_t)e * I2 * H, blockIdx.x * kGateRows + rg, c, H, I2, gu + (size_t)slot * I2);
 }
 
 // grid (H / CH, T), 64 k threads: wave j = slot j of the token.  NG = ceil(I / 128).
@@ -188,16 +126,18 @@ __global__ __launch_bounds__(64 * kMaxK) void down_few_kernel(const float* __res
   }
 }
 
+// gate_up_done: launch_router_gateup has run
 template <typename T>
 hipError_t launch_t(const T* x, const T* wgu, const T* wd, const float* theta, const int32_t* idx, const float* w,
-                    const CombineArgs& a, int Tn, int H, int E, int k, int I, int act, float* gu, T* out, hipStream_t s) {
+                    const CombineArgs& a, int Tn, int H, int E, int k, int I, int act, float* gu, T* out, bool gate_up_done, hipStream_t s) {
   auto gateup = [&](auto ng) {
     hipLaunchKernelGGL((gateup_few_kernel<T, decltype(ng)::value>), dim3((2 * I + kGateRows - 1) / kGateRows, Tn * k), dim3(256), 0, s, x,
                        wgu, idx, k, H, 2 * I, E, gu);
   };
   using std::integral_constant;
   const int nh = (H + 127) / 128;
-  if (nh <= 2) gateup(integral_constant<int, 2>{});
+  if (gate_up_done) {
+  } else if (nh <= 2) gateup(integral_constant<int, 2>{});
   else if (nh <= 4) gateup(integral_constant<int, 4>{});
   else if (nh <= 6) gateup(integral_constant<int, 6>{});
   else gateup(integral_constant<int, 8>{});
@@ -221,12 +161,12 @@ bool few_supported(int T, int H, int k, int I) {
 
 hipError_t launch_experts_few(const void* x, const void* wgu, const void* wd, const float* theta, const int32_t* idx, const float* w,
                               const CombineArgs& a, int T, int H, int E, int k, int I, int dtype, int act, float* gu, void* out,
-                              hipStream_t s) {
+                              bool gate_up_done, hipStream_t s) {
   if (dtype == BIBO_DTYPE_BF16)
     return launch_t(static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(wgu), static_cast<const bf16_t*>(wd), theta, idx, w, a, T,
-                    H, E, k, I, act, gu, static_cast<bf16_t*>(out), s);
+                    H, E, k, I, act, gu, static_cast<bf16_t*>(out), gate_up_done, s);
   return launch_t(static_cast<const float*>(x), static_cast<const float*>(wgu), static_cast<const float*>(wd), theta, idx, w, a, T, H, E,
-                  k, I, act, gu, static_cast<float*>(out), s);
+                  k, I, act, gu, static_cast<float*>(out), gate_up_done, s);
 }
 
 }  // namespace bibo

@@ -1,7 +1,7 @@
 // Kernel 1: fused router.  fp32 logits x @ w_router^T, canonical sigmoid, selection on score + bias
 // (ties to the lowest expert index), gather of the unbiased scores, normalisation.
 // Follows BiBoMoERouter.forward, src/modeling/ffn/router.py:25-51 of the reference.
-#include "tile_f32.h"
+#include "few.h"
 
 namespace bibo {
 namespace {
@@ -397,6 +397,70 @@ __global__ __launch_bounds__(256) void router_ring_kernel(const bf16_t* __restri
   router_finish<TOK>(acc, sc, bias_s, T, E, k, norm_mode, t0, logits, idx, w, gap, chunk_hist);
 }
 
+// A token's routing with the first pass of its experts behind it, for the few-token kernels: every workgroup works out the routing of its
+// slot's token for itself and goes on to blocks of 32 rows of the slot's gate/up weights.  All of w_router (98 KB at E = 64, H = 768) comes
+// from L2 to each workgroup at once, every request on its way before the first wait, and a launch and the gap behind it are saved.  One
+// workgroup a CU at most (the LDS holds w_router), so with more slots each takes more blocks.  Kernels of a layer, router + gate/up launch
+// -> this, weights from HBM, us: H = 768, I = 384, k = 6: 16.7 -> 14.7 (T = 1), 21.1 -> 19.4 (4), 26.5 -> 25.8 (8); H = 512, I = 256:
+// 13.3 -> 10.6 (1), 18.1 -> 17.7 (8); H = 1024, I = 512, k = 8: 22.0 -> 17.4 (1), 30.8 -> 26.0 (4).  The host is through sooner too: the
+// layer of one token at H = 768 takes 12.2 us instead of 15.6.  Same products in the same order as router_mfma_kernel and
+// gateup_few_kernel.  Grid (blocks of rows shared out, T k); NG = H / 128.
+template <int NG>
+__global__ __launch_bounds__(256) void router_gateup_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ wr,
+                                                            const float* __restrict__ bias, int Et, int k, int norm_mode,
+                                                            float* __restrict__ logits, int32_t* __restrict__ idx,
+                                                            float* __restrict__ w, const bf16_t* __restrict__ wgu, int E, int I2,
+                                                            float* __restrict__ gu) {
+  constexpr int H = NG * kRouterKC, kGran = H / 8;
+  __shared__ __attribute__((aligned(16))) bf16_t ws[kMaxE * H];
+  __shared__ __attribute__((aligned(16))) bf16_t xs[H];
+  __shared__ float sc[16 * kRowPad];
+  __shared__ float bias_s[kMaxE];
+  __shared__ int32_t idx_s[kMaxK];
+  __shared__ float w_s[kMaxK];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int slot = blockIdx.y, t = slot / k, j = slot - t * k;
+  const bf16_t* xr = x + (size_t)t * H;
+  // chunk-major stages as in router_mfma_kernel: granule c of a row sits at position c ^ (row & 15)
+#pragma unroll
+  for (int c = 0; c < NG; ++c)
+#pragma unroll
+    for (int i = 0; i < kMaxE / 16; ++i) {
+      const int row = i * 16 + (tid >> 4), g = (tid & 15) ^ (row & 15);
+      __builtin_amdgcn_global_load_lds((router_gbl_void*)(wr + (size_t)min(row, Et - 1) * H + c * kRouterKC + g * 8),
+                                       (router_lds_void*)(ws + ((c * kMaxE + i * 16) * 16 + wave * 64) * 8), 16, 0, 0);
+    }
+  const int c16 = tid & 15, rg = tid >> 4;
+  Raw8<bf16_t> xv[NG];
+#pragma unroll
+  for (int u = 0; u < NG; ++u) xv[u].load(xr + (u * 16 + c16) * 8);
+  if (tid < kGran) *reinterpret_cast<bf16x8*>(xs + tid * 8) = *reinterpret_cast<const bf16x8*>(xr + tid * 8);
+  if (tid < kMaxE) bias_s[tid] = tid < Et ? bias[tid] : 0.f;
+  __syncthreads();
+  const int r16 = lane & 15, kc = lane >> 4;
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < NG; ++c)
+#pragma unroll
+    for (int s = 0; s < kRouterKC / 32; ++s) {
+      const bf16x8 a = *reinterpret_cast<const bf16x8*>(xs + c * kRouterKC + (s * 4 + kc) * 8);    // sixteen times the token's row
+      const bf16x8 b = *reinterpret_cast<const bf16x8*>(ws + (c * kMaxE + wave * 16 + r16) * kRouterKC + ((s * 4 + kc) ^ r16) * 8);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
+    }
+  const bool first = blockIdx.x == 0 && j == 0;
+  router_finish<16>(acc, sc, bias_s, 1, Et, k, norm_mode, 0, first && logits != nullptr ? logits + (size_t)t * Et : nullptr, idx_s, w_s,
+                    nullptr, nullptr);
+  __syncthreads();
+  if (first && tid < k) {
+    idx[(size_t)t * k + tid] = idx_s[tid];
+    w[(size_t)t * k + tid] = w_s[tid];
+  }
+  const int e = __builtin_amdgcn_readfirstlane(idx_s[j]);
+  if ((unsigned)e >= (unsigned)E) return;                      // no GLU expert
+  for (int row = blockIdx.x * kGateRows; row < I2; row += gridDim.x * kGateRows)
+    gateup_rows<bf16_t, NG>(xv, wgu + (size_t)e * I2 * H, row + rg, c16, H, I2, gu + (size_t)slot * I2);
+}
+
 // ---- MFMA router with the block's input RMSNorm in front (the caller's seam) ----------------------
 // out = h + moe(post_attention_layernorm(h)) (src/modeling/layers.py:57-64) needs the normalised rows twice: as the
 // router's operand and as the rows the expert kernels gather.  This kernel reads the raw rows once: all H elements of
@@ -629,6 +693,34 @@ hipError_t launch_router_norm(const void* h, Vec norm_weight, float eps, const v
   if (e != hipSuccess) return e;
   if (hist_tokens != nullptr && chunk_hist != nullptr) *hist_tokens = T >= 32 * 256 ? 32 : 16;
   return hipSuccess;
+}
+
+bool router_gateup_supported(int T, int H, int k, int I, int dtype, const void* x, const void* w_router) {
+  return dtype == BIBO_DTYPE_BF16 && H % kRouterKC == 0 && H <= 8 * kRouterKC && T >= 1 &&
+         ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w_router)) & 15) == 0;
+}
+
+hipError_t launch_router_gateup(const void* x, const void* w_router, const float* bias, int T, int H, int Et, int k, int norm_mode,
+                                float* logits, int32_t* idx, float* w, const void* wgu, int E, int I, float* gu, hipStream_t s) {
+  const int blocks = (2 * I + kGateRows - 1) / kGateRows, most = kCUs / (T * k), each = (blocks + most - 1) / most;
+  auto launch = [&](auto ng) {
+    hipLaunchKernelGGL((router_gateup_kernel<decltype(ng)::value>), dim3((blocks + each - 1) / each, T * k), dim3(256), 0, s,
+                       static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w_router), bias, Et, k, norm_mode, logits, idx, w,
+                       static_cast<const bf16_t*>(wgu), E, 2 * I, gu);
+  };
+  using std::integral_constant;
+  switch (H / kRouterKC) {
+    case 1: launch(integral_constant<int, 1>{}); break;
+    case 2: launch(integral_constant<int, 2>{}); break;
+    case 3: launch(integral_constant<int, 3>{}); break;
+    case 4: launch(integral_constant<int, 4>{}); break;
+    case 5: launch(integral_constant<int, 5>{}); break;
+    case 6: launch(integral_constant<int, 6>{}); break;
+    case 7: launch(integral_constant<int, 7>{}); break;
+    case 8: launch(integral_constant<int, 8>{}); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
 }
 
 hipError_t launch_router(const void* x, const void* w_router, const float* bias, int T, int H, int E, int k, int dtype,
