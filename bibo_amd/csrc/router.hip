@@ -126,8 +126,7 @@ __device__ __forceinline__ unsigned long long select_tokens16(const float* __res
 
 // Histogram of the selections of this workgroup's TOK tokens (16 threads each), for the permutation kernel.
 template <int TOK>
-__device__ __forceinline__ void write_chunk_hist(unsigned long long mask, int32_t* __restrict__ chunk_hist) {
-  __shared__ unsigned long long mask_s[TOK];
+__device__ __forceinline__ void write_chunk_hist(unsigned long long mask, int32_t* __restrict__ chunk_hist, unsigned long long* mask_s) {
   const int tid = threadIdx.x;
   if ((tid & 15) == 0) mask_s[tid >> 4] = mask;
   __syncthreads();
@@ -159,7 +158,7 @@ template <int TOK>
 __device__ __forceinline__ void router_finish(const floatx4& acc, float* sc, const float* bias_s, int T, int E, int k,
                                               int norm_mode, int t0, float* __restrict__ logits, int32_t* __restrict__ idx,
                                               float* __restrict__ w, float* __restrict__ gap,
-                                              int32_t* __restrict__ chunk_hist) {
+                                              int32_t* __restrict__ chunk_hist, unsigned long long* mask_s) {
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   const int tm = wave >> 2, en = wave & 3;
@@ -176,7 +175,7 @@ __device__ __forceinline__ void router_finish(const floatx4& acc, float* sc, con
   }
   __syncthreads();
   const unsigned long long mask = select_tokens16(sc, bias_s, E, k, norm_mode, t0, ntok, idx, w, gap);
-  if (chunk_hist != nullptr) write_chunk_hist<TOK>(mask, chunk_hist);
+  if (chunk_hist != nullptr) write_chunk_hist<TOK>(mask, chunk_hist, mask_s);
 }
 
 // ---- generic router: any H, bf16 or fp32 inputs, fp32 arithmetic ---------------------------------
@@ -252,7 +251,8 @@ __global__ __launch_bounds__(256) void router_f32_kernel(const TIn* __restrict__
     if (h0 + kGenKC < H) chunk(integral_constant<int, 1>{}, h0 + kGenKC);
     if (h0 + 2 * kGenKC < H) chunk(integral_constant<int, 2>{}, h0 + 2 * kGenKC);
   }
-  router_finish<kGenTokens>(acc, sc, bias_s, T, E, k, norm_mode, t0, logits, idx, w, gap, chunk_hist);
+  __shared__ unsigned long long mask_s[kGenTokens];
+  router_finish<kGenTokens>(acc, sc, bias_s, T, E, k, norm_mode, t0, logits, idx, w, gap, chunk_hist, mask_s);
 }
 
 template <int TOK>
@@ -317,7 +317,8 @@ __global__ __launch_bounds__(TOK * 16) void router_mfma_kernel(const bf16_t* __r
       multiply(st1);
     }
   }
-  router_finish<TOK>(acc, sc, bias_s, T, E, k, norm_mode, t0, logits, idx, w, gap, chunk_hist);
+  __shared__ unsigned long long mask_s[TOK];
+  router_finish<TOK>(acc, sc, bias_s, T, E, k, norm_mode, t0, logits, idx, w, gap, chunk_hist, mask_s);
 }
 
 // The same for calls of at most one workgroup per CU, which are a chain of memory latencies, one a chunk with two stages: here the first
@@ -394,7 +395,8 @@ __global__ __launch_bounds__(256) void router_ring_kernel(const bf16_t* __restri
       }
     });
   if (tid < kMaxE) bias_s[tid] = my_bias;
-  router_finish<TOK>(acc, sc, bias_s, T, E, k, norm_mode, t0, logits, idx, w, gap, chunk_hist);
+  __shared__ unsigned long long mask_s[TOK];
+  router_finish<TOK>(acc, sc, bias_s, T, E, k, norm_mode, t0, logits, idx, w, gap, chunk_hist, mask_s);
 }
 
 // A token's routing with the first pass of its experts behind it, for the few-token kernels: every workgroup works out the routing of its
@@ -449,7 +451,7 @@ __global__ __launch_bounds__(256) void router_gateup_kernel(const bf16_t* __rest
     }
   const bool first = blockIdx.x == 0 && j == 0;
   router_finish<16>(acc, sc, bias_s, 1, Et, k, norm_mode, 0, first && logits != nullptr ? logits + (size_t)t * Et : nullptr, idx_s, w_s,
-                    nullptr, nullptr);
+                    nullptr, nullptr, nullptr);
   __syncthreads();
   if (first && tid < k) {
     idx[(size_t)t * k + tid] = idx_s[tid];
@@ -469,7 +471,15 @@ __global__ __launch_bounds__(256) void router_gateup_kernel(const bf16_t* __rest
 // row back to LDS in place and to `xn` in memory, and the logits are then multiplied from the resident rows while
 // w_router streams through two LDS stages as in router_mfma_kernel.  x rows are stored as H/128 chunks of
 // [TOK][128], granule c of a chunk row r at position c ^ (r & 15).
-template <int TOK, typename TN>
+// What the selection needs lies where the rows were: 80 KB of LDS at TOK = 32 and H = 768, so that two workgroups share a CU and one's
+// round trips pass behind the other's arithmetic (one a CU: 30.0 -> 21.7 us at T = 16384, 26.9 -> 19.9 at 12000).  RING: six chunks of
+// w_router requested behind the rows, as in router_ring_kernel (H = 512, T = 1024: 10.8 -> 9.5 us; H = 768: 12.2 -> 11.4;
+// T = 16: 9.8 -> 10.8, so not there).
+constexpr int kNormRouterMaxH = 1024, kNormGran = kNormRouterMaxH / 8 / kWave;
+template <int TOK>
+constexpr int kNormTail = (TOK * kRowPad + kMaxE) * (int)sizeof(float) + TOK * (int)sizeof(unsigned long long);
+
+template <int TOK, typename TN, bool RING>
 __global__ __launch_bounds__(TOK * 16) void router_norm_mfma_kernel(const bf16_t* __restrict__ h, const TN* __restrict__ nw,
                                                                     float eps, const bf16_t* __restrict__ wr,
                                                                     const float* __restrict__ bias, int T, int H, int E,
@@ -480,15 +490,29 @@ __global__ __launch_bounds__(TOK * 16) void router_norm_mfma_kernel(const bf16_t
   constexpr int kThreads = TOK * 16;
   constexpr int kWPer = kMaxE * kRouterGran / kThreads;      // w_router load instructions per thread and chunk
   extern __shared__ __attribute__((aligned(16))) bf16_t xs[];                 // [H/128][TOK][128]
+  constexpr int kRingElems = RING ? kMaxE * kRouterKC : 8;
   __shared__ __attribute__((aligned(16))) bf16_t wst0[kMaxE * kRouterKC];
   __shared__ __attribute__((aligned(16))) bf16_t wst1[kMaxE * kRouterKC];
-  __shared__ float sc[TOK * kRowPad];
-  __shared__ float bias_s[kMaxE];
+  __shared__ __attribute__((aligned(16))) bf16_t wst2[kRingElems];
+  __shared__ __attribute__((aligned(16))) bf16_t wst3[kRingElems];
+  __shared__ __attribute__((aligned(16))) bf16_t wst4[kRingElems];
+  __shared__ __attribute__((aligned(16))) bf16_t wst5[kRingElems];
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   const int t0 = blockIdx.x * TOK;
   const int nchunks = H / kRouterKC;
-  if (tid < kMaxE) bias_s[tid] = (tid < E) ? bias[tid] : 0.f;
+  const int ngran = H / 8;
+  const float my_bias = tid < E ? bias[tid] : 0.f;
+  TN wv[kNormGran][8];                                 // the norm's weights of this lane's granules u*64 + lane, for all of the wave's rows
+#pragma unroll
+  for (int u = 0; u < kNormGran; ++u) {
+    const int c = min(u * kWave + lane, ngran - 1);
+    if constexpr (sizeof(TN) == 2) *reinterpret_cast<bf16x8*>(wv[u]) = reinterpret_cast<const bf16x8*>(nw)[c];
+    else
+#pragma unroll
+      for (int q = 0; q < 8; ++q) wv[u][q] = nw[c * 8 + q];
+  }
+  __builtin_amdgcn_sched_barrier(0);                   // requested in front of w_router: a wait for them is none for that
 
   // w_router chunk loads: thread t of instruction i fills granule i*kThreads + t = (row, position t % 16)
   const bf16_t* wsrc[kWPer];
@@ -503,7 +527,12 @@ __global__ __launch_bounds__(TOK * 16) void router_norm_mfma_kernel(const bf16_t
       __builtin_amdgcn_global_load_lds((router_gbl_void*)(wsrc[i] + k0), (router_lds_void*)(st + (i * kThreads + wave * 64) * 8),
                                        16, 0, 0);
   };
-  issue_w(0, wst0);
+  auto stage = [&](auto ic) -> bf16_t* {
+    constexpr int i = decltype(ic)::value;
+    if constexpr (i == 0) return wst0; else if constexpr (i == 1) return wst1; else if constexpr (i == 2) return wst2;
+    else if constexpr (i == 3) return wst3; else if constexpr (i == 4) return wst4; else return wst5;
+  };
+  if constexpr (!RING) issue_w(0, wst0);
   // the raw rows: instruction i is chunk i of every row (TOK * 16 granules = one per thread)
   {
     const int row = tid >> 4;
@@ -512,19 +541,30 @@ __global__ __launch_bounds__(TOK * 16) void router_norm_mfma_kernel(const bf16_t
       __builtin_amdgcn_global_load_lds((router_gbl_void*)(src + i * kRouterKC),
                                        (router_lds_void*)(xs + (i * kThreads + wave * 64) * 8), 16, 0, 0);
   }
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
+  if constexpr (RING) {
+    for_each<kRouterRing>([&](auto ic) { if (decltype(ic)::value < nchunks) issue_w(decltype(ic)::value * kRouterKC, stage(ic)); });
+    switch (min(nchunks, kRouterRing)) {               // the rows have arrived
+      case 1: sync_keep_loads<kWPer>(); break;
+      case 2: sync_keep_loads<2 * kWPer>(); break;
+      case 3: sync_keep_loads<3 * kWPer>(); break;
+      case 4: sync_keep_loads<4 * kWPer>(); break;
+      case 5: sync_keep_loads<5 * kWPer>(); break;
+      default: sync_keep_loads<6 * kWPer>();
+    }
+  } else {
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+  }
   // RMSNorm, one wave per row, four rows per wave; lane takes logical granules u*64 + lane of the row
   {
-    const int ngran = H / 8;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int r = wave * 4 + j;
-      bf16x8 v[4];
-      bf16_t* loc[4];
+      bf16x8 v[kNormGran];
+      bf16_t* loc[kNormGran];
       float ss = 0.f;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < kNormGran; ++u) {
         const int c = u * kWave + lane;
         if (c < ngran) {
           loc[u] = xs + (((c >> 4) * TOK + r) * kRouterGran + ((c & 15) ^ (r & 15))) * 8;
@@ -537,17 +577,12 @@ __global__ __launch_bounds__(TOK * 16) void router_norm_mfma_kernel(const bf16_t
       const float rinv = rsqrtf(ss / (float)H + eps);                                   // norm.py:22-23
       const bool live = t0 + r < T;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < kNormGran; ++u) {
         const int c = u * kWave + lane;
         if (c < ngran) {
           bf16x8 o;
-          TN wv[8];
-          if constexpr (sizeof(TN) == 2) *reinterpret_cast<bf16x8*>(wv) = reinterpret_cast<const bf16x8*>(nw)[c];
-          else
 #pragma unroll
-            for (int q = 0; q < 8; ++q) wv[q] = nw[c * 8 + q];
-#pragma unroll
-          for (int q = 0; q < 8; ++q) o[q] = (bf16_t)((float)wv[q] * (float)(bf16_t)((float)v[u][q] * rinv));   // norm.py:24
+          for (int q = 0; q < 8; ++q) o[q] = (bf16_t)((float)wv[u][q] * (float)(bf16_t)((float)v[u][q] * rinv));   // norm.py:24
           *reinterpret_cast<bf16x8*>(loc[u]) = o;
           if (live) *reinterpret_cast<bf16x8*>(xn + (size_t)(t0 + r) * H + c * 8) = o;
         }
@@ -568,19 +603,48 @@ __global__ __launch_bounds__(TOK * 16) void router_norm_mfma_kernel(const bf16_t
       acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
     }
   };
-  for (int c0 = 0; c0 < nchunks; c0 += 2) {
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();                                   // first pass: also the normalised rows of the other waves
-    if (c0 + 1 < nchunks) issue_w((c0 + 1) * kRouterKC, wst1);
-    multiply(xs + (size_t)c0 * TOK * kRouterKC, wst0);
-    if (c0 + 1 < nchunks) {
+  if constexpr (RING) {
+    for (int c0 = 0; c0 < nchunks; c0 += kRouterRing)
+      for_each<kRouterRing>([&](auto ic) {
+        const int c = c0 + decltype(ic)::value;
+        if (c >= nchunks) return;
+        if (c == 0) __builtin_amdgcn_s_waitcnt(0xc07f);          // this wave's normalised rows are in LDS
+        switch (min(nchunks - 1 - c, kRouterRing - 1)) {         // chunks that may still be on their way (stores of rows do no harm)
+          case 0: sync_keep_loads<0>(); break;
+          case 1: sync_keep_loads<kWPer>(); break;
+          case 2: sync_keep_loads<2 * kWPer>(); break;
+          case 3: sync_keep_loads<3 * kWPer>(); break;
+          case 4: sync_keep_loads<4 * kWPer>(); break;
+          default: sync_keep_loads<5 * kWPer>();
+        }
+        multiply(xs + (size_t)c * TOK * kRouterKC, stage(ic));
+        if (c + kRouterRing < nchunks) {
+          __builtin_amdgcn_s_waitcnt(0xc07f);                    // this wave's reads of the stage have returned
+          __builtin_amdgcn_s_barrier();
+          issue_w((c + kRouterRing) * kRouterKC, stage(ic));
+        }
+      });
+  } else {
+    for (int c0 = 0; c0 < nchunks; c0 += 2) {
       __builtin_amdgcn_s_waitcnt(0);
-      __syncthreads();
-      if (c0 + 2 < nchunks) issue_w((c0 + 2) * kRouterKC, wst0);
-      multiply(xs + (size_t)(c0 + 1) * TOK * kRouterKC, wst1);
+      __syncthreads();                                   // first pass: also the normalised rows of the other waves
+      if (c0 + 1 < nchunks) issue_w((c0 + 1) * kRouterKC, wst1);
+      multiply(xs + (size_t)c0 * TOK * kRouterKC, wst0);
+      if (c0 + 1 < nchunks) {
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        if (c0 + 2 < nchunks) issue_w((c0 + 2) * kRouterKC, wst0);
+        multiply(xs + (size_t)(c0 + 1) * TOK * kRouterKC, wst1);
+      }
     }
   }
-  router_finish<TOK>(acc, sc, bias_s, T, E, k, norm_mode, t0, logits, idx, w, gap, chunk_hist);
+  // the rows' LDS holds what is left to do: scores, bias, selections
+  __syncthreads();
+  float* sc = reinterpret_cast<float*>(xs);
+  float* bias_s = sc + TOK * kRowPad;
+  unsigned long long* mask_s = reinterpret_cast<unsigned long long*>(bias_s + kMaxE);
+  if (tid < kMaxE) bias_s[tid] = my_bias;
+  router_finish<TOK>(acc, sc, bias_s, T, E, k, norm_mode, t0, logits, idx, w, gap, chunk_hist, mask_s);
 }
 
 // ---- MFMA router for H % 32 == 0 but not % 128: operands straight to registers, K split over 4 waves ----
@@ -647,13 +711,11 @@ __global__ __launch_bounds__(256) void router_mfma_split_kernel(const bf16_t* __
   }
   __syncthreads();
   const unsigned long long mask = select_tokens16(sc, bias_s, E, k, norm_mode, t0, ntok, idx, w, gap);
-  if (chunk_hist != nullptr) write_chunk_hist<kMfmaTokens>(mask, chunk_hist);
+  __shared__ unsigned long long mask_s[kMfmaTokens];
+  if (chunk_hist != nullptr) write_chunk_hist<kMfmaTokens>(mask, chunk_hist, mask_s);
 }
 
 }  // namespace
-
-// The widest hidden size whose TOK raw rows fit LDS next to the w_router stages (TOK = 32: 64 KB of rows).
-constexpr int kNormRouterMaxH = 1024;
 
 bool router_norm_supported(int H, int dtype, const void* h, const void* w_router, const void* xn) {
   const bool aligned = ((reinterpret_cast<uintptr_t>(h) | reinterpret_cast<uintptr_t>(w_router) |
@@ -662,10 +724,10 @@ bool router_norm_supported(int H, int dtype, const void* h, const void* w_router
 }
 
 // the kernel's TOK whole rows sit in dynamic LDS: allowed once per device, for the widest rows it takes
-template <int TOK, typename TN>
+template <int TOK, typename TN, bool RING>
 hipError_t allow_dynamic_lds() {
   static LdsLimitOnce once;
-  return once.raise(reinterpret_cast<const void*>(&router_norm_mfma_kernel<TOK, TN>), (int)(TOK * kNormRouterMaxH * sizeof(bf16_t)));
+  return once.raise(reinterpret_cast<const void*>(&router_norm_mfma_kernel<TOK, TN, RING>), (int)(TOK * kNormRouterMaxH * sizeof(bf16_t)));
 }
 
 // RMSNorm + router in one launch (see router_norm_mfma_kernel); `xn` receives the normalised rows.
@@ -677,19 +739,24 @@ hipError_t launch_router_norm(const void* h, Vec norm_weight, float eps, const v
   const bf16_t* hp = static_cast<const bf16_t*>(h);
   const bf16_t* wp = static_cast<const bf16_t*>(w_router);
   bf16_t* xp = static_cast<bf16_t*>(xn);
-  auto launch = [&](auto tok, auto* nw) -> hipError_t {
+  auto launch = [&](auto tok, auto ring, auto* nw) -> hipError_t {
     constexpr int TOK = decltype(tok)::value;
+    constexpr bool RING = decltype(ring)::value;
     using TN = std::remove_const_t<std::remove_pointer_t<decltype(nw)>>;
-    const hipError_t e = allow_dynamic_lds<TOK, TN>();
+    const hipError_t e = allow_dynamic_lds<TOK, TN, RING>();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((router_norm_mfma_kernel<TOK, TN>), dim3((T + TOK - 1) / TOK), dim3(TOK * 16), (size_t)TOK * H * sizeof(bf16_t), s,
-                       hp, nw, eps, wp, bias, T, H, E, k, norm_mode, xp, logits, idx, w, nullptr, chunk_hist);
+    const size_t rows = (size_t)TOK * H * sizeof(bf16_t), lds = rows > (size_t)kNormTail<TOK> ? rows : (size_t)kNormTail<TOK>;
+    hipLaunchKernelGGL((router_norm_mfma_kernel<TOK, TN, RING>), dim3((T + TOK - 1) / TOK), dim3(TOK * 16), lds, s, hp, nw, eps, wp, bias, T, H, E, k, norm_mode, xp, logits, idx, w, nullptr, chunk_hist);
     return hipGetLastError();
   };
-  auto typed = [&](auto tok) {
-    return norm_weight.bf16 ? launch(tok, static_cast<const bf16_t*>(norm_weight.p)) : launch(tok, static_cast<const float*>(norm_weight.p));
+  auto typed = [&](auto tok, auto ring) {
+    return norm_weight.bf16 ? launch(tok, ring, static_cast<const bf16_t*>(norm_weight.p))
+                            : launch(tok, ring, static_cast<const float*>(norm_weight.p));
   };
-  const hipError_t e = T >= 32 * 256 ? typed(std::integral_constant<int, 32>()) : typed(std::integral_constant<int, 16>());
+  using std::integral_constant;
+  const hipError_t e = T >= 32 * 256 ? typed(integral_constant<int, 32>(), std::false_type())
+                       : T >= kRingLeast && T <= 16 * kCUs ? typed(integral_constant<int, 16>(), std::true_type())
+                                        : typed(integral_constant<int, 16>(), std::false_type());
   if (e != hipSuccess) return e;
   if (hist_tokens != nullptr && chunk_hist != nullptr) *hist_tokens = T >= 32 * 256 ? 32 : 16;
   return hipSuccess;

@@ -30,3 +30,24 @@ def test_ring(H, T, E, k):
     assert bool(((logits.double() - x.double() @ wr.double().t()).abs() <= bound).all())
     oi, ow, _ = O.route_from_logits(logits.numpy(), bias.numpy(), k, "sum")
     assert np.array_equal(idx.numpy(), oi) and np.array_equal(w.numpy(), ow)
+
+
+@pytest.mark.parametrize("H", [128, 640, 768, 896, 1024])
+@pytest.mark.parametrize("T,E,k", [(127, 9, 2), (128, 64, 6), (1000, 64, 6), (4096, 64, 8), (4097, 33, 4), (8192, 64, 6), (8197, 64, 6)])
+def test_behind_the_norm(H, T, E, k):
+    """The same kernel shapes with the RMSNorm in front: the bits of the norm and the router on their own."""
+    g = torch.Generator().manual_seed(H + T)
+    I = 128
+    x = torch.randn(T, H, generator=g).bfloat16().to(DEV)
+    nw = (torch.rand(H, generator=g) + 0.5).to(DEV)
+    wr = (torch.randn(E, H, generator=g) * 0.1).bfloat16().to(DEV)
+    bias = (torch.rand(E, generator=g) * 0.02 - 0.01).to(DEV)
+    gu = (torch.randn(E, 2 * I, H, generator=g) * 0.05).bfloat16().to(DEV)
+    dn = (torch.randn(E, H, I, generator=g) * 0.05).bfloat16().to(DEV)
+    th = torch.zeros(E, device=DEV)
+    got = ops.ffn_forward(x, nw, 1e-6, wr, bias, gu, dn, th, k, want_routing=True)
+    xn = ops.rmsnorm_fwd(x, nw, 1e-6)
+    idx, w, _, _ = ops.router_fwd(xn, wr, bias, k, "sum")
+    assert torch.equal(got[1], idx) and torch.equal(got[2], w)
+    out = ops.moe_forward(xn, wr, bias, gu, dn, th, k)[0]
+    assert float((got[0].double() - (x.double() + out.double())).abs().max()) <= 2.0 ** -7 * float((x.double() + out.double()).abs().max())
