@@ -344,15 +344,17 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
                         (long long)T * k <= (a == BIBO_ALGO_FUSED ? kScanSlots : kScanSlots / 2) &&
                         (state != nullptr ? Eg == E : counts_out == nullptr) && aligned16(x) && aligned16(w_gate_up) && aligned16(w_down);
   const bool want_hist = may_scan || (need_permute && T > 0 && permute_takes_router_hist(T, k));
-  if (T > 0 && norm_src != nullptr) {
-    rc = hip_rc(launch_router_norm(norm_src, norm_weight, eps, w_router, bias, T, H, E, k, norm_mode, const_cast<void*>(x),
-                                   logits_out, idx, w, want_hist ? hist : nullptr, &hist_tokens, s));
-    if (rc != BIBO_OK) return rc;
-  } else if (few && !want_hist && router_gateup_supported(T, H, k, I, dtype, x, w_router)) {
-    rc = hip_rc(launch_router_gateup(x, w_router, bias, T, H, E, k, norm_mode, logits_out, idx, w, w_gate_up, Eg, I,
-                                     reinterpret_cast<float*>(base + ws.gu), s));
+  const void* rows = norm_src != nullptr ? norm_src : x;
+  void* xn = norm_src != nullptr ? const_cast<void*>(x) : nullptr;
+  if (few && !want_hist && router_gateup_supported(T, H, k, I, dtype, rows, w_router)) {
+    rc = hip_rc(launch_router_gateup(rows, w_router, bias, T, H, E, k, norm_mode, logits_out, idx, w, w_gate_up, Eg, I,
+                                     reinterpret_cast<float*>(base + ws.gu), norm_weight, eps, xn, s));
     if (rc != BIBO_OK) return rc;
     gate_up_done = true;
+  } else if (T > 0 && norm_src != nullptr) {
+    rc = hip_rc(launch_router_norm(norm_src, norm_weight, eps, w_router, bias, T, H, E, k, norm_mode, xn, logits_out, idx, w,
+                                   want_hist ? hist : nullptr, &hist_tokens, s));
+    if (rc != BIBO_OK) return rc;
   } else if (T > 0 && (rc = hip_rc(launch_router(x, w_router, bias, T, H, E, k, dtype, norm_mode, logits_out, idx, w, nullptr,
                                                  want_hist ? hist : nullptr, &hist_tokens, s))) != BIBO_OK)
     return rc;

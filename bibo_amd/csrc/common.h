@@ -211,10 +211,11 @@ hipError_t launch_down_generic(const void* hidden, const void* wd, const float* 
                                const int32_t* perm_slot, int T, int H, int E, int k, int I, int dtype, float* yw,
                                hipStream_t s);
 bool tile_f32_supported(int H, int I);
-// launch_router and the gate/up launch of launch_experts_few in one, where every workgroup has a CU to itself
+// launch_router (xn: launch_router_norm, and the rows it leaves; NULL: no norm) and the gate/up launch of launch_experts_few in one
 bool router_gateup_supported(int T, int H, int k, int I, int dtype, const void* x, const void* w_router);
 hipError_t launch_router_gateup(const void* x, const void* w_router, const float* bias, int T, int H, int Et, int k, int norm_mode,
-                                float* logits, int32_t* idx, float* w, const void* wgu, int E, int I, float* gu, hipStream_t s);
+                                float* logits, int32_t* idx, float* w, const void* wgu, int E, int I, float* gu, Vec norm_weight, float eps,
+                                void* xn, hipStream_t s);
 bool few_supported(int T, int H, int k, int I);
 hipError_t launch_experts_tiled(const void* x, const void* wgu, const void* wd, const float* theta, const float* w,
                                 const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int T, int H,

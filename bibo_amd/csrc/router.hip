@@ -399,6 +399,8 @@ __global__ __launch_bounds__(256) void router_ring_kernel(const bf16_t* __restri
   router_finish<TOK>(acc, sc, bias_s, T, E, k, norm_mode, t0, logits, idx, w, gap, chunk_hist, mask_s);
 }
 
+constexpr int kNormRouterMaxH = 1024, kNormGran = kNormRouterMaxH / 8 / kWave;
+
 // A token's routing with the first pass of its experts behind it, for the few-token kernels: every workgroup works out the routing of its
 // slot's token for itself and goes on to blocks of 32 rows of the slot's gate/up weights.  All of w_router (98 KB at E = 64, H = 768) comes
 // from L2 to each workgroup at once, every request on its way before the first wait, and a launch and the gap behind it are saved.  One
@@ -407,12 +409,18 @@ __global__ __launch_bounds__(256) void router_ring_kernel(const bf16_t* __restri
 // 13.3 -> 10.6 (1), 18.1 -> 17.7 (8); H = 1024, I = 512, k = 8: 22.0 -> 17.4 (1), 30.8 -> 26.0 (4).  The host is through sooner too: the
 // layer of one token at H = 768 takes 12.2 us instead of 15.6.  Same products in the same order as router_mfma_kernel and
 // gateup_few_kernel.  Grid (blocks of rows shared out, T k); NG = H / 128.
-template <int NG>
+// TN (the type of the norm's weights; void: no norm): the token's row goes through the block's input RMSNorm first, in every wave, with the
+// arithmetic and the summation order of router_norm_mfma_kernel; the first workgroup of a token leaves it in `xn`.
+// Kernels of norm + layer + sum, norm and router in a launch of their own -> this, us: H = 768, I = 384: 17.6 -> 13.3 (T = 1), 24.2 -> 19.2 (4),
+// 28.2 -> 26.1 (8); H = 512, I = 256: 15.2 -> 11.5, 17.1 -> 13.0, 19.4 -> 16.6; H = 1024, I = 512, k = 8: 20.7 -> 16.5 (1), 32.7 -> 26.3 (4).
+template <int NG, typename TN>
 __global__ __launch_bounds__(256) void router_gateup_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ wr,
                                                             const float* __restrict__ bias, int Et, int k, int norm_mode,
                                                             float* __restrict__ logits, int32_t* __restrict__ idx,
                                                             float* __restrict__ w, const bf16_t* __restrict__ wgu, int E, int I2,
-                                                            float* __restrict__ gu) {
+                                                            float* __restrict__ gu, const void* __restrict__ norm_weight, float eps,
+                                                            bf16_t* __restrict__ xn) {
+  constexpr bool kNorm = !std::is_same_v<TN, void>;
   constexpr int H = NG * kRouterKC, kGran = H / 8;
   __shared__ __attribute__((aligned(16))) bf16_t ws[kMaxE * H];
   __shared__ __attribute__((aligned(16))) bf16_t xs[H];
@@ -423,6 +431,23 @@ __global__ __launch_bounds__(256) void router_gateup_kernel(const bf16_t* __rest
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int slot = blockIdx.y, t = slot / k, j = slot - t * k;
   const bf16_t* xr = x + (size_t)t * H;
+  const bool first = blockIdx.x == 0 && j == 0;
+  bf16x8 row[kNormGran];                               // granules u*64 + lane
+  float nw[kNormGran][8];
+  if constexpr (kNorm) {
+#pragma unroll
+    for (int u = 0; u < kNormGran; ++u) {
+      const int c = min(u * kWave + lane, kGran - 1);
+      row[u] = *reinterpret_cast<const bf16x8*>(xr + c * 8);
+      TN v[8];
+      if constexpr (sizeof(TN) == 2) *reinterpret_cast<bf16x8*>(v) = reinterpret_cast<const bf16x8*>(norm_weight)[c];
+      else
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = static_cast<const TN*>(norm_weight)[c * 8 + q];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) nw[u][q] = (float)v[q];
+    }
+  }
   // chunk-major stages as in router_mfma_kernel: granule c of a row sits at position c ^ (row & 15)
 #pragma unroll
   for (int c = 0; c < NG; ++c)
@@ -434,11 +459,37 @@ __global__ __launch_bounds__(256) void router_gateup_kernel(const bf16_t* __rest
     }
   const int c16 = tid & 15, rg = tid >> 4;
   Raw8<bf16_t> xv[NG];
+  if constexpr (kNorm) {
+    float ss = 0.f;
 #pragma unroll
-  for (int u = 0; u < NG; ++u) xv[u].load(xr + (u * 16 + c16) * 8);
-  if (tid < kGran) *reinterpret_cast<bf16x8*>(xs + tid * 8) = *reinterpret_cast<const bf16x8*>(xr + tid * 8);
+    for (int u = 0; u < kNormGran; ++u)
+      if (u * kWave + lane < kGran)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) ss = fmaf((float)row[u][q], (float)row[u][q], ss);
+    ss = wave_sum(ss);
+    const float rinv = rsqrtf(ss / (float)H + eps);                                               // norm.py:22-23
+#pragma unroll
+    for (int u = 0; u < kNormGran; ++u) {
+      const int c = u * kWave + lane;
+      if (wave == u && c < kGran) {
+        bf16x8 o;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) o[q] = (bf16_t)(nw[u][q] * (float)(bf16_t)((float)row[u][q] * rinv));    // norm.py:24
+        *reinterpret_cast<bf16x8*>(xs + c * 8) = o;
+        if (first) *reinterpret_cast<bf16x8*>(xn + (size_t)t * H + c * 8) = o;
+      }
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < NG; ++u) xv[u].load(xr + (u * 16 + c16) * 8);
+    if (tid < kGran) *reinterpret_cast<bf16x8*>(xs + tid * 8) = *reinterpret_cast<const bf16x8*>(xr + tid * 8);
+  }
   if (tid < kMaxE) bias_s[tid] = tid < Et ? bias[tid] : 0.f;
   __syncthreads();
+  if constexpr (kNorm) {
+#pragma unroll
+    for (int u = 0; u < NG; ++u) xv[u].v = *reinterpret_cast<const bf16x8*>(xs + (u * 16 + c16) * 8);
+  }
   const int r16 = lane & 15, kc = lane >> 4;
   floatx4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -449,7 +500,6 @@ __global__ __launch_bounds__(256) void router_gateup_kernel(const bf16_t* __rest
       const bf16x8 b = *reinterpret_cast<const bf16x8*>(ws + (c * kMaxE + wave * 16 + r16) * kRouterKC + ((s * 4 + kc) ^ r16) * 8);
       acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
     }
-  const bool first = blockIdx.x == 0 && j == 0;
   router_finish<16>(acc, sc, bias_s, 1, Et, k, norm_mode, 0, first && logits != nullptr ? logits + (size_t)t * Et : nullptr, idx_s, w_s,
                     nullptr, nullptr, nullptr);
   __syncthreads();
@@ -475,7 +525,6 @@ __global__ __launch_bounds__(256) void router_gateup_kernel(const bf16_t* __rest
 // round trips pass behind the other's arithmetic (one a CU: 30.0 -> 21.7 us at T = 16384, 26.9 -> 19.9 at 12000).  RING: six chunks of
 // w_router requested behind the rows, as in router_ring_kernel (H = 512, T = 1024: 10.8 -> 9.5 us; H = 768: 12.2 -> 11.4;
 // T = 16: 9.8 -> 10.8, so not there).
-constexpr int kNormRouterMaxH = 1024, kNormGran = kNormRouterMaxH / 8 / kWave;
 template <int TOK>
 constexpr int kNormTail = (TOK * kRowPad + kMaxE) * (int)sizeof(float) + TOK * (int)sizeof(unsigned long long);
 
@@ -768,12 +817,19 @@ bool router_gateup_supported(int T, int H, int k, int I, int dtype, const void* 
 }
 
 hipError_t launch_router_gateup(const void* x, const void* w_router, const float* bias, int T, int H, int Et, int k, int norm_mode,
-                                float* logits, int32_t* idx, float* w, const void* wgu, int E, int I, float* gu, hipStream_t s) {
+                                float* logits, int32_t* idx, float* w, const void* wgu, int E, int I, float* gu, Vec norm_weight, float eps,
+                                void* xn, hipStream_t s) {
   const int blocks = (2 * I + kGateRows - 1) / kGateRows, most = kCUs / (T * k), each = (blocks + most - 1) / most;
-  auto launch = [&](auto ng) {
-    hipLaunchKernelGGL((router_gateup_kernel<decltype(ng)::value>), dim3((blocks + each - 1) / each, T * k), dim3(256), 0, s,
+  auto typed = [&](auto ng, auto* tn) {
+    using TN = std::remove_pointer_t<decltype(tn)>;
+    hipLaunchKernelGGL((router_gateup_kernel<decltype(ng)::value, TN>), dim3((blocks + each - 1) / each, T * k), dim3(256), 0, s,
                        static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w_router), bias, Et, k, norm_mode, logits, idx, w,
-                       static_cast<const bf16_t*>(wgu), E, 2 * I, gu);
+                       static_cast<const bf16_t*>(wgu), E, 2 * I, gu, norm_weight.p, eps, static_cast<bf16_t*>(xn));
+  };
+  auto launch = [&](auto ng) {
+    if (xn == nullptr) typed(ng, static_cast<void*>(nullptr));
+    else if (norm_weight.bf16) typed(ng, static_cast<bf16_t*>(nullptr));
+    else typed(ng, static_cast<float*>(nullptr));
   };
   using std::integral_constant;
   switch (H / kRouterKC) {

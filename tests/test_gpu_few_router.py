@@ -29,3 +29,11 @@ def test_token_by_token(H, Eg, pairs, k, I):
             assert torch.equal(one[i], whole[i][t:t + 1])
         if t % 2 == 1:
             assert torch.equal(one[3], torch.bincount(one[1].flatten().long(), minlength=E).int())
+    # behind the norm: the bits of the norm, the layer and the sum on their own
+    nw = (torch.rand(H, generator=g) + 0.5).to(DEV)
+    kw = dict(n_pos=pairs, n_neg=pairs)
+    xn = ops.rmsnorm_fwd(x, nw, 1e-6)
+    seam = ops.ffn_forward(x, nw, 1e-6, *args, k, want_routing=True, residual=False, **kw)
+    ref = ops.moe_forward(xn, *args, k, want_routing=True, **kw)
+    for a, b in zip(seam[:3], ref[:3]):
+        assert torch.equal(a, b)
