@@ -243,8 +243,9 @@ hipError_t launch_gateup_mfma(const void* x, const void* wgu, const float* theta
 hipError_t launch_down_mfma(const void* hidden, const void* wd, const float* w, const int32_t* offsets,
                             const int32_t* perm_slot, int T, int H, int E, int k, int I, void* yw, hipStream_t s);
 
-// For a call that fills one round of the fused kernel's tiles at most (half of it on average: kScanSlots of 128-row tiles, half as many of
-// 64) and needs no permutation otherwise: the workgroups find their rows in the routing itself.  hist: the router's histograms, one per 16
+// For calls that need no permutation otherwise: the fused kernel's workgroups find their rows in the routing itself.  kScanSlots is half of
+// what one round of 128-row tiles holds (64-row tiles: half as many slots): beyond one round a CU would look twice, and the permutation's
+// launch is small beside the rest (figures at experts_fused_kernel).  hist: the router's histograms, one per 16
 // tokens.  Left behind for who reads them later: perm_slot and offsets by launch_gateup_raw (for launch_down_act), those, perm_token and
 // counts by a training forward (its experts all have weights: nobody would place the slots of the others).
 constexpr int kScanSlots = 16384;
