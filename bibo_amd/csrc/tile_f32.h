@@ -137,10 +137,16 @@ template <typename T> struct Planes { static constexpr int n = 3; typedef floatx
 template <> struct Planes<bf16_t> { static constexpr int n = 1; typedef bf16x4 raw; };
 __device__ __forceinline__ floatx4 widen4(floatx4 v) { return v; }
 __device__ __forceinline__ floatx4 widen4(bf16x4 v) { return floatx4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]}; }
-// Plane p of four consecutive elements, which v holds less the planes before it, to LDS; v keeps the rest.
+// Plane p of four consecutive elements, which v holds less the planes before it, to LDS; v keeps the rest.  A number whose lowest bit lies
+// below 2^-133, bf16's smallest subnormal, is not the sum of three parts (all others are: the rest behind two parts has eight bits at
+// most).  The rest then is an fp32 subnormal with some of its low 16 bits set, which no other third part has: `rests` collects them.
 template <int P>
-__device__ __forceinline__ void put_plane(bf16_t* to, floatx4& v) {
+__device__ __forceinline__ void put_plane(bf16_t* to, floatx4& v, unsigned& rests) {
   typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+  if constexpr (P == 2) {
+    rests |= __float_as_uint(v[0]) | __float_as_uint(v[1]);
+    rests |= __float_as_uint(v[2]) | __float_as_uint(v[3]);
+  }
   const u32x2 u = {__builtin_bit_cast(unsigned, bf16x2{(bf16_t)v[0], (bf16_t)v[1]}), __builtin_bit_cast(unsigned, bf16x2{(bf16_t)v[2], (bf16_t)v[3]})};
   *reinterpret_cast<u32x2*>(to) = u;
   if constexpr (P < 2) {
@@ -151,7 +157,8 @@ __device__ __forceinline__ void put_plane(bf16_t* to, floatx4& v) {
   }
 }
 template <int P>
-__device__ __forceinline__ void put_plane(bf16_t* to, bf16x4& v) { *reinterpret_cast<bf16x4*>(to) = v; }
+__device__ __forceinline__ void put_plane(bf16_t* to, bf16x4& v, unsigned&) { *reinterpret_cast<bf16x4*>(to) = v; }
+__device__ __forceinline__ bool bits_lost(unsigned rests) { return (rests & 0xffffu) != 0; }
 
 // Element offset of the four k from 4 c on of row r in a [rows][32] plane: 64-byte rows, 16-byte granules as in the stripe layout.
 __device__ __forceinline__ int aswz(int r, int c) { return r * kFK + (((c >> 1) ^ ((r >> 2) & 3)) << 3) + ((c & 1) << 2); }
@@ -242,16 +249,17 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ggemm_split_kernel(const TA* 
       }
     }
   };
+  unsigned rests = 0;
   // one plane of one of a thread's A_PER + W_PER quadruples to its stage
   auto put = [&](auto set_c, auto q_c) {
     constexpr int set = decltype(set_c)::value, q = decltype(q_c)::value;
     if constexpr (q < A_PER * PA) {
       constexpr int i = q / PA, p = q % PA;
-      put_plane<p>(As[set] + p * (BM * kFK) + aswz(ar + kThreads / 8 * i, ac), ra[set][i]);
+      put_plane<p>(As[set] + p * (BM * kFK) + aswz(ar + kThreads / 8 * i, ac), ra[set][i], rests);
     } else if constexpr (q < A_PER * PA + W_PER * PW) {
       constexpr int i = (q - A_PER * PA) / PW, p = (q - A_PER * PA) % PW;
       const int g = tid + kThreads * i;
-      put_plane<p>(Ws[set] + p * (BN * kFK) + (W_KM ? kswz<BN>(g / (BN / 4), g % (BN / 4)) : aswz(ar + kThreads / 8 * i, ac)), rw[set][i]);
+      put_plane<p>(Ws[set] + p * (BN * kFK) + (W_KM ? kswz<BN>(g / (BN / 4), g % (BN / 4)) : aswz(ar + kThreads / 8 * i, ac)), rw[set][i], rests);
     }
   };
   const int wm = wave % WM, wn = wave / WM, l32 = lane & 31, h = lane >> 5;
@@ -358,13 +366,15 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ggemm_split_kernel(const TA* 
     for (int j = 0; j < NTW; ++j) acc[1][j] = acc[0][j];
     fold();
   }
-  // An infinity, a NaN or a value that rounds to infinity has no three bf16 parts: a tile whose sums are not all finite is multiplied
-  // again by fp32 MFMAs, whose infinities and NaNs are those of the products.
+  // An infinity, a NaN, a value that rounds to infinity or one with bits below 2^-133 (from 2^-110 down) has no three bf16 parts: a tile
+  // whose sums are not all finite, or that has met such bits, is multiplied again by fp32 MFMAs, whose infinities and NaNs are those of
+  // the products.  (The bf16 MFMAs keep subnormal operands, products and sums: small results need nothing of the kind.)  Collecting the bits
+  // costs 1 % (the layer of T = 2048 above: 258.7 -> 261.3 us).
   if constexpr (PA + PW > 2) {
     bool finite = true;
 #pragma unroll
     for (int f = 0; f < 16 * NTW; ++f) finite = finite && fabs(sum[f / 16][f % 16]) <= 3.402823466e38;
-    if (__syncthreads_or(!finite)) {
+    if (__syncthreads_or(!finite || bits_lost(rests))) {
       float* const af = reinterpret_cast<float*>(As);
       float* const wf = reinterpret_cast<float*>(Ws);
 #pragma unroll
@@ -492,16 +502,17 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void wgrad_split_kernel(const TP* 
     }
   };
   constexpr int kPuts = P_PER * PP + Q_PER * PQ;
+  unsigned rests = 0;
   auto put = [&](auto set_c, auto q_c) {
     constexpr int set = decltype(set_c)::value, q = decltype(q_c)::value;
     if constexpr (q < P_PER * PP) {
       constexpr int i = q / PP, p = q % PP;
       const int g = tid + kThreads * i;
-      put_plane<p>(Ps[set] + p * (BP * kFK) + kswz<BP>(g / (BP / 4), g % (BP / 4)), rp[set][i]);
+      put_plane<p>(Ps[set] + p * (BP * kFK) + kswz<BP>(g / (BP / 4), g % (BP / 4)), rp[set][i], rests);
     } else if constexpr (q < kPuts) {
       constexpr int i = (q - P_PER * PP) / PQ, p = (q - P_PER * PP) % PQ;
       const int g = tid + kThreads * i;
-      put_plane<p>(Qs[set] + p * (BQ * kFK) + kswz<BQ>(g / (BQ / 4), g % (BQ / 4)), rq[set][i]);
+      put_plane<p>(Qs[set] + p * (BQ * kFK) + kswz<BQ>(g / (BQ / 4), g % (BQ / 4)), rq[set][i], rests);
     }
   };
   const int wm = wave % WM, wn = wave / WM, l32 = lane & 31, h = lane >> 5;
@@ -562,13 +573,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void wgrad_split_kernel(const TP* 
       if (s + 1 < nsteps) turn(c1, s + 1);
     }
   }
-  if constexpr (PP + PQ > 2) {                           // infinities and NaNs, as in ggemm_split_kernel
+  if constexpr (PP + PQ > 2) {                           // numbers without three parts, as in ggemm_split_kernel
     bool finite = true;
 #pragma unroll
     for (int j = 0; j < NTW; ++j)
 #pragma unroll
       for (int i = 0; i < 16; ++i) finite = finite && fabsf(acc[j][i]) <= 3.402823466e38f;
-    if (__syncthreads_or(!finite)) {
+    if (__syncthreads_or(!finite || bits_lost(rests))) {
       float* const pf = reinterpret_cast<float*>(Ps);
       float* const qf = reinterpret_cast<float*>(Qs);
 #pragma unroll

@@ -85,3 +85,31 @@ def test_infinities_and_nans_stay_where_they_are(rows):
     x[a, 1] = float("nan")
     out = _forward({**p, "x": x}, idx, w).cpu()
     assert torch.isnan(out[a]).all() and torch.isfinite(out[rest]).all()
+
+
+# bf16 ends at 2^-133, so a number below 2^-110 is not the sum of three bf16 parts.  2^-118 loses bits from 2^-15 of it down, 2^-130 is a
+# subnormal itself.  The results are in the usual range, or as far above 2^-149 as their bound needs
+@pytest.mark.parametrize("e", [112, 118, 130])
+@pytest.mark.parametrize("rows", [(400, 800), (2000, 2400)])
+def test_small_numbers(rows, e):
+    p, idx, w = _inputs(516, 260, rows, 7)
+    p["x"] *= 2.0 ** (e - 8)
+    p["w_gate_up"] *= 2.0 ** -e
+    ref = O.experts_forward(p["x"], idx, w, p["w_gate_up"], p["w_down"], p["theta"], dtype=torch.float64)
+    assert _rel(_forward(p, idx, w), ref) <= 1.2e-6
+    p, idx, w = _inputs(516, 260, rows, 8)
+    p["w_down"] *= 2.0 ** -min(e, 118)
+    ref = O.experts_forward(p["x"], idx, w, p["w_gate_up"], p["w_down"], p["theta"], dtype=torch.float64)
+    assert _rel(_forward(p, idx, w), ref) <= 1.2e-6
+
+
+@pytest.mark.parametrize("T,H,I,E,k", [(777, 192, 88, 16, 3), (1200, 640, 256, 9, 2)])
+def test_small_gradients(T, H, I, E, k):
+    p = O.make_inputs(T=T, H=H, E=E, k=k, I=I, bias="uniform", theta="normal", seed=T, dtype=torch.float32)
+    d = torch.randn(T, H, generator=torch.Generator().manual_seed(T)) * 2.0 ** -112
+    args = [p[n].to(DEV) for n in NAMES]
+    got = ops.moe_backward(p["x"].to(DEV), d.to(DEV), *args, k)
+    idx = ops.moe_forward(p["x"].to(DEV), *args, k, want_routing=True)[1].cpu().numpy()
+    ref = O.moe_backward(p["x"], p["w_router"], p["w_gate_up"], p["w_down"], p["theta"], idx, d)
+    for name, a in zip(("x", "w_router", "w_gate_up", "w_down"), got):
+        assert _rel(a, ref[name]) <= 2e-6, name
