@@ -140,13 +140,15 @@ __device__ __forceinline__ floatx4 widen4(bf16x4 v) { return floatx4{(float)v[0]
 // Plane p of four consecutive elements, which v holds less the planes before it, to LDS; v keeps the rest.  A number whose lowest bit lies
 // below 2^-133, bf16's smallest subnormal, is not the sum of three parts (all others are: the rest behind two parts has eight bits at
 // most).  The rest then is an fp32 subnormal with some of its low 16 bits set, which no other third part has: `rests` collects them.
-template <int P>
+// NEG: of their negatives.
+template <int P, bool NEG = false>
 __device__ __forceinline__ void put_plane(bf16_t* to, floatx4& v, unsigned& rests) {
   typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
   if constexpr (P == 2) {
     rests |= __float_as_uint(v[0]) | __float_as_uint(v[1]);
     rests |= __float_as_uint(v[2]) | __float_as_uint(v[3]);
   }
+  if constexpr (NEG && P == 0) v = -v;
   const u32x2 u = {__builtin_bit_cast(unsigned, bf16x2{(bf16_t)v[0], (bf16_t)v[1]}), __builtin_bit_cast(unsigned, bf16x2{(bf16_t)v[2], (bf16_t)v[3]})};
   *reinterpret_cast<u32x2*>(to) = u;
   if constexpr (P < 2) {
@@ -156,8 +158,8 @@ __device__ __forceinline__ void put_plane(bf16_t* to, floatx4& v, unsigned& rest
     v[3] -= __uint_as_float(u[1] & 0xffff0000u);
   }
 }
-template <int P>
-__device__ __forceinline__ void put_plane(bf16_t* to, bf16x4& v, unsigned&) { *reinterpret_cast<bf16x4*>(to) = v; }
+template <int P, bool NEG = false>
+__device__ __forceinline__ void put_plane(bf16_t* to, bf16x4& v, unsigned&) { *reinterpret_cast<bf16x4*>(to) = NEG ? -v : v; }
 __device__ __forceinline__ bool bits_lost(unsigned rests) { return (rests & 0xffffu) != 0; }
 
 // Element offset of the four k from 4 c on of row r in a [rows][32] plane: 64-byte rows, 16-byte granules as in the stripe layout.
@@ -255,7 +257,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ggemm_split_kernel(const TA* 
     constexpr int set = decltype(set_c)::value, q = decltype(q_c)::value;
     if constexpr (q < A_PER * PA) {
       constexpr int i = q / PA, p = q % PA;
-      put_plane<p>(As[set] + p * (BM * kFK) + aswz(ar + kThreads / 8 * i, ac), ra[set][i], rests);
+      put_plane<p, set == 1>(As[set] + p * (BM * kFK) + aswz(ar + kThreads / 8 * i, ac), ra[set][i], rests);
     } else if constexpr (q < A_PER * PA + W_PER * PW) {
       constexpr int i = (q - A_PER * PA) / PW, p = (q - A_PER * PA) % PW;
       const int g = tid + kThreads * i;
@@ -281,6 +283,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ggemm_split_kernel(const TA* 
     if constexpr (W_KM) return kplane_frag<BN>(plane, lane, nb, ks);
     else return *reinterpret_cast<const bf16x8*>(plane + aswz(nb + l32, 2 * (2 * ks + h)));
   };
+  // What a bf16 MFMA adds to a sum much smaller than itself cuts off that sum's bits below its own towards minus infinity (0.12 of a last
+  // place on average; fp32 MFMAs round to nearest).  Over the steps, and over the k rows of a token, that adds up: d_x of 98 tokens, H = 536,
+  // I = 400, E = 64, k = 8, was off by 2.14e-7 where fp32 MFMAs are by 2.05e-7, of 2 experts by 1.76e-7 and 1.84e-7.  So every other step
+  // multiplies the negatives of A's rows and is subtracted.
   // Step s multiplies stage st = s % 2.  Between its MFMAs, two at a time, go the next step's planes from registers to the other stage and
   // the previous step's sums into the fp64 ones: vector instructions that would otherwise wait for the MFMA pipe and it for them.
   floatx16 acc[2][NTW];
@@ -315,7 +321,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ggemm_split_kernel(const TA* 
       constexpr int kF = (16 * NTW + kChunks - 1) / kChunks;
 #pragma unroll
       for (int f = c * kF; f < (c + 1) * kF; ++f)
-        if (f < 16 * NTW) sum[f / 16][f % 16] += (double)acc[st ^ 1][f / 16][f % 16];
+        if (f < 16 * NTW) sum[f / 16][f % 16] += (double)(st == 0 ? -acc[1][f / 16][f % 16] : acc[0][f / 16][f % 16]);
       __builtin_amdgcn_sched_barrier(0);
     };
     for_each<kChunks>(chunk);
@@ -345,25 +351,25 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ggemm_split_kernel(const TA* 
       if (s + 1 < full) turn(c1, s + 1);
       else {
 #pragma unroll
-        for (int j = 0; j < NTW; ++j) acc[1][j] = acc[0][j];
+        for (int j = 0; j < NTW; ++j) acc[1][j] = -acc[0][j];
       }
     }
   }
   auto fold = [&]() {
 #pragma unroll
-    for (int f = 0; f < 16 * NTW; ++f) sum[f / 16][f % 16] += (double)acc[1][f / 16][f % 16];
+    for (int f = 0; f < 16 * NTW; ++f) sum[f / 16][f % 16] -= (double)acc[1][f / 16][f % 16];
   };
   fold();
-  if (K % kFK != 0) {
-    load(c0, std::true_type{}, full * kFK);
-    put_all(c0);
+  if (K % kFK != 0) {                                            // (a negated step: it follows an even number of steps or the last of an odd one)
     load(c1, std::true_type{}, full * kFK);
+    put_all(c1);
+    load(c0, std::true_type{}, full * kFK);
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < NTW; ++j) acc[1][j] = none;
-    if (busy) step(c0);
+    for (int j = 0; j < NTW; ++j) acc[0][j] = none;
 #pragma unroll
-    for (int j = 0; j < NTW; ++j) acc[1][j] = acc[0][j];
+    for (int j = 0; j < NTW; ++j) acc[1][j] = none;
+    if (busy) step(c1);
     fold();
   }
   // An infinity, a NaN, a value that rounds to infinity or one with bits below 2^-133 (from 2^-110 down) has no three bf16 parts: a tile

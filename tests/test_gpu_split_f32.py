@@ -113,3 +113,14 @@ def test_small_gradients(T, H, I, E, k):
     ref = O.moe_backward(p["x"], p["w_router"], p["w_gate_up"], p["w_down"], p["theta"], idx, d)
     for name, a in zip(("x", "w_router", "w_gate_up", "w_down"), got):
         assert _rel(a, ref[name]) <= 2e-6, name
+
+
+# The mean of n independent errors of either sign lies within 5 of their root mean square / sqrt(n).  (The rows' own errors reach a result
+# through weights of either sign, so they count as independent.)  Even numbers of steps of 32: an odd one leaves the share of one step.
+@pytest.mark.parametrize("H,I", [(512, 256), (1024, 512), (64, 64)])
+@pytest.mark.parametrize("rows", [(400, 800), (2000, 2400)])
+def test_errors_have_no_sign(H, I, rows):
+    p, idx, w = _inputs(H, I, rows, 9)
+    ref = O.experts_forward(p["x"], idx, w, p["w_gate_up"], p["w_down"], p["theta"], dtype=torch.float64)
+    err = _forward(p, idx, w).double().cpu() - ref
+    assert abs(float(err.mean())) <= 5 * float(err.pow(2).mean() / err.numel()) ** 0.5
