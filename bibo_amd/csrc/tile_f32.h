@@ -514,7 +514,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void wgrad_split_kernel(const TP* 
     if constexpr (q < P_PER * PP) {
       constexpr int i = q / PP, p = q % PP;
       const int g = tid + kThreads * i;
-      put_plane<p>(Ps[set] + p * (BP * kFK) + kswz<BP>(g / (BP / 4), g % (BP / 4)), rp[set][i], rests);
+      put_plane<p, set == 1>(Ps[set] + p * (BP * kFK) + kswz<BP>(g / (BP / 4), g % (BP / 4)), rp[set][i], rests);
     } else if constexpr (q < kPuts) {
       constexpr int i = (q - P_PER * PP) / PQ, p = (q - P_PER * PP) % PQ;
       const int g = tid + kThreads * i;
@@ -522,12 +522,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void wgrad_split_kernel(const TP* 
     }
   };
   const int wm = wave % WM, wn = wave / WM, l32 = lane & 31, h = lane >> 5;
-  floatx16 acc[NTW], none;
+  // every other step's negatives in a sum of their own, for the same reason as in ggemm_split_kernel
+  floatx16 acc[2][NTW], none;
 #pragma unroll
   for (int i = 0; i < 16; ++i) none[i] = 0.f;
 #pragma unroll
-  for (int j = 0; j < NTW; ++j) acc[j] = none;
-  // as a step of ggemm_split_kernel, but into one running sum: 24 roundings a step where 32 FMAs would make 32
+  for (int j = 0; j < NTW; ++j) acc[0][j] = acc[1][j] = none;
+  // as a step of ggemm_split_kernel, but into a running sum: 24 roundings a step where 32 FMAs would make 32
   auto step = [&](auto st_c) {
     constexpr int st = decltype(st_c)::value;
     constexpr int kProducts = PP * PQ == 9 ? 6 : PP * PQ == 3 ? 3 : 1, kChunks = 2 * kProducts;
@@ -548,7 +549,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void wgrad_split_kernel(const TP* 
       constexpr int pp = PP == 3 && PQ == 3 ? (q == 0 ? 2 : q == 2 || q == 3 ? 1 : 0) : PP == 3 ? 2 - q : 0;
       constexpr int pq = PP == 3 && PQ == 3 ? (q == 1 ? 2 : q == 2 || q == 4 ? 1 : 0) : PQ == 3 ? 2 - q : 0;
 #pragma unroll
-      for (int j = 0; j < NTW; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[ks][pp], b[ks][j][pq], acc[j], 0, 0, 0);
+      for (int j = 0; j < NTW; ++j) acc[st][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[ks][pp], b[ks][j][pq], acc[st][j], 0, 0, 0);
       constexpr int kP = (kPuts + kChunks - 1) / kChunks;
       for_each<kP>([&](auto i_c) { put(integral_constant<int, st ^ 1>{}, integral_constant<int, c * kP + decltype(i_c)::value>{}); });
       __builtin_amdgcn_sched_barrier(0);
@@ -579,17 +580,19 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void wgrad_split_kernel(const TP* 
       if (s + 1 < nsteps) turn(c1, s + 1);
     }
   }
+#pragma unroll
+  for (int j = 0; j < NTW; ++j) acc[0][j] -= acc[1][j];
   if constexpr (PP + PQ > 2) {                           // numbers without three parts, as in ggemm_split_kernel
     bool finite = true;
 #pragma unroll
     for (int j = 0; j < NTW; ++j)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) finite = finite && fabsf(acc[j][i]) <= 3.402823466e38f;
+      for (int i = 0; i < 16; ++i) finite = finite && fabsf(acc[0][j][i]) <= 3.402823466e38f;
     if (__syncthreads_or(!finite || bits_lost(rests))) {
       float* const pf = reinterpret_cast<float*>(Ps);
       float* const qf = reinterpret_cast<float*>(Qs);
 #pragma unroll
-      for (int j = 0; j < NTW; ++j) acc[j] = none;
+      for (int j = 0; j < NTW; ++j) acc[0][j] = none;
       for (int r0 = lo; r0 < hi; r0 += kFK) {
         lookup(c0, r0);
         load(c0, r0);
@@ -602,8 +605,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void wgrad_split_kernel(const TP* 
         for (int k = 0; k < kFK; k += 2)
 #pragma unroll
           for (int j = 0; j < NTW; ++j)
-            acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(pf[(k + h) * BP + wm * 32 + l32], qf[(k + h) * BQ + (wn * NTW + j) * 32 + l32],
-                                                          acc[j], 0, 0, 0);
+            acc[0][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(pf[(k + h) * BP + wm * 32 + l32], qf[(k + h) * BQ + (wn * NTW + j) * 32 + l32],
+                                                             acc[0][j], 0, 0, 0);
       }
     }
   }
@@ -614,7 +617,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void wgrad_split_kernel(const TP* 
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int n = n0 + wm * 32 + acc_row(i, lane);
-        if (n < N) dW[((size_t)e * N + n) * M + m] = from_float<TOut>(acc[j][i]);
+        if (n < N) dW[((size_t)e * N + n) * M + m] = from_float<TOut>(acc[0][j][i]);
       }
     }
   }
