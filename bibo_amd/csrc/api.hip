@@ -81,6 +81,7 @@ inline bool stream_eligible(int T, int H, int E, int k, int I, int dtype, bool d
 // tiles: H = 512, I = 256, E = 64: 31 -> 31 us at 9 rows per expert with weights in the Infinity Cache, 34 -> 35 at 12 and 39 -> 36 at 18
 // from HBM; E = 32: 27 -> 31 at 12, 32 -> 30 at 20; E = 16: 28 -> 30 at 20, 36 -> 29 at 36; E = 9: 24 -> 25 at 14, 30 -> 29 at 28.
 // H = 1024, I = 512, E = 64: 63 -> 63 at 10, 69 -> 63 at 12, 80 -> 63 at 16; E = 9: 30 -> 34 at 11, 38 -> 34 at 14.
+// Those tiles hand fp32 rows to the combine, as streaming does (f32_rows); the others' are bf16.
 inline long long stream_slots(int E, int H, int I, int dtype) {
   if (H <= 512 && I <= 512) return 24 * E < 704 ? 24 * E : 704;
   return (fused_wide_supported(H, I, dtype) ? 11LL : 17LL) * E;
@@ -172,8 +173,8 @@ Workspace carve(int T, int H, int E, int k, int I, int dtype) {
   ws.yw = o;
   ws.least = o + align_up(S * (size_t)H * sizeof(float));
   ws.total = o + align_up(S * (size_t)(generic_tiles(H, I, dtype) && 2 * I > H ? 2 * I : H) * sizeof(float));
-  // fp32 pre-activations of a call whose tiles are cut by columns: behind its slot rows, which are bf16
-  ws.pre = o + align_up(S * (size_t)H * sizeof(bf16_t));
+  // fp32 pre-activations of a call whose tiles are cut by columns: behind its slot rows, fp32 where `auto` streamed before, else bf16
+  ws.pre = o + align_up(S * (size_t)H * (stream_eligible(T, H, E, k, I, dtype, true) ? sizeof(float) : sizeof(bf16_t)));
   if (dtype == BIBO_DTYPE_BF16 && mfma_supported(H, I, dtype) && split_columns(T * k, E, H, I)) {
     const size_t end = ws.pre + align_up(S * (size_t)2 * I * sizeof(float));
     if (end > ws.total) ws.total = end;
@@ -217,7 +218,8 @@ int experts_dispatch(const void* x, const void* wgu, const void* wd, const float
                      const float* w, const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token,
                      const void* residual, bool idx_trusted, int T, int H, int Eg, int np, int nn, int k, int I, int dtype,
                      int algo, int act, int flags, void* out, char* base, const Workspace& ws, size_t ws_bytes,
-                     hipStream_t s, void* preact = nullptr, const ScanArgs& scan = ScanArgs(), bool gate_up_done = false) {
+                     hipStream_t s, bool f32_rows = false, void* preact = nullptr, const ScanArgs& scan = ScanArgs(),
+                     bool gate_up_done = false) {
   float* yw = reinterpret_cast<float*>(base + ws.yw);
   CombineArgs ca;
   ca.residual = residual;
@@ -245,14 +247,16 @@ int experts_dispatch(const void* x, const void* wgu, const void* wd, const float
     void* pre = base + ws.pre;
     hipError_t e = launch_gateup_raw(x, wgu, offsets, perm_token, T, H, Eg, k, I, pre, true, true, s, scan);
     if (e != hipSuccess) return (int)e;
-    if ((e = launch_down_act(pre, wd, theta, w, offsets, perm_slot, T * k, H, Eg, I, act, yw, preact, s)) != hipSuccess) return (int)e;
-    return hip_rc(launch_combine(yw, 1, ca, T, H, k, dtype, out, s));
+    if ((e = launch_down_act(pre, wd, theta, w, offsets, perm_slot, T * k, H, Eg, I, act, yw, f32_rows, preact, s)) != hipSuccess)
+      return (int)e;
+    return hip_rc(launch_combine(yw, f32_rows ? 0 : 1, ca, T, H, k, dtype, out, s));
   }
   if (algo == BIBO_ALGO_FUSED || algo == kAlgoFusedWide) {
     if (!aligned16(x) || !aligned16(wgu) || !aligned16(wd)) return BIBO_ERR_MISALIGNED;
-    hipError_t e = launch_experts_fused(x, wgu, wd, theta, w, offsets, perm_slot, perm_token, T, H, Eg, k, I, act, yw, preact, s, scan);
+    hipError_t e = launch_experts_fused(x, wgu, wd, theta, w, offsets, perm_slot, perm_token, T, H, Eg, k, I, act, yw, f32_rows, preact, s,
+                                        scan);
     if (e != hipSuccess) return (int)e;
-    return hip_rc(launch_combine(yw, 1, ca, T, H, k, dtype, out, s));
+    return hip_rc(launch_combine(yw, f32_rows ? 0 : 1, ca, T, H, k, dtype, out, s));
   }
   // (a bf16 shape of the MFMA families that a caller asks the generic one for runs the row kernels, like the stage calls)
   if (algo == BIBO_ALGO_GENERIC && generic_tiles(H, I, dtype) && aligned16(x) && aligned16(wgu) && aligned16(wd) &&
@@ -304,7 +308,9 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
   if (norm_mode < BIBO_NORM_NONE || norm_mode > BIBO_NORM_SOFTMAX || !act_ok(sh->act)) return BIBO_ERR_UNSUPPORTED;
   int a;
   if ((rc = resolve_algo(algo, T, H, E, k, I, dtype, true, true, &a)) != BIBO_OK) return rc;
+  const int resolved = a;
   a = composite_algo(algo == BIBO_ALGO_AUTO || (state != nullptr && (sh->flags & BIBO_FLAG_TRAIN_AUTO) != 0), a, T, H, E, k, I, dtype);
+  const bool f32_rows = resolved == BIBO_ALGO_STREAM && a != BIBO_ALGO_STREAM;
   if (a == kAlgoSplit && workspace_bytes < carve(T, H, E, k, I, dtype).total) a = BIBO_ALGO_FUSED;
   if (!workspace) return BIBO_ERR_NULL_POINTER;
   if (!aligned_ws(workspace)) return BIBO_ERR_MISALIGNED;
@@ -380,7 +386,8 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
   }
   if (T == 0) return BIBO_OK;
   return experts_dispatch(x, w_gate_up, w_down, theta, idx, w, offsets, perm_slot, perm_token, residual, true, T, H, Eg,
-                          sh->n_pos, sh->n_neg, k, I, dtype, a, sh->act, sh->flags, out, base, ws, workspace_bytes, s, preact, scan, gate_up_done);
+                          sh->n_pos, sh->n_neg, k, I, dtype, a, sh->act, sh->flags, out, base, ws, workspace_bytes, s, f32_rows, preact, scan,
+                          gate_up_done);
 }
 
 
@@ -630,7 +637,7 @@ int bibo_moe_gateup_down_fwd(const void* x, const void* w_gate_up, const void* w
     return BIBO_ERR_NULL_POINTER;
   if (!aligned16(x) || !aligned16(w_gate_up) || !aligned16(w_down) || !aligned16(yw)) return BIBO_ERR_MISALIGNED;
   return hip_rc(launch_experts_fused(x, w_gate_up, w_down, theta, w, offsets, perm_slot, perm_token, T, H, E, k, I, act,
-                                     yw, nullptr, static_cast<hipStream_t>(stream)));
+                                     yw, false, nullptr, static_cast<hipStream_t>(stream)));
 }
 
 int bibo_moe_combine_fwd(const void* yw, int yw_is_bf16, int T, int H, int k, int dtype, void* out, void* stream) {
@@ -669,7 +676,9 @@ int bibo_moe_experts_fwd(const void* x, const int32_t* idx, const float* w, cons
   int a;
   // a caller's indices may repeat an expert inside a token (moe.py:46-71 accepts that)
   if ((rc = resolve_algo(algo, T, H, E, k, I, dtype, true, false, &a)) != BIBO_OK) return rc;
+  const int resolved = a;
   a = composite_algo(algo == BIBO_ALGO_AUTO, a, T, H, E, k, I, dtype);
+  const bool f32_rows = resolved == BIBO_ALGO_STREAM && a != BIBO_ALGO_STREAM;
   if (a == kAlgoSplit && workspace_bytes < carve(T, H, E, k, I, dtype).total) a = BIBO_ALGO_FUSED;
   if (!workspace) return BIBO_ERR_NULL_POINTER;
   if (!aligned_ws(workspace)) return BIBO_ERR_MISALIGNED;
@@ -691,7 +700,7 @@ int bibo_moe_experts_fwd(const void* x, const int32_t* idx, const float* w, cons
     return rc;
   if (T == 0) return BIBO_OK;
   return experts_dispatch(x, w_gate_up, w_down, theta, idx, w, offsets, perm_slot, perm_token, nullptr, false, T, H, Eg,
-                          sh->n_pos, sh->n_neg, k, I, dtype, a, sh->act, 0, out, base, ws, workspace_bytes, s);
+                          sh->n_pos, sh->n_neg, k, I, dtype, a, sh->act, 0, out, base, ws, workspace_bytes, s, f32_rows);
 }
 
 int bibo_moe_forward(const void* x, const void* w_router, const float* bias, const void* w_gate_up, const void* w_down,

@@ -265,10 +265,11 @@ hipError_t launch_gateup_raw(const void* x, const void* wgu, const int32_t* offs
 // whether a tile's columns are cut over several workgroups (launch_gateup_raw + launch_down_act instead of the fused kernel)
 bool split_columns(int S, int E, int H, int I);
 hipError_t launch_down_act(const void* gu, const void* wd, const float* theta, const float* w, const int32_t* offsets,
-                           const int32_t* perm_slot, int S, int H, int E, int I, int act, void* yw, void* preact, hipStream_t s);
+                           const int32_t* perm_slot, int S, int H, int E, int I, int act, void* yw, bool f32_rows, void* preact,
+                           hipStream_t s);
 hipError_t launch_experts_fused(const void* x, const void* wgu, const void* wd, const float* theta, const float* w,
                                 const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int T,
-                                int H, int E, int k, int I, int act, void* yw, void* preact, hipStream_t s,
+                                int H, int E, int k, int I, int act, void* yw, bool f32_rows, void* preact, hipStream_t s,
                                 const ScanArgs& scan = ScanArgs());
 bool stream_supported(int H, int I, int dtype);
 hipError_t launch_gateup_stream(const void* x, const void* wgu, const int32_t* idx, int T, int H, int E, int k, int I,

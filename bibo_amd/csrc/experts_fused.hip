@@ -133,10 +133,12 @@ __device__ __forceinline__ bf16x8 to_operand_lanes(bf16x8 v, int sel) {
 // One block of F::BN2 output columns (from column n0 on) for the first NRT 16-row tiles of a tile whose activations sit in LDS
 // (`slice(i)`: columns [128 i, 128 i + 128) of all rows), and its way out through the staging buffers O0 and O1 (moe.py:92-93).
 // wb: the first D K blocks of this wave's w_down rows, already requested; with `more`, the next column block's are on return.
+// f32_rows: the rows leave in fp32, 16-byte stores from the accumulators, 64 bytes of a row by four of them.
 template <typename F, int CT, int KB, int D, int NB, int NRT, typename Slice>
 __device__ __forceinline__ void down_block(Slice slice, WBlock<CT> (&wb)[NB], const bf16_t*& wp, size_t tile_stride, bool more, int n0,
                                            const float* w_s, const int* slot_s, int rows, bf16_t* O0, bf16_t* O1, int H,
-                                           bf16_t* __restrict__ yw) {
+                                           void* __restrict__ yw_, bool f32_rows) {
+  bf16_t* const yw = static_cast<bf16_t*>(yw_);
   constexpr int I = F::I;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int r16 = lane & 15, g4 = lane >> 4;
@@ -228,6 +230,18 @@ __device__ __forceinline__ void down_block(Slice slice, WBlock<CT> (&wb)[NB], co
     }
   };
   constexpr int NR = NRT * 16 / F::kOutRows;
+  if (f32_rows) {
+#pragma unroll
+    for (int rt = 0; rt < NRT; ++rt) {
+      const int m = rt * 16 + r16o;
+      if (m >= rows) continue;
+      const float ws = w_s[m];
+      float* const dst = static_cast<float*>(yw_) + (size_t)slot_s[m] * H + n0 + wave * (16 * CT) + 4 * g4o;
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) *reinterpret_cast<floatx4*>(dst + 16 * ct) = ws * acc2[ct][rt];
+    }
+    return;
+  }
   stage_rows(0);
 #pragma unroll
   for (int hf = 0; hf < NR; ++hf) {
@@ -258,7 +272,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
                                                             const int32_t* __restrict__ offsets,
                                                             const int32_t* __restrict__ perm_slot,
                                                             const int32_t* __restrict__ perm_token, int H, int E,
-                                                            int act, unsigned x_bytes, bf16_t* __restrict__ yw,
+                                                            int act, unsigned x_bytes, void* __restrict__ yw, int f32_rows,
                                                             bf16_t* __restrict__ preact, int column_blocks, ScanArgs scan) {
   using FT = FusedShape<NT, CT, MTP>;
   constexpr int BM = FT::BM, I = FT::I, BK = FT::BK;
@@ -675,7 +689,8 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
   // ---- phase 3: down projection, routing weight, scatter to slot order (moe.py:92-93) ----
   const int nblk = H / F::BN2;
   for (int nb = 0; nb < nblk; ++nb)
-    down_block<F, CT, KB, D, NB, 2 * kBlocks>(slice, wb, wp, tile_stride, nb + 1 < nblk, nb * F::BN2, w_s, slot_s, rows, A0, A1, H, yw);
+    down_block<F, CT, KB, D, NB, 2 * kBlocks>(slice, wb, wp, tile_stride, nb + 1 < nblk, nb * F::BN2, w_s, slot_s, rows, A0, A1, H, yw,
+                                                  MODE == 0 && SCAN <= 8 && f32_rows != 0);   // (calls of at most 24 kMaxE slots)
   };   // body
   if (MTP == 2 && nblocks == 4) body(std::integral_constant<int, 2 * MTP>{});
   else if (MTP == 2 && nblocks == 3) body(std::integral_constant<int, 2 * MTP - 1>{});
@@ -693,7 +708,7 @@ template <int NT, int CT, int MTP>
 __global__ __launch_bounds__(512) void down_act_kernel(const float* __restrict__ gu, const bf16_t* __restrict__ wd,
                                                        const float* __restrict__ theta, const float* __restrict__ w,
                                                        const int32_t* __restrict__ offsets, const int32_t* __restrict__ perm_slot,
-                                                       int H, int E, int act, bf16_t* __restrict__ yw,
+                                                       int H, int E, int act, void* __restrict__ yw, int f32_rows,
                                                        bf16_t* __restrict__ preact) {
   using F = FusedShape<NT, CT, MTP>;
   constexpr int BM = F::BM, I = F::I;
@@ -788,7 +803,7 @@ __global__ __launch_bounds__(512) void down_act_kernel(const float* __restrict__
   auto slice = [&](int i) -> const bf16_t* { return acts + i * (BM * 128); };
   auto body = [&](auto nblocks_c) {
     down_block<F, CT, KB, KB, KB, 2 * decltype(nblocks_c)::value>(slice, wb, wp, tile_stride, false, nb * F::BN2, w_s, slot_s, rows, O0,
-                                                                 O1, H, yw);
+                                                                 O1, H, yw, f32_rows != 0);
   };
   const int nblocks = (rows + 31) >> 5;
   if (MTP == 2 && nblocks == 4) body(std::integral_constant<int, 2 * MTP>{});
@@ -799,14 +814,14 @@ __global__ __launch_bounds__(512) void down_act_kernel(const float* __restrict__
 
 template <int NT>
 void launch_down_act_nt(const float* gu, const bf16_t* wd, const float* theta, const float* w, const int32_t* offsets,
-                        const int32_t* perm_slot, int S, int H, int E, int act, bf16_t* yw, bf16_t* preact,
+                        const int32_t* perm_slot, int S, int H, int E, int act, void* yw, bool f32_rows, bf16_t* preact,
                         hipStream_t s) {
   auto launch = [&](auto mt, auto ct) {
     constexpr int MT = decltype(mt)::value, CT = decltype(ct)::value;
     const int tiles = S / (64 * MT) + E < S ? S / (64 * MT) + E : S;
     const int grid = ((tiles * (H / (128 * CT)) + 7) & ~7) + 8;
     hipLaunchKernelGGL((down_act_kernel<NT, CT, MT>), dim3(grid), dim3(512), 0, s, gu, wd, theta, w, offsets, perm_slot, H, E, act, yw,
-                       preact);
+                       (int)f32_rows, preact);
   };
   // 64-row tiles while they and their column blocks leave no workgroup waiting for a CU: shorter, and more of them pull weights
   using std::integral_constant;
@@ -832,19 +847,19 @@ void scan_variant(int S, Launch launch) {
 template <int NT, int CT, int MT>
 void launch_fused_t(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const float* theta, const float* w,
                     const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int S, int H, int E,
-                    int act, unsigned x_bytes, bf16_t* yw, bf16_t* preact, const ScanArgs& scan, hipStream_t s) {
+                    int act, unsigned x_bytes, void* yw, bool f32_rows, bf16_t* preact, const ScanArgs& scan, hipStream_t s) {
   const int grid = round_tiles_most(S, E, 64 * MT);
   auto launch = [&](auto mode) {
     constexpr int MODE = decltype(mode)::value;
     if (scan.idx != nullptr) {
       scan_variant(S, [&](auto per) {
         hipLaunchKernelGGL((experts_fused_kernel<NT, CT, MODE, MT, decltype(per)::value>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta,
-                           w, nullptr, nullptr, nullptr, H, E, act, x_bytes, yw, preact, 1, scan);
+                           w, nullptr, nullptr, nullptr, H, E, act, x_bytes, yw, (int)f32_rows, preact, 1, scan);
       });
       return;
     }
     hipLaunchKernelGGL((experts_fused_kernel<NT, CT, MODE, MT>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta, w, offsets, perm_slot,
-                       perm_token, H, E, act, x_bytes, yw, preact, 1, scan);
+                       perm_token, H, E, act, x_bytes, yw, (int)f32_rows, preact, 1, scan);
   };
   if constexpr (NT < 4) {                    // (a state-keeping forward has I <= 384)
     if (preact != nullptr) {
@@ -858,10 +873,11 @@ void launch_fused_t(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const 
 template <int NT>
 void launch_fused_nt(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const float* theta, const float* w,
                      const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int S, int H, int E,
-                     int act, unsigned x_bytes, bf16_t* yw, bf16_t* preact, const ScanArgs& scan, hipStream_t s) {
+                     int act, unsigned x_bytes, void* yw, bool f32_rows, bf16_t* preact, const ScanArgs& scan, hipStream_t s) {
   constexpr int MT = NT == 4 ? 1 : 2;
   auto launch = [&](auto ct) {
-    launch_fused_t<NT, decltype(ct)::value, MT>(x, wgu, wd, theta, w, offsets, perm_slot, perm_token, S, H, E, act, x_bytes, yw, preact, scan, s);
+    launch_fused_t<NT, decltype(ct)::value, MT>(x, wgu, wd, theta, w, offsets, perm_slot, perm_token, S, H, E, act, x_bytes, yw, f32_rows,
+                                               preact, scan, s);
   };
   // (blocks of 256 columns leave room for the third x buffer of the deeper ring where I is not 384)
   if constexpr (NT != 4) {
@@ -884,13 +900,13 @@ void launch_raw_nt(const bf16_t* x, const bf16_t* wgu, const int32_t* offsets, c
     if (scan.idx != nullptr) {
       scan_variant(S, [&](auto per) {
         hipLaunchKernelGGL((experts_fused_kernel<NT, 1, MODE, MT, decltype(per)::value>), dim3(grid), dim3(512), 0, s, x, wgu, nullptr,
-                           nullptr, nullptr, nullptr, nullptr, nullptr, H, E, 0, x_bytes, nullptr, gu, column_blocks, scan);
+                           nullptr, nullptr, nullptr, nullptr, nullptr, H, E, 0, x_bytes, nullptr, 0, gu, column_blocks, scan);
       });
       return;
     }
   }
   hipLaunchKernelGGL((experts_fused_kernel<NT, 1, MODE, MT>), dim3(grid), dim3(512), 0, s, x, wgu, nullptr, nullptr, nullptr,
-                     offsets, nullptr, perm_token, H, E, 0, x_bytes, nullptr, gu, column_blocks, scan);
+                     offsets, nullptr, perm_token, H, E, 0, x_bytes, nullptr, 0, gu, column_blocks, scan);
 }
 
 }  // namespace
@@ -944,20 +960,20 @@ bool split_columns(int S, int E, int H, int I) {
   return I >= 256 && S <= 3600 && S <= hi * (46 + E) / 10 && S <= hi * hi * E / 763;
 }
 
-// gu [S, 2I] fp32 -> routing-weighted rows in slot order, and with `preact` their bf16 copy (down_act_kernel; I <= 384); shapes as
+// gu [S, 2I] fp32 -> routing-weighted rows in slot order (bf16 or, with f32_rows, fp32), and with `preact` their bf16 copy (down_act_kernel; I <= 384); shapes as
 // launch_gateup_raw takes them, I = 256 to 512
 hipError_t launch_down_act(const void* gu, const void* wd, const float* theta, const float* w, const int32_t* offsets,
-                           const int32_t* perm_slot, int S, int H, int E, int I, int act, void* yw, void* preact, hipStream_t s) {
+                           const int32_t* perm_slot, int S, int H, int E, int I, int act, void* yw, bool f32_rows, void* preact,
+                           hipStream_t s) {
   if (S == 0) return hipSuccess;
   if (I == 512 && preact != nullptr) return hipErrorInvalidValue;
   const float* gp = static_cast<const float*>(gu);
   bf16_t* pp = static_cast<bf16_t*>(preact);
   const bf16_t* dp = static_cast<const bf16_t*>(wd);
-  bf16_t* yp = static_cast<bf16_t*>(yw);
   switch (I) {
-    case 256: launch_down_act_nt<2>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yp, pp, s); break;
-    case 384: launch_down_act_nt<3>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yp, pp, s); break;
-    case 512: launch_down_act_nt<4>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yp, pp, s); break;
+    case 256: launch_down_act_nt<2>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yw, f32_rows, pp, s); break;
+    case 384: launch_down_act_nt<3>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yw, f32_rows, pp, s); break;
+    case 512: launch_down_act_nt<4>(gp, dp, theta, w, offsets, perm_slot, S, H, E, act, yw, f32_rows, pp, s); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -973,7 +989,8 @@ bool fused_wide_supported(int H, int I, int dtype) { return dtype == BIBO_DTYPE_
 
 hipError_t launch_experts_fused(const void* x, const void* wgu, const void* wd, const float* theta, const float* w,
                                 const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int T,
-                                int H, int E, int k, int I, int act, void* yw, void* preact, hipStream_t s, const ScanArgs& scan) {
+                                int H, int E, int k, int I, int act, void* yw, bool f32_rows, void* preact, hipStream_t s,
+                                const ScanArgs& scan) {
   const int S = T * k;
   if (S == 0) return hipSuccess;
   if ((unsigned long long)T * H * sizeof(bf16_t) >= (1ull << 32)) return hipErrorInvalidValue;   // 32-bit byte offsets into x
@@ -982,13 +999,12 @@ hipError_t launch_experts_fused(const void* x, const void* wgu, const void* wd, 
   const bf16_t* xp = static_cast<const bf16_t*>(x);
   const bf16_t* gp = static_cast<const bf16_t*>(wgu);
   const bf16_t* dp = static_cast<const bf16_t*>(wd);
-  bf16_t* yp = static_cast<bf16_t*>(yw);
   bf16_t* pp = static_cast<bf16_t*>(preact);
   switch (I) {
-    case 128: launch_fused_nt<1>(xp, gp, dp, theta, w, offsets, perm_slot, perm_token, S, H, E, act, xb, yp, pp, scan, s); break;
-    case 256: launch_fused_nt<2>(xp, gp, dp, theta, w, offsets, perm_slot, perm_token, S, H, E, act, xb, yp, pp, scan, s); break;
-    case 384: launch_fused_nt<3>(xp, gp, dp, theta, w, offsets, perm_slot, perm_token, S, H, E, act, xb, yp, pp, scan, s); break;
-    case 512: launch_fused_nt<4>(xp, gp, dp, theta, w, offsets, perm_slot, perm_token, S, H, E, act, xb, yp, pp, scan, s); break;
+    case 128: launch_fused_nt<1>(xp, gp, dp, theta, w, offsets, perm_slot, perm_token, S, H, E, act, xb, yw, f32_rows, pp, scan, s); break;
+    case 256: launch_fused_nt<2>(xp, gp, dp, theta, w, offsets, perm_slot, perm_token, S, H, E, act, xb, yw, f32_rows, pp, scan, s); break;
+    case 384: launch_fused_nt<3>(xp, gp, dp, theta, w, offsets, perm_slot, perm_token, S, H, E, act, xb, yw, f32_rows, pp, scan, s); break;
+    case 512: launch_fused_nt<4>(xp, gp, dp, theta, w, offsets, perm_slot, perm_token, S, H, E, act, xb, yw, f32_rows, pp, scan, s); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
