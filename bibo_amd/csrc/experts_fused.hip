@@ -946,18 +946,26 @@ hipError_t launch_gateup_raw(const void* x, const void* wgu, const int32_t* offs
 // weights then, at HBM's latency where no other tile of the expert runs beside it.  Cut (launch_gateup_raw, launch_down_act), each CU pulls a
 // part of them, the pre-activations make a round trip and every column block computes the activations again.  So the limit, in routed slots,
 // goes with the weights of an expert, H x I; with the experts, because many of them share what the chip's L2s deliver; and with few experts
-// as the square of H x I, because their tiles are short streams then that the second launch outweighs.  At I = 512 the second half's tiles
-// of 64 rows come to two rounds from about 3600 slots on.  Sum of the layer's kernels, uncut -> cut, cold weights, bf16:
-//   E = 64, k = 6: H = 768, I = 384: 60 -> 46 us at 768 slots, 61 -> 56 at 3072, 57 -> 59 at 3600; H = 512, I = 384: 47 -> 46 at 1920,
-//     46 -> 47 at 2400; H = 1024, I = 256: 56 -> 53 at 2700, 55 -> 56 at 3072; H = 512, I = 256: 36 -> 35 at 768, 36 -> 37 at 1152
-//   E = 64, k = 8, H = 1024, I = 512: 90 -> 68 at 2048, 89 -> 72 at 2800, 84 -> 86 at 3600
-//   E = 16, k = 3: H = 768, I = 384: 42 -> 32 at 192, 44 -> 43 at 1536, 44 -> 45 at 1800; H = 768, I = 256: 37 -> 33 at 384, 35 -> 36 at 576;
-//     H = 512, I = 256: 30 -> 29 at 384, 29 -> 33 at 576; H = 1024, I = 512: 59 -> 53 at 3072, 60 -> 66 at 4095
-//   E = 9, k = 2, H = 512, I = 256: 29 -> 29 at 256, 30 -> 34 at 384, 30 -> 40 at 2048
+// as the square of H x I, because their tiles are short streams then that the second launch outweighs (the divisors: where the two meet
+// up to 1.5 MB of weights an expert, and above them a line below which it pays off at every size measured).  At I = 512 the second half's tiles
+// of 64 rows come to two rounds from about 3600 slots on.  A layer replayed from a graph, cold weights, bf16, uncut -> cut, us:
+//   E = 64, k = 6: H = 768, I = 384: 58 -> 49 at 1800 slots, 58 -> 53 at 3120; H = 1024, I = 256: 53 -> 48 at 1800, 53 -> 50 at 2640;
+//     H = 768, I = 256: 45 -> 42 at 1440, 45 -> 44 at 2100; H = 512, I = 384: 43 -> 39 at 1200, 43 -> 43 at 1920; H = 512, I = 256: 34 -> 32 at
+//     780, 35 -> 35 at 1350
+//   E = 64, k = 8, H = 1024, I = 512, sum of the kernels: 90 -> 68 at 2048, 89 -> 72 at 2800, 84 -> 86 at 3600
+//   E = 32, k = 4: H = 768, I = 384: 54 -> 40 at 800, 50 -> 46 at 2000; H = 1024, I = 256: 48 -> 42 at 1200, 48 -> 46 at 1960; H = 768, I = 256:
+//     32 -> 29 at 600, 32 -> 34 at 1200; H = 512, I = 384: 31 -> 31 at 800, 31 -> 32 at 1120
+//   E = 16, k = 3: H = 768, I = 384: 38 -> 33 at 600, 38 -> 38 at 1350, 38 -> 39 at 1710; H = 1024, I = 256: 36 -> 34 at 600, 37 -> 38 at 1200; H = 768, I = 256:
+//     31 -> 29 at 384, 31 -> 31 at 576, 32 -> 33 at 750; H = 512, I = 384: 30 -> 29 at 390, 30 -> 31 at 570
+//   E = 48, k = 4, H = 512, I = 256: 26 -> 27 at 712
+//   E = 9, k = 2: H = 768, I = 384: 37 -> 33 at 400, 38 -> 36 at 600, 38 -> 38 at 880; H = 512, I = 512: 34 -> 35 at 600
+// and with larger weights, which it pays off for longer: E = 9, k = 2: H = 640, I = 512: 42 -> 37 at 1180; H = 768, I = 512: 47 -> 41 at 1700;
+//   H = 896, I = 512: 51 -> 46 at 2100, 51 -> 50 at 2300; H = 1024, I = 384: 45 -> 43 at 1700; H = 1024, I = 512: 54 -> 46 at 2300;
+//   E = 16, k = 3: H = 640, I = 512: 43 -> 38 at 1950; H = 1024, I = 384: 46 -> 48 at 2160, 48 -> 47 at 2370; H = 1024, I = 512: 62 -> 53 at 3120
 // Pre-activations in bf16 were 1 to 5 us faster and half again as far from the exact result (3.5e-3 against 2.3e-3).
 bool split_columns(int S, int E, int H, int I) {
   const long long hi = (long long)H * I / 1024;
-  return I >= 256 && S <= 3600 && S <= hi * (46 + E) / 10 && S <= hi * hi * E / 763;
+  return I >= 256 && S <= 3600 && S <= hi * (46 + E) / 10 && S <= hi * hi * E / (hi <= 256 ? 1100 : 763);
 }
 
 // gu [S, 2I] fp32 -> routing-weighted rows in slot order (bf16 or, with f32_rows, fp32), and with `preact` their bf16 copy (down_act_kernel; I <= 384); shapes as

@@ -17,9 +17,15 @@ def _rel(a, ref):
     return float((a.double().cpu() - ref.double()).abs().max() / ref.double().abs().max().clamp_min(1e-30))
 
 
-@pytest.mark.parametrize("H,I", [(128, 256), (640, 384), (768, 384), (1024, 512), (1024, 256)])
+def _with_idle_experts(rows):
+    """So many that `auto` cuts these rows at every size here: past streaming's rows per expert, within split_columns."""
+    return rows + (0,) * ((8 if sum(rows) < 300 else 16) - len(rows))
+
+
+@pytest.mark.parametrize("H,I", [(768, 256), (640, 384), (768, 384), (1024, 512), (1024, 256)])
 @pytest.mark.parametrize("rows", [(40, 1, 0, 200), (31, 32, 33, 64), (65, 128, 129, 127), (300, 0, 0, 96)])
 def test_cut_tiles(H, I, rows):
+    rows = _with_idle_experts(rows)
     E, k = len(rows), 1
     T = sum(rows)
     p = O.make_inputs(T=T, H=H, E=E, k=k, I=I, theta="normal", seed=T + H)
@@ -44,7 +50,7 @@ def test_cut_tiles_lose_no_precision(H, I):
     """Pre-activations cross memory in fp32: the same sums as the uncut kernel's registers hold, activated in the same order but
     for the sum of squares, so results differ only where that tips a rounding.  (Rounded to bf16 on the way, their 2^-9 shows up
     as 4e-3 here.)"""
-    rows = (65, 128, 129, 127)
+    rows = _with_idle_experts((65, 128, 129, 127))
     T, E = sum(rows), len(rows)
     p = O.make_inputs(T=T, H=H, E=E, k=1, I=I, theta="normal", seed=T + H)
     args = [torch.from_numpy(np.repeat(np.arange(E, dtype=np.int32), rows).reshape(T, 1)).to(DEV), torch.ones(T, 1, device=DEV),
