@@ -485,6 +485,7 @@ __global__ __launch_bounds__(256) void router_gateup_kernel(const bf16_t* __rest
     if (tid < kGran) *reinterpret_cast<bf16x8*>(xs + tid * 8) = *reinterpret_cast<const bf16x8*>(xr + tid * 8);
   }
   if (tid < kMaxE) bias_s[tid] = tid < Et ? bias[tid] : 0.f;
+  __builtin_amdgcn_s_waitcnt(0);                               // vmcnt(0): this thread's transfers of w_router have landed
   __syncthreads();
   if constexpr (kNorm) {
 #pragma unroll
