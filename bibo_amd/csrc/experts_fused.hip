@@ -24,7 +24,7 @@
 // activations already fill most of the LDS.
 // Each block of columns is scaled by the routing weight, staged through LDS 32 rows at a time (in the two x
 // buffers, which are idle by then) and scattered to slot order as 256-byte row segments.
-// A tile may hold fewer than 128 rows: make_round_tile_map chooses the height of a call's tiles by the rounds of the chip they come to, and
+// A tile may hold fewer than 128 rows: count_round_tiles chooses the height of a call's tiles by the rounds of the chip they come to, and
 // an expert's last tile takes what is left.  32-row blocks without rows are not multiplied: the kernel body exists once per number of blocks
 // (1 to 4), with the MFMAs, activations, down projection row tiles and output rounds of the missing blocks left out, and of up to two blocks
 // each M wave takes one; every wave still issues its share of the weight requests, which is most of what a tile costs.

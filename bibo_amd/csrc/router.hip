@@ -403,7 +403,7 @@ constexpr int kNormRouterMaxH = 1024, kNormGran = kNormRouterMaxH / 8 / kWave;
 
 // A token's routing with the first pass of its experts behind it, for the few-token kernels: every workgroup works out the routing of its
 // slot's token for itself and goes on to blocks of 32 rows of the slot's gate/up weights.  All of w_router (98 KB at E = 64, H = 768) comes
-// from L2 to each workgroup at once, every request on its way before the first wait, and a launch and the gap behind it are saved.  One
+// from L2 to each workgroup at once (behind a norm three of 24 go out after the first wait at H = 768), and a launch and the gap behind it are saved.  One
 // workgroup a CU at most (the LDS holds w_router), so with more slots each takes more blocks.  Kernels of a layer, router + gate/up launch
 // -> this, weights from HBM, us: H = 768, I = 384, k = 6: 16.7 -> 14.7 (T = 1), 21.1 -> 19.4 (4), 26.5 -> 25.8 (8); H = 512, I = 256:
 // 13.3 -> 10.6 (1), 18.1 -> 17.7 (8); H = 1024, I = 512, k = 8: 22.0 -> 17.4 (1), 30.8 -> 26.0 (4).  The host is through sooner too: the
@@ -525,7 +525,9 @@ __global__ __launch_bounds__(256) void router_gateup_kernel(const bf16_t* __rest
 // What the selection needs lies where the rows were: 80 KB of LDS at TOK = 32 and H = 768, so that two workgroups share a CU and one's
 // round trips pass behind the other's arithmetic (one a CU: 30.0 -> 21.7 us at T = 16384, 26.9 -> 19.9 at 12000).  RING: six chunks of
 // w_router requested behind the rows, as in router_ring_kernel (H = 512, T = 1024: 10.8 -> 9.5 us; H = 768: 12.2 -> 11.4;
-// T = 16: 9.8 -> 10.8, so not there).
+// T = 16: 9.8 -> 10.8, so not there).  The chunks arrive together, not behind the norm's arithmetic: the first use of the norm's weights,
+// registers whose loads are older, is compiled into a wait for everything, and with fp32 weights so is each later one, which then waits for
+// the stores of the row before (H = 768, T = 2049: 11.8 us, where router_ring_kernel takes 8 without the norm).
 template <int TOK>
 constexpr int kNormTail = (TOK * kRowPad + kMaxE) * (int)sizeof(float) + TOK * (int)sizeof(unsigned long long);
 
@@ -562,7 +564,7 @@ __global__ __launch_bounds__(TOK * 16) void router_norm_mfma_kernel(const bf16_t
 #pragma unroll
       for (int q = 0; q < 8; ++q) wv[u][q] = nw[c * 8 + q];
   }
-  __builtin_amdgcn_sched_barrier(0);                   // requested in front of w_router: a wait for them is none for that
+  __builtin_amdgcn_sched_barrier(0);                   // requested in front of w_router and of the rows
 
   // w_router chunk loads: thread t of instruction i fills granule i*kThreads + t = (row, position t % 16)
   const bf16_t* wsrc[kWPer];

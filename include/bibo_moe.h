@@ -82,16 +82,17 @@ enum bibo_flags {
 /* kernel family for the expert GEMMs */
 enum bibo_algo {
   BIBO_ALGO_AUTO = 0,    /* pick by shape */
-  BIBO_ALGO_GENERIC = 1, /* fp32 arithmetic, any H and I, bf16 or fp32: tiles of fp32 matrix instructions where H and I are
-                            multiples of 4 (bf16: and no MFMA tile divides them), else one workgroup per routed row */
+  BIBO_ALGO_GENERIC = 1, /* fp32 precision, any H and I, bf16 or fp32: tiles of matrix instructions (three bf16 parts per fp32 number,
+                            or fp32 ones where experts have few rows) where H and I are multiples of 4 (bf16: and no MFMA tile
+                            divides them), else one workgroup per routed row */
   BIBO_ALGO_MFMA = 2,    /* grouped bf16 MFMA tiles, one kernel per GEMM; needs bf16, H % 128 == 0 and
                             I in {128,256,384,512} */
   BIBO_ALGO_STREAM = 3,  /* weight-streaming kernels for few rows per expert (decode); bf16, H and I
                             multiples of 64 up to 1728; only the composite entry points; at most 4096 slots and
                             2048 rows per expert: T <= 2048 for bibo_moe_forward / bibo_moe_ffn_forward (a token's experts are
                             distinct), T*k <= 2048 for bibo_moe_experts_fwd (a caller's indices may repeat) */
-  BIBO_ALGO_FUSED = 4    /* both GEMMs of a 128-row tile in one kernel, activations stay in LDS; bf16,
-                            H % 128 == 0, I in {128,256,384}; only bibo_moe_experts_fwd / bibo_moe_forward */
+  BIBO_ALGO_FUSED = 4    /* both GEMMs of a tile of up to 128 rows in one kernel, activations stay in LDS; bf16,
+                            H % 128 == 0, I in {128,256,384}; only the composite entry points */
 };
 
 enum bibo_error {
@@ -129,8 +130,11 @@ const char* bibo_moe_strerror(int code);
 int bibo_moe_workspace_bytes(const bibo_moe_shape* shape, size_t* bytes);
 
 /*
- * The kernel family the composite entry points (bibo_moe_experts_fwd, bibo_moe_forward, bibo_moe_ffn_forward) run
- * for this shape when asked for `algo`: *selected is one of BIBO_ALGO_GENERIC / MFMA / STREAM / FUSED (never AUTO).
+ * The kernel family that `algo` names for this shape in the composite entry points (bibo_moe_experts_fwd, bibo_moe_forward,
+ * bibo_moe_ffn_forward): *selected is one of BIBO_ALGO_GENERIC / MFMA / STREAM / FUSED (never AUTO).  A family asked for by its
+ * name runs its own kernels.  BIBO_ALGO_AUTO may run others at that family's precision where they are faster: the few-token
+ * kernels (up to 48 slots; STREAM and GENERIC, also by name), tiles with fp32 rows behind them above 704 slots at H, I <= 512 and above 11 rows
+ * per expert at I = 512 (STREAM), tiles cut by columns (FUSED, MFMA), the fused kernel on 64-row tiles at I = 512 (MFMA).
  * Returns BIBO_ERR_UNSUPPORTED when `algo` names a family that cannot run the shape.  Host-side only; no
  * counterpart in the reference (its choice between eager and patched paths is made by the caller,
  * ablate/common/patches.py:402-417).
@@ -238,8 +242,9 @@ int bibo_moe_forward(const void* x, const void* w_router, const float* bias, con
  * Same arguments and results as bibo_moe_forward, without `workspace`: the intermediates (routing, permutation,
  * pre-activations, slot rows) live in a static device array of BIBO_MOE_STATIC_SCRATCH_BYTES that every GPU the
  * library runs on holds until the process ends.  The call allocates and frees nothing.  A shape whose
- * bibo_moe_workspace_bytes() exceeds the array is refused with BIBO_ERR_STATIC_SCRATCH before anything is
- * launched (decode-size shapes fit: T=64, H=1024, I=512 needs 2.8 MB).  All calls on one GPU share that GPU's
+ * intermediates do not fit the array is refused with BIBO_ERR_STATIC_SCRATCH before anything is
+ * launched (decode-size shapes fit: T=64, H=1024, I=512 needs 2.8 MB; kernels that want more room than a shape's others, which
+ * bibo_moe_workspace_bytes() counts in, give way to those where it is short).  All calls on one GPU share that GPU's
  * array, on whatever stream: calls that may overlap on one GPU race and must be ordered by the caller.  Nothing
  * in the array has to start at zero (every segment is written before it is read within a call), so it is
  * never cleared.  The first call on a device looks the array's address up (no stream work); make that call
