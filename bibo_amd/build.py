@@ -17,7 +17,10 @@ BUILD = HERE / "csrc" / "build"
 LIB = HERE / "libbibo_moe.so"
 NATIVE = HERE / "_native.so"
 
-SOURCES = ["router.hip", "permute.hip", "experts_generic.hip", "experts_mfma.hip", "experts_fused.hip", "experts_stream.hip", "experts_few.hip", "ffn.hip", "exp_attention.hip", "backward.hip", "backward_generic.hip", "api.hip"]
+# longest first
+SOURCES = ["experts_fused_384.hip", "experts_fused_256.hip", "experts_fused_128.hip", "experts_fused_512.hip", "backward.hip", "router.hip", "backward_generic.hip",
+           "experts_generic.hip", "experts_mfma.hip", "exp_attention.hip", "experts_stream.hip", "experts_few.hip", "ffn.hip", "permute.hip",
+           "experts_fused.hip", "api.hip"]
 
 # -packed-fp32-ops is switched off on purpose: hipcc -O3 otherwise forms v_pk_*_f32 from scalar float code.
 HIPCC_FLAGS = [

@@ -1,0 +1,13 @@
+// The launches of experts_fused_launch.h at I = 256.
+#include "experts_fused.h"
+
+namespace bibo {
+
+template void launch_fused_nt<2>(const bf16_t*, const bf16_t*, const bf16_t*, const float*, const float*, const int32_t*, const int32_t*,
+                                 const int32_t*, int, int, int, int, unsigned, void*, bool, bf16_t*, const ScanArgs&, hipStream_t);
+template void launch_raw_nt<2, 1>(const bf16_t*, const bf16_t*, const int32_t*, const int32_t*, int, int, int, unsigned, bf16_t*, int,
+                                  hipStream_t, const ScanArgs&);
+template void launch_down_act_nt<2>(const float*, const bf16_t*, const float*, const float*, const int32_t*, const int32_t*, int, int,
+                                    int, int, void*, bool, bf16_t*, hipStream_t);
+
+}  // namespace bibo
