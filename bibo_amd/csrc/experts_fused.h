@@ -233,7 +233,7 @@ __device__ __forceinline__ void down_block(Slice slice, WBlock<CT> (&wb)[NB], co
     }
   };
   constexpr int NR = NRT * 16 / F::kOutRows;
-  if (f32_rows) {
+  if (__builtin_expect(f32_rows, false)) {
 #pragma unroll
     for (int rt = 0; rt < NRT; ++rt) {
       const int m = rt * 16 + r16o;
