@@ -233,7 +233,7 @@ __device__ __forceinline__ void down_block(Slice slice, WBlock<CT> (&wb)[NB], co
     }
   };
   constexpr int NR = NRT * 16 / F::kOutRows;
-  if (__builtin_expect(f32_rows, false)) {
+  if (f32_rows) {
 #pragma unroll
     for (int rt = 0; rt < NRT; ++rt) {
       const int m = rt * 16 + r16o;
@@ -267,7 +267,7 @@ __device__ __forceinline__ void down_block(Slice slice, WBlock<CT> (&wb)[NB], co
 // I = 256, k = 6: 30.8 -> 27.5 (T = 256), 33.0 -> 29.1 (800), 38.3 -> 37.0 (2000); H = 768, I = 384: 49.9 -> 47.4, 57.3 -> 54.7,
 // 61.1 -> 60.7; nine experts, k = 2: 31.8 -> 26.5, 30.2 -> 26.6, 32.1 -> 28.4.  Beyond one round of tiles a CU would look twice: level at
 // 16,000 slots of H = 1024, I = 512.
-template <int NT, int CT, int MODE = 0, int MTP = 2, int SCAN = 0>
+template <int NT, int CT, int MODE = 0, int MTP = 2, int SCAN = 0, bool F32_ROWS = false>
 __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ wgu,
                                                             const bf16_t* __restrict__ wd,
                                                             const float* __restrict__ theta,
@@ -275,7 +275,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
                                                             const int32_t* __restrict__ offsets,
                                                             const int32_t* __restrict__ perm_slot,
                                                             const int32_t* __restrict__ perm_token, int H, int E,
-                                                            int act, unsigned x_bytes, void* __restrict__ yw, int f32_rows,
+                                                            int act, unsigned x_bytes, void* __restrict__ yw,
                                                             bf16_t* __restrict__ preact, int column_blocks, ScanArgs scan) {
   using FT = FusedShape<NT, CT, MTP>;
   constexpr int BM = FT::BM, I = FT::I, BK = FT::BK;
@@ -693,7 +693,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
   const int nblk = H / F::BN2;
   for (int nb = 0; nb < nblk; ++nb)
     down_block<F, CT, KB, D, NB, 2 * kBlocks>(slice, wb, wp, tile_stride, nb + 1 < nblk, nb * F::BN2, w_s, slot_s, rows, A0, A1, H, yw,
-                                                  MODE == 0 && SCAN <= 8 && f32_rows != 0);   // (calls of at most 24 kMaxE slots)
+                                                  F32_ROWS);
   };   // body
   if (MTP == 2 && nblocks == 4) body(std::integral_constant<int, 2 * MTP>{});
   else if (MTP == 2 && nblocks == 3) body(std::integral_constant<int, 2 * MTP - 1>{});
@@ -828,25 +828,32 @@ void launch_fused_t(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const 
                     const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int S, int H, int E,
                     int act, unsigned x_bytes, void* yw, bool f32_rows, bf16_t* preact, const ScanArgs& scan, hipStream_t s) {
   const int grid = round_tiles_most(S, E, 64 * MT);
-  auto launch = [&](auto mode) {
-    constexpr int MODE = decltype(mode)::value;
-    if (scan.idx != nullptr) {
-      scan_variant(S, [&](auto per) {
-        hipLaunchKernelGGL((experts_fused_kernel<NT, CT, MODE, MT, decltype(per)::value>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta,
-                           w, nullptr, nullptr, nullptr, H, E, act, x_bytes, yw, (int)f32_rows, preact, 1, scan);
-      });
-      return;
-    }
-    hipLaunchKernelGGL((experts_fused_kernel<NT, CT, MODE, MT>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta, w, offsets, perm_slot,
-                       perm_token, H, E, act, x_bytes, yw, (int)f32_rows, preact, 1, scan);
+  auto launch = [&](auto mode, auto f32, auto per) {
+    constexpr int MODE = decltype(mode)::value, SCAN = decltype(per)::value;
+    hipLaunchKernelGGL((experts_fused_kernel<NT, CT, MODE, MT, SCAN, decltype(f32)::value>), dim3(grid), dim3(512), 0, s, x, wgu, wd, theta,
+                       w, offsets, perm_slot, perm_token, H, E, act, x_bytes, yw, preact, 1, scan);
   };
+  const std::false_type bf16_rows;
+  const bool find = scan.idx != nullptr;
+  const std::integral_constant<int, 0> permuted;
   if constexpr (NT < 4) {                    // (a state-keeping forward has I <= 384)
     if (preact != nullptr) {
-      launch(std::integral_constant<int, 2>());
+      const std::integral_constant<int, 2> train;
+      if (find) scan_variant(S, [&](auto per) { launch(train, bf16_rows, per); });
+      else launch(train, bf16_rows, permuted);
       return;
     }
   }
-  launch(std::integral_constant<int, 0>());
+  const std::integral_constant<int, 0> forward;
+  if (f32_rows) {                            // (kernels of their own: as a branch of the usual ones it cost those 0.3 to 0.5 % at I = 512)
+    static_assert(kStreamMaxSlots <= 8 * 512, "calls that may stream fit the shortest scan");
+    if (find) launch(forward, std::true_type(), std::integral_constant<int, 8>());
+    else launch(forward, std::true_type(), permuted);
+  } else if (find) {
+    scan_variant(S, [&](auto per) { launch(forward, bf16_rows, per); });
+  } else {
+    launch(forward, bf16_rows, permuted);
+  }
 }
 
 }  // namespace
@@ -905,13 +912,13 @@ void launch_raw_nt(const bf16_t* x, const bf16_t* wgu, const int32_t* offsets, c
     if (scan.idx != nullptr) {
       scan_variant(S, [&](auto per) {
         hipLaunchKernelGGL((experts_fused_kernel<NT, 1, MODE, MT, decltype(per)::value>), dim3(grid), dim3(512), 0, s, x, wgu, nullptr,
-                           nullptr, nullptr, nullptr, nullptr, nullptr, H, E, 0, x_bytes, nullptr, 0, gu, column_blocks, scan);
+                           nullptr, nullptr, nullptr, nullptr, nullptr, H, E, 0, x_bytes, nullptr, gu, column_blocks, scan);
       });
       return;
     }
   }
   hipLaunchKernelGGL((experts_fused_kernel<NT, 1, MODE, MT>), dim3(grid), dim3(512), 0, s, x, wgu, nullptr, nullptr, nullptr,
-                     offsets, nullptr, perm_token, H, E, 0, x_bytes, nullptr, 0, gu, column_blocks, scan);
+                     offsets, nullptr, perm_token, H, E, 0, x_bytes, nullptr, gu, column_blocks, scan);
 }
 
 }  // namespace bibo

@@ -95,6 +95,7 @@ hipError_t launch_experts_fused(const void* x, const void* wgu, const void* wd, 
   if (S == 0) return hipSuccess;
   if ((unsigned long long)T * H * sizeof(bf16_t) >= (1ull << 32)) return hipErrorInvalidValue;   // 32-bit byte offsets into x
   if (I == 512 && preact != nullptr) return hipErrorInvalidValue;
+  if (f32_rows && (preact != nullptr || S > kStreamMaxSlots)) return hipErrorInvalidValue;   // compiled for calls that may stream
   const unsigned xb = (unsigned)((size_t)T * H * sizeof(bf16_t));
   const bf16_t* xp = static_cast<const bf16_t*>(x);
   const bf16_t* gp = static_cast<const bf16_t*>(wgu);
