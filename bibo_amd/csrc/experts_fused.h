@@ -70,10 +70,6 @@ __device__ __forceinline__ void dma16_buf(__amdgpu_buffer_rsrc_t rsrc, unsigned 
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void*)l, 16, voff, soff, 0, 0);
 }
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, unsigned bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);   // raw buffer, 32-bit data format
-}
-
 // What one thread needs to request a weight stage and the x rows of a K step.
 template <typename F>
 struct SubLoader {

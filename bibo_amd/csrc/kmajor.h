@@ -64,8 +64,13 @@ __device__ __forceinline__ bf16x8 kfrag_read_s(const bf16_t* sub, int off, int s
 
 // One K stage (two k16 steps) of a wave's MT x NTW tiles as a software pipeline: the fragments of the second step
 // are read while the first is multiplied, two LDS reads behind every MFMA.  read_a(s, mt) / read_b(s, j) return the
-// fragments.
-template <int MT, int NTW, typename ReadA, typename ReadB>
+// fragments.  ROW_LANES: operands swapped, a lane ends up with columns of ONE row of A; else with rows of one row of B.
+template <bool ROW_LANES>
+__device__ __forceinline__ floatx16 mfma_pair(bf16x8 a, bf16x8 b, floatx16 c) {
+  return ROW_LANES ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, a, c, 0, 0, 0) : __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+template <int MT, int NTW, bool ROW_LANES, typename ReadA, typename ReadB>
 __device__ __forceinline__ void multiply_stage(floatx16 (&acc)[MT][NTW], ReadA read_a, ReadB read_b) {
   constexpr int kSteps = kKS / 16;
   bf16x8 af[2][MT], bfr[2][NTW];
@@ -85,7 +90,7 @@ __device__ __forceinline__ void multiply_stage(floatx16 (&acc)[MT][NTW], ReadA r
     for (int j = 0; j < NTW; ++j)
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
-        acc[mt][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[s & 1][j], af[s & 1][mt], acc[mt][j], 0, 0, 0);
+        acc[mt][j] = mfma_pair<ROW_LANES>(af[s & 1][mt], bfr[s & 1][j], acc[mt][j]);
     // order for the scheduler: an MFMA, then the next two LDS reads, and so on
 #pragma unroll
     for (int i = 0; i < MT * NTW; ++i) {
@@ -99,7 +104,7 @@ __device__ __forceinline__ void multiply_stage(floatx16 (&acc)[MT][NTW], ReadA r
 // fragment, so the row operand is read one fragment ahead and only the column operand is held for a whole k16 step;
 // the column fragments of the next step are read during the first NTW pairs of this one.  kARd = LDS reads per row
 // fragment (1: a 16-byte read, 2: a pair of transposing reads).
-template <int MT, int NTW, int kARd, typename ReadA, typename ReadB>
+template <int MT, int NTW, bool ROW_LANES, int kARd, typename ReadA, typename ReadB>
 __device__ __forceinline__ void multiply_stage_tall(floatx16 (&acc)[MT][NTW], ReadA read_a, ReadB read_b) {
   constexpr int kSteps = kKS / 16, kPairs = kSteps * MT;
   static_assert(MT >= NTW, "a step's pairs carry the next step's column fragments");
@@ -115,7 +120,7 @@ __device__ __forceinline__ void multiply_stage_tall(floatx16 (&acc)[MT][NTW], Re
     if (more_b) bfr[(s + 1) & 1][mt] = read_b(s + 1, mt);
 #pragma unroll
     for (int j = 0; j < NTW; ++j)
-      acc[mt][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[s & 1][j], af[p & 1], acc[mt][j], 0, 0, 0);
+      acc[mt][j] = mfma_pair<ROW_LANES>(af[p & 1], bfr[s & 1][j], acc[mt][j]);
     if (more_a) __builtin_amdgcn_sched_group_barrier(0x100, kARd, 0);
     if (more_b) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
     __builtin_amdgcn_sched_group_barrier(0x008, NTW, 0);
@@ -228,8 +233,8 @@ __device__ __forceinline__ void dgrad_block(const Ring& ring, int* dst_s, int bl
     const bf16_t* bt = bbuf(bc);
     auto read_a = [&](int s, int mt) { return *reinterpret_cast<const bf16x8*>(at + aoff + mt * 32 * kKS + (apos0 ^ (s * 16))); };
     auto read_b = [&](int s, int j) { return kfrag_read_s(bt, boff[j], s); };
-    if constexpr (MT == 2) multiply_stage<MT, NTW>(acc, read_a, read_b);      // nstages is a multiple of 4
-    else if (stage < nstages) multiply_stage_tall<MT, NTW, 1>(acc, read_a, read_b);
+    if constexpr (MT == 2) multiply_stage<MT, NTW, true>(acc, read_a, read_b);      // nstages is a multiple of 4
+    else if (stage < nstages) multiply_stage_tall<MT, NTW, true, 1>(acc, read_a, read_b);
   };
   for (int i = 0; i < nstages; i += R) {
     step(integral_constant<int, 0>{}, i);
@@ -337,6 +342,11 @@ __device__ __forceinline__ void wgrad_plan(const int32_t* __restrict__ offsets, 
   if (lane < E) list[slots + E + lane] = int4v{first, mine, 0, 0};
 }
 
+// the neighbour's value: lanes 2 i and 2 i + 1 trade
+__device__ __forceinline__ float quad_swap(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true));
+}
+
 template <int MT, int NTW, bool GATHER_P, bool GATHER_Q>
 __device__ __forceinline__ void wgrad_block(const Ring& ring, int block, const bf16_t* __restrict__ P, const bf16_t* __restrict__ Q,
                                             const int32_t* __restrict__ index, const bf16_t* __restrict__ zrow, int N, int M, int E,
@@ -432,8 +442,8 @@ __device__ __forceinline__ void wgrad_block(const Ring& ring, int block, const b
         const bf16_t* qt = qbuf(bc);
         auto read_p = [&](int s, int mt) { return kfrag_read_s(pt, poff[mt], s); };
         auto read_q = [&](int s, int j) { return kfrag_read_s(qt, qoff[j], s); };
-        if constexpr (MT == 2) multiply_stage<MT, NTW>(acc, read_p, read_q);
-        else multiply_stage_tall<MT, NTW, 2>(acc, read_p, read_q);
+        if constexpr (MT == 2) multiply_stage<MT, NTW, false>(acc, read_p, read_q);
+        else multiply_stage_tall<MT, NTW, false, 2>(acc, read_p, read_q);
       }
     };
     for (int i = 0; i < nstages; i += R) {
@@ -444,35 +454,41 @@ __device__ __forceinline__ void wgrad_block(const Ring& ring, int block, const b
     }
     __builtin_amdgcn_s_waitcnt(0);       // the repeated requests of the last steps land before the workgroup ends
   }
-  // accumulators transposed: lane = row n0 + wm MT 32 + 32 mt + lane % 32, register 4 q + r = column
-  // m0 + (wn NTW + j) 32 + 8 q + 4 (lane / 32) + r
+  // lane = column m0 + (wn NTW + j) 32 + lane % 32, register 4 q + r = row n0 + (wm MT + mt) 32 + 8 q + 4 (lane / 32) + r: a store's 32
+  // lanes leave 128 contiguous bytes of a row in fp32, and in bf16 (lane pairs trade the odd row of one for the even row of the other, two
+  // columns a lane) 64.  With a lane per row, 16 bytes of each in a store, XXX.
   const int n = lane & 31, hh = lane >> 5;
-  const size_t oofs = ((size_t)n0 + wm * MT * 32 + n) * M + m0 + wn * NTW * 32 + 4 * hh;
+  const unsigned row = n0 + wm * MT * 32 + 4 * hh, col = m0 + wn * NTW * 32 + n;
   if (e_chunks == 1 && !f32) {
-    bf16_t* orow = static_cast<bf16_t*>(dW) + (size_t)e * N * M + oofs;
+    const __amdgpu_buffer_rsrc_t dst = make_rsrc(uniform(static_cast<bf16_t*>(dW) + (size_t)e * N * M), (unsigned)N * M * sizeof(bf16_t));
+    const bool odd = n & 1;
+    const unsigned voff = ((row + odd) * M + (col & ~1u)) * sizeof(bf16_t);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int j = 0; j < NTW; ++j)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          bf16x4 v;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] = (bf16_t)acc[mt][j][4 * q + r];
-          *reinterpret_cast<bf16x4*>(orow + (size_t)mt * 32 * M + j * 32 + 8 * q) = v;
+        for (int i = 0; i < 16; i += 2) {
+          const float lo = acc[mt][j][i], hi2 = acc[mt][j][i + 1];
+          const float got = quad_swap(odd ? lo : hi2);
+          typedef bf16_t bf16x2 __attribute__((ext_vector_type(2)));
+          const bf16x2 v = {(bf16_t)(odd ? got : lo), (bf16_t)(odd ? hi2 : got)};
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), dst, voff,
+                                                ((mt * 32 + 8 * (i >> 2) + (i & 3)) * M + j * 32) * (unsigned)sizeof(bf16_t), 0);
         }
   } else {
-    float* prow = (e_chunks == 1 ? static_cast<float*>(dW) + (size_t)e * N * M : part + (size_t)cg * N * M) + oofs;
+    float* const base = e_chunks == 1 ? static_cast<float*>(dW) + (size_t)e * N * M : part + (size_t)cg * N * M;
+    const __amdgpu_buffer_rsrc_t dst = make_rsrc(uniform(base), (unsigned)N * M * sizeof(float));
+    const unsigned voff = (row * M + col) * sizeof(float);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int j = 0; j < NTW; ++j)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          floatx4 v;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] = acc[mt][j][4 * q + r];
-          *reinterpret_cast<floatx4*>(prow + (size_t)mt * 32 * M + j * 32 + 8 * q) = v;
+        for (int i = 0; i < 16; ++i) {
+          const float v = acc[mt][j][i];         // (a bit_cast of the element itself reads element 0)
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), dst, voff,
+                                                ((mt * 32 + 8 * (i >> 2) + (i & 3)) * M + j * 32) * (unsigned)sizeof(float), 0);
         }
   }
 }

@@ -100,6 +100,18 @@ __device__ __forceinline__ void dma16(const bf16_t* g, bf16_t* l) {
   __builtin_amdgcn_global_load_lds((gbl_void*)g, (lds_void*)l, 16, 0, 0);
 }
 
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);   // raw buffer, 32-bit data format
+}
+
+// a pointer that is the same in every lane, in scalar registers
+template <typename T>
+__device__ __forceinline__ T* uniform(T* p) {
+  const unsigned long long a = (unsigned long long)p;
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)a), hi = __builtin_amdgcn_readfirstlane((unsigned)(a >> 32));
+  return (T*)((unsigned long long)hi << 32 | lo);
+}
+
 // WM waves along M (each MT 32-row tiles) x 4 waves along N (each NTW 32-column tiles).
 template <int MT, int NTW, int WM, int BK_ = kBK>
 struct Stripe {
