@@ -9,7 +9,7 @@
 //     dx_t += W_gate_up[e]^T [dg, du]  (grouped GEMM over the TRANSPOSED gate/up weights)
 //     dW_down[e] += (w d_t) h^T,  dW_gate_up[e] += [dg, du] x_t^T   (grouped GEMMs that contract over an expert's rows)
 //     dlogit from dw (router.py:41-47), dW_router += dlogit^T x, dx += dlogit W_router.
-// Every GEMM here runs on LDS-DMA stages and 32x32x16 MFMAs.  The pre-activations are recomputed with the forward's
+// Every GEMM here runs on LDS-DMA stages and MFMAs.  The pre-activations are recomputed with the forward's
 // operand layout (both operands contiguous along the contraction).  The input gradients contract over the middle
 // dimension of the weight tensors and the weight gradients over the ROWS of row-major activations: those operands go
 // to LDS as they lie in memory and are read through transposing LDS reads (kmajor.h), so nothing is transposed in
@@ -172,13 +172,17 @@ inline int sub_tiles(int n) { return n % 384 == 0 ? 3 : n % 256 == 0 ? 2 : 1; }
 // dx of every slot and both weight gradients (kmajor.h: backward_gemms_kernel).  256-row tiles, which stream the other operand half as
 // often and take 1.75 times as long, where the experts hold 192 rows on average and the launch is several rounds of workgroups, whose last
 // one the three products share.
-hipError_t launch_backward_gemms(BackwardGemms g, int S, int slots, hipStream_t s) {
+// Tall launches address rows by 32-bit offsets (kmajor.h: SMALL): from the first token of x and d_out, from the first row of a chunk in the
+// others.
+hipError_t launch_backward_gemms(BackwardGemms g, int T, int S, int chunk, int slots, hipStream_t s) {
   const int H = g.H, I = g.I, E = g.E, nh = sub_tiles(H), ni = sub_tiles(I), bh = kSubW * nh, bi = kSubW * ni;
   auto pad8 = [](long long n) { return (int)((n + 7) & ~7ll); };
   auto dx = [&](int rows) { return ((long long)S / rows + E) * (H / bh); };
   auto gu = [&](int rows) { return (long long)slots * (2 * I / rows) * (H / bh); };
   auto down = [&](int rows) { return (long long)slots * (H / rows) * (I / bi); };
-  const bool tall = (long long)S >= 192ll * E && dx(128) + gu(128) + down(128) > 3 * kCUs;
+  const long long widest = (long long)sizeof(bf16_t) * (H > 2 * I ? H : 2 * I);
+  const bool near = T * widest < kNoRow && chunk * widest < kNoRow;
+  const bool tall = near && (long long)S >= 192ll * E && dx(128) + gu(128) + down(128) > 3 * kCUs;
   g.tall_dx = tall;
   g.tall_gu = tall && 2 * I % 256 == 0;
   g.tall_d = tall && H % 256 == 0;
@@ -582,7 +586,7 @@ hipError_t launch_backward(const void* x, const void* d_out, const void* w_route
   float* part_gu = b.wgrad_part + (size_t)slots * H * I;
   BackwardGemms gemms{xp, dop, dgu, hidden, wgup, zrow, offsets, perm_slot, perm_token, b.wgrad_plan, dxs, d_wgu, d_wd, part_gu,
                       b.wgrad_part, H, I, E, grad_f32, 0, 0, false, false, false};
-  if ((err = launch_backward_gemms(gemms, S, slots, s)) != hipSuccess) return err;
+  if ((err = launch_backward_gemms(gemms, T, S, backward_chunk_rows(S, Et), slots, s)) != hipSuccess) return err;
   const bool with_router = w_router != nullptr;      // else: the experts alone, the caller owns the routing
   const int parts = (H / 8 + kWave - 1) / kWave;     // runs of columns a lane each
   auto token_bwd = [&](auto kc) {

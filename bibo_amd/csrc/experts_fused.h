@@ -64,12 +64,6 @@ struct FusedShape {
   static_assert(MT == 2 ? NT <= 3 : NT <= 4, "accumulators and activations of a tile");
 };
 
-// LDS-DMA through a buffer descriptor: the address is descriptor base + 32-bit per-thread byte offset (one
-// vector register) + a wave-uniform byte offset (scalar), so the loop keeps no 64-bit per-thread addresses.
-__device__ __forceinline__ void dma16_buf(__amdgpu_buffer_rsrc_t rsrc, unsigned voff, unsigned soff, bf16_t* l) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void*)l, 16, voff, soff, 0, 0);
-}
-
 // What one thread needs to request a weight stage and the x rows of a K step.
 template <typename F>
 struct SubLoader {

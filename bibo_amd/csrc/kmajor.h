@@ -36,96 +36,89 @@ __device__ __forceinline__ void kfill_subtile(const bf16_t* row, bf16_t* sub) {
   dma16(row, sub + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * 64 * 8);
 }
 
-// Per-lane element offset, inside a sub-tile, of the first transposed read of the 32 (n) x 16 (k) fragment whose
-// first column is nbase (a multiple of 32): k16 step s and half ks add (16 s + 4 ks) * kSubW elements.
+// Per-lane element offset, inside a sub-tile, of the first transposed read of the 16 (n) x 32 (k) fragment whose first column is
+// nbase (a multiple of 16): the four k behind those it hands a lane are 4 * kSubW elements on.
 __device__ __forceinline__ int kfrag_offset(int lane, int nbase) {
-  const int r = lane & 15, g16 = lane >> 4;
-  const int kg = g16 >> 1, nblk = g16 & 1;
-  const int krow = 8 * kg + (r >> 2);
-  const int n = nbase + 16 * nblk + 4 * (r & 3);
-  const int pos = (n >> 3) ^ ((r >> 2) << 2);                  // (k & 3) == r / 4 for every read of the fragment
+  const int r = lane & 15, krow = 8 * (lane >> 4) + (r >> 2);
+  const int n = nbase + 4 * (r & 3);
+  const int pos = (n >> 3) ^ ((r >> 2) << 2);                  // (k & 3) == r / 4 for both reads of the fragment
   return krow * kSubW + pos * 8 + (n & 4);
 }
 
-// The fragment of k16 step S: lane (n = lane % 32, kg = lane / 32) gets k = 16 S + 8 kg .. + 8 of column nbase + n.
-template <int S>
+// The fragment of a stage: lane (n = lane % 16, g = lane / 16) gets k = 8 g .. + 8 of column nbase + n.
 __device__ __forceinline__ bf16x8 kfrag_read(const bf16_t* sub, int off) {
-  const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(sub + off + (16 * S) * kSubW));
-  const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(sub + off + (16 * S + 4) * kSubW));
+  const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(sub + off));
+  const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(sub + off + 4 * kSubW));
   typedef short v8i16 __attribute__((ext_vector_type(8)));
   const v8i16 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
   return __builtin_bit_cast(bf16x8, v);
 }
 
-// the same with the step as a loop variable of an unrolled loop (folds to one of the two)
-__device__ __forceinline__ bf16x8 kfrag_read_s(const bf16_t* sub, int off, int s) {
-  return s == 0 ? kfrag_read<0>(sub, off) : kfrag_read<1>(sub, off);
-}
-
-// One K stage (two k16 steps) of a wave's MT x NTW tiles as a software pipeline: the fragments of the second step
-// are read while the first is multiplied, two LDS reads behind every MFMA.  read_a(s, mt) / read_b(s, j) return the
-// fragments.  ROW_LANES: operands swapped, a lane ends up with columns of ONE row of A; else with rows of one row of B.
+// 16 x 16 x 32 and not 32 x 32 x 16: the chip's clock gives way to the power of its matrix pipes, and on operands that are not zeros a loop of
+// nothing but the one runs at 1.97 GHz (2.0 PFLOP/s), of the other at 1.75 (1.78).  ROW_LANES: operands swapped, a lane ends up with columns of ONE row of A; else with rows of one row of B.
 template <bool ROW_LANES>
-__device__ __forceinline__ floatx16 mfma_pair(bf16x8 a, bf16x8 b, floatx16 c) {
-  return ROW_LANES ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, a, c, 0, 0, 0) : __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+__device__ __forceinline__ floatx4 mfma_pair(bf16x8 a, bf16x8 b, floatx4 c) {
+  return ROW_LANES ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a, c, 0, 0, 0) : __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-template <int MT, int NTW, bool ROW_LANES, typename ReadA, typename ReadB>
-__device__ __forceinline__ void multiply_stage(floatx16 (&acc)[MT][NTW], ReadA read_a, ReadB read_b) {
-  constexpr int kSteps = kKS / 16;
-  bf16x8 af[2][MT], bfr[2][NTW];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) af[0][mt] = read_a(0, mt);
-#pragma unroll
-  for (int j = 0; j < NTW; ++j) bfr[0][j] = read_b(0, j);
-#pragma unroll
-  for (int s = 0; s < kSteps; ++s) {
-    if (s + 1 < kSteps) {
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) af[(s + 1) & 1][mt] = read_a(s + 1, mt);
-#pragma unroll
-      for (int j = 0; j < NTW; ++j) bfr[(s + 1) & 1][j] = read_b(s + 1, j);
-    }
-#pragma unroll
-    for (int j = 0; j < NTW; ++j)
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-        acc[mt][j] = mfma_pair<ROW_LANES>(af[s & 1][mt], bfr[s & 1][j], acc[mt][j]);
-    // order for the scheduler: an MFMA, then the next two LDS reads, and so on
-#pragma unroll
-    for (int i = 0; i < MT * NTW; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      if (s + 1 < kSteps) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-    }
-  }
-}
+// The multiplication of a wave's RT x CT tiles of 16 x 16 as one software pipeline over the row tiles of ALL stages (a stage is one MFMA
+// deep): a row fragment is read two row tiles ahead of its MFMAs, the column fragments are held for the whole stage, and in its last row
+// tile the next stage's take their places one by one behind their last MFMAs.  Two row tiles before a stage ends every row fragment of
+// it has been read and its column fragments are held, so that is where the waves meet (`meet`: the next stage has landed, the one just
+// read may be filled again), and 2 CT MFMAs run while the next stage's first fragments are on their way.  The order is pinned: left to
+// itself the compiler reads a fragment into the registers of the last one and waits for it on the spot.  The loop over a ring's stages has
+// no other way in or out of its middle, because where two ways meet the compiler waits for every transfer before the next LDS read.
+// T = 8192, H = 768, I = 384, E = 64, k = 6: dh' 41.0 -> 35.0 us (pinned order 40.0, with these MFMAs 37.0), backward_gemms_kernel 195 -> 163.
+template <int RT, int CT, bool ROW_LANES>
+struct StagePipe {
+  static constexpr int NA = RT % 3 == 2 ? 3 : 4;           // row fragments in flight; divides the row tiles of a ring
+  bf16x8 af[NA], bfr[CT];
 
-// The same for a tall tile (MT = 4 row tiles per wave): 192 accumulator registers leave no room for two sets of every
-// fragment, so the row operand is read one fragment ahead and only the column operand is held for a whole k16 step;
-// the column fragments of the next step are read during the first NTW pairs of this one.  kARd = LDS reads per row
-// fragment (1: a 16-byte read, 2: a pair of transposing reads).
-template <int MT, int NTW, bool ROW_LANES, int kARd, typename ReadA, typename ReadB>
-__device__ __forceinline__ void multiply_stage_tall(floatx16 (&acc)[MT][NTW], ReadA read_a, ReadB read_b) {
-  constexpr int kSteps = kKS / 16, kPairs = kSteps * MT;
-  static_assert(MT >= NTW, "a step's pairs carry the next step's column fragments");
-  bf16x8 af[2], bfr[2][NTW];
+  template <typename ReadA, typename ReadB>
+  __device__ __forceinline__ void begin(ReadA read_a, ReadB read_b) {
 #pragma unroll
-  for (int j = 0; j < NTW; ++j) bfr[0][j] = read_b(0, j);
-  af[0] = read_a(0, 0);
-#pragma unroll
-  for (int p = 0; p < kPairs; ++p) {
-    const int s = p / MT, mt = p % MT;
-    const bool more_a = p + 1 < kPairs, more_b = s + 1 < kSteps && mt < NTW;
-    if (more_a) af[(p + 1) & 1] = read_a((p + 1) / MT, (p + 1) % MT);
-    if (more_b) bfr[(s + 1) & 1][mt] = read_b(s + 1, mt);
-#pragma unroll
-    for (int j = 0; j < NTW; ++j)
-      acc[mt][j] = mfma_pair<ROW_LANES>(af[p & 1], bfr[s & 1][j], acc[mt][j]);
-    if (more_a) __builtin_amdgcn_sched_group_barrier(0x100, kARd, 0);
-    if (more_b) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-    __builtin_amdgcn_sched_group_barrier(0x008, NTW, 0);
+    for (int j = 0; j < CT; ++j) bfr[j] = read_b(j);
+    af[0] = read_a(0);
+    af[1] = read_a(1);
+    __builtin_amdgcn_sched_barrier(0);
   }
-}
+  // Transfer q of a refill is issued q row tiles behind the meeting that allows it, the last ones together where a stage has fewer.
+  static constexpr int slot(int q) { return q < RT ? q : RT - 1; }
+  // FIRST: running number of the stage's first row tile, mod NA.  refill(q): transfer q into the buffer of this stage;
+  // refill_before(q): of the stage before.
+  template <int FIRST, int OPS, typename Meet, typename ReadA, typename NextA, typename NextB, typename Refill, typename Before>
+  __device__ __forceinline__ void stage(floatx4 (&acc)[RT][CT], Meet meet, ReadA read_a, NextA next_a, NextB next_b, Refill refill,
+                                        Before refill_before) {
+#pragma unroll
+    for (int p = 0; p < RT; ++p) {
+      if (p == RT - 2) {
+        meet();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      af[(FIRST + p + 2) % NA] = p < RT - 2 ? read_a(p + 2) : next_a(p + 2 - RT);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < CT; ++j) {
+        acc[p][j] = mfma_pair<ROW_LANES>(af[(FIRST + p) % NA], bfr[j], acc[p][j]);
+        if (p == RT - 1) {
+          __builtin_amdgcn_sched_barrier(0);
+          bfr[j] = next_b(j);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (j == 0) {
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int q = 0; q < OPS; ++q) {
+            if (slot(q) != (p + 2) % RT) continue;
+            if (p >= RT - 2) refill(q); else refill_before(q);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+};
 
 // Row-major operand tile [128 rows][32 k] in the stripe layout for 64-byte rows (granule c of row r at
 // c ^ ((r >> 2) & 3)): thread t of the fill writes row t / 4, position t % 4.  `row` = that row's K extent, already
@@ -135,11 +128,11 @@ __device__ __forceinline__ void afill(const bf16_t* row, bf16_t* tile) {
   dma16(row, tile + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * 64 * 8);
 }
 
-// The stages form a ring of four, each a __shared__ variable of its own (the compiler orders an LDS-DMA transfer
-// against later reads of the same variable with a full wait).  Step i of the K loop waits until the transfers of
-// stage i have landed (those of stages i + 1 and i + 2 may stay in flight: loads complete in order), meets the other
-// waves, requests stage i + 3 into the buffer stage i - 1 was read from, and multiplies stage i.  Every step issues
-// the same number of transfers (a request past the last stage repeats the last one), so the wait count is a constant.
+// The stages form a ring, each a __shared__ variable of its own (the compiler orders an LDS-DMA transfer against later reads of the same
+// variable with a full wait).  Where the waves meet in stage i (StagePipe), the transfers of stage i + 1 have landed, those of the R - 2
+// stages behind it may stay in flight (loads complete in order), and stage i + R is requested into the buffer that stage i has just been
+// read from.  Every stage issues the same number of transfers (a request past the last stage repeats the last one), so the wait count is a
+// constant.
 
 // The stages of a ring, a row operand's and a column operand's each, as a kernel declares them; the fourth ones only for rings of four.
 struct Ring {
@@ -150,10 +143,11 @@ struct Ring {
 
 // ---- input gradients: out[dst(r), n] = sum_k A[src(r), k] W[e][k, n] for the rows r of expert e ----------------
 // A row-major (K contiguous), W K-major as stored: [K, N] per expert.  src(r) = a_index[r] (GATHER) or r; dst(r) =
-// out_index[r] (SCATTER) or r.  Workgroup = 64 MT rows x 128 NTW columns, 2 x 4 waves, 32x32x16 MFMA, operands swapped
+// out_index[r] (SCATTER) or r.  Workgroup = 64 MT rows x 128 NTW columns, 2 x 4 waves, 16x16x32 MFMA, operands swapped
 // so that a lane owns one output row.  K is a multiple of 128.  MT = 2: 128-row tiles, ring of four stages.  MT = 4:
 // 256-row tiles for experts with many rows - an expert's weights then pass through LDS once per 256 rows instead of
-// once per 128, which is what these kernels are bound by; 192 accumulator registers and 40 KB stages, ring of three.
+// once per 128; 192 accumulator registers and 40 KB stages, ring of three.  With the transfers or the LDS reads left out the tall tiles are
+// 10 % faster, with neither (MFMAs alone) 14 %: they are bound by the matrix pipes at the clock these leave.
 template <int MT, int NTW, bool GATHER, bool SCATTER>
 __device__ __forceinline__ void dgrad_block(const Ring& ring, int* dst_s, int block, const bf16_t* __restrict__ A,
                                             const int32_t* __restrict__ a_index, const bf16_t* __restrict__ W,
@@ -191,62 +185,73 @@ __device__ __forceinline__ void dgrad_block(const Ring& ring, int* dst_s, int bl
   const int nstages = K / kKS;
   auto abuf = [&](auto bc) -> bf16_t* { return ring.template a<decltype(bc)::value>(); };
   auto bbuf = [&](auto bc) -> bf16_t* { return ring.template b<decltype(bc)::value>(); };
-  auto fill = [&](auto bc, int stage) {
+  // transfer q of a stage into buffer bc
+  auto fill = [&](auto bc, int stage, int q) {
     const int k0 = min(stage, nstages - 1) * kKS;
-#pragma unroll
-    for (int hb = 0; hb < kAOps; ++hb) afill(arow[hb] + k0, abuf(bc) + hb * kATile);
-    const bf16_t* w0 = wrow + (size_t)k0 * N;
-#pragma unroll
-    for (int j = 0; j < NTW; ++j) kfill_subtile(w0 + j * kSubW, bbuf(bc) + j * kSubElems);
+    if (q < kAOps) afill(arow[q] + k0, abuf(bc) + q * kATile);
+    else kfill_subtile(wrow + (size_t)k0 * N + (q - kAOps) * kSubW, bbuf(bc) + (q - kAOps) * kSubElems);
   };
   using std::integral_constant;
-  fill(integral_constant<int, 0>{}, 0);
-  fill(integral_constant<int, 1>{}, 1);
-  if constexpr (R == 4) fill(integral_constant<int, 2>{}, 2);
+  auto fill_all = [&](auto bc, int stage) {
+#pragma unroll
+    for (int q = 0; q < kOps; ++q) fill(bc, stage, q);
+  };
+  fill_all(integral_constant<int, 0>{}, 0);
+  fill_all(integral_constant<int, 1>{}, 1);
+  if constexpr (R == 4) fill_all(integral_constant<int, 2>{}, 2);
+  constexpr int kFirst = 2;                               // transfers that stage 0 does not issue for the one before it
+#pragma unroll
+  for (int q = 0; q < kFirst; ++q) fill(integral_constant<int, R - 1>{}, R - 1, q);
 
-  floatx16 acc[MT][NTW];
+  constexpr int RT = 2 * MT, CT = 2 * NTW;                // a wave's tiles of 16 x 16
+  floatx4 acc[RT][CT];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
+  for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int j = 0; j < NTW; ++j)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[mt][j][i] = 0.f;
+    for (int j = 0; j < CT; ++j) acc[rt][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  // fragment side.  A: lane (n, h) reads logical granule 2 s + h of row mbase + 32 mt + n.  W: wave wn's tile j is
-  // columns (wn NTW + j) 32 of the block = sub-tile (wn NTW + j) / 4, column ((wn NTW + j) % 4) 32 inside it.
-  const int n = lane & 31, h = lane >> 5;
+  // fragment side.  A: lane (n, g) reads granule g of row mbase + 16 rt + n.  W: wave wn's tile j is columns (wn CT + j) 16 of the block =
+  // sub-tile (wn CT + j) / 8, column ((wn CT + j) % 8) 16 inside it.
+  const int n = lane & 15, g4 = lane >> 4;
   const int mbase = wm * MT * 32;
-  const int apos0 = (h ^ ((n >> 2) & 3)) * 8;
-  const int aoff = (mbase + n) * kKS;
-  int boff[NTW];
+  const int aoff = (mbase + n) * kKS + (g4 ^ ((n >> 2) & 3)) * 8;
+  int boff[CT / 2];                                        // of the even tiles: an odd one is 16 elements on
 #pragma unroll
-  for (int j = 0; j < NTW; ++j) {
-    const int t32 = wn * NTW + j;
-    boff[j] = (t32 >> 2) * kSubElems + kfrag_offset(lane, (t32 & 3) * 32);
+  for (int t = 0; t < CT / 2; ++t) {
+    const int t16 = wn * CT + 2 * t;
+    boff[t] = (t16 >> 3) * kSubElems + kfrag_offset(lane, (t16 & 7) * 16);
   }
-  // step `stage` reads buffer stage % R and requests stage + R - 1 into the buffer stage - 1 was read from
+  auto read_a = [&](auto bc, int rt) { return *reinterpret_cast<const bf16x8*>(abuf(bc) + aoff + rt * 16 * kKS); };
+  auto read_b = [&](auto bc, int j) { return kfrag_read(bbuf(bc) + (j & 1) * 16, boff[j >> 1]); };
+  using Pipe = StagePipe<RT, CT, true>;
+  Pipe pipe;
+  sync_keep_loads<(R - 2) * kOps + kFirst>();
+  {
+    const integral_constant<int, 0> b0;
+    pipe.begin([&](int rt) { return read_a(b0, rt); }, [&](int j) { return read_b(b0, j); });
+  }
   auto step = [&](auto bc, int stage) {
     constexpr int b = decltype(bc)::value;
-    sync_keep_loads<(R - 2) * kOps>();
-    fill(integral_constant<int, (b + R - 1) % R>{}, stage + R - 1);
-    const bf16_t* at = abuf(bc);
-    const bf16_t* bt = bbuf(bc);
-    auto read_a = [&](int s, int mt) { return *reinterpret_cast<const bf16x8*>(at + aoff + mt * 32 * kKS + (apos0 ^ (s * 16))); };
-    auto read_b = [&](int s, int j) { return kfrag_read_s(bt, boff[j], s); };
-    if constexpr (MT == 2) multiply_stage<MT, NTW, true>(acc, read_a, read_b);      // nstages is a multiple of 4
-    else if (stage < nstages) multiply_stage_tall<MT, NTW, true, 1>(acc, read_a, read_b);
+    const integral_constant<int, (b + 1) % R> nc;
+    const integral_constant<int, (b + R - 1) % R> pc;
+    pipe.template stage<b * RT % Pipe::NA, kOps>(
+        acc, [&]() { sync_keep_loads<(R - 2) * kOps>(); }, [&](int rt) { return read_a(bc, rt); }, [&](int rt) { return read_a(nc, rt); },
+        [&](int j) { return read_b(nc, j); }, [&](int q) { fill(bc, stage + R, q); }, [&](int q) { fill(pc, stage + R - 1, q); });
   };
-  for (int i = 0; i < nstages; i += R) {
+  int i = 0;
+  for (; i + R <= nstages; i += R) {
     step(integral_constant<int, 0>{}, i);
     step(integral_constant<int, 1>{}, i + 1);
     step(integral_constant<int, 2>{}, i + 2);
     if constexpr (R == 4) step(integral_constant<int, 3>{}, i + 3);
   }
+  if (i < nstages) step(integral_constant<int, 0>{}, i);
+  if (i + 1 < nstages) step(integral_constant<int, 1>{}, i + 1);
+  if constexpr (R == 4) if (i + 2 < nstages) step(integral_constant<int, 2>{}, i + 2);
   wait_loads_and_sync();                 // the repeated requests of the last steps have landed; every wave is done reading
 
   // Epilogue (accumulators transposed: lane = row, four consecutive columns per register quad): 32 rows at a time
   // through a wave-private LDS tile, out as 16-byte row segments.
-  const int hh = lane >> 5;
   constexpr int kOutCols = NTW * 32;
   constexpr int kOutStride = kOutCols + 8;          // +16 bytes staggers the rows over the banks
   static_assert(3 * 32 * kOutStride <= NTW * kSubElems, "output staging does not fit a weight stage");
@@ -258,13 +263,13 @@ __device__ __forceinline__ void dgrad_block(const Ring& ring, int* dst_s, int bl
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
-    for (int j = 0; j < NTW; ++j)
+    for (int j = 0; j < CT; ++j)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
+      for (int q = 0; q < 2; ++q) {
         bf16x4 hv;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) hv[r] = (bf16_t)acc[mt][j][4 * q + r];
-        *reinterpret_cast<bf16x4*>(otile + n * kOutStride + j * 32 + 8 * q + 4 * hh) = hv;
+        for (int r = 0; r < 4; ++r) hv[r] = (bf16_t)acc[2 * mt + q][j][r];
+        *reinterpret_cast<bf16x4*>(otile + (16 * q + n) * kOutStride + j * 16 + 4 * g4) = hv;
       }
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
     __builtin_amdgcn_wave_barrier();
@@ -280,6 +285,10 @@ __device__ __forceinline__ void dgrad_block(const Ring& ring, int* dst_s, int bl
   }
 }
 
+// The compiler lays LDS variables out by alignment: the row operand's stages come first, so that their addresses fit the 16-bit offset of a
+// read and need no registers of their own.
+constexpr int kLowLds = 1024;
+
 // Elements of a stage's row and column operand.
 constexpr int ring_a(int MT) { return MT / 2 * kATile; }
 constexpr int ring_b(int NTW) { return NTW * kSubElems; }
@@ -290,10 +299,10 @@ __global__ __launch_bounds__(512) void dgrad_kmajor_kernel(const bf16_t* __restr
                                                            const int32_t* __restrict__ out_index, int K, int N, int E, int nblk_n,
                                                            bf16_t* __restrict__ out) {
   constexpr bool four = MT == 2;
-  __shared__ __attribute__((aligned(16))) bf16_t a0[ring_a(MT)];
-  __shared__ __attribute__((aligned(16))) bf16_t a1[ring_a(MT)];
-  __shared__ __attribute__((aligned(16))) bf16_t a2[ring_a(MT)];
-  __shared__ __attribute__((aligned(16))) bf16_t a3[four ? ring_a(MT) : 8];
+  __shared__ __attribute__((aligned(kLowLds))) bf16_t a0[ring_a(MT)];
+  __shared__ __attribute__((aligned(kLowLds))) bf16_t a1[ring_a(MT)];
+  __shared__ __attribute__((aligned(kLowLds))) bf16_t a2[ring_a(MT)];
+  __shared__ __attribute__((aligned(kLowLds))) bf16_t a3[four ? ring_a(MT) : 8];
   __shared__ __attribute__((aligned(16))) bf16_t b0[ring_b(NTW)];
   __shared__ __attribute__((aligned(16))) bf16_t b1[ring_b(NTW)];
   __shared__ __attribute__((aligned(16))) bf16_t b2[ring_b(NTW)];
@@ -347,7 +356,11 @@ __device__ __forceinline__ float quad_swap(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true));
 }
 
-template <int MT, int NTW, bool GATHER_P, bool GATHER_Q>
+// SMALL: an operand's rows lie within kNoRow bytes of its first one, so that a transfer's address is a descriptor and one 32-bit offset, and a row
+// past the end is an offset past the descriptor's, which reads zeros.  (With 64-bit addresses the tall tiles spill, and a spilled
+// register's reload waits for every transfer before it.)
+constexpr unsigned kNoRow = 0xffffff00u;
+template <int MT, int NTW, bool GATHER_P, bool GATHER_Q, bool SMALL>
 __device__ __forceinline__ void wgrad_block(const Ring& ring, int block, const bf16_t* __restrict__ P, const bf16_t* __restrict__ Q,
                                             const int32_t* __restrict__ index, const bf16_t* __restrict__ zrow, int N, int M, int E,
                                             const int* __restrict__ plan, float* __restrict__ part, void* __restrict__ dW, int f32) {
@@ -374,121 +387,149 @@ __device__ __forceinline__ void wgrad_block(const Ring& ring, int block, const b
   const int e_chunks = __builtin_amdgcn_readfirstlane(entry[3]);
   const int n0 = (rest % nblk_n) * BM, m0 = (rest / nblk_n) * BN;
   const int wn = wave & 3, wm = wave >> 2;
-  floatx16 acc[MT][NTW];
+  constexpr int RT = 2 * MT, CT = 2 * NTW;                // a wave's tiles of 16 x 16
+  floatx4 acc[RT][CT];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
+  for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int j = 0; j < NTW; ++j)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[mt][j][i] = 0.f;
+    for (int j = 0; j < CT; ++j) acc[rt][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
   auto pbuf = [&](auto bc) -> bf16_t* { return ring.template a<decltype(bc)::value>(); };
   auto qbuf = [&](auto bc) -> bf16_t* { return ring.template b<decltype(bc)::value>(); };
   const int nstages = (hi - lo + kKS - 1) / kKS;
   const int gofs = kfill_granule(tid) * 8;
-  // This thread's row of stage `stage` (row tid / 16 of the stage's 32), the expert's last row past its end.
-  auto stage_row = [&](int stage) { return lo + min(stage, nstages - 1) * kKS + (tid >> 4); };
-  auto lookup = [&](int stage) {
-    return (GATHER_P || GATHER_Q) ? index[min(stage_row(stage), hi - 1)] : 0;
+  // This thread's row of stage `stage` (row tid / 16 of the stage's 32), counted from lo
+  const int count = hi - lo;
+  auto stage_row = [&](int stage) { return min(stage, nstages - 1) * kKS + (tid >> 4); };
+  auto lookup = [&](int stage) { return (GATHER_P || GATHER_Q) ? index[lo + min(stage_row(stage), count - 1)] : 0; };
+  // transfer q of a stage into buffer bc, the row index ix looked up before
+  const int wave_elems = __builtin_amdgcn_readfirstlane(tid >> 6) * 64 * 8;
+  const unsigned gbytes = gofs * sizeof(bf16_t);
+  const __amdgpu_buffer_rsrc_t p_rsrc = make_rsrc(uniform(P + (GATHER_P ? 0 : (size_t)lo * N) + n0), SMALL ? kNoRow : 0);
+  const __amdgpu_buffer_rsrc_t q_rsrc = make_rsrc(uniform(Q + (GATHER_Q ? 0 : (size_t)lo * M) + m0), SMALL ? kNoRow : 0);
+  unsigned pv = 0, qv = 0;
+  auto fill = [&](auto bc, int stage, int ix, int q) {
+    if constexpr (SMALL) {
+      if (q == 0) {
+        const int r = stage_row(stage);
+        pv = r < count ? (unsigned)(GATHER_P ? ix : r) * (unsigned)(N * (int)sizeof(bf16_t)) + gbytes : kNoRow;
+        qv = r < count ? (unsigned)(GATHER_Q ? ix : r) * (unsigned)(M * (int)sizeof(bf16_t)) + gbytes : kNoRow;
+      }
+      const int sub = q < kPOps ? q : q - kPOps;
+      bf16_t* const dst = (q < kPOps ? pbuf(bc) : qbuf(bc)) + sub * kSubElems + wave_elems;
+      dma16_buf(q < kPOps ? p_rsrc : q_rsrc, q < kPOps ? pv : qv, sub * kSubW * (unsigned)sizeof(bf16_t), dst);
+    } else {
+      const int r = lo + stage_row(stage);
+      const bool live = r < hi;
+      const int rc = live ? r : hi - 1;
+      if (q < kPOps) {
+        const bf16_t* prow = live ? P + (size_t)(GATHER_P ? ix : rc) * N + n0 : zrow;
+        kfill_subtile(prow + q * kSubW + gofs, pbuf(bc) + q * kSubElems);
+      } else {
+        const bf16_t* qrow = Q + (size_t)(GATHER_Q ? ix : rc) * M + m0;
+        kfill_subtile(qrow + (q - kPOps) * kSubW + gofs, qbuf(bc) + (q - kPOps) * kSubElems);
+      }
+    }
   };
-  auto fill = [&](auto bc, int stage, int ix) {
-    const int r = stage_row(stage);
-    const bool live = r < hi;
-    const int rc = live ? r : hi - 1;
-    const bf16_t* prow = live ? P + (size_t)(GATHER_P ? ix : rc) * N + n0 : zrow;
-    const bf16_t* qrow = Q + (size_t)(GATHER_Q ? ix : rc) * M + m0;
+  int poff[RT / 2], qoff[CT / 2];                          // of the even tiles: an odd one is 16 elements on
 #pragma unroll
-    for (int j = 0; j < kPOps; ++j) kfill_subtile(prow + j * kSubW + gofs, pbuf(bc) + j * kSubElems);
-#pragma unroll
-    for (int j = 0; j < NTW; ++j) kfill_subtile(qrow + j * kSubW + gofs, qbuf(bc) + j * kSubElems);
-  };
-  int poff[MT], qoff[NTW];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const int t32 = wm * MT + mt;
-    poff[mt] = (t32 >> 2) * kSubElems + kfrag_offset(lane, (t32 & 3) * 32);
+  for (int t = 0; t < RT / 2; ++t) {
+    const int t16 = wm * RT + 2 * t;
+    poff[t] = (t16 >> 3) * kSubElems + kfrag_offset(lane, (t16 & 7) * 16);
   }
 #pragma unroll
-  for (int j = 0; j < NTW; ++j) {
-    const int t32 = wn * NTW + j;
-    qoff[j] = (t32 >> 2) * kSubElems + kfrag_offset(lane, (t32 & 3) * 32);
+  for (int t = 0; t < CT / 2; ++t) {
+    const int t16 = wn * CT + 2 * t;
+    qoff[t] = (t16 >> 3) * kSubElems + kfrag_offset(lane, (t16 & 7) * 16);
   }
   using std::integral_constant;
   if (nstages > 0) {                                               // an idle expert's gradient is zero
-    // The row index of a gathered operand is loaded R - 1 steps before the transfers that use it (R values rotate
-    // through ix[], the index of stage s in ix[s % R]): step s requests stage s + R - 1 with the index loaded at step
-    // s - R + 1 and loads the one of stage s + 2 (R - 1).  That load is one more vector-memory operation per step, so
-    // the ring's wait counts it.
+    // The row index of a gathered operand is loaded R stages before the transfers that use it: the index of stage s sits in ix[s % R], and
+    // where stage s + R is requested with it the one of stage s + 2 R is loaded.  That load is one more vector-memory operation per
+    // stage, so the ring's wait counts it.
     constexpr int kVm = kOps + ((GATHER_P || GATHER_Q) ? 1 : 0);
     int ix[R];
-    // prologue, oldest request first: stage 0, index R - 1, stage 1, index R, ... stage R - 2, index 2 R - 3
+    using Pipe = StagePipe<RT, CT, false>;
 #pragma unroll
-    for (int i = 0; i < R - 1; ++i) ix[i] = lookup(i);
-    auto prologue = [&](auto ic) {
-      constexpr int i = decltype(ic)::value;
-      fill(integral_constant<int, i>{}, i, ix[i]);
-      ix[(i + R - 1) % R] = lookup(i + R - 1);
+    for (int i = 0; i < R; ++i) ix[i] = lookup(i);
+    auto request = [&](auto bc, int stage, int q) {       // operation q of a stage: its transfers, then the lookup
+      constexpr int b = decltype(bc)::value;
+      if (q < kOps) fill(bc, stage, ix[b], q);
+      else ix[b] = lookup(stage + R);
+      __builtin_amdgcn_sched_barrier(0);                   // (in the order that the wait counts assume)
     };
-    prologue(integral_constant<int, 0>{});
-    prologue(integral_constant<int, 1>{});
-    if constexpr (R == 4) prologue(integral_constant<int, 2>{});
+    auto request_all = [&](auto bc, int stage) {
+#pragma unroll
+      for (int q = 0; q < kVm; ++q) request(bc, stage, q);
+    };
+    request_all(integral_constant<int, 0>{}, 0);
+    request_all(integral_constant<int, 1>{}, 1);
+    if constexpr (R == 4) request_all(integral_constant<int, 2>{}, 2);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) request(integral_constant<int, R - 1>{}, R - 1, q);
+    auto read_p = [&](auto bc, int rt) { return kfrag_read(pbuf(bc) + (rt & 1) * 16, poff[rt >> 1]); };
+    auto read_q = [&](auto bc, int j) { return kfrag_read(qbuf(bc) + (j & 1) * 16, qoff[j >> 1]); };
+    Pipe pipe;
+    sync_keep_loads<(R - 2) * kVm + 2>();
+    {
+      const integral_constant<int, 0> b0;
+      pipe.begin([&](int rt) { return read_p(b0, rt); }, [&](int j) { return read_q(b0, j); });
+    }
     auto step = [&](auto bc, int stage) {
       constexpr int b = decltype(bc)::value;
-      sync_keep_loads<(R - 2) * kVm>();
-      fill(integral_constant<int, (b + R - 1) % R>{}, stage + R - 1, ix[(b + R - 1) % R]);
-      ix[(b + R - 2) % R] = lookup(stage + 2 * (R - 1));
-      if (stage < nstages) {
-        const bf16_t* pt = pbuf(bc);
-        const bf16_t* qt = qbuf(bc);
-        auto read_p = [&](int s, int mt) { return kfrag_read_s(pt, poff[mt], s); };
-        auto read_q = [&](int s, int j) { return kfrag_read_s(qt, qoff[j], s); };
-        if constexpr (MT == 2) multiply_stage<MT, NTW, false>(acc, read_p, read_q);
-        else multiply_stage_tall<MT, NTW, false, 2>(acc, read_p, read_q);
-      }
+      const integral_constant<int, (b + 1) % R> nc;
+      const integral_constant<int, (b + R - 1) % R> pc;
+      pipe.template stage<b * RT % Pipe::NA, kVm>(
+          acc, [&]() { sync_keep_loads<(R - 2) * kVm>(); }, [&](int rt) { return read_p(bc, rt); }, [&](int rt) { return read_p(nc, rt); },
+          [&](int j) { return read_q(nc, j); }, [&](int q) { request(bc, stage + R, q); }, [&](int q) { request(pc, stage + R - 1, q); });
     };
-    for (int i = 0; i < nstages; i += R) {
+    int i = 0;
+    for (; i + R <= nstages; i += R) {
       step(integral_constant<int, 0>{}, i);
       step(integral_constant<int, 1>{}, i + 1);
       step(integral_constant<int, 2>{}, i + 2);
       if constexpr (R == 4) step(integral_constant<int, 3>{}, i + 3);
     }
+    if (i < nstages) step(integral_constant<int, 0>{}, i);
+    if (i + 1 < nstages) step(integral_constant<int, 1>{}, i + 1);
+    if constexpr (R == 4) if (i + 2 < nstages) step(integral_constant<int, 2>{}, i + 2);
     __builtin_amdgcn_s_waitcnt(0);       // the repeated requests of the last steps land before the workgroup ends
   }
-  // lane = column m0 + (wn NTW + j) 32 + lane % 32, register 4 q + r = row n0 + (wm MT + mt) 32 + 8 q + 4 (lane / 32) + r: a store's 32
-  // lanes leave 128 contiguous bytes of a row in fp32, and in bf16 (lane pairs trade the odd row of one for the even row of the other, two
-  // columns a lane) 64.  With a lane per row, 16 bytes of each in a store, XXX.
-  const int n = lane & 31, hh = lane >> 5;
-  const unsigned row = n0 + wm * MT * 32 + 4 * hh, col = m0 + wn * NTW * 32 + n;
+  // lane = column m0 + (wn CT + j) 16 + lane % 16, register r = row n0 + (wm RT + rt) 16 + 4 (lane / 16) + r: 16 lanes of a store leave 64
+  // contiguous bytes of a row in fp32, and in bf16 (lane pairs trade the odd row of one for the even row of the other, two columns a lane)
+  // 32.  With a lane per row, 16 bytes of each in a store, the launch took 207 us instead of 195 at T = 8192, H = 768, I = 384, E = 64, k = 6.
+  const int n = lane & 15, g4 = lane >> 4;
+  const unsigned row = n0 + wm * MT * 32 + 4 * g4, col = m0 + wn * NTW * 32 + n;
   if (e_chunks == 1 && !f32) {
     const __amdgpu_buffer_rsrc_t dst = make_rsrc(uniform(static_cast<bf16_t*>(dW) + (size_t)e * N * M), (unsigned)N * M * sizeof(bf16_t));
     const bool odd = n & 1;
     const unsigned voff = ((row + odd) * M + (col & ~1u)) * sizeof(bf16_t);
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-      for (int j = 0; j < NTW; ++j)
+      for (int i = 0; i < 4; i += 2)
 #pragma unroll
-        for (int i = 0; i < 16; i += 2) {
-          const float lo = acc[mt][j][i], hi2 = acc[mt][j][i + 1];
+        for (int j = 0; j < CT; ++j) {
+          const float lo = acc[rt][j][i], hi2 = acc[rt][j][i + 1];
           const float got = quad_swap(odd ? lo : hi2);
           typedef bf16_t bf16x2 __attribute__((ext_vector_type(2)));
           const bf16x2 v = {(bf16_t)(odd ? got : lo), (bf16_t)(odd ? hi2 : got)};
           __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), dst, voff,
-                                                ((mt * 32 + 8 * (i >> 2) + (i & 3)) * M + j * 32) * (unsigned)sizeof(bf16_t), 0);
+                                                ((rt * 16 + i) * M + j * 16) * (unsigned)sizeof(bf16_t), 0);
         }
   } else {
     float* const base = e_chunks == 1 ? static_cast<float*>(dW) + (size_t)e * N * M : part + (size_t)cg * N * M;
     const __amdgpu_buffer_rsrc_t dst = make_rsrc(uniform(base), (unsigned)N * M * sizeof(float));
     const unsigned voff = (row * M + col) * sizeof(float);
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-      for (int j = 0; j < NTW; ++j)
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const float v = acc[mt][j][i];         // (a bit_cast of the element itself reads element 0)
-          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), dst, voff,
-                                                ((mt * 32 + 8 * (i >> 2) + (i & 3)) * M + j * 32) * (unsigned)sizeof(float), 0);
+        for (int j = 0; j < CT; ++j) {
+          const float v = acc[rt][j][i];         // (a bit_cast of the element itself reads element 0)
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), dst, voff, ((rt * 16 + i) * M + j * 16) * (unsigned)sizeof(float),
+                                                0);
         }
   }
 }
@@ -514,10 +555,10 @@ struct BackwardGemms {
 template <int NH, int NI, bool TALL>
 __global__ __launch_bounds__(512) void backward_gemms_kernel(BackwardGemms g) {
   constexpr int MT = TALL ? 4 : 2, NB = NH > NI ? NH : NI;
-  __shared__ __attribute__((aligned(16))) bf16_t a0[ring_a(MT)];
-  __shared__ __attribute__((aligned(16))) bf16_t a1[ring_a(MT)];
-  __shared__ __attribute__((aligned(16))) bf16_t a2[ring_a(MT)];
-  __shared__ __attribute__((aligned(16))) bf16_t a3[ring_a(2)];
+  __shared__ __attribute__((aligned(kLowLds))) bf16_t a0[ring_a(MT)];
+  __shared__ __attribute__((aligned(kLowLds))) bf16_t a1[ring_a(MT)];
+  __shared__ __attribute__((aligned(kLowLds))) bf16_t a2[ring_a(MT)];
+  __shared__ __attribute__((aligned(kLowLds))) bf16_t a3[ring_a(2)];
   __shared__ __attribute__((aligned(16))) bf16_t b0[ring_b(NB)];
   __shared__ __attribute__((aligned(16))) bf16_t b1[ring_b(NB)];
   __shared__ __attribute__((aligned(16))) bf16_t b2[ring_b(NB)];
@@ -539,12 +580,12 @@ __global__ __launch_bounds__(512) void backward_gemms_kernel(BackwardGemms g) {
     });
   else if (block < g.n_dx + g.n_gu)
     either(g.tall_gu, [&](auto mt) {
-      wgrad_block<decltype(mt)::value, NH, false, true>(ring, block - g.n_dx, g.dgu, g.x, g.perm_token, g.zrow, 2 * g.I, g.H, g.E, g.plan,
+      wgrad_block<decltype(mt)::value, NH, false, true, TALL>(ring, block - g.n_dx, g.dgu, g.x, g.perm_token, g.zrow, 2 * g.I, g.H, g.E, g.plan,
                                                         g.part_gu, g.dwgu, g.f32);
     });
   else
     either(g.tall_d, [&](auto mt) {
-      wgrad_block<decltype(mt)::value, NI, true, false>(ring, block - g.n_dx - g.n_gu, g.d_out, g.hidden, g.perm_token, g.zrow, g.H, g.I, g.E,
+      wgrad_block<decltype(mt)::value, NI, true, false, TALL>(ring, block - g.n_dx - g.n_gu, g.d_out, g.hidden, g.perm_token, g.zrow, g.H, g.I, g.E,
                                                         g.plan, g.part_d, g.dwd, g.f32);
     });
 }

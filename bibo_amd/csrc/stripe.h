@@ -104,6 +104,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, un
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);   // raw buffer, 32-bit data format
 }
 
+// LDS-DMA through a buffer descriptor: the address is descriptor base + 32-bit per-thread byte offset (one
+// vector register) + a wave-uniform byte offset (scalar), so the loop keeps no 64-bit per-thread addresses.
+__device__ __forceinline__ void dma16_buf(__amdgpu_buffer_rsrc_t rsrc, unsigned voff, unsigned soff, bf16_t* l) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void*)l, 16, voff, soff, 0, 0);
+}
+
 // a pointer that is the same in every lane, in scalar registers
 template <typename T>
 __device__ __forceinline__ T* uniform(T* p) {

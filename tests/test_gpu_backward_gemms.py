@@ -1,8 +1,11 @@
 """The three products of the backward pass that share a launch (dx of every slot, dW_gate_up, dW_down), on 128-row tiles and on 256-row ones
 (experts of 192 rows and more, several rounds of workgroups), over the widths their workgroups divide into; against autograd in fp32."""
+import ctypes
+
 import pytest
 import torch
 
+from bibo_amd import _lib as L
 from bibo_amd import ops
 from oracle import bibo_moe_oracle as O
 
@@ -39,3 +42,41 @@ def test_products(T, H, I, E, k):
     for name, a, ref in zip(("dx", "dW_gate_up", "dW_down"), (dx, dgu, ddn), _reference(x, d, idx, w, wgu, wd, theta)):
         assert float((a.float() - ref).norm() / ref.norm()) <= 1e-2, name
         assert float((a.float() - ref).abs().max() / ref.abs().max()) <= 2e-2, name
+
+
+def _weight_grads_f32(x, d, idx, w, wgu, wd, theta):
+    """Both weight gradients of bibo_moe_experts_backward in fp32, as for the masters of mixed-precision training."""
+    (T, H), (E, _, I), k = x.shape, wd.shape, idx.shape[1]
+    sh = L.Shape(T, H, E, k, I, 0, 0, 0, 0, L.FLAG_GRAD_F32)
+    need = ctypes.c_size_t(0)
+    L.check(L.lib().bibo_moe_backward_workspace_bytes(ctypes.byref(sh), ctypes.byref(need)), "bytes")
+    ws = torch.empty(need.value + 256, dtype=torch.uint8, device=DEV)
+    dx, dw, dth = torch.empty_like(x), torch.empty_like(w), torch.empty_like(theta)
+    dgu, ddn = (torch.empty(t.shape, dtype=torch.float32, device=DEV) for t in (wgu, wd))
+    ptr = [ctypes.c_void_p(t.data_ptr()) for t in (x, d, idx, w, wgu, wd, theta)]
+    out = [ctypes.c_void_p(t.data_ptr()) for t in (dx, dw, dgu, ddn, dth)]
+    L.check(L.lib().bibo_moe_experts_backward(*ptr, ctypes.byref(sh), *out, ctypes.c_void_p((ws.data_ptr() + 255) & ~255), need.value,
+                                              ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "bibo_moe_experts_backward")
+    return dx, None, dgu, ddn
+
+
+# An expert's rows are a loop over stages of 32 in rings of four (128-row tiles) or three (256-row ones): no stage, less than a ring, every
+# remainder, and last stages of one row and of all but one.
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("H,I,counts", [(256, 128, [0, 1, 2, 31, 32, 33, 63, 64, 65, 96, 97, 127, 128, 129, 159, 161, 225, 256]),
+                                        (768, 384, [0, 1, 33] + [193 + 5 * i for i in range(61)])])
+def test_rows_of_an_expert(H, I, counts, f32):
+    E, T = len(counts), sum(counts)
+    p = O.make_inputs(T=8, H=H, E=E, k=1, I=I, theta="normal", seed=E)
+    g = torch.Generator().manual_seed(E)
+    x, d = (torch.randn(T, H, generator=g).bfloat16().to(DEV) for _ in range(2))
+    idx = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(T, generator=g)].to(torch.int32)[:, None].to(DEV)
+    w = torch.rand(T, 1, generator=g).to(DEV)
+    wgu, wd, theta = (p[n].to(DEV) for n in ("w_gate_up", "w_down", "theta"))
+    dx, _, dgu, ddn = (_weight_grads_f32 if f32 else ops.experts_backward)(x, d, idx, w, wgu, wd, theta)[:4]
+    for name, a, ref in zip(("dx", "dW_gate_up", "dW_down"), (dx, dgu, ddn), _reference(x, d, idx, w, wgu, wd, theta)):
+        assert float((a.float() - ref).norm() / ref.norm()) <= 1e-2, name
+        if name == "dx":
+            continue
+        for e in range(E):          # an expert at a time: a row too many or too few of one does not drown in the others
+            assert float((a[e].float() - ref[e]).norm()) <= 2e-2 * float(ref[e].norm()) + 1e-6, (name, e, counts[e])
