@@ -136,6 +136,16 @@ __device__ __forceinline__ void sync_keep_loads() {
   __builtin_amdgcn_s_barrier();
 }
 
+// The same where the compiler does not see the transfers as writes to LDS: no LDS access moves across it.
+template <int N>
+__device__ __forceinline__ void meet_waves() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  sync_keep_loads<N>();
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+}
+
 // Map a workgroup id to a tile so that the workgroups of one XCD (ids congruent mod 8 are dispatched
 // to the same XCD) walk a contiguous range of tiles: tiles of one expert then share that XCD's L2.
 __device__ __forceinline__ int xcd_tile(int bid, int total) {

@@ -34,6 +34,7 @@
 #include <type_traits>
 
 #include "experts_fused_launch.h"
+#include "experts_wide.h"
 #include "stripe.h"
 
 namespace bibo {
@@ -872,12 +873,22 @@ void launch_down_act_nt(const float* gu, const bf16_t* wd, const float* theta, c
   if (two) launch(integral_constant<int, 1>{}, integral_constant<int, 2>{}); else launch(integral_constant<int, 1>{}, integral_constant<int, 1>{});
 }
 
+// I = 512 has a kernel of its own behind the calls that find their rows themselves.  H = 1024, E = 64, k = 8, layer, this kernel -> that one, on
+// one card: 89.4 -> 89.0 us (T = 1025), 87.8 -> 86.0 (1500), 139.7 -> 133.6 (2047), 150.0 -> 143.6 (3001), 274 -> 257 (6000), 574 -> 541 (16,000);
+// H = 768, E = 32, k = 4: 106.7 -> 102.7 (4100); H = 640, E = 16, k = 2: 55.9 -> 53.9 (4200); H = 512, E = 8, k = 1: 48.1 -> 48.1 (9000).
 template <int NT>
 void launch_fused_nt(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const float* theta, const float* w,
                      const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int S, int H, int E,
                      int act, unsigned x_bytes, void* yw, bool f32_rows, bf16_t* preact, const ScanArgs& scan, hipStream_t s) {
   constexpr int MT = NT == 4 ? 1 : 2;
   auto launch = [&](auto ct) {
+    if constexpr (NT == 4) {
+      if (S > kScanSlots / 2) {
+        static_assert(kStreamMaxSlots <= kScanSlots / 2, "fp32 rows go with the few rows of a streaming call");
+        launch_wide_t<decltype(ct)::value>(x, wgu, wd, theta, w, offsets, perm_slot, perm_token, S, H, E, act, x_bytes, yw, s);
+        return;
+      }
+    }
     launch_fused_t<NT, decltype(ct)::value, MT>(x, wgu, wd, theta, w, offsets, perm_slot, perm_token, S, H, E, act, x_bytes, yw, f32_rows,
                                                preact, scan, s);
   };

@@ -1,0 +1,42 @@
+"""The fused kernel of I = 512 with more than 8192 slots: output blocks of every width and the ends of its tile heights, with idle experts;
+against the fp32 oracle and against the first rows alone, which the kernel for fewer slots takes."""
+import numpy as np
+import pytest
+import torch
+
+from bibo_amd import ops
+from oracle import bibo_moe_oracle as O
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+ROWS = {
+    "one slot more than the limit": [1161, 0, 1025, 1023, 1024, 1026, 1434, 1500],
+    "one block each": [128] * 63 + [130],
+    "ragged": [0, 1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 1400, 7] * 4,
+    "one expert": [0, 16385, 0],
+}
+
+
+@pytest.mark.parametrize("H", [128, 256, 384, 640, 768])
+@pytest.mark.parametrize("name", ROWS)
+def test_many_slots(H, name):
+    rows, I = ROWS[name], 512
+    E, T = len(rows), sum(rows)
+    assert T > 8192
+    p = O.make_inputs(T=T, H=H, E=E, k=1, I=I, theta="normal", seed=H + I)
+    idx = np.repeat(np.arange(E, dtype=np.int32), rows)
+    np.random.default_rng(I).shuffle(idx)
+    idx, w = idx.reshape(T, 1), np.random.default_rng(H).random((T, 1)).astype(np.float32)
+
+    def run(keep):
+        args = [p["x"][keep].to(DEV), torch.from_numpy(idx[keep]).to(DEV), torch.from_numpy(w[keep]).to(DEV),
+                *(p[n].to(DEV) for n in ("w_gate_up", "w_down", "theta"))]
+        return ops.experts_fwd(*args, algo="auto")[0].float().cpu()
+
+    got, few = run(slice(None)), run(slice(0, 1500))
+    ref = O.experts_forward(p["x"], idx, w, p["w_gate_up"], p["w_down"], p["theta"]).float()
+    top = float(ref.abs().max())
+    assert float((got - ref).abs().max()) <= 2e-2 * top
+    # sums in another order: an activation and an output may round to the neighbouring bf16 value, 2^-7 of the value each
+    assert float((few - got[:1500]).abs().max()) <= 2 * 2.0 ** -7 * top
