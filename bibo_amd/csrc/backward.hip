@@ -170,8 +170,11 @@ hipError_t launch_dgrad(const bf16_t* A, const int32_t* a_index, const bf16_t* W
 inline int sub_tiles(int n) { return n % 384 == 0 ? 3 : n % 256 == 0 ? 2 : 1; }
 
 // dx of every slot and both weight gradients (kmajor.h: backward_gemms_kernel).  256-row tiles, which stream the other operand half as
-// often and take 1.75 times as long, where the experts hold 192 rows on average and the launch is several rounds of workgroups, whose last
-// one the three products share.
+// often, from 128 rows per expert on, where the average expert fills a row tile of the lower ones and begins another, if the launch is several
+// rounds of workgroups, whose last one the three products share.  Lower -> taller tiles, us, E = 64, k = 6 and rows per expert in brackets:
+// H = 768, I = 384: 56 -> 59 (122), 60.5 -> 59.6 (131), 70 -> 63 (159), 79 -> 67 (192), 189 -> 151 (768); H = 512, I = 256: 31.6 -> 28.8 (131),
+// 100 -> 86 (768); H = 768, I = 128: 29.6 -> 24.7 (131); H = 1024, I = 512, k = 8: 106 -> 95 (100), 122 -> 102 (150), 260 -> 211 (512).  In
+// launches of one round and a bit (H = 512, I = 256, E = 9, k = 2): 13.9 -> 18.6 (494), 30.8 -> 33.1 (1333).
 // Tall launches address rows by 32-bit offsets (kmajor.h: SMALL): from the first token of x and d_out, from the first row of a chunk in the
 // others.
 hipError_t launch_backward_gemms(BackwardGemms g, int T, int S, int chunk, int slots, hipStream_t s) {
@@ -182,7 +185,7 @@ hipError_t launch_backward_gemms(BackwardGemms g, int T, int S, int chunk, int s
   auto down = [&](int rows) { return (long long)slots * (H / rows) * (I / bi); };
   const long long widest = (long long)sizeof(bf16_t) * (H > 2 * I ? H : 2 * I);
   const bool near = T * widest < kNoRow && chunk * widest < kNoRow;
-  const bool tall = near && (long long)S >= 192ll * E && dx(128) + gu(128) + down(128) > 3 * kCUs;
+  const bool tall = near && (long long)S >= 128ll * E && dx(128) + gu(128) + down(128) > 3 * kCUs;
   g.tall_dx = tall;
   g.tall_gu = tall && 2 * I % 256 == 0;
   g.tall_d = tall && H % 256 == 0;

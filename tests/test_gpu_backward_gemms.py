@@ -64,7 +64,9 @@ def _weight_grads_f32(x, d, idx, w, wgu, wd, theta):
 # remainder, and last stages of one row and of all but one.
 @pytest.mark.parametrize("f32", [False, True])
 @pytest.mark.parametrize("H,I,counts", [(256, 128, [0, 1, 2, 31, 32, 33, 63, 64, 65, 96, 97, 127, 128, 129, 159, 161, 225, 256]),
-                                        (768, 384, [0, 1, 33] + [193 + 5 * i for i in range(61)])])
+                                        (768, 384, [0, 1, 33] + [193 + 5 * i for i in range(61)]),
+                                        (512, 256, [0, 1, 255, 256, 257] + [98 + i for i in range(59)]),       # 128 rows and more on average
+                                        (512, 256, [0, 1, 255, 256, 257] + [96 + i for i in range(59)])])      # and less
 def test_rows_of_an_expert(H, I, counts, f32):
     E, T = len(counts), sum(counts)
     p = O.make_inputs(T=8, H=H, E=E, k=1, I=I, theta="normal", seed=E)
