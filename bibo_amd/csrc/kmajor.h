@@ -453,9 +453,12 @@ __device__ __forceinline__ void wgrad_block(const Ring& ring, int block, const b
   using std::integral_constant;
   if (nstages > 0) {                                               // an idle expert's gradient is zero
     // The row index of a gathered operand is loaded R stages before the transfers that use it: the index of stage s sits in ix[s % R], and
-    // where stage s + R is requested with it the one of stage s + 2 R is loaded.  That load is one more vector-memory operation per
-    // stage, so the ring's wait counts it.
-    constexpr int kVm = kOps + ((GATHER_P || GATHER_Q) ? 1 : 0);
+    // where stage s + R is requested with it the one of stage s + 2 R is loaded.  No wait counts these loads: the compiler drops the ones
+    // that nothing behind them uses, as in the last stages, and moves others, and a wait that counts a load it has dropped lets the last
+    // transfer of the stage that is read next stay in flight.  Counted by transfers alone, which are all issued at their places, a wait
+    // is for R - 2 operations more than it need be where the loads are there: no difference in time (T = 8192, H = 768, I = 384, E = 64, k = 6:
+    // 154 to 170 us either way).
+    constexpr int kVm = kOps + ((GATHER_P || GATHER_Q) ? 1 : 0);           // operations of a stage
     int ix[R];
     using Pipe = StagePipe<RT, CT, false>;
 #pragma unroll
@@ -464,7 +467,7 @@ __device__ __forceinline__ void wgrad_block(const Ring& ring, int block, const b
       constexpr int b = decltype(bc)::value;
       if (q < kOps) fill(bc, stage, ix[b], q);
       else ix[b] = lookup(stage + R);
-      __builtin_amdgcn_sched_barrier(0);                   // (in the order that the wait counts assume)
+      __builtin_amdgcn_sched_barrier(0);                   // (stage by stage, as the waits assume)
     };
     auto request_all = [&](auto bc, int stage) {
 #pragma unroll
@@ -478,7 +481,7 @@ __device__ __forceinline__ void wgrad_block(const Ring& ring, int block, const b
     auto read_p = [&](auto bc, int rt) { return kfrag_read(pbuf(bc) + (rt & 1) * 16, poff[rt >> 1]); };
     auto read_q = [&](auto bc, int j) { return kfrag_read(qbuf(bc) + (j & 1) * 16, qoff[j >> 1]); };
     Pipe pipe;
-    sync_keep_loads<(R - 2) * kVm + 2>();
+    sync_keep_loads<(R - 2) * kOps + 2>();
     {
       const integral_constant<int, 0> b0;
       pipe.begin([&](int rt) { return read_p(b0, rt); }, [&](int j) { return read_q(b0, j); });
@@ -488,7 +491,7 @@ __device__ __forceinline__ void wgrad_block(const Ring& ring, int block, const b
       const integral_constant<int, (b + 1) % R> nc;
       const integral_constant<int, (b + R - 1) % R> pc;
       pipe.template stage<b * RT % Pipe::NA, kVm>(
-          acc, [&]() { sync_keep_loads<(R - 2) * kVm>(); }, [&](int rt) { return read_p(bc, rt); }, [&](int rt) { return read_p(nc, rt); },
+          acc, [&]() { sync_keep_loads<(R - 2) * kOps>(); }, [&](int rt) { return read_p(bc, rt); }, [&](int rt) { return read_p(nc, rt); },
           [&](int j) { return read_q(nc, j); }, [&](int q) { request(bc, stage + R, q); }, [&](int q) { request(pc, stage + R - 1, q); });
     };
     int i = 0;

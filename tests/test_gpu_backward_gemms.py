@@ -66,7 +66,15 @@ def _weight_grads_f32(x, d, idx, w, wgu, wd, theta):
 @pytest.mark.parametrize("H,I,counts", [(256, 128, [0, 1, 2, 31, 32, 33, 63, 64, 65, 96, 97, 127, 128, 129, 159, 161, 225, 256]),
                                         (768, 384, [0, 1, 33] + [193 + 5 * i for i in range(61)]),
                                         (512, 256, [0, 1, 255, 256, 257] + [98 + i for i in range(59)]),       # 128 rows and more on average
-                                        (512, 256, [0, 1, 255, 256, 257] + [96 + i for i in range(59)])])      # and less
+                                        (512, 256, [0, 1, 255, 256, 257] + [96 + i for i in range(59)]),       # and less
+                                        # 128-row tiles of dW_down (H no multiple of 256) beside 256-row ones of the others: three stages behind
+                                        # the last full ring of four, the loads of their row indices gone
+                                        (640, 128, [65 + i for i in range(32)] + [193 + i for i in range(32)]),
+                                        (640, 256, [65 + i for i in range(32)] + [193 + i for i in range(32)]),
+                                        (384, 384, [65 + i for i in range(32)] + [193 + i for i in range(32)]),
+                                        (384, 256, [193 + i for i in range(32)] + [321 + i for i in range(32)]),
+                                        # two stages, fewer than a ring of three: in whole experts and in the last chunk of cut ones
+                                        (768, 384, [33 + i for i in range(32)] + [545 + i for i in range(32)])])
 def test_rows_of_an_expert(H, I, counts, f32):
     E, T = len(counts), sum(counts)
     p = O.make_inputs(T=8, H=H, E=E, k=1, I=I, theta="normal", seed=E)
