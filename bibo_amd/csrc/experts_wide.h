@@ -55,7 +55,7 @@ struct WideShape {
 // meetings of phase 1 do exactly and for a buffer of the ring that is chosen at run time.  l: byte address in LDS of the wave's 1 KB.
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void dma16_unseen(i32x4 rsrc, unsigned voff, unsigned soff, unsigned l) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(l), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(l), "v"(voff), "s"(rsrc), "s"(soff) : "m0", "memory");
 }
 __device__ __forceinline__ i32x4 make_words(const void* base, unsigned bytes) {      // make_rsrc for it
   const unsigned long long a = (unsigned long long)uniform(base);
