@@ -61,7 +61,8 @@ __device__ __forceinline__ i32x4 make_words(const void* base, unsigned bytes) { 
   const unsigned long long a = (unsigned long long)uniform(base);
   return i32x4{(int)(unsigned)a, (int)(unsigned)(a >> 32), (int)bytes, 0x00020000};
 }
-constexpr unsigned kPastEnd = 0xff000000u;       // an offset past any descriptor's end: reads zeros
+// a lane's offset that lies past the descriptor's end whatever is in range of it is added: reads zeros
+__device__ __forceinline__ unsigned past_end(i32x4 words) { return (unsigned)words[2]; }
 __device__ __forceinline__ unsigned lds_address(bf16_t* p) { return (unsigned)(unsigned long long)(lds_void*)p; }
 
 // The w_down rows of a wave's 16*CT output columns in blocks of 128 K elements, on their way from memory order to MFMA operand order.  A
@@ -96,10 +97,10 @@ struct DownWeights {
   // load i of block kb of the rows `rows_on` behind the first ones; with `none`, no memory is read
   __device__ __forceinline__ void load(int buf, int i, int kb, unsigned rows_on, bool none = false) {
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)((unsigned long long)(unsigned)words[0] | (unsigned long long)(unsigned)words[1] << 32), 0, words[2], words[3]);
-    const unsigned v = none ? kPastEnd : voff, at = base + (i * I + kb * 128) * (unsigned)sizeof(bf16_t);
+    const unsigned v = none ? past_end(words) : voff, at = none ? 0u : base + (i * I + kb * 128 + rows_on * I) * (unsigned)sizeof(bf16_t);
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct)
-      w[buf][ct][i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc, v, at + (rows_on + 16 * ct) * I * (unsigned)sizeof(bf16_t), 0));
+      w[buf][ct][i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc, v, at + 16 * ct * I * (unsigned)sizeof(bf16_t), 0));
   }
   // 32-bit word d of the four registers of column tile ct
   __device__ __forceinline__ void transpose(int buf, int ct, int d) {
@@ -259,13 +260,14 @@ __global__ __launch_bounds__(512) void experts_wide_kernel(const bf16_t* __restr
     const unsigned s_lds = lds_address(S) + wave_bytes, a_lds = lds_address(A) + wave_bytes;
     const unsigned a_voff = (unsigned)perm_token[row0 + min(drow, rows - 1)] * hb + chunk * 16;   // gather, moe.py:81 (rows past the end: the last one)
     // the transfers of sub-step (s, t) into stage `st` and of step s into x buffer `xb`; for steps past the last one, whose buffers nobody
-    // reads again, they lie past the descriptors' ends and touch no memory: every sub-step issues the same number
+    // reads again, they lie past the descriptors' ends and touch no memory (where x is close to 2^32 bytes and the sum of the offsets wraps,
+    // they read from its first row): every sub-step issues the same number
     auto request_w = [&](int q, int t, int s, unsigned st) {
-      dma16_unseen(w_rsrc, s < nsteps ? b_voff : kPastEnd, (unsigned)block_of(t) * 32 * hb + (unsigned)s * kb + q * bstep,
+      dma16_unseen(w_rsrc, s < nsteps ? b_voff : past_end(w_rsrc), (unsigned)block_of(t) * 32 * hb + (unsigned)s * kb + q * bstep,
                    s_lds + st * (F::kStageElems * (unsigned)sizeof(bf16_t)) + q * 8192);
     };
     auto request_x = [&](int s, unsigned xb) {
-      dma16_unseen(x_rsrc, s < nsteps ? a_voff : kPastEnd, (unsigned)s * kb, a_lds + xb * (F::kAElems * (unsigned)sizeof(bf16_t)));
+      dma16_unseen(x_rsrc, s < nsteps ? a_voff : past_end(x_rsrc), (unsigned)s * kb, a_lds + xb * (F::kAElems * (unsigned)sizeof(bf16_t)));
     };
     // One pipeline over eight groups (k32 step, 16-column tile) a sub-step, RT MFMAs each.  A group's weight fragment is read D groups ahead,
     // across the ends of sub-steps: D groups before a sub-step ends the waves meet (the next stage has landed, every fragment of

@@ -40,3 +40,27 @@ def test_many_slots(H, name):
     assert float((got - ref).abs().max()) <= 2e-2 * top
     # sums in another order: an activation and an output may round to the neighbouring bf16 value, 2^-7 of the value each
     assert float((few - got[:1500]).abs().max()) <= 2 * 2.0 ** -7 * top
+
+
+def test_x_of_almost_4_gib():
+    """Rows of x beyond byte 0xff000000, the last tokens among them: the requests behind the last K step lie past x whatever its size.  A
+    row's sums do not depend on its tile, so the ends of the call are the same bits as those tokens alone."""
+    H, I, E, part = 1024, 512, 8, 9000
+    T = 0xff000000 // (2 * H) + 3
+    p = O.make_inputs(T=8, H=H, E=E, k=1, I=I, theta="normal", seed=5)
+    wgu, wd, theta = (p[n].to(DEV) for n in ("w_gate_up", "w_down", "theta"))
+    g = torch.Generator(device=DEV).manual_seed(6)
+    try:
+        x = torch.randn(T, H, generator=g, device=DEV, dtype=torch.bfloat16)
+        idx = torch.randint(E, (T, 1), generator=g, device=DEV, dtype=torch.int32)
+        w = torch.rand(T, 1, generator=g, device=DEV)
+        out = ops.experts_fwd(x, idx, w, wgu, wd, theta)[0]
+        for a in (0, T // 2, T - part):
+            few = slice(a, a + part)
+            assert torch.equal(ops.experts_fwd(x[few], idx[few], w[few], wgu, wd, theta)[0], out[few]), a
+        tail = slice(T - 64, T)
+        ref = O.experts_forward(x[tail].cpu(), idx[tail].cpu(), w[tail].cpu(), p["w_gate_up"], p["w_down"], p["theta"]).float()
+        assert float((out[tail].float().cpu() - ref).abs().max()) <= 2e-2 * float(ref.abs().max())
+    finally:
+        ops._workspaces.clear()                      # 4 GB of workspace: not kept for the tests that follow
+        torch.cuda.empty_cache()
