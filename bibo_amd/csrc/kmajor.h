@@ -510,9 +510,11 @@ __device__ __forceinline__ void wgrad_block(const Ring& ring, int block, const b
   // contiguous bytes of a row in fp32, and in bf16 (lane pairs trade the odd row of one for the even row of the other, two columns a lane)
   // 32.  With a lane per row, 16 bytes of each in a store, the launch took 207 us instead of 195 at T = 8192, H = 768, I = 384, E = 64, k = 6.
   const int n = lane & 15, g4 = lane >> 4;
-  const unsigned row = n0 + wm * MT * 32 + 4 * g4, col = m0 + wn * NTW * 32 + n;
+  // Offsets count from the tile's first element: an expert's matrix may hold 2^32 bytes and more.
+  const unsigned row = wm * MT * 32 + 4 * g4, col = wn * NTW * 32 + n;
+  const size_t tile = (size_t)n0 * M + m0;
   if (e_chunks == 1 && !f32) {
-    const __amdgpu_buffer_rsrc_t dst = make_rsrc(uniform(static_cast<bf16_t*>(dW) + (size_t)e * N * M), (unsigned)N * M * sizeof(bf16_t));
+    const __amdgpu_buffer_rsrc_t dst = make_rsrc(uniform(static_cast<bf16_t*>(dW) + (size_t)e * N * M + tile), kNoRow);
     const bool odd = n & 1;
     const unsigned voff = ((row + odd) * M + (col & ~1u)) * sizeof(bf16_t);
 #pragma unroll
@@ -530,7 +532,7 @@ __device__ __forceinline__ void wgrad_block(const Ring& ring, int block, const b
         }
   } else {
     float* const base = e_chunks == 1 ? static_cast<float*>(dW) + (size_t)e * N * M : part + (size_t)cg * N * M;
-    const __amdgpu_buffer_rsrc_t dst = make_rsrc(uniform(base), (unsigned)N * M * sizeof(float));
+    const __amdgpu_buffer_rsrc_t dst = make_rsrc(uniform(base + tile), kNoRow);
     const unsigned voff = (row * M + col) * sizeof(float);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)

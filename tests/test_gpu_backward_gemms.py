@@ -90,3 +90,20 @@ def test_rows_of_an_expert(H, I, counts, f32):
             continue
         for e in range(E):          # an expert at a time: a row too many or too few of one does not drown in the others
             assert float((a[e].float() - ref[e]).norm()) <= 2e-2 * float(ref[e].norm()) + 1e-6, (name, e, counts[e])
+
+
+def test_weight_gradients_of_4_gib():
+    """One expert whose fp32 gate/up gradient holds 2^32 bytes: offsets into it do not fit 32 bits."""
+    T, H, E, I = 40, 1 << 20, 1, 512
+    g = torch.Generator(device=DEV).manual_seed(1)
+    rand = lambda *shape: torch.randn(*shape, generator=g, device=DEV, dtype=torch.bfloat16)
+    try:
+        x, d, wgu, wd = rand(T, H), rand(T, H), rand(E, 2 * I, H) * 1e-3, rand(E, H, I) * 1e-3
+        idx, w = torch.zeros(T, 1, dtype=torch.int32, device=DEV), torch.rand(T, 1, generator=g, device=DEV)
+        theta = torch.zeros(E, device=DEV)
+        dx, _, dgu, ddn = _weight_grads_f32(x, d, idx, w, wgu, wd, theta)
+        assert dgu.numel() * dgu.element_size() >= 2 ** 32
+        for name, a, ref in zip(("dx", "dW_gate_up", "dW_down"), (dx, dgu, ddn), _reference(x, d, idx, w, wgu, wd, theta)):
+            assert float((a.float() - ref).norm() / ref.norm()) <= 1e-2, name
+    finally:
+        torch.cuda.empty_cache()
