@@ -186,17 +186,16 @@ hipError_t launch_backward_gemms(BackwardGemms g, int T, int S, int chunk, int s
   const long long widest = (long long)sizeof(bf16_t) * (H > 2 * I ? H : 2 * I);
   const bool near = T * widest < kNoRow && chunk * widest < kNoRow;
   const bool tall = near && (long long)S >= 128ll * E && dx(128) + gu(128) + down(128) > 3 * kCUs;
-  g.tall_dx = tall;
-  g.tall_gu = tall && 2 * I % 256 == 0;
+  const int rows = tall ? 256 : 128;                     // (2 I is a multiple of both: backward_supported)
   g.tall_d = tall && H % 256 == 0;
-  g.n_dx = pad8(dx(g.tall_dx ? 256 : 128));
-  g.n_gu = pad8(gu(g.tall_gu ? 256 : 128));
+  g.n_dx = pad8(dx(rows));
+  g.n_gu = pad8(gu(rows));
   const int n_d = pad8(down(g.tall_d ? 256 : 128));
   const dim3 grid((unsigned)(g.n_dx + g.n_gu + n_d));
   using std::integral_constant;
   auto launch = [&](auto hc, auto ic) {
     constexpr int NH = decltype(hc)::value, NI = decltype(ic)::value;
-    if (g.tall_dx || g.tall_gu || g.tall_d) hipLaunchKernelGGL((backward_gemms_kernel<NH, NI, true>), grid, dim3(512), 0, s, g);
+    if (tall) hipLaunchKernelGGL((backward_gemms_kernel<NH, NI, true>), grid, dim3(512), 0, s, g);
     else hipLaunchKernelGGL((backward_gemms_kernel<NH, NI, false>), grid, dim3(512), 0, s, g);
   };
   auto by_i = [&](auto hc) {
@@ -588,7 +587,7 @@ hipError_t launch_backward(const void* x, const void* d_out, const void* w_route
   // [dg, du]^T x (x gathered by token)
   float* part_gu = b.wgrad_part + (size_t)slots * H * I;
   BackwardGemms gemms{xp, dop, dgu, hidden, wgup, zrow, offsets, perm_slot, perm_token, b.wgrad_plan, dxs, d_wgu, d_wd, part_gu,
-                      b.wgrad_part, H, I, E, grad_f32, 0, 0, false, false, false};
+                      b.wgrad_part, H, I, E, grad_f32, 0, 0, false};
   if ((err = launch_backward_gemms(gemms, T, S, backward_chunk_rows(S, Et), slots, s)) != hipSuccess) return err;
   const bool with_router = w_router != nullptr;      // else: the experts alone, the caller owns the routing
   const int parts = (H / 8 + kWave - 1) / kWave;     // runs of columns a lane each

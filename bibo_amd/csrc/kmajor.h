@@ -551,7 +551,7 @@ __device__ __forceinline__ void wgrad_block(const Ring& ring, int block, const b
 // dx of every slot = [dg, du] W_gate_up (blocks [0, n_dx)), dW_gate_up = [dg, du]^T x (the next n_gu), dW_down = d^T (w h) (the rest).
 // They need nothing from one another, and a workgroup fills a CU in each: as launches of their own each ended with a round in which most
 // CUs had none, and a small call spent three launches on three handfuls of workgroups.  Longest workgroups first.  NH, NI: what 128-column
-// sub-tiles H and I divide into.  TALL: each of the three has 256-row tiles by its flag, else none (their rings are smaller).  The three
+// sub-tiles H and I divide into.  TALL: 256-row tiles in all three, dW_down's only where they divide H (tall_d); else in none.  The three
 // launches -> this one: T = 8192, H = 768, I = 384, E = 64, k = 6: 259 -> 233 us; T = 2500: 118 -> 90; T = 1111, H = 512, I = 256, E = 9,
 // k = 2: 36 -> 14; T = 16000, H = 1024, I = 512, E = 64, k = 8: 750 -> 731.
 struct BackwardGemms {
@@ -562,7 +562,7 @@ struct BackwardGemms {
   void *dwgu, *dwd;
   float *part_gu, *part_d;
   int H, I, E, f32, n_dx, n_gu;
-  bool tall_dx, tall_gu, tall_d;
+  bool tall_d;
 };
 
 template <int NH, int NI, bool TALL>
@@ -579,28 +579,20 @@ __global__ __launch_bounds__(512) void backward_gemms_kernel(BackwardGemms g) {
   __shared__ int dst_s[64 * MT];
   const Ring ring{a0, a1, a2, a3, b0, b1, b2, b3};
   const int block = blockIdx.x;
-  using std::integral_constant;
-  auto either = [](bool tall, auto run) {
-    if constexpr (TALL) {
-      if (tall) { run(integral_constant<int, 4>{}); return; }
-    }
-    run(integral_constant<int, 2>{});
+  auto down = [&](auto mt) {
+    wgrad_block<decltype(mt)::value, NI, true, false, TALL>(ring, block - g.n_dx - g.n_gu, g.d_out, g.hidden, g.perm_token, g.zrow, g.H, g.I, g.E,
+                                                            g.plan, g.part_d, g.dwd, g.f32);
   };
   if (block < g.n_dx)
-    either(g.tall_dx, [&](auto mt) {
-      dgrad_block<decltype(mt)::value, NH, false, true>(ring, dst_s, block, g.dgu, nullptr, g.wgu, g.offsets, g.perm_slot, 2 * g.I, g.H, g.E,
-                                                        g.H / (kSubW * NH), g.dxs);
-    });
+    dgrad_block<MT, NH, false, true>(ring, dst_s, block, g.dgu, nullptr, g.wgu, g.offsets, g.perm_slot, 2 * g.I, g.H, g.E, g.H / (kSubW * NH),
+                                     g.dxs);
   else if (block < g.n_dx + g.n_gu)
-    either(g.tall_gu, [&](auto mt) {
-      wgrad_block<decltype(mt)::value, NH, false, true, TALL>(ring, block - g.n_dx, g.dgu, g.x, g.perm_token, g.zrow, 2 * g.I, g.H, g.E, g.plan,
-                                                        g.part_gu, g.dwgu, g.f32);
-    });
+    wgrad_block<MT, NH, false, true, TALL>(ring, block - g.n_dx, g.dgu, g.x, g.perm_token, g.zrow, 2 * g.I, g.H, g.E, g.plan, g.part_gu, g.dwgu,
+                                           g.f32);
+  else if (!TALL || g.tall_d)
+    down(std::integral_constant<int, MT>{});
   else
-    either(g.tall_d, [&](auto mt) {
-      wgrad_block<decltype(mt)::value, NI, true, false, TALL>(ring, block - g.n_dx - g.n_gu, g.d_out, g.hidden, g.perm_token, g.zrow, g.H, g.I, g.E,
-                                                        g.plan, g.part_d, g.dwd, g.f32);
-    });
+    down(std::integral_constant<int, 2>{});
 }
 
 // For the experts that were cut into chunks (none, when the tokens are spread evenly): dW[e] = the sum of expert e's
