@@ -806,12 +806,17 @@ __global__ __launch_bounds__(512) void down_act_kernel(const float* __restrict__
   else body(std::integral_constant<int, 1>{});
 }
 
-// slots a thread of a SCAN kernel looks at, 512 threads
-template <typename Launch>
+// slots a thread of a SCAN kernel looks at, 512 threads; MOST: slots of the largest call that finds its rows itself
+template <int MOST, typename Launch>
 void scan_variant(int S, Launch launch) {
-  if (S <= 8 * 512) launch(std::integral_constant<int, 8>());
-  else if (S <= 16 * 512) launch(std::integral_constant<int, 16>());
-  else launch(std::integral_constant<int, 32>());
+  static_assert(MOST <= 32 * 512, "slots of a scan");
+  if constexpr (MOST > 16 * 512) {
+    if (S > 16 * 512) { launch(std::integral_constant<int, 32>()); return; }
+  }
+  if constexpr (MOST > 8 * 512) {
+    if (S > 8 * 512) { launch(std::integral_constant<int, 16>()); return; }
+  }
+  launch(std::integral_constant<int, 8>());
 }
 
 template <int NT, int CT, int MT>
@@ -830,7 +835,7 @@ void launch_fused_t(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const 
   if constexpr (NT < 4) {                    // (a state-keeping forward has I <= 384)
     if (preact != nullptr) {
       const std::integral_constant<int, 2> train;
-      if (find) scan_variant(S, [&](auto per) { launch(train, bf16_rows, per); });
+      if (find) scan_variant<kScanSlots>(S, [&](auto per) { launch(train, bf16_rows, per); });
       else launch(train, bf16_rows, permuted);
       return;
     }
@@ -841,7 +846,7 @@ void launch_fused_t(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const 
     if (find) launch(forward, std::true_type(), std::integral_constant<int, 8>());
     else launch(forward, std::true_type(), permuted);
   } else if (find) {
-    scan_variant(S, [&](auto per) { launch(forward, bf16_rows, per); });
+    scan_variant<NT == 4 ? kScanSlots / 2 : kScanSlots>(S, [&](auto per) { launch(forward, bf16_rows, per); });
   } else {
     launch(forward, bf16_rows, permuted);
   }
@@ -911,7 +916,7 @@ void launch_raw_nt(const bf16_t* x, const bf16_t* wgu, const int32_t* offsets, c
   const int grid = MODE == 3 || column_blocks > 1 ? ((tiles * column_blocks + 7) & ~7) + 8 : round_tiles_most(S, E, 64 * MT);
   if constexpr (MODE == 3) {
     if (scan.idx != nullptr) {
-      scan_variant(S, [&](auto per) {
+      scan_variant<kSplitSlots>(S, [&](auto per) {
         hipLaunchKernelGGL((experts_fused_kernel<NT, 1, MODE, MT, decltype(per)::value>), dim3(grid), dim3(512), 0, s, x, wgu, nullptr,
                            nullptr, nullptr, nullptr, nullptr, nullptr, H, E, 0, x_bytes, nullptr, gu, column_blocks, scan);
       });

@@ -15,7 +15,7 @@ hipError_t launch_gateup_raw(const void* x, const void* wgu, const int32_t* offs
   const bf16_t* xp = static_cast<const bf16_t*>(x);
   const bf16_t* gp = static_cast<const bf16_t*>(wgu);
   bf16_t* out = static_cast<bf16_t*>(gu);
-  if ((f32 && !split) || (scan.idx != nullptr && !f32)) return hipErrorInvalidValue;
+  if ((f32 && !split) || (scan.idx != nullptr && (!f32 || S > kSplitSlots))) return hipErrorInvalidValue;
   if (f32) {
     launch_raw_nt<1, 3>(xp, gp, offsets, perm_token, S, H, E, xb, out, I / 128, s, scan);
     return hipGetLastError();
@@ -57,7 +57,7 @@ hipError_t launch_gateup_raw(const void* x, const void* wgu, const int32_t* offs
 // Pre-activations in bf16 were 1 to 5 us faster and half again as far from the exact result (3.5e-3 against 2.3e-3).
 bool split_columns(int S, int E, int H, int I) {
   const long long hi = (long long)H * I / 1024;
-  return I >= 256 && S <= 3600 && S <= hi * (46 + E) / 10 && S <= hi * hi * E / (hi <= 256 ? 1100 : 763);
+  return I >= 256 && S <= kSplitSlots && S <= hi * (46 + E) / 10 && S <= hi * hi * E / (hi <= 256 ? 1100 : 763);
 }
 
 // gu [S, 2I] fp32 -> routing-weighted rows in slot order (bf16 or, with f32_rows, fp32), and with `preact` their bf16 copy (down_act_kernel; I <= 384); shapes as

@@ -6,6 +6,8 @@
 
 namespace bibo {
 
+constexpr int kSplitSlots = 3600;       // routed slots up to which a tile's columns may be cut (split_columns)
+
 // MODE 1: pre-activations in bf16; MODE 3: in fp32 (experts_fused_kernel)
 template <int NT>
 void launch_fused_nt(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const float* theta, const float* w,
