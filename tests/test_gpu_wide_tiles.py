@@ -42,6 +42,34 @@ def test_many_slots(H, name):
     assert float((few - got[:1500]).abs().max()) <= 2 * 2.0 ** -7 * top
 
 
+@pytest.mark.parametrize("act", ["radial", "tanh", "silu"])
+@pytest.mark.parametrize("T,H,E,k,n_pos,n_neg", [(1201, 1024, 62, 8, 1, 1), (1500, 256, 9, 6, 0, 0), (4100, 384, 3, 2, 0, 1)])
+def test_what_a_call_may_hold(T, H, E, k, n_pos, n_neg, act):
+    """Every activation, several experts per token, +/-Identity experts and slots without an expert; each token on its own, so that a wrong
+    row of one does not drown in the others."""
+    I, Et = 512, E + n_pos + n_neg
+    assert T * k > 8192
+    p = O.make_inputs(T=T, H=H, E=E, k=k, I=I, theta="normal", seed=T)
+    rng = np.random.default_rng(T)
+    idx = np.argsort(rng.random((T, Et)) + np.linspace(0, 0.2, Et), axis=1)[:, :k].astype(np.int32)
+    w = rng.random((T, k)).astype(np.float32)
+    w_of, bad = w.copy(), idx.copy()
+    for rows, j, e in ((slice(0, None, 3), 1, Et), (slice(1, None, 5), 0, -1), (slice(T - 1, T), slice(None), Et + 7)):
+        bad[rows, j], w_of[rows, j] = e, 0.0
+    ops.workspace(DEV, 64 << 20).fill_(0x7f)                  # an unwritten slot row does not pass by luck
+    out, counts = ops.experts_fwd(p["x"].to(DEV), torch.from_numpy(bad).to(DEV), torch.from_numpy(w).to(DEV),
+                                  *(p[n].to(DEV) for n in ("w_gate_up", "w_down", "theta")), want_counts=True, n_pos=n_pos, n_neg=n_neg, act=act)
+    got = out.float().cpu()
+    ref = O.experts_forward(p["x"], idx, w_of, p["w_gate_up"], p["w_down"], p["theta"], n_pos=n_pos, n_neg=n_neg, act=act).float()
+    assert np.array_equal(counts.cpu().numpy(), np.bincount(bad[(bad >= 0) & (bad < Et)], minlength=Et))
+    assert float((got - ref).abs().max()) <= 2e-2 * float(ref.abs().max())
+    # per token: activation, slot row and output are rounded to bf16, up to 2^-9 each and independent: 3.4e-3 of a slot, and of the sum of k
+    # independent ones; six times that, for slots that cancel
+    size = ref.norm(dim=1) + 1e-3 * float(ref.norm(dim=1).max())
+    assert float(((got - ref).norm(dim=1) / size).max()) <= 2e-2
+    assert not got[T - 1].any()                                # no expert at all
+
+
 def test_x_of_almost_4_gib():
     """Rows of x beyond byte 0xff000000, the last tokens among them: the requests behind the last K step lie past x whatever its size.  A
     row's sums do not depend on its tile, so the ends of the call are the same bits as those tokens alone."""
