@@ -81,7 +81,9 @@ enum bibo_flags {
 
 /* kernel family for the expert GEMMs */
 enum bibo_algo {
-  BIBO_ALGO_AUTO = 0,    /* pick by shape */
+  BIBO_ALGO_AUTO = 0,    /* pick by shape: which kernels run, and so the last bits of a token's output, may go with T, k, E and the
+                            layer's sizes.  In bf16 the limits are, in routed slots T*k: 48 (few tokens), those of streaming and of cut
+                            tiles, and at I = 512 also 8192 */
   BIBO_ALGO_GENERIC = 1, /* fp32 precision, any H and I, bf16 or fp32: tiles of matrix instructions (three bf16 parts per fp32 number,
                             or fp32 ones where experts have few rows) where H and I are multiples of 4 (bf16: and no MFMA tile
                             divides them), else one workgroup per routed row */
