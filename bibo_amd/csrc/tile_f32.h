@@ -334,8 +334,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ggemm_split_kernel(const TA* 
   const integral_constant<int, 1> c1;
   const std::false_type whole;
   const int full = K / kFK;                                      // whole steps
+  // (both: a wave without rows multiplies nothing, and after an odd number of steps what acc[0] happened to hold would count as its sums:
+  // where that was no number the tile was multiplied again, and its last bits went with what had run before)
 #pragma unroll
-  for (int j = 0; j < NTW; ++j) acc[1][j] = none;
+  for (int j = 0; j < NTW; ++j) acc[0][j] = acc[1][j] = none;
   if (full > 0) {
     load(c0, whole, 0);
     load(c1, whole, full > 1 ? kFK : 0);
