@@ -129,10 +129,13 @@ hipError_t launch_ggemm(const bf16_t* A, const int32_t* a_index, const bf16_t* W
   return launch_ggemm_t<1, GATHER, SCATTER>(A, a_index, W, offsets, out_index, S_rows, K, N, E, out, s);
 }
 
-// 256-row tiles stream an expert's weights through LDS half as often as 128-row tiles but take about 1.75 times as
-// long each, and the workgroups of a launch run in rounds of one per CU (256 on this chip): the tall tiles pay when
-// their rounds, weighted so, are fewer.  Only for experts that hold 192 rows on average (a 256-row tile is then at
-// least half full where it matters).
+// 256-row tiles stream an expert's weights through LDS half as often as 128-row tiles, and the workgroups of a launch run in rounds of one
+// per CU (256 on this chip): the tall tiles pay when their rounds, weighted by 1.75, are fewer.  A round of them takes 1.4 to 1.5 times as long
+// where both heights need one, and what the weight leaves out is not worth a call: dh' GEMM, lower -> taller tiles, us, E = 64, k = 6 and
+// rounds in brackets: H = 768, I = 384: 19.4 -> 28.5 (T = 2048, 1 and 1), 21.9 -> 31.4 (4096, 1 and 1), 35.0 -> 31.8 (5000, 2 and 1),
+// 39.8 -> 36.3 (8192, 2 and 1), 59.7 -> 61.6 (12,000, 3 and 2: stays low), 79.9 -> 68.7 (16,384, 4 and 2); H = 512, I = 256: 23.4 -> 20.4 (8192);
+// H = 1024, I = 512: 45.6 -> 38.7 (4000), 77.3 -> 65.1 (8192); H = 640, I = 128: 16.2 -> 16.4 (8192).  Only for experts that hold 192 rows on
+// average (a 256-row tile is then at least half full where it matters).
 inline bool tall_tiles(int S_rows, int E, long long tiles_short, long long tiles_tall) {
   constexpr long long kCUs = 256;
   const long long rs = (tiles_short + kCUs - 1) / kCUs, rt = (tiles_tall + kCUs - 1) / kCUs;

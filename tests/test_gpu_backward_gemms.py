@@ -1,5 +1,5 @@
 """The three products of the backward pass that share a launch (dx of every slot, dW_gate_up, dW_down), on 128-row tiles and on 256-row ones
-(experts of 192 rows and more, several rounds of workgroups), over the widths their workgroups divide into; against autograd in fp32."""
+(experts of 128 rows and more on average, several rounds of workgroups), over the widths their workgroups divide into; against autograd in fp32."""
 import ctypes
 
 import pytest
