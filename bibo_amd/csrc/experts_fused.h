@@ -878,9 +878,10 @@ void launch_down_act_nt(const float* gu, const bf16_t* wd, const float* theta, c
   if (two) launch(integral_constant<int, 1>{}, integral_constant<int, 2>{}); else launch(integral_constant<int, 1>{}, integral_constant<int, 1>{});
 }
 
-// I = 512 has a kernel of its own behind the calls that find their rows themselves.  H = 1024, E = 64, k = 8, layer, this kernel -> that one, on
-// one card: 89.4 -> 89.0 us (T = 1025), 87.8 -> 86.0 (1500), 139.7 -> 133.6 (2047), 150.0 -> 143.6 (3001), 274 -> 257 (6000), 574 -> 541 (16,000);
-// H = 768, E = 32, k = 4: 106.7 -> 102.7 (4100); H = 640, E = 16, k = 2: 55.9 -> 53.9 (4200); H = 512, E = 8, k = 1: 48.1 -> 48.1 (9000).
+// I = 512 has a kernel of its own behind the calls that find their rows themselves.  H = 1024, E = 64, k = 8, layer, this kernel -> that one, the
+// same weights again and again, in turn on one card: 74.2 -> 72.1 us (T = 1025), 77.2 -> 74.6 (1500), 130.7 -> 122.3 (2047), 145.6 -> 137.5 (3001),
+// 264 -> 245 (6000), 582 -> 551 (16,000); H = 768, E = 32, k = 4: 107.6 -> 102.3 (4100); H = 640, E = 16, k = 2: 57.1 -> 53.9 (4200); H = 512, E = 8,
+// k = 1: 48.9 -> 48.9 (9000).  Cards differ, as the clock their power leaves does: T = 3001 on others 150.0 -> 143.6, 149.5 -> 144.6, 140.4 -> 139.3.
 template <int NT>
 void launch_fused_nt(const bf16_t* x, const bf16_t* wgu, const bf16_t* wd, const float* theta, const float* w,
                      const int32_t* offsets, const int32_t* perm_slot, const int32_t* perm_token, int S, int H, int E,

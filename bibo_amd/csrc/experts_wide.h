@@ -2,8 +2,8 @@
 // takes up to 64 permuted rows of one expert through the gate/up projection, Radial NormSiLU and the down projection without the
 // activations leaving the CU.  The same tiles, requests and layout of the activations as experts_fused_kernel, with the instructions of both
 // products in an order of their own.  What bounds it: the weights of an expert, which every 64 of its rows pull through a CU, and the matrix
-// pipes beside them.  H = 1024, E = 64, k = 8, layer, experts_fused_kernel -> this one: 133.8 -> 131.1 us (T = 2049), 263.7 -> 253.1 (6000),
-// 592 -> 568 (16,000); on another card 142 -> 136, 274 -> 257, 574 -> 541.
+// pipes beside them.  H = 1024, E = 64, k = 8, layer, experts_fused_kernel -> this one: 145.6 -> 137.5 us (T = 3001), 264 -> 245 (6000), 582 -> 551
+// (16,000); on other cards 263.7 -> 253.1 and 274 -> 257 (6000), 592 -> 568 and 574 -> 541 (16,000), and between 150.0 -> 143.6 and 140.4 -> 139.3 (3001).
 //
 // Phase 1 (gate/up GEMM, 2 x 4 waves, v_mfma_f32_16x16x32_bf16, operands swapped so that a lane ends up with
 // one ROW's values) walks K in steps of 64 elements, so every row an LDS-DMA instruction fetches is a whole

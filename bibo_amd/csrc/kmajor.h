@@ -70,7 +70,8 @@ __device__ __forceinline__ floatx4 mfma_pair(bf16x8 a, bf16x8 b, floatx4 c) {
 // read may be filled again), and 2 CT MFMAs run while the next stage's first fragments are on their way.  The order is pinned: left to
 // itself the compiler reads a fragment into the registers of the last one and waits for it on the spot.  The loop over a ring's stages has
 // no other way in or out of its middle, because where two ways meet the compiler waits for every transfer before the next LDS read.
-// T = 8192, H = 768, I = 384, E = 64, k = 6: dh' 41.0 -> 35.0 us (pinned order 40.0, with these MFMAs 37.0), backward_gemms_kernel 195 -> 163.
+// T = 8192, H = 768, I = 384, E = 64, k = 6, best times: dh' 41.0 -> 35.0 us (pinned order 40.0, with these MFMAs 37.0), backward_gemms_kernel
+// 195 -> 163.  In traces of training passes on several cards they average 39 to 41 and 181 to 199, cold first pass included.
 template <int RT, int CT, bool ROW_LANES>
 struct StagePipe {
   static constexpr int NA = RT % 3 == 2 ? 3 : 4;           // row fragments in flight; divides the row tiles of a ring
