@@ -24,8 +24,8 @@
 // activations already fill most of the LDS.
 // Each block of columns is scaled by the routing weight, staged through LDS 32 rows at a time (in the two x
 // buffers, which are idle by then) and scattered to slot order as 256-byte row segments.
-// A tile may hold fewer than 128 rows: count_round_tiles chooses the height of a call's tiles by the rounds of the chip they come to, and
-// an expert's last tile takes what is left.  32-row blocks without rows are not multiplied: the kernel body exists once per number of blocks
+// A tile may hold fewer than 128 rows: find_round_tile chooses the heights of a call's tiles by the rounds of the chip they come to, and
+// an expert's last tile may have less.  32-row blocks without rows are not multiplied: the kernel body exists once per number of blocks
 // (1 to 4), with the MFMAs, activations, down projection row tiles and output rounds of the missing blocks left out, and of up to two blocks
 // each M wave takes one; every wave still issues its share of the weight requests, which is most of what a tile costs.
 // Reference: BiBoFusedExperts.forward, src/modeling/ffn/moe.py:81-93.
@@ -258,6 +258,7 @@ __device__ __forceinline__ void down_block(Slice slice, WBlock<CT> (&wb)[NB], co
 // I = 256, k = 6: 30.8 -> 27.5 (T = 256), 33.0 -> 29.1 (800), 38.3 -> 37.0 (2000); H = 768, I = 384: 49.9 -> 47.4, 57.3 -> 54.7,
 // 61.1 -> 60.7; nine experts, k = 2: 31.8 -> 26.5, 30.2 -> 26.6, 32.1 -> 28.4.  Beyond one round of tiles a CU would look twice: level at
 // 16,000 slots of H = 1024, I = 512.
+static_assert(kScanSlots / 128 + kMaxE <= kCUs && kScanSlots / 2 / 64 + kMaxE <= kCUs, "tiles of a call that finds its rows itself fit a round");
 template <int NT, int CT, int MODE = 0, int MTP = 2, int SCAN = 0, bool F32_ROWS = false>
 __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ wgu,
                                                             const bf16_t* __restrict__ wd,
@@ -316,9 +317,6 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
   } else {
     tm = load_tile_map(offsets, E);
   }
-  if (MODE == 3 || ncb > 1) count_tiles(tm, BM);
-  else count_round_tiles<BM>(tm);
-  const int flat = xcd_tile(blockIdx.x, tm.total * ncb);
   if constexpr (SCAN > 0 && MODE >= 2) {
     if (blockIdx.x == 0 && threadIdx.x < (unsigned)E) {   // (also where every slot went to an expert that has no weights)
       scan.offsets[threadIdx.x] = tm.lo;
@@ -326,10 +324,19 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
       if (scan.counts != nullptr) scan.counts[threadIdx.x] = tm.n;
     }
   }
-  if (flat >= tm.total * ncb) return;
-  const int tile = flat / ncb, cb = flat - tile * ncb;
-  int e, row0, rows, tile_e;                            // the same for every lane, in scalar registers
-  find_tile(tm, tile, e, row0, rows, tile_e);
+  int e, first, rows, tile_e, cb = 0;                   // the same for every lane, in scalar registers; first: the tile's first row in its expert
+  if (MODE == 3 || ncb > 1) {
+    count_tiles(tm, BM);
+    const int flat = xcd_tile(blockIdx.x, tm.total * ncb);
+    if (flat >= tm.total * ncb) return;
+    const int tile = flat / ncb;
+    cb = flat - tile * ncb;
+    find_tile(tm, tile, e, first, rows, tile_e);
+    first = tile_e * BM;
+  } else if (!find_round_tile<BM, (SCAN > 0)>(tm, blockIdx.x, e, first, rows, tile_e)) {
+    return;
+  }
+  const int row0 = __builtin_amdgcn_readlane(tm.lo, e) + first;
   // The tiles of an expert walk the weights of a K step from different blocks of columns on: of the tiles that run side by side on an XCD,
   // one pays HBM's latency for a line and the others find it in L2.  A CU keeps about 40 KB of misses in flight, 47 GB/s from HBM and 90
   // from L2.  (Not from different K offsets on: a row's sums would then depend on its place in the tile.)  Layer, weights from HBM, all tiles
@@ -346,7 +353,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
     if (lane == 0) found[wave] = count;
     if (tid < BM) slot_s[tid] = 0;
     __syncthreads();
-    int r0 = -tile_e * tm.height;
+    int r0 = -first;
 #pragma unroll
     for (int v = 0; v < 7; ++v) r0 += v < wave ? found[v] : 0;
 #pragma unroll

@@ -221,12 +221,10 @@ __global__ __launch_bounds__(512) void experts_wide_kernel(const bf16_t* __restr
   __shared__ float rinv_s[BM], gain_s[BM], w_s[BM];
   __shared__ int slot_s[BM];
 
-  TileMap tm = load_tile_map(offsets, E);
-  count_round_tiles<BM>(tm);
-  const int tile = xcd_tile(blockIdx.x, tm.total);
-  if (tile >= tm.total) return;
-  int e, row0, rows, tile_e;                            // the same for every lane, in scalar registers
-  find_tile(tm, tile, e, row0, rows, tile_e);
+  const TileMap tm = load_tile_map(offsets, E);
+  int e, first, rows, tile_e;                           // the same for every lane, in scalar registers
+  if (!find_round_tile<BM, false>(tm, blockIdx.x, e, first, rows, tile_e)) return;
+  const int row0 = __builtin_amdgcn_readlane(tm.lo, e) + first;
   // the tiles of an expert walk the weights of a K step from different blocks of columns on (experts_fused_kernel says why)
   const int rot = tile_e % NT;
   const int nblocks = (rows + 31) >> 5;                 // 32-row blocks that hold rows: 1 or 2

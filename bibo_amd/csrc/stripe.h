@@ -44,26 +44,65 @@ __device__ __forceinline__ TileMap make_tile_map(const int32_t* __restrict__ off
   return tm;
 }
 
-// Tile heights for a kernel whose workgroups fill a CU each, in whole 32-row blocks up to BM.  What a tile costs is first of all the
-// stream of its expert's weights through its CU, whatever its rows (64 experts, H = 768, I = 384, 256 tiles: 38 us at 32 rows, 44 at 64,
-// 50 at 96, 57 at 128), so the rounds of kCUs tiles count first, and within them the height: the lowest tiles that still fit the rounds
-// that tiles of BM rows take.  Counted from the rows as routed: one tile more than a round is a round more.  T = 1024, k = 6: 57 -> 38 us,
-// 2049: 57 -> 45, 3001: 57 -> 50, 6000: 106 -> 88.
+// Tiles for a kernel whose workgroups fill a CU each, up to BM rows in whole 32-row blocks, and the tile of workgroup `bid`, if there is one
+// (first: its first row in its expert).  The rounds of kCUs tiles that tiles of BM rows would take are filled.
+// Heights: all tiles but an expert's last get the least number of blocks with which the call still fits those rounds.  T = 1024, k = 6 (H = 768,
+// I = 384): 57 -> 38 us, 2049: 57 -> 45, 3001: 57 -> 50.  Where two or more quarters of a block less would fit on average (one of 64-row tiles, and
+// those in two rounds), an expert's blocks are spread over so many tiles instead, two heights of them, and no CU waits for a last round of a few
+// tall ones.  (Full rounds take 29, 38, 51 and 67 us at one to four blocks: lower tiles cost a block little more.)  Layer, four layers' weights in
+// turn, one height -> two: T = 12,000: 214.6 -> 205.8 us, the same with four experts that every token picks: 213.2 -> 201.1, 16,384: 280.6 ->
+// 264.7; H = 512, I = 256: 160.1 -> 157.3 (16,384); H = 1024, I = 512, k = 8: 144.6 -> 136.5 (2500), 149.4 -> 147.1 (3001).  For one quarter less
+// the tiles' weights cost what it gives (T = 40,000 and 16,384 of 32 experts: 0 to 2 % slower), and so they do on 64-row tiles in four rounds
+// (T = 6000: 2 %).  In two rounds at T = 8192 it comes to nothing either way.
+// Order: an XCD (ids congruent mod 8) has a contiguous range of the tiles, whose experts' weights share its L2.  (The tall ones in front, so
+// that the CUs end together, brings an expert's weights through the L2 once for each height: with weights from HBM 1 to 2 % slower in two
+// rounds, as fast in three and 5 % slower in eight.)
 constexpr int kCUs = 256, kBlockRows = 32;
-template <int BM>
-__device__ __forceinline__ void count_round_tiles(TileMap& tm) {
+template <int BM, bool ONE_ROUND>
+__device__ __forceinline__ bool find_round_tile(const TileMap& tm, int bid, int& expert, int& first, int& rows, int& tile_e) {
   static_assert(BM == 64 || BM == 128, "two or four blocks");
-  count_tiles(tm, BM);
-  const int room = (int)((unsigned)(tm.total + kCUs - 1) / kCUs * kCUs);
-  count_tiles(tm, kBlockRows);
-  if (tm.total <= room) return;
-  if constexpr (BM == 128) {
-    count_tiles(tm, 2 * kBlockRows);
-    if (tm.total <= room) return;
-    count_tiles(tm, 3 * kBlockRows);
-    if (tm.total <= room) return;
+  constexpr int kMost = BM / kBlockRows;
+  const int blocks = (tm.n + kBlockRows - 1) / kBlockRows;
+  int t = (blocks + kMost - 1) / kMost, incl = wave_inclusive_scan(t), total = __builtin_amdgcn_readlane(incl, kWave - 1);
+  const int rounds = ONE_ROUND ? 1 : (int)((unsigned)(total + kCUs - 1) / kCUs), room = rounds * kCUs;
+  auto fits = [&](unsigned quarters) {       // tiles of so many quarter blocks
+    const int v = (int)((4u * blocks + quarters - 1) / quarters), scan = wave_inclusive_scan(v);
+    const int n = __builtin_amdgcn_readlane(scan, kWave - 1);
+    if (n > room) return false;
+    t = v;
+    incl = scan;
+    total = n;
+    return true;
+  };
+  int low = kMost;                           // blocks of a tile
+#pragma unroll
+  for (int c = 1; c < kMost; ++c) {
+    if (fits(4 * c)) {
+      low = c;
+      break;
+    }
   }
-  count_tiles(tm, BM);
+  bool two = false;
+  if (!ONE_ROUND && rounds > 1 && (kMost == 4 || rounds == 2)) {
+    const unsigned all = __builtin_amdgcn_readlane(wave_inclusive_scan(blocks), kWave - 1);
+    for (unsigned quarters = max(4u * low - 3, (4u * all + room - 1) / (unsigned)room); quarters <= 4u * low - (kMost == 4 ? 2 : 1) && !two; ++quarters)
+      two = fits(quarters);
+  }
+  const int at = xcd_tile(bid, total);
+  if (at >= total) return false;
+  int tall = 0;                              // with two heights, tall tiles of low + 1 blocks, then the others of `low` blocks
+  if (two) {
+    low = 0;
+#pragma unroll
+    for (int c = 1; c <= kMost; ++c) low += blocks >= c * t;
+    tall = blocks - low * t;
+  }
+  expert = __ffsll((long long)__ballot(incl > at)) - 1;
+  tile_e = at - (__builtin_amdgcn_readlane(incl, expert) - __builtin_amdgcn_readlane(t, expert));
+  const int l = __builtin_amdgcn_readlane(low, expert), h = __builtin_amdgcn_readlane(tall, expert);
+  first = (tile_e * l + min(tile_e, h)) * kBlockRows;
+  rows = min((l + (tile_e < h)) * kBlockRows, __builtin_amdgcn_readlane(tm.n, expert) - first);
+  return true;
 }
 // What such a map can come to, for the grid: the rounds that tiles of BM rows are sure to fit, or every tile at its lowest.
 inline int round_tiles_most(int S, int E, int BM) {
@@ -71,8 +110,7 @@ inline int round_tiles_most(int S, int E, int BM) {
   return (int)((rounds * kCUs < low ? rounds * kCUs : low) + 7) & ~7;
 }
 
-// tile < tm.total required; tile_e: which of its expert's tiles it is.  (Rows spread evenly over an expert's tiles were 1 to 2 us slower:
-// the short last tiles end early.)
+// tile < tm.total required; tile_e: which of its expert's tiles it is
 __device__ __forceinline__ void find_tile(const TileMap& tm, int tile, int& expert, int& row0, int& rows, int& tile_e) {
   expert = __ffsll((long long)__ballot(tm.incl > tile)) - 1;
   tile_e = tile - (__builtin_amdgcn_readlane(tm.incl, expert) - __builtin_amdgcn_readlane(tm.ntile, expert));
