@@ -219,7 +219,7 @@ int experts_dispatch(const void* x, const void* wgu, const void* wd, const float
                      const void* residual, bool idx_trusted, int T, int H, int Eg, int np, int nn, int k, int I, int dtype,
                      int algo, int act, int flags, void* out, char* base, const Workspace& ws, size_t ws_bytes,
                      hipStream_t s, bool f32_rows = false, void* preact = nullptr, const ScanArgs& scan = ScanArgs(),
-                     bool gate_up_done = false) {
+                     bool gate_up_done = false, float* keep_gu = nullptr) {
   float* yw = reinterpret_cast<float*>(base + ws.yw);
   CombineArgs ca;
   ca.residual = residual;
@@ -261,8 +261,8 @@ int experts_dispatch(const void* x, const void* wgu, const void* wd, const float
   // (a bf16 shape of the MFMA families that a caller asks the generic one for runs the row kernels, like the stage calls)
   if (algo == BIBO_ALGO_GENERIC && generic_tiles(H, I, dtype) && aligned16(x) && aligned16(wgu) && aligned16(wd) &&
       ws_bytes >= ws.total) {
-    hipError_t e = launch_experts_tiled(x, wgu, wd, theta, w, offsets, perm_slot, perm_token, T, H, Eg, k, I, dtype, act, yw,
-                                        base + ws.hidden, yw, s);
+    hipError_t e = launch_experts_tiled(x, wgu, wd, theta, w, offsets, perm_slot, perm_token, T, H, Eg, k, I, dtype, act,
+                                        keep_gu != nullptr ? keep_gu : yw, base + ws.hidden, yw, s);
     if (e != hipSuccess) return (int)e;
     return hip_rc(launch_combine(yw, 0, ca, T, H, k, dtype, out, s));
   }
@@ -272,12 +272,26 @@ int experts_dispatch(const void* x, const void* wgu, const void* wd, const float
 }
 
 // What a training forward leaves for its backward pass in a caller-owned buffer: the routing (selection, combine
-// weights, fp32 logits), the permutation and the bf16 gate/up pre-activations of every routed row.
+// weights, fp32 logits), the permutation and, of every routed row, the gate/up pre-activations: in bf16 where the fused forward kernel
+// and the MFMA backward both take the shape; where a caller asks for every shape, in fp32 if the tile kernels of the generic family run,
+// whose forward has them in memory anyway, and else none.
+enum class Keeps { kNothing, kBf16, kF32, kRouting };
+
+Keeps kept_state(const bibo_moe_shape* sh) {
+  const bool fast = backward_supported(sh->H, sh->I, sh->k, sh->dtype);      // the MFMA backward family
+  if (fast && fused_supported(sh->H, sh->I, sh->dtype) && fused_fits(sh->T, sh->H)) return Keeps::kBf16;
+  if ((sh->flags & BIBO_FLAG_KEEP_ANY) == 0) return Keeps::kNothing;
+  int algo;
+  const bool tiled = resolve_algo(BIBO_ALGO_AUTO, sh->T, sh->H, sh->E, sh->k, sh->I, sh->dtype, true, true, &algo) == BIBO_OK &&
+                     algo == BIBO_ALGO_GENERIC && generic_tiles(sh->H, sh->I, sh->dtype) && !few_supported(sh->T, sh->H, sh->k, sh->I);
+  return !fast && tiled ? Keeps::kF32 : Keeps::kRouting;
+}
+
 struct TrainState {
   size_t idx, w, logits, offsets, perm_slot, perm_token, gu, total;
 };
 
-TrainState carve_state(int T, int E, int k, int I) {
+TrainState carve_state(int T, int E, int k, int I, Keeps keeps) {
   const size_t S = (size_t)T * k;
   TrainState st;
   size_t o = 0;
@@ -287,7 +301,7 @@ TrainState carve_state(int T, int E, int k, int I) {
   st.offsets = o;    o += align_up((kMaxE + 1) * sizeof(int32_t));
   st.perm_slot = o;  o += align_up(S * sizeof(int32_t));
   st.perm_token = o; o += align_up(S * sizeof(int32_t));
-  st.gu = o;         o += align_up(S * 2 * (size_t)I * sizeof(bf16_t));
+  st.gu = o;         o += align_up(S * 2 * (size_t)I * (keeps == Keeps::kBf16 ? sizeof(bf16_t) : keeps == Keeps::kF32 ? sizeof(float) : 0));
   st.total = o;
   return st;
 }
@@ -327,19 +341,22 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
   int32_t* perm_slot = reinterpret_cast<int32_t*>(base + ws.perm_slot);
   int32_t* perm_token = reinterpret_cast<int32_t*>(base + ws.perm_token);
   void* preact = nullptr;
+  float* keep_gu = nullptr;
   if (state != nullptr) {                // a training forward: what the backward pass needs lands in the caller's state buffer
-    const TrainState st = carve_state(T, E, k, I);
+    const Keeps keeps = kept_state(sh);
+    const TrainState st = carve_state(T, E, k, I, keeps);
     idx = reinterpret_cast<int32_t*>(state + st.idx);
     w = reinterpret_cast<float*>(state + st.w);
     logits_out = reinterpret_cast<float*>(state + st.logits);
     offsets = reinterpret_cast<int32_t*>(state + st.offsets);
     perm_slot = reinterpret_cast<int32_t*>(state + st.perm_slot);
     perm_token = reinterpret_cast<int32_t*>(state + st.perm_token);
-    preact = state + st.gu;
+    if (keeps == Keeps::kBf16) preact = state + st.gu;
+    if (keeps == Keeps::kF32) keep_gu = reinterpret_cast<float*>(state + st.gu);
   }
   // the streaming and few-token kernels find their rows themselves; the permutation then only serves the counts
   const bool few = few_taken(a, T, H, k, I, dtype, x, w_gate_up, w_down);
-  const bool need_permute = (a != BIBO_ALGO_STREAM && !few) || counts_out != nullptr || T == 0;
+  const bool need_permute = (a != BIBO_ALGO_STREAM && !few) || counts_out != nullptr || state != nullptr || T == 0;
   // the router kernel can leave per-workgroup histograms of its selections, which save the permutation its
   // histogram launch and its counting pass
   int32_t* hist = reinterpret_cast<int32_t*>(base + ws.hist);
@@ -348,7 +365,7 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
   // with few slots, the fused kernel and its first half find their rows themselves; of a permutation they leave what a backward pass reads
   const bool may_scan = (a == BIBO_ALGO_FUSED || a == kAlgoFusedWide || a == kAlgoSplit) && T > 0 &&
                         (long long)T * k <= (a == BIBO_ALGO_FUSED ? kScanSlots : kScanSlots / 2) &&
-                        (state != nullptr ? Eg == E : counts_out == nullptr) && aligned16(x) && aligned16(w_gate_up) && aligned16(w_down);
+                        (state != nullptr ? Eg == E && (preact != nullptr || a == kAlgoSplit) : counts_out == nullptr) && aligned16(x) && aligned16(w_gate_up) && aligned16(w_down);
   const bool want_hist = may_scan || (need_permute && T > 0 && permute_takes_router_hist(T, k));
   const void* rows = norm_src != nullptr ? norm_src : x;
   void* xn = norm_src != nullptr ? const_cast<void*>(x) : nullptr;
@@ -387,7 +404,7 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
   if (T == 0) return BIBO_OK;
   return experts_dispatch(x, w_gate_up, w_down, theta, idx, w, offsets, perm_slot, perm_token, residual, true, T, H, Eg,
                           sh->n_pos, sh->n_neg, k, I, dtype, a, sh->act, sh->flags, out, base, ws, workspace_bytes, s, f32_rows, preact, scan,
-                          gate_up_done);
+                          gate_up_done, keep_gu);
 }
 
 
@@ -486,14 +503,15 @@ int backward_mfma(const void* x, const void* d_out, const void* w_router, const 
   const int32_t* idx; const float* w; const float* logits; const int32_t* offsets; const int32_t* perm_slot;
   const int32_t* perm_token; const void* gu_saved = nullptr;
   if (state != nullptr) {
-    const TrainState st = carve_state(T, E, k, I);
+    const Keeps keeps = kept_state(sh);
+    const TrainState st = carve_state(T, E, k, I, keeps);
     idx = reinterpret_cast<const int32_t*>(state + st.idx);
     w = reinterpret_cast<const float*>(state + st.w);
     logits = reinterpret_cast<const float*>(state + st.logits);
     offsets = reinterpret_cast<const int32_t*>(state + st.offsets);
     perm_slot = reinterpret_cast<const int32_t*>(state + st.perm_slot);
     perm_token = reinterpret_cast<const int32_t*>(state + st.perm_token);
-    gu_saved = state + st.gu;
+    if (keeps == Keeps::kBf16) gu_saved = state + st.gu;
   } else {
     int32_t* idx_w = reinterpret_cast<int32_t*>(base + ws.idx);
     float* w_w = reinterpret_cast<float*>(base + ws.w);
@@ -529,9 +547,55 @@ int backward_mfma(const void* x, const void* d_out, const void* w_router, const 
                                 d_w_router, d_w_gate_up, d_w_down, d_theta, (sh->flags & BIBO_FLAG_GRAD_F32) != 0, s, gu_saved));
 }
 
-// whether a shape has the training forward that keeps its state: the fused forward kernel and the MFMA backward both take it
-inline bool train_state_supported(const bibo_moe_shape* sh) {
-  return backward_fast(sh) && fused_supported(sh->H, sh->I, sh->dtype) && fused_fits(sh->T, sh->H);
+// The generic family, likewise.
+int backward_generic(const void* x, const void* d_out, const void* w_router, const float* bias, const void* w_gate_up, const void* w_down,
+                     const float* theta, const bibo_moe_shape* sh, int norm_mode, const char* state, void* d_x, void* d_w_router,
+                     void* d_w_gate_up, void* d_w_down, float* d_theta, float* d_w_out, void* workspace, size_t workspace_bytes,
+                     void* stream) {
+  const int T = sh->T, H = sh->H, E = sh->E, k = sh->k, I = sh->I;
+  const GenericBackwardWorkspace ws = carve_backward_generic(T, H, E, k, I);
+  if (workspace_bytes < ws.total) return BIBO_ERR_WORKSPACE_TOO_SMALL;
+  char* base = static_cast<char*>(workspace);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int32_t* idx; const float* w; const float* logits; const int32_t* offsets; const int32_t* perm_slot; const int32_t* perm_token;
+  GenericBackwardBuffers b;
+  if (state != nullptr) {
+    const Keeps keeps = kept_state(sh);
+    const TrainState st = carve_state(T, E, k, I, keeps);
+    idx = reinterpret_cast<const int32_t*>(state + st.idx);
+    w = reinterpret_cast<const float*>(state + st.w);
+    logits = reinterpret_cast<const float*>(state + st.logits);
+    offsets = reinterpret_cast<const int32_t*>(state + st.offsets);
+    perm_slot = reinterpret_cast<const int32_t*>(state + st.perm_slot);
+    perm_token = reinterpret_cast<const int32_t*>(state + st.perm_token);
+    if (keeps == Keeps::kF32) b.gu_saved = reinterpret_cast<const float*>(state + st.gu);
+  } else {
+    int32_t* idx_w = reinterpret_cast<int32_t*>(base + ws.idx);
+    float* w_w = reinterpret_cast<float*>(base + ws.w);
+    float* logits_w = reinterpret_cast<float*>(base + ws.logits);
+    int32_t* offsets_w = reinterpret_cast<int32_t*>(base + ws.offsets);
+    int32_t* slot_w = reinterpret_cast<int32_t*>(base + ws.perm_slot);
+    int32_t* token_w = reinterpret_cast<int32_t*>(base + ws.perm_token);
+    int32_t* counts = reinterpret_cast<int32_t*>(base + ws.counts);
+    int32_t* hist = reinterpret_cast<int32_t*>(base + ws.hist);
+    int hist_tokens = 0, rc;
+    const bool want_hist = T > 0 && permute_takes_router_hist(T, k);
+    if (T > 0 && (rc = hip_rc(launch_router(x, w_router, bias, T, H, E, k, sh->dtype, norm_mode, logits_w, idx_w, w_w, nullptr,
+                                            want_hist ? hist : nullptr, &hist_tokens, s))) != BIBO_OK)
+      return rc;
+    if ((rc = hip_rc((want_hist && hist_tokens > 0)
+                         ? launch_permute_from_hist(idx_w, T, E, k, hist, hist_tokens, counts, offsets_w, slot_w, token_w, s)
+                         : launch_permute(idx_w, T, E, k, counts, offsets_w, slot_w, token_w, hist, s))) != BIBO_OK)
+      return rc;
+    idx = idx_w; w = w_w; logits = logits_w; offsets = offsets_w; perm_slot = slot_w; perm_token = token_w;
+  }
+  b.dgu = reinterpret_cast<float*>(base + ws.dgu); b.hw = reinterpret_cast<float*>(base + ws.hw);
+  b.dxs = reinterpret_cast<float*>(base + ws.dxs);
+  b.dw_slot = d_w_out ? d_w_out : reinterpret_cast<float*>(base + ws.dw_slot);
+  b.dl = reinterpret_cast<float*>(base + ws.dl); b.dtheta_row = reinterpret_cast<float*>(base + ws.dtheta_row);
+  return hip_rc(launch_backward_generic(x, d_out, w_router, w_gate_up, w_down, theta, logits, idx, w, offsets, perm_slot, perm_token, T, H,
+                                        E - sh->n_pos - sh->n_neg, sh->n_pos, sh->n_neg, k, I, sh->dtype, norm_mode, sh->act, b, d_x,
+                                        d_w_router, d_w_gate_up, d_w_down, d_theta, (sh->flags & BIBO_FLAG_GRAD_F32) != 0, s));
 }
 
 }  // namespace
@@ -784,45 +848,17 @@ int bibo_moe_backward(const void* x, const void* d_out, const void* w_router, co
                       const void* w_down, const float* theta, const bibo_moe_shape* sh, int norm_mode, void* d_x,
                       void* d_w_router, void* d_w_gate_up, void* d_w_down, float* d_theta, float* d_w_out,
                       void* workspace, size_t workspace_bytes, void* stream) {
-  int rc = backward_check(sh, norm_mode);
+  const int rc = backward_check(sh, norm_mode);
   if (rc != BIBO_OK) return rc;
-  const int T = sh->T, H = sh->H, E = sh->E, k = sh->k, I = sh->I;
+  const int T = sh->T;
   if (!workspace) return BIBO_ERR_NULL_POINTER;
   if (!aligned_ws(workspace)) return BIBO_ERR_MISALIGNED;
   if (!d_w_router || !d_w_gate_up || !d_w_down || !d_theta) return BIBO_ERR_NULL_POINTER;
   if (T > 0 && (!x || !d_out || !w_router || !bias || !w_gate_up || !w_down || !d_x)) return BIBO_ERR_NULL_POINTER;
   if (T > 0 && !theta && sh->act != BIBO_ACT_SILU) return BIBO_ERR_NULL_POINTER;
   if (!backward_fast(sh)) {
-    const GenericBackwardWorkspace gw = carve_backward_generic(T, H, E, k, I);
-    if (workspace_bytes < gw.total) return BIBO_ERR_WORKSPACE_TOO_SMALL;
-    char* gb = static_cast<char*>(workspace);
-    hipStream_t gs = static_cast<hipStream_t>(stream);
-    int32_t* g_idx = reinterpret_cast<int32_t*>(gb + gw.idx);
-    float* g_w = reinterpret_cast<float*>(gb + gw.w);
-    float* g_logits = reinterpret_cast<float*>(gb + gw.logits);
-    int32_t* g_offsets = reinterpret_cast<int32_t*>(gb + gw.offsets);
-    int32_t* g_slot = reinterpret_cast<int32_t*>(gb + gw.perm_slot);
-    int32_t* g_token = reinterpret_cast<int32_t*>(gb + gw.perm_token);
-    int32_t* g_counts = reinterpret_cast<int32_t*>(gb + gw.counts);
-    int32_t* g_hist = reinterpret_cast<int32_t*>(gb + gw.hist);
-    int hist_tokens = 0;
-    const bool want_hist = T > 0 && permute_takes_router_hist(T, k);
-    if (T > 0 && (rc = hip_rc(launch_router(x, w_router, bias, T, H, E, k, sh->dtype, norm_mode, g_logits, g_idx, g_w, nullptr,
-                                            want_hist ? g_hist : nullptr, &hist_tokens, gs))) != BIBO_OK)
-      return rc;
-    if ((rc = hip_rc((want_hist && hist_tokens > 0)
-                         ? launch_permute_from_hist(g_idx, T, E, k, g_hist, hist_tokens, g_counts, g_offsets, g_slot, g_token, gs)
-                         : launch_permute(g_idx, T, E, k, g_counts, g_offsets, g_slot, g_token, g_hist, gs))) != BIBO_OK)
-      return rc;
-    GenericBackwardBuffers g;
-    g.dgu = reinterpret_cast<float*>(gb + gw.dgu); g.hw = reinterpret_cast<float*>(gb + gw.hw);
-    g.dxs = reinterpret_cast<float*>(gb + gw.dxs);
-    g.dw_slot = d_w_out ? d_w_out : reinterpret_cast<float*>(gb + gw.dw_slot);
-    g.dl = reinterpret_cast<float*>(gb + gw.dl); g.dtheta_row = reinterpret_cast<float*>(gb + gw.dtheta_row);
-    return hip_rc(launch_backward_generic(x, d_out, w_router, w_gate_up, w_down, theta, g_logits, g_idx, g_w, g_offsets, g_slot,
-                                          g_token, T, H, E - sh->n_pos - sh->n_neg, sh->n_pos, sh->n_neg, k, I, sh->dtype,
-                                          norm_mode, sh->act, g, d_x, d_w_router, d_w_gate_up, d_w_down, d_theta,
-                                          (sh->flags & BIBO_FLAG_GRAD_F32) != 0, gs));
+    return backward_generic(x, d_out, w_router, bias, w_gate_up, w_down, theta, sh, norm_mode, nullptr, d_x, d_w_router, d_w_gate_up,
+                            d_w_down, d_theta, d_w_out, workspace, workspace_bytes, stream);
   }
   return backward_mfma(x, d_out, w_router, bias, w_gate_up, w_down, theta, sh, norm_mode, nullptr, d_x, d_w_router,
                        d_w_gate_up, d_w_down, d_theta, d_w_out, workspace, workspace_bytes, stream);
@@ -832,8 +868,9 @@ int bibo_moe_train_state_bytes(const bibo_moe_shape* sh, size_t* bytes) {
   if (bytes == nullptr) return BIBO_ERR_NULL_POINTER;
   const int rc = backward_check(sh, BIBO_NORM_SUM);
   if (rc != BIBO_OK) return rc;
-  if (!train_state_supported(sh)) return BIBO_ERR_UNSUPPORTED;
-  *bytes = carve_state(sh->T, sh->E, sh->k, sh->I).total;
+  const Keeps keeps = kept_state(sh);
+  if (keeps == Keeps::kNothing) return BIBO_ERR_UNSUPPORTED;
+  *bytes = carve_state(sh->T, sh->E, sh->k, sh->I, keeps).total;
   return BIBO_OK;
 }
 
@@ -842,12 +879,17 @@ int bibo_moe_forward_train(const void* x, const void* w_router, const float* bia
                            void* state, size_t state_bytes, void* workspace, size_t workspace_bytes, void* stream) {
   const int rc = backward_check(sh, norm_mode);
   if (rc != BIBO_OK) return rc;
-  if (!train_state_supported(sh)) return BIBO_ERR_UNSUPPORTED;
+  const Keeps keeps = kept_state(sh);
+  if (keeps == Keeps::kNothing) return BIBO_ERR_UNSUPPORTED;
   if (state == nullptr) return BIBO_ERR_NULL_POINTER;
   if (!aligned_ws(state)) return BIBO_ERR_MISALIGNED;
-  if (state_bytes < carve_state(sh->T, sh->E, sh->k, sh->I).total) return BIBO_ERR_WORKSPACE_TOO_SMALL;
-  return forward_impl(x, w_router, bias, w_gate_up, w_down, theta, sh, norm_mode, BIBO_ALGO_FUSED, nullptr, out, nullptr,
-                      nullptr, counts_out, nullptr, workspace, workspace_bytes, stream, nullptr, Vec{nullptr, 0}, 0.f,
+  if (state_bytes < carve_state(sh->T, sh->E, sh->k, sh->I, keeps).total) return BIBO_ERR_WORKSPACE_TOO_SMALL;
+  if (keeps != Keeps::kBf16) {             // (the tile kernels, whose pre-activations are kept, need both)
+    if (!aligned16(x) || !aligned16(w_gate_up) || !aligned16(w_down)) return BIBO_ERR_MISALIGNED;
+    if (workspace_bytes < carve(sh->T, sh->H, sh->E, sh->k, sh->I, sh->dtype).total) return BIBO_ERR_WORKSPACE_TOO_SMALL;
+  }
+  return forward_impl(x, w_router, bias, w_gate_up, w_down, theta, sh, norm_mode, keeps == Keeps::kBf16 ? BIBO_ALGO_FUSED : BIBO_ALGO_AUTO,
+                      nullptr, out, nullptr, nullptr, counts_out, nullptr, workspace, workspace_bytes, stream, nullptr, Vec{nullptr, 0}, 0.f,
                       static_cast<char*>(state));
 }
 
@@ -857,16 +899,18 @@ int bibo_moe_backward_saved(const void* x, const void* d_out, const void* w_rout
                             float* d_theta, float* d_w_out, void* workspace, size_t workspace_bytes, void* stream) {
   const int rc = backward_check(sh, norm_mode);
   if (rc != BIBO_OK) return rc;
-  if (!train_state_supported(sh)) return BIBO_ERR_UNSUPPORTED;
+  const Keeps keeps = kept_state(sh);
+  if (keeps == Keeps::kNothing) return BIBO_ERR_UNSUPPORTED;
   const int T = sh->T;
   if (!workspace || !state) return BIBO_ERR_NULL_POINTER;
   if (!aligned_ws(workspace) || !aligned_ws(state)) return BIBO_ERR_MISALIGNED;
-  if (state_bytes < carve_state(T, sh->E, sh->k, sh->I).total) return BIBO_ERR_WORKSPACE_TOO_SMALL;
+  if (state_bytes < carve_state(T, sh->E, sh->k, sh->I, keeps).total) return BIBO_ERR_WORKSPACE_TOO_SMALL;
   if (!d_w_router || !d_w_gate_up || !d_w_down || !d_theta) return BIBO_ERR_NULL_POINTER;
   if (T > 0 && (!x || !d_out || !w_router || !w_gate_up || !w_down || !d_x)) return BIBO_ERR_NULL_POINTER;
   if (T > 0 && !theta && sh->act != BIBO_ACT_SILU) return BIBO_ERR_NULL_POINTER;
-  return backward_mfma(x, d_out, w_router, nullptr, w_gate_up, w_down, theta, sh, norm_mode, static_cast<const char*>(state),
-                       d_x, d_w_router, d_w_gate_up, d_w_down, d_theta, d_w_out, workspace, workspace_bytes, stream);
+  return (backward_fast(sh) ? backward_mfma : backward_generic)(x, d_out, w_router, nullptr, w_gate_up, w_down, theta, sh, norm_mode,
+                                                                static_cast<const char*>(state), d_x, d_w_router, d_w_gate_up, d_w_down,
+                                                                d_theta, d_w_out, workspace, workspace_bytes, stream);
 }
 
 int bibo_moe_experts_backward(const void* x, const void* d_out, const int32_t* idx, const float* w, const void* w_gate_up,

@@ -122,10 +122,10 @@ __global__ __launch_bounds__(256) void row_bwd_generic_kernel(const TIn* __restr
   }
 }
 
-// Radial NormSiLU backward of one permuted row per wave (formulas at the top of row_bwd_generic_kernel and backward.hip), in
-// place: gu [S, 2I] holds [g, u] and receives [dg, du], dhp [S, I] holds dh' and receives w h.  The row is read three times,
+// Radial NormSiLU backward of one permuted row per wave (formulas at the top of row_bwd_generic_kernel and backward.hip): gu [S, 2I] holds
+// [g, u], dgu receives [dg, du] (it may be gu), dhp [S, I] holds dh' and receives w h.  The row is read three times,
 // from L1 after the first.
-__global__ __launch_bounds__(256) void act_bwd_f32_kernel(float* __restrict__ gu, float* __restrict__ dhp,
+__global__ __launch_bounds__(256) void act_bwd_f32_kernel(const float* gu, float* dgu, float* __restrict__ dhp,
                                                           const float* __restrict__ w, const float* __restrict__ theta,
                                                           const int32_t* __restrict__ offsets,
                                                           const int32_t* __restrict__ perm_slot, int S, int E, int I, int act,
@@ -137,7 +137,8 @@ __global__ __launch_bounds__(256) void act_bwd_f32_kernel(float* __restrict__ gu
   if (e < 0) return;
   const int slot = perm_slot[row];
   const float ws = w[slot];
-  float* gr = gu + (size_t)row * 2 * I;
+  const float* gr = gu + (size_t)row * 2 * I;
+  float* go = dgu + (size_t)row * 2 * I;
   float* dr = dhp + (size_t)row * I;
   float ss = 0.f;
   for (int c = lane * 4; c < I; c += 4 * kWave) {
@@ -184,8 +185,8 @@ __global__ __launch_bounds__(256) void act_bwd_f32_kernel(float* __restrict__ gu
       ou[q] = dh * gain * a;
       oh[q] = (float)((double)ws * gain * a * u[q]);
     }
-    store4(gr + c, og);
-    store4(gr + I + c, ou);
+    store4(go + c, og);
+    store4(go + I + c, ou);
     store4(dr + c, oh);
   }
   if (lane == 0) {
@@ -372,11 +373,15 @@ hipError_t launch_t(const void* x_, const void* d_out_, const void* w_router_, c
                                                     reinterpret_cast<uintptr_t>(wgu) | reinterpret_cast<uintptr_t>(wd)) & 15) == 0;
   hipError_t err = hipSuccess;
   if (tiles) {
-    // gu = x W_gate_up^T; dh' = d W_down; [dg, du] and w h in their places; dx of every slot = [dg, du] W_gate_up
-    if ((err = launch_ggemm_f32<TIn, TIn, false, true, false>(x, perm_token, wgu, offsets, nullptr, nullptr, S, H, 2 * I, E, b.dgu, s)) != hipSuccess) return err;
+    // gu = x W_gate_up^T, where the forward has not kept it; dh' = d W_down; [dg, du] and w h in their places; dx of every slot = [dg, du] W_gate_up
+    const float* gu = b.gu_saved;
+    if (gu == nullptr) {
+      gu = b.dgu;
+      if ((err = launch_ggemm_f32<TIn, TIn, false, true, false>(x, perm_token, wgu, offsets, nullptr, nullptr, S, H, 2 * I, E, b.dgu, s)) != hipSuccess) return err;
+    }
     if ((err = launch_ggemm_f32<TIn, TIn, true, true, false>(d_out, perm_token, wd, offsets, nullptr, nullptr, S, H, I, E, b.hw, s)) != hipSuccess) return err;
-    hipLaunchKernelGGL(act_bwd_f32_kernel, dim3((S + 3) / 4), dim3(256), 0, s, b.dgu, b.hw, w, theta, offsets, perm_slot, S, E, I, act,
-                       b.dw_slot, b.dtheta_row);
+    hipLaunchKernelGGL(act_bwd_f32_kernel, dim3((S + 3) / 4), dim3(256), 0, s, gu, b.dgu, b.hw, w, theta, offsets, perm_slot, S, E, I,
+                       act, b.dw_slot, b.dtheta_row);
     if ((err = launch_ggemm_f32<float, TIn, true, false, true>(b.dgu, nullptr, wgu, offsets, perm_slot, nullptr, S, 2 * I, H, E, b.dxs, s)) != hipSuccess) return err;
   } else {
     const size_t shm = (size_t)(2 * H + 5 * I) * sizeof(float);

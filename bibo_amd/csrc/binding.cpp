@@ -238,10 +238,11 @@ py::tuple ffn_forward(const Tensor& h, const Tensor& norm_weight, double eps, co
 
 // ---- training: the whole layer as one autograd node --------------------------------------------------------------
 // Gradients are what autograd gives the reference's eager layer with the selection held fixed (moe.py:157-183); the
-// balancing bias gets none (router.py:38).  Two ways through the library: with `keep` and a shape that has the pair,
-// forward = bibo_moe_forward_train, which leaves routing, permutation and pre-activations in a state tensor (about 4 I
-// bytes per routed slot), and backward = bibo_moe_backward_saved; otherwise forward = bibo_moe_forward and backward =
-// bibo_moe_backward, which computes all of that again from the saved input rows.  The same gradients, bit for bit.
+// balancing bias gets none (router.py:38).  Two ways through the library: with `keep`,
+// forward = bibo_moe_forward_train, which leaves routing, permutation and, for most shapes, pre-activations in a state tensor (about 4 I
+// bytes per routed slot, 8 I for the fp32 tile kernels), and backward = bibo_moe_backward_saved; otherwise forward = bibo_moe_forward and
+// backward = bibo_moe_backward, which computes all of that again from the saved input rows.  The same gradients, bit for bit.
+// H = 192, I = 88, 16 experts, k = 3, T = 777 in fp32, forward and backward: 19 launches without, 15 with.
 struct TrainCall {
   Layer l;               // kernel-dtype copies of the parameters (the parameters themselves where they have that dtype)
   at::ScalarType compute;
@@ -256,7 +257,10 @@ class LayerFn : public torch::autograd::Function<LayerFn> {
     const Layer& l = c->l;
     const Tensor xb = in_dtype(x, c->compute);
     // a family that was asked for by name runs in training as well
-    const bibo_moe_shape sh = shape_of(xb, l, l.algo == BIBO_ALGO_AUTO ? BIBO_FLAG_TRAIN_AUTO : 0);
+    const bool aligned = ((reinterpret_cast<uintptr_t>(xb.data_ptr()) | reinterpret_cast<uintptr_t>(l.w_gate_up.data_ptr()) |
+                           reinterpret_cast<uintptr_t>(l.w_down.data_ptr())) & 15) == 0;
+    const int any = aligned ? BIBO_FLAG_KEEP_ANY : 0;
+    const bibo_moe_shape sh = shape_of(xb, l, l.algo == BIBO_ALGO_AUTO ? BIBO_FLAG_TRAIN_AUTO | any : 0);
     Tensor out = at::empty_like(xb);
     hipStream_t s = c10::hip::getCurrentHIPStream(xb.device().index()).stream();
     size_t bytes = 0, state_bytes = 0;
@@ -283,7 +287,7 @@ class LayerFn : public torch::autograd::Function<LayerFn> {
     }
     ctx->save_for_backward({xb, l.w_router, l.w_gate_up, l.w_down, l.theta, last});
     auto& d = ctx->saved_data;
-    d["conf"] = std::vector<int64_t>{l.k, l.norm, l.n_pos, l.n_neg, l.act, saved ? 1 : 0};
+    d["conf"] = std::vector<int64_t>{l.k, l.norm, l.n_pos, l.n_neg, l.act, saved ? 1 : 0, sh.flags & BIBO_FLAG_KEEP_ANY};
     d["dtypes"] = std::vector<int64_t>{(int64_t)x.scalar_type(), (int64_t)w_router.scalar_type(), (int64_t)w_gate_up.scalar_type(),
                                        (int64_t)w_down.scalar_type(), (int64_t)theta.scalar_type()};
     return out;
@@ -305,7 +309,7 @@ class LayerFn : public torch::autograd::Function<LayerFn> {
                           dtypes[3] == (int64_t)at::kFloat;
     const bibo_moe_shape sh{(int32_t)(x.numel() / x.size(-1)), (int32_t)x.size(-1), (int32_t)(Eg + l.n_pos + l.n_neg), l.k,
                             (int32_t)(l.w_gate_up.size(1) / 2), dtype_code(x), l.n_pos, l.n_neg, l.act,
-                            grad_f32 ? BIBO_FLAG_GRAD_F32 : 0};
+                            (grad_f32 ? BIBO_FLAG_GRAD_F32 : 0) | (int)conf[6]};
     const at::TensorOptions wopt = l.w_gate_up.options().requires_grad(false).dtype(grad_f32 ? at::kFloat : x.scalar_type());
     Tensor d_x = at::empty_like(x), d_wr = at::empty(l.w_router.sizes(), wopt), d_gu = at::empty(l.w_gate_up.sizes(), wopt),
            d_dn = at::empty(l.w_down.sizes(), wopt), d_th = at::empty_like(l.theta);

@@ -319,6 +319,7 @@ int backward_dwr_split();
 struct GenericBackwardBuffers {
   float *dgu, *hw, *dxs;                                            // [S,2I], [S,I], [S,H]
   float *dw_slot, *dl, *dtheta_row;                                 // [T*k] each
+  const float* gu_saved = nullptr;                                  // [S,2I] the forward's pre-activations, or NULL
 };
 bool backward_generic_supported(int H, int I, int k);
 hipError_t launch_backward_generic(const void* x, const void* d_out, const void* w_router, const void* wgu, const void* wd,

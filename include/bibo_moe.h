@@ -76,7 +76,10 @@ enum bibo_flags {
      workgroups) instead of always running the fused kernel. */
   BIBO_FLAG_TRAIN_AUTO = 8,
   /* bibo_moe_ffn_forward only: norm_weight points to bf16 values, 16-byte aligned (used in fp32, as the fp32 ones are). */
-  BIBO_FLAG_NORM_BF16 = 16
+  BIBO_FLAG_NORM_BF16 = 16,
+  /* bibo_moe_train_state_bytes, bibo_moe_forward_train and bibo_moe_backward_saved: every shape that bibo_moe_backward takes, not only
+   * those of the fused kernel (see there) */
+  BIBO_FLAG_KEEP_ANY = 32
 };
 
 /* kernel family for the expert GEMMs */
@@ -320,6 +323,10 @@ int bibo_moe_backward(const void* x, const void* d_out, const void* w_router, co
  * bibo_moe_backward, whose results bibo_moe_backward_saved reproduces bit for bit.  Shapes: bf16, H a multiple of 128,
  * I in {128, 256, 384}; BIBO_ERR_UNSUPPORTED otherwise (use bibo_moe_forward + bibo_moe_backward).  The reference keeps
  * its activations through torch.autograd; this pair is that choice made explicit.
+ * With BIBO_FLAG_KEEP_ANY in shape->flags of all three calls the pair takes every shape that bibo_moe_backward takes.  Where the fused kernel
+ * does not run, out is that of bibo_moe_forward with BIBO_ALGO_AUTO, and the state holds the routing and the permutation and, for the fp32 tile
+ * kernels (H and I multiples of four, more than a few routed slots), the fp32 pre-activations too (about 8 I bytes per routed slot); the
+ * backward pass computes what the state does not hold.  x, w_gate_up and w_down have to be 16-byte aligned then.
  */
 int bibo_moe_train_state_bytes(const bibo_moe_shape* shape, size_t* bytes);
 int bibo_moe_forward_train(const void* x, const void* w_router, const float* bias, const void* w_gate_up, const void* w_down,
