@@ -14,7 +14,7 @@ NORM_NONE, NORM_SUM, NORM_SOFTMAX = 0, 1, 2
 ALGO_AUTO, ALGO_GENERIC, ALGO_MFMA, ALGO_STREAM, ALGO_FUSED = 0, 1, 2, 3, 4
 MAX_EXPERTS, MAX_TOPK = 64, 8
 ACT_RADIAL_SIGMOID, ACT_RADIAL_TANH, ACT_SILU = 0, 1, 2
-FLAG_ROUND_BLOCK_OUT, FLAG_NO_RESIDUAL, FLAG_GRAD_F32, FLAG_TRAIN_AUTO, FLAG_NORM_BF16 = 1, 2, 4, 8, 16
+FLAG_ROUND_BLOCK_OUT, FLAG_NO_RESIDUAL, FLAG_GRAD_F32, FLAG_TRAIN_AUTO, FLAG_NORM_BF16, FLAG_KEEP_ANY = 1, 2, 4, 8, 16, 32
 ABI_VERSION = 3
 
 # every symbol include/bibo_moe.h declares
@@ -23,7 +23,7 @@ SYMBOLS = (
     "bibo_moe_permute", "bibo_moe_gateup_fwd", "bibo_moe_down_combine_fwd", "bibo_moe_gateup_down_fwd",
     "bibo_moe_combine_fwd", "bibo_moe_combine_ex_fwd", "bibo_moe_experts_fwd", "bibo_moe_forward", "bibo_moe_rmsnorm_fwd",
     "bibo_moe_ffn_workspace_bytes", "bibo_moe_ffn_forward", "bibo_moe_forward_static", "bibo_moe_backward_workspace_bytes", "bibo_moe_backward", "bibo_moe_experts_backward",
-    "bibo_moe_train_state_bytes", "bibo_moe_forward_train", "bibo_moe_backward_saved",
+    "bibo_moe_train_state_bytes", "bibo_moe_forward_train", "bibo_moe_forward_train_balance", "bibo_moe_backward_saved",
     "bibo_moe_exp_attn_res_fwd", "bibo_moe_balance_step",
     "bibo_moe_exp_attn_res_norm_fwd", "bibo_moe_exp_carry_fwd", "bibo_moe_exp_silu_mul_fwd", "bibo_moe_exp_qk_norm_rope",
     "bibo_moe_exp_attention_fwd", "bibo_moe_exp_rope_tables",

@@ -219,9 +219,10 @@ int experts_dispatch(const void* x, const void* wgu, const void* wd, const float
                      const void* residual, bool idx_trusted, int T, int H, int Eg, int np, int nn, int k, int I, int dtype,
                      int algo, int act, int flags, void* out, char* base, const Workspace& ws, size_t ws_bytes,
                      hipStream_t s, bool f32_rows = false, void* preact = nullptr, const ScanArgs& scan = ScanArgs(),
-                     bool gate_up_done = false, float* keep_gu = nullptr) {
+                     bool gate_up_done = false, float* keep_gu = nullptr, const BalanceArgs& balance = BalanceArgs()) {
   float* yw = reinterpret_cast<float*>(base + ws.yw);
   CombineArgs ca;
+  ca.balance = balance;
   ca.residual = residual;
   ca.round_block = (residual != nullptr && (flags & BIBO_FLAG_ROUND_BLOCK_OUT)) ? 1 : 0;   // layers.py:62-63
   // indices that come straight from the router kernel are in range; a caller's may hold padding values, whose
@@ -229,8 +230,9 @@ int experts_dispatch(const void* x, const void* wgu, const void* wd, const float
   if (!idx_trusted || np + nn > 0) { ca.idx = idx; ca.w = w; ca.x = x; ca.E_glu = Eg; ca.n_pos = np; ca.n_neg = nn; }
   if (few_taken(algo, T, H, k, I, dtype, x, wgu, wd)) {
     ca.x = x; ca.n_pos = np; ca.n_neg = nn;
-    return hip_rc(launch_experts_few(x, wgu, wd, theta, idx, w, ca, T, H, Eg, k, I, dtype, act, reinterpret_cast<float*>(base + ws.gu),
-                                     out, gate_up_done, s));
+    const hipError_t e = launch_experts_few(x, wgu, wd, theta, idx, w, ca, T, H, Eg, k, I, dtype, act, reinterpret_cast<float*>(base + ws.gu),
+                                            out, gate_up_done, s);
+    return hip_rc(e == hipSuccess && balance.counts != nullptr ? launch_balance_step(balance, s) : e);
   }
   if (algo == BIBO_ALGO_STREAM) {
     if (!aligned16(x) || !aligned16(wgu) || !aligned16(wd)) return BIBO_ERR_MISALIGNED;
@@ -313,7 +315,7 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
                  const float* theta, const bibo_moe_shape* sh, int norm_mode, int algo, const void* residual, void* out,
                  int32_t* idx_out, float* w_out, int32_t* counts_out, float* logits_out, void* workspace,
                  size_t workspace_bytes, void* stream, const void* norm_src = nullptr, Vec norm_weight = Vec{nullptr, 0},
-                 float eps = 0.f, char* state = nullptr) {
+                 float eps = 0.f, char* state = nullptr, const bibo_moe_balance* moves = nullptr) {
   if (sh == nullptr) return BIBO_ERR_NULL_POINTER;
   const int T = sh->T, H = sh->H, E = sh->E, k = sh->k, I = sh->I, dtype = sh->dtype;
   int rc = check_dims(T, H, E, k, I, dtype, sh->n_pos, sh->n_neg);
@@ -401,10 +403,12 @@ int forward_impl(const void* x, const void* w_router, const float* bias, const v
                              : launch_permute(idx, T, E, k, counts, offsets, perm_slot, perm_token, hist, s);
     if (e != hipSuccess) return (int)e;
   }
-  if (T == 0) return BIBO_OK;
+  BalanceArgs balance;
+  if (moves != nullptr) balance = BalanceArgs{counts, moves->accumulated, moves->bias, E, moves->factor, moves->update};
+  if (T == 0) return moves != nullptr ? hip_rc(launch_balance_step(balance, s)) : BIBO_OK;
   return experts_dispatch(x, w_gate_up, w_down, theta, idx, w, offsets, perm_slot, perm_token, residual, true, T, H, Eg,
                           sh->n_pos, sh->n_neg, k, I, dtype, a, sh->act, sh->flags, out, base, ws, workspace_bytes, s, f32_rows, preact, scan,
-                          gate_up_done, keep_gu);
+                          gate_up_done, keep_gu, balance);
 }
 
 
@@ -874,9 +878,9 @@ int bibo_moe_train_state_bytes(const bibo_moe_shape* sh, size_t* bytes) {
   return BIBO_OK;
 }
 
-int bibo_moe_forward_train(const void* x, const void* w_router, const float* bias, const void* w_gate_up, const void* w_down,
-                           const float* theta, const bibo_moe_shape* sh, int norm_mode, void* out, int32_t* counts_out,
-                           void* state, size_t state_bytes, void* workspace, size_t workspace_bytes, void* stream) {
+static int forward_train(const void* x, const void* w_router, const float* bias, const void* w_gate_up, const void* w_down, const float* theta,
+                         const bibo_moe_shape* sh, int norm_mode, void* out, int32_t* counts_out, const bibo_moe_balance* balance,
+                         void* state, size_t state_bytes, void* workspace, size_t workspace_bytes, void* stream) {
   const int rc = backward_check(sh, norm_mode);
   if (rc != BIBO_OK) return rc;
   const Keeps keeps = kept_state(sh);
@@ -890,7 +894,23 @@ int bibo_moe_forward_train(const void* x, const void* w_router, const float* bia
   }
   return forward_impl(x, w_router, bias, w_gate_up, w_down, theta, sh, norm_mode, keeps == Keeps::kBf16 ? BIBO_ALGO_FUSED : BIBO_ALGO_AUTO,
                       nullptr, out, nullptr, nullptr, counts_out, nullptr, workspace, workspace_bytes, stream, nullptr, Vec{nullptr, 0}, 0.f,
-                      static_cast<char*>(state));
+                      static_cast<char*>(state), balance);
+}
+
+int bibo_moe_forward_train(const void* x, const void* w_router, const float* bias, const void* w_gate_up, const void* w_down,
+                           const float* theta, const bibo_moe_shape* sh, int norm_mode, void* out, int32_t* counts_out,
+                           void* state, size_t state_bytes, void* workspace, size_t workspace_bytes, void* stream) {
+  return forward_train(x, w_router, bias, w_gate_up, w_down, theta, sh, norm_mode, out, counts_out, nullptr, state, state_bytes, workspace,
+                       workspace_bytes, stream);
+}
+
+int bibo_moe_forward_train_balance(const void* x, const void* w_router, const float* bias, const void* w_gate_up, const void* w_down,
+                                   const float* theta, const bibo_moe_shape* sh, int norm_mode, void* out, int32_t* counts_out,
+                                   const bibo_moe_balance* balance, void* state, size_t state_bytes, void* workspace,
+                                   size_t workspace_bytes, void* stream) {
+  if (balance == nullptr || balance->accumulated == nullptr || balance->bias == nullptr) return BIBO_ERR_NULL_POINTER;
+  return forward_train(x, w_router, bias, w_gate_up, w_down, theta, sh, norm_mode, out, counts_out, balance, state, state_bytes, workspace,
+                       workspace_bytes, stream);
 }
 
 int bibo_moe_backward_saved(const void* x, const void* d_out, const void* w_router, const void* w_gate_up, const void* w_down,
@@ -975,7 +995,7 @@ int bibo_moe_experts_backward(const void* x, const void* d_out, const int32_t* i
 int bibo_moe_balance_step(const int32_t* counts, float* accumulated, float* bias, int E, float factor, int update, void* stream) {
   if (E < 1 || E > kMaxE) return BIBO_ERR_BAD_SHAPE;
   if (!counts || !accumulated || !bias) return BIBO_ERR_NULL_POINTER;
-  return hip_rc(launch_balance_step(counts, accumulated, bias, E, factor, update, static_cast<hipStream_t>(stream)));
+  return hip_rc(launch_balance_step(BalanceArgs{counts, accumulated, bias, E, factor, update}, static_cast<hipStream_t>(stream)));
 }
 
 int bibo_moe_exp_attn_res_norm_fwd(const void* const* candidates, int n_candidates, const void* score_a, const void* score_b,

@@ -248,6 +248,8 @@ struct TrainCall {
   at::ScalarType compute;
   bool keep;
   Tensor counts;         // int32 [E] to fill, or undefined
+  const bibo_moe_balance* balance = nullptr;   // the balancing step behind the forward, which a saved one takes along,
+  bool balanced = false;                       // and whether it has
 };
 
 class LayerFn : public torch::autograd::Function<LayerFn> {
@@ -271,11 +273,19 @@ class LayerFn : public torch::autograd::Function<LayerFn> {
     if (saved) {
       last = at::empty({(int64_t)std::max<size_t>(state_bytes, 256)}, xb.options().dtype(at::kByte));
       const Scratch ws(xb.device(), s, bytes);
-      check(bibo_moe_forward_train(xb.data_ptr(), l.w_router.data_ptr(), f32(l.bias), l.w_gate_up.data_ptr(), l.w_down.data_ptr(),
-                                   f32(l.theta), &sh, l.norm, out.data_ptr(), int_ptr(c->counts), last.data_ptr(),
-                                   (size_t)last.numel(), ws.data_ptr(), (size_t)ws.numel(), s),
-            "bibo_moe_forward_train");
+      if (c->balance != nullptr)
+        check(bibo_moe_forward_train_balance(xb.data_ptr(), l.w_router.data_ptr(), f32(l.bias), l.w_gate_up.data_ptr(), l.w_down.data_ptr(),
+                                             f32(l.theta), &sh, l.norm, out.data_ptr(), nullptr, c->balance, last.data_ptr(),
+                                             (size_t)last.numel(), ws.data_ptr(), (size_t)ws.numel(), s),
+              "bibo_moe_forward_train_balance");
+      else
+        check(bibo_moe_forward_train(xb.data_ptr(), l.w_router.data_ptr(), f32(l.bias), l.w_gate_up.data_ptr(), l.w_down.data_ptr(),
+                                     f32(l.theta), &sh, l.norm, out.data_ptr(), int_ptr(c->counts), last.data_ptr(),
+                                     (size_t)last.numel(), ws.data_ptr(), (size_t)ws.numel(), s),
+              "bibo_moe_forward_train");
+      c->balanced = c->balance != nullptr;
     } else {
+      if (c->balance != nullptr) c->counts = counts_for(xb, sh);       // for a step behind this call
       // A private copy: the layer's balancing step writes gate.bias in place later in the same forward, and the backward
       // pass has to route with the values the forward saw.
       last = l.bias.detach().clone();
@@ -337,16 +347,32 @@ class LayerFn : public torch::autograd::Function<LayerFn> {
   }
 };
 
-// x and the parameters as the caller holds them, then their kernel-dtype copies -> (out like x in compute dtype, counts or None)
+// x and the parameters as the caller holds them, then their kernel-dtype copies -> (out like x in compute dtype, counts or None, whether the
+// balancing step is done).  accumulated, balance_bias, factor, update: the arguments of balance_step, where the caller leaves the step to this
+// call; counts only come back if it could not take it.
 py::tuple layer_train(const Tensor& x, const Tensor& w_router, const Tensor& w_gate_up, const Tensor& w_down, const Tensor& theta,
                       const Tensor& wr_k, const Tensor& bias_k, const Tensor& gu_k, const Tensor& dn_k, const Tensor& th_k, int k,
-                      int norm, int algo, int n_pos, int n_neg, int act, bool want_counts, at::ScalarType compute, bool keep) {
+                      int norm, int algo, int n_pos, int n_neg, int act, bool want_counts, at::ScalarType compute, bool keep,
+                      const c10::optional<Tensor>& accumulated, const c10::optional<Tensor>& balance_bias, double factor, bool update) {
   TORCH_CHECK(x.is_cuda(), "x must live on the GPU (got ", x.device(), "); bibo_amd has no CPU path");
   c10::DeviceGuard guard(x.device());
   TrainCall c{{wr_k, bias_k, gu_k, dn_k, th_k, k, norm, algo, n_pos, n_neg, act}, compute, keep, Tensor()};
-  if (want_counts) c.counts = at::empty({gu_k.size(0) + n_pos + n_neg}, x.options().dtype(at::kInt).requires_grad(false));
+  const int64_t E = gu_k.size(0) + n_pos + n_neg;
+  bibo_moe_balance balance;
+  if (accumulated.has_value() && balance_bias.has_value()) {
+    check_tensor(*accumulated, "accumulated_tpe", at::kFloat, {E});
+    check_tensor(*balance_bias, "bias", at::kFloat, {E});
+    balance = {static_cast<float*>(accumulated->data_ptr()), static_cast<float*>(balance_bias->data_ptr()), (float)factor, update ? 1 : 0};
+    c.balance = &balance;
+  } else if (want_counts) {
+    c.counts = at::empty({E}, x.options().dtype(at::kInt).requires_grad(false));
+  }
   Tensor out = LayerFn::apply(x, w_router, w_gate_up, w_down, theta, &c);
-  return py::make_tuple(out, maybe(c.counts));
+  if (c.balanced) {                                      // written in place
+    accumulated->unsafeGetTensorImpl()->bump_version();
+    if (update) balance_bias->unsafeGetTensorImpl()->bump_version();
+  }
+  return py::make_tuple(out, maybe(c.counts), c.balanced);
 }
 
 // accumulated += counts; with `update`, bias += factor * (mean(load) - load) for load = accumulated / max(sum, 1), and

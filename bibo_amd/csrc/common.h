@@ -194,6 +194,26 @@ __device__ __forceinline__ void load8(const Vec& v, size_t at, float (&out)[8]) 
   }
 }
 
+// The balancing step behind a training forward (moe.py:131-155); counts NULL: none.
+struct BalanceArgs {
+  const int32_t* counts = nullptr;   // [E] of the call
+  float* accumulated = nullptr;      // [E]
+  float* bias = nullptr;             // [E]
+  int E = 0;
+  float factor = 0.f;
+  int update = 0;
+};
+// accumulated += counts and, with `update`, the proportional bias step on the normalised loads; one wave, lane = expert
+__device__ __forceinline__ void balance_step(const BalanceArgs& b) {
+  const int lane = lane_id();
+  const float acc = lane < b.E ? b.accumulated[lane] + (float)b.counts[lane] : 0.f;
+  const float load = acc / fmaxf(wave_sum(acc), 1.f);
+  const float mean = wave_sum(load) / (float)b.E;
+  if (lane >= b.E) return;
+  b.accumulated[lane] = b.update ? 0.f : acc;
+  if (b.update) b.bias[lane] += b.factor * (mean - load);
+}
+
 // ---- host-side launchers (one per translation unit) -------------------------------------------
 // `chunk_hist` (or NULL): per-workgroup histograms of the selected experts, [ceil(T / *hist_tokens)][64]; *hist_tokens
 // comes back 0 when the kernel that ran does not write them.
@@ -212,8 +232,7 @@ bool permute_takes_router_hist(int T, int k);
 hipError_t launch_permute_from_hist(const int32_t* idx, int T, int E, int k, int32_t* hist, int hist_tokens,
                                     int32_t* counts, int32_t* offsets, int32_t* perm_slot, int32_t* perm_token,
                                     hipStream_t s);
-hipError_t launch_balance_step(const int32_t* counts, float* accumulated, float* bias, int E, float factor, int update,
-                               hipStream_t s);
+hipError_t launch_balance_step(const BalanceArgs& b, hipStream_t s);
 hipError_t launch_gateup_generic(const void* x, const void* wgu, const float* theta, const int32_t* offsets,
                                  const int32_t* perm_token, int T, int H, int E, int k, int I, int dtype, int act,
                                  void* hidden, hipStream_t s);
@@ -238,6 +257,7 @@ struct CombineArgs {
   int E_glu = 0, n_pos = 0, n_neg = 0;
   const void* residual = nullptr;  // [T,H] in the output dtype
   int round_block = 0;             // round the sum of the slot rows to the output dtype before the residual is added
+  BalanceArgs balance;             // taken by a workgroup of its own behind the others
 };
 hipError_t launch_experts_few(const void* x, const void* wgu, const void* wd, const float* theta, const int32_t* idx, const float* w,
                               const CombineArgs& a, int T, int H, int E, int k, int I, int dtype, int act, float* gu, void* out,

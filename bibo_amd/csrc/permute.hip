@@ -217,24 +217,13 @@ __global__ __launch_bounds__(64) void permute_small_kernel(const int32_t* __rest
   }
 }
 
-// accumulated += counts and, with `update`, the proportional bias step on the normalised loads (moe.py:131-155); lane =
-// expert.  One launch of one wave for what takes eight elementwise launches of tensor operations.
-__global__ __launch_bounds__(64) void balance_step_kernel(const int32_t* __restrict__ counts, float* __restrict__ accumulated,
-                                                          float* __restrict__ bias, int E, float factor, int update) {
-  const int lane = threadIdx.x;
-  const float acc = lane < E ? accumulated[lane] + (float)counts[lane] : 0.f;
-  const float load = acc / fmaxf(wave_sum(acc), 1.f);
-  const float mean = wave_sum(load) / (float)E;
-  if (lane >= E) return;
-  accumulated[lane] = update ? 0.f : acc;
-  if (update) bias[lane] += factor * (mean - load);
-}
+// One launch of one wave for what takes eight elementwise launches of tensor operations (calls that end in a combine kernel need none).
+__global__ __launch_bounds__(64) void balance_step_kernel(BalanceArgs b) { balance_step(b); }
 
 }  // namespace
 
-hipError_t launch_balance_step(const int32_t* counts, float* accumulated, float* bias, int E, float factor, int update,
-                               hipStream_t s) {
-  hipLaunchKernelGGL(balance_step_kernel, dim3(1), dim3(64), 0, s, counts, accumulated, bias, E, factor, update);
+hipError_t launch_balance_step(const BalanceArgs& b, hipStream_t s) {
+  hipLaunchKernelGGL(balance_step_kernel, dim3(1), dim3(64), 0, s, b);
   return hipGetLastError();
 }
 

@@ -388,21 +388,34 @@ class BiBoMoELayer(nn.Module):
         self.accumulated_tpe.zero_()
         return tpe
 
-    def _balance(self, counts, num_tokens):
-        """_balance_step and update_bias of this forward in one launch, where neither is overridden or replaced, the state is fp32 on
-        the GPU and no process group has to see the counts first."""
+    def _native_balance(self, num_tokens, device):
+        """(accumulated counts, bias, factor, whether the bias moves) of this forward's balancing step as one native call, and the cadence
+        it was worked out with, where neither half is overridden or replaced, the state is fp32 on the GPU and no process group has to
+        see the counts first; else None.  Changes nothing."""
         cls, bias, acc = type(self), _param(self._modules["gate"], "bias"), self.accumulated_tpe
-        if ((cls._balance_step, cls.update_bias) == _BALANCING
-                and "update_bias" not in self.__dict__ and "_balance_step" not in self.__dict__
-                and counts is not None and counts.is_cuda and acc.device == bias.device == counts.device
-                and acc.dtype == bias.dtype == torch.float32 and acc.is_contiguous() and bias.is_contiguous()):
-            if self._update_every is None:
-                self._update_every = max(1, round(self.bias_update_threshold / max(num_tokens, 1)))
-            fires = (self._fwd_step + 1) % self._update_every == 0
-            if not (fires and torch.distributed.is_available() and torch.distributed.is_initialized()):
-                self._fwd_step += 1
-                L.native().balance_step(counts, acc, bias, self.bias_update_factor, fires)
-                return
+        if ((cls._balance_step, cls.update_bias) != _BALANCING or "update_bias" in self.__dict__ or "_balance_step" in self.__dict__
+                or device.type != "cuda" or not (acc.device == bias.device == device) or not (acc.dtype == bias.dtype == torch.float32)
+                or not (acc.is_contiguous() and bias.is_contiguous())):
+            return None
+        every = self._update_every
+        if every is None:
+            every = max(1, round(self.bias_update_threshold / max(num_tokens, 1)))
+        fires = (self._fwd_step + 1) % every == 0
+        if fires and torch.distributed.is_available() and torch.distributed.is_initialized():
+            return None
+        return (acc, bias, self.bias_update_factor, fires), every
+
+    def _balance_is_ours(self) -> bool:
+        return type(self)._balance is _BALANCE and "_balance" not in self.__dict__
+
+    def _balance(self, counts, num_tokens):
+        """_balance_step and update_bias of this forward, in one launch where that is allowed."""
+        native = self._native_balance(num_tokens, counts.device) if counts is not None else None
+        if native is not None:
+            self._update_every = native[1]
+            self._fwd_step += 1
+            L.native().balance_step(counts, *native[0])
+            return
         tpe = self._balance_step(None, num_tokens, counts=counts)
         if tpe is not None:
             self.update_bias(tpe)
@@ -454,7 +467,13 @@ class BiBoMoELayer(nn.Module):
             if torch.is_grad_enabled() and (hidden_states.requires_grad or any(p.requires_grad for p in params[:4])):
                 if not self._differentiable(cd):
                     raise NotImplementedError(_NO_BACKWARD)
-                out, counts = L.native().layer_train(hidden_states, *params[:4], *operands, *settings, self.keep_activations)
+                native = self._native_balance(num_tokens, hidden_states.device) if balancing and self._balance_is_ours() else None
+                out, counts, done = L.native().layer_train(hidden_states, *params[:4], *operands, *settings, self.keep_activations,
+                                                           *(native[0] if native is not None else (None, None, 0.0, False)))
+                if done:                                       # with the forward's own launches
+                    self._update_every = native[1]
+                    self._fwd_step += 1
+                    balancing = False
             else:
                 out, counts = L.native().layer_forward(hidden_states, *operands, *settings)
             out = out if out.dtype == hidden_states.dtype else out.to(hidden_states.dtype)
@@ -513,4 +532,5 @@ class BiBoMoELayer(nn.Module):
         return out.to(torch.bfloat16) if bf16_stream else out
 
 
-_BALANCING = (BiBoMoELayer._balance_step, BiBoMoELayer.update_bias)      # unless somebody replaces them on the class
+# unless somebody replaces them on the class
+_BALANCING, _BALANCE = (BiBoMoELayer._balance_step, BiBoMoELayer.update_bias), BiBoMoELayer._balance

@@ -332,6 +332,18 @@ int bibo_moe_train_state_bytes(const bibo_moe_shape* shape, size_t* bytes);
 int bibo_moe_forward_train(const void* x, const void* w_router, const float* bias, const void* w_gate_up, const void* w_down,
                            const float* theta, const bibo_moe_shape* shape, int norm_mode, void* out, int32_t* counts_out,
                            void* state, size_t state_bytes, void* workspace, size_t workspace_bytes, void* stream);
+/* bibo_moe_forward_train and, from the counts of that call, bibo_moe_balance_step with these arguments, without a launch of its own where the
+ * call ends in a combine kernel.  balance->bias may be the `bias` the call routes with: it is read before it is written. */
+typedef struct bibo_moe_balance {
+  float* accumulated;   /* [E] */
+  float* bias;          /* [E] */
+  float factor;
+  int32_t update;
+} bibo_moe_balance;
+int bibo_moe_forward_train_balance(const void* x, const void* w_router, const float* bias, const void* w_gate_up, const void* w_down,
+                                   const float* theta, const bibo_moe_shape* shape, int norm_mode, void* out, int32_t* counts_out,
+                                   const bibo_moe_balance* balance, void* state, size_t state_bytes, void* workspace,
+                                   size_t workspace_bytes, void* stream);
 int bibo_moe_backward_saved(const void* x, const void* d_out, const void* w_router, const void* w_gate_up, const void* w_down,
                             const float* theta, const bibo_moe_shape* shape, int norm_mode, const void* state,
                             size_t state_bytes, void* d_x, void* d_w_router, void* d_w_gate_up, void* d_w_down,

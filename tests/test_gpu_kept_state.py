@@ -78,6 +78,7 @@ def test_which_shapes_keep_what():
     tiles, rows, wide = (777, 192, 16, 3, 88, L.DTYPE_F32), (60, 50, 5, 2, 30, L.DTYPE_F32), (1500, 256, 8, 4, 512, L.DTYPE_BF16)
     for dims in (tiles, rows, wide):
         assert size(0, *dims) == -6
+    assert L.FLAG_KEEP_ANY == 32
     assert size(32, *tiles) >= 777 * 3 * (2 * 88 * 4 + 16)
     assert 0 < size(32, *rows) < 60 * 2 * 2 * 30 * 4 + 8192
     assert 0 < size(32, *wide) < 1500 * 4 * 2 * 512
