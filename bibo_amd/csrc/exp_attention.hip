@@ -203,7 +203,8 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const bf16_t* __restr
     float mx = st[0];
 #pragma unroll
     for (int i = 1; i < 16; ++i) mx = fmaxf(mx, st[i]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave)) * scale_log2;
+    const Pair mxs = lanes32(mx);
+    mx = fmaxf(mxs.a, mxs.b) * scale_log2;
     if (__any(mx > m + 8.f)) {
       const float mn = fmaxf(m, mx), al = __builtin_amdgcn_exp2f(m - mn);
       m = mn;
@@ -247,7 +248,8 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const bf16_t* __restr
   }
   // y = O / l, then XSA: y -= tanh(alpha) <y, vn> vn with vn = v / |v| of the query's own token
   const int qi = q0w + n;
-  l += __shfl_xor(l, 32, kWave);
+  const Pair ls = lanes32(l);
+  l = ls.a + ls.b;
   const float inv = 1.f / l;
   if (xsa_alpha.p != nullptr) {
     const bf16_t* vrow = vbase + (size_t)min(qi, S - 1) * ld + 4 * h;
@@ -266,8 +268,9 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const bf16_t* __restr
         vv = fmaf(f, f, vv);
         yv = fmaf(f, o[dt][i], yv);
       }
-    vv += __shfl_xor(vv, 32, kWave);
-    yv += __shfl_xor(yv, 32, kWave);
+    const Pair vvs = lanes32(vv), yvs = lanes32(yv);
+    vv = vvs.a + vvs.b;
+    yv = yvs.a + yvs.b;
     const float vn = 1.f / fmaxf(sqrtf(vv), 1e-12f);            // F.normalize
     const float coeff = yv * vn * vn * tanhf(xsa_alpha[head]);
 #pragma unroll

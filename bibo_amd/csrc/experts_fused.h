@@ -632,7 +632,8 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
       for (int j = 1; j < NT; ++j) v = block_of(j) == b ? part[j] : v;
       sq += v;
     }
-    sq += __shfl_xor(sq, 32, kWave);
+    const Pair halves = lanes32(sq);
+    sq = halves.a + halves.b;
     if (hh == 0) ssq[wn * BM + mbase + mt * 32 + n] = sq;
   }
   __syncthreads();

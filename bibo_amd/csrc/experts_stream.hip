@@ -296,7 +296,7 @@ __device__ __forceinline__ void stage_activated(const bf16_t* __restrict__ gu, f
 #pragma unroll
         for (int q = 0; q < 8; ++q) ss = fmaf((float)g[j][q], (float)g[j][q], ss);
       }
-    for (int o = tpr >> 1; o > 0; o >>= 1) ss += __shfl_xor(ss, o, kWave);   // the row's threads are adjacent lanes
+    ss = tpr == 64 ? wave_sum(ss) : half_wave_sum(ss);                       // the row's threads are adjacent lanes
     float rinv, gain;                                                                     // 1/r, r^p (moe.py:88-89)
     radial_row_scalars(ss, I, p, act, rinv, gain);
     const float nrl = -1.4426950408889634f * rinv, rg = rinv * gain;

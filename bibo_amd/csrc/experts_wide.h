@@ -388,8 +388,10 @@ __global__ __launch_bounds__(512) void experts_wide_kernel(const bf16_t* __restr
       for (int j = 1; j < NT; ++j) v = block_of(j) == b ? part[j] : v;
       sq += v;
     }
-    sq += __shfl_xor(sq, 16, kWave);
-    sq += __shfl_xor(sq, 32, kWave);
+    Pair p = lanes16(sq);
+    sq = p.a + p.b;
+    p = lanes32(sq);
+    sq = p.a + p.b;
     if (g4 == 0) ssq[wn * BM + mbase + rt * 16 + n] = sq;
   }
   __syncthreads();
