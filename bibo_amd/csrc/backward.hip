@@ -312,6 +312,91 @@ __device__ __forceinline__ float lane_value(float v, int lane) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
 }
 
+// dlogit of slot j of a token (router.py:31,41-47) from the scores s, weights w and weight gradients dw of its slots, the sums in ascending order
+template <int K>
+__device__ __forceinline__ float weight_to_score_grad(float dw, float w, float sum, float dot, int norm_mode) {
+  if (K > 1 && norm_mode == BIBO_NORM_SUM) return (dw - dot) / (sum + 1e-20f);
+  if (K > 1 && norm_mode == BIBO_NORM_SOFTMAX) return w * (dw - dot);
+  return dw;
+}
+__device__ __forceinline__ float score_of(float logit) { return 1.f / (1.f + __expf(-logit)); }
+
+// dW_router[e, c] = sum over the rows r of expert e of dl[slot(r)] x[token(r), c], in two steps.  Step 1: block (g, z) takes the z-th of
+// kDwrSplit equal row ranges of row chunk g of the plan (kmajor.h: an expert's rows, cut where an expert holds many); 32 threads share a
+// row, 256 columns at a time, the eight partial sums meet in LDS in a fixed order -> part[g][z][c] fp32.  Step 2 adds the ranges of an
+// expert's chunks in order.  A row's token and dl go through LDS, 256 rows at a time: as loads of each of its threads they were three of four
+// load instructions, 16 cycles of a CU's address unit each.
+constexpr int kDwrSplit = 8, kDwrRows = 4, kDwrTurns = 4;
+struct DwrShared {
+  float red[8][256], d[256];
+  int token[256];
+};
+template <typename SlotGrad>
+__device__ __forceinline__ void dwr_block(DwrShared& sh, const bf16_t* __restrict__ x, SlotGrad slot_grad, const int* __restrict__ plan,
+                                          const int32_t* __restrict__ perm_slot, const int32_t* __restrict__ perm_token, int H, int g, int z,
+                                          float* __restrict__ part) {
+  if (g >= plan[0]) return;
+  const int tid = threadIdx.x, cg = tid & 31, rl = tid >> 5;
+  const int lo_e = plan[4 + 4 * g + 1], n = plan[4 + 4 * g + 2] - lo_e;
+  const int per = (n + kDwrSplit - 1) / kDwrSplit;
+  const int lo = lo_e + min(z * per, n), hi = lo_e + min((z + 1) * per, n);
+  for (int h0 = 0; h0 < H; h0 += 256 * kDwrTurns) {             // (once up to H = 1024)
+    float acc[kDwrTurns][8];
+#pragma unroll
+    for (int i = 0; i < kDwrTurns; ++i)
+#pragma unroll
+      for (int q = 0; q < 8; ++q) acc[i][q] = 0.f;
+    for (int r0 = lo; r0 < hi; r0 += 256) {
+      const int rows = min(hi - r0, 256);
+      __syncthreads();                                          // the rows before have been read
+      if (tid < rows) {
+        sh.token[tid] = perm_token[r0 + tid];
+        sh.d[tid] = slot_grad(perm_slot[r0 + tid]);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < kDwrTurns; ++i) {
+        const int c = h0 + i * 256 + cg * 8;
+        if (c >= H) continue;
+        const bf16_t* const xc = x + c;
+        auto add = [&](float d, const bf16x8& v) {
+#pragma unroll
+          for (int q = 0; q < 8; ++q) acc[i][q] = fmaf(d, (float)v[q], acc[i][q]);
+        };
+        int r = rl;
+        for (; r + 8 * (kDwrRows - 1) < rows; r += 8 * kDwrRows) {   // several rows on their way together
+          bf16x8 v[kDwrRows];
+#pragma unroll
+          for (int u = 0; u < kDwrRows; ++u) v[u] = *reinterpret_cast<const bf16x8*>(xc + (size_t)sh.token[r + 8 * u] * H);
+#pragma unroll
+          for (int u = 0; u < kDwrRows; ++u) add(sh.d[r + 8 * u], v[u]);
+        }
+        for (; r < rows; r += 8) add(sh.d[r], *reinterpret_cast<const bf16x8*>(xc + (size_t)sh.token[r] * H));
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kDwrTurns; ++i) {
+      if (h0 + i * 256 >= H) break;
+      __syncthreads();                                          // the sums before have been read
+#pragma unroll
+      for (int q = 0; q < 8; ++q) sh.red[rl][cg * 8 + q] = acc[i][q];
+      __syncthreads();
+      const int col = h0 + i * 256 + tid;
+      if (col < H)
+        part[((size_t)g * kDwrSplit + z) * H + col] = ((sh.red[0][tid] + sh.red[1][tid]) + (sh.red[2][tid] + sh.red[3][tid])) +
+                                                      ((sh.red[4][tid] + sh.red[5][tid]) + (sh.red[6][tid] + sh.red[7][tid]));
+    }
+  }
+}
+
+// where +/-Identity experts make a slot's gradient a dot product, which token_bwd_kernel works out
+__global__ __launch_bounds__(256) void dwr_partial_kernel(const bf16_t* __restrict__ x, const float* __restrict__ dl, const int* __restrict__ plan,
+                                                          const int32_t* __restrict__ perm_slot, const int32_t* __restrict__ perm_token,
+                                                          int H, float* __restrict__ part) {
+  __shared__ DwrShared sh;
+  dwr_block(sh, x, [&](int slot) { return dl[slot]; }, plan, perm_slot, perm_token, H, blockIdx.x, blockIdx.y, part);
+}
+
 // Everything per token behind the experts, one wave per token and run of up to 512 columns (`parts` runs of equal length):
 //   +/-Identity slots (moe.py:95-99): dw = +/- <d_out[t], x[t]>, their share of dx is +/- w d_out[t];
 //   router (router.py:31,41-47; w_router == NULL: none): lane j < k turns the gradients of the combine weights into dlogit of
@@ -322,15 +407,46 @@ __device__ __forceinline__ float lane_value(float v, int lane) {
 // scalars, the first one stores them.  Bound by reading the slots' dx rows (T = 8192, H = 768, k = 6: 75 MB), which are requested
 // before the indices that decide about them are back.  K = k at compile time, and no load under a condition: the compiler
 // drains all loads where a branch around one ends (k at run time: 26 us at that size, 21 like this).
-template <int K>
+// DWR: the first nb_dwr workgroups are dwr_partial_kernel's (the ranges of a chunk next to each other) and work out
+// dl of their rows' slots themselves, so that they need not wait for this launch.  Both launches -> this one, us: 40.0 -> 31.4 (T = 8192, H = 768,
+// k = 6), 20.4 -> 13.2 (6000, 512, 6), 29.3 -> 25.7 (4000, 1024, 8), 8.7 -> 6.2 (1111, 512, 2); with 256 columns a workgroup, each of which
+// works dl out again, 35.3, 14.0, 28.8 and 5.0; with dl from workgroups behind the GEMMs' 32.6, 15.0, 26.9 and 4.4, and 1 to 7 more in the GEMMs.
+template <int K, bool DWR>
 __global__ __launch_bounds__(256) void token_bwd_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ d_out,
                                                         const bf16_t* __restrict__ dxs, const float* __restrict__ logits,
                                                         const int32_t* __restrict__ idx, const float* __restrict__ w,
                                                         const bf16_t* __restrict__ w_router, int T, int H, int E, int n_pos,
                                                         int n_neg, int norm_mode, int parts, float* __restrict__ dw_slot,
-                                                        float* __restrict__ dl, bf16_t* __restrict__ dx) {
+                                                        float* __restrict__ dl, bf16_t* __restrict__ dx, int nb_dwr,
+                                                        const int* __restrict__ plan, const int32_t* __restrict__ perm_slot,
+                                                        const int32_t* __restrict__ perm_token, float* __restrict__ dwr_part) {
+  if constexpr (DWR) {
+    __shared__ DwrShared sh;
+    if (blockIdx.x < (unsigned)nb_dwr) {
+      dwr_block(sh, x, [&](int slot) {
+        const int t = slot / K, mine = slot - t * K;
+        float s[K], dw[K], wj[K], sum = 0.f, dot = 0.f;
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+          s[j] = logits[(size_t)t * E + min((unsigned)idx[t * K + j], (unsigned)E - 1u)];
+          dw[j] = dw_slot[t * K + j];
+          wj[j] = w[t * K + j];
+        }
+        float s_ = 0.f, dw_ = 0.f, w_ = 0.f;
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+          s[j] = score_of(s[j]);
+          sum += s[j];
+          dot = fmaf(dw[j], wj[j], dot);
+          if (j == mine) { s_ = s[j]; dw_ = dw[j]; w_ = wj[j]; }
+        }
+        return weight_to_score_grad<K>(dw_, w_, sum, dot, norm_mode) * s_ * (1.f - s_);
+      }, plan, perm_slot, perm_token, H, blockIdx.x / kDwrSplit, blockIdx.x % kDwrSplit, dwr_part);
+      return;
+    }
+  }
   const int lane = threadIdx.x & 63;
-  const int unit = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  const int unit = __builtin_amdgcn_readfirstlane((blockIdx.x - (DWR ? nb_dwr : 0)) * 4 + (threadIdx.x >> 6));
   const int t = unit / parts, part = unit - t * parts;
   if (t >= T) return;
   const int Et = E + n_pos + n_neg, gran = H / 8, run = (gran + parts - 1) / parts;
@@ -354,7 +470,7 @@ __global__ __launch_bounds__(256) void token_bwd_kernel(const bf16_t* __restrict
 #pragma unroll
     for (int j = 0; j < K; ++j)
       r[j] = reinterpret_cast<const bf16x8*>(w_router)[(size_t)max(__builtin_amdgcn_readlane(e_, j), 0) * gran + cc];
-    s_ = 1.f / (1.f + __expf(-logit));
+    s_ = score_of(logit);
   }
   if (__ballot(e_ >= E) != 0ull) {
     float dot = 0.f;
@@ -375,12 +491,9 @@ __global__ __launch_bounds__(256) void token_bwd_kernel(const bf16_t* __restrict
       sum += lane_value(s_, j);
       dot = fmaf(lane_value(dw_, j), lane_value(w_, j), dot);
     }
-    float ds = dw_;
-    if (K > 1 && norm_mode == BIBO_NORM_SUM) ds = (ds - dot) / (sum + 1e-20f);
-    else if (K > 1 && norm_mode == BIBO_NORM_SOFTMAX) ds = w_ * (ds - dot);
-    dl_ = ds * s_ * (1.f - s_);
+    dl_ = weight_to_score_grad<K>(dw_, w_, sum, dot, norm_mode) * s_ * (1.f - s_);
   }
-  if (part == 0 && lane < K) {
+  if (!DWR && part == 0 && lane < K) {
     if (e_ < 0 || e_ >= E) dw_slot[t * K + lane] = dw_;
     if (w_router != nullptr) dl[t * K + lane] = dl_;
   }
@@ -409,44 +522,6 @@ __global__ __launch_bounds__(256) void token_bwd_kernel(const bf16_t* __restrict
 #pragma unroll
   for (int q = 0; q < 8; ++q) o[q] = (bf16_t)acc[q];
   reinterpret_cast<bf16x8*>(dx)[(size_t)t * gran + c] = o;
-}
-
-// dW_router[e, c] = sum over the rows r of expert e of dl[slot(r)] x[token(r), c], in two steps.  Step 1, grid =
-// (H / 256, chunks, kDwrSplit): block (., g, z) takes the z-th of kDwrSplit equal row ranges of row chunk g of the plan
-// (kmajor.h: an expert's rows, cut where an expert holds many); thread (rl = t / 32, cg = t % 32) adds up rows rl,
-// rl + 8, .. of the range for columns 8 cg .. + 8 of the block's 256, the eight partial sums meet in LDS in a fixed
-// order -> part[g][z][c] fp32.  Step 2 adds the ranges of an expert's chunks in order.
-constexpr int kDwrSplit = 8;
-
-__global__ __launch_bounds__(256) void dwr_partial_kernel(const bf16_t* __restrict__ x, const float* __restrict__ dl,
-                                                          const int* __restrict__ plan,
-                                                          const int32_t* __restrict__ perm_slot,
-                                                          const int32_t* __restrict__ perm_token, int H,
-                                                          float* __restrict__ part) {
-  __shared__ float red[8][256];
-  const int g = blockIdx.y, z = blockIdx.z, cg = threadIdx.x & 31, rl = threadIdx.x >> 5;
-  if (g >= plan[0]) return;
-  const int c = blockIdx.x * 256 + cg * 8;
-  const int lo_e = plan[4 + 4 * g + 1], n = plan[4 + 4 * g + 2] - lo_e;
-  const int per = (n + kDwrSplit - 1) / kDwrSplit;
-  const int lo = lo_e + min(z * per, n), hi = lo_e + min((z + 1) * per, n);
-  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  if (c < H)
-    for (int r = lo + rl; r < hi; r += 8) {
-      const float d = dl[perm_slot[r]];
-      const bf16x8 v = *reinterpret_cast<const bf16x8*>(x + (size_t)perm_token[r] * H + c);
-#pragma unroll
-      for (int q = 0; q < 8; ++q) acc[q] = fmaf(d, (float)v[q], acc[q]);
-    }
-#pragma unroll
-  for (int q = 0; q < 8; ++q) red[rl][cg * 8 + q] = acc[q];
-  __syncthreads();
-  const int col = blockIdx.x * 256 + threadIdx.x;
-  if (col < H) {
-    const int t = threadIdx.x;
-    part[((size_t)g * kDwrSplit + z) * H + col] =
-        ((red[0][t] + red[1][t]) + (red[2][t] + red[3][t])) + ((red[4][t] + red[5][t]) + (red[6][t] + red[7][t]));
-  }
 }
 
 // The last launch of the backward pass: every sum that ends one, by ranges of workgroups.
@@ -594,25 +669,33 @@ hipError_t launch_backward(const void* x, const void* d_out, const void* w_route
                       b.wgrad_part, H, I, E, grad_f32, 0, 0, false};
   if ((err = launch_backward_gemms(gemms, T, S, backward_chunk_rows(S, Et), slots, s)) != hipSuccess) return err;
   const bool with_router = w_router != nullptr;      // else: the experts alone, the caller owns the routing
+  const bool merged = with_router && E == Et;        // the router's partial sums beside the tokens: their slots are the experts'
   const int parts = (H / 8 + kWave - 1) / kWave;     // runs of columns a lane each
-  auto token_bwd = [&](auto kc) {
-    hipLaunchKernelGGL(token_bwd_kernel<decltype(kc)::value>, dim3((unsigned)(((long long)T * parts + 3) / 4)), dim3(256), 0, s, xp, dop,
-                       dxs, logits, idx, w, wrp, T, H, E, n_pos, n_neg, norm_mode, parts, b.dw_slot, b.dl, static_cast<bf16_t*>(dx));
+  const int nb_dwr = slots * kDwrSplit;
+  auto token_bwd = [&](auto kc, auto with_dwr) {
+    constexpr bool DWR = decltype(with_dwr)::value;
+    hipLaunchKernelGGL((token_bwd_kernel<decltype(kc)::value, DWR>), dim3((unsigned)(((long long)T * parts + 3) / 4) + (DWR ? nb_dwr : 0)), dim3(256),
+                       0, s, xp, dop, dxs, logits, idx, w, wrp, T, H, E, n_pos, n_neg, norm_mode, parts, b.dw_slot, b.dl,
+                       static_cast<bf16_t*>(dx), nb_dwr, b.wgrad_plan, perm_slot, perm_token, b.dwr_part);
+  };
+  auto token_launch = [&](auto kc) {
+    if (merged) token_bwd(kc, std::true_type());
+    else token_bwd(kc, std::false_type());
   };
   static_assert(kMaxK == 8, "a case per k");
   using std::integral_constant;
   switch (k) {
-    case 1: token_bwd(integral_constant<int, 1>{}); break;
-    case 2: token_bwd(integral_constant<int, 2>{}); break;
-    case 3: token_bwd(integral_constant<int, 3>{}); break;
-    case 4: token_bwd(integral_constant<int, 4>{}); break;
-    case 5: token_bwd(integral_constant<int, 5>{}); break;
-    case 6: token_bwd(integral_constant<int, 6>{}); break;
-    case 7: token_bwd(integral_constant<int, 7>{}); break;
-    default: token_bwd(integral_constant<int, 8>{});
+    case 1: token_launch(integral_constant<int, 1>{}); break;
+    case 2: token_launch(integral_constant<int, 2>{}); break;
+    case 3: token_launch(integral_constant<int, 3>{}); break;
+    case 4: token_launch(integral_constant<int, 4>{}); break;
+    case 5: token_launch(integral_constant<int, 5>{}); break;
+    case 6: token_launch(integral_constant<int, 6>{}); break;
+    case 7: token_launch(integral_constant<int, 7>{}); break;
+    default: token_launch(integral_constant<int, 8>{});
   }
-  if (with_router)
-    hipLaunchKernelGGL(dwr_partial_kernel, dim3((H + 255) / 256, slots, kDwrSplit), dim3(256), 0, s, xp, b.dl, b.wgrad_plan,
+  if (with_router && !merged)
+    hipLaunchKernelGGL(dwr_partial_kernel, dim3(slots, kDwrSplit), dim3(256), 0, s, xp, b.dl, b.wgrad_plan,
                        perm_slot, perm_token, H, b.dwr_part);
   // the sums that end the pass: cut experts' partial tiles, dtheta, the router's weight gradient
   const int nb_w = (int)(((size_t)2 * I * H / 4 + 255) / 256);
