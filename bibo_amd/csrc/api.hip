@@ -1073,7 +1073,8 @@ int bibo_moe_exp_rope_tables(const void* inv_freq, int inv_freq_dtype, int S, in
 int bibo_moe_exp_attention_fwd(const void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, int window,
                                float scale, const void* xsa_alpha, int alpha_dtype, void* out, void* stream) {
   if (B < 0 || S < 0 || window < 0 || (long long)B * S * n_heads > 0x3fffffffLL) return BIBO_ERR_BAD_SHAPE;
-  if (!exp_attention_supported(n_heads, n_kv_heads, head_dim) || ld < (n_heads + 2 * n_kv_heads) * head_dim || ld % 8 != 0)
+  if (!exp_attention_supported(n_heads, n_kv_heads, head_dim) || ld < (n_heads + 2 * n_kv_heads) * head_dim || ld % 8 != 0 ||
+      ld > kAttnMaxLd)
     return BIBO_ERR_UNSUPPORTED;
   if (B == 0 || S == 0) return BIBO_OK;
   if (!qkv || !out) return BIBO_ERR_NULL_POINTER;

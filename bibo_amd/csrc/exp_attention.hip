@@ -103,16 +103,23 @@ __global__ __launch_bounds__(256) void rope_tables_kernel(Vec inv_freq, int S, i
 // 1.661e-3 here and 2.349e-3 there).  Causal layers' library kernel rounded them to bf16, as the other variant does.
 // The running maximum is raised (and O rescaled, D/32 x 16 multiplies) only when a row's maximum passes it by more than 8
 // in log2 units: the sums stay exact, the probabilities at most 256.
-// K and V blocks arrive by LDS-DMA in two stages; the next one is requested right after the barrier that frees its stage.
+// K and V blocks arrive by LDS-DMA in three stages, requested two blocks ahead right after the barrier that frees the stage, by transfers that the
+// compiler does not see: it waited for all of them in front of the values' reads, that is for the block behind the present one.  A wave's chain
+// of a block (12 dependent MFMAs, maximum, 16 exponentials, 12 MFMAs) bounds the causal layers, whose last queries take 64 of them: six key
+// fragments are read in front of the first MFMA, and the masks select instead of branching.  Two stages, reads in pairs -> now, us,
+// D = 192, 4 and 2 heads, S = 2048: causal 8 x 83.9 -> 74.7, 1 x 65.3 -> 60.4, window 128 8 x 31.8 -> 30.9, 1 x 17.6 -> 15.9; D = 128, 8 and 2
+// heads, 4 x 1024 35.9 -> 30.8.  Tried: a block's scores beside the block before's exponentials (registers; reads next to their use: 89.5).
 // 16-byte granule g of a K row r sits at g ^ swz, so the 16 rows of a fragment read hit distinct banks; V rows are
 // swizzled so that the four rows of a transposing read do.
-// Two workgroups per CU (D = 192: 48 KB of LDS, 96 accumulator and 48 query registers per lane): one's softmax runs beside the
+// Two workgroups per CU (D = 192: 72 KB of LDS, 96 accumulator and 48 query registers per lane): one's softmax runs beside the
 // other's MFMAs.  Causal blocks are dealt longest first, then shortest first, so that the two of a CU add up alike.
 typedef short attn_v4i16 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) attn_v4i16 attn_lds_v4i16;
 
 template <int D> __device__ __forceinline__ int kswz(int row) { return D == 128 ? (row & 15) : ((row >> 1) & 7); }
 template <int D> __device__ __forceinline__ int vswz(int row) { return D == 128 ? ((row & 3) << 2) : (((row >> 1) & 1) << 2); }
+
+constexpr int kAttnStages = 3;
 
 template <int D, bool FINE>
 __global__ __launch_bounds__(256, 2) void attention_kernel(const bf16_t* __restrict__ qkv, int ld, int S, int nq, int nkv, int hpw,
@@ -121,10 +128,8 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const bf16_t* __restr
   constexpr int KB = 32, GPR = D / 8, NI = KB * GPR / 256;      // keys per block, granules per row, DMA instructions per operand
   constexpr int DT = D / 32, KS = D / 16;
   static_assert(KB * GPR % 256 == 0, "a block does not divide over the threads");
-  __shared__ __attribute__((aligned(16))) bf16_t K0[KB * D];
-  __shared__ __attribute__((aligned(16))) bf16_t K1[KB * D];
-  __shared__ __attribute__((aligned(16))) bf16_t V0[KB * D];
-  __shared__ __attribute__((aligned(16))) bf16_t V1[KB * D];
+  __shared__ __attribute__((aligned(16))) bf16_t K[kAttnStages][KB * D];
+  __shared__ __attribute__((aligned(16))) bf16_t V[kAttnStages][KB * D];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
@@ -142,32 +147,39 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const bf16_t* __restr
   const bf16_t* kbase = base + (size_t)(nq + kvh) * D;
   const bf16_t* vbase = base + (size_t)(nq + nkv + kvh) * D;
 
-  int krow[NI], kg[NI], vg[NI];                                 // this thread's row of a block and source granules
-#pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const int p = i * 256 + tid, row = p / GPR, pos = p - row * GPR;
-    krow[i] = row;
-    kg[i] = (pos ^ kswz<D>(row)) * 8;
-    vg[i] = (pos ^ vswz<D>(row)) * 8;
-  }
-  auto request = [&](int kv0, bf16_t* ks, bf16_t* vs) {
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const size_t o = (size_t)min(kv0 + krow[i], S - 1) * ld;
-      dma16(kbase + o + kg[i], ks + (i * 256 + wave * 64) * 8);
-      dma16(vbase + o + vg[i], vs + (i * 256 + wave * 64) * 8);
-    }
-  };
-  const int kv_first = window > 0 ? max(0, (q0 - window + 1)) & ~(KB - 1) : 0;
-  const int kv_end = min(q0 + QB, S);                           // keys [kv_first, kv_end)
-  request(kv_first, K0, V0);
-
   bf16x8 q[KS];
   {
     const bf16_t* qrow = base + (size_t)min(q0w + n, S - 1) * ld + head * D + h * 8;
 #pragma unroll
     for (int s = 0; s < KS; ++s) q[s] = *reinterpret_cast<const bf16x8*>(qrow + s * 16);
   }
+  const unsigned row_bytes = (unsigned)ld * (unsigned)sizeof(bf16_t);
+  unsigned koff[NI], voff[NI];                                  // this thread's granules of a block, in bytes from its first row
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int p = i * 256 + tid, row = p / GPR, pos = p - row * GPR;
+    koff[i] = row * row_bytes + (pos ^ kswz<D>(row)) * 16;
+    voff[i] = row * row_bytes + (pos ^ vswz<D>(row)) * 16;
+  }
+  // keys [kv0, kv0 + KB) into a stage; rows past the last one lie past the descriptor's end and read as zeros
+  auto request = [&](int kv0, auto stage_c) __attribute__((always_inline)) {
+    constexpr int st = decltype(stage_c)::value;
+    const unsigned long long left = (unsigned long long)(S - kv0) * row_bytes;
+    const unsigned bytes = left < 0xffffffffull ? (unsigned)left : 0xffffffffu;
+    const i32x4 kd = make_words(kbase + (size_t)kv0 * ld, bytes), vd = make_words(vbase + (size_t)kv0 * ld, bytes);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      dma16_unseen(kd, koff[i], 0, lds_address(K[st]) + (i * 256 + wave * 64) * 16);
+      dma16_unseen(vd, voff[i], 0, lds_address(V[st]) + (i * 256 + wave * 64) * 16);
+    }
+  };
+  const int kv_first = window > 0 ? max(0, (q0 - window + 1)) & ~(KB - 1) : 0;
+  const int kv_end = min(q0 + QB, S);                           // keys [kv_first, kv_end)
+  using std::integral_constant;
+  request(kv_first, integral_constant<int, 0>{});
+  if (kv_first + KB < kv_end) request(kv_first + KB, integral_constant<int, 1>{});
+#pragma unroll
+  for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(q[s]));   // q has arrived: a wait in the loop, where the compiler cannot know, would be for all transfers
   floatx16 o[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
@@ -180,25 +192,31 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const bf16_t* __restr
   const int vsw = vswz<D>(r16 >> 2);                            // the same for every key this lane reads (keys = r16 / 4 mod 4)
   const int ksw = kswz<D>(n);
 
-  auto block = [&](int kv0, const bf16_t* ks, const bf16_t* vs) {
+  auto block = [&](int kv0, const bf16_t* ks, const bf16_t* vs) __attribute__((always_inline)) {
     // nothing of this block is visible to this wave's queries?
     if (kv0 > q0w + 31 || (window > 0 && kv0 + KB - 1 <= q0w - window)) return;
     floatx16 st;
 #pragma unroll
     for (int i = 0; i < 16; ++i) st[i] = 0.f;
+    // (left to itself the compiler reads two fragments at a time and waits for them)
+    constexpr int kAhead = KS < 6 ? KS : 6;
+    bf16x8 kf[KS];
+    auto kread = [&](int s) __attribute__((always_inline)) { kf[s] = *reinterpret_cast<const bf16x8*>(ks + n * D + (((2 * s + h) ^ ksw) << 3)); };
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s) kread(s);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
-      const bf16x8 kf = *reinterpret_cast<const bf16x8*>(ks + n * D + (((2 * s + h) ^ ksw) << 3));
-      st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, q[s], st, 0, 0, 0);
+      st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s], q[s], st, 0, 0, 0);
+      if (s + kAhead < KS) kread(s + kAhead);
+      __builtin_amdgcn_sched_barrier(0);
     }
     // register i: key kv0 + 8 (i / 4) + 4 h + i % 4
     if (kv0 + KB - 1 > q0w || (window > 0 && q0w + 31 - kv0 >= window)) {
-      const int qi = q0w + n;
+      const int past = q0w + n - kv0 - 4 * h;                     // key 8 (i / 4) + i % 4 is seen from here on and up to `window` - 1 before
+      const unsigned seen = window > 0 ? window : 0x80000000u;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int key = kv0 + 8 * (i >> 2) + 4 * h + (i & 3);
-        if (key > qi || (window > 0 && qi - key >= window)) st[i] = -INFINITY;
-      }
+      for (int i = 0; i < 16; ++i) st[i] = (unsigned)(past - (8 * (i >> 2) + (i & 3))) < seen ? st[i] : -INFINITY;
     }
     float mx = st[0];
 #pragma unroll
@@ -236,15 +254,18 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const bf16_t* __restr
         if constexpr (FINE) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, v), pf[kk], o[dt], 0, 0, 0);
       }
   };
-  for (int kv0 = kv_first; kv0 < kv_end; kv0 += 2 * KB) {
-    sync_keep_loads<0>();                    // block kv0 has landed in every wave; nobody reads the other stage any more
-    if (kv0 + KB < kv_end) request(kv0 + KB, K1, V1);
-    block(kv0, K0, V0);
-    if (kv0 + KB < kv_end) {
-      sync_keep_loads<0>();
-      if (kv0 + 2 * KB < kv_end) request(kv0 + 2 * KB, K0, V0);
-      block(kv0 + KB, K1, V1);
-    }
+  // block kv0 has landed in every wave, nobody reads the stage of the block before it any more, and the block behind it may be on its way
+  auto turn = [&](int kv0, auto stage_c) __attribute__((always_inline)) {
+    constexpr int st = decltype(stage_c)::value;
+    if (kv0 + KB < kv_end) meet_waves<2 * NI>();
+    else meet_waves<0>();
+    if (kv0 + 2 * KB < kv_end) request(kv0 + 2 * KB, integral_constant<int, (st + 2) % kAttnStages>{});
+    block(kv0, K[st], V[st]);
+  };
+  for (int kv0 = kv_first; kv0 < kv_end; kv0 += kAttnStages * KB) {
+    turn(kv0, integral_constant<int, 0>{});
+    if (kv0 + KB < kv_end) turn(kv0 + KB, integral_constant<int, 1>{});
+    if (kv0 + 2 * KB < kv_end) turn(kv0 + 2 * KB, integral_constant<int, 2>{});
   }
   // y = O / l, then XSA: y -= tanh(alpha) <y, vn> vn with vn = v / |v| of the query's own token
   const int qi = q0w + n;

@@ -51,22 +51,8 @@ struct WideShape {
   static_assert(NT * BM * 128 <= kRing * kStageElems, "the activations lie in the stages");
 };
 
-// LDS-DMA that the compiler does not see as a write to LDS: it makes every LDS read that may meet one wait for all transfers, which the
-// meetings of phase 1 do exactly and for a buffer of the ring that is chosen at run time.  l: byte address in LDS of the wave's 1 KB.
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"      // that m0 is a reserved register: it may be written between the uses the compiler makes of it
-__device__ __forceinline__ void dma16_unseen(i32x4 rsrc, unsigned voff, unsigned soff, unsigned l) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(l), "v"(voff), "s"(rsrc), "s"(soff) : "m0", "memory");
-}
-#pragma clang diagnostic pop
-__device__ __forceinline__ i32x4 make_words(const void* base, unsigned bytes) {      // make_rsrc for it
-  const unsigned long long a = (unsigned long long)uniform(base);
-  return i32x4{(int)(unsigned)a, (int)(unsigned)(a >> 32), (int)bytes, 0x00020000};
-}
 // a lane's offset that lies past the descriptor's end whatever is in range of it is added: reads zeros
 __device__ __forceinline__ unsigned past_end(i32x4 words) { return (unsigned)words[2]; }
-__device__ __forceinline__ unsigned lds_address(bf16_t* p) { return (unsigned)(unsigned long long)(lds_void*)p; }
 
 // The w_down rows of a wave's 16*CT output columns in blocks of 128 K elements, on their way from memory order to MFMA operand order.  A
 // load gives each quad of lanes (a = lane / 16, b = lane / 4 % 4) 64 contiguous bytes, segment k_segment(a) of row 4 b + i in load i: the

@@ -156,6 +156,21 @@ __device__ __forceinline__ T* uniform(T* p) {
   return (T*)((unsigned long long)hi << 32 | lo);
 }
 
+// LDS-DMA that the compiler does not see as a write to LDS: it makes every LDS read that may meet one wait for all transfers, which
+// kernels that use it do exactly, and for a buffer that is chosen at run time.  l: byte address in LDS of the wave's 1 KB.
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"      // that m0 is a reserved register: it may be written between the uses the compiler makes of it
+__device__ __forceinline__ void dma16_unseen(i32x4 rsrc, unsigned voff, unsigned soff, unsigned l) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(l), "v"(voff), "s"(rsrc), "s"(soff) : "m0", "memory");
+}
+#pragma clang diagnostic pop
+__device__ __forceinline__ i32x4 make_words(const void* base, unsigned bytes) {      // make_rsrc for it
+  const unsigned long long a = (unsigned long long)uniform(base);
+  return i32x4{(int)(unsigned)a, (int)(unsigned)(a >> 32), (int)bytes, 0x00020000};
+}
+__device__ __forceinline__ unsigned lds_address(bf16_t* p) { return (unsigned)(unsigned long long)(lds_void*)p; }
+
 // WM waves along M (each MT 32-row tiles) x 4 waves along N (each NTW 32-column tiles).
 template <int MT, int NTW, int WM, int BK_ = kBK>
 struct Stripe {
