@@ -26,7 +26,7 @@ SYMBOLS = (
     "bibo_moe_train_state_bytes", "bibo_moe_forward_train", "bibo_moe_forward_train_balance", "bibo_moe_backward_saved",
     "bibo_moe_exp_attn_res_fwd", "bibo_moe_balance_step",
     "bibo_moe_exp_attn_res_norm_fwd", "bibo_moe_exp_carry_fwd", "bibo_moe_exp_silu_mul_fwd", "bibo_moe_exp_qk_norm_rope",
-    "bibo_moe_exp_attention_fwd", "bibo_moe_exp_rope_tables",
+    "bibo_moe_exp_attention_fwd", "bibo_moe_exp_norm_attention_fwd", "bibo_moe_exp_rope_tables",
 )
 STATIC_SCRATCH_BYTES = 16 << 20
 
@@ -97,7 +97,9 @@ def _declare(l):
                        ("bibo_moe_exp_silu_mul_fwd", [vp, ci, ci, vp, vp]),
                        ("bibo_moe_exp_qk_norm_rope", [vp, ci, ci, ci, ci, ci, ci, vp, vp, ci, cf, vp, vp, ci, ci, vp]),
                        ("bibo_moe_exp_rope_tables", [vp, ci, ci, ci, vp, vp, vp]),
-                       ("bibo_moe_exp_attention_fwd", [vp, ci, ci, ci, ci, ci, ci, ci, cf, vp, ci, vp, vp])):
+                       ("bibo_moe_exp_attention_fwd", [vp, ci, ci, ci, ci, ci, ci, ci, cf, vp, ci, vp, vp]),
+                       ("bibo_moe_exp_norm_attention_fwd", [vp, ci, ci, ci, ci, ci, ci, vp, vp, ci, cf, vp, vp, ci, ci, ci, cf, vp, ci, vp,
+                                                            vp])):
         getattr(l, name).restype, getattr(l, name).argtypes = ci, args
     l.bibo_moe_balance_step.restype = ci
     l.bibo_moe_balance_step.argtypes = [vp, vp, vp, ci, ctypes.c_float, ci, vp]

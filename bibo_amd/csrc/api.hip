@@ -1046,9 +1046,8 @@ int bibo_moe_exp_silu_mul_fwd(const void* gate_up, int T, int I, void* out, void
   return hip_rc(launch_silu_mul(gate_up, T, I, out, static_cast<hipStream_t>(stream)));
 }
 
-int bibo_moe_exp_qk_norm_rope(void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, const void* q_weight,
-                              const void* k_weight, int weight_dtype, float eps, const void* cos, const void* sin, int rope_dtype,
-                              int ld_rope, void* stream) {
+static int qk_norm_rope(void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, const void* q_weight, const void* k_weight,
+                        int weight_dtype, float eps, const void* cos, const void* sin, int rope_dtype, int ld_rope, bool keys_only, void* stream) {
   if (B < 0 || S < 0 || (long long)B * S > 0x3fffffffLL) return BIBO_ERR_BAD_SHAPE;
   if (!exp_attention_supported(n_heads, n_kv_heads, head_dim) || ld < (n_heads + 2 * n_kv_heads) * head_dim || ld % 8 != 0 ||
       (cos == nullptr) != (sin == nullptr) || (cos != nullptr && (ld_rope < head_dim / 2 || ld_rope % 8 != 0)))
@@ -1058,9 +1057,17 @@ int bibo_moe_exp_qk_norm_rope(void* qkv, int ld, int B, int S, int n_heads, int 
   if (!aligned16(qkv) || !vec_ok(q_weight, weight_dtype) || !vec_ok(k_weight, weight_dtype) || !vec_ok(cos, rope_dtype) ||
       !vec_ok(sin, rope_dtype))
     return BIBO_ERR_MISALIGNED;
+  if (keys_only && k_weight == nullptr && cos == nullptr) return BIBO_OK;
   return hip_rc(launch_qk_norm_rope(qkv, ld, B * S, S, n_heads, n_kv_heads, head_dim, vec(q_weight, weight_dtype),
-                                    vec(k_weight, weight_dtype), eps, vec(cos, rope_dtype), vec(sin, rope_dtype), ld_rope,
+                                    vec(k_weight, weight_dtype), eps, vec(cos, rope_dtype), vec(sin, rope_dtype), ld_rope, keys_only,
                                     static_cast<hipStream_t>(stream)));
+}
+
+int bibo_moe_exp_qk_norm_rope(void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, const void* q_weight,
+                              const void* k_weight, int weight_dtype, float eps, const void* cos, const void* sin, int rope_dtype,
+                              int ld_rope, void* stream) {
+  return qk_norm_rope(qkv, ld, B, S, n_heads, n_kv_heads, head_dim, q_weight, k_weight, weight_dtype, eps, cos, sin, rope_dtype, ld_rope, false,
+                      stream);
 }
 
 int bibo_moe_exp_rope_tables(const void* inv_freq, int inv_freq_dtype, int S, int half, void* cos, void* sin, void* stream) {
@@ -1070,8 +1077,8 @@ int bibo_moe_exp_rope_tables(const void* inv_freq, int inv_freq_dtype, int S, in
   return hip_rc(launch_rope_tables(vec(inv_freq, inv_freq_dtype), S, half, cos, sin, static_cast<hipStream_t>(stream)));
 }
 
-int bibo_moe_exp_attention_fwd(const void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, int window,
-                               float scale, const void* xsa_alpha, int alpha_dtype, void* out, void* stream) {
+static int attention(const void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, int window, float scale,
+                     const void* xsa_alpha, int alpha_dtype, Vec q_weight, float eps, Vec cos, Vec sin, int ld_rope, void* out, void* stream) {
   if (B < 0 || S < 0 || window < 0 || (long long)B * S * n_heads > 0x3fffffffLL) return BIBO_ERR_BAD_SHAPE;
   if (!exp_attention_supported(n_heads, n_kv_heads, head_dim) || ld < (n_heads + 2 * n_kv_heads) * head_dim || ld % 8 != 0 ||
       ld > kAttnMaxLd)
@@ -1079,8 +1086,33 @@ int bibo_moe_exp_attention_fwd(const void* qkv, int ld, int B, int S, int n_head
   if (B == 0 || S == 0) return BIBO_OK;
   if (!qkv || !out) return BIBO_ERR_NULL_POINTER;
   if (!aligned16(qkv) || !aligned16(out)) return BIBO_ERR_MISALIGNED;
-  return hip_rc(launch_exp_attention(qkv, ld, B, S, n_heads, n_kv_heads, head_dim, window, scale, vec(xsa_alpha, alpha_dtype), out,
-                                     static_cast<hipStream_t>(stream)));
+  return hip_rc(launch_exp_attention(qkv, ld, B, S, n_heads, n_kv_heads, head_dim, window, scale, vec(xsa_alpha, alpha_dtype), q_weight, eps, cos,
+                                     sin, ld_rope, out, static_cast<hipStream_t>(stream)));
+}
+
+int bibo_moe_exp_attention_fwd(const void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, int window,
+                               float scale, const void* xsa_alpha, int alpha_dtype, void* out, void* stream) {
+  const Vec none{nullptr, 0};
+  return attention(qkv, ld, B, S, n_heads, n_kv_heads, head_dim, window, scale, xsa_alpha, alpha_dtype, none, 0.f, none, none, 0, out, stream);
+}
+
+int bibo_moe_exp_norm_attention_fwd(void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, const void* q_weight,
+                                    const void* k_weight, int weight_dtype, float eps, const void* cos, const void* sin, int rope_dtype,
+                                    int ld_rope, int window, float scale, const void* xsa_alpha, int alpha_dtype, void* out, void* stream) {
+  // what the second half refuses, before the first has written anything
+  if (B < 0 || S < 0 || window < 0 || (long long)B * S * n_heads > 0x3fffffffLL) return BIBO_ERR_BAD_SHAPE;
+  if (ld > kAttnMaxLd) return BIBO_ERR_UNSUPPORTED;
+  if (B > 0 && S > 0 && !out) return BIBO_ERR_NULL_POINTER;
+  if (!aligned16(out)) return BIBO_ERR_MISALIGNED;
+  const bool here = (long long)B * S * n_heads * head_dim >= kQueryElems;
+  if (q_weight != nullptr || k_weight != nullptr || cos != nullptr) {
+    const int rc = qk_norm_rope(qkv, ld, B, S, n_heads, n_kv_heads, head_dim, q_weight, k_weight, weight_dtype, eps, cos, sin, rope_dtype, ld_rope,
+                                here, stream);
+    if (rc != BIBO_OK) return rc;
+  }
+  const Vec none{nullptr, 0};
+  return attention(qkv, ld, B, S, n_heads, n_kv_heads, head_dim, window, scale, xsa_alpha, alpha_dtype, here ? vec(q_weight, weight_dtype) : none, eps,
+                   here ? vec(cos, rope_dtype) : none, here ? vec(sin, rope_dtype) : none, ld_rope, out, stream);
 }
 
 }  // extern "C"

@@ -472,7 +472,7 @@ py::tuple exp_rope_tables(const Tensor& inv_freq, int64_t S) {
   return py::make_tuple(cos, sin);
 }
 
-// x [B, S, H] -> attention output [B, S, H]: one projection to q|k|v rows, norm and RoPE in place, attention with XSA, output
+// x [B, S, H] -> attention output [B, S, H]: one projection to q|k|v rows, attention of their norms and rotations with XSA, output
 // projection (the two products are library GEMMs)
 Tensor exp_attention(const Tensor& x, const Tensor& w_q, const Tensor& w_k, const Tensor& w_v, const Tensor& w_o, const c10::optional<Tensor>& q_weight,
                      const c10::optional<Tensor>& k_weight, double eps, const c10::optional<Tensor>& cos,
@@ -488,14 +488,11 @@ Tensor exp_attention(const Tensor& x, const Tensor& w_q, const Tensor& w_k, cons
   check_rows(qkv, "q|k|v rows", (int64_t)(n_heads + 2 * n_kv_heads) * head_dim);
   const int ld = (int)qkv.size(-1);
   hipStream_t s = stream_of(x);
-  if (q_weight.has_value() || k_weight.has_value() || cos.has_value())
-    check(bibo_moe_exp_qk_norm_rope(qkv.data_ptr(), ld, (int)B, (int)S, n_heads, n_kv_heads, head_dim, norm[0], norm[1], norm.dtype,
-                                    (float)eps, rope[0], rope[1], rope.dtype, head_dim, s),
-          "bibo_moe_exp_qk_norm_rope");
   const Tensor y = at::empty({B, S, (int64_t)n_heads * head_dim}, x.options());
-  check(bibo_moe_exp_attention_fwd(qkv.data_ptr(), ld, (int)B, (int)S, n_heads, n_kv_heads, head_dim, window, (float)scale, alpha[0],
-                                   alpha.dtype, y.data_ptr(), s),
-        "bibo_moe_exp_attention_fwd");
+  check(bibo_moe_exp_norm_attention_fwd(qkv.data_ptr(), ld, (int)B, (int)S, n_heads, n_kv_heads, head_dim, norm[0], norm[1], norm.dtype,
+                                        (float)eps, rope[0], rope[1], rope.dtype, head_dim, window, (float)scale, alpha[0], alpha.dtype,
+                                        y.data_ptr(), s),
+        "bibo_moe_exp_norm_attention_fwd");
   return at::linear(y, w_o);
 }
 

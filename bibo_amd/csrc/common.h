@@ -340,11 +340,12 @@ hipError_t launch_carry(const void* attn_read, const void* a, Vec theta, const v
 hipError_t launch_silu_mul(const void* gu, int T, int I, void* out, hipStream_t s);
 bool exp_attention_supported(int nq, int nkv, int D);
 constexpr int kAttnMaxLd = 1 << 26;      // 32 rows of keys lie within 32-bit byte offsets
+constexpr long long kQueryElems = 3 << 20;   // elements of the queries from which on the attention normalises and rotates them (measured at norm_rope_query)
 hipError_t launch_qk_norm_rope(void* qkv, int ld, int T, int S, int nq, int nkv, int D, Vec qw, Vec kw, float eps, Vec cos, Vec sin,
-                               int ld_rope, hipStream_t s);
+                               int ld_rope, bool keys_only, hipStream_t s);
 hipError_t launch_rope_tables(Vec inv_freq, int S, int half, void* cos, void* sin, hipStream_t s);
 hipError_t launch_exp_attention(const void* qkv, int ld, int B, int S, int nq, int nkv, int D, int window, float scale,
-                                Vec xsa_alpha, void* out, hipStream_t s);
+                                Vec xsa_alpha, Vec qw, float eps, Vec cos, Vec sin, int ld_rope, void* out, hipStream_t s);
 
 // ---- backward pass (backward.hip) ----
 struct BackwardBuffers {

@@ -17,17 +17,17 @@ __device__ __forceinline__ float row16_sum(float v) {      // sum over a DPP row
 }
 
 // ---- QK-norm (norm.py:19-24 on head rows) and RoPE (attn/rope.py, rotate-half), in place --------------------------
-// rows of qkv: [T, ld], the nq query heads first, then the nkv key heads, D elements each.  Sixteen lanes per head row; lane
+// rows of qkv: [T, ld], the nq query heads first, then the nkv key heads, D elements each; heads [first, nq + nkv).  Sixteen lanes per head row; lane
 // c < D / 16 owns elements 8c .. 8c + 7 of the first half and of the second half, i.e. whole rotation pairs.  Memory-bound:
-// one read and one write of the q and k columns.  qw, kw: [D], or NULL: no norm; cos, sin: rows of D / 2 at stride ld_rope, or NULL.
+// one read and one write of the columns (in front of attention_kernel from kQueryElems on only the keys': it takes the queries on their way).  qw, kw: [D], or NULL: no norm; cos, sin: rows of D / 2 at stride ld_rope, or NULL.
 template <int D>
-__global__ __launch_bounds__(256) void qk_norm_rope_kernel(bf16_t* __restrict__ qkv, int ld, int T, int S, int nq, int nkv,
+__global__ __launch_bounds__(256) void qk_norm_rope_kernel(bf16_t* __restrict__ qkv, int ld, int T, int S, int first, int nq, int nkv,
                                                            Vec qw, Vec kw, float eps, Vec cos, Vec sin, int ld_rope) {
   constexpr int kLanes = D / 16;
-  const int heads = nq + nkv;
+  const int heads = nq + nkv - first;
   const long long g = ((long long)blockIdx.x * 256 + threadIdx.x) >> 4;
   if (g >= (long long)T * heads) return;                   // whole groups of 16 lanes
-  const int t = (int)(g / heads), hd = (int)(g - (long long)t * heads);
+  const int t = (int)(g / heads), hd = first + (int)(g - (long long)t * heads);
   const int c = threadIdx.x & 15;
   const bool live = c < kLanes;
   bf16_t* row = qkv + (size_t)t * ld + hd * D;
@@ -121,10 +121,72 @@ template <int D> __device__ __forceinline__ int vswz(int row) { return D == 128 
 
 constexpr int kAttnStages = 3;
 
+// QK-norm and RoPE of the queries, as in qk_norm_rope_kernel; weight, cos, sin may be NULL
+struct QueryNorm {
+  Vec weight;
+  float eps;
+  Vec cos, sin;
+  int ld_rope;
+};
+
+// The fragments of row `pos` of a head: the half-waves h of lane n hold granules 2 s + h.  The same sums in the same order as in
+// qk_norm_rope_kernel, whose lane c holds granules c and c + D / 16, hence the same bits.  In place they
+// are read and written once more, here they lengthen the chain in front of a wave's first product.  Both launches, us, queries in place / here,
+// 4 and 2 heads of 192, causal with norm and window 128 with norm and RoPE: T = 16384: 88.1 / 80.4 and 47.6 / 44.0; 8192: 76.8 / 71.6 and 32.2 /
+// 30.3; 4096: 71.6 / 70.2 and 26.8 / 26.5; 2048: 67.0 / 67.8 and 22.7 / 24.4; 128: 15.1 / 18.2.  Hence kQueryElems, the 4096 tokens of these.
+// weights(s, first half's 8, second half's 8), tables(s, cos, sin): of granule 2 s + h.
+template <int KS, typename Weights, typename Tables>
+__device__ __forceinline__ void norm_rope_query(const QueryNorm& nr, bf16x8 (&q)[KS], Weights weights, Tables tables) {
+  constexpr int KH = KS / 2, D = 16 * KS;
+  float rinv = 0.f;
+  if (nr.weight.p != nullptr) {
+    float t[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < KH; ++s) {
+      float ss = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float a = (float)q[s][e], b = (float)q[s + KH][e];
+        ss = fmaf(a, a, fmaf(b, b, ss));
+      }
+      const Pair p = lanes32(ss);
+      t[s] = p.a + p.b;
+    }
+    rinv = rsqrtf((((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]))) / (float)D + nr.eps);
+  }
+#pragma unroll
+  for (int s = 0; s < KH; ++s) {
+    float a[8], b[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) { a[e] = (float)q[s][e]; b[e] = (float)q[s + KH][e]; }
+    if (nr.weight.p != nullptr) {
+      float wa[8], wb[8];
+      weights(s, wa, wb);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        a[e] = wa[e] * (float)(bf16_t)(a[e] * rinv);
+        b[e] = wb[e] * (float)(bf16_t)(b[e] * rinv);
+      }
+    }
+    if (nr.cos.p != nullptr) {
+      float co[8], si[8];
+      tables(s, co, si);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float x = a[e], y = b[e];
+        a[e] = x * co[e] - y * si[e];
+        b[e] = y * co[e] + x * si[e];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) { q[s][e] = (bf16_t)a[e]; q[s + KH][e] = (bf16_t)b[e]; }
+  }
+}
+
 template <int D, bool FINE>
 __global__ __launch_bounds__(256, 2) void attention_kernel(const bf16_t* __restrict__ qkv, int ld, int S, int nq, int nkv, int hpw,
                                                            int heads, int nqb, int window, float scale_log2,
-                                                           Vec xsa_alpha, bf16_t* __restrict__ out) {
+                                                           Vec xsa_alpha, QueryNorm nr, bf16_t* __restrict__ out) {
   constexpr int KB = 32, GPR = D / 8, NI = KB * GPR / 256;      // keys per block, granules per row, DMA instructions per operand
   constexpr int DT = D / 32, KS = D / 16;
   static_assert(KB * GPR % 256 == 0, "a block does not divide over the threads");
@@ -178,8 +240,43 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const bf16_t* __restr
   using std::integral_constant;
   request(kv_first, integral_constant<int, 0>{});
   if (kv_first + KB < kv_end) request(kv_first + KB, integral_constant<int, 1>{});
+  // the tables of this lane's granules, requested with the queries (bf16 ones; load by load behind them it all took 8 us)
+  constexpr int KH = KS / 2;
+  const int pos = min(q0w + n, S - 1);
+  const bool fetched = (nr.weight.p == nullptr || nr.weight.bf16) && (nr.cos.p == nullptr || (nr.cos.bf16 && nr.sin.bf16));
+  const size_t at = (size_t)pos * nr.ld_rope + h * 8;
+  bf16x8 ct[KH], sn[KH];
+  if (fetched && nr.cos.p != nullptr)
+#pragma unroll
+    for (int s = 0; s < KH; ++s) {
+      ct[s] = *reinterpret_cast<const bf16x8*>(static_cast<const bf16_t*>(nr.cos.p) + at + s * 16);
+      sn[s] = *reinterpret_cast<const bf16x8*>(static_cast<const bf16_t*>(nr.sin.p) + at + s * 16);
+    }
 #pragma unroll
   for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(q[s]));   // q has arrived: a wait in the loop, where the compiler cannot know, would be for all transfers
+  if (nr.weight.p != nullptr || nr.cos.p != nullptr) {
+    auto widen = [](bf16x8 v, float (&to)[8]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) to[e] = (float)v[e];
+    };
+    if (fetched) {
+      bf16x8 wt[KS];
+      if (nr.weight.p != nullptr)
+#pragma unroll
+        for (int s = 0; s < KS; ++s) wt[s] = *reinterpret_cast<const bf16x8*>(static_cast<const bf16_t*>(nr.weight.p) + s * 16 + h * 8);
+      norm_rope_query<KS>(nr, q, [&](int s, float (&a)[8], float (&b)[8]) __attribute__((always_inline)) { widen(wt[s], a); widen(wt[s + KH], b); },
+                          [&](int s, float (&c)[8], float (&d)[8]) __attribute__((always_inline)) { widen(ct[s], c); widen(sn[s], d); });
+    } else
+      norm_rope_query<KS>(nr, q,
+                          [&](int s, float (&a)[8], float (&b)[8]) __attribute__((always_inline)) {
+                            load8(nr.weight, s * 16 + h * 8, a);
+                            load8(nr.weight, D / 2 + s * 16 + h * 8, b);
+                          },
+                          [&](int s, float (&c)[8], float (&d)[8]) __attribute__((always_inline)) {
+                            load8(nr.cos, at + s * 16, c);
+                            load8(nr.sin, at + s * 16, d);
+                          });
+  }
   floatx16 o[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
@@ -322,15 +419,19 @@ bool exp_attention_supported(int nq, int nkv, int D) {
 }
 
 hipError_t launch_qk_norm_rope(void* qkv, int ld, int T, int S, int nq, int nkv, int D, Vec qw, Vec kw, float eps, Vec cos, Vec sin,
-                               int ld_rope, hipStream_t s) {
-  const long long groups = (long long)T * (nq + nkv);
+                               int ld_rope, bool keys_only, hipStream_t s) {
+  const int first = keys_only ? nq : 0;
+  const long long groups = (long long)T * (nq + nkv - first);
   if (groups == 0) return hipSuccess;
   const dim3 grid((unsigned)((groups + 15) / 16));
   bf16_t* p = static_cast<bf16_t*>(qkv);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, p, ld, T, S, first, nq, nkv, qw, kw, eps, cos, sin, ld_rope);
+  };
   switch (D) {
-    case 64: hipLaunchKernelGGL(qk_norm_rope_kernel<64>, grid, dim3(256), 0, s, p, ld, T, S, nq, nkv, qw, kw, eps, cos, sin, ld_rope); break;
-    case 128: hipLaunchKernelGGL(qk_norm_rope_kernel<128>, grid, dim3(256), 0, s, p, ld, T, S, nq, nkv, qw, kw, eps, cos, sin, ld_rope); break;
-    case 192: hipLaunchKernelGGL(qk_norm_rope_kernel<192>, grid, dim3(256), 0, s, p, ld, T, S, nq, nkv, qw, kw, eps, cos, sin, ld_rope); break;
+    case 64: launch(qk_norm_rope_kernel<64>); break;
+    case 128: launch(qk_norm_rope_kernel<128>); break;
+    case 192: launch(qk_norm_rope_kernel<192>); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -345,7 +446,7 @@ hipError_t launch_rope_tables(Vec inv_freq, int S, int half, void* cos, void* si
 }
 
 hipError_t launch_exp_attention(const void* qkv, int ld, int B, int S, int nq, int nkv, int D, int window, float scale,
-                                Vec xsa_alpha, void* out, hipStream_t s) {
+                                Vec xsa_alpha, Vec qw, float eps, Vec cos, Vec sin, int ld_rope, void* out, hipStream_t s) {
   if (B == 0 || S == 0) return hipSuccess;
   const int g = nq / nkv;
   const int hpw = g % 4 == 0 ? 4 : (g % 2 == 0 ? 2 : 1);
@@ -355,7 +456,7 @@ hipError_t launch_exp_attention(const void* qkv, int ld, int B, int S, int nq, i
   const bf16_t* p = static_cast<const bf16_t*>(qkv);
   bf16_t* o = static_cast<bf16_t*>(out);
   auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, p, ld, S, nq, nkv, hpw, heads, nqb, window, sl, xsa_alpha, o);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, p, ld, S, nq, nkv, hpw, heads, nqb, window, sl, xsa_alpha, QueryNorm{qw, eps, cos, sin, ld_rope}, o);
   };
   const bool fine = window > 0;
   switch (D) {

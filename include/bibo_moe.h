@@ -398,6 +398,8 @@ int bibo_moe_exp_attn_res_fwd(const void* const* candidates, int n_candidates, c
  *   last `window` keys), softmax in fp32, with the XSA correction y - tanh(alpha) <y, vn> vn (xsa_alpha [n_heads] or NULL;
  *   src/modeling/attn/xsa.py:41-54).  head_dim in {64, 128, 192}; n_heads / n_kv_heads = 1 or even; ld at most 2^26
  *   (BIBO_ERR_UNSUPPORTED otherwise).
+ * bibo_moe_exp_norm_attention_fwd: bibo_moe_exp_qk_norm_rope and bibo_moe_exp_attention_fwd of the same rows, the same bits; of many
+ *   rows only the keys are normalised and rotated in place, the queries on their way into the attention (qkv then keeps them as they were).
  */
 int bibo_moe_exp_attn_res_norm_fwd(const void* const* candidates, int n_candidates, const void* score_a, const void* score_b,
                                    float eps, const void* norm_weight, float norm_eps, int weight_dtype, int T, int H, int dtype,
@@ -411,6 +413,9 @@ int bibo_moe_exp_qk_norm_rope(void* qkv, int ld, int B, int S, int n_heads, int 
 int bibo_moe_exp_rope_tables(const void* inv_freq, int inv_freq_dtype, int S, int half, void* cos, void* sin, void* stream);
 int bibo_moe_exp_attention_fwd(const void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, int window,
                                float scale, const void* xsa_alpha, int alpha_dtype, void* out, void* stream);
+int bibo_moe_exp_norm_attention_fwd(void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, const void* q_weight,
+                                    const void* k_weight, int weight_dtype, float eps, const void* cos, const void* sin, int rope_dtype,
+                                    int ld_rope, int window, float scale, const void* xsa_alpha, int alpha_dtype, void* out, void* stream);
 
 #ifdef __cplusplus
 }

@@ -94,6 +94,33 @@ def test_banded_attention_is_as_exact_as_its_output_type(B, S, nq, nkv, D, windo
     assert float((out.cpu().double() - ref).norm()) <= 1.001 * float((ref.bfloat16().double() - ref).norm())
 
 
+@pytest.mark.parametrize("D,nq,nkv", [(64, 2, 2), (128, 4, 2), (192, 4, 2)])
+@pytest.mark.parametrize("S,window,many", [(1, 0, True), (33, 16, True), (97, 0, True), (200, 64, True), (97, 64, False)])
+@pytest.mark.parametrize("normed,rope,bf16", [(True, True, True), (True, False, False), (False, True, False), (False, False, True)])
+def test_attention_takes_the_queries_as_the_norm_kernel_does(D, nq, nkv, S, window, many, normed, rope, bf16):
+    """One call and two leave the same bits: the queries' norm and rotation inside the attention add in the norm kernel's order.  Rows
+    wider than their heads, tables wider than D / 2; from 3 << 20 elements of queries on the one call leaves the queries alone."""
+    B = -(-(3 << 20) // (S * nq * D)) if many else 2
+    ld, ldr = (nq + 2 * nkv) * D + 8, D
+    g = torch.Generator(device=DEV).manual_seed(S + D)
+    dt = torch.bfloat16 if bf16 else torch.float32
+    rows = torch.randn(B * S, ld, generator=g, device=DEV).bfloat16()
+    qw, kw = ((torch.rand(D, generator=g, device=DEV) + 0.5).to(dt) for _ in range(2)) if normed else (None, None)
+    ang = torch.rand(S, ldr, generator=g, device=DEV) * 6
+    cos, sin = (ang.cos().to(dt), ang.sin().to(dt)) if rope else (None, None)
+    xsa = torch.randn(nq, generator=g, device=DEV)
+    pp = lambda t: None if t is None else _ptr(t)
+    code = 0 if bf16 else 1                                        # BIBO_DTYPE_BF16, BIBO_DTYPE_F32
+    norm = (pp(qw), pp(kw), code, ctypes.c_float(1e-6), pp(cos), pp(sin), code, ldr)
+    one, two = rows.clone(), rows.clone()
+    out = [torch.empty(B * S, nq * D, device=DEV, dtype=torch.bfloat16) for _ in range(2)]
+    _call("bibo_moe_exp_norm_attention_fwd", _ptr(one), ld, B, S, nq, nkv, D, *norm, window, ctypes.c_float(D ** -0.5), _ptr(xsa), 1, _ptr(out[0]))
+    _call("bibo_moe_exp_qk_norm_rope", _ptr(two), ld, B, S, nq, nkv, D, *norm)
+    _call("bibo_moe_exp_attention_fwd", _ptr(two), ld, B, S, nq, nkv, D, window, ctypes.c_float(D ** -0.5), _ptr(xsa), 1, _ptr(out[1]))
+    assert torch.equal(out[0], out[1])
+    assert torch.equal(one[:, :nq * D], (rows if many else two)[:, :nq * D]) and torch.equal(one[:, nq * D:], two[:, nq * D:])
+
+
 def test_attention_refuses_what_it_does_not_take():
     args = lambda nq, nkv, D: (None, 4096, 1, 4, nq, nkv, D, 0, ctypes.c_float(1.0), None, 1, None, None)
     for nq, nkv, D in ((4, 2, 96), (3, 2, 64), (3, 1, 64), (4, 0, 64)):
