@@ -520,7 +520,10 @@ __global__ __launch_bounds__(256) void router_gateup_kernel(const bf16_t* __rest
 // its TOK rows arrive in LDS by LDS-DMA, one wave per row computes BiBoRMSNorm (src/modeling/norm.py:19-24) with the
 // arithmetic and the summation order of rmsnorm_bf16x8_kernel (so both produce the same bits), writes the normalised
 // row back to LDS in place and to `xn` in memory, and the logits are then multiplied from the resident rows while
-// w_router streams through two LDS stages as in router_mfma_kernel.  x rows are stored as H/128 chunks of
+// w_router streams through two LDS stages, two chunks a round trip, the first two requested in front of the rows.  A wave's four rows pass
+// through the norm side by side and leave for memory behind the products: one row after the other and a chunk a round trip the whole seam
+// took, us: H = 768, I = 384, k = 6: T = 16: 38.5 -> 37.7, 64: 43.2 -> 41.9, 2049: 66.0 -> 64.6, 6000: 127.2 -> 125.7; H = 512, I = 256, T = 512:
+// 30.9 -> 29.7 (all with the sums over a wave in common.h, which are 0.2 to 0.8 of it).  x rows are stored as H/128 chunks of
 // [TOK][128], granule c of a chunk row r at position c ^ (r & 15).
 // What the selection needs lies where the rows were: 80 KB of LDS at TOK = 32 and H = 768, so that two workgroups share a CU and one's
 // round trips pass behind the other's arithmetic (one a CU: 30.0 -> 21.7 us at T = 16384, 26.9 -> 19.9 at 12000).  RING: six chunks of
@@ -584,7 +587,10 @@ __global__ __launch_bounds__(TOK * 16) void router_norm_mfma_kernel(const bf16_t
     if constexpr (i == 0) return wst0; else if constexpr (i == 1) return wst1; else if constexpr (i == 2) return wst2;
     else if constexpr (i == 3) return wst3; else if constexpr (i == 4) return wst4; else return wst5;
   };
-  if constexpr (!RING) issue_w(0, wst0);
+  if constexpr (!RING) {
+    issue_w(0, wst0);
+    if (nchunks > 1) issue_w(kRouterKC, wst1);
+  }
   // the raw rows: instruction i is chunk i of every row (TOK * 16 granules = one per thread)
   {
     const int row = tid >> 4;
@@ -607,38 +613,43 @@ __global__ __launch_bounds__(TOK * 16) void router_norm_mfma_kernel(const bf16_t
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
   }
-  // RMSNorm, one wave per row, four rows per wave; lane takes logical granules u*64 + lane of the row
+  // RMSNorm, one wave per row, four rows per wave, which pass through each step side by side (one after the other their reads wait for the
+  // writes of the row before); lane takes logical granules u*64 + lane of the row.  They leave for memory behind the products, whose waits for
+  // w_router would be for them too.
+  bf16x8 v[4][kNormGran];
   {
+    float rinv[4];
+    auto place = [&](int j, int u) {
+      const int c = u * kWave + lane, r = wave * 4 + j;
+      return xs + (((c >> 4) * TOK + r) * kRouterGran + ((c & 15) ^ (r & 15))) * 8;
+    };
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int u = 0; u < kNormGran; ++u)
+        if (u * kWave + lane < ngran) v[j][u] = *reinterpret_cast<const bf16x8*>(place(j, u));
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int r = wave * 4 + j;
-      bf16x8 v[kNormGran];
-      bf16_t* loc[kNormGran];
       float ss = 0.f;
 #pragma unroll
-      for (int u = 0; u < kNormGran; ++u) {
-        const int c = u * kWave + lane;
-        if (c < ngran) {
-          loc[u] = xs + (((c >> 4) * TOK + r) * kRouterGran + ((c & 15) ^ (r & 15))) * 8;
-          v[u] = *reinterpret_cast<const bf16x8*>(loc[u]);
+      for (int u = 0; u < kNormGran; ++u)
+        if (u * kWave + lane < ngran)
 #pragma unroll
-          for (int q = 0; q < 8; ++q) ss = fmaf((float)v[u][q], (float)v[u][q], ss);
+          for (int q = 0; q < 8; ++q) ss = fmaf((float)v[j][u][q], (float)v[j][u][q], ss);
+      rinv[j] = ss;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) rinv[j] = rsqrtf(wave_sum(rinv[j]) / (float)H + eps);       // norm.py:22-23
+#pragma unroll
+    for (int u = 0; u < kNormGran; ++u) {
+      const int c = u * kWave + lane;
+      if (c < ngran)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+          for (int q = 0; q < 8; ++q) v[j][u][q] = (bf16_t)((float)wv[u][q] * (float)(bf16_t)((float)v[j][u][q] * rinv[j]));   // norm.py:24
+          *reinterpret_cast<bf16x8*>(place(j, u)) = v[j][u];
         }
-      }
-      ss = wave_sum(ss);
-      const float rinv = rsqrtf(ss / (float)H + eps);                                   // norm.py:22-23
-      const bool live = t0 + r < T;
-#pragma unroll
-      for (int u = 0; u < kNormGran; ++u) {
-        const int c = u * kWave + lane;
-        if (c < ngran) {
-          bf16x8 o;
-#pragma unroll
-          for (int q = 0; q < 8; ++q) o[q] = (bf16_t)((float)wv[u][q] * (float)(bf16_t)((float)v[u][q] * rinv));   // norm.py:24
-          *reinterpret_cast<bf16x8*>(loc[u]) = o;
-          if (live) *reinterpret_cast<bf16x8*>(xn + (size_t)(t0 + r) * H + c * 8) = o;
-        }
-      }
     }
   }
   const int tm = wave >> 2, en = wave & 3;
@@ -661,7 +672,7 @@ __global__ __launch_bounds__(TOK * 16) void router_norm_mfma_kernel(const bf16_t
         const int c = c0 + decltype(ic)::value;
         if (c >= nchunks) return;
         if (c == 0) __builtin_amdgcn_s_waitcnt(0xc07f);          // this wave's normalised rows are in LDS
-        switch (min(nchunks - 1 - c, kRouterRing - 1)) {         // chunks that may still be on their way (stores of rows do no harm)
+        switch (min(nchunks - 1 - c, kRouterRing - 1)) {         // chunks that may still be on their way
           case 0: sync_keep_loads<0>(); break;
           case 1: sync_keep_loads<kWPer>(); break;
           case 2: sync_keep_loads<2 * kWPer>(); break;
@@ -677,19 +688,25 @@ __global__ __launch_bounds__(TOK * 16) void router_norm_mfma_kernel(const bf16_t
         }
       });
   } else {
-    for (int c0 = 0; c0 < nchunks; c0 += 2) {
+    for (int c0 = 0; c0 < nchunks; c0 += 2) {            // two chunks a round trip; the first two are requested in front of the rows
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();                                   // first pass: also the normalised rows of the other waves
-      if (c0 + 1 < nchunks) issue_w((c0 + 1) * kRouterKC, wst1);
       multiply(xs + (size_t)c0 * TOK * kRouterKC, wst0);
-      if (c0 + 1 < nchunks) {
-        __builtin_amdgcn_s_waitcnt(0);
+      if (c0 + 1 < nchunks) multiply(xs + (size_t)(c0 + 1) * TOK * kRouterKC, wst1);
+      if (c0 + 2 < nchunks) {
         __syncthreads();
-        if (c0 + 2 < nchunks) issue_w((c0 + 2) * kRouterKC, wst0);
-        multiply(xs + (size_t)(c0 + 1) * TOK * kRouterKC, wst1);
+        issue_w((c0 + 2) * kRouterKC, wst0);
+        if (c0 + 3 < nchunks) issue_w((c0 + 3) * kRouterKC, wst1);
       }
     }
   }
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int u = 0; u < kNormGran; ++u) {
+      const int c = u * kWave + lane, t = t0 + wave * 4 + j;
+      if (c < ngran && t < T) *reinterpret_cast<bf16x8*>(xn + (size_t)t * H + c * 8) = v[j][u];
+    }
   // the rows' LDS holds what is left to do: scores, bias, selections
   __syncthreads();
   float* sc = reinterpret_cast<float*>(xs);
