@@ -31,6 +31,7 @@
 // Reference: BiBoFusedExperts.forward, src/modeling/ffn/moe.py:81-93.
 #pragma once
 
+#include <climits>
 #include <type_traits>
 
 #include "experts_fused_launch.h"
@@ -333,7 +334,7 @@ __global__ __launch_bounds__(512) void experts_fused_kernel(const bf16_t* __rest
     cb = flat - tile * ncb;
     find_tile(tm, tile, e, first, rows, tile_e);
     first = tile_e * BM;
-  } else if (!find_round_tile<BM, (SCAN > 0)>(tm, blockIdx.x, e, first, rows, tile_e)) {
+  } else if (!find_round_tile<BM, (NT == 2 ? 2 : 3), (SCAN > 0 ? 0 : NT == 1 ? 1 : INT_MAX), (NT == 2 ? 2 : 3)>(tm, blockIdx.x, e, first, rows, tile_e)) {
     return;
   }
   const int row0 = __builtin_amdgcn_readlane(tm.lo, e) + first;

@@ -209,7 +209,7 @@ __global__ __launch_bounds__(512) void experts_wide_kernel(const bf16_t* __restr
 
   const TileMap tm = load_tile_map(offsets, E);
   int e, first, rows, tile_e;                           // the same for every lane, in scalar registers
-  if (!find_round_tile<BM, false>(tm, blockIdx.x, e, first, rows, tile_e)) return;
+  if (!find_round_tile<BM, 2, 2, 1>(tm, blockIdx.x, e, first, rows, tile_e)) return;
   const int row0 = __builtin_amdgcn_readlane(tm.lo, e) + first;
   // the tiles of an expert walk the weights of a K step from different blocks of columns on (experts_fused_kernel says why)
   const int rot = tile_e % NT;

@@ -13,11 +13,14 @@ DEV = torch.device("cuda:0")
 # rows per expert, 64 experts.  128-row tiles:
 ROWS = {
     "two rounds": [768] * 32 + [769] * 32,               # 3.25 blocks a tile: 8 of 3, or 7 of 3 and one of 4
-    "two rounds, 2.5 blocks": [560] * 64,                                   # 18 blocks in 7 or 8 tiles
-    "three rounds": [1120, 1121, 1, 0, 31, 1500, 1100, 1152] * 8,
-    "four rounds, hot experts": [16000] * 4 + [540] * 30 + [33] * 30,       # 3.25 blocks a tile
-    "four rounds": [1500] * 64,
-    "one expert": [65536 + 100] + [0] * 63,                                 # 513 tiles of 128: three rounds, 2.75 blocks
+    "two rounds, 2.25 blocks": [560] * 64,                                  # 18 blocks in 8 tiles
+    "two rounds, idle experts": [1120, 1121, 1, 0, 31, 1500, 1100, 1152] * 8,
+    "two rounds, 3.5 blocks": [870] * 64,                                   # 28 blocks in 8 tiles
+    "three rounds": [1170] * 32 + [1160, 1180] * 16,                        # 37 blocks in 12 tiles
+    "four rounds": [1540] * 60 + [0, 33, 3000, 1540],                       # 49 blocks in 16 tiles
+    "four rounds, hot experts": [16384] * 4 + [540] * 60,                   # 512 blocks in 158 tiles, 17 in 6
+    "one height": [1500] * 64,                                              # 47 blocks in 12 tiles, three full rounds
+    "one expert": [65536 + 100] + [0] * 63,
 }
 
 
@@ -42,7 +45,7 @@ def _check(rows, H, I, algo):
     return run, got
 
 
-@pytest.mark.parametrize("H,I", [(128, 128), (128, 384)])
+@pytest.mark.parametrize("H,I", [(128, 128), (128, 256), (128, 384)])      # one height; two from two rounds on; from three on
 @pytest.mark.parametrize("name", ROWS)
 def test_two_heights(name, H, I):
     run, got = _check(ROWS[name], H, I, "fused")
