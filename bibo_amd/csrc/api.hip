@@ -1080,8 +1080,7 @@ int bibo_moe_exp_rope_tables(const void* inv_freq, int inv_freq_dtype, int S, in
 static int attention(const void* qkv, int ld, int B, int S, int n_heads, int n_kv_heads, int head_dim, int window, float scale,
                      const void* xsa_alpha, int alpha_dtype, Vec q_weight, float eps, Vec cos, Vec sin, int ld_rope, void* out, void* stream) {
   if (B < 0 || S < 0 || window < 0 || (long long)B * S * n_heads > 0x3fffffffLL) return BIBO_ERR_BAD_SHAPE;
-  if (!exp_attention_supported(n_heads, n_kv_heads, head_dim) || ld < (n_heads + 2 * n_kv_heads) * head_dim || ld % 8 != 0 ||
-      ld > kAttnMaxLd)
+  if (!exp_attention_supported(n_heads, n_kv_heads, head_dim) || ld < (n_heads + 2 * n_kv_heads) * head_dim || ld % 8 != 0)
     return BIBO_ERR_UNSUPPORTED;
   if (B == 0 || S == 0) return BIBO_OK;
   if (!qkv || !out) return BIBO_ERR_NULL_POINTER;
@@ -1101,7 +1100,6 @@ int bibo_moe_exp_norm_attention_fwd(void* qkv, int ld, int B, int S, int n_heads
                                     int ld_rope, int window, float scale, const void* xsa_alpha, int alpha_dtype, void* out, void* stream) {
   // what the second half refuses, before the first has written anything
   if (B < 0 || S < 0 || window < 0 || (long long)B * S * n_heads > 0x3fffffffLL) return BIBO_ERR_BAD_SHAPE;
-  if (ld > kAttnMaxLd) return BIBO_ERR_UNSUPPORTED;
   if (B > 0 && S > 0 && !out) return BIBO_ERR_NULL_POINTER;
   if (!aligned16(out)) return BIBO_ERR_MISALIGNED;
   const bool here = (long long)B * S * n_heads * head_dim >= kQueryElems;

@@ -339,7 +339,7 @@ hipError_t launch_carry(const void* attn_read, const void* a, Vec theta, const v
                         void* prefix_out, hipStream_t s);
 hipError_t launch_silu_mul(const void* gu, int T, int I, void* out, hipStream_t s);
 bool exp_attention_supported(int nq, int nkv, int D);
-constexpr int kAttnMaxLd = 1 << 26;      // 32 rows of keys lie within 32-bit byte offsets
+constexpr int kAttnNearLd = 1 << 26;     // up to here 32 rows of keys lie within 32-bit byte offsets
 constexpr long long kQueryElems = 3 << 20;   // elements of the queries from which on the attention normalises and rotates them (measured at norm_rope_query)
 hipError_t launch_qk_norm_rope(void* qkv, int ld, int T, int S, int nq, int nkv, int D, Vec qw, Vec kw, float eps, Vec cos, Vec sin,
                                int ld_rope, bool keys_only, hipStream_t s);

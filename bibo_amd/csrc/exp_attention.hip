@@ -195,7 +195,8 @@ __device__ __forceinline__ Granules swap_halves(u32x4 v) {
   return {{(unsigned)x[0], (unsigned)y[0]}, {(unsigned)x[1], (unsigned)y[1]}};
 }
 
-template <int D, bool FINE>
+// FAR: rows further apart than kAttnNearLd, by 64-bit addresses.
+template <int D, bool FINE, bool FAR>
 __global__ __launch_bounds__(256, 2) void attention_kernel(const bf16_t* __restrict__ qkv, int ld, int S, int nq, int nkv, int hpw,
                                                            int heads, int nqb, int window, float scale_log2,
                                                            Vec xsa_alpha, QueryNorm nr, bf16_t* __restrict__ out) {
@@ -238,6 +239,16 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const bf16_t* __restr
   // keys [kv0, kv0 + KB) into a stage; rows past the last one lie past the descriptor's end and read as zeros
   auto request = [&](int kv0, auto stage_c) __attribute__((always_inline)) {
     constexpr int st = decltype(stage_c)::value;
+    if constexpr (FAR) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int p = i * 256 + tid, row = p / GPR, pos = p - row * GPR;
+        const size_t o = (size_t)min(kv0 + row, S - 1) * ld;
+        dma16(kbase + o + (pos ^ kswz<D>(row)) * 8, K[st] + (i * 256 + wave * 64) * 8);
+        dma16(vbase + o + (pos ^ vswz<D>(row)) * 8, V[st] + (i * 256 + wave * 64) * 8);
+      }
+      return;
+    }
     const unsigned long long left = (unsigned long long)(S - kv0) * row_bytes;
     const unsigned bytes = left < 0xffffffffull ? (unsigned)left : 0xffffffffu;
     const i32x4 kd = make_words(kbase + (size_t)kv0 * ld, bytes), vd = make_words(vbase + (size_t)kv0 * ld, bytes);
@@ -478,11 +489,18 @@ hipError_t launch_exp_attention(const void* qkv, int ld, int B, int S, int nq, i
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, p, ld, S, nq, nkv, hpw, heads, nqb, window, sl, xsa_alpha, QueryNorm{qw, eps, cos, sin, ld_rope}, o);
   };
-  const bool fine = window > 0;
+  auto pick = [&](auto d) {
+    constexpr int HD = decltype(d)::value;
+    if (ld > kAttnNearLd) {
+      if (window > 0) launch(attention_kernel<HD, true, true>); else launch(attention_kernel<HD, false, true>);
+    } else {
+      if (window > 0) launch(attention_kernel<HD, true, false>); else launch(attention_kernel<HD, false, false>);
+    }
+  };
   switch (D) {
-    case 64: if (fine) launch(attention_kernel<64, true>); else launch(attention_kernel<64, false>); break;
-    case 128: if (fine) launch(attention_kernel<128, true>); else launch(attention_kernel<128, false>); break;
-    case 192: if (fine) launch(attention_kernel<192, true>); else launch(attention_kernel<192, false>); break;
+    case 64: pick(std::integral_constant<int, 64>{}); break;
+    case 128: pick(std::integral_constant<int, 128>{}); break;
+    case 192: pick(std::integral_constant<int, 192>{}); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

@@ -396,8 +396,8 @@ int bibo_moe_exp_attn_res_fwd(const void* const* candidates, int n_candidates, c
  * bibo_moe_exp_rope_tables: cos, sin bf16 [S, 2 half] of position * inv_freq[half] in fp32, both halves of a row alike.
  * bibo_moe_exp_attention_fwd: out [B*S, n_heads * head_dim] = causal attention of those rows (window > 0: restricted to the
  *   last `window` keys), softmax in fp32, with the XSA correction y - tanh(alpha) <y, vn> vn (xsa_alpha [n_heads] or NULL;
- *   src/modeling/attn/xsa.py:41-54).  head_dim in {64, 128, 192}; n_heads / n_kv_heads = 1 or even; ld at most 2^26
- *   (BIBO_ERR_UNSUPPORTED otherwise).
+ *   src/modeling/attn/xsa.py:41-54).  head_dim in {64, 128, 192}; n_heads / n_kv_heads = 1 or even (BIBO_ERR_UNSUPPORTED
+ *   otherwise).
  * bibo_moe_exp_norm_attention_fwd: bibo_moe_exp_qk_norm_rope and bibo_moe_exp_attention_fwd of the same rows, the same bits; of many
  *   rows only the keys are normalised and rotated in place, the queries on their way into the attention (qkv then keeps them as they were).
  */

@@ -121,6 +121,19 @@ def test_attention_takes_the_queries_as_the_norm_kernel_does(D, nq, nkv, S, wind
     assert torch.equal(one[:, :nq * D], (rows if many else two)[:, :nq * D]) and torch.equal(one[:, nq * D:], two[:, nq * D:])
 
 
+@pytest.mark.parametrize("D,nq,nkv,S,window", [(64, 2, 1, 33, 0), (192, 2, 2, 31, 16)])
+def test_attention_of_rows_far_apart(D, nq, nkv, S, window):
+    """Rows whose 32-key blocks span more than 2^32 bytes leave the bits of packed rows."""
+    w, far = (nq + 2 * nkv) * D, (1 << 26) + 8
+    packed = torch.randn(S, w, generator=torch.Generator(device=DEV).manual_seed(S), device=DEV).bfloat16()
+    apart = torch.empty((S - 1) * far + w, dtype=torch.bfloat16, device=DEV)
+    apart.as_strided((S, w), (far, 1)).copy_(packed)
+    out = [torch.empty(S, nq * D, dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+    for rows, ld, o in ((packed, w, out[0]), (apart, far, out[1])):
+        _call("bibo_moe_exp_attention_fwd", _ptr(rows), ld, 1, S, nq, nkv, D, window, ctypes.c_float(D ** -0.5), None, 1, _ptr(o))
+    assert torch.isfinite(out[0]).all() and torch.equal(*out)
+
+
 def test_attention_refuses_what_it_does_not_take():
     args = lambda nq, nkv, D: (None, 4096, 1, 4, nq, nkv, D, 0, ctypes.c_float(1.0), None, 1, None, None)
     for nq, nkv, D in ((4, 2, 96), (3, 2, 64), (3, 1, 64), (4, 0, 64)):
