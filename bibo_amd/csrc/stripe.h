@@ -46,15 +46,16 @@ __device__ __forceinline__ TileMap make_tile_map(const int32_t* __restrict__ off
 
 // Tiles for a kernel whose workgroups fill a CU each, up to BM rows in whole 32-row blocks, and the tile of workgroup `bid`, if there is one
 // (first: its first row in its expert).  The rounds of kCUs tiles that tiles of BM rows would take are filled.
-// Heights: all tiles but an expert's last get the least number of blocks with which the call still fits those rounds.  T = 1024, k = 6 (H = 768,
-// I = 384): 57 -> 38 us, 2049: 57 -> 45, 3001: 57 -> 50.  Where LESS quarters of a block less would fit on average (and the rounds are FROM to TO), an expert's blocks are spread over so many tiles instead, two heights of them, and no CU waits for a last round of a few
-// tall ones.  (Full rounds take 29, 38, 51 and 67 us at one to four blocks: lower tiles cost a block little more.)  Layer, four layers' weights in
-// turn, one height -> two: T = 12,000: 214.6 -> 205.8 us, the same with four experts that every token picks: 213.2 -> 201.1, 16,384: 280.6 ->
-// 264.7; H = 512, I = 256: 160.1 -> 157.3 (16,384); H = 1024, I = 512, k = 8: 144.6 -> 136.5 (2500), 149.4 -> 147.1 (3001).  For less the
-// tiles' weights cost what it gives (one quarter: T = 40,000 and 16,384 of 32 experts 0 to 2 % slower; two: I = 384, T = 14,000 0.7 % slower, but
-// I = 256, H = 1024, T = 8192 4.6 against 2.2 % faster with three), and so they do on 64-row tiles in four rounds (T = 6000: 2 %).  In two rounds it gives 2 to 4 % at I = 256 (H = 512, T = 8192: 84.0 -> 81.6; H = 1024, T = 8192: 142.4 -> 137.2), at I = 384
-// -2 to 2 by the card (T = 8192: 142.8 -> 139.7, 135.1 -> 137.5), and at I = 128 up to 2 % less than nothing in two to four rounds (H = 640:
-// 112.5 -> 114.8 at T = 12,000).  TO == 0: all tiles fit one round.
+// Heights: all tiles but an expert's last get the least number of blocks with which the call still fits those rounds.  T = 1024, k = 6 (H = 768, I =
+// 384): 57 -> 38 us, 2049: 57 -> 45, 3001: 57 -> 50.  Where LESS quarters of a block less would fit on average (and the rounds are FROM to TO), an
+// expert's blocks are spread over so many tiles instead, two heights of them, and no CU waits for a last round of a few tall ones.  (Full rounds
+// take 29, 38, 51 and 67 us at one to four blocks: lower tiles cost a block little more.)  Layer, four layers' weights in turn, one height -> two: T
+// = 12,000: 214.6 -> 205.8 us, the same with four experts that every token picks: 213.2 -> 201.1, 16,384: 280.6 -> 264.7; H = 512, I = 256: 160.1 ->
+// 157.3 (16,384); H = 1024, I = 512, k = 8: 144.6 -> 136.5 (2500), 149.4 -> 147.1 (3001).  For less the tiles' weights cost what it gives (one
+// quarter: T = 40,000 and 16,384 of 32 experts 0 to 2 % slower; two: I = 384, T = 14,000 0.7 % slower, but I = 256, H = 1024, T = 8192 4.6 against
+// 2.2 % faster with three), and so they do on 64-row tiles in four rounds (T = 6000: 2 %).  In two rounds it gives 2 to 4 % at I = 256 (H = 512, T =
+// 8192: 84.0 -> 81.6; H = 1024, T = 8192: 142.4 -> 137.2), at I = 384 -2 to 2 by the card (T = 8192: 142.8 -> 139.7, 135.1 -> 137.5), and at I = 128
+// up to 2 % less than nothing in two to four rounds (H = 640: 112.5 -> 114.8 at T = 12,000).  TO == 0: all tiles fit one round.
 // Order: an XCD (ids congruent mod 8) has a contiguous range of the tiles, whose experts' weights share its L2.  (The tall ones in front, so
 // that the CUs end together, brings an expert's weights through the L2 once for each height: with weights from HBM 1 to 2 % slower in two
 // rounds, as fast in three and 5 % slower in eight.)
