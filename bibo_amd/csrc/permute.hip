@@ -58,8 +58,19 @@ __global__ __launch_bounds__(256) void hist_blocksum_kernel(const int32_t* __res
 // with ballots), 16 or 32 for the histograms the router kernel wrote per workgroup (a wave's count is the sum
 // of its 32/HT histograms and no counting pass is needed).
 // BATCH = histograms a wave requests together.  They are read whether a call has them or not (past the end: the last one again,
-// counted as zero), and each costs the wave 40 ns, so few histograms get a short batch: 6.7 -> 4.2 us at 32 of them (T = 512),
+// counted as zero), and each cost the wave 40 ns when it was a load of its own, so few histograms get a short batch: 6.7 -> 4.2 us at 32 of them (T = 512),
 // 6.3 -> 4.7 at 49.  Wave index and bounds are scalar: under per-lane conditions 256 of them took 7.3 us instead of 6.5 (T = 8192).
+// A load is four histograms, 16 bytes a lane, and up to 512 of them come in one round trip: one to a load, two round trips from 257 on -> now, us
+// under the profiler: 5.9 -> 5.3 at 256 (T = 8192), 9.5 -> 8.7 at 512, 6.3 -> 5.6 at 188 (T = 3001), 6.0 -> 5.4 at 128; layers by 0.2 to 0.6 %.
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef i32x4 i32x4_dword __attribute__((aligned(4)));       // a caller's workspace may start at any dword
+// the sum of what lanes l % 16 of the four rows of 16 hold, in all of them
+__device__ __forceinline__ int sum_rows16(int v) {
+  const auto a = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+  const unsigned s = a[0] + a[1];
+  const auto b = __builtin_amdgcn_permlane32_swap(s, s, false, false);
+  return (int)(b[0] + b[1]);
+}
 template <int HT, int BATCH>
 __global__ __launch_bounds__(256) void scatter_kernel(const int32_t* __restrict__ idx, int S, int E, int k,
                                                       const int32_t* __restrict__ hist, int nhist,
@@ -67,7 +78,7 @@ __global__ __launch_bounds__(256) void scatter_kernel(const int32_t* __restrict_
                                                       int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
                                                       int32_t* __restrict__ perm_slot, int32_t* __restrict__ perm_token) {
   static_assert(kPermTokens == 128 && (HT == kPermTokens || HT == 16 || HT == 32), "a wave owns 32 tokens");
-  __shared__ int part_tot[4][kMaxE], part_bef[4][kMaxE], wave_cnt[4][kMaxE];
+  __shared__ __attribute__((aligned(16))) int part_tot[4][kMaxE], part_bef[4][kMaxE], wave_cnt[4][kMaxE];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int b = blockIdx.x;
   const int s0 = (b * kPermTokens + wave * (kPermTokens / 4)) * k;
@@ -105,28 +116,38 @@ __global__ __launch_bounds__(256) void scatter_kernel(const int32_t* __restrict_
   }
   wave_cnt[wave][lane] = mycnt;
 
-  int tot = 0, bef = 0;
   constexpr int kBatch = BATCH;                    // histograms requested together: one memory latency per batch
-  if (BATCH < 64 || block_sum == nullptr) {
-    for (int bb0 = wave; bb0 < nhist; bb0 += 4 * kBatch) {
-      int v[kBatch];
+  if (BATCH != 64 || block_sum == nullptr) {
+    // a load is four histograms: lanes 16 q .. 16 q + 15 hold the four experts from 4 (lane % 16) on of the q-th
+    const int q = lane >> 4, c4 = (lane & 15) * 4;
+    i32x4 t4 = {0, 0, 0, 0}, b4 = {0, 0, 0, 0};
+    for (int bb0 = wave * 4 + q; bb0 - q < nhist; bb0 += 4 * kBatch) {
+      i32x4 v[kBatch / 4];
 #pragma unroll
-      for (int u = 0; u < kBatch; ++u) {
-        const int bb = min(bb0 + 4 * u, nhist - 1);
-        v[u] = (hist + (size_t)bb * kMaxE)[lane];
-      }
+      for (int u = 0; u < kBatch / 4; ++u)
+        v[u] = *reinterpret_cast<const i32x4_dword*>(hist + (unsigned)(min(bb0 + 16 * u, nhist - 1) * kMaxE + c4));
 #pragma unroll
-      for (int u = 0; u < kBatch; ++u) {
-        const int bb = bb0 + 4 * u;
-        tot += v[u] & (bb < nhist ? -1 : 0);
-        bef += v[u] & (bb < min(h0, nhist) ? -1 : 0);
+      for (int u = 0; u < kBatch / 4; ++u) {
+        const int bb = bb0 + 16 * u, all = bb < nhist ? -1 : 0, front = bb < min(h0, nhist) ? -1 : 0;
+        t4 += v[u] & i32x4{all, all, all, all};
+        b4 += v[u] & i32x4{front, front, front, front};
       }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      t4[i] = sum_rows16(t4[i]);
+      b4[i] = sum_rows16(b4[i]);
+    }
+    if (q == 0) {
+      *reinterpret_cast<i32x4*>(&part_tot[wave][c4]) = t4;
+      *reinterpret_cast<i32x4*>(&part_bef[wave][c4]) = b4;
     }
   } else if constexpr (BATCH == 64) {
     // two levels: the sums of whole blocks of histograms, then the histograms of this workgroup's own block in front
     // of its first one
     static_assert(kHistBlock == 4 * kBatch, "one batch per wave covers a block");
     const int nblk = (nhist + kHistBlock - 1) / kHistBlock, hb = h0 / kHistBlock;
+    int tot = 0, bef = 0;
     int v[kBatch];
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
@@ -140,9 +161,9 @@ __global__ __launch_bounds__(256) void scatter_kernel(const int32_t* __restrict_
     }
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) bef += v[u];
+    part_tot[wave][lane] = tot;
+    part_bef[wave][lane] = bef;
   }
-  part_tot[wave][lane] = tot;
-  part_bef[wave][lane] = bef;
   __syncthreads();
   const int total = (part_tot[0][lane] + part_tot[1][lane]) + (part_tot[2][lane] + part_tot[3][lane]);
   const int before = (part_bef[0][lane] + part_bef[1][lane]) + (part_bef[2][lane] + part_bef[3][lane]);
@@ -255,7 +276,8 @@ static void launch_scatter(const int32_t* idx, int S, int E, int k, const int32_
   if (nhist <= 4 * 8) launch(std::integral_constant<int, 8>());
   else if (nhist <= 4 * 24) launch(std::integral_constant<int, 24>());
   else if (nhist <= 4 * 48) launch(std::integral_constant<int, 48>());
-  else launch(std::integral_constant<int, 64>());
+  else if (nhist <= 4 * 64 || block_sum != nullptr) launch(std::integral_constant<int, 64>());
+  else launch(std::integral_constant<int, 128>());
 }
 
 hipError_t launch_permute(const int32_t* idx, int T, int E, int k, int32_t* counts, int32_t* offsets,

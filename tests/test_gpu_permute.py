@@ -78,3 +78,9 @@ def test_histogram_counts_around_the_batches(n):
     again, counts2 = ops.experts_fwd(x, idx, w, *ops_in[2:], algo="fused", want_counts=True)
     assert torch.equal(counts, counts2) and torch.equal(out, again)
     assert np.array_equal(counts.cpu().numpy(), np.bincount(idx.cpu().numpy().ravel(), minlength=16))
+
+
+@pytest.mark.parametrize("n", [3, 258, 259, 511, 512, 513, 1023])
+def test_histograms_four_to_a_load(n):
+    """A load is four histograms: counts that leave one to three over, and up to two rounds of 512."""
+    _check(_random_idx(128 * n - 5, 16, 2, n), 16)
