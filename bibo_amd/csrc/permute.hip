@@ -59,7 +59,7 @@ __global__ __launch_bounds__(256) void hist_blocksum_kernel(const int32_t* __res
 // of its 32/HT histograms and no counting pass is needed).
 // BATCH = histograms a wave requests together.  They are read whether a call has them or not (past the end: the last one again,
 // counted as zero), and each cost the wave 40 ns when it was a load of its own, so few histograms get a short batch: 6.7 -> 4.2 us at 32 of them (T = 512),
-// 6.3 -> 4.7 at 49.  Wave index and bounds are scalar: under per-lane conditions 256 of them took 7.3 us instead of 6.5 (T = 8192).
+// 6.3 -> 4.7 at 49.
 // A load is four histograms, 16 bytes a lane, and up to 512 of them come in one round trip: one to a load, two round trips from 257 on -> now, us
 // under the profiler: 5.9 -> 5.3 at 256 (T = 8192), 9.5 -> 8.7 at 512, 6.3 -> 5.6 at 188 (T = 3001), 6.0 -> 5.4 at 128; layers by 0.2 to 0.6 %.
 typedef int i32x4 __attribute__((ext_vector_type(4)));
