@@ -218,9 +218,9 @@ hipError_t launch_backward_gemms(BackwardGemms g, int T, int S, int chunk, int s
 //   dtheta (the row's share) = p'(theta) ln r sum_i q_i r^p a_i;  dw = <dh', h>, dh = w dh'.
 // `hidden` receives w h, the row the down projection's weight gradient contracts with d_out.
 // act = SiLU: h = SiLU(g) u, dg = q a'(g), no theta.  Rows of I <= kActMaxI elements.
-// Bound by the 12 I bytes of a row's way in and out (T = 8192, k = 6, I = 384: 226 MB) once the vector instructions are few: the reciprocal
-// unit instead of divisions, as in the forward, and two sums over the row beside that of its squares.  57 -> 40 us at that size, 5.6 TB/s
-// (37 -> 26 at T = 6000, I = 256; 37 -> 33 at T = 4000, k = 8, I = 512), every gradient as far from fp64 as before.
+// Bound by its vector instructions: the divisions are IEEE ones and the row has three sums besides that of its squares.  T = 8192, k = 6, I = 384:
+// 57 us for 226 MB, 4 TB/s; on the reciprocal unit, with two sums, 40 us.  That costs precision: a quotient off by an ulp in 14 of 525 rows
+// of one element where these are the nearest floats, and gradients that are other numbers by 1e-4 of their norm.
 constexpr int kActMaxI = 512;   // one 16-byte granule of the row per lane
 
 __global__ __launch_bounds__(256) void act_bwd_kernel(const bf16_t* __restrict__ gu, const bf16_t* __restrict__ dhp,
@@ -271,40 +271,42 @@ __global__ __launch_bounds__(256) void act_bwd_kernel(const bf16_t* __restrict__
     p = radial_exponent(theta, e, act);
     radial_row_scalars(ss, I, p, act, rinv, gain);             // 1 / r and r^p
   }
-  // with X = sum_i dh'_i u_i a_i and Y = sum_i dh'_i u_i a'_i z_i: dw = r^p X, the bracket of dg w r^(p-1) (p X - Y)
-  const float nrl = -1.44269504f * rinv;
-  float x_sum = 0.f, y_sum = 0.f;
+  const float r = 1.f / rinv;
+  float dot_h = 0.f, sum_qa = 0.f, inner = 0.f;
   float a_[8], ad_[8];
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
     const float z = g[q] * rinv;
-    const float s = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(g[q] * nrl));
+    const float s = 1.f / (1.f + __expf(-z));
     a_[q] = z * s;
-    ad_[q] = fmaf(a_[q], 1.f - s, s);
-    const float du = d[q] * u[q];
-    x_sum = fmaf(du, a_[q], x_sum);
-    y_sum = fmaf(du * ad_[q], z, y_sum);
+    ad_[q] = s * (1.f + z * (1.f - s));
+    dot_h = fmaf(d[q], gain * a_[q] * u[q], dot_h);
+    const float qq = ws * d[q] * u[q];
+    sum_qa = fmaf(qq, a_[q], sum_qa);
+    inner = fmaf(qq, gain * rinv * (p * a_[q] - ad_[q] * z), inner);    // p r^(p-1) a - r^(p-2) a' g = r^(p-1) (p a - a' z)
   }
-  x_sum = wave_sum(x_sum);
-  y_sum = wave_sum(y_sum);
-  const float wg = ws * gain, wgr = wg * rinv;
+  dot_h = wave_sum(dot_h);
+  sum_qa = wave_sum(sum_qa);
+  inner = wave_sum(inner);
   if (live) {
-    const float across = radial ? wgr * rinv * (p * x_sum - y_sum) * (1.f / (float)I) : 0.f;
     bf16x8 og, ou, oh;
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-      og[q] = (bf16_t)fmaf(g[q], across, wgr * (d[q] * u[q] * ad_[q]));
-      ou[q] = (bf16_t)(wg * (d[q] * a_[q]));
-      oh[q] = (bf16_t)(wg * (a_[q] * u[q]));                   // w h: the weight gradient's operand (moe.py:92-93)
+      const float dh = ws * d[q];
+      float dg = dh * u[q] * gain * rinv * ad_[q];
+      if (radial) dg = fmaf(g[q] * rinv / (float)I, inner, dg);
+      og[q] = (bf16_t)dg;
+      ou[q] = (bf16_t)(dh * gain * a_[q]);
+      oh[q] = (bf16_t)(ws * gain * a_[q] * u[q]);              // w h: the weight gradient's operand (moe.py:92-93)
     }
     *reinterpret_cast<bf16x8*>(dgu + (size_t)row * 2 * I + lane * 8) = og;
     *reinterpret_cast<bf16x8*>(dgu + (size_t)row * 2 * I + I + lane * 8) = ou;
     *reinterpret_cast<bf16x8*>(hidden + (size_t)row * I + lane * 8) = oh;
   }
   if (lane == 0) {
-    dw_slot[slot] = gain * x_sum;
+    dw_slot[slot] = dot_h;
     const float dp = act == BIBO_ACT_RADIAL_TANH ? 1.f - p * p : p * (1.f - p);
-    dtheta_row[row] = radial ? dp * __logf(1.f / rinv) * wg * x_sum : 0.f;
+    dtheta_row[row] = radial ? dp * __logf(r) * gain * sum_qa : 0.f;
   }
 }
 
