@@ -4,6 +4,7 @@
 // what bounded every call below a few thousand tokens.
 //
 // Nothing here computes: tensors are checked, results allocated, one library function called.
+#include <ATen/SavedTensorHooks.h>
 #include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/extension.h>
@@ -349,7 +350,7 @@ class LayerFn : public torch::autograd::Function<LayerFn> {
 
 // x and the parameters as the caller holds them, then their kernel-dtype copies -> (out like x in compute dtype, counts or None, whether the
 // balancing step is done).  accumulated, balance_bias, factor, update: the arguments of balance_step, where the caller leaves the step to this
-// call; counts only come back if it could not take it.
+// call; counts only come back if it did not take it.
 py::tuple layer_train(const Tensor& x, const Tensor& w_router, const Tensor& w_gate_up, const Tensor& w_down, const Tensor& theta,
                       const Tensor& wr_k, const Tensor& bias_k, const Tensor& gu_k, const Tensor& dn_k, const Tensor& th_k, int k,
                       int norm, int algo, int n_pos, int n_neg, int act, bool want_counts, at::ScalarType compute, bool keep,
@@ -359,7 +360,10 @@ py::tuple layer_train(const Tensor& x, const Tensor& w_router, const Tensor& w_g
   TrainCall c{{wr_k, bias_k, gu_k, dn_k, th_k, k, norm, algo, n_pos, n_neg, act}, compute, keep, Tensor()};
   const int64_t E = gu_k.size(0) + n_pos + n_neg;
   bibo_moe_balance balance;
-  if (accumulated.has_value() && balance_bias.has_value()) {
+  // A pack hook may end this call behind the forward's launches, as activation checkpointing ends a recomputation with the last tensor it
+  // needs: the caller then counts no step, so none may have been taken.
+  const bool hooked = !at::SavedTensorDefaultHooks::get_tls_state().stack.empty();
+  if (accumulated.has_value() && balance_bias.has_value() && !hooked) {
     check_tensor(*accumulated, "accumulated_tpe", at::kFloat, {E});
     check_tensor(*balance_bias, "bias", at::kFloat, {E});
     balance = {static_cast<float*>(accumulated->data_ptr()), static_cast<float*>(balance_bias->data_ptr()), (float)factor, update ? 1 : 0};

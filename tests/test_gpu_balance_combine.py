@@ -2,6 +2,7 @@
 of its own: the same counts and biases, bit for bit, with updates in between, through every combine kernel."""
 import pytest
 import torch
+import torch.utils.checkpoint
 
 import bibo_amd
 
@@ -45,3 +46,34 @@ def test_replaced_balance_is_called():
     layer._balance = lambda counts, n: seen.append((int(counts.sum()), n))
     layer(torch.randn(1, 60, 128, device=DEV))
     assert seen == [(240, 60)] and float(layer.accumulated_tpe.abs().max()) == 0
+
+
+def _small(**kw):
+    cfg = bibo_amd.BiBoMoEConfig(hidden_size=128, moe_intermediate_size=128, num_routed_experts=16, num_experts_per_tok=4, special_expert_pairs=0, **kw)
+    layer = bibo_amd.BiBoMoELayer(cfg).to(DEV).train()
+    for p in (layer.gate.gate_proj.weight, layer.experts.gate_up_proj, layer.experts.down_proj):
+        p.data = p.data.bfloat16()
+    return layer, torch.randn(1, 60, 128, device=DEV, dtype=torch.bfloat16, requires_grad=True)
+
+
+def test_a_recomputation_takes_no_step_of_its_own():
+    """Checkpointing ends the recomputation with the last tensor it needs, in front of the balancing step: with a cadence of two forwards the
+    bias moves with every second one, from the counts of two."""
+    layer, x = _small(bias_update_threshold=120)
+    plain, _ = _small(bias_update_threshold=120)
+    plain.load_state_dict(layer.state_dict())
+    for step in range(4):
+        torch.utils.checkpoint.checkpoint(layer, x, use_reentrant=False).sum().backward()
+        plain(x)
+        assert layer._fwd_step == plain._fwd_step == step + 1
+        assert torch.equal(layer.accumulated_tpe, plain.accumulated_tpe) and torch.equal(layer.gate.bias, plain.gate.bias)
+    assert float(layer.gate.bias.abs().max()) > 0
+
+
+def test_a_forward_that_a_hook_ends_takes_no_step():
+    layer, x = _small(bias_update_threshold=1)
+    def refuse(t):
+        raise RuntimeError("refused")
+    with pytest.raises(RuntimeError, match="refused"), torch.autograd.graph.saved_tensors_hooks(refuse, lambda t: t):
+        layer(x)
+    assert layer._fwd_step == 0 and float(layer.gate.bias.abs().max()) == 0 and float(layer.accumulated_tpe.abs().max()) == 0
