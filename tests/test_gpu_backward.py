@@ -37,7 +37,8 @@ def _run(T, H, E, k, I, norm="sum", act="radial", seed=0, theta="normal", scale=
 
 @pytest.mark.parametrize("T,H,E,k,I", [(300, 256, 16, 4, 128), (512, 512, 64, 6, 256), (64, 384, 8, 2, 384), (1000, 768, 64, 6, 384),
                                        (200, 1024, 16, 4, 512),      # the widest rows the backward pass takes
-                                       (600, 256, 4, 2, 128), (700, 768, 5, 3, 384)])   # 300 / 420 rows per expert: 256-row tiles
+                                       (600, 256, 4, 2, 128), (700, 768, 5, 3, 384),    # 300 / 420 rows per expert: 256-row tiles
+                                       (9000, 1152, 4, 2, 128)])     # w_router's gradient: columns beyond 1024, row ranges of more than 256
 def test_backward_matches_oracle(T, H, E, k, I):
     got, ref, _ = _run(T, H, E, k, I, seed=T)
     for name in ("w", "x", "w_down", "w_gate_up", "w_router", "theta"):
@@ -45,7 +46,8 @@ def test_backward_matches_oracle(T, H, E, k, I):
 
 
 @pytest.mark.parametrize("T,H,Eg,n_pos,n_neg,k,I,norm", [(300, 256, 6, 1, 1, 3, 128, "sum"), (1000, 768, 62, 1, 1, 6, 384, "sum"),
-                                                         (200, 256, 5, 2, 0, 4, 128, "softmax"), (64, 384, 3, 0, 2, 2, 256, False)])
+                                                         (200, 256, 5, 2, 0, 4, 128, "softmax"), (64, 384, 3, 0, 2, 2, 256, False),
+                                                         (6000, 1152, 3, 1, 1, 2, 128, "sum")])
 def test_backward_with_identity_experts_matches_oracle(T, H, Eg, n_pos, n_neg, k, I, norm):
     """+/-Identity experts (moe.py:95-99, on by default in the reference's configuration): a slot routed to one sends
     +/- w d_out to d_x and +/- <d_out, x> to its combine weight, hence to the router; its router row gets a gradient,

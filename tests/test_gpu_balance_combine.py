@@ -15,6 +15,8 @@ DEV = torch.device("cuda:0")
     (torch.bfloat16, 40, 256, 512, 9, 2, 1),       # fp32 slot rows, 4 columns a thread
     (torch.float32, 777, 64, 32, 63, 3, 0),
     (torch.float32, 60, 50, 30, 5, 2, 1),          # one column a thread
+    (torch.bfloat16, 60, 50, 30, 5, 2, 1),
+    (torch.bfloat16, 300, 1024, 512, 8, 2, 0),     # counts from workgroups that find their rows themselves
     (torch.float32, 4, 64, 32, 8, 3, 0),           # few tokens: no combine
     (torch.bfloat16, 1, 256, 128, 8, 2, 0),
 ])

@@ -121,10 +121,11 @@ def test_attention_takes_the_queries_as_the_norm_kernel_does(D, nq, nkv, S, wind
     assert torch.equal(one[:, :nq * D], (rows if many else two)[:, :nq * D]) and torch.equal(one[:, nq * D:], two[:, nq * D:])
 
 
+@pytest.mark.parametrize("far", [1 << 26, (1 << 26) + 8])
 @pytest.mark.parametrize("D,nq,nkv,S,window", [(64, 2, 1, 33, 0), (192, 2, 2, 31, 16)])
-def test_attention_of_rows_far_apart(D, nq, nkv, S, window):
-    """Rows whose 32-key blocks span more than 2^32 bytes leave the bits of packed rows."""
-    w, far = (nq + 2 * nkv) * D, (1 << 26) + 8
+def test_attention_of_rows_far_apart(D, nq, nkv, S, window, far):
+    """Rows so far apart that the last row of a 32-key block is just in reach of 32-bit offsets, and just out of it, leave the bits of packed rows."""
+    w = (nq + 2 * nkv) * D
     packed = torch.randn(S, w, generator=torch.Generator(device=DEV).manual_seed(S), device=DEV).bfloat16()
     apart = torch.empty((S - 1) * far + w, dtype=torch.bfloat16, device=DEV)
     apart.as_strided((S, w), (far, 1)).copy_(packed)

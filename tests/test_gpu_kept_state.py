@@ -22,6 +22,7 @@ CASES = [  # dtype, T, H, I, E, k, pairs
     (BF16, 200, 200, 72, 8, 2, 0),      # bf16 on fp32 tiles
     (BF16, 40, 256, 512, 8, 2, 0),      # I = 512: streaming, then tiles cut by columns, one round of tiles and several
     (BF16, 300, 256, 512, 8, 2, 1),
+    (BF16, 300, 1024, 512, 8, 2, 0),    # whose workgroups find their rows themselves
     (BF16, 1500, 256, 512, 8, 4, 0),
     (BF16, 9000, 128, 512, 40, 4, 0),
 ]
