@@ -323,11 +323,11 @@ __device__ __forceinline__ float weight_to_score_grad(float dw, float w, float s
 }
 __device__ __forceinline__ float score_of(float logit) { return 1.f / (1.f + __expf(-logit)); }
 
-// dW_router[e, c] = sum over the rows r of expert e of dl[slot(r)] x[token(r), c], in two steps.  Step 1: block (g, z) takes the z-th of
-// kDwrSplit equal row ranges of row chunk g of the plan (kmajor.h: an expert's rows, cut where an expert holds many); 32 threads share a
-// row, 256 columns at a time, the eight partial sums meet in LDS in a fixed order -> part[g][z][c] fp32.  Step 2 adds the ranges of an
-// expert's chunks in order.  A row's token and dl go through LDS, 256 rows at a time: as loads of each of its threads they were three of four
-// load instructions, 16 cycles of a CU's address unit each.
+// dW_router[e, c] = sum over the rows r of expert e of dl[slot(r)] x[token(r), c], in two steps.  Step 1: a block takes the z-th of
+// kDwrSplit equal row ranges of row chunk g of the plan (kmajor.h: an expert's rows, cut where an expert holds many) and `width` columns
+// (dwr_width); 32 threads share a row, 256 columns at a time, the eight partial sums meet in LDS in a fixed order -> part[g][z][c] fp32.
+// Step 2 adds the ranges of an expert's chunks in order.  A row's token and dl go through LDS, 256 rows at a time: as loads of each of
+// its threads they were three of four load instructions, 16 cycles of a CU's address unit each.
 constexpr int kDwrSplit = 8, kDwrRows = 4, kDwrTurns = 4;
 struct DwrShared {
   float red[8][256], d[256];
@@ -335,68 +335,80 @@ struct DwrShared {
 };
 template <typename SlotGrad>
 __device__ __forceinline__ void dwr_block(DwrShared& sh, const bf16_t* __restrict__ x, SlotGrad slot_grad, const int* __restrict__ plan,
-                                          const int32_t* __restrict__ perm_slot, const int32_t* __restrict__ perm_token, int H, int g, int z,
-                                          float* __restrict__ part) {
+                                          const int32_t* __restrict__ perm_slot, const int32_t* __restrict__ perm_token, int H, int width,
+                                          int block, float* __restrict__ part) {
+  const int across = (H + width - 1) / width, range = block / across;
+  const int g = range / kDwrSplit, z = range % kDwrSplit, c0 = (block - range * across) * width, c1 = min(c0 + width, H);
   if (g >= plan[0]) return;
   const int tid = threadIdx.x, cg = tid & 31, rl = tid >> 5;
   const int lo_e = plan[4 + 4 * g + 1], n = plan[4 + 4 * g + 2] - lo_e;
   const int per = (n + kDwrSplit - 1) / kDwrSplit;
   const int lo = lo_e + min(z * per, n), hi = lo_e + min((z + 1) * per, n);
-  for (int h0 = 0; h0 < H; h0 += 256 * kDwrTurns) {             // (once up to H = 1024)
-    float acc[kDwrTurns][8];
+  float acc[kDwrTurns][8];
 #pragma unroll
-    for (int i = 0; i < kDwrTurns; ++i)
+  for (int i = 0; i < kDwrTurns; ++i)
 #pragma unroll
-      for (int q = 0; q < 8; ++q) acc[i][q] = 0.f;
-    for (int r0 = lo; r0 < hi; r0 += 256) {
-      const int rows = min(hi - r0, 256);
-      __syncthreads();                                          // the rows before have been read
-      if (tid < rows) {
-        sh.token[tid] = perm_token[r0 + tid];
-        sh.d[tid] = slot_grad(perm_slot[r0 + tid]);
-      }
-      __syncthreads();
-#pragma unroll
-      for (int i = 0; i < kDwrTurns; ++i) {
-        const int c = h0 + i * 256 + cg * 8;
-        if (c >= H) continue;
-        const bf16_t* const xc = x + c;
-        auto add = [&](float d, const bf16x8& v) {
-#pragma unroll
-          for (int q = 0; q < 8; ++q) acc[i][q] = fmaf(d, (float)v[q], acc[i][q]);
-        };
-        int r = rl;
-        for (; r + 8 * (kDwrRows - 1) < rows; r += 8 * kDwrRows) {   // several rows on their way together
-          bf16x8 v[kDwrRows];
-#pragma unroll
-          for (int u = 0; u < kDwrRows; ++u) v[u] = *reinterpret_cast<const bf16x8*>(xc + (size_t)sh.token[r + 8 * u] * H);
-#pragma unroll
-          for (int u = 0; u < kDwrRows; ++u) add(sh.d[r + 8 * u], v[u]);
-        }
-        for (; r < rows; r += 8) add(sh.d[r], *reinterpret_cast<const bf16x8*>(xc + (size_t)sh.token[r] * H));
-      }
+    for (int q = 0; q < 8; ++q) acc[i][q] = 0.f;
+  for (int r0 = lo; r0 < hi; r0 += 256) {
+    const int rows = min(hi - r0, 256);
+    __syncthreads();                                            // the rows before have been read
+    if (tid < rows) {
+      sh.token[tid] = perm_token[r0 + tid];
+      sh.d[tid] = slot_grad(perm_slot[r0 + tid]);
     }
+    __syncthreads();
 #pragma unroll
     for (int i = 0; i < kDwrTurns; ++i) {
-      if (h0 + i * 256 >= H) break;
-      __syncthreads();                                          // the sums before have been read
+      const int c = c0 + i * 256 + cg * 8;
+      if (c >= c1) continue;
+      const bf16_t* const xc = x + c;
+      auto add = [&](float d, const bf16x8& v) {
 #pragma unroll
-      for (int q = 0; q < 8; ++q) sh.red[rl][cg * 8 + q] = acc[i][q];
-      __syncthreads();
-      const int col = h0 + i * 256 + tid;
-      if (col < H)
-        part[((size_t)g * kDwrSplit + z) * H + col] = ((sh.red[0][tid] + sh.red[1][tid]) + (sh.red[2][tid] + sh.red[3][tid])) +
-                                                      ((sh.red[4][tid] + sh.red[5][tid]) + (sh.red[6][tid] + sh.red[7][tid]));
+        for (int q = 0; q < 8; ++q) acc[i][q] = fmaf(d, (float)v[q], acc[i][q]);
+      };
+      int r = rl;
+      for (; r + 8 * (kDwrRows - 1) < rows; r += 8 * kDwrRows) {     // several rows on their way together
+        bf16x8 v[kDwrRows];
+#pragma unroll
+        for (int u = 0; u < kDwrRows; ++u) v[u] = *reinterpret_cast<const bf16x8*>(xc + (size_t)sh.token[r + 8 * u] * H);
+#pragma unroll
+        for (int u = 0; u < kDwrRows; ++u) add(sh.d[r + 8 * u], v[u]);
+      }
+      for (; r < rows; r += 8) add(sh.d[r], *reinterpret_cast<const bf16x8*>(xc + (size_t)sh.token[r] * H));
     }
   }
+#pragma unroll
+  for (int i = 0; i < kDwrTurns; ++i) {
+    if (c0 + i * 256 >= c1) break;
+    __syncthreads();                                            // the sums before have been read
+#pragma unroll
+    for (int q = 0; q < 8; ++q) sh.red[rl][cg * 8 + q] = acc[i][q];
+    __syncthreads();
+    const int col = c0 + i * 256 + tid;
+    if (col < c1)
+      part[((size_t)g * kDwrSplit + z) * H + col] = ((sh.red[0][tid] + sh.red[1][tid]) + (sh.red[2][tid] + sh.red[3][tid])) +
+                                                    ((sh.red[4][tid] + sh.red[5][tid]) + (sh.red[6][tid] + sh.red[7][tid]));
+  }
+}
+
+// Columns of a block: all turns, fewer where less than two blocks a CU would come of it, which then read for longer than the rest of their
+// launch takes.  All columns in a block -> this, backward pass, us: T = 16384, H = 4096, four experts: 953 -> 621; 8192, 2048, eight: 256 -> 213;
+// 8192, 1536, four: 267 -> 205; 300, 1024, sixteen: 72 -> 69; with +/-Identity experts 8192, 2048, nine: 262 -> 226.  Half as many blocks at
+// least, or twice as many: the same within 1 %.
+constexpr int kDwrLeast = 512;
+int dwr_blocks(int slots, int H, int width) { return slots * kDwrSplit * ((H + width - 1) / width); }
+int dwr_width(int slots, int H) {
+  int width = 256 * kDwrTurns;
+  while (width > 256 && dwr_blocks(slots, H, width) < kDwrLeast) width /= 2;
+  return width;
 }
 
 // where +/-Identity experts make a slot's gradient a dot product, which token_bwd_kernel works out
 __global__ __launch_bounds__(256) void dwr_partial_kernel(const bf16_t* __restrict__ x, const float* __restrict__ dl, const int* __restrict__ plan,
                                                           const int32_t* __restrict__ perm_slot, const int32_t* __restrict__ perm_token,
-                                                          int H, float* __restrict__ part) {
+                                                          int H, int width, float* __restrict__ part) {
   __shared__ DwrShared sh;
-  dwr_block(sh, x, [&](int slot) { return dl[slot]; }, plan, perm_slot, perm_token, H, blockIdx.x, blockIdx.y, part);
+  dwr_block(sh, x, [&](int slot) { return dl[slot]; }, plan, perm_slot, perm_token, H, width, blockIdx.x, part);
 }
 
 // Everything per token behind the experts, one wave per token and run of up to 512 columns (`parts` runs of equal length):
@@ -406,20 +418,22 @@ __global__ __launch_bounds__(256) void dwr_partial_kernel(const bf16_t* __restri
 //   dx[t, c] = sum_j (dx row of slot j + dl[t, j] W_router[idx[t, j], c]).
 // A slot whose expert id lies outside [0, E + n_pos + n_neg) (padding in a caller's indices, which the forward pass skips) has no
 // dx row and no combine-weight gradient: it is left out and its dw_slot entry set to zero.  Every wave of a token works out the k
-// scalars, the first one stores them.  Bound by reading the slots' dx rows (T = 8192, H = 768, k = 6: 75 MB), which are requested
+// scalars, the first one stores them (without DWR).  Bound by reading the slots' dx rows (T = 8192, H = 768, k = 6: 75 MB), which are requested
 // before the indices that decide about them are back.  K = k at compile time, and no load under a condition: the compiler
 // drains all loads where a branch around one ends (k at run time: 26 us at that size, 21 like this).
 // DWR: the first nb_dwr workgroups are dwr_partial_kernel's (the ranges of a chunk next to each other) and work out
 // dl of their rows' slots themselves, so that they need not wait for this launch.  Both launches -> this one, us: 40.0 -> 31.4 (T = 8192, H = 768,
-// k = 6), 20.4 -> 13.2 (6000, 512, 6), 29.3 -> 25.7 (4000, 1024, 8), 8.7 -> 6.2 (1111, 512, 2); with 256 columns a workgroup, each of which
-// works dl out again, 35.3, 14.0, 28.8 and 5.0; with dl from workgroups behind the GEMMs' 32.6, 15.0, 26.9 and 4.4, and 1 to 7 more in the GEMMs.
+// k = 6), 20.4 -> 13.2 (6000, 512, 6), 29.3 -> 25.7 (4000, 1024, 8); with 256 columns a workgroup, each of which
+// works dl out again, 35.3, 14.0 and 28.8; with dl from workgroups behind the GEMMs' 32.6, 15.0 and 26.9, and 1 to 7 more in the GEMMs.  (1111, 512, 2,
+// sixteen experts: 8.7 -> 5.0 with 256 columns, which dwr_width takes there.)  Neither dl nor dw_slot is written then: every slot must be an
+// expert's with weights (E is all there is, the indices the router's), whose dw_slot entry act_bwd_kernel has left.
 template <int K, bool DWR>
 __global__ __launch_bounds__(256) void token_bwd_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ d_out,
                                                         const bf16_t* __restrict__ dxs, const float* __restrict__ logits,
                                                         const int32_t* __restrict__ idx, const float* __restrict__ w,
                                                         const bf16_t* __restrict__ w_router, int T, int H, int E, int n_pos,
                                                         int n_neg, int norm_mode, int parts, float* __restrict__ dw_slot,
-                                                        float* __restrict__ dl, bf16_t* __restrict__ dx, int nb_dwr,
+                                                        float* __restrict__ dl, bf16_t* __restrict__ dx, int nb_dwr, int dwr_cols,
                                                         const int* __restrict__ plan, const int32_t* __restrict__ perm_slot,
                                                         const int32_t* __restrict__ perm_token, float* __restrict__ dwr_part) {
   if constexpr (DWR) {
@@ -443,7 +457,7 @@ __global__ __launch_bounds__(256) void token_bwd_kernel(const bf16_t* __restrict
           if (j == mine) { s_ = s[j]; dw_ = dw[j]; w_ = wj[j]; }
         }
         return weight_to_score_grad<K>(dw_, w_, sum, dot, norm_mode) * s_ * (1.f - s_);
-      }, plan, perm_slot, perm_token, H, blockIdx.x / kDwrSplit, blockIdx.x % kDwrSplit, dwr_part);
+      }, plan, perm_slot, perm_token, H, dwr_cols, blockIdx.x, dwr_part);
       return;
     }
   }
@@ -673,12 +687,12 @@ hipError_t launch_backward(const void* x, const void* d_out, const void* w_route
   const bool with_router = w_router != nullptr;      // else: the experts alone, the caller owns the routing
   const bool merged = with_router && E == Et;        // the router's partial sums beside the tokens: their slots are the experts'
   const int parts = (H / 8 + kWave - 1) / kWave;     // runs of columns a lane each
-  const int nb_dwr = slots * kDwrSplit;
+  const int dwr_cols = dwr_width(slots, H), nb_dwr = dwr_blocks(slots, H, dwr_cols);
   auto token_bwd = [&](auto kc, auto with_dwr) {
     constexpr bool DWR = decltype(with_dwr)::value;
     hipLaunchKernelGGL((token_bwd_kernel<decltype(kc)::value, DWR>), dim3((unsigned)(((long long)T * parts + 3) / 4) + (DWR ? nb_dwr : 0)), dim3(256),
                        0, s, xp, dop, dxs, logits, idx, w, wrp, T, H, E, n_pos, n_neg, norm_mode, parts, b.dw_slot, b.dl,
-                       static_cast<bf16_t*>(dx), nb_dwr, b.wgrad_plan, perm_slot, perm_token, b.dwr_part);
+                       static_cast<bf16_t*>(dx), nb_dwr, dwr_cols, b.wgrad_plan, perm_slot, perm_token, b.dwr_part);
   };
   auto token_launch = [&](auto kc) {
     if (merged) token_bwd(kc, std::true_type());
@@ -697,8 +711,7 @@ hipError_t launch_backward(const void* x, const void* d_out, const void* w_route
     default: token_launch(integral_constant<int, 8>{});
   }
   if (with_router && !merged)
-    hipLaunchKernelGGL(dwr_partial_kernel, dim3(slots, kDwrSplit), dim3(256), 0, s, xp, b.dl, b.wgrad_plan,
-                       perm_slot, perm_token, H, b.dwr_part);
+    hipLaunchKernelGGL(dwr_partial_kernel, dim3(nb_dwr), dim3(256), 0, s, xp, b.dl, b.wgrad_plan, perm_slot, perm_token, H, dwr_cols, b.dwr_part);
   // the sums that end the pass: cut experts' partial tiles, dtheta, the router's weight gradient
   const int nb_w = (int)(((size_t)2 * I * H / 4 + 255) / 256);
   const int nb_r = with_router ? (Et * H + 255) / 256 : 0;
