@@ -60,8 +60,10 @@ __global__ __launch_bounds__(256) void hist_blocksum_kernel(const int32_t* __res
 // BATCH = histograms a wave requests together.  They are read whether a call has them or not (past the end: the last one again,
 // counted as zero), and each cost the wave 40 ns when it was a load of its own, so few histograms get a short batch: 6.7 -> 4.2 us at 32 of them (T = 512),
 // 6.3 -> 4.7 at 49.
-// A load is four histograms, 16 bytes a lane, and up to 512 of them come in one round trip: one to a load, two round trips from 257 on -> now, us
-// under the profiler: 5.9 -> 5.3 at 256 (T = 8192), 9.5 -> 8.7 at 512, 6.3 -> 5.6 at 188 (T = 3001), 6.0 -> 5.4 at 128; layers by 0.2 to 0.6 %.
+// A load is four histograms, 16 bytes a lane, and up to 384 of them come in one round trip.  A load for each, 256 a round trip -> now, us under the
+// profiler, 64 experts, k = 6: 7.8 -> 5.4 at 284 histograms (T = 9000), 8.4 -> 6.6 at 512, 9.7 -> 6.0 at 628, 9.8 -> 6.1 at 752, 11.9 -> 7.9 at 1020;
+// 5.9 -> 5.3 at 256, 6.3 -> 5.6 at 188, 6.0 -> 5.4 at 128.  (512 a round trip are compiled into loads one behind the other: 7.8 at 512, 10.1 at
+// 628, 11.3 at 752; 256 take 5.8, 6.0, 7.0 and 7.2 from 284 on.)
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef i32x4 i32x4_dword __attribute__((aligned(4)));       // a caller's workspace may start at any dword
 // the sum of what lanes l % 16 of the four rows of 16 hold, in all of them
@@ -277,7 +279,7 @@ static void launch_scatter(const int32_t* idx, int S, int E, int k, const int32_
   else if (nhist <= 4 * 24) launch(std::integral_constant<int, 24>());
   else if (nhist <= 4 * 48) launch(std::integral_constant<int, 48>());
   else if (nhist <= 4 * 64 || block_sum != nullptr) launch(std::integral_constant<int, 64>());
-  else launch(std::integral_constant<int, 128>());
+  else launch(std::integral_constant<int, 96>());
 }
 
 hipError_t launch_permute(const int32_t* idx, int T, int E, int k, int32_t* counts, int32_t* offsets,

@@ -80,7 +80,7 @@ def test_histogram_counts_around_the_batches(n):
     assert np.array_equal(counts.cpu().numpy(), np.bincount(idx.cpu().numpy().ravel(), minlength=16))
 
 
-@pytest.mark.parametrize("n", [3, 258, 259, 511, 512, 513, 1023])
+@pytest.mark.parametrize("n", [3, 258, 259, 384, 385, 511, 512, 513, 768, 769, 1023])
 def test_histograms_four_to_a_load(n):
-    """A load is four histograms: counts that leave one to three over, and up to two rounds of 512."""
+    """A load is four histograms: counts that leave one to three over, and up to three rounds of 384."""
     _check(_random_idx(128 * n - 5, 16, 2, n), 16)
