@@ -243,7 +243,8 @@ py::tuple ffn_forward(const Tensor& h, const Tensor& norm_weight, double eps, co
 // forward = bibo_moe_forward_train, which leaves routing, permutation and, for most shapes, pre-activations in a state tensor (about 4 I
 // bytes per routed slot, 8 I for the fp32 tile kernels), and backward = bibo_moe_backward_saved; otherwise forward = bibo_moe_forward and
 // backward = bibo_moe_backward, which computes all of that again from the saved input rows.  The same gradients, bit for bit.
-// H = 192, I = 88, 16 experts, k = 3, T = 777 in fp32, forward and backward: 19 launches without, 15 with.
+// H = 192, I = 88, 16 experts, k = 3, T = 777 in fp32, forward and backward: 19 launches without, 13 with (one of them less for the
+// balancing step, which rides on the forward's combine, and one for the copy of the biases).
 struct TrainCall {
   Layer l;               // kernel-dtype copies of the parameters (the parameters themselves where they have that dtype)
   at::ScalarType compute;

@@ -134,6 +134,9 @@ struct QueryNorm {
 // are read and written once more, here they lengthen the chain in front of a wave's first product.  Both launches, us, queries in place / here,
 // 4 and 2 heads of 192, causal with norm and window 128 with norm and RoPE: T = 16384: 88.1 / 80.4 and 47.6 / 44.0; 8192: 76.8 / 71.6 and 32.2 /
 // 30.3; 4096: 71.6 / 70.2 and 26.8 / 26.5; 2048: 67.0 / 67.8 and 22.7 / 24.4; 128: 15.1 / 18.2.  Hence kQueryElems, the 4096 tokens of these.
+// Other heads, as long a call or longer, causal and window 128, 8 x 2048 tokens: 64 wide, 8 and 2: 65.4 / 54.6 and 39.3 / 27.7, 32 and 8: 231 / 185 and
+// 122 / 79; 128 wide, 2 and 2: 61.8 / 58.6 and 28.5 / 26.4, 32 and 8: 363 / 326 and 188 / 148.  Of 84 such calls the longest on this side of
+// the line is one sequence of 8192 in a window, 192 wide, 2 and 2 heads: 27.5 / 29.4.
 // weights(s, first half's 8, second half's 8), tables(s, cos, sin): of granule 2 s + h.
 template <int KS, typename Weights, typename Tables>
 __device__ __forceinline__ void norm_rope_query(const QueryNorm& nr, bf16x8 (&q)[KS], Weights weights, Tables tables) {

@@ -529,8 +529,8 @@ __global__ __launch_bounds__(256) void router_gateup_kernel(const bf16_t* __rest
 // round trips pass behind the other's arithmetic (one a CU: 30.0 -> 21.7 us at T = 16384, 26.9 -> 19.9 at 12000).  RING: six chunks of
 // w_router requested behind the rows, as in router_ring_kernel (H = 512, T = 1024: 10.8 -> 9.5 us; H = 768: 12.2 -> 11.4;
 // T = 16: 9.8 -> 10.8, so not there).  The chunks arrive together, not behind the norm's arithmetic: the first use of the norm's weights,
-// registers whose loads are older, is compiled into a wait for everything, and with fp32 weights so is each later one, which then waits for
-// the stores of the row before (H = 768, T = 2049: 11.8 us, where router_ring_kernel takes 8 without the norm).
+// registers whose loads are older, is compiled into a wait for everything (H = 768, T = 2049: 10.2 us, where router_ring_kernel takes 8 without
+// the norm).
 template <int TOK>
 constexpr int kNormTail = (TOK * kRowPad + kMaxE) * (int)sizeof(float) + TOK * (int)sizeof(unsigned long long);
 

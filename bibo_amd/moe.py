@@ -340,9 +340,11 @@ class BiBoMoELayer(nn.Module):
         self.register_buffer("accumulated_tpe", torch.zeros(config.num_routed_experts, dtype=torch.float))
         self._fwd_step = 0
         self._update_every = None
-        # Training forwards keep routing, permutation and gate/up pre-activations for their backward pass (about
-        # 4 * moe_intermediate_size bytes per routed slot until that backward has run), as autograd keeps the reference
-        # layer's activations; False makes the backward pass compute them again from the input rows instead.
+        # Training forwards keep what their backward pass would compute again, until that backward has run, as autograd keeps
+        # the reference layer's activations: every shape its routing and permutation; bf16 with sizes of the fused kernel
+        # (hidden a multiple of 128, expert 128, 256 or 384) also the gate/up pre-activations in bf16, 4 * moe_intermediate_size
+        # bytes per routed slot; fp32 and odd sizes on the fp32 tiles (multiples of four, more than 48 slots) in fp32, 8 * that
+        # (151 MB a layer at 8192 tokens, k = 6, 384 wide).  False makes the backward pass compute all of it from the input rows.
         self.keep_activations = True
         self.experts = BiBoFusedExperts(config)
         self.use_shared_expert = getattr(config, "use_shared_expert", False)
