@@ -469,7 +469,9 @@ class BiBoMoELayer(nn.Module):
             if torch.is_grad_enabled() and (hidden_states.requires_grad or any(p.requires_grad for p in params[:4])):
                 if not self._differentiable(cd):
                     raise NotImplementedError(_NO_BACKWARD)
-                native = self._native_balance(num_tokens, hidden_states.device) if balancing and self._balance_is_ours() else None
+                # (a shared expert may still raise, or its hooks look at the layer: the step then comes behind it)
+                ours = balancing and not self.use_shared_expert and self._balance_is_ours()
+                native = self._native_balance(num_tokens, hidden_states.device) if ours else None
                 out, counts, done = L.native().layer_train(hidden_states, *params[:4], *operands, *settings, self.keep_activations,
                                                            *(native[0] if native is not None else (None, None, 0.0, False)))
                 if done:                                       # with the forward's own launches

@@ -79,3 +79,18 @@ def test_a_forward_that_a_hook_ends_takes_no_step():
     with pytest.raises(RuntimeError, match="refused"), torch.autograd.graph.saved_tensors_hooks(refuse, lambda t: t):
         layer(x)
     assert layer._fwd_step == 0 and float(layer.gate.bias.abs().max()) == 0 and float(layer.accumulated_tpe.abs().max()) == 0
+
+
+def test_the_step_follows_the_shared_expert():
+    layer, x = _small(bias_update_threshold=1, use_shared_expert=True)
+    layer.shared_experts_list[0].bfloat16()
+    seen = []
+    def refuse(module, args):
+        seen.append((layer._fwd_step, float(layer.gate.bias.abs().max())))
+        if len(seen) == 1:
+            raise RuntimeError("refused")
+    layer.shared_experts_list[0].register_forward_pre_hook(refuse)
+    with pytest.raises(RuntimeError, match="refused"):
+        layer(x)
+    layer(x)
+    assert seen == [(0, 0.0), (0, 0.0)] and layer._fwd_step == 1 and float(layer.gate.bias.abs().max()) > 0
